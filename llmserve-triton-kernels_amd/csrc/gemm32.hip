@@ -1,0 +1,245 @@
+// 32-bit matrix products on the matrix cores:  C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]), float in, float out.
+// v_mfma_f32_16x16x4_f32 multiplies and adds in 32-bit (no reduced-precision mode) at the rate of the vector units, but takes
+// its operands from registers that a wave fills with 16-byte loads, so nothing but memory bounds the products of few rows.
+//
+//   gemm32_stream  M <= 64: the weight is read once, straight into the matrix instruction; a workgroup owns 16 or 32 weight
+//                  rows, its waves share K out in chunks of 32 and add their sums up in LDS in a fixed order.
+//   gemm32_tile    more rows: tiles through LDS, the next tile's loads in flight while the present one is multiplied.
+//
+// Both: K and the row stride of A multiples of 4, A and W 16-byte aligned (the host checks; what does not fit goes to
+// gemm_fma); M and N are arbitrary.  Loads go through a buffer that ends with the workgroup's last row; rows and columns that
+// do not exist are asked for beyond its end, which brings zeros and touches no memory (and no branch surrounds a load).
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+// Operand layout: lane l holds A[i = l % 16][k = l / 16] and B[k = l / 16][j = l % 16]; result D[i = 4 (l / 16) + r][j = l % 16].
+// A lane's four consecutive columns 4g .. 4g + 3 (one 16-byte load) serve four instructions: the sum over K takes the columns
+// of a group of 16 in another order, the same one for both operands.  i = weight row, j = row of A.
+__device__ __forceinline__ void fma_16x16x16(f32x4& acc, f32x4 w, f32x4 x) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[r], x[r], acc, 0, 0, 0);
+}
+
+#define NOWHERE 0x80000000u
+// The rows first .. first + rows - 1 (those below `all`) of a matrix with `ld` columns a row, `cols` of them used.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_buffer(const float* p, int first, int rows, int all, int ld, int cols) {
+    const unsigned bytes = (unsigned)(min(rows, all - first) - 1) * (unsigned)ld * 4u + (unsigned)cols * 4u;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p + (size_t)first * ld), 0, bytes, 0x00020000);
+}
+// four columns from k on of the row that starts `row` bytes into the buffer
+__device__ __forceinline__ f32x4 load_columns(__amdgpu_buffer_rsrc_t b, unsigned row, int k, int K) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, k < K ? row + (unsigned)k * 4u : NOWHERE, 0, 0));
+}
+__device__ __forceinline__ unsigned row_offset(int row, int rows, int ld) { return row < rows ? (unsigned)row * ld * 4u : NOWHERE / 2; }
+
+// ------------------------------------------------------------------------------ few rows
+// Bound by reading the weight: 32000 x 2048 (262 MB) at 2 rows takes 48 microseconds (5.4 TB/s), 11264 x 2048 22 (4.1 TB/s),
+// 2048 x 2048 9 (a launch and one wait for memory); the multiply-add kernel, whose workgroup brings 64 weight rows through
+// LDS 4 bytes a load whatever the number of rows, takes 282, 216 and 197.  At 64 rows 111, 56 and 23: from some 20 rows on
+// every workgroup's reading of all rows of X out of L2 weighs more than the weight.
+template <int MB, int NT, int WAVES, int UNROLL>
+__global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* __restrict__ C, const float* __restrict__ X,
+                                                                         const float* __restrict__ W,
+                                                                         const float* __restrict__ bias, int M, int N, int K,
+                                                                         int ldx, int ldc, int wide) {
+    __shared__ f32x4 red[WAVES][NT * MB][LLMS_WAVE];
+    const int wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE;
+    const int r16 = lane % 16, g = lane / 16;
+    const int n0 = blockIdx.x * 16 * NT;
+    const __amdgpu_buffer_rsrc_t w_buf = rows_buffer(W, n0, 16 * NT, N, K, K), x_buf = rows_buffer(X, 0, 16 * MB, M, ldx, K);
+    unsigned wrow[NT], xrow[MB];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wrow[t] = row_offset(t * 16 + r16, N - n0, K);
+#pragma unroll
+    for (int b = 0; b < MB; ++b) xrow[b] = row_offset(b * 16 + r16, M, ldx);
+    f32x4 acc[NT][MB];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) acc[t][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+    const int chunks = (K + 31) / 32;
+    for (int c0 = wave; c0 < chunks; c0 += WAVES * UNROLL) {
+        f32x4 wv[UNROLL][NT][2];
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) wv[u][t][s] = load_columns(w_buf, wrow[t], (c0 + u * WAVES) * 32 + s * 16 + g * 4, K);
+        __builtin_amdgcn_sched_barrier(0);  // (all of them are asked for before the first is used)
+#pragma unroll
+        for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int k = (c0 + u * WAVES) * 32 + s * 16 + g * 4;
+#pragma unroll
+                for (int b = 0; b < MB; ++b) {
+                    const f32x4 xv = load_columns(x_buf, xrow[b], k, K);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) fma_16x16x16(acc[t][b], wv[u][t][s], xv);
+                }
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int b = 0; b < MB; ++b) red[wave][t * MB + b][lane] = acc[t][b];
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < NT * MB * LLMS_WAVE; idx += WAVES * LLMS_WAVE) {
+        const int part = idx / LLMS_WAVE, l = idx % LLMS_WAVE;
+        const int n = n0 + (part / MB) * 16 + 4 * (l / 16), m = (part % MB) * 16 + l % 16;
+        if (m >= M || n >= N) continue;
+        f32x4 s = red[0][part][l];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) s += red[w][part][l];
+        float* c = C + (size_t)m * ldc + n;
+        if (wide && n + 4 <= N) {
+            if (bias)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[r] += bias[n + r];
+            *reinterpret_cast<f32x4*>(c) = s;
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (n + r < N) c[r] = s[r] + (bias ? bias[n + r] : 0.f);
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------ tiles
+// Bound by the matrix cores (157 TFLOP/s in 32-bit) once there are tiles for every compute unit: an instruction of 32 cycles
+// needs 8 bytes of LDS per lane, so one buffer and a plain order of stages are enough.  Measured: 4096 x 4096 at 2,048 rows 502
+// microseconds (137 TFLOP/s), 11264 x 2048 at 130 rows 106 (56; the multiply-add kernel 378), 2048 x 2048 at 130 rows 31 (220).
+template <int BM, int BN, int BK, int WM>
+__global__ __launch_bounds__(256) void gemm32_tile_kernel(float* __restrict__ C, const float* __restrict__ A,
+                                                          const float* __restrict__ W, const float* __restrict__ bias, int M,
+                                                          int N, int K, int lda, int ldc, int tiles_m, int wide) {
+    constexpr int WN = 4 / WM, TM = BM / WM / 16, TN = BN / WN / 16, LD = BK + 4;
+    constexpr int PER_ROW = BK / 4, CA = BM * PER_ROW / 256, CB = BN * PER_ROW / 256, STEP = 256 / PER_ROW;
+    __shared__ __attribute__((aligned(16))) float As[BM * LD];
+    __shared__ __attribute__((aligned(16))) float Bs[BN * LD];
+    // workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, rows fastest, so that the tiles
+    // which share a weight slab share an L2
+    const int nblk = gridDim.x, pid = blockIdx.x;
+    const int full = nblk / 8, rem = nblk % 8, xcd = pid % 8;
+    const int t = xcd * full + min(xcd, rem) + pid / 8;
+    const int m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
+    const int tid = threadIdx.x, wave = tid / LLMS_WAVE, lane = tid % LLMS_WAVE;
+    const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
+    const int r16 = lane % 16, g = lane / 16;
+    const int row = tid / PER_ROW, col = (tid % PER_ROW) * 4;
+
+    const __amdgpu_buffer_rsrc_t a_buf = rows_buffer(A, m0, BM, M, lda, K), w_buf = rows_buffer(W, n0, BN, N, K, K);
+    unsigned ap[CA], wp[CB];
+#pragma unroll
+    for (int c = 0; c < CA; ++c) ap[c] = row_offset(row + c * STEP, M - m0, lda);
+#pragma unroll
+    for (int c = 0; c < CB; ++c) wp[c] = row_offset(row + c * STEP, N - n0, K);
+    f32x4 ra[CA], rb[CB], acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int c = 0; c < CA; ++c) ra[c] = load_columns(a_buf, ap[c], k0 + col, K);
+#pragma unroll
+        for (int c = 0; c < CB; ++c) rb[c] = load_columns(w_buf, wp[c], k0 + col, K);
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += BK) {
+        __syncthreads();  // (every wave is done with the tile before)
+#pragma unroll
+        for (int c = 0; c < CA; ++c) *reinterpret_cast<f32x4*>(&As[(row + c * STEP) * LD + col]) = ra[c];
+#pragma unroll
+        for (int c = 0; c < CB; ++c) *reinterpret_cast<f32x4*>(&Bs[(row + c * STEP) * LD + col]) = rb[c];
+        __syncthreads();
+        if (k0 + BK < K) fetch(k0 + BK);
+#pragma unroll
+        for (int s = 0; s < BK / 16; ++s) {
+            f32x4 xf[TM], wf[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) xf[i] = *reinterpret_cast<const f32x4*>(&As[(wm + i * 16 + r16) * LD + s * 16 + g * 4]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wf[j] = *reinterpret_cast<const f32x4*>(&Bs[(wn + j * 16 + r16) * LD + s * 16 + g * 4]);
+            // (four columns of K for every tile before the next four: a tile's instructions do not follow on one another)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][r], xf[i][r], acc[i][j], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = m0 + wm + i * 16 + r16;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = n0 + wn + j * 16 + g * 4;
+            f32x4 s = acc[i][j];
+            float* c = C + (size_t)m * ldc + n;
+            if (wide && n + 4 <= N) {
+                if (bias)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[r] += bias[n + r];
+                *reinterpret_cast<f32x4*>(c) = s;
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < N) c[r] = s[r] + (bias ? bias[n + r] : 0.f);
+            }
+        }
+    }
+}
+
+template <int BM, int BN, int BK, int WM>
+static int launch_tile(float* C, const float* A, const float* W, const float* bias, int M, int N, int K, int lda, int ldc, int wide,
+                       hipStream_t stream) {
+    const int tiles_m = (M + BM - 1) / BM;
+    const long long blocks = (long long)tiles_m * ((N + BN - 1) / BN);
+    LLMS_REQUIRE(blocks < (1ll << 31), "gemm32: too many tiles");
+    gemm32_tile_kernel<BM, BN, BK, WM><<<(unsigned)blocks, 256, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, tiles_m, wide);
+    LLMS_LAUNCH_CHECK();
+}
+
+extern "C" {
+
+int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int N, int K, int lda, int ldc, int cus,
+                hipStream_t stream) {
+    LLMS_REQUIRE(M > 0 && N > 0 && K > 0, "gemm32: sizes must be positive");
+    LLMS_REQUIRE(K % 4 == 0 && lda % 4 == 0, "gemm32: K and the row stride of A must be multiples of 4");
+    LLMS_REQUIRE((uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0, "gemm32: A and W must be 16-byte aligned");
+    LLMS_REQUIRE(lda >= K && ldc >= N, "gemm32: leading dimensions too small");
+    LLMS_REQUIRE(cus > 0, "gemm32: no compute units");
+    // (offsets within a tile of 128 rows stay below the one that stands for nothing)
+    LLMS_REQUIRE((long long)lda * 4 * 128 < (1ll << 30) && (long long)K * 4 * 128 < (1ll << 30), "gemm32: rows are too long");
+    float* C = (float*)c;
+    const float *A = (const float*)a, *W = (const float*)w, *bias = (const float*)b;
+    const int wide = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
+    if (M <= 64) {
+        const unsigned tiles = (N + 15) / 16, pairs = (N + 31) / 32;
+        if (M <= 16) {
+            // 16 waves a tile while the tiles alone do not fill the chip, 8 beyond
+            if (tiles <= 2u * cus) gemm32_stream_kernel<1, 1, 16, 4><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+            else gemm32_stream_kernel<1, 1, 8, 4><<<tiles, 512, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+        } else if (M <= 32) {
+            if (tiles <= 2u * cus) gemm32_stream_kernel<2, 1, 16, 4><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+            else gemm32_stream_kernel<2, 2, 8, 2><<<pairs, 512, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+        } else {
+            if (tiles <= 2u * cus) gemm32_stream_kernel<4, 1, 16, 2><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+            else gemm32_stream_kernel<4, 2, 8, 2><<<pairs, 512, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+        }
+        LLMS_LAUNCH_CHECK();
+    }
+    // the largest tile of which there are two for every compute unit (a larger tile reads each operand less often)
+    const auto tiles_of = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+    if (tiles_of(128, 128) >= 2ll * cus) return launch_tile<128, 128, 32, 2>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+    if (tiles_of(64, 64) >= 2ll * cus) return launch_tile<64, 64, 64, 2>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+    return launch_tile<32, 64, 64, 1>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+}
+
+}  // extern "C"

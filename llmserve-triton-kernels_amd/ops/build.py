@@ -41,7 +41,7 @@ HIPCC_FLAGS = [
 # kernels.  Parts add their own (`Part.libraries`: an attention its kernels, a 32-bit stream its own), so a model
 # compiles what it runs and no more; the sampler's library is built when something is first sampled.
 BASE = {
-    "float32": ("elementwise", "gemm"),
+    "float32": ("elementwise", "gemm", "gemm32"),
     "bfloat16": ("elementwise", "gemm", "gemm_stream", "gemm_decode"),
 }
 # (everything the built-in parts of the Llama decoder load: what `ensure_built(dtype)` without a model builds)

@@ -301,6 +301,36 @@ def gemm_fma(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: torch.Te
     return out
 
 
+def gemm32_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the 32-bit matrix-core kernels take these operands (else `gemm_fma` does): 16-byte pieces of rows, and rows of
+    less than 8 MB (offsets within a tile are 32-bit)."""
+    k = a.shape[1]
+    return (a.dtype == torch.float32 and w.dtype == torch.float32 and k % 4 == 0 and a.stride(0) % 4 == 0 and
+            a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and max(k, a.stride(0)) < (1 << 21))
+
+
+def gemm32(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """out[M,N] = a[M,K] w[N,K]^T (+ bias), float32 throughout: multiply-adds in 32-bit on the matrix cores."""
+    dev = _dev(out, a, w, bias)
+    if a.dim() != 2 or a.stride(1) != 1 or out.dim() != 2 or out.stride(1) != 1:
+        raise ValueError("a and out must be 2-d with unit inner stride")
+    _rows(w, "w", a.shape[1])
+    m, k = a.shape
+    n = w.shape[0]
+    if tuple(out.shape) != (m, n):
+        raise ValueError(f"out shape {tuple(out.shape)} is not {(m, n)}")
+    if out.dtype != torch.float32 or not gemm32_supported(a, w):
+        raise ValueError("gemm32 takes float32 operands with rows of multiples of 4 elements, 16-byte aligned")
+    if bias is not None:
+        _f32(bias, "bias", n)
+    if m == 0:
+        return out
+    _check(load("gemm32").llms_gemm32(
+        _ptr(out), _ptr(a), _ptr(w), _ptr(bias), c_int(m), c_int(n), c_int(k), c_int(a.stride(0)), c_int(out.stride(0)),
+        c_int(compute_units(dev)), _stream(dev)), "gemm32")
+    return out
+
+
 def gemm_bf16_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the matrix-core kernels take these operands (else `gemm_fma` does)."""
     k = a.shape[1]

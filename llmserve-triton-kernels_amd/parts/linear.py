@@ -1,6 +1,7 @@
 """y = x W^T (+ b) for the parts: picks the matrix product by dtype and shape.
 
-float32: the 32-bit multiply-add kernel, always (no reduced-precision matrix mode).
+float32: the 32-bit matrix-core kernels (ops.gemm32: multiply-adds in 32-bit, no reduced-precision mode), or the
+  multiply-add kernel of the vector units where rows are no multiples of 16 bytes.
 bfloat16, up to 16 rows of up to 6,144 columns, 17 to 32 rows of up to 4,096, or 33 to 64 rows of up to 2,048:
   ops.gemm_decode, one workgroup per compute unit, with the activation or the rotation and cache store in
   its epilogue; up to 16 rows it also norms its rows on the way in and adds its result to the residual
@@ -144,4 +145,6 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
         if bias is None:
             return torch.mm(x, weight.t(), out_dtype=out.dtype, out=out)
         return torch.addmm(bias.to(out.dtype), x, weight.t(), out_dtype=out.dtype, out=out)
+    if out.dtype == torch.float32 and ops.gemm32_supported(x, weight):
+        return ops.gemm32(out, x, weight, bias)
     return ops.gemm_fma(out, x, weight, bias)

@@ -221,6 +221,23 @@ def test_gemm_fma(m, n, k):
     assert (out.float().cpu().double() - ref).abs().max() <= 2.0 ** -8 * float(ref.abs().max())
 
 
+# rows around the kernels' blocks of 16, 32 and 64, tiles of 32, 64 and 128; N beside a tile's end; K no multiple of a chunk
+@pytest.mark.parametrize("m,n,k", [(1, 333, 4), (2, 16, 36), (16, 2560, 2048), (17, 100, 96), (32, 8300, 68), (33, 333, 1000),
+                                   (64, 8210, 132), (65, 65, 20), (130, 4100, 100), (300, 513, 1000), (2050, 4098, 36)])
+def test_gemm32(m, n, k):
+    a, w, b = rnd(m, k + 4, seed=8)[:, :k], rnd(n, k, seed=9), rnd(n, seed=10)
+    ref = a.double() @ w.double().t() + b.double()
+    out = torch.full((m, n + 3), 7.0, device=DEV)  # (rows that do not start on 16 bytes)
+    ops().gemm32(out[:, :n], a.to(DEV), w.to(DEV), b.to(DEV))
+    # a sum of k products in 32-bit, in any order: k roundings of 2^-24 of sums that grow with sqrt(k)
+    bound = 2e-6 * math.sqrt(k) * float(ref.abs().max())
+    assert (out[:, :n].cpu().double() - ref).abs().max() <= bound and bool((out[:, n:] == 7.0).all())
+    whole = ops().gemm32(torch.empty(m, n, device=DEV), a.to(DEV), w.to(DEV), b.to(DEV))
+    assert torch.equal(whole, out[:, :n])
+    with pytest.raises(ValueError):
+        ops().gemm32(whole, a.bfloat16().to(DEV), w.bfloat16().to(DEV))
+
+
 @pytest.mark.parametrize("kernel,m", [("skinny", 1), ("skinny", 7), ("skinny", 16), ("skinny", 17), ("skinny", 33),
                                       ("skinny", 64), ("tile", 5), ("tile", 65), ("tile", 128), ("tile", 300)])
 @pytest.mark.parametrize("n,k", [(16, 64), (333, 96), (100, 176), (2056, 2048), (512, 5632)])
