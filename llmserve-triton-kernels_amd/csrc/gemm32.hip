@@ -2,9 +2,10 @@
 // v_mfma_f32_16x16x4_f32 multiplies and adds in 32-bit (no reduced-precision mode) at the rate of the vector units, but takes
 // its operands from registers that a wave fills with 16-byte loads, so nothing but memory bounds the products of few rows.
 //
-//   gemm32_stream  M <= 64: the weight is read once, straight into the matrix instruction; a workgroup owns 16 or 32 weight
+//   gemm32_stream  M <= 64, K >= 512: the weight is read once, straight into the matrix instruction; a workgroup owns 16 or 32 weight
 //                  rows, its waves share K out in chunks of 32 and add their sums up in LDS in a fixed order.
-//   gemm32_tile    more rows: tiles through LDS, the next tile's loads in flight while the present one is multiplied.
+//   gemm32_tile    the rest: tiles through LDS, the next tile's loads in flight while the present one is multiplied; a result is
+//                  the sum of its products from the first column to the last, to the bit what gemm_fma gives.
 //
 // Both: K and the row stride of A multiples of 4, A and W 16-byte aligned (the host checks; what does not fit goes to
 // gemm_fma); M and N are arbitrary.  Loads go through a buffer that ends with the workgroup's last row; rows and columns that
@@ -14,8 +15,9 @@
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 // Operand layout: lane l holds A[i = l % 16][k = l / 16] and B[k = l / 16][j = l % 16]; result D[i = 4 (l / 16) + r][j = l % 16].
-// A lane's four consecutive columns 4g .. 4g + 3 (one 16-byte load) serve four instructions: the sum over K takes the columns
-// of a group of 16 in another order, the same one for both operands.  i = weight row, j = row of A.
+// i = weight row, j = row of A.  One instruction adds its four products one after the other, each rounded.  In the stream a
+// lane's four consecutive columns 4g .. 4g + 3 (one 16-byte load) serve four instructions: the sum over K takes the columns
+// of a group of 16 in another order, the same one for both operands.
 __device__ __forceinline__ void fma_16x16x16(f32x4& acc, f32x4 w, f32x4 x) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[r], x[r], acc, 0, 0, 0);
@@ -91,9 +93,13 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
         const int part = idx / LLMS_WAVE, l = idx % LLMS_WAVE;
         const int n = n0 + (part / MB) * 16 + 4 * (l / 16), m = (part % MB) * 16 + l % 16;
         if (m >= M || n >= N) continue;
-        f32x4 s = red[0][part][l];
+        // (added up in 64 bits and rounded once: the few sums of a thread wait for LDS, not for arithmetic)
+        double wide_sum[4] = {};
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) s += red[w][part][l];
+        for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) wide_sum[r] += (double)red[w][part][l][r];
+        f32x4 s = {(float)wide_sum[0], (float)wide_sum[1], (float)wide_sum[2], (float)wide_sum[3]};
         float* c = C + (size_t)m * ldc + n;
         if (wide && n + 4 <= N) {
             if (bias)
@@ -129,7 +135,7 @@ __global__ __launch_bounds__(256) void gemm32_tile_kernel(float* __restrict__ C,
     const int tid = threadIdx.x, wave = tid / LLMS_WAVE, lane = tid % LLMS_WAVE;
     const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
     const int r16 = lane % 16, g = lane / 16;
-    const int row = tid / PER_ROW, col = (tid % PER_ROW) * 4;
+    const int row = tid / PER_ROW, col = (tid % PER_ROW) * 4, place = (col & ~15) + (col & 15) / 4;
 
     const __amdgpu_buffer_rsrc_t a_buf = rows_buffer(A, m0, BM, M, lda, K), w_buf = rows_buffer(W, n0, BN, N, K, K);
     unsigned ap[CA], wp[CB];
@@ -151,10 +157,16 @@ __global__ __launch_bounds__(256) void gemm32_tile_kernel(float* __restrict__ C,
     fetch(0);
     for (int k0 = 0; k0 < K; k0 += BK) {
         __syncthreads();  // (every wave is done with the tile before)
+        // column 4 q + r of a group of 16 lies at 4 r + q: what a lane reads in one piece, its instructions take in the order
+        // of the columns, so that a result is the sum of its products from the first column to the last
 #pragma unroll
-        for (int c = 0; c < CA; ++c) *reinterpret_cast<f32x4*>(&As[(row + c * STEP) * LD + col]) = ra[c];
+        for (int c = 0; c < CA; ++c)
 #pragma unroll
-        for (int c = 0; c < CB; ++c) *reinterpret_cast<f32x4*>(&Bs[(row + c * STEP) * LD + col]) = rb[c];
+            for (int r = 0; r < 4; ++r) As[(row + c * STEP) * LD + place + 4 * r] = ra[c][r];
+#pragma unroll
+        for (int c = 0; c < CB; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Bs[(row + c * STEP) * LD + place + 4 * r] = rb[c][r];
         __syncthreads();
         if (k0 + BK < K) fetch(k0 + BK);
 #pragma unroll
@@ -220,7 +232,10 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
     float* C = (float*)c;
     const float *A = (const float*)a, *W = (const float*)w, *bias = (const float*)b;
     const int wide = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
-    if (M <= 64) {
+    // Rows of fewer than 512 columns give the stream's waves a chunk each at most.  Tiles take some microseconds more there (2
+    // rows of 508 columns against 512 weight rows 8.6, of 512 columns in the stream 5.4; 40 rows 8.8 and 8.1; the multiply-add
+    // kernel 43 to 51), and what they sum in the order of the columns stays to the bit what small models gave before.
+    if (M <= 64 && K >= 512) {
         const unsigned tiles = (N + 15) / 16, pairs = (N + 31) / 32;
         if (M <= 16) {
             // 16 waves a tile while the tiles alone do not fill the chip, 8 beyond

@@ -1,0 +1,411 @@
+// bfloat16 matrix products of many rows (prompts, portions of prompts, large decode batches):  X[M,K] * W[N,K]^T on the
+// matrix cores with 32-bit sums, and what used to be a kernel behind the product in its epilogue:
+//
+//   plain    C[M,N] (+ bias), bfloat16 or float
+//   parts    K shared out to several workgroups a tile, one array of 32-bit sums per part, for a norm to add up
+//   gated    W = [gate; up]: C[M,N/2] = silu(gate) * up (or the clamped unit, or gelu(gate) * up)
+//   rotary   W = [q; k; v]: C = rotated q; rotated k and v go to the tokens' cache slots
+//
+// Arrangement.  A workgroup of 4 or 8 waves owns a tile of BM rows of X by BN rows of W and walks K in steps of 64.  A step's
+// rows come into one of S buffers of LDS by loads that go there directly (8 rows of 128 bytes an instruction), S - 1 steps
+// ahead; a piece of 16 bytes lies at its place XOR the row, so that the 16 rows of a matrix operand are read without bank
+// conflicts.  Fragments are held twice: while the first half of a step is multiplied its second half is read, and while
+// that is multiplied the next step's first half is, so LDS and matrix cores work side by side and a step needs one barrier.
+// The buffers are variables of their own, and the loop is unrolled over them: only so does the compiler know that a read
+// of one buffer need not wait for the loads into another.  Instructions per wave tile of (BM / WM) x (BN / WN): the larger,
+// the fewer bytes of LDS per product (a 64 x 64 wave tile already asks LDS for as much as it can give), so the large tiles
+// run at 1.4 PFLOP/s in the loop and the small ones fill the chip when there are few rows.
+//
+// Measured (microseconds, weights from memory; in brackets the library's product, and with it the kernel behind):
+//   1.1B shape    333 rows: q, k, v 9 (12), o_proj in 2 parts 8 (12), gate and up with SiLU 28 (32 + 5), down_proj in 4 parts 16 (25)
+//                 512 rows: 10 (15), 9 (12), 31 (33 + 6), 22 (27);  2,048 rows: 26 (28), 20 (22), 87 (92 + 13), 50 (50 to 60)
+//   7B shape      330 rows: q, k, v 50 (56), o_proj 21 (26), down_proj 40 (60);  2,048 rows: gate and up 310 (402), down_proj 155 (167)
+// What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times
+// its matrix instructions); beyond, LDS and matrix cores together, and how evenly the tiles fill 256 compute units.
+//
+// K must be a multiple of 64 S (the host checks), N of 16, rows of X and W 16-byte aligned; M is arbitrary: rows beyond M
+// are read as zeros or as row 0 and never stored.
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+
+#define GT_PLAIN 0
+#define GT_FLOAT 1  // plain or parts, 32-bit result
+#define GT_GATED 2
+#define GT_ROTARY 3
+
+struct TilesArgs {
+    const bf16* X;
+    const bf16* W;
+    const bf16* bias;
+    void* C;
+    int M, N, K, ldx, ldc;
+    int tiles_m, tiles;          // tiles along M, tiles in all (of one part)
+    int steps;                   // of 64 columns, of one part
+    long long part_stride;       // elements from one part's sums to the next's
+    int inter, unit;             // GATED; unit 0 SiLU, 1 clamped, 3 gelu
+    float limit;
+    int n_heads, n_kv_heads, head_dim, block_size, bs_shift;  // ROTARY (bs_shift: log2 of the page size, or -1)
+    const float* angles;         // [M][head_dim / 2] (sine, cosine), or null: nothing turns
+    const int* slots;            // or null: nothing is stored
+    bf16 *k_pool, *v_pool;
+};
+
+template <int N>
+struct Number {
+    static constexpr int n = N;
+};
+
+// Row of W behind row `r` (a multiple of 8) of the product's columns in the order the epilogue wants them: blocks of 16
+// columns that belong together (gate and up, both halves of a head) alternate.
+template <int EPI>
+__device__ __forceinline__ int gt_weight_row(const TilesArgs& a, int r) {
+    const int block = r / 16, within = r % 16;
+    if (EPI == GT_GATED) return (block & 1) * a.inter + (block / 2) * 16 + within;
+    if (EPI == GT_ROTARY) {
+        const int halves = a.head_dim / 32, turned = 2 * (a.n_heads + a.n_kv_heads) * halves;  // blocks of q and k
+        if (block < turned) {
+            const int pair = block / 2, head = pair / halves;
+            return head * a.head_dim + (pair - head * halves) * 16 + (block & 1) * (a.head_dim / 2) + within;
+        }
+    }
+    return r;
+}
+
+__device__ __forceinline__ void gt_store4(bf16* p, float a, float b, float c, float d) {
+    *reinterpret_cast<u32x2*>(p) = (u32x2){pack_bf16x2(a, b), pack_bf16x2(c, d)};
+}
+
+__device__ __forceinline__ float gt_unit(const TilesArgs& a, float gate, float up) {
+    if (a.unit == 1) {
+        const float g = fminf(gate, a.limit), v = fminf(fmaxf(up, -a.limit), a.limit);
+        return g / (1.f + expf(-1.702f * g)) * (v + 1.f);
+    }
+    if (a.unit == 3) return gelu_tanh(gate) * up;
+    gate = round_to<bf16>(gate);  // (the projections' results and SiLU are bfloat16 before they are multiplied)
+    return round_to<bf16>(gate / (1.f + expf(-gate))) * round_to<bf16>(up);
+}
+
+template <int BM, int BN, int WM, int WN, int S, int EPI>
+__global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const TilesArgs a) {
+    constexpr int NW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
+    constexpr int LM = BM / 8 / NW, LN = BN / 8 / NW;  // loads of 8 rows, per wave
+    static_assert(LM * NW * 8 == BM && LN * NW * 8 == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile does not divide");
+    static_assert(TN % 2 == 0, "columns that belong together lie in one wave");
+    static_assert(S == 2 || S == 4, "buffers");
+    constexpr int TILE = (BM + BN) * 128;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds0[TILE];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds1[TILE];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds2[S > 2 ? TILE : 16];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds3[S > 2 ? TILE : 16];
+
+    const int part = EPI == GT_FLOAT ? blockIdx.x / a.tiles : 0, pid = blockIdx.x - part * a.tiles;
+    const int first = part * a.steps, steps = min(a.steps, a.K / 64 - first);
+    // workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, rows fastest, so that the tiles
+    // which share weight rows share an L2
+    const int full = a.tiles / 8, rem = a.tiles % 8, xcd = pid % 8;
+    const int t = xcd * full + min(xcd, rem) + pid / 8;
+    const int m0 = (t % a.tiles_m) * BM, n0 = (t / a.tiles_m) * BN;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / LLMS_WAVE), lane = tid % LLMS_WAVE;
+    const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
+    const int r16 = lane % 16, g = lane / 16;
+
+    // A load brings 8 rows: lane l row l / 8, the piece (l % 8) ^ (l / 8) of its 128 bytes, to place l.  Each load has a
+    // buffer of its own that starts with its first row and ends with the matrix (groups of rows beyond it: with row 0).
+    const int lr = lane / 8, lc = ((lane % 8) ^ lr) * 16;
+    const unsigned x_off = (unsigned)(lr * a.ldx * 2 + lc), w_off = (unsigned)(lr * a.K * 2 + lc);
+    __amdgpu_buffer_rsrc_t xb[LM], wb[LN];
+#pragma unroll
+    for (int i = 0; i < LM; ++i) {
+        int r = m0 + (wave * LM + i) * 8;
+        r = r < a.M ? r : 0;
+        xb[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.X + (size_t)r * a.ldx), 0,
+                                                  (unsigned)((min(8, a.M - r) - 1) * a.ldx + a.K) * 2u, 0x00020000);
+    }
+#pragma unroll
+    for (int i = 0; i < LN; ++i) {
+        const int c = n0 + (wave * LN + i) * 8;
+        const int r = c < a.N ? gt_weight_row<EPI>(a, c) : 0;
+        wb[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.W + (size_t)r * a.K), 0, (unsigned)(8 * a.K) * 2u, 0x00020000);
+    }
+    auto fetch = [&](uint8_t* lds, int step) {
+        const int so = (first + step) * 128;
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+        for (int i = 0; i < LM; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xb[i], (__attribute__((address_space(3))) void*)(lds + (wave * LM + i) * 1024), 16,
+                                                     x_off, so, 0, 0);
+#pragma unroll
+        for (int i = 0; i < LN; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                wb[i], (__attribute__((address_space(3))) void*)(lds + BM * 128 + (wave * LN + i) * 1024), 16, w_off, so, 0, 0);
+#endif
+    };
+
+    // v_mfma_f32_16x16x32_bf16 as everywhere in this folder: i = weight row (4 g + register), j = row of X (lane % 16)
+    f32x4 acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    bf16x8 wf[2][TN], xf[2][TM];
+    auto read = [&](const uint8_t* lds, int half) {
+        const int q = ((half * 4 + g) ^ (r16 & 7)) * 16;
+#pragma unroll
+        for (int i = 0; i < TN; ++i) wf[half][i] = *reinterpret_cast<const bf16x8*>(lds + BM * 128 + (wn + i * 16 + r16) * 128 + q);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) xf[half][j] = *reinterpret_cast<const bf16x8*>(lds + (wm + j * 16 + r16) * 128 + q);
+    };
+    auto multiply = [&](int half) {
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+            for (int i = 0; i < TN; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[half][i], xf[half][j], acc[i][j], 0, 0, 0);
+    };
+    // the order in which the scheduler puts a stage: some matrix instructions, one LDS read, one load, and again
+    auto interleave = [&](auto loads) {
+        constexpr int READS = TM + TN, EACH = TM * TN / READS > 0 ? TM * TN / READS : 1;
+#pragma unroll
+        for (int i = 0; i < READS; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, EACH, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (i < decltype(loads)::n) __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x8, TM * TN, 0);
+    };
+    // waits until at most `left` steps' loads of this wave are in flight (and its LDS reads are done), then for all waves
+    auto arrive = [&](auto left) {
+        constexpr int n = decltype(left)::n * (LM + LN);
+        static_assert(n < 64, "the counter of loads in flight");
+        __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | 0x0070);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // One step: `now` holds it, its first half is in registers; `next` holds the step behind it.  At the barrier every wave
+    // has read all of `now`, which then takes the step S further on.
+    int step = 0;
+    auto one = [&](uint8_t* now, uint8_t* next, auto left, auto more, auto last) {
+        constexpr bool MORE = decltype(more)::n, LAST = decltype(last)::n;
+        read(now, 1);
+        multiply(0);
+        interleave(Number<0>());
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (LAST) {
+            multiply(1);
+        } else {
+            arrive(left);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (MORE) fetch(now, step + S);
+            read(next, 0);
+            multiply(1);
+            interleave(Number<MORE ? LM + LN : 0>());
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ++step;
+    };
+    typedef Number<1> Yes;
+    typedef Number<0> No;
+    fetch(lds0, 0);
+    fetch(lds1, 1);
+    if constexpr (S > 2) {
+        fetch(lds2, 2);
+        fetch(lds3, 3);
+    }
+    arrive(Number<S - 1>());
+    read(lds0, 0);
+    for (int rounds = steps / S - 1; rounds > 0; --rounds) {
+        if constexpr (S == 2) {
+            one(lds0, lds1, Number<0>(), Yes(), No());
+            one(lds1, lds0, Number<0>(), Yes(), No());
+        } else {
+            one(lds0, lds1, Number<2>(), Yes(), No());
+            one(lds1, lds2, Number<2>(), Yes(), No());
+            one(lds2, lds3, Number<2>(), Yes(), No());
+            one(lds3, lds0, Number<2>(), Yes(), No());
+        }
+    }
+    if constexpr (S == 2) {
+        one(lds0, lds1, Number<0>(), No(), No());
+        one(lds1, lds0, Number<0>(), No(), Yes());
+    } else {
+        one(lds0, lds1, Number<2>(), No(), No());
+        one(lds1, lds2, Number<1>(), No(), No());
+        one(lds2, lds3, Number<0>(), No(), No());
+        one(lds3, lds0, Number<0>(), No(), Yes());
+    }
+
+    // ---- epilogue: a lane holds 4 consecutive columns of row m in each acc[i][j]; blocks i and i + 1 (i even) belong together
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        const int m = m0 + wm + j * 16 + r16;
+        if (m >= a.M) continue;
+        if constexpr (EPI == GT_GATED) {
+#pragma unroll
+            for (int i = 0; i < TN; i += 2) {
+                const int n = (n0 + wn) / 2 + i * 8 + g * 4;
+                if (n >= a.inter) continue;
+                const f32x4 lo = acc[i][j], hi = acc[i + 1][j];
+                gt_store4(reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + n, gt_unit(a, lo[0], hi[0]), gt_unit(a, lo[1], hi[1]),
+                          gt_unit(a, lo[2], hi[2]), gt_unit(a, lo[3], hi[3]));
+            }
+        } else if constexpr (EPI == GT_ROTARY) {
+            const int D = a.head_dim, half = D / 2, bs = a.block_size, nkv = a.n_kv_heads;
+            const int slot = a.slots ? a.slots[m] : -1;
+            const int page = a.bs_shift >= 0 ? slot >> a.bs_shift : slot / bs, off = slot - page * bs;  // (used where slot >= 0)
+#pragma unroll
+            for (int i = 0; i < TN; i += 2) {
+                const int c = n0 + wn + i * 16;  // (the same for all lanes: the branches below are uniform)
+                if (c >= a.N) continue;
+                f32x4 lo = acc[i][j], hi = acc[i + 1][j];
+                const int row_lo = gt_weight_row<EPI>(a, c) + g * 4, row_hi = gt_weight_row<EPI>(a, c + 16) + g * 4;
+                if (a.bias) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        lo[r] += bf16_bits_to_f32(a.bias[row_lo + r].bits);
+                        hi[r] += bf16_bits_to_f32(a.bias[row_hi + r].bits);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {  // (the projection's result is bfloat16 before it is rotated)
+                    lo[r] = round_to<bf16>(lo[r]);
+                    hi[r] = round_to<bf16>(hi[r]);
+                }
+                if (c < (a.n_heads + nkv) * D) {
+                    const int head = row_lo / D, d = row_lo - head * D;
+                    if (a.angles) {
+                        const f32x4* table = reinterpret_cast<const f32x4*>(a.angles + ((size_t)m * half + d) * 2);
+                        const f32x4 s0 = table[0], s1 = table[1];
+                        const float sn[4] = {s0[0], s0[2], s1[0], s1[2]}, cs[4] = {s0[1], s0[3], s1[1], s1[3]};
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float2 v = rotate_pair(lo[r], hi[r], cs[r], sn[r]);
+                            lo[r] = v.x;
+                            hi[r] = v.y;
+                        }
+                    }
+                    bf16* to = nullptr;
+                    if (head < a.n_heads) to = reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + head * D + d;
+                    else if (slot >= 0) to = a.k_pool + (((size_t)page * nkv + (head - a.n_heads)) * bs + off) * D + d;
+                    if (to) {
+                        gt_store4(to, lo[0], lo[1], lo[2], lo[3]);
+                        gt_store4(to + half, hi[0], hi[1], hi[2], hi[3]);
+                    }
+                } else if (slot >= 0) {
+                    // a page holds [kv head][dimension][token]: 16 lanes are 16 tokens, mostly side by side in a page
+                    bf16* v = a.v_pool + (size_t)page * nkv * D * bs + off;
+                    const int f_lo = row_lo - (a.n_heads + nkv) * D, f_hi = row_hi - (a.n_heads + nkv) * D;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        v[(size_t)(f_lo + r) * bs].bits = f32_to_bf16_bits(lo[r]);
+                        v[(size_t)(f_hi + r) * bs].bits = f32_to_bf16_bits(hi[r]);
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const int n = n0 + wn + i * 16 + g * 4;
+                if (n >= a.N) continue;
+                f32x4 s = acc[i][j];
+                if (a.bias) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[r] += bf16_bits_to_f32(a.bias[n + r].bits);
+                }
+                if constexpr (EPI == GT_FLOAT)
+                    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.C) + part * a.part_stride + (size_t)m * a.ldc + n) = s;
+                else
+                    gt_store4(reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + n, s[0], s[1], s[2], s[3]);
+            }
+        }
+    }
+}
+
+template <int BM, int BN, int WM, int WN, int S>
+static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
+    LLMS_REQUIRE(a.K % (64 * S) == 0, "gemm_tiles: K does not divide into this tile's steps");
+    const int tiles_n = (a.N + BN - 1) / BN, groups = a.K / 64 / S;
+    a.tiles_m = (a.M + BM - 1) / BM;
+    LLMS_REQUIRE((long long)a.tiles_m * tiles_n * parts < (1ll << 31), "gemm_tiles: too many tiles");
+    a.tiles = a.tiles_m * tiles_n;
+    a.steps = (groups + parts - 1) / parts * S;
+    LLMS_REQUIRE((long long)(parts - 1) * a.steps < a.K / 64, "gemm_tiles: a part of K is empty");
+    const dim3 grid((unsigned)(a.tiles * parts)), block(WM * WN * LLMS_WAVE);
+    if (epilogue == GT_PLAIN) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_PLAIN><<<grid, block, 0, stream>>>(a);
+    else if (epilogue == GT_FLOAT) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_FLOAT><<<grid, block, 0, stream>>>(a);
+    else if (epilogue == GT_GATED) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_GATED><<<grid, block, 0, stream>>>(a);
+    else gemm_tiles_kernel<BM, BN, WM, WN, S, GT_ROTARY><<<grid, block, 0, stream>>>(a);
+    LLMS_LAUNCH_CHECK();
+}
+
+extern "C" {
+
+// epilogue: 0 plain bfloat16, 1 plain float (parts > 1: `parts` arrays of sums, part_stride elements apart), 2 gated, 3 rotary.
+// tile: a place in the table of ops/library.py (GEMM_TILES).
+int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* W, const void* bias, int M, int N, int K, int ldx,
+                    int ldc, int parts, long long part_stride, int unit, float limit, int n_heads, int n_kv_heads, int head_dim,
+                    int block_size, const float* angles, const int* slots, void* k_pool, void* v_pool, hipStream_t stream) {
+    LLMS_REQUIRE(M > 0 && N > 0 && K > 0 && parts > 0, "gemm_tiles: sizes must be positive");
+    LLMS_REQUIRE(N % 16 == 0 && ldx % 8 == 0 && ldx >= K, "gemm_tiles: N in multiples of 16, rows of X of multiples of 8");
+    LLMS_REQUIRE((uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0, "gemm_tiles: X and W must be 16-byte aligned");
+    LLMS_REQUIRE(ldx < (1 << 26) && K < (1 << 26), "gemm_tiles: rows are too long");
+    LLMS_REQUIRE(epilogue >= GT_PLAIN && epilogue <= GT_ROTARY, "gemm_tiles: epilogue");
+    LLMS_REQUIRE(parts == 1 || (epilogue == GT_FLOAT && bias == nullptr), "gemm_tiles: only plain 32-bit sums come in parts");
+    LLMS_REQUIRE(C != nullptr && ldc % 4 == 0 && (uintptr_t)C % (epilogue == GT_FLOAT ? 16 : 8) == 0 && part_stride % 4 == 0,
+                 "gemm_tiles: rows of the result must start on 4 elements");
+    const int cols = epilogue == GT_GATED ? N / 2 : epilogue == GT_ROTARY ? n_heads * head_dim : N;
+    LLMS_REQUIRE(ldc >= cols, "gemm_tiles: leading dimension of the result too small");
+    TilesArgs a{};
+    a.X = (const bf16*)X;
+    a.W = (const bf16*)W;
+    a.bias = (const bf16*)bias;
+    a.C = C;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.ldx = ldx;
+    a.ldc = ldc;
+    a.part_stride = part_stride;
+    if (epilogue == GT_GATED) {
+        LLMS_REQUIRE(N % 32 == 0 && bias == nullptr, "gemm_tiles: the gated epilogue takes blocks of 16 units and no bias");
+        LLMS_REQUIRE(unit == 0 || unit == 1 || unit == 3, "gemm_tiles: unit 0, 1 or 3");
+        a.inter = N / 2;
+        a.unit = unit;
+        a.limit = limit;
+    }
+    if (epilogue == GT_ROTARY) {
+        LLMS_REQUIRE(n_heads > 0 && n_kv_heads > 0 && head_dim > 0 && head_dim % 32 == 0 && N == (n_heads + 2 * n_kv_heads) * head_dim,
+                     "gemm_tiles: the rotary epilogue takes q, k and v of heads in multiples of 32");
+        LLMS_REQUIRE(slots == nullptr || (k_pool && v_pool && block_size > 0 && (uintptr_t)k_pool % 8 == 0), "gemm_tiles: slots without pools");
+        LLMS_REQUIRE((uintptr_t)angles % 16 == 0, "gemm_tiles: the table of angles must be 16-byte aligned");
+        a.n_heads = n_heads;
+        a.n_kv_heads = n_kv_heads;
+        a.head_dim = head_dim;
+        a.block_size = block_size;
+        a.bs_shift = -1;
+        for (int s = 0; s < 31; ++s)
+            if ((1 << s) == block_size) a.bs_shift = s;
+        a.angles = angles;
+        a.slots = slots;
+        a.k_pool = (bf16*)k_pool;
+        a.v_pool = (bf16*)v_pool;
+    }
+    switch (tile) {
+        case 0: return launch<64, 64, 2, 2, 4>(epilogue, a, parts, stream);
+        case 1: return launch<96, 64, 2, 2, 4>(epilogue, a, parts, stream);
+        case 2: return launch<128, 64, 2, 2, 4>(epilogue, a, parts, stream);
+        case 3: return launch<96, 128, 2, 2, 4>(epilogue, a, parts, stream);
+        case 4: return launch<128, 128, 2, 2, 4>(epilogue, a, parts, stream);
+        case 5: return launch<128, 192, 2, 2, 4>(epilogue, a, parts, stream);
+        case 6: return launch<192, 128, 2, 2, 4>(epilogue, a, parts, stream);
+        case 7: return launch<160, 128, 2, 2, 2>(epilogue, a, parts, stream);
+        case 8: return launch<192, 128, 2, 2, 2>(epilogue, a, parts, stream);
+        case 9: return launch<256, 192, 2, 2, 2>(epilogue, a, parts, stream);
+        case 10: return launch<256, 256, 2, 4, 2>(epilogue, a, parts, stream);
+    }
+    LLMS_REQUIRE(false, "gemm_tiles: no such tile");
+}
+
+}  // extern "C"

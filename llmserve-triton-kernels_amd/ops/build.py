@@ -42,7 +42,7 @@ HIPCC_FLAGS = [
 # compiles what it runs and no more; the sampler's library is built when something is first sampled.
 BASE = {
     "float32": ("elementwise", "gemm", "gemm32"),
-    "bfloat16": ("elementwise", "gemm", "gemm_stream", "gemm_decode"),
+    "bfloat16": ("elementwise", "gemm", "gemm_stream", "gemm_decode", "gemm_tiles"),
 }
 # (everything the built-in parts of the Llama decoder load: what `ensure_built(dtype)` without a model builds)
 GROUPS = {

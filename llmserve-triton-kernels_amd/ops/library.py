@@ -9,6 +9,7 @@ Kernels run on the current torch stream of the tensors' device.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 import os
 import threading
@@ -599,6 +600,128 @@ def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias
 
 
 SLICE_K = 512  # what one workgroup of gemm_slices takes of K
+
+
+# Tiles of ops.gemm_tiles (the order is the launcher's): rows of x, rows of w, workgroups a compute unit holds, steps of 64
+# columns its LDS holds, and the microseconds a step takes with one workgroup on every compute unit and with all it holds:
+# fitted to 150 products (65 to 2,048 rows; K of 2,048 to 11,008, N of 2,048 to 22,016), over which the plan below is 1 % off
+# the best tile in the mean and 18 % at worst.
+GEMM_TILES = ((64, 64, 2, 4, 0.23, 0.37), (96, 64, 2, 4, 0.245, 0.43), (128, 64, 1, 4, 0.32, 0.32), (96, 128, 1, 4, 0.40, 0.40),
+              (128, 128, 1, 4, 0.52, 0.52), (128, 192, 1, 4, 0.70, 0.70), (192, 128, 1, 4, 0.60, 0.60), (160, 128, 2, 2, 1.08, 0.90),
+              (192, 128, 2, 2, 1.57, 1.00), (256, 192, 1, 2, 1.31, 1.31), (256, 256, 1, 2, 1.33, 1.33))
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256) -> tuple[int, int]:
+    """(tile, parts of K) for m rows against a weight [n, k]: the least of what the rounds over the compute units cost.  A
+    round takes a tile's steps; the last one as much as its fullest compute unit has.  Parts of K (2 or 4, where the caller
+    takes partial sums) fill the chip when there are few tiles, and cost writing and reading their 32-bit sums (2048 x 5632
+    with the norm behind it at 128 rows: 16.6 microseconds in four parts, 33 in one; at 1,024 rows 42 and 37.6).  A rule by
+    sizes alone."""
+    best = None
+    for tile, (bm, bn, held, stages, one, full) in enumerate(GEMM_TILES):
+        groups = k // (64 * stages)
+        if k % (64 * stages):
+            continue
+        for parts in (1, 2, 4):
+            if parts > most_parts or parts > groups or (parts - 1) * -(-groups // parts) >= groups:
+                continue
+            steps = -(-groups // parts) * stages
+            workgroups = -(-m // bm) * -(-n // bn) * parts
+            rounds, rest = divmod(workgroups, held * cus)
+            cost = steps * (rounds * full + (0.0 if rest == 0 else one if rounds == 0 and rest <= cus else full)) + rounds + (rest > 0)
+            if parts > 1:
+                cost += m * n * (7.4 * parts - 4) / 4.0e6
+            if best is None or cost < best[0]:
+                best = (cost, tile, parts)
+    return best[1:]
+
+
+def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 128, blocks of 16 weight rows, 16-byte rows."""
+    return gemm_bf16_supported(x, w) and x.shape[1] % 128 == 0 and w.shape[0] % 16 == 0 and w.dtype == torch.bfloat16
+
+
+def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *, swiglu: bool = False,
+               rope: dict | None = None, limit: float | None = None, gelu: bool = False, tile: int | None = None) -> torch.Tensor:
+    """The product of many bfloat16 rows, and what follows it fused in.
+
+    plain:   out[M, N] = x w^T (+ bias), bfloat16 or float32; float32 [parts, M, N]: the sums of that many parts of K.
+    swiglu:  w = [gate; up] ([2I, K], I a multiple of 16); out[M, I] = silu(gate) * up, or with `limit` or `gelu` the units of
+             `silu_mul` (in 32-bit, rounded once).
+    rope:    as for `gemm_decode` (head_dim a multiple of 32): out[M, n_heads * head_dim] = rotated q, rotated k and v go to
+             the tokens' cache slots.
+    `tile`: a place in GEMM_TILES; default by gemm_tiles_plan."""
+    dev = _dev(out, x, w, bias)
+    if x.dim() != 2 or x.stride(1) != 1 or out.dim() not in (2, 3) or out.stride(-1) != 1:
+        raise ValueError("x must be 2-d, x and out with unit inner stride")
+    _rows(w, "w", x.shape[1])
+    m, k = x.shape
+    n = w.shape[0]
+    parts, part_stride = 1, 0
+    if out.dim() == 3:
+        parts = out.shape[0]
+        if swiglu or rope is not None or bias is not None or out.dtype != torch.float32 or not out.is_contiguous():
+            raise ValueError("parts of K leave plain sums in a contiguous float32 [parts, M, N] tensor, without a bias")
+        part_stride = out.stride(0)
+    if x.dtype != torch.bfloat16 or not gemm_tiles_supported(x, w):
+        raise ValueError(f"gemm_tiles takes bfloat16 operands, 16-byte aligned, K ({k}) a multiple of 128, N ({n}) of 16")
+    if out.dtype != torch.bfloat16 and (out.dtype != torch.float32 or swiglu or rope is not None):
+        raise ValueError("out must be bfloat16, or float32 with the plain epilogue")
+    if out.stride(-2) % 4 or out.data_ptr() % (4 * out.element_size()):
+        raise ValueError("rows of out must start on 4 elements")
+    if bias is not None and (bias.dtype != torch.bfloat16 or bias.numel() != n or not bias.is_contiguous()):
+        raise ValueError("bias must be a contiguous bfloat16 vector of N elements")
+    if swiglu and rope is not None or ((limit is not None or gelu) and not swiglu):
+        raise ValueError("one epilogue at a time; a limit and gelu go with the gated one")
+    epilogue, cols = (1 if out.dtype == torch.float32 else 0), n
+    r = dict(n_heads=0, n_kv_heads=0, head_dim=0, block_size=1, inv_freq=None, positions=None, slots=None, k_pool=None, v_pool=None,
+             angles=None)
+    if swiglu:
+        if n % 32 or bias is not None:
+            raise ValueError("the gated epilogue needs gate and up in blocks of 16 rows and no bias")
+        epilogue, cols = 2, n // 2
+    elif rope is not None:
+        r.update(rope)
+        nh, nkv, d = r["n_heads"], r["n_kv_heads"], r["head_dim"]
+        if d % 32 or n != (nh + 2 * nkv) * d:
+            raise ValueError("the rotary epilogue needs head_dim in multiples of 32 and N = (heads + 2 kv heads) * head_dim")
+        if r["angles"] is None and r["inv_freq"] is not None:
+            _i32(r["positions"], "positions", m)
+            _f32(r["inv_freq"], "inv_freq", d // 2)
+            r["angles"] = rotary_angles(r["positions"], r["inv_freq"])
+        if r["angles"] is not None:
+            _f32(r["angles"], "angles", m * d)
+        if r["slots"] is not None:
+            _i32(r["slots"], "slots", m)
+            bs, kp, vp = r["block_size"], r["k_pool"], r["v_pool"]
+            pages = kp.shape[0]
+            if (tuple(kp.shape) != (pages, nkv, bs, d) or tuple(vp.shape) != (pages, nkv, d, bs) or kp.dtype != torch.bfloat16
+                    or vp.dtype != torch.bfloat16 or not kp.is_contiguous() or not vp.is_contiguous()):
+                raise ValueError("k_pool and v_pool must be contiguous bfloat16 pools of these heads and pages")
+            if kp.device != dev or vp.device != dev or r["slots"].device != dev:
+                raise ValueError("pools and slots must be on the operands' device")
+        epilogue, cols = 3, nh * d
+    if tuple(out.shape[-2:]) != (m, cols):
+        raise ValueError(f"out shape {tuple(out.shape)} does not end in {(m, cols)}")
+    if m == 0:
+        return out
+    if tile is None:
+        tile = gemm_tiles_plan(m, n, k, 1, compute_units(dev))[0] if parts == 1 else _tile_for_parts(m, n, k, parts, compute_units(dev))
+    _check(load("gemm_tiles").llms_gemm_tiles(
+        c_int(tile), c_int(epilogue), _ptr(out), _ptr(x), _ptr(w), _ptr(bias), c_int(m), c_int(n), c_int(k), c_int(x.stride(0)),
+        c_int(out.stride(-2)), c_int(parts), ctypes.c_longlong(part_stride), c_int(_gated_unit(limit, gelu)),
+        c_float(0.0 if limit is None else limit), c_int(r["n_heads"]), c_int(r["n_kv_heads"]), c_int(r["head_dim"]),
+        c_int(r["block_size"]), _ptr(r["angles"]), _ptr(r["slots"]), _ptr(r["k_pool"]), _ptr(r["v_pool"]), _stream(dev)),
+        "gemm_tiles")
+    return out
+
+
+def _tile_for_parts(m: int, n: int, k: int, parts: int, cus: int) -> int:
+    tile, planned = gemm_tiles_plan(m, n, k, 4, cus)
+    if planned != parts:
+        raise ValueError(f"{m} rows against [{n}, {k}] are planned in {planned} parts of K; for {parts} name the tile")
+    return tile
 
 
 def gemm_slices(parts: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -16,7 +16,7 @@ import math
 import torch
 
 from ..ops import library as ops
-from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums
+from .linear import STREAM_ROWS, adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums
 from .registry import ADDED_IN_PLACE, POSITION_ENCODINGS, DeferredNorm, Mixer, register_mixer
 from .spec import PagedCacheSpec, ParamInfo
 
@@ -74,7 +74,7 @@ class Attention(Mixer):
         view = batch.groups[cache.group_id]
         slots = view.slots if cache.store else None
         deferred = x if isinstance(x, DeferredNorm) else None  # (then the result goes to a norm, which takes partial sums)
-        q = self.project_few_rows(x, batch, cache, slots)
+        q = self.project_and_store(x, batch, cache, slots)
         if q is None:
             if deferred is not None:
                 x = deferred.materialize()
@@ -97,12 +97,17 @@ class Attention(Mixer):
     def _few_rows_unfit(self, rows) -> bool:
         if rows.dtype != torch.bfloat16 or self.head_dim % 16 != 0 or not ops.gemm_bf16_supported(rows, self.qkv_weight):
             return True
-        return not (decode_product(rows, self.qkv_weight) or few_rows(rows.shape[0], self.qkv_weight))
+        return not (decode_product(rows, self.qkv_weight) or few_rows(rows.shape[0], self.qkv_weight) or self._fits_tiles(rows))
 
-    def project_few_rows(self, x, batch, cache, slots):
-        """With few bfloat16 rows one kernel does the projection, the rotation and the cache store
-        (ops.gemm_decode, which also norms its rows on the way in, or ops.gemm_stream).  Returns the rotated
-        queries, or None when neither kernel applies."""
+    def _fits_tiles(self, rows) -> bool:
+        # (whatever the weight's size: the rotation and the cache store that the library's product leaves to a kernel of their
+        # own cost more than it gains)
+        return rows.shape[0] > STREAM_ROWS and self.head_dim % 32 == 0 and ops.gemm_tiles_supported(rows, self.qkv_weight)
+
+    def project_and_store(self, x, batch, cache, slots):
+        """With bfloat16 rows one kernel does the projection, the rotation and the cache store
+        (ops.gemm_decode, which also norms its rows on the way in, ops.gemm_stream or ops.gemm_tiles).  Returns the rotated
+        queries, or None when none of them applies."""
         deferred = isinstance(x, DeferredNorm)
         rows = x.residual if deferred else x
         m = rows.shape[0]
@@ -121,11 +126,15 @@ class Attention(Mixer):
                     inv_freq=frequencies() if frequencies is not None else None, positions=batch.positions,
                     slots=slots, k_pool=cache.k_pool, v_pool=cache.v_pool, block_size=cache.block_size)
         q = torch.empty((m, self.num_heads * self.head_dim), dtype=rows.dtype, device=rows.device)
-        if decode:
+        tiles = not decode and not few_rows(m, self.qkv_weight)
+        if decode or tiles:
             angles = getattr(self.position, "rotary_angles", None)
             if angles is not None and getattr(batch, "shared", None) is not None:
                 rope["angles"] = angles(batch)  # worked out once per step, not once per layer and workgroup
-            ops.gemm_decode(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, norm=norm)
+            if tiles:
+                ops.gemm_tiles(q, rows, self.qkv_weight, self.qkv_bias, rope=rope)
+            else:
+                ops.gemm_decode(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, norm=norm)
         else:
             ops.gemm_stream(q, rows, self.qkv_weight, self.qkv_bias, rope=rope)
         return q

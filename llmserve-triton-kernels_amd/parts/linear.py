@@ -13,15 +13,15 @@ bfloat16, few rows otherwise: the hand-written kernel that streams the weight on
   the norm kernel adds up (linear_partial_sums): that fills the chip for a short, wide weight; for 17 to
   64 rows it is ops.gemm_decode with K shared out to 2 to 8 sets of workgroups (ops.gemm_slices, which
   keeps a slice of all rows in LDS, where that kernel is switched off).
-bfloat16, more rows: the library's matrix product (hipBLASLt through torch.mm), which is
-  where the reference's engine uses a library too (nn.Linear, src/llmserve/model/llama.py:64-67);
-  sums are 32-bit, the result bfloat16 or, for logits, float32.
+bfloat16, more rows: ops.gemm_tiles, tiles on the matrix cores with the activation, the rotation and cache store, or the
+  partial sums of a product that goes to a norm in the epilogue; the library's matrix product (hipBLASLt through
+  torch.mm), which is where the reference's engine uses a library too (nn.Linear, src/llmserve/model/llama.py:64-67), only
+  for the sizes where it is still the faster one (library_is_faster) and for K or N that the tiles cannot take.
 Operands the matrix-core kernels cannot take (K not a multiple of 8) fall to the 32-bit
 multiply-add kernel, which takes anything.
 
-LLMSERVE_GEMM=own in the environment keeps the library out altogether: products the streaming
-kernel does not take then go to this repository's tiled matrix-core kernels (ops.gemm_bf16), a
-few times slower than hipBLASLt on large shapes but free of any library.
+LLMSERVE_GEMM=own in the environment keeps the library out altogether: what neither the streaming kernel nor the tiles
+take then goes to this repository's plain tiled kernels (ops.gemm_bf16).
 """
 
 from __future__ import annotations
@@ -71,6 +71,31 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
         return m > 0
     return m <= STREAM_MAX_ROWS and -(-m // 16) * weight.numel() * 2 <= STREAM_REREAD_BYTES
 
+# Where a weight is large enough to give the library's products (which share the last round's tiles out) tiles for every
+# compute unit several times over.  Plain products (microseconds, tiles and library): 32000 x 2048 41 and 42 at 160 rows, 54
+# and 44 at 256, 68 and 65 at 512, 259 and 252 at 2,048; 12288 x 4096 55 and 56 at 512, 79 and 62 at 640, 80 and 74 at 768.
+# Below that size the tiles win or tie: 4608 x 2048 10 and 14 at 128, 17 and 22 at 640.  Gated products, with the activation
+# that the library's leaves to a kernel of its own: 22016 x 4096 62 and 66 at 200, 90 and 82 at 333, 102 and 99 at 512, 146 and
+# 133 at 640, 147 and 162 at 768, 321 and 428 at 2,048; 11264 x 2048 wins or ties from 65 rows (20 and 33) to 2,048 (99 and
+# 106), 640 rows excepted (49 and 43).
+LIBRARY_PLAIN_WEIGHT = 48e6
+LIBRARY_PLAIN_ROWS = 160
+LIBRARY_GATED_WEIGHT = 64e6
+LIBRARY_GATED_ROWS = (256, 768)  # beyond the first, below the second
+
+
+def library_is_faster(m: int, weight: torch.Tensor, gated: bool = False) -> bool:
+    if gated:
+        return weight.numel() >= LIBRARY_GATED_WEIGHT and LIBRARY_GATED_ROWS[0] < m < LIBRARY_GATED_ROWS[1]
+    return weight.numel() >= LIBRARY_PLAIN_WEIGHT and m >= LIBRARY_PLAIN_ROWS
+
+
+def tiles_product(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
+    """Whether x [M, K] against weight goes to ops.gemm_tiles, once the kernels for few rows have declined."""
+    return (x.shape[0] > STREAM_ROWS and ops.gemm_tiles_supported(x, weight) and (not gated or weight.shape[0] % 32 == 0)
+            and (OWN_KERNELS_ONLY or not library_is_faster(x.shape[0], weight, gated)))
+
+
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and
 # down_proj: 128), and long rows make each workgroup wait for several rounds of loads.  Sharing K out to
 # several workgroups per tile fills the chip: measured 4.3 -> 3.2 microseconds of reading for 2048 x 2048 and
@@ -117,6 +142,11 @@ def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor):
         parts = torch.empty((-(-weight.shape[1] // ops.SLICE_K), m, weight.shape[0]), dtype=torch.float32, device=x.device)
         return PartialSums(ops.gemm_slices(parts, x, weight), x.dtype)
     if not few_rows(m, weight):
+        if tiles_product(x, weight):
+            k_parts = ops.gemm_tiles_plan(m, weight.shape[0], weight.shape[1], 4, ops.compute_units(x.device))[1]
+            if k_parts > 1:
+                parts = torch.empty((k_parts, m, weight.shape[0]), dtype=torch.float32, device=x.device)
+                return PartialSums(ops.gemm_tiles(parts, x, weight), x.dtype)
         return None
     splits = k_splits_for(m, weight)
     if splits < 2:
@@ -140,6 +170,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
             return ops.gemm_decode(out, x, weight, bias)
         if few_rows(m, weight):
             return ops.gemm_stream(out, x, weight, bias)
+        if tiles_product(x, weight) and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0:
+            return ops.gemm_tiles(out, x, weight, bias)
         if OWN_KERNELS_ONLY:
             return ops.gemm_bf16(out, x, weight, bias, kernel="skinny" if m <= 64 else "tile")
         if bias is None:

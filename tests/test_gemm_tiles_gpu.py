@@ -1,0 +1,143 @@
+"""The tiled bfloat16 product of many rows: every tile and epilogue at the edges of tiles, and the plan that picks tiles."""
+
+import math
+
+import pytest
+import torch
+
+DEV = "cuda:0"
+
+
+def ops():
+    from llmserve.ops import library
+
+    return library
+
+
+def rnd(*shape, seed=0, scale=1.0):
+    return (scale * torch.randn(*shape, generator=torch.Generator().manual_seed(seed))).to(torch.bfloat16)
+
+
+def product(x, w, bias=None):
+    y = x.double() @ w.double().t()
+    return y if bias is None else y + bias.double()
+
+
+def close(got, want, k, rounded=True):
+    """32-bit sums of k products of bfloat16 numbers in some order, then (rounded) one rounding to bfloat16."""
+    top = float(want.abs().max())
+    bound = 2e-6 * math.sqrt(k) * top + (2.0 ** -8 * top if rounded else 0.0)
+    assert (got.cpu().double() - want).abs().max() <= bound
+
+
+TILES = range(11)
+
+
+def sizes_of(tile):
+    bm, bn, _, stages, *_ = ops().GEMM_TILES[tile]
+    return bm, bn, 64 * stages
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+def test_plain_and_parts(tile):
+    bm, bn, step = sizes_of(tile)
+    # one row, a row less and more than a tile, several tiles; N of one block, beside a tile's end, several tiles; K of one,
+    # two and five rounds of the buffers
+    for m, n, k in ((1, 16, step), (bm - 1, bn + 16, 2 * step), (bm + 1, bn - 16, step), (2 * bm + 9, 3 * bn + 48, 5 * step)):
+        x, w, b = rnd(m, k + 8, seed=m)[:, :k], rnd(n, k, seed=n), rnd(n, seed=3)
+        xd = rnd(m, k + 8, seed=m).to(DEV)[:, :k]
+        want = product(x, w, b)
+        for dtype in (torch.bfloat16, torch.float32):
+            out = torch.full((m + 1, n + 4), 7.0, dtype=dtype, device=DEV)
+            ops().gemm_tiles(out[:m, :n], xd, w.to(DEV), b.to(DEV), tile=tile)
+            close(out[:m, :n], want, k, dtype == torch.bfloat16)
+            assert bool((out[m:] == 7.0).all()) and bool((out[:, n:] == 7.0).all())
+        want = product(x, w)
+        for parts in (2, 3, 5):
+            if parts <= k // step and (parts - 1) * -(-(k // step) // parts) < k // step:
+                sums = torch.full((parts, m, n), 7.0, device=DEV)
+                ops().gemm_tiles(sums, xd, w.to(DEV), tile=tile)
+                close(sums.double().sum(0), want, k, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("limit,gelu", [(None, False), (1.5, False), (None, True)])
+def test_gated(tile, limit, gelu):
+    bm, bn, step = sizes_of(tile)
+    for m, inter, k in ((1, 16, step), (bm + 3, bn // 2 + 16, 3 * step), (bm - 1, bn + 32, step)):
+        x, w = rnd(m, k, seed=5), rnd(2 * inter, k, seed=6, scale=k ** -0.5)
+        y = product(x, w)
+        gate, up = y[:, :inter], y[:, inter:]
+        if limit is not None:
+            g = gate.clamp(max=limit)
+            want = g * torch.sigmoid(1.702 * g) * (up.clamp(-limit, limit) + 1)
+        elif gelu:
+            want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+        else:
+            want = torch.nn.functional.silu(gate) * up
+        out = torch.full((m, inter + 4), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops().gemm_tiles(out[:, :inter], x.to(DEV), w.to(DEV), swiglu=True, limit=limit, gelu=gelu, tile=tile)
+        # roundings of gate, up, silu and the result: four of 2^-9 of the factors' size
+        bound = 4 * 2.0 ** -9 * float((gate.abs().max() + 1) * (up.abs().max() + 1))
+        assert (out[:, :inter].cpu().double() - want).abs().max() <= bound and bool((out[:, inter:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("nh,nkv,d,bs,bias", [(4, 2, 64, 16, True), (3, 1, 32, 8, False), (2, 2, 128, 5, True), (5, 1, 96, 32, False)])
+def test_rotary(tile, nh, nkv, d, bs, bias):
+    """To the bit what the plain product followed by the rotation's own kernel gives."""
+    bm, _, step = sizes_of(tile)
+    m, k, n = bm + 21, 2 * step, (nh + 2 * nkv) * d
+    x, w = rnd(m, k, seed=7).to(DEV), rnd(n, k, seed=8, scale=k ** -0.5).to(DEV)
+    b = rnd(n, seed=9).to(DEV) if bias else None
+    positions = (torch.arange(m, dtype=torch.int32) * 7 % 4096).to(DEV)
+    inv_freq = (1.0 / (1e4 ** (torch.arange(0, d, 2, dtype=torch.float32) / d))).to(DEV)
+    pages = -(-(m + 4) // bs) + 1
+    slots = torch.arange(3, m + 3, dtype=torch.int32)  # (a run that starts inside a page, with a hole and a jump)
+    slots[m // 2] = -1
+    slots[-1] = pages * bs - 1
+    slots = slots.to(DEV)
+    pools = [torch.full(shape, 7.0, dtype=torch.bfloat16, device=DEV)
+             for shape in ((pages, nkv, bs, d), (pages, nkv, d, bs)) for _ in range(2)]
+    for freq in (inv_freq, None):
+        qkv = ops().gemm_tiles(torch.empty(m, n, dtype=torch.bfloat16, device=DEV), x, w, b, tile=tile)
+        ops().rope_store(qkv, freq, positions, slots, pools[0], pools[2], nh, nkv, d, bs)
+        rope = dict(n_heads=nh, n_kv_heads=nkv, head_dim=d, inv_freq=freq, positions=positions, slots=slots, k_pool=pools[1],
+                    v_pool=pools[3], block_size=bs)
+        q = ops().gemm_tiles(torch.empty(m, nh * d, dtype=torch.bfloat16, device=DEV), x, w, b, rope=rope, tile=tile)
+        assert torch.equal(q, qkv[:, :nh * d])
+        assert torch.equal(pools[0], pools[1]) and torch.equal(pools[2], pools[3])
+    # without slots nothing is stored
+    rope.update(slots=None, inv_freq=inv_freq)
+    ops().gemm_tiles(q, x, w, b, rope=rope, tile=tile)
+    assert torch.equal(pools[0], pools[1]) and torch.equal(pools[2], pools[3])
+
+
+@pytest.mark.gpu
+def test_what_the_kernel_cannot_take_is_refused():
+    x, w = rnd(70, 256).to(DEV), rnd(64, 256).to(DEV)
+    out = torch.empty(70, 64, dtype=torch.bfloat16, device=DEV)
+    for bad in (lambda: ops().gemm_tiles(out, x[:, :192], w[:, :192].contiguous()),            # K in steps of 128
+                lambda: ops().gemm_tiles(out[:, :56], x, w[:56].contiguous()),                  # N in blocks of 16
+                lambda: ops().gemm_tiles(out, x.float(), w.float()),
+                lambda: ops().gemm_tiles(out[:, :48], x, w),
+                lambda: ops().gemm_tiles(torch.empty(70, 66, dtype=torch.bfloat16, device=DEV)[:, 1:65], x, w),
+                lambda: ops().gemm_tiles(out, x, w, w[0, :64], swiglu=True),
+                lambda: ops().gemm_tiles(torch.empty(2, 70, 64, device=DEV, dtype=torch.bfloat16), x, w)):
+        with pytest.raises(ValueError):
+            bad()
+
+
+def test_plan():
+    """The plan names a tile whose buffers divide K, and no more parts than were allowed or than K has."""
+    for m in (17, 64, 65, 128, 333, 512, 2048, 8191):
+        for n, k in ((16, 128), (2560, 2048), (2048, 5632), (22016, 4096), (4096, 11008), (160, 384)):
+            for most in (1, 2, 4):
+                tile, parts = ops().gemm_tiles_plan(m, n, k, most)
+                groups = k // (64 * ops().GEMM_TILES[tile][3])
+                assert k % (64 * ops().GEMM_TILES[tile][3]) == 0 and 1 <= parts <= min(most, groups)
+                assert (parts - 1) * -(-groups // parts) < groups
+    assert ops().gemm_tiles_plan(128, 2048, 5632, 4)[1] == 4 and ops().gemm_tiles_plan(2048, 2048, 2048, 4)[1] == 1

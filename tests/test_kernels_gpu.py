@@ -223,7 +223,7 @@ def test_gemm_fma(m, n, k):
 
 # rows around the kernels' blocks of 16, 32 and 64, tiles of 32, 64 and 128; N beside a tile's end; K no multiple of a chunk
 @pytest.mark.parametrize("m,n,k", [(1, 333, 4), (2, 16, 36), (16, 2560, 2048), (17, 100, 96), (32, 8300, 68), (33, 333, 1000),
-                                   (64, 8210, 132), (65, 65, 20), (130, 4100, 100), (300, 513, 1000), (2050, 4098, 36)])
+                                   (64, 8210, 516), (40, 70, 508), (65, 65, 20), (130, 4100, 100), (300, 513, 1000), (2050, 4098, 36)])
 def test_gemm32(m, n, k):
     a, w, b = rnd(m, k + 4, seed=8)[:, :k], rnd(n, k, seed=9), rnd(n, seed=10)
     ref = a.double() @ w.double().t() + b.double()
@@ -234,6 +234,8 @@ def test_gemm32(m, n, k):
     assert (out[:, :n].cpu().double() - ref).abs().max() <= bound and bool((out[:, n:] == 7.0).all())
     whole = ops().gemm32(torch.empty(m, n, device=DEV), a.to(DEV), w.to(DEV), b.to(DEV))
     assert torch.equal(whole, out[:, :n])
+    if m > 64 or k < 512:  # (tiles: the products in the order of the columns, as the multiply-add kernel sums them)
+        assert torch.equal(whole, ops().gemm_fma(torch.empty(m, n, device=DEV), a.to(DEV), w.to(DEV), b.to(DEV)))
     with pytest.raises(ValueError):
         ops().gemm32(whole, a.bfloat16().to(DEV), w.bfloat16().to(DEV))
 
