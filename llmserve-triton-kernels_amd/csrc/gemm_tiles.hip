@@ -23,7 +23,7 @@
 // What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times
 // its matrix instructions); beyond, LDS and matrix cores together, and how evenly the tiles fill 256 compute units.
 //
-// K must be a multiple of 64 S (the host checks), N of 16, rows of X and W 16-byte aligned; M is arbitrary: rows beyond M
+// K must be a multiple of 64 (the host checks), N of 16, rows of X and W 16-byte aligned; M is arbitrary: rows beyond M
 // are read as zeros or as row 0 and never stored.
 #include "common.h"
 
@@ -94,12 +94,12 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     constexpr int LM = BM / 8 / NW, LN = BN / 8 / NW;  // loads of 8 rows, per wave
     static_assert(LM * NW * 8 == BM && LN * NW * 8 == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile does not divide");
     static_assert(TN % 2 == 0, "columns that belong together lie in one wave");
-    static_assert(S == 2 || S == 4, "buffers");
+    static_assert(S >= 2 && S <= 4, "buffers");
     constexpr int TILE = (BM + BN) * 128;
     __shared__ __attribute__((aligned(1024))) uint8_t lds0[TILE];
     __shared__ __attribute__((aligned(1024))) uint8_t lds1[TILE];
     __shared__ __attribute__((aligned(1024))) uint8_t lds2[S > 2 ? TILE : 16];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds3[S > 2 ? TILE : 16];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds3[S > 3 ? TILE : 16];
 
     const int part = EPI == GT_FLOAT ? blockIdx.x / a.tiles : 0, pid = blockIdx.x - part * a.tiles;
     const int first = part * a.steps, steps = min(a.steps, a.K / 64 - first);
@@ -112,8 +112,15 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
     const int r16 = lane % 16, g = lane / 16;
 
+    int slots[TM];  // (asked for here, used in the epilogue)
+    if constexpr (EPI == GT_ROTARY) {
+#pragma unroll
+        for (int j = 0; j < TM; ++j) slots[j] = a.slots ? a.slots[min(m0 + wm + j * 16 + r16, a.M - 1)] : -1;
+    }
+
     // A load brings 8 rows: lane l row l / 8, the piece (l % 8) ^ (l / 8) of its 128 bytes, to place l.  Each load has a
     // buffer of its own that starts with its first row and ends with the matrix (groups of rows beyond it: with row 0).
+    // Steps beyond the last are asked for beyond the buffers' ends: zeros, and no memory is touched.
     const int lr = lane / 8, lc = ((lane % 8) ^ lr) * 16;
     const unsigned x_off = (unsigned)(lr * a.ldx * 2 + lc), w_off = (unsigned)(lr * a.K * 2 + lc);
     __amdgpu_buffer_rsrc_t xb[LM], wb[LN];
@@ -127,20 +134,22 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
 #pragma unroll
     for (int i = 0; i < LN; ++i) {
         const int c = n0 + (wave * LN + i) * 8;
-        const int r = c < a.N ? gt_weight_row<EPI>(a, c) : 0;
-        wb[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.W + (size_t)r * a.K), 0, (unsigned)(8 * a.K) * 2u, 0x00020000);
+        wb[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.W + (size_t)(c < a.N ? gt_weight_row<EPI>(a, c) : 0) * a.K), 0,
+                                                  (unsigned)(8 * a.K) * 2u, 0x00020000);
     }
     auto fetch = [&](uint8_t* lds, int step) {
-        const int so = (first + step) * 128;
 #if defined(__HIP_DEVICE_COMPILE__)
+        const bool live = step < steps;
+        const int so = live ? (first + step) * 128 : 0;
+        const unsigned xo = live ? x_off : 0x80000000u, wo = live ? w_off : 0x80000000u;
 #pragma unroll
         for (int i = 0; i < LM; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xb[i], (__attribute__((address_space(3))) void*)(lds + (wave * LM + i) * 1024), 16,
-                                                     x_off, so, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xb[i], (__attribute__((address_space(3))) void*)(lds + (wave * LM + i) * 1024), 16, xo,
+                                                     so, 0, 0);
 #pragma unroll
         for (int i = 0; i < LN; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                wb[i], (__attribute__((address_space(3))) void*)(lds + BM * 128 + (wave * LN + i) * 1024), 16, w_off, so, 0, 0);
+                wb[i], (__attribute__((address_space(3))) void*)(lds + BM * 128 + (wave * LN + i) * 1024), 16, wo, so, 0, 0);
 #endif
     };
 
@@ -187,97 +196,93 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     // One step: `now` holds it, its first half is in registers; `next` holds the step behind it.  At the barrier every wave
     // has read all of `now`, which then takes the step S further on.
     int step = 0;
-    auto one = [&](uint8_t* now, uint8_t* next, auto left, auto more, auto last) {
-        constexpr bool MORE = decltype(more)::n, LAST = decltype(last)::n;
+    auto one = [&](uint8_t* now, uint8_t* next) {
         read(now, 1);
         multiply(0);
         interleave(Number<0>());
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (LAST) {
-            multiply(1);
-        } else {
-            arrive(left);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (MORE) fetch(now, step + S);
-            read(next, 0);
-            multiply(1);
-            interleave(Number<MORE ? LM + LN : 0>());
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        arrive(Number<S - 2>());
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(now, step + S);
+        read(next, 0);
+        multiply(1);
+        interleave(Number<LM + LN>());
+        __builtin_amdgcn_sched_barrier(0);
         ++step;
     };
-    typedef Number<1> Yes;
-    typedef Number<0> No;
     fetch(lds0, 0);
     fetch(lds1, 1);
-    if constexpr (S > 2) {
-        fetch(lds2, 2);
-        fetch(lds3, 3);
-    }
+    if constexpr (S > 2) fetch(lds2, 2);
+    if constexpr (S > 3) fetch(lds3, 3);
     arrive(Number<S - 1>());
     read(lds0, 0);
-    for (int rounds = steps / S - 1; rounds > 0; --rounds) {
+    for (int rounds = (steps + S - 1) / S; rounds > 0; --rounds) {
+        one(lds0, lds1);
         if constexpr (S == 2) {
-            one(lds0, lds1, Number<0>(), Yes(), No());
-            one(lds1, lds0, Number<0>(), Yes(), No());
+            one(lds1, lds0);
+        } else if constexpr (S == 3) {
+            one(lds1, lds2);
+            one(lds2, lds0);
         } else {
-            one(lds0, lds1, Number<2>(), Yes(), No());
-            one(lds1, lds2, Number<2>(), Yes(), No());
-            one(lds2, lds3, Number<2>(), Yes(), No());
-            one(lds3, lds0, Number<2>(), Yes(), No());
+            one(lds1, lds2);
+            one(lds2, lds3);
+            one(lds3, lds0);
         }
     }
-    if constexpr (S == 2) {
-        one(lds0, lds1, Number<0>(), No(), No());
-        one(lds1, lds0, Number<0>(), No(), Yes());
-    } else {
-        one(lds0, lds1, Number<2>(), No(), No());
-        one(lds1, lds2, Number<1>(), No(), No());
-        one(lds2, lds3, Number<0>(), No(), No());
-        one(lds3, lds0, Number<0>(), No(), Yes());
-    }
+    arrive(Number<0>());  // (no load may find the workgroup gone)
 
     // ---- epilogue: a lane holds 4 consecutive columns of row m in each acc[i][j]; blocks i and i + 1 (i even) belong together
+    if constexpr (EPI == GT_ROTARY) {
+        const int D = a.head_dim, half = D / 2, bs = a.block_size, nkv = a.n_kv_heads, turned = (a.n_heads + nkv) * D;
+        // The angles of a pair of blocks are asked for before the pair in front of them is stored: behind the stores, each row's
+        // would be waited for on its own (the compiler cannot know that they do not overlap), which took 10 microseconds of
+        // the 36 that q, k and v of 2,048 rows of the 1.1B shape took.
+        constexpr int AHEAD = NW == 4 ? 2 : 1;  // (8 waves leave no registers for a second pair's)
+        f32x4 table[AHEAD][TM][2];
+        auto ask = [&](int i) {
+            const int c = n0 + wn + i * 16;  // (the same for all lanes: the branches on it are uniform)
+            if (!a.angles || c >= turned) return;
+            const int row = gt_weight_row<EPI>(a, c) + g * 4, d = row % D;
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-        const int m = m0 + wm + j * 16 + r16;
-        if (m >= a.M) continue;
-        if constexpr (EPI == GT_GATED) {
-#pragma unroll
-            for (int i = 0; i < TN; i += 2) {
-                const int n = (n0 + wn) / 2 + i * 8 + g * 4;
-                if (n >= a.inter) continue;
-                const f32x4 lo = acc[i][j], hi = acc[i + 1][j];
-                gt_store4(reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + n, gt_unit(a, lo[0], hi[0]), gt_unit(a, lo[1], hi[1]),
-                          gt_unit(a, lo[2], hi[2]), gt_unit(a, lo[3], hi[3]));
+            for (int j = 0; j < TM; ++j) {
+                const int m = min(m0 + wm + j * 16 + r16, a.M - 1);
+                const f32x4* from = reinterpret_cast<const f32x4*>(a.angles + ((size_t)m * half + d) * 2);
+                table[(i / 2) % AHEAD][j][0] = from[0];
+                table[(i / 2) % AHEAD][j][1] = from[1];
             }
-        } else if constexpr (EPI == GT_ROTARY) {
-            const int D = a.head_dim, half = D / 2, bs = a.block_size, nkv = a.n_kv_heads;
-            const int slot = a.slots ? a.slots[m] : -1;
-            const int page = a.bs_shift >= 0 ? slot >> a.bs_shift : slot / bs, off = slot - page * bs;  // (used where slot >= 0)
+        };
+        if (AHEAD == 2) ask(0);
 #pragma unroll
-            for (int i = 0; i < TN; i += 2) {
-                const int c = n0 + wn + i * 16;  // (the same for all lanes: the branches below are uniform)
-                if (c >= a.N) continue;
-                f32x4 lo = acc[i][j], hi = acc[i + 1][j];
-                const int row_lo = gt_weight_row<EPI>(a, c) + g * 4, row_hi = gt_weight_row<EPI>(a, c + 16) + g * 4;
-                if (a.bias) {
+        for (int i = 0; i < TN; i += 2) {
+            if (AHEAD == 1) ask(i);
+            else if (i + 2 < TN) ask(i + 2);
+            const int c = n0 + wn + i * 16;
+            if (c >= a.N) continue;
+            const int row_lo = gt_weight_row<EPI>(a, c) + g * 4, row_hi = gt_weight_row<EPI>(a, c + 16) + g * 4;
+            const int head = row_lo / D, d = row_lo - head * D;
+            float b_lo[4] = {}, b_hi[4] = {};
+            if (a.bias) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        lo[r] += bf16_bits_to_f32(a.bias[row_lo + r].bits);
-                        hi[r] += bf16_bits_to_f32(a.bias[row_hi + r].bits);
-                    }
+                for (int r = 0; r < 4; ++r) {
+                    b_lo[r] = bf16_bits_to_f32(a.bias[row_lo + r].bits);
+                    b_hi[r] = bf16_bits_to_f32(a.bias[row_hi + r].bits);
                 }
+            }
+#pragma unroll
+            for (int j = 0; j < TM; ++j) {
+                const int m = m0 + wm + j * 16 + r16;
+                if (m >= a.M) continue;
+                const int slot = slots[j];
+                const int page = a.bs_shift >= 0 ? slot >> a.bs_shift : slot / bs, off = slot - page * bs;  // (used where slot >= 0)
+                float lo[4], hi[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {  // (the projection's result is bfloat16 before it is rotated)
-                    lo[r] = round_to<bf16>(lo[r]);
-                    hi[r] = round_to<bf16>(hi[r]);
+                    lo[r] = round_to<bf16>(acc[i][j][r] + b_lo[r]);
+                    hi[r] = round_to<bf16>(acc[i + 1][j][r] + b_hi[r]);
                 }
-                if (c < (a.n_heads + nkv) * D) {
-                    const int head = row_lo / D, d = row_lo - head * D;
+                if (c < turned) {
                     if (a.angles) {
-                        const f32x4* table = reinterpret_cast<const f32x4*>(a.angles + ((size_t)m * half + d) * 2);
-                        const f32x4 s0 = table[0], s1 = table[1];
+                        const f32x4 s0 = table[(i / 2) % AHEAD][j][0], s1 = table[(i / 2) % AHEAD][j][1];
                         const float sn[4] = {s0[0], s0[2], s1[0], s1[2]}, cs[4] = {s0[1], s0[3], s1[1], s1[3]};
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
@@ -296,13 +301,28 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
                 } else if (slot >= 0) {
                     // a page holds [kv head][dimension][token]: 16 lanes are 16 tokens, mostly side by side in a page
                     bf16* v = a.v_pool + (size_t)page * nkv * D * bs + off;
-                    const int f_lo = row_lo - (a.n_heads + nkv) * D, f_hi = row_hi - (a.n_heads + nkv) * D;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        v[(size_t)(f_lo + r) * bs].bits = f32_to_bf16_bits(lo[r]);
-                        v[(size_t)(f_hi + r) * bs].bits = f32_to_bf16_bits(hi[r]);
+                        v[(size_t)(row_lo - turned + r) * bs].bits = f32_to_bf16_bits(lo[r]);
+                        v[(size_t)(row_hi - turned + r) * bs].bits = f32_to_bf16_bits(hi[r]);
                     }
                 }
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        const int m = m0 + wm + j * 16 + r16;
+        if (m >= a.M) continue;
+        if constexpr (EPI == GT_GATED) {
+#pragma unroll
+            for (int i = 0; i < TN; i += 2) {
+                const int n = (n0 + wn) / 2 + i * 8 + g * 4;
+                if (n >= a.inter) continue;
+                const f32x4 lo = acc[i][j], hi = acc[i + 1][j];
+                gt_store4(reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + n, gt_unit(a, lo[0], hi[0]), gt_unit(a, lo[1], hi[1]),
+                          gt_unit(a, lo[2], hi[2]), gt_unit(a, lo[3], hi[3]));
             }
         } else {
 #pragma unroll
@@ -325,12 +345,12 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
 
 template <int BM, int BN, int WM, int WN, int S>
 static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
-    LLMS_REQUIRE(a.K % (64 * S) == 0, "gemm_tiles: K does not divide into this tile's steps");
-    const int tiles_n = (a.N + BN - 1) / BN, groups = a.K / 64 / S;
+    LLMS_REQUIRE(a.K % 64 == 0, "gemm_tiles: K must be a multiple of 64");
+    const int tiles_n = (a.N + BN - 1) / BN;
     a.tiles_m = (a.M + BM - 1) / BM;
     LLMS_REQUIRE((long long)a.tiles_m * tiles_n * parts < (1ll << 31), "gemm_tiles: too many tiles");
     a.tiles = a.tiles_m * tiles_n;
-    a.steps = (groups + parts - 1) / parts * S;
+    a.steps = (a.K / 64 + parts - 1) / parts;
     LLMS_REQUIRE((long long)(parts - 1) * a.steps < a.K / 64, "gemm_tiles: a part of K is empty");
     const dim3 grid((unsigned)(a.tiles * parts)), block(WM * WN * LLMS_WAVE);
     if (epilogue == GT_PLAIN) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_PLAIN><<<grid, block, 0, stream>>>(a);
@@ -400,10 +420,11 @@ int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* 
         case 4: return launch<128, 128, 2, 2, 4>(epilogue, a, parts, stream);
         case 5: return launch<128, 192, 2, 2, 4>(epilogue, a, parts, stream);
         case 6: return launch<192, 128, 2, 2, 4>(epilogue, a, parts, stream);
-        case 7: return launch<160, 128, 2, 2, 2>(epilogue, a, parts, stream);
-        case 8: return launch<192, 128, 2, 2, 2>(epilogue, a, parts, stream);
-        case 9: return launch<256, 192, 2, 2, 2>(epilogue, a, parts, stream);
-        case 10: return launch<256, 256, 2, 4, 2>(epilogue, a, parts, stream);
+        case 7: return launch<192, 128, 2, 2, 2>(epilogue, a, parts, stream);
+        case 8: return launch<256, 128, 2, 2, 3>(epilogue, a, parts, stream);
+        case 9: return launch<160, 192, 2, 2, 3>(epilogue, a, parts, stream);
+        case 10: return launch<192, 192, 2, 2, 3>(epilogue, a, parts, stream);
+        case 11: return launch<256, 256, 2, 4, 2>(epilogue, a, parts, stream);
     }
     LLMS_REQUIRE(false, "gemm_tiles: no such tile");
 }

@@ -605,10 +605,10 @@ SLICE_K = 512  # what one workgroup of gemm_slices takes of K
 # Tiles of ops.gemm_tiles (the order is the launcher's): rows of x, rows of w, workgroups a compute unit holds, steps of 64
 # columns its LDS holds, and the microseconds a step takes with one workgroup on every compute unit and with all it holds:
 # fitted to 150 products (65 to 2,048 rows; K of 2,048 to 11,008, N of 2,048 to 22,016), over which the plan below is 1 % off
-# the best tile in the mean and 18 % at worst.
-GEMM_TILES = ((64, 64, 2, 4, 0.23, 0.37), (96, 64, 2, 4, 0.245, 0.43), (128, 64, 1, 4, 0.32, 0.32), (96, 128, 1, 4, 0.40, 0.40),
-              (128, 128, 1, 4, 0.52, 0.52), (128, 192, 1, 4, 0.70, 0.70), (192, 128, 1, 4, 0.60, 0.60), (160, 128, 2, 2, 1.08, 0.90),
-              (192, 128, 2, 2, 1.57, 1.00), (256, 192, 1, 2, 1.31, 1.31), (256, 256, 1, 2, 1.33, 1.33))
+# the best tile in the mean.
+GEMM_TILES = ((64, 64, 2, 4, 0.20, 0.33), (96, 64, 2, 4, 0.255, 0.40), (128, 64, 1, 4, 0.31, 0.31), (96, 128, 1, 4, 0.39, 0.39),
+              (128, 128, 1, 4, 0.50, 0.50), (128, 192, 1, 4, 0.755, 0.755), (192, 128, 1, 4, 0.62, 0.62), (192, 128, 2, 2, 0.94, 1.23),
+              (256, 128, 1, 3, 0.85, 0.85), (160, 192, 1, 3, 0.81, 0.81), (192, 192, 1, 3, 0.90, 0.90), (256, 256, 1, 2, 1.47, 1.47))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -620,26 +620,24 @@ def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256)
     sizes alone."""
     best = None
     for tile, (bm, bn, held, stages, one, full) in enumerate(GEMM_TILES):
-        groups = k // (64 * stages)
-        if k % (64 * stages):
-            continue
         for parts in (1, 2, 4):
-            if parts > most_parts or parts > groups or (parts - 1) * -(-groups // parts) >= groups:
+            steps = -(-(k // 64) // parts)
+            if parts > most_parts or (parts - 1) * steps >= k // 64:
                 continue
-            steps = -(-groups // parts) * stages
+            steps = -(-steps // stages) * stages
             workgroups = -(-m // bm) * -(-n // bn) * parts
             rounds, rest = divmod(workgroups, held * cus)
             cost = steps * (rounds * full + (0.0 if rest == 0 else one if rounds == 0 and rest <= cus else full)) + rounds + (rest > 0)
             if parts > 1:
-                cost += m * n * (7.4 * parts - 4) / 4.0e6
+                cost += m * n * (6 * parts - 4) / 5.0e6
             if best is None or cost < best[0]:
                 best = (cost, tile, parts)
     return best[1:]
 
 
 def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 128, blocks of 16 weight rows, 16-byte rows."""
-    return gemm_bf16_supported(x, w) and x.shape[1] % 128 == 0 and w.shape[0] % 16 == 0 and w.dtype == torch.bfloat16
+    """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 64, blocks of 16 weight rows, 16-byte rows."""
+    return gemm_bf16_supported(x, w) and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0 and w.dtype == torch.bfloat16
 
 
 def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *, swiglu: bool = False,
@@ -665,7 +663,7 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
             raise ValueError("parts of K leave plain sums in a contiguous float32 [parts, M, N] tensor, without a bias")
         part_stride = out.stride(0)
     if x.dtype != torch.bfloat16 or not gemm_tiles_supported(x, w):
-        raise ValueError(f"gemm_tiles takes bfloat16 operands, 16-byte aligned, K ({k}) a multiple of 128, N ({n}) of 16")
+        raise ValueError(f"gemm_tiles takes bfloat16 operands, 16-byte aligned, K ({k}) a multiple of 64, N ({n}) of 16")
     if out.dtype != torch.bfloat16 and (out.dtype != torch.float32 or swiglu or rope is not None):
         raise ValueError("out must be bfloat16, or float32 with the plain epilogue")
     if out.stride(-2) % 4 or out.data_ptr() % (4 * out.element_size()):

@@ -16,7 +16,7 @@ bfloat16, few rows otherwise: the hand-written kernel that streams the weight on
 bfloat16, more rows: ops.gemm_tiles, tiles on the matrix cores with the activation, the rotation and cache store, or the
   partial sums of a product that goes to a norm in the epilogue; the library's matrix product (hipBLASLt through
   torch.mm), which is where the reference's engine uses a library too (nn.Linear, src/llmserve/model/llama.py:64-67), only
-  for the sizes where it is still the faster one (library_is_faster) and for K or N that the tiles cannot take.
+  for the sizes where it is still the faster one (tiles_product) and for K or N that the tiles cannot take.
 Operands the matrix-core kernels cannot take (K not a multiple of 8) fall to the 32-bit
 multiply-add kernel, which takes anything.
 
@@ -71,29 +71,25 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
         return m > 0
     return m <= STREAM_MAX_ROWS and -(-m // 16) * weight.numel() * 2 <= STREAM_REREAD_BYTES
 
-# Where a weight is large enough to give the library's products (which share the last round's tiles out) tiles for every
-# compute unit several times over.  Plain products (microseconds, tiles and library): 32000 x 2048 41 and 42 at 160 rows, 54
-# and 44 at 256, 68 and 65 at 512, 259 and 252 at 2,048; 12288 x 4096 55 and 56 at 512, 79 and 62 at 640, 80 and 74 at 768.
-# Below that size the tiles win or tie: 4608 x 2048 10 and 14 at 128, 17 and 22 at 640.  Gated products, with the activation
-# that the library's leaves to a kernel of its own: 22016 x 4096 62 and 66 at 200, 90 and 82 at 333, 102 and 99 at 512, 146 and
-# 133 at 640, 147 and 162 at 768, 321 and 428 at 2,048; 11264 x 2048 wins or ties from 65 rows (20 and 33) to 2,048 (99 and
-# 106), 640 rows excepted (49 and 43).
-LIBRARY_PLAIN_WEIGHT = 48e6
-LIBRARY_PLAIN_ROWS = 160
-LIBRARY_GATED_WEIGHT = 64e6
-LIBRARY_GATED_ROWS = (256, 768)  # beyond the first, below the second
+# A plain product against a weight this large (the vocabulary's) stays with the library from some rows on: it has tiles for
+# every compute unit several times over, and the library shares the last round's out.  Microseconds, tiles and library:
+# 32000 x 2048 40 and 39 at 160 rows, 54 and 44 at 256, 68 and 65 at 512, 268 and 262 at 2,048; 12288 x 4096 53 and 53 at
+# 333, 56 and 55 at 512, 97 and 87 at 1,024.  Smaller weights win or tie (2048 x 5632 22 and 28 at 333, 56 and 60 at
+# 2,048; 4608 x 2048 12 and 22 at 200), and gated products mostly, with the activation that the library's leaves to a kernel
+# of its own (11264 x 2048 34 and 40 at 333, 101 and 103 at 2,048; 22016 x 4096 75 and 82 at 333, 111 and 96 at 512, 197 and
+# 183 at 1,024, 321 and 424 at 2,048).
+LIBRARY_WEIGHT = 48e6
+LIBRARY_ROWS = 160
 
 
-def library_is_faster(m: int, weight: torch.Tensor, gated: bool = False) -> bool:
-    if gated:
-        return weight.numel() >= LIBRARY_GATED_WEIGHT and LIBRARY_GATED_ROWS[0] < m < LIBRARY_GATED_ROWS[1]
-    return weight.numel() >= LIBRARY_PLAIN_WEIGHT and m >= LIBRARY_PLAIN_ROWS
+def tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether x [M, K] against weight may go to ops.gemm_tiles, once the kernels for few rows have declined."""
+    return x.shape[0] > STREAM_ROWS and ops.gemm_tiles_supported(x, weight)
 
 
-def tiles_product(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
-    """Whether x [M, K] against weight goes to ops.gemm_tiles, once the kernels for few rows have declined."""
-    return (x.shape[0] > STREAM_ROWS and ops.gemm_tiles_supported(x, weight) and (not gated or weight.shape[0] % 32 == 0)
-            and (OWN_KERNELS_ONLY or not library_is_faster(x.shape[0], weight, gated)))
+def tiles_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether a plain product goes there."""
+    return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or not (weight.numel() >= LIBRARY_WEIGHT and x.shape[0] >= LIBRARY_ROWS))
 
 
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and

@@ -30,7 +30,7 @@ def close(got, want, k, rounded=True):
     assert (got.cpu().double() - want).abs().max() <= bound
 
 
-TILES = range(11)
+TILES = range(12)
 
 
 def sizes_of(tile):
@@ -42,9 +42,10 @@ def sizes_of(tile):
 @pytest.mark.parametrize("tile", TILES)
 def test_plain_and_parts(tile):
     bm, bn, step = sizes_of(tile)
-    # one row, a row less and more than a tile, several tiles; N of one block, beside a tile's end, several tiles; K of one,
-    # two and five rounds of the buffers
-    for m, n, k in ((1, 16, step), (bm - 1, bn + 16, 2 * step), (bm + 1, bn - 16, step), (2 * bm + 9, 3 * bn + 48, 5 * step)):
+    # one row, a row less and more than a tile, several tiles; N of one block, beside a tile's end, several tiles; K of one
+    # step, one round of the buffers, a step more and less than two, ten
+    for m, n, k in ((1, 16, 64), (bm - 1, bn + 16, step), (bm + 1, bn - 16, 2 * step + 64), (17, 48, 2 * step - 64),
+                    (2 * bm + 9, 3 * bn + 48, 10 * step)):
         x, w, b = rnd(m, k + 8, seed=m)[:, :k], rnd(n, k, seed=n), rnd(n, seed=3)
         xd = rnd(m, k + 8, seed=m).to(DEV)[:, :k]
         want = product(x, w, b)
@@ -55,7 +56,7 @@ def test_plain_and_parts(tile):
             assert bool((out[m:] == 7.0).all()) and bool((out[:, n:] == 7.0).all())
         want = product(x, w)
         for parts in (2, 3, 5):
-            if parts <= k // step and (parts - 1) * -(-(k // step) // parts) < k // step:
+            if (parts - 1) * -(-(k // 64) // parts) < k // 64:
                 sums = torch.full((parts, m, n), 7.0, device=DEV)
                 ops().gemm_tiles(sums, xd, w.to(DEV), tile=tile)
                 close(sums.double().sum(0), want, k, False)
@@ -66,7 +67,7 @@ def test_plain_and_parts(tile):
 @pytest.mark.parametrize("limit,gelu", [(None, False), (1.5, False), (None, True)])
 def test_gated(tile, limit, gelu):
     bm, bn, step = sizes_of(tile)
-    for m, inter, k in ((1, 16, step), (bm + 3, bn // 2 + 16, 3 * step), (bm - 1, bn + 32, step)):
+    for m, inter, k in ((1, 16, 64), (bm + 3, bn // 2 + 16, 2 * step + 64), (bm - 1, bn + 32, step)):
         x, w = rnd(m, k, seed=5), rnd(2 * inter, k, seed=6, scale=k ** -0.5)
         y = product(x, w)
         gate, up = y[:, :inter], y[:, inter:]
@@ -120,7 +121,7 @@ def test_rotary(tile, nh, nkv, d, bs, bias):
 def test_what_the_kernel_cannot_take_is_refused():
     x, w = rnd(70, 256).to(DEV), rnd(64, 256).to(DEV)
     out = torch.empty(70, 64, dtype=torch.bfloat16, device=DEV)
-    for bad in (lambda: ops().gemm_tiles(out, x[:, :192], w[:, :192].contiguous()),            # K in steps of 128
+    for bad in (lambda: ops().gemm_tiles(out, x[:, :96], w[:, :96].contiguous()),              # K in steps of 64
                 lambda: ops().gemm_tiles(out[:, :56], x, w[:56].contiguous()),                  # N in blocks of 16
                 lambda: ops().gemm_tiles(out, x.float(), w.float()),
                 lambda: ops().gemm_tiles(out[:, :48], x, w),
@@ -132,12 +133,11 @@ def test_what_the_kernel_cannot_take_is_refused():
 
 
 def test_plan():
-    """The plan names a tile whose buffers divide K, and no more parts than were allowed or than K has."""
+    """The plan names a tile, and no more parts than were allowed or than K has steps for."""
     for m in (17, 64, 65, 128, 333, 512, 2048, 8191):
         for n, k in ((16, 128), (2560, 2048), (2048, 5632), (22016, 4096), (4096, 11008), (160, 384)):
             for most in (1, 2, 4):
                 tile, parts = ops().gemm_tiles_plan(m, n, k, most)
-                groups = k // (64 * ops().GEMM_TILES[tile][3])
-                assert k % (64 * ops().GEMM_TILES[tile][3]) == 0 and 1 <= parts <= min(most, groups)
-                assert (parts - 1) * -(-groups // parts) < groups
+                assert 0 <= tile < len(ops().GEMM_TILES) and 1 <= parts <= most
+                assert (parts - 1) * -(-(k // 64) // parts) < k // 64
     assert ops().gemm_tiles_plan(128, 2048, 5632, 4)[1] == 4 and ops().gemm_tiles_plan(2048, 2048, 2048, 4)[1] == 1
