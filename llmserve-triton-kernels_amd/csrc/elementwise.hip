@@ -167,6 +167,50 @@ __global__ void rmsnorm_bf16_vec_kernel(bf16* __restrict__ out, const bf16* x, c
     }
 }
 
+// The same for float rows of hidden % 4 == 0 and hidden <= 4 * RV_CHUNKS * 256: the row, what is added to
+// it and the norm's weight are asked for at once (one wait for memory; the plain kernel waits three times: rows of 2,048
+// take 4.8 microseconds under the profiler, 5.7 there).
+__global__ __launch_bounds__(256) void rmsnorm_f32_vec_kernel(float* __restrict__ out, const float* x, const float* __restrict__ delta,
+                                                              float* resid_out, const float* __restrict__ weight,
+                                                              const int* __restrict__ rows, float eps, int hidden,
+                                                              const float* __restrict__ parts, int n_parts, size_t part_stride) {
+    __shared__ float red[16];
+    const int r = blockIdx.x;
+    const size_t s = rows ? rows[r] : r;
+    float4 v[RV_CHUNKS], d[RV_CHUNKS], w[RV_CHUNKS];
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int c = 0; c < RV_CHUNKS; ++c) {
+        const int i = 4 * (threadIdx.x + c * 256);
+        const bool in = i < hidden;
+        w[c] = in ? *reinterpret_cast<const float4*>(weight + i) : zero;
+        v[c] = in ? *reinterpret_cast<const float4*>(x + s * hidden + i) : zero;
+        d[c] = (in && delta) ? *reinterpret_cast<const float4*>(delta + s * hidden + i) : zero;
+        if (in && parts)  // (partial sums, added up in order)
+            for (int p = 0; p < n_parts; ++p) {
+                const float4 a = *reinterpret_cast<const float4*>(parts + p * part_stride + s * hidden + i);
+                d[c].x += a.x, d[c].y += a.y, d[c].z += a.z, d[c].w += a.w;
+            }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < RV_CHUNKS; ++c) {
+        const int i = 4 * (threadIdx.x + c * 256);
+        v[c].x += d[c].x, v[c].y += d[c].y, v[c].z += d[c].z, v[c].w += d[c].w;
+        if (resid_out && i < hidden) *reinterpret_cast<float4*>(resid_out + s * hidden + i) = v[c];
+        ss += v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
+    }
+    ss = block_sum(ss, red);
+    const float inv = rsqrtf(ss / (float)hidden + eps);
+#pragma unroll
+    for (int c = 0; c < RV_CHUNKS; ++c) {
+        const int i = 4 * (threadIdx.x + c * 256);
+        if (i < hidden)
+            *reinterpret_cast<float4*>(out + (size_t)r * hidden + i) =
+                make_float4(w[c].x * (v[c].x * inv), w[c].y * (v[c].y * inv), w[c].z * (v[c].z * inv), w[c].w * (v[c].w * inv));
+    }
+}
+
 // ------------------------------------------------------------------ rotary encoding + cache store
 // qkv row n = [q heads | k heads | v heads], head_dim wide each.
 //   q, k: x' = x*cos + rotate_half(x)*sin with pairs (i, i + D/2) and angle
@@ -526,6 +570,12 @@ int llms_rmsnorm(int dtype, void* out, const void* x, const void* delta, void* r
         rmsnorm_bf16_vec_kernel<<<n_rows, threads, 0, stream>>>((bf16*)out, (const bf16*)x, (const bf16*)delta,
                                                                 (bf16*)resid_out, (const bf16*)weight, rows, eps,
                                                                 hidden, parts, n_parts, part_stride);
+        LLMS_LAUNCH_CHECK();
+    }
+    if (dtype == 0 && (!parts || (((uintptr_t)parts % 16) == 0 && part_stride % 4 == 0)) && hidden % 4 == 0 && hidden <= 4 * RV_CHUNKS * 256 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
+        ((uintptr_t)weight % 16) == 0 && ((uintptr_t)delta % 16) == 0 && ((uintptr_t)resid_out % 16) == 0) {
+        rmsnorm_f32_vec_kernel<<<n_rows, 256, 0, stream>>>((float*)out, (const float*)x, (const float*)delta, (float*)resid_out,
+                                                           (const float*)weight, rows, eps, hidden, parts, n_parts, part_stride);
         LLMS_LAUNCH_CHECK();
     }
     const int threads = hidden >= 2048 ? 512 : 256;
