@@ -1,0 +1,521 @@
+// The composed attention on the matrix cores, bfloat16, where a column meets the values before heads are mixed.
+//
+// With mixed heads a result is sum_g talk[h, g] sum_j w_g(j) v_h(j).  Mixing the weights w_g first needs them normalised, so
+// two walks over the keys, and every head's weights of a token through LDS.  Here each score column g is multiplied with the
+// values of *all* key/value heads in one walk, u_g[k] = sum_j w_g(j) v_k(j), and the results are mixed once at the end:
+// o_h = sum_g talk[h, g] u_g[kv(h)].  That is kv_heads times the value products (4 of 20 matrix instructions become 16 of 20 at 4
+// key/value heads) and nothing else per key: a plain online softmax whose values are kv_heads * dv wide.  Up to 256 columns
+// of values (64 registers of results a lane) it is the faster way.  Two score maps are the same walk with a map's columns as
+// columns of their own, over the values of their key/value head.
+//
+// A unit is 16 columns that share a key row: `tpw` neighbouring tokens times the `grp` query heads of a key/value head.  Per
+// step of 32 keys (two tiles of 16) a wave forms S^T = K Q^T with v_mfma_f32_16x16x32_bf16; a lane then holds keys 4 q4 .. + 3 of
+// both tiles for its column, which is the B operand of O^T = V^T P^T when the values' A operand takes its 8 keys in the
+// same order.  Pages hold a multiple of 16 keys, so a tile's page and place are scalars and a lane adds its own fixed offset.
+//
+//   attend_wide_kernel<.., PARTS = true>   requests that bring one token: the keys go to `shares` workgroups, whose maxima, sums
+//       and results (32-bit) a second kernel joins: combine_mixed_kernel or combine_maps_kernel.
+//   PARTS = false   portions of prompts.  With mixed heads a workgroup holds all heads of its tokens, and mixes in LDS (32-bit
+//       matrix instructions), one key/value head's values at a time; else it holds a key/value head's one or two maps.
+//
+// Why it is a kernel of its own, and a short one: attention_composed_mfma.hip is 31 to 41 KB of straight code that a decoding wave
+// goes through once or twice (twice the waves a request and keys asked for a group ahead left its time as it was: it waits for
+// its instructions), and its places are looked up lane by lane; this one is 5 to 9 KB.  What bounds it now: for single tokens the
+// chain of two launches and of lengths -> table -> keys -> results; for portions the answers to a step's values.
+// Measured against that kernel, microseconds (mixed: 32 heads of 64 on 4 key/value heads; maps: 16 heads of two maps of 64 on 2,
+// values of 128):
+//     4 requests, one token behind   300 keys    mixed 22.0 -> 11.6    maps 18.4 ->  9.0
+//     4 requests, one token behind 1,000 keys    mixed 24.1 -> 12.0    maps 31.7 ->  9.5
+//   256 requests, one token behind 1,000 keys    mixed  130 ->   72    maps 50.4 -> 51.1 (5 TB/s of keys and values)
+//     a prompt of   333 tokens                   mixed  153 ->   26    maps 35.6 -> 13.0
+//     a prompt of 2,048 tokens                   mixed  821 ->  206    maps  284 ->   97
+// The weights are rounded to bfloat16 as the operand of the value product there as here, there after the mixing and here before
+// it.  Against 64 bits (100 to 3,000 keys, mixing of 0.3 to 3 times the identity's size): 1.8 to 2.3e-3 of the result's norm here,
+// 2.2 to 2.4e-3 there; two maps 2.2 to 2.5e-3 both.
+//
+// Masks as in attention_composed_mfma.hip: a column at position i sees j <= i with j >= its chunk's start and (i - j < window or
+// j < keep_first).
+#include "common.h"
+
+#define LOG2E 1.4426950408889634f
+#define NOTHING_YET (-1.0e30f)
+#define AW_SHARES 16  // most workgroups that share a request's keys
+#define AW_NO_KEY 0x40000000
+
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((ext_vector_type(8))) short s16x8;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+
+struct WideArgs {
+    bf16* out;
+    const bf16* q;
+    const bf16* k_pool;
+    const bf16* v_pool;
+    const int* block_tables;
+    const int* table_rows;
+    const int* cu_seqlens;
+    const int* context_lens;
+    const float* slopes;
+    const float* talk;
+    float* ws_o;      // [share][request][heads * maps][DT * 16]
+    float* ws_stats;  // [share][request][heads * maps][2]: maximum (units of log 2) and sum
+    int out_stride, q_stride, max_blocks;
+    int seq_begin, n_seqs, blocks_per_seq;
+    int heads, grp, maps, score_heads, heads_per_wg;
+    int dv, block_size, k_page, v_page;  // k_page, v_page: elements of a page
+    int window, keep_first, chunk;
+    int tok, tpw, shares;
+    unsigned bs_magic;  // ceil(2^32 / block_size)
+    float scale, lambda, eps, out_scale;
+    int head_norm, sink;
+};
+
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+__device__ __forceinline__ uint32_t low_half_mask(int keep) { return keep <= 0 ? 0u : keep == 1 ? 0xffffu : 0xffffffffu; }
+
+template <int TK, int DT, int U, bool PARTS>
+__global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const WideArgs a) {
+    extern __shared__ float lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
+    const int nwaves = blockDim.x / LLMS_WAVE;
+    const int col = lane % 16, q4 = lane / 16;
+    const int bi = blockIdx.x % a.n_seqs, b = a.seq_begin + bi, blk = a.blocks_per_seq - 1 - blockIdx.x / a.n_seqs;
+    const int row0 = a.cu_seqlens[b], count = a.cu_seqlens[b + 1] - row0, end = a.context_lens[b];
+    const int t0 = blk * a.tok;
+    if (t0 >= count || end <= 0) return;  // (the same for every thread of the workgroup)
+    const int ntok = count - t0 < a.tok ? count - t0 : a.tok;
+    const int pos_lo = end - count + t0, pos_hi = pos_lo + ntok - 1;
+    const int* table = a.block_tables + (size_t)(a.table_rows ? a.table_rows[b] : b) * a.max_blocks;
+    const int head = blockIdx.z * a.heads_per_wg + wave;
+    if (PARTS && head >= a.score_heads) return;
+    const int kvh = head / a.maps, map = head - kvh * a.maps;
+    const int share = blockIdx.y, bs = a.block_size;
+    constexpr int DK = 32 * TK, HALVES = (DT > 8 && !PARTS) ? 2 : 1;  // (16 tiles of values and their results fill a wave's registers)
+
+    // tiles of 16 keys: the kept first keys that the window has passed, then what the first token reaches to the last's own
+    const int lo_chunk = a.chunk > 0 ? pos_lo / a.chunk * a.chunk : 0;
+    const int lo_win = (a.window > 0 && pos_lo - a.window + 1 > 0) ? pos_lo - a.window + 1 : 0;
+    const int main_begin = (lo_chunk > lo_win ? lo_chunk : lo_win) / 16, main_end = pos_hi / 16 + 1;
+    const int sink_begin = lo_chunk / 16;
+    int sink_end = (a.keep_first + 15) / 16;
+    if (sink_end > main_begin) sink_end = main_begin;
+    if (a.window <= 0 || sink_end < sink_begin) sink_end = sink_begin;
+    const int n_sink = sink_end - sink_begin, n_tiles = n_sink + main_end - main_begin, n_steps = (n_tiles + 1) / 2;
+    auto tile_start = [&](int i) { return 16 * (i < n_sink ? sink_begin + i : main_begin + (i - n_sink)); };
+
+    bool valid[U];
+    int pos[U], pmin[U], pmax[U], chunk_lo[U];
+    bf16x8v qf[U][TK];
+    const int h = kvh * a.grp + col % a.grp;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int first = u * a.tpw, tl = first + col / a.grp;
+        valid[u] = col < a.tpw * a.grp && tl < ntok;
+        pos[u] = pos_lo + tl;
+        pmin[u] = pos_lo + first;
+        pmax[u] = pmin[u] + a.tpw - 1 < pos_hi ? pmin[u] + a.tpw - 1 : pos_hi;
+        chunk_lo[u] = a.chunk > 0 ? pos[u] / a.chunk * a.chunk : 0;
+        const bf16* qrow = a.q + (size_t)(row0 + t0 + tl) * a.q_stride + (size_t)(h * a.maps + map) * DK + 8 * q4;
+#pragma unroll
+        for (int t = 0; t < TK; ++t)
+            qf[u][t] = valid[u] ? *reinterpret_cast<const bf16x8v*>(qrow + 32 * t) : __builtin_bit_cast(bf16x8v, s16x8{0, 0, 0, 0, 0, 0, 0, 0});
+    }
+    const bool sloped = a.slopes != nullptr;
+    const float slope = sloped ? a.slopes[h] * LOG2E : 0.f;
+    const float scale2 = a.scale * LOG2E;
+
+    const bf16* k_head = a.k_pool + (size_t)head * bs * DK + col * DK + 8 * q4;
+    const bf16* v_head = a.v_pool + (size_t)(DT * 16 == a.dv ? kvh : 0) * a.dv * bs + col * bs + 4 * q4;
+    struct Place {
+        int page, in_page;
+    };
+    // a step's second tile may not exist: it reads the last one again, and its keys lie behind every position
+    auto place_of = [&](int i) {
+        const int j = tile_start(i < n_tiles ? i : n_tiles - 1), block = (int)__umulhi((unsigned)j, a.bs_magic);
+        const int page = table[block];
+        return Place{page < 0 ? 0 : page, j - block * bs};
+    };
+    auto ask_keys = [&](const Place at[2], bf16x8v kf[2][TK]) {
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int t = 0; t < TK; ++t)
+                kf[tt][t] = *reinterpret_cast<const bf16x8v*>(k_head + (size_t)at[tt].page * a.k_page + at[tt].in_page * DK + 32 * t);
+    };
+
+    f32x4 o[U][DT];
+    float run_m[U], run_l[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        run_m[u] = NOTHING_YET, run_l[u] = 0.f;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+
+    bf16x8v kf[2][TK];
+    Place at[2];
+    if (share < n_steps) {
+        at[0] = place_of(2 * share), at[1] = place_of(2 * share + 1);
+        ask_keys(at, kf);
+    }
+    for (int step = share; step < n_steps; step += a.shares) {
+        s16x4 vf[HALVES][2][DT / HALVES];
+        auto ask_values = [&](int half) {
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                const bf16* vt = v_head + (size_t)at[tt].page * a.v_page + at[tt].in_page + (size_t)half * (DT / HALVES) * 16 * bs;
+#pragma unroll
+                for (int d = 0; d < DT / HALVES; ++d) vf[half][tt][d] = *reinterpret_cast<const s16x4*>(vt + (size_t)16 * d * bs);
+            }
+        };
+        ask_values(0);
+        int j0[2];
+        j0[0] = tile_start(2 * step), j0[1] = 2 * step + 1 < n_tiles ? tile_start(2 * step + 1) : AW_NO_KEY;
+        bf16x8v pf[U];
+        float corr[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float sc[2][4], mx = -INFINITY;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < TK; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[tt][t], qf[u][t], acc, 0, 0, 0);
+                const int key0 = j0[tt] + 4 * q4;
+                // every column of the unit sees all 16 keys (the same answer in every lane)
+                const bool whole = j0[tt] + 15 <= pmin[u] && (a.chunk <= 0 || j0[tt] >= pmax[u] / a.chunk * a.chunk) &&
+                                   (a.window <= 0 || pmax[u] - j0[tt] < a.window);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sc[tt][r] = acc[r] * scale2;
+                if (sloped) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sc[tt][r] -= slope * ((float)(pos[u] - key0) - (float)r);
+                }
+                if (!whole) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int key = key0 + r;
+                        const bool seen = key <= pos[u] && key >= chunk_lo[u] && (a.window <= 0 || pos[u] - key < a.window || key < a.keep_first);
+                        sc[tt][r] = seen ? sc[tt][r] : -INFINITY;
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, sc[tt][r]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, LLMS_WAVE));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, LLMS_WAVE));
+            const float m_new = fmaxf(fmaxf(run_m[u], mx), NOTHING_YET);
+            corr[u] = fast_exp2(run_m[u] - m_new);
+            float p[2][4], sum = 0.f;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[tt][r] = fast_exp2(sc[tt][r] - m_new), sum += p[tt][r];
+            run_l[u] = run_l[u] * corr[u] + sum;
+            run_m[u] = m_new;
+            pf[u] = __builtin_bit_cast(bf16x8v, u32x4{pack_bf16x2(p[0][0], p[0][1]), pack_bf16x2(p[0][2], p[0][3]),
+                                                      pack_bf16x2(p[1][0], p[1][1]), pack_bf16x2(p[1][2], p[1][3])});
+        }
+        if (HALVES == 2) ask_values(1);
+        if (step + a.shares < n_steps) {  // the next step's keys, before this step's values are waited for
+            const int next = step + a.shares;
+            at[0] = place_of(2 * next), at[1] = place_of(2 * next + 1);
+            ask_keys(at, kf);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (__any(corr[u] != 1.f)) {
+#pragma unroll
+                for (int d = 0; d < DT; ++d) o[u][d] *= corr[u];
+            }
+        const bool tail = j0[0] + 15 >= end || j0[1] + 15 >= end;  // values behind the request's end may be anything, also NaN
+#pragma unroll
+        for (int half = 0; half < HALVES; ++half) {
+            if (tail) {
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt) {
+                    const int keep = end - (j0[tt] + 4 * q4);
+                    const uint32_t lo = low_half_mask(keep), hi = low_half_mask(keep - 2);
+#pragma unroll
+                    for (int d = 0; d < DT / HALVES; ++d) {
+                        u32x2 v = __builtin_bit_cast(u32x2, vf[half][tt][d]);
+                        v.x &= lo, v.y &= hi;
+                        vf[half][tt][d] = __builtin_bit_cast(s16x4, v);
+                    }
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < DT / HALVES; ++d) {
+                const bf16x8v v = __builtin_bit_cast(bf16x8v, __builtin_shufflevector(vf[half][0][d], vf[half][1][d], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    f32x4& to = o[u][half * (DT / HALVES) + d];
+                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf[u], to, 0, 0, 0);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        run_l[u] += __shfl_xor(run_l[u], 16, LLMS_WAVE);
+        run_l[u] += __shfl_xor(run_l[u], 32, LLMS_WAVE);
+    }
+
+    if constexpr (PARTS) {
+        if (!valid[0]) return;
+        const size_t at_col = ((size_t)share * a.n_seqs + bi) * (a.heads * a.maps) + h * a.maps + map;
+        if (q4 == 0) a.ws_stats[2 * at_col] = run_m[0], a.ws_stats[2 * at_col + 1] = run_l[0];
+        float* part = a.ws_o + at_col * (DT * 16) + 4 * q4;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(part + 16 * d) = o[0][d];
+    } else if (!a.talk) {
+        // the second map's waves leave their results in LDS, lane by lane, for those of the first with the same columns
+        float mul[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) mul[u] = 1.f / (a.sink ? run_l[u] + fast_exp2(-run_m[u]) : run_l[u]);
+        f32x4* other = reinterpret_cast<f32x4*>(lds) + lane;
+        if (a.maps == 2) {
+            if (map == 1) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int d = 0; d < DT; ++d) other[(u * DT + d) * LLMS_WAVE] = o[u][d] * (mul[u] * a.lambda);
+            }
+            __syncthreads();
+            if (map == 1) return;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float ss = 0.f;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                o[u][d] *= mul[u];
+                if (a.maps == 2) o[u][d] -= other[(u * DT + d) * LLMS_WAVE];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ss = fmaf(o[u][d][r], o[u][d][r], ss);
+            }
+            ss += __shfl_xor(ss, 16, LLMS_WAVE);
+            ss += __shfl_xor(ss, 32, LLMS_WAVE);
+            const float norm = a.head_norm ? a.out_scale / sqrtf(ss / (float)(DT * 16) + a.eps) : 1.f;
+            if (!valid[u]) continue;
+            bf16* orow = a.out + (size_t)(row0 + t0 + u * a.tpw + col / a.grp) * a.out_stride + (size_t)h * (DT * 16) + 4 * q4;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const f32x4 v = o[u][d] * norm;
+                *reinterpret_cast<u32x2*>(orow + 16 * d) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            }
+        }
+    } else {
+        // one key/value head's values at a time: [token][head g][dv + 16] in LDS (the pad puts 4 heads on different banks),
+        // then a job is a token's 16 dimensions of that key/value head's query heads, 4 heads g an instruction
+        const int H = a.heads, dv = a.dv, dvt = dv / 16, pad = dv + 16, G = H / a.grp;
+        float* talk_s = lds + (size_t)a.tok * H * pad;  // [g][h]
+        for (int i = threadIdx.x; i < H * H; i += blockDim.x) talk_s[(i % H) * H + i / H] = a.talk[i];
+        float inv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) inv[u] = 1.f / run_l[u];
+        for (int k = 0; k < G; ++k) {
+            if (k) __syncthreads();
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (valid[u]) {
+                    float* at_col = lds + ((size_t)(u * a.tpw + col / a.grp) * H + h) * pad + 4 * q4;
+#pragma unroll
+                    for (int d = 0; d < DT; ++d)  // (constant indexes of the results: the others are skipped)
+                        if (d / dvt == k) *reinterpret_cast<f32x4*>(at_col + 16 * (d - k * dvt)) = o[u][d] * inv[u];
+                }
+            __syncthreads();
+            for (int job = wave; job < ntok * dvt; job += nwaves) {
+                const int tl = job / dvt, d0 = 16 * (job - tl * dvt);
+                const bool mine = col < a.grp;
+                const int ho = k * a.grp + (mine ? col : 0);
+                const float* from = lds + (size_t)tl * H * pad + d0 + col;
+                f32x4 mixed = {0.f, 0.f, 0.f, 0.f};
+                for (int g0 = 0; g0 < H; g0 += 4) {
+                    const int g = g0 + q4;
+                    const float ug = g < H ? from[g * pad] : 0.f, tg = g < H ? talk_s[g * H + ho] : 0.f;
+                    mixed = __builtin_amdgcn_mfma_f32_16x16x4f32(ug, tg, mixed, 0, 0, 0);
+                }
+                if (mine) {
+                    *reinterpret_cast<u32x2*>(a.out + (size_t)(row0 + t0 + tl) * a.out_stride + (size_t)ho * dv + d0 + 4 * q4) =
+                        u32x2{pack_bf16x2(mixed[0], mixed[1]), pack_bf16x2(mixed[2], mixed[3])};
+                }
+            }
+        }
+    }
+}
+
+// A column's factors for its shares' results: exp2(m_s - max m) / sum, 0 for a share that saw no key (its results are not used).
+template <bool SINK>
+__device__ __forceinline__ void share_factors(const float* stats, size_t stride, int shares, float f[AW_SHARES]) {
+    float m[AW_SHARES], l[AW_SHARES], top = NOTHING_YET, total = 0.f;
+#pragma unroll
+    for (int s = 0; s < AW_SHARES; ++s) {
+        const float2 ml = *reinterpret_cast<const float2*>(stats + (s < shares ? s : shares - 1) * stride);
+        m[s] = ml.x, l[s] = s < shares ? ml.y : 0.f;
+    }
+#pragma unroll
+    for (int s = 0; s < AW_SHARES; ++s) top = fmaxf(top, l[s] > 0.f ? m[s] : NOTHING_YET);
+#pragma unroll
+    for (int s = 0; s < AW_SHARES; ++s) {
+        f[s] = l[s] > 0.f ? fast_exp2(m[s] - top) : 0.f;
+        total += f[s] * l[s];
+    }
+    if (SINK) total += fast_exp2(-top);
+    const float inv = 1.f / total;
+#pragma unroll
+    for (int s = 0; s < AW_SHARES; ++s) f[s] *= inv;
+}
+
+// Mixed heads: a workgroup takes one request, the query heads of one key/value head and 16 of its dimensions.
+__global__ __launch_bounds__(256) void combine_mixed_kernel(const WideArgs a, int width) {
+    extern __shared__ float lds[];  // [g][16 + 4] results, then this key/value head's rows of the mixing matrix [grp][H]
+    const int b = a.seq_begin + blockIdx.x, H = a.heads, grp = a.grp, k = blockIdx.y, d0 = k * a.dv + 16 * blockIdx.z;
+    const int row = a.cu_seqlens[b];
+    if (a.cu_seqlens[b + 1] <= row || a.context_lens[b] <= 0) return;
+    float* talk_s = lds + H * 20;
+    for (int i = threadIdx.x; i < grp * H; i += blockDim.x) talk_s[i] = a.talk[(size_t)k * grp * H + i];
+    for (int i = threadIdx.x; i < 4 * H; i += blockDim.x) {
+        const int g = i / 4, c = 4 * (i % 4);
+        const size_t col = (size_t)blockIdx.x * H + g, stride = (size_t)a.n_seqs * H;
+        f32x4 part[AW_SHARES];
+#pragma unroll
+        for (int s = 0; s < AW_SHARES; ++s)  // (a share that does not exist reads the last one and counts for nothing)
+            part[s] = *reinterpret_cast<const f32x4*>(a.ws_o + (col + (s < a.shares ? s : a.shares - 1) * stride) * width + d0 + c);
+        float f[AW_SHARES];
+        share_factors<false>(a.ws_stats + 2 * col, 2 * stride, a.shares, f);
+        f32x4 u = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < AW_SHARES; ++s) u += f[s] * part[s];
+        *reinterpret_cast<f32x4*>(lds + g * 20 + c) = u;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < grp * 16; i += blockDim.x) {
+        const int hh = i / 16, d = i % 16;
+        float sum = 0.f;
+        for (int g = 0; g < H; ++g) sum = fmaf(talk_s[hh * H + g], lds[g * 20 + d], sum);
+        a.out[(size_t)row * a.out_stride + (size_t)(k * grp + hh) * a.dv + 16 * blockIdx.z + d] = from_f32<bf16>(sum);
+    }
+}
+
+// One or two maps: a wave takes a request's head; a half of it is a map, a lane 4 dimensions (dv <= 128).
+template <bool SINK>
+__global__ __launch_bounds__(64) void combine_maps_kernel(const WideArgs a) {
+    const int b = a.seq_begin + blockIdx.x, h = blockIdx.y, lane = threadIdx.x, map = lane / 32, c = 4 * (lane % 32);
+    const int row = a.cu_seqlens[b];
+    if (a.cu_seqlens[b + 1] <= row || a.context_lens[b] <= 0) return;
+    const bool mine = map < a.maps && c < a.dv;
+    const int n = a.heads * a.maps;
+    const size_t col = (size_t)blockIdx.x * n + h * a.maps + (map < a.maps ? map : 0), stride = (size_t)a.n_seqs * n;
+    f32x4 part[AW_SHARES];
+#pragma unroll
+    for (int s = 0; s < AW_SHARES; ++s)
+        part[s] = *reinterpret_cast<const f32x4*>(a.ws_o + (col + (s < a.shares ? s : a.shares - 1) * stride) * a.dv + (mine ? c : 0));
+    float f[AW_SHARES];
+    share_factors<SINK>(a.ws_stats + 2 * col, 2 * stride, a.shares, f);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < AW_SHARES; ++s) o += f[s] * part[s];
+    if (!mine) o = f32x4{0.f, 0.f, 0.f, 0.f};
+    float ss = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float other = __shfl_xor(o[r], 32, LLMS_WAVE);
+        if (a.maps == 2) o[r] -= a.lambda * other;  // (the upper half's numbers are not used)
+        ss = fmaf(o[r], o[r], ss);
+    }
+#pragma unroll
+    for (int mask = 1; mask < 32; mask *= 2) ss += __shfl_xor(ss, mask, LLMS_WAVE);
+    const float norm = a.head_norm ? a.out_scale / sqrtf(ss / (float)a.dv + a.eps) : 1.f;
+    if (map == 0 && mine) {
+        *reinterpret_cast<u32x2*>(a.out + (size_t)row * a.out_stride + (size_t)h * a.dv + c) =
+            u32x2{pack_bf16x2(o[0] * norm, o[1] * norm), pack_bf16x2(o[2] * norm, o[3] * norm)};
+    }
+}
+
+template <int U, bool PARTS>
+static int launch(const WideArgs& a, int dk, int width, dim3 grid, int threads, size_t lds, hipStream_t stream) {
+#define AW_LAUNCH(TK, DT)                                                                                              \
+    do {                                                                                                               \
+        auto kernel = attend_wide_kernel<TK, DT, U, PARTS>;                                                            \
+        if (lds > 48 * 1024)                                                                                           \
+            LLMS_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+        kernel<<<grid, threads, lds, stream>>>(a);                                                                     \
+    } while (0)
+    if (width == 256) {
+        if constexpr (U == 1) {
+            if (dk == 64) AW_LAUNCH(2, 16);
+            else AW_LAUNCH(4, 16);
+        }
+    } else if (dk == 64 && width == 64) AW_LAUNCH(2, 4);
+    else if (dk == 64) AW_LAUNCH(2, 8);
+    else if (width == 64) AW_LAUNCH(4, 4);
+    else AW_LAUNCH(4, 8);
+#undef AW_LAUNCH
+    LLMS_LAUNCH_CHECK();
+}
+
+extern "C" {
+
+// `units` > 0: portions of prompts, workgroups of `units` (1, or 2 up to 128 columns of values) units of tokens.  units = 0:
+// requests that bring one token, their keys shared out to `shares` workgroups, with the workspaces ws_o and ws_stats.
+int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_stride, const void* k_pool, const void* v_pool,
+                              const int* block_tables, const int* table_rows, int max_blocks, const int* cu_seqlens,
+                              const int* context_lens, int seq_begin, int n_seqs, int max_new, int heads, int kv_heads, int maps,
+                              int dk, int dv, int block_size, int window, int keep_first, int chunk, float scale,
+                              const float* slopes, const float* talk, float lambda, int head_norm, float eps, float out_scale,
+                              int sink, int units, int shares, float* ws_o, float* ws_stats, hipStream_t stream) {
+    const int width = talk ? kv_heads * dv : dv;
+    LLMS_REQUIRE(n_seqs > 0 && max_new > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads / kv_heads <= 16,
+                 "attend_composed_wide: up to 16 query heads per key/value head");
+    LLMS_REQUIRE((maps == 1 || maps == 2) && !(talk && (maps != 1 || sink || head_norm)), "attend_composed_wide: one or two maps; mixed heads with one, no sink and no norm");
+    LLMS_REQUIRE((dk == 64 || dk == 128) && dv > 0 && dv % 16 == 0 && (width == 64 || width == 128 || width == 256) && (talk || dv <= 128),
+                 "attend_composed_wide: keys of 64 or 128, values of 64, 128 or 256 a column");
+    LLMS_REQUIRE(block_size > 0 && block_size % 16 == 0 && max_blocks > 0, "attend_composed_wide: pages of a multiple of 16 keys");
+    LLMS_REQUIRE(q_stride % 8 == 0 && out_stride % 4 == 0, "attend_composed_wide: query rows must be 16-byte aligned, result rows 8-byte");
+    LLMS_REQUIRE(window >= 0 && keep_first >= 0 && chunk >= 0, "attend_composed_wide: window, keep_first and chunk are >= 0");
+    LLMS_REQUIRE((size_t)kv_heads * maps * block_size * dk < (1u << 31) && (size_t)kv_heads * dv * block_size < (1u << 31),
+                 "attend_composed_wide: a page is too large");
+    WideArgs a;
+    a.out = (bf16*)out, a.q = (const bf16*)q, a.k_pool = (const bf16*)k_pool, a.v_pool = (const bf16*)v_pool;
+    a.block_tables = block_tables, a.table_rows = table_rows, a.cu_seqlens = cu_seqlens, a.context_lens = context_lens;
+    a.slopes = slopes, a.talk = talk, a.ws_o = ws_o, a.ws_stats = ws_stats;
+    a.out_stride = out_stride, a.q_stride = q_stride, a.max_blocks = max_blocks, a.seq_begin = seq_begin, a.n_seqs = n_seqs;
+    a.heads = heads, a.grp = heads / kv_heads, a.maps = maps, a.score_heads = kv_heads * maps;
+    a.dv = dv, a.block_size = block_size, a.k_page = kv_heads * maps * block_size * dk, a.v_page = kv_heads * dv * block_size;
+    a.window = window, a.keep_first = keep_first, a.chunk = chunk;
+    a.scale = scale, a.lambda = lambda, a.eps = eps, a.out_scale = out_scale, a.head_norm = head_norm, a.sink = sink;
+    a.tpw = 16 / a.grp;
+    a.bs_magic = (unsigned)((0x100000000ull + block_size - 1) / block_size);
+    if (units > 0) {
+        a.heads_per_wg = talk ? kv_heads : maps, a.shares = 1;
+        LLMS_REQUIRE((units == 1 || (units == 2 && width <= 128)) && a.heads_per_wg <= 8, "attend_composed_wide: up to 8 waves, of two units up to 128 columns of values");
+        a.tok = units * a.tpw, a.blocks_per_seq = (max_new + a.tok - 1) / a.tok;
+        const size_t lds = talk        ? ((size_t)a.tok * heads * (dv + 16) + (size_t)heads * heads) * sizeof(float)
+                           : maps == 2 ? (size_t)units * 16 * dv * sizeof(float)
+                                       : 0;
+        LLMS_REQUIRE(lds <= 160 * 1024, "attend_composed_wide: too many heads for the LDS");
+        const dim3 grid(n_seqs * a.blocks_per_seq, 1, talk ? 1 : kv_heads);
+        return units == 2 ? launch<2, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream)
+                          : launch<1, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream);
+    }
+    LLMS_REQUIRE(max_new == 1 && shares >= 1 && shares <= AW_SHARES && ws_o && ws_stats, "attend_composed_wide: one token a request, up to 16 shares, and their workspaces");
+    a.heads_per_wg = a.score_heads < 4 ? a.score_heads : 4;
+    a.tok = 1, a.blocks_per_seq = 1, a.shares = shares;
+    const int zs = (a.score_heads + a.heads_per_wg - 1) / a.heads_per_wg;
+    LLMS_REQUIRE(zs <= 65535 && heads <= 65535, "attend_composed_wide: too many heads");
+    const size_t mix_lds = ((size_t)heads * 20 + (size_t)a.grp * heads) * sizeof(float);
+    LLMS_REQUIRE(!talk || mix_lds <= 48 * 1024, "attend_composed_wide: too many heads for the LDS");
+    const int rc = launch<1, true>(a, dk, width, dim3(n_seqs, shares, zs), a.heads_per_wg * LLMS_WAVE, 0, stream);
+    if (rc != LLMS_OK) return rc;
+    if (talk) combine_mixed_kernel<<<dim3(n_seqs, kv_heads, dv / 16), 256, mix_lds, stream>>>(a, width);
+    else if (sink) combine_maps_kernel<true><<<dim3(n_seqs, heads), 64, 0, stream>>>(a);
+    else combine_maps_kernel<false><<<dim3(n_seqs, heads), 64, 0, stream>>>(a);
+    LLMS_LAUNCH_CHECK();
+}
+
+}  // extern "C"

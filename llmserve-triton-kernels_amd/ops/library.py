@@ -1365,23 +1365,9 @@ def attend_composed_mfma_tokens(heads: int, kv_heads: int, dk: int, dv: int, max
         c_int(heads), c_int(kv_heads), c_int(dk), c_int(dv), c_int(max_new)))
 
 
-def attend_composed_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
-                         block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
-                         seq_begin: int, n_seqs: int, max_new: int, *, heads: int, kv_heads: int, dk: int, dv: int,
-                         block_size: int, scale: float, maps: int = 1, window: int = 0, keep_first: int = 0,
-                         chunk: int = 0, slopes: torch.Tensor | None = None, talk: torch.Tensor | None = None,
-                         lam: float = 0.0, head_norm: bool = False, eps: float = 0.0, out_scale: float = 1.0,
-                         table_rows: torch.Tensor | None = None, shares: int = 1, dist_bias: torch.Tensor | None = None,
-                         gate: torch.Tensor | None = None, sink: bool = False, gate_heads: bool = False) -> torch.Tensor:
-    """`attend_composed` on the matrix cores (bfloat16) for requests [seq_begin, seq_begin + n_seqs) of a step: request
-    b owns rows cu_seqlens[b] .. cu_seqlens[b+1] of q and out, brings at most `max_new` tokens and is context_lens[b]
-    long after the step (0: padding, left alone).  Same arguments and arithmetic otherwise; the weights are rounded
-    to bfloat16 as the operand of the value product.  `shares` > 1 (where the heads' weights are mixed): the keys
-    of every block of tokens are shared out to that many workgroups in two launches (maxima and sums; weights and
-    values), their 32-bit parts added up by a third."""
-    dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, slopes, talk, table_rows, dist_bias, gate)
-    if not attend_composed_mfma_supported(q.dtype, heads, kv_heads, dk, dv, block_size, talk is not None):
-        raise ValueError("attend_composed_mfma does not take these sizes; see attend_composed_mfma_supported")
+def _composed_checks(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, seq_begin, n_seqs, slopes, talk, table_rows,
+                     heads, kv_heads, maps, dk, dv, block_size):
+    """What both matrix-core kernels of the composed attention ask of their tensors."""
     if q.dim() != 2 or q.stride(1) != 1 or q.shape[1] < heads * maps * dk or q.stride(0) % 4 or q.data_ptr() % 8:
         raise ValueError("q must be [N, >= heads*maps*dk] with unit inner stride and 8-byte aligned rows")
     _rows(out, "out", heads * dv)
@@ -1411,6 +1397,27 @@ def attend_composed_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
         _f32(slopes, "slopes", heads)
     if talk is not None:
         _f32(talk, "talk", heads * heads)
+
+
+def attend_composed_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                         block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
+                         seq_begin: int, n_seqs: int, max_new: int, *, heads: int, kv_heads: int, dk: int, dv: int,
+                         block_size: int, scale: float, maps: int = 1, window: int = 0, keep_first: int = 0,
+                         chunk: int = 0, slopes: torch.Tensor | None = None, talk: torch.Tensor | None = None,
+                         lam: float = 0.0, head_norm: bool = False, eps: float = 0.0, out_scale: float = 1.0,
+                         table_rows: torch.Tensor | None = None, shares: int = 1, dist_bias: torch.Tensor | None = None,
+                         gate: torch.Tensor | None = None, sink: bool = False, gate_heads: bool = False) -> torch.Tensor:
+    """`attend_composed` on the matrix cores (bfloat16) for requests [seq_begin, seq_begin + n_seqs) of a step: request
+    b owns rows cu_seqlens[b] .. cu_seqlens[b+1] of q and out, brings at most `max_new` tokens and is context_lens[b]
+    long after the step (0: padding, left alone).  Same arguments and arithmetic otherwise; the weights are rounded
+    to bfloat16 as the operand of the value product.  `shares` > 1 (where the heads' weights are mixed): the keys
+    of every block of tokens are shared out to that many workgroups in two launches (maxima and sums; weights and
+    values), their 32-bit parts added up by a third."""
+    dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, slopes, talk, table_rows, dist_bias, gate)
+    if not attend_composed_mfma_supported(q.dtype, heads, kv_heads, dk, dv, block_size, talk is not None):
+        raise ValueError("attend_composed_mfma does not take these sizes; see attend_composed_mfma_supported")
+    _composed_checks(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, seq_begin, n_seqs, slopes, talk, table_rows,
+                     heads, kv_heads, maps, dk, dv, block_size)
     if dist_bias is not None and (dist_bias.dtype != torch.float32 or dist_bias.dim() != 2 or dist_bias.shape[0] != heads
                                   or dist_bias.shape[1] < 1 or not dist_bias.is_contiguous()):
         raise ValueError("dist_bias must be a contiguous float32 [heads, reach + 1] tensor")
@@ -1438,6 +1445,66 @@ def attend_composed_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
         _ptr(gate), c_int(gate.stride(0) if gate is not None else 0), c_int(1 if gate_heads else 0), c_int(1 if sink else 0),
         _stream(dev)), "attend_composed_mfma")
     return out
+
+
+def attend_composed_wide_supported(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, heads: int, kv_heads: int, dk: int,
+                                   dv: int, block_size: int, talk: bool) -> bool:
+    """Whether `attend_composed_wide` takes this attention: bfloat16, keys of 64 or 128, pages of a multiple of 16 keys, aligned
+    rows; one token a request, or mixed heads; and 64, 128 or 256 columns of values for a score column: those of its key/value
+    head, with mixed heads those of all.  (With 512 a lane's results would need 128 registers, and the value products would be 8
+    of 9: the kernel that mixes weights has 1 in 3.)"""
+    width = kv_heads * dv if talk else dv
+    return (q.dtype == torch.bfloat16 and heads % kv_heads == 0 and heads // kv_heads <= 16 and dk in (64, 128) and dv % 16 == 0
+            and dv <= 128 and width in (64, 128, 256) and block_size % 16 == 0 and kv_heads <= 8 and heads <= 128
+            and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0 and k_pool.data_ptr() % 16 == 0 and v_pool.data_ptr() % 16 == 0)
+
+
+def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                         block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
+                         seq_begin: int, n_seqs: int, max_new: int, *, heads: int, kv_heads: int, dk: int, dv: int,
+                         block_size: int, scale: float, maps: int = 1, window: int = 0, keep_first: int = 0,
+                         chunk: int = 0, slopes: torch.Tensor | None = None, talk: torch.Tensor | None = None,
+                         lam: float = 0.0, head_norm: bool = False, eps: float = 0.0, out_scale: float = 1.0,
+                         table_rows: torch.Tensor | None = None, sink: bool = False, shares: int = 1) -> torch.Tensor:
+    """`attend_composed_mfma` for one token a request (`max_new` = 1; their keys shared out to `shares` workgroups), and for
+    portions of prompts with mixed heads, in one walk over the keys: a head's weights meet the values of all key/value heads
+    and the results are mixed, not the weights.  Same arguments and results; see attend_composed_wide_supported."""
+    dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, slopes, talk, table_rows)
+    if not attend_composed_wide_supported(q, k_pool, v_pool, heads, kv_heads, dk, dv, block_size, talk is not None):
+        raise ValueError("attend_composed_wide does not take these sizes; see attend_composed_wide_supported")
+    if talk is not None and (sink or head_norm):
+        raise ValueError("mixed heads have no sink and no norm of their results here")
+    _composed_checks(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, seq_begin, n_seqs, slopes, talk, table_rows,
+                     heads, kv_heads, maps, dk, dv, block_size)
+    if n_seqs == 0 or max_new <= 0 or q.shape[0] == 0:
+        return out
+    ws_o = ws_stats = None
+    units = 0
+    if max_new == 1:
+        shares = max(1, min(int(shares), 16))
+        columns = shares * n_seqs * heads * maps
+        ws_o = torch.empty(columns * (kv_heads * dv if talk is not None else dv), dtype=torch.float32, device=dev)
+        ws_stats = torch.empty(2 * columns, dtype=torch.float32, device=dev)
+    else:
+        units = wide_prompt_units(heads, kv_heads, dv, talk is not None, n_seqs, max_new, compute_units(dev))
+    _check(load("attention_composed_wide").llms_attend_composed_wide(
+        _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
+        _ptr(table_rows), c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), c_int(seq_begin),
+        c_int(n_seqs), c_int(max_new), c_int(heads), c_int(kv_heads), c_int(maps), c_int(dk), c_int(dv),
+        c_int(block_size), c_int(window), c_int(keep_first), c_int(chunk), c_float(scale), _ptr(slopes), _ptr(talk),
+        c_float(lam), c_int(1 if head_norm else 0), c_float(eps), c_float(out_scale), c_int(1 if sink else 0),
+        c_int(units), c_int(shares), _ptr(ws_o), _ptr(ws_stats), _stream(dev)), "attend_composed_wide")
+    return out
+
+
+def wide_prompt_units(heads: int, kv_heads: int, dv: int, talk: bool, n_seqs: int, max_new: int, cus: int) -> int:
+    """Units of 16 columns a wave of `attend_composed_wide` takes over portions of prompts.  Two share every key and value a wave
+    reads, one gives twice the workgroups (16 heads of two maps over 64, values of 128: 2,000 tokens of 4 requests in 440
+    workgroups of two 56 microseconds, in 890 of one 105; 100 tokens in 112 or 224 of them 48 and 39).  The results of two
+    units of 256 columns do not fit a wave's registers."""
+    tpw, width = 16 // (heads // kv_heads), kv_heads * dv if talk else dv
+    workgroups = n_seqs * -(-max_new // (2 * tpw)) * (1 if talk else kv_heads)
+    return 2 if width <= 128 and workgroups >= cus else 1
 
 
 # ------------------------------------------------------------------------------ sampling

@@ -224,7 +224,7 @@ class ComposedAttention(Mixer):
             return ("attention_composed",)
         if self.plain_but_for_head_gate and self.head_dim % 16 == 0 and self.head_dim <= 256:
             return ("attention_composed", "attention_gated" if self.gate_heads else "attention_mfma")
-        names = ("attention_composed", "attention_composed_mfma")
+        names = ("attention_composed", "attention_composed_mfma", "attention_composed_wide")
         return names + ("attention_biased",) if self.plain_but_for_bias_and_gate else names
 
     @property
@@ -390,9 +390,19 @@ class ComposedAttention(Mixer):
         args = (out, q, paged.k_pool, paged.v_pool, view.block_tables, batch.cu_seqlens, batch.context_lens)
         common.update(dist_bias=self.dist_bias, gate=gate, sink=self.sink, gate_heads=self.gate_heads)
         n_dec = batch.num_decode
+        # one walk over the keys by a short kernel, and the results mixed, wherever it takes the sizes: it was the faster one from 1
+        # request to 256, 64 keys to 4,000 and 16 tokens to 2,048 (12 against 24 microseconds for 4 decoding requests behind
+        # 1,000 keys, 26 against 153 for a prompt of 333)
+        wide = self.dist_bias is None and gate is None and not (self.talking and self.head_norm_eps is not None) and \
+            ops.attend_composed_wide_supported(q, paged.k_pool, paged.v_pool, self.num_heads, self.num_kv_heads, self.head_dim,
+                                               self.value_dim, paged.block_size, self.talking)
+        plain = {k: v for k, v in common.items() if k not in ("dist_bias", "gate", "gate_heads")}
         if n_dec:
-            ops.attend_composed_mfma(*args, 0, n_dec, 1, shares=self.decode_shares(n_dec, batch.max_decode_context,
-                                                                                  ops.compute_units(q.device)), **common)
+            shares = self.decode_shares(n_dec, batch.max_decode_context, ops.compute_units(q.device))
+            if wide:
+                ops.attend_composed_wide(*args, 0, n_dec, 1, shares=shares, **plain)
+            else:
+                ops.attend_composed_mfma(*args, 0, n_dec, 1, shares=shares if self.talking else 1, **common)
         if n_dec < batch.num_seqs and self.plain_but_for_bias_and_gate and not self.gate_heads and \
                 ops.attention_prompt_biased_supported(q.dtype, self.head_dim, self.value_dim, paged.block_size) and \
                 (gate is None or (gate.data_ptr() % 16 == 0 and gate.stride(0) % 4 == 0)) and q.stride(0) % 8 == 0:
@@ -403,7 +413,9 @@ class ComposedAttention(Mixer):
                                         head_dim=self.head_dim, block_size=paged.block_size, scale=self.scale,
                                         dist_bias=self.dist_bias, gate=gate, table_rows=batch.state_slots)
             return
-        if n_dec < batch.num_seqs:
+        if n_dec < batch.num_seqs and batch.max_count > 1 and wide:
+            ops.attend_composed_wide(*args, n_dec, batch.num_seqs - n_dec, batch.max_count, **plain)
+        elif n_dec < batch.num_seqs:
             shares = self.prompt_shares(batch.num_seqs - n_dec, batch.max_count, batch.max_context,
                                         ops.compute_units(q.device))
             ops.attend_composed_mfma(*args, n_dec, batch.num_seqs - n_dec, batch.max_count, shares=shares, **common)
@@ -437,13 +449,12 @@ class ComposedAttention(Mixer):
         return max(1, min(4, cus // max(blocks, 1), int(reach) // 256))
 
     def decode_shares(self, n_requests: int, max_context: int, cus: int = 256) -> int:
-        """Workgroups that share the keys of one decoding request when the heads' weights are mixed.  Such a request is
-        one workgroup (all its heads must meet for the mixing), which alone keeps one compute unit busy for as long
-        as its keys last; while the batch leaves compute units idle its keys go to several, down to one group of 64
-        keys a share, at the price of two more launches (measured at batch 8 behind 520 keys, 32 heads of 64: 71
-        microseconds in one workgroup of 16 waves, 43 in 4 shares, 26 in 12)."""
-        if not self.talking:
-            return 1
+        """Workgroups that share the keys of one decoding request.  Such a request (with mixed heads, and a key/value head of it
+        without) is one workgroup, which alone keeps one compute unit busy for as long as its keys last; while the batch
+        leaves compute units idle its keys go to several, down to one group of 64 keys a share, at the price of one more
+        launch, or two more where the heads' weights are mixed and not their results.  Measured, microseconds: 4 requests
+        behind 1,000 keys, 32 heads of 64 mixed: 49 in one share, 19 in 4, 12 in 16; 64 requests 53, 24, 33; 256 requests
+        72, 84, 136."""
         reach = min(x for x in (max_context, self.chunk, None if self.window is None else self.window + self.keep_first)
                     if x is not None)
         return max(1, min(16, cus // max(n_requests, 1), -(-int(reach) // 64)))

@@ -1,0 +1,117 @@
+"""The composed attention whose columns meet the values before heads are mixed, against the plain implementation in float64
+(tests/plain_dibepel.py), at the edges of its steps of 32 keys, its shares and its blocks of tokens.
+
+Tolerance as for the kernel that mixes weights (test_dibepel_gpu.close): operands and results rounded to bfloat16 once."""
+import pytest
+import torch
+
+import plain_dibepel as pd
+from test_dibepel_gpu import DEV, F64, attend_mfma, close, rnd, rounded
+
+pytestmark = pytest.mark.gpu
+
+
+# (context, first new row): one token at the edges of tiles, steps and shares; then portions of prompts
+REQUESTS = [(1, 0), (16, 15), (17, 16), (33, 32), (200, 199), (90, 0), (58, 33), (40, 38), (131, 64)]
+
+
+def run(seqs, bs, shares=1, **kw):
+    from llmserve.ops import library as ops
+
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(ops, "attend_composed_mfma", ops.attend_composed_wide)
+        return attend_mfma(seqs, bs, shares=shares, **kw)
+
+
+TALK = [  # heads, kv_heads, dk, dv, chunk, block size
+    (32, 4, 64, 64, 128, 16),
+    (4, 2, 64, 32, 20, 16),
+    (3, 1, 128, 128, None, 32),  # 5 tokens a unit, a padded column, heads not a multiple of 4
+    (16, 1, 64, 64, 48, 16),  # a unit is one token
+    (8, 8, 128, 32, None, 48),  # pages that are no power of two
+    (12, 2, 64, 128, 64, 16),
+]
+
+
+@pytest.mark.parametrize("heads,kv,dk,dv,chunk,bs", TALK)
+def test_mixed_heads(heads, kv, dk, dv, chunk, bs, monkeypatch):
+    from llmserve.ops import library as ops
+
+    dt = torch.bfloat16
+    talk = torch.eye(heads, dtype=F64) + rnd(heads, heads, seed=33, scale=0.3 / heads ** 0.5)
+    slopes = pd.distance_slopes(heads)
+    seqs, refs = [], []
+    for i, (t, first) in enumerate(REQUESTS):
+        q, k, v = (rounded(x, dt) for x in (rnd(t, heads, dk, seed=60 + i), rnd(t, kv, dk, seed=70 + i), rnd(t, kv, dv, seed=80 + i)))
+        ref = pd.talking_heads(q, k, v, pd.visible_chunk(t, chunk), 0.1, slopes, talk)
+        refs.append(ref.reshape(t, -1)[first:])
+        seqs.append((q, k, v, first, t - first))
+    for shares, units in ((1, 1), (3, 2 if kv * dv <= 128 else 1), (16, 1)):
+        monkeypatch.setattr(ops, "wide_prompt_units", lambda *a: units)
+        got = run(seqs, bs, shares=shares, heads=heads, kv_heads=kv, chunk=chunk or 0, scale=0.1, slopes=slopes.float().to(DEV),
+                  talk=talk.float().to(DEV))
+        for i, (g, r) in enumerate(zip(got, refs)):
+            close(g, r, dt, f"request {i}, {shares} shares, {units} units")
+
+
+MAPS = [  # heads, kv_heads, maps, dk, dv, window, keep_first, block size
+    (16, 2, 2, 64, 128, 33, 20, 16),
+    (3, 1, 2, 128, 64, 48, 0, 16),
+    (4, 4, 2, 64, 64, None, 0, 32),
+    (10, 5, 2, 64, 128, 100, 16, 16),  # ten score heads: three workgroups of up to four
+]
+
+
+@pytest.mark.parametrize("heads,kv,maps,dk,dv,window,keep,bs", MAPS)
+def test_two_maps(heads, kv, maps, dk, dv, window, keep, bs, monkeypatch):
+    from llmserve.ops import library as ops
+
+    dt = torch.bfloat16
+    lam, diff, eps, scale = 0.83, 0.3, 1e-5, 0.1
+    seqs, refs = [], []
+    for i, (t, first) in enumerate(REQUESTS):
+        q, k, v = (rounded(x, dt) for x in (rnd(t, heads, 2, dk, seed=60 + i), rnd(t, kv, 2, dk, seed=70 + i), rnd(t, kv, dv, seed=80 + i)))
+        ref = pd.differential_heads(q, k, v, pd.visible_window(t, window, keep), scale, lam, diff, eps)
+        refs.append(ref.reshape(t, -1)[first:])
+        seqs.append((q.reshape(t, heads * 2, dk), k.reshape(t, kv * 2, dk), v, first, t - first))
+    for shares, units in ((1, 1), (2, 2), (16, 1)):
+        monkeypatch.setattr(ops, "wide_prompt_units", lambda *a: units)
+        got = run(seqs, bs, shares=shares, heads=heads, kv_heads=kv, maps=2, window=window or 0, keep_first=keep, scale=scale, lam=lam,
+                  head_norm=True, eps=eps, out_scale=1 - diff)
+        for i, (g, r) in enumerate(zip(got, refs)):
+            close(g, r, dt, f"request {i}, {shares} shares, {units} units")
+
+
+@pytest.mark.parametrize("sink", [False, True])
+def test_one_map_with_a_sink_as_the_other_kernel(sink):
+    """One map without a mixture: the same results as the kernel that takes any size, in bfloat16 (two roundings apart)."""
+    heads, kv, dk, dv, bs = 8, 2, 64, 64, 16
+    seqs = []
+    for i, (t, first) in enumerate(REQUESTS):
+        q, k, v = (rounded(x, torch.bfloat16) for x in (rnd(t, heads, dk, seed=1 + i), rnd(t, kv, dk, seed=20 + i), rnd(t, kv, dv, seed=40 + i)))
+        seqs.append((q, k, v, first, t - first))
+    kw = dict(heads=heads, kv_heads=kv, scale=0.1, chunk=64, slopes=pd.distance_slopes(heads).float().to(DEV), sink=sink)
+    for i, (g, r) in enumerate(zip(run(seqs, bs, shares=4, **kw), attend_mfma(seqs, bs, **kw))):
+        close(g, r.double().cpu(), torch.bfloat16, f"request {i}")
+
+
+def test_values_behind_the_end_and_pages_of_other_requests_are_not_seen():
+    """NaN in every place of the pools that the request does not own stays out of its result."""
+    from llmserve.ops import library as ops
+
+    heads, kv, d, bs, t = 8, 2, 64, 16, 37
+    g = torch.Generator().manual_seed(3)
+    k_pool = torch.full((6, kv, bs, d), float("nan"), dtype=torch.bfloat16)
+    v_pool = torch.full((6, kv, d, bs), float("nan"), dtype=torch.bfloat16)
+    for j in range(t):
+        k_pool[j // bs, :, j % bs] = torch.randn(kv, d, generator=g).bfloat16()
+        v_pool[j // bs, :, :, j % bs] = torch.randn(kv, d, generator=g).bfloat16()
+    talk = (torch.eye(heads) + 0.1 * torch.randn(heads, heads, generator=g)).to(DEV)
+    table = torch.tensor([[0, 1, 2, 5]], dtype=torch.int32, device=DEV)
+    for new in (1, 7):
+        q = torch.randn(new, heads * d, generator=g).bfloat16().to(DEV)
+        out = torch.empty(new, heads * d, dtype=torch.bfloat16, device=DEV)
+        i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+        ops.attend_composed_wide(out, q, k_pool.to(DEV), v_pool.to(DEV), table, i32(0, new), i32(t), 0, 1, new, heads=heads, kv_heads=kv,
+                                 dk=d, dv=d, block_size=bs, scale=0.1, talk=talk, shares=2)
+        assert torch.isfinite(out.float()).all()
