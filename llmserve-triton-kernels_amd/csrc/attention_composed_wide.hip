@@ -25,10 +25,10 @@
 // Measured against that kernel, microseconds (mixed: 32 heads of 64 on 4 key/value heads; maps: 16 heads of two maps of 64 on 2,
 // values of 128):
 //     4 requests, one token behind   300 keys    mixed 22.0 -> 11.6    maps 18.4 ->  9.0
-//     4 requests, one token behind 1,000 keys    mixed 24.1 -> 12.0    maps 31.7 ->  9.5
+//     4 requests, one token behind 1,000 keys    mixed 24.1 -> 12.3    maps 31.7 ->  9.8
 //   256 requests, one token behind 1,000 keys    mixed  130 ->   72    maps 50.4 -> 51.1 (5 TB/s of keys and values)
-//     a prompt of   333 tokens                   mixed  153 ->   26    maps 35.6 -> 13.0
-//     a prompt of 2,048 tokens                   mixed  821 ->  206    maps  284 ->   97
+//     a prompt of   333 tokens                   mixed  153 ->   26    maps 35.7 -> 13.5
+//     a prompt of 2,048 tokens                   mixed  821 ->  154    maps  284 ->   99
 // The weights are rounded to bfloat16 as the operand of the value product there as here, there after the mixing and here before
 // it.  Against 64 bits (100 to 3,000 keys, mixing of 0.3 to 3 times the identity's size): 1.8 to 2.3e-3 of the result's norm here,
 // 2.2 to 2.4e-3 there; two maps 2.2 to 2.5e-3 both.
@@ -77,7 +77,7 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 
 __device__ __forceinline__ uint32_t low_half_mask(int keep) { return keep <= 0 ? 0u : keep == 1 ? 0xffffu : 0xffffffffu; }
 
-template <int TK, int DT, int U, bool PARTS>
+template <int TK, int DT, int U, bool PARTS, bool SHARED>
 __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const WideArgs a) {
     extern __shared__ float lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
@@ -89,12 +89,15 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
     if (t0 >= count || end <= 0) return;  // (the same for every thread of the workgroup)
     const int ntok = count - t0 < a.tok ? count - t0 : a.tok;
     const int pos_lo = end - count + t0, pos_hi = pos_lo + ntok - 1;
-    const int* table = a.block_tables + (size_t)(a.table_rows ? a.table_rows[b] : b) * a.max_blocks;
+    // (the constant address space: a page's number stays a scalar load also behind a barrier, where the compiler would take it for
+    // memory that may have changed, load it as a vector and wait for every load in flight before it)
+    const auto table = (const __attribute__((address_space(4))) int*)(uintptr_t)(
+        a.block_tables + (size_t)(a.table_rows ? a.table_rows[b] : b) * a.max_blocks);
     const int head = blockIdx.z * a.heads_per_wg + wave;
     if (PARTS && head >= a.score_heads) return;
     const int kvh = head / a.maps, map = head - kvh * a.maps;
     const int share = blockIdx.y, bs = a.block_size;
-    constexpr int DK = 32 * TK, HALVES = (DT > 8 && !PARTS) ? 2 : 1;  // (16 tiles of values and their results fill a wave's registers)
+    constexpr int DK = 32 * TK, HALVES = (DT > 8 && !PARTS && !SHARED) ? 2 : 1;  // (16 tiles of values and their results fill a wave's registers)
 
     // tiles of 16 keys: the kept first keys that the window has passed, then what the first token reaches to the last's own
     const int lo_chunk = a.chunk > 0 ? pos_lo / a.chunk * a.chunk : 0;
@@ -156,13 +159,54 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         for (int d = 0; d < DT; ++d) o[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    bf16x8v kf[2][TK];
-    Place at[2];
+    // SHARED: a step's values go through LDS (2,048 tokens of 32 heads on 4: 201 -> 154 microseconds), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
+    // (one per key/value head, at least 4) all read all of them.  A chunk is 32 dimensions of a tile, 16 bytes a lane;
+    // the two halves of dimensions 8 to 15 of every 16 change places, so that 32 lanes read 64 banks.
+    constexpr int CHUNKS = SHARED ? DT / 4 : 1;
+    uint16_t* v_lds = reinterpret_cast<uint16_t*>(lds);
+    u32x4 staged[CHUNKS];
+    int staged_keep[CHUNKS];  // keys of a lane's 8 that lie before the request's end
+    auto ask_chunks = [&](const Place at[2], int step) {
+#pragma unroll
+        for (int i = 0; i < CHUNKS; ++i) {
+            const int own = wave + i * nwaves, c = own < DT ? own : DT - 1, tt = c / (DT / 2), dim = 32 * (c - tt * (DT / 2)) + lane / 2;
+            const Place& p = tt ? at[1] : at[0];
+            staged[i] = *reinterpret_cast<const u32x4*>(a.v_pool + (size_t)p.page * a.v_page + (size_t)dim * bs + p.in_page + 8 * (lane % 2));
+            staged_keep[i] = (2 * step + tt < n_tiles ? end - tile_start(2 * step + tt) : 0) - 8 * (lane % 2);
+        }
+    };
+    auto store_chunks = [&](int turn) {
+#pragma unroll
+        for (int i = 0; i < CHUNKS; ++i) {
+            const int c = wave + i * nwaves;
+            if (c >= DT) continue;
+            u32x4 v = staged[i];
+            if (__any(staged_keep[i] < 8)) {  // values behind the request's end may be anything, also NaN
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] &= low_half_mask(staged_keep[i] - 2 * e);
+            }
+            *reinterpret_cast<u32x4*>(v_lds + turn * (DT * 512) + c * 512 + lane / 2 * 16 + 8 * ((lane ^ (lane >> 4)) & 1)) = v;
+        }
+    };
+
+    // A step asks for the next step's keys (and values, where they are shared) before anything else; the places of the step after
+    // that are looked up at the same time, so that no step waits for a page's number.
+    bf16x8v kf[2][TK], next_kf[2][TK];
+    Place at[2], next_at[2];
     if (share < n_steps) {
         at[0] = place_of(2 * share), at[1] = place_of(2 * share + 1);
+        next_at[0] = place_of(2 * (share + a.shares)), next_at[1] = place_of(2 * (share + a.shares) + 1);
+        if constexpr (SHARED) ask_chunks(at, share);
         ask_keys(at, kf);
+        if constexpr (SHARED) store_chunks(0);
     }
+    int turn = 0;
     for (int step = share; step < n_steps; step += a.shares) {
+        const int next = step + a.shares;
+        if constexpr (SHARED) {
+            __syncthreads();  // this step's values are in LDS, and the turn before has been read
+            if (next < n_steps) ask_chunks(next_at, next);
+        }
         s16x4 vf[HALVES][2][DT / HALVES];
         auto ask_values = [&](int half) {
 #pragma unroll
@@ -172,7 +216,16 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
                 for (int d = 0; d < DT / HALVES; ++d) vf[half][tt][d] = *reinterpret_cast<const s16x4*>(vt + (size_t)16 * d * bs);
             }
         };
-        ask_values(0);
+        if constexpr (!SHARED) ask_values(0);
+        if (next < n_steps) ask_keys(next_at, next_kf);
+        if constexpr (SHARED) {  // (all of them, asked for before the scores: their way through LDS passes beside the softmax)
+            const uint16_t* from = v_lds + turn * (DT * 512) + col * 16 + 4 * (q4 ^ (2 * (col / 8)));
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+                vf[0][0][d] = *reinterpret_cast<const s16x4*>(from + 256 * d), vf[0][1][d] = *reinterpret_cast<const s16x4*>(from + 256 * (DT + d));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const Place after_at[2] = {place_of(2 * (next + a.shares)), place_of(2 * (next + a.shares) + 1)};
         int j0[2];
         j0[0] = tile_start(2 * step), j0[1] = 2 * step + 1 < n_tiles ? tile_start(2 * step + 1) : AW_NO_KEY;
         bf16x8v pf[U];
@@ -221,11 +274,6 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
                                                       pack_bf16x2(p[1][0], p[1][1]), pack_bf16x2(p[1][2], p[1][3])});
         }
         if (HALVES == 2) ask_values(1);
-        if (step + a.shares < n_steps) {  // the next step's keys, before this step's values are waited for
-            const int next = step + a.shares;
-            at[0] = place_of(2 * next), at[1] = place_of(2 * next + 1);
-            ask_keys(at, kf);
-        }
 #pragma unroll
         for (int u = 0; u < U; ++u)
             if (__any(corr[u] != 1.f)) {
@@ -235,7 +283,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         const bool tail = j0[0] + 15 >= end || j0[1] + 15 >= end;  // values behind the request's end may be anything, also NaN
 #pragma unroll
         for (int half = 0; half < HALVES; ++half) {
-            if (tail) {
+            if (!SHARED && tail) {
 #pragma unroll
                 for (int tt = 0; tt < 2; ++tt) {
                     const int keep = end - (j0[tt] + 4 * q4);
@@ -257,6 +305,16 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
                     to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf[u], to, 0, 0, 0);
                 }
             }
+        }
+        if constexpr (SHARED) {
+            turn ^= 1;
+            if (next < n_steps) store_chunks(turn);
+        }
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            at[tt] = next_at[tt], next_at[tt] = after_at[tt];
+#pragma unroll
+            for (int t = 0; t < TK; ++t) kf[tt][t] = next_kf[tt][t];
         }
     }
 #pragma unroll
@@ -314,12 +372,13 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         // then a job is a token's 16 dimensions of that key/value head's query heads, 4 heads g an instruction
         const int H = a.heads, dv = a.dv, dvt = dv / 16, pad = dv + 16, G = H / a.grp;
         float* talk_s = lds + (size_t)a.tok * H * pad;  // [g][h]
+        if (SHARED) __syncthreads();  // (the values' place is free)
         for (int i = threadIdx.x; i < H * H; i += blockDim.x) talk_s[(i % H) * H + i / H] = a.talk[i];
         float inv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) inv[u] = 1.f / run_l[u];
         for (int k = 0; k < G; ++k) {
-            if (k) __syncthreads();
+            if (SHARED || k) __syncthreads();
 #pragma unroll
             for (int u = 0; u < U; ++u)
                 if (valid[u]) {
@@ -441,7 +500,7 @@ template <int U, bool PARTS>
 static int launch(const WideArgs& a, int dk, int width, dim3 grid, int threads, size_t lds, hipStream_t stream) {
 #define AW_LAUNCH(TK, DT)                                                                                              \
     do {                                                                                                               \
-        auto kernel = attend_wide_kernel<TK, DT, U, PARTS>;                                                            \
+        auto kernel = attend_wide_kernel<TK, DT, U, PARTS, false>;                                                            \
         if (lds > 48 * 1024)                                                                                           \
             LLMS_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
         kernel<<<grid, threads, lds, stream>>>(a);                                                                     \
@@ -468,7 +527,7 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
                               const int* context_lens, int seq_begin, int n_seqs, int max_new, int heads, int kv_heads, int maps,
                               int dk, int dv, int block_size, int window, int keep_first, int chunk, float scale,
                               const float* slopes, const float* talk, float lambda, int head_norm, float eps, float out_scale,
-                              int sink, int units, int shares, float* ws_o, float* ws_stats, hipStream_t stream) {
+                              int sink, int units, int shared, int shares, float* ws_o, float* ws_stats, hipStream_t stream) {
     const int width = talk ? kv_heads * dv : dv;
     LLMS_REQUIRE(n_seqs > 0 && max_new > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads / kv_heads <= 16,
                  "attend_composed_wide: up to 16 query heads per key/value head");
@@ -500,6 +559,15 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
                                        : 0;
         LLMS_REQUIRE(lds <= 160 * 1024, "attend_composed_wide: too many heads for the LDS");
         const dim3 grid(n_seqs * a.blocks_per_seq, 1, talk ? 1 : kv_heads);
+        if (shared) {
+            LLMS_REQUIRE(talk && units == 1 && kv_heads >= 4 && dk == 64 && width == 256, "attend_composed_wide: shared values with 4 to 8 mixed key/value heads, keys of 64 and 256 columns of values");
+            const size_t turns = 2 * (size_t)width * 64, all = lds > turns ? lds : turns;
+            auto kernel = attend_wide_kernel<2, 16, 1, false, true>;
+            if (all > 48 * 1024)
+                LLMS_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)all));
+            kernel<<<grid, kv_heads * LLMS_WAVE, all, stream>>>(a);
+            LLMS_LAUNCH_CHECK();
+        }
         return units == 2 ? launch<2, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream)
                           : launch<1, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream);
     }

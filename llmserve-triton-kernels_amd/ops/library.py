@@ -1479,7 +1479,7 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
     if n_seqs == 0 or max_new <= 0 or q.shape[0] == 0:
         return out
     ws_o = ws_stats = None
-    units = 0
+    units = shared = 0
     if max_new == 1:
         shares = max(1, min(int(shares), 16))
         columns = shares * n_seqs * heads * maps
@@ -1487,13 +1487,14 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
         ws_stats = torch.empty(2 * columns, dtype=torch.float32, device=dev)
     else:
         units = wide_prompt_units(heads, kv_heads, dv, talk is not None, n_seqs, max_new, compute_units(dev))
+        shared = wide_prompt_shared(heads, kv_heads, dk, dv, talk is not None, n_seqs, max_new, compute_units(dev))
     _check(load("attention_composed_wide").llms_attend_composed_wide(
         _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
         _ptr(table_rows), c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), c_int(seq_begin),
         c_int(n_seqs), c_int(max_new), c_int(heads), c_int(kv_heads), c_int(maps), c_int(dk), c_int(dv),
         c_int(block_size), c_int(window), c_int(keep_first), c_int(chunk), c_float(scale), _ptr(slopes), _ptr(talk),
         c_float(lam), c_int(1 if head_norm else 0), c_float(eps), c_float(out_scale), c_int(1 if sink else 0),
-        c_int(units), c_int(shares), _ptr(ws_o), _ptr(ws_stats), _stream(dev)), "attend_composed_wide")
+        c_int(units), c_int(1 if shared else 0), c_int(shares), _ptr(ws_o), _ptr(ws_stats), _stream(dev)), "attend_composed_wide")
     return out
 
 
@@ -1505,6 +1506,16 @@ def wide_prompt_units(heads: int, kv_heads: int, dv: int, talk: bool, n_seqs: in
     tpw, width = 16 // (heads // kv_heads), kv_heads * dv if talk else dv
     workgroups = n_seqs * -(-max_new // (2 * tpw)) * (1 if talk else kv_heads)
     return 2 if width <= 128 and workgroups >= cus else 1
+
+
+def wide_prompt_shared(heads: int, kv_heads: int, dk: int, dv: int, talk: bool, n_seqs: int, max_new: int, cus: int) -> bool:
+    """Whether the waves of a workgroup of `attend_composed_wide` share the values of a step through LDS (256 columns of values, all
+    read by at least 4 waves).  Where a SIMD has two waves or more, reading them once a workgroup counts for more than the
+    barrier a step and the way through LDS (microseconds, each wave for itself -> shared, 32 heads of 64 on 4: 1,100 tokens 84 -> 71,
+    2,048 tokens 201 -> 154; 8 heads on 8 of 32: 333 tokens 45 -> 41); a single wave a SIMD waits for each step's barrier (333
+    tokens 25.9 -> 29.2, 512 behind 488 others 53 -> 61)."""
+    workgroups = n_seqs * -(-max_new // (16 // (heads // kv_heads)))
+    return talk and dk == 64 and kv_heads * dv == 256 and kv_heads >= 4 and (kv_heads > 4 or workgroups > cus)
 
 
 # ------------------------------------------------------------------------------ sampling

@@ -30,6 +30,7 @@ TALK = [  # heads, kv_heads, dk, dv, chunk, block size
     (16, 1, 64, 64, 48, 16),  # a unit is one token
     (8, 8, 128, 32, None, 48),  # pages that are no power of two
     (12, 2, 64, 128, 64, 16),
+    (8, 8, 64, 32, 100, 32),  # eight waves on one turn of values
 ]
 
 
@@ -46,8 +47,10 @@ def test_mixed_heads(heads, kv, dk, dv, chunk, bs, monkeypatch):
         ref = pd.talking_heads(q, k, v, pd.visible_chunk(t, chunk), 0.1, slopes, talk)
         refs.append(ref.reshape(t, -1)[first:])
         seqs.append((q, k, v, first, t - first))
-    for shares, units in ((1, 1), (3, 2 if kv * dv <= 128 else 1), (16, 1)):
+    can_share = kv >= 4 and kv * dv == 256 and dk == 64
+    for shares, units, shared in ((1, 1, False), (3, 2 if kv * dv <= 128 else 1, False), (16, 1, can_share)):
         monkeypatch.setattr(ops, "wide_prompt_units", lambda *a: units)
+        monkeypatch.setattr(ops, "wide_prompt_shared", lambda *a: shared)
         got = run(seqs, bs, shares=shares, heads=heads, kv_heads=kv, chunk=chunk or 0, scale=0.1, slopes=slopes.float().to(DEV),
                   talk=talk.float().to(DEV))
         for i, (g, r) in enumerate(zip(got, refs)):
