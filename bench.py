@@ -481,13 +481,17 @@ def gemv(args) -> int:
             x = torch.randn(m, k, device=dev, dtype=torch.bfloat16)
             decode = lin.decode_product(x, weights[0])
             norm = (norm_weight, 1e-5) if decode and m <= ops.GEMM_DECODE_NORM_ROWS else None
-            how = "gemm_decode" if decode else "gemm_stream" if lin.few_rows(m, weights[0]) else "library"
+            how = "gemm_decode" if decode else "gemm_stream" if lin.few_rows(m, weights[0]) else \
+                "gemm_tiles" if lin.tiles_product(x, weights[0]) else "library"
             if name == "gate_up":
                 out = torch.empty(m, inter, device=dev, dtype=torch.bfloat16)
                 if decode:
                     run = lambda w: ops.gemm_decode(out, x, w, swiglu=True, norm=norm)  # noqa: E731
                 elif lin.few_rows(m, weights[0]):
                     run = lambda w: ops.gemm_stream(out, x, w, swiglu=True)  # noqa: E731
+                elif lin.tiles_fit(x, weights[0]):
+                    run = lambda w: ops.gemm_tiles(out, x, w, swiglu=True)  # noqa: E731
+                    how = "gemm_tiles"
                 else:
                     wide = torch.empty(m, n, device=dev, dtype=torch.bfloat16)
                     run = lambda w: ops.silu_mul(out, torch.mm(x, w.t(), out=wide))  # noqa: E731
@@ -505,6 +509,10 @@ def gemv(args) -> int:
                     run = lambda w: ops.gemm_decode(q, x, w, rope=rope, norm=norm)  # noqa: E731
                 elif lin.few_rows(m, weights[0]):
                     run = lambda w: ops.gemm_stream(q, x, w, rope=rope)  # noqa: E731
+                elif lin.tiles_fit(x, weights[0]) and d % 32 == 0:
+                    rope["angles"] = ops.rotary_angles(positions, inv_freq)
+                    run = lambda w: ops.gemm_tiles(q, x, w, rope=rope)  # noqa: E731
+                    how = "gemm_tiles"
                 else:
                     wide = torch.empty(m, n, device=dev, dtype=torch.bfloat16)
                     run = lambda w: ops.rope_store(torch.mm(x, w.t(), out=wide), inv_freq, positions, slots, k_pool,  # noqa: E731
