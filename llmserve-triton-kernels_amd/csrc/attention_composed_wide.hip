@@ -3,10 +3,17 @@
 // With mixed heads a result is sum_g talk[h, g] sum_j w_g(j) v_h(j).  Mixing the weights w_g first needs them normalised, so
 // two walks over the keys, and every head's weights of a token through LDS.  Here each score column g is multiplied with the
 // values of *all* key/value heads in one walk, u_g[k] = sum_j w_g(j) v_k(j), and the results are mixed once at the end:
-// o_h = sum_g talk[h, g] u_g[kv(h)].  That is kv_heads times the value products (4 of 20 matrix instructions become 16 of 20 at 4
-// key/value heads) and nothing else per key: a plain online softmax whose values are kv_heads * dv wide.  Up to 256 columns
-// of values (64 registers of results a lane) it is the faster way.  Two score maps are the same walk with a map's columns as
-// columns of their own, over the values of their key/value head.
+// o_h = sum_g talk[h, g] u_g[kv(h)]: a plain online softmax whose values are kv_heads * dv wide.  Up to 256 columns of values (64
+// registers of results a lane) it is the faster way.  Two score maps are the same walk with a map's columns as columns of their
+// own, over the values of their key/value head.
+//
+// Mixing may subtract heads that are nearly alike, and then a rounding of each head's weights is not small beside what is left.  So
+// with mixed heads a weight is two bfloat16 numbers, itself rounded and the remainder rounded (2^-18 of it is lost), and the values
+// are multiplied with both: at 4 key/value heads of 64, 32 of 36 matrix instructions are value products, where the kernel that
+// mixes weights has 4 of 12 in its two walks.  Relative error of the result in the norm against 64 bits, 32 heads of 64 on 4, 100 and
+// 1,000 keys: 1.6 to 2.0e-3 for the identity with noise, random matrices, heads minus their mean and minus the next head with
+// queries of 0.01 to 1, and pairs of heads subtracted whose queries are 0.01 to 0.3 apart; where the mixed weights are rounded 2.2
+// to 2.5e-3; with one rounded number a weight 2.0e-3 to 1.2e-1, the pairs up to 0.7.  A third number changes the fourth digit.
 //
 // A unit is 16 columns that share a key row: `tpw` neighbouring tokens times the `grp` query heads of a key/value head.  Per
 // step of 32 keys (two tiles of 16) a wave forms S^T = K Q^T with v_mfma_f32_16x16x32_bf16; a lane then holds keys 4 q4 .. + 3 of
@@ -24,14 +31,13 @@
 // chain of two launches and of lengths -> table -> keys -> results; for portions the answers to a step's values.
 // Measured against that kernel, microseconds (mixed: 32 heads of 64 on 4 key/value heads; maps: 16 heads of two maps of 64 on 2,
 // values of 128):
-//     4 requests, one token behind   300 keys    mixed 22.0 -> 11.6    maps 18.4 ->  9.0
-//     4 requests, one token behind 1,000 keys    mixed 24.1 -> 12.3    maps 31.7 ->  9.8
+//     4 requests, one token behind   300 keys    mixed 22.1 -> 12.1    maps 18.4 ->  9.0
+//     4 requests, one token behind 1,000 keys    mixed 24.9 -> 12.5    maps 31.7 ->  9.8
 //   256 requests, one token behind 1,000 keys    mixed  130 ->   72    maps 50.4 -> 51.1 (5 TB/s of keys and values)
-//     a prompt of   333 tokens                   mixed  153 ->   26    maps 35.7 -> 13.5
-//     a prompt of 2,048 tokens                   mixed  821 ->  154    maps  284 ->   99
-// The weights are rounded to bfloat16 as the operand of the value product there as here, there after the mixing and here before
-// it.  Against 64 bits (100 to 3,000 keys, mixing of 0.3 to 3 times the identity's size): 1.8 to 2.3e-3 of the result's norm here,
-// 2.2 to 2.4e-3 there; two maps 2.2 to 2.5e-3 both.
+//     a prompt of   333 tokens                   mixed  152 ->   27    maps 35.7 -> 13.5
+//     a prompt of 2,048 tokens                   mixed  819 ->  167    maps  284 ->   99
+// (Mixed with one number a weight: 11.8, 12.3, 72, 26 and 154.)  Two maps, whose weights are one number in both kernels, are 2.2 to
+// 2.5e-3 from 64 bits in both.
 //
 // Masks as in attention_composed_mfma.hip: a column at position i sees j <= i with j >= its chunk's start and (i - j < window or
 // j < keep_first).
@@ -41,6 +47,7 @@
 #define NOTHING_YET (-1.0e30f)
 #define AW_SHARES 16  // most workgroups that share a request's keys
 #define AW_NO_KEY 0x40000000
+#define AW_PIECES 2  // of a weight, where heads are mixed behind the value products
 
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
@@ -75,9 +82,26 @@ struct WideArgs {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Four weights of two tiles each as operands of the value products, rounded to bfloat16; the first is the weights rounded, each
+// further one what is then left of them.
+template <int PIECES>
+__device__ __forceinline__ void weight_pieces(float p[2][4], bf16x8v pf[PIECES]) {
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        u32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float &a = p[e / 2][2 * (e % 2)], &b = p[e / 2][2 * (e % 2) + 1];
+            w[e] = pack_bf16x2(a, b);
+            a -= __uint_as_float(w[e] << 16), b -= __uint_as_float(w[e] & 0xffff0000u);
+        }
+        pf[i] = __builtin_bit_cast(bf16x8v, w);
+    }
+}
+
 __device__ __forceinline__ uint32_t low_half_mask(int keep) { return keep <= 0 ? 0u : keep == 1 ? 0xffffu : 0xffffffffu; }
 
-template <int TK, int DT, int U, bool PARTS, bool SHARED>
+template <int TK, int DT, int U, bool PARTS, bool SHARED, bool MIXED>
 __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const WideArgs a) {
     extern __shared__ float lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
@@ -97,6 +121,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
     if (PARTS && head >= a.score_heads) return;
     const int kvh = head / a.maps, map = head - kvh * a.maps;
     const int share = blockIdx.y, bs = a.block_size;
+    constexpr int PIECES = MIXED ? AW_PIECES : 1;
     constexpr int DK = 32 * TK, HALVES = (DT > 8 && !PARTS && !SHARED) ? 2 : 1;  // (16 tiles of values and their results fill a wave's registers)
 
     // tiles of 16 keys: the kept first keys that the window has passed, then what the first token reaches to the last's own
@@ -132,7 +157,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
     const float scale2 = a.scale * LOG2E;
 
     const bf16* k_head = a.k_pool + (size_t)head * bs * DK + col * DK + 8 * q4;
-    const bf16* v_head = a.v_pool + (size_t)(DT * 16 == a.dv ? kvh : 0) * a.dv * bs + col * bs + 4 * q4;
+    const bf16* v_head = a.v_pool + (size_t)(MIXED ? 0 : kvh) * a.dv * bs + col * bs + 4 * q4;
     struct Place {
         int page, in_page;
     };
@@ -159,7 +184,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         for (int d = 0; d < DT; ++d) o[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // SHARED: a step's values go through LDS (2,048 tokens of 32 heads on 4: 201 -> 154 microseconds), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
+    // SHARED: a step's values go through LDS (2,048 tokens of 32 heads on 4: 206 -> 167 microseconds), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
     // (one per key/value head, at least 4) all read all of them.  A chunk is 32 dimensions of a tile, 16 bytes a lane;
     // the two halves of dimensions 8 to 15 of every 16 change places, so that 32 lanes read 64 banks.
     constexpr int CHUNKS = SHARED ? DT / 4 : 1;
@@ -228,7 +253,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         const Place after_at[2] = {place_of(2 * (next + a.shares)), place_of(2 * (next + a.shares) + 1)};
         int j0[2];
         j0[0] = tile_start(2 * step), j0[1] = 2 * step + 1 < n_tiles ? tile_start(2 * step + 1) : AW_NO_KEY;
-        bf16x8v pf[U];
+        bf16x8v pf[U][PIECES];
         float corr[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -270,8 +295,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
                 for (int r = 0; r < 4; ++r) p[tt][r] = fast_exp2(sc[tt][r] - m_new), sum += p[tt][r];
             run_l[u] = run_l[u] * corr[u] + sum;
             run_m[u] = m_new;
-            pf[u] = __builtin_bit_cast(bf16x8v, u32x4{pack_bf16x2(p[0][0], p[0][1]), pack_bf16x2(p[0][2], p[0][3]),
-                                                      pack_bf16x2(p[1][0], p[1][1]), pack_bf16x2(p[1][2], p[1][3])});
+            weight_pieces<PIECES>(p, pf[u]);
         }
         if (HALVES == 2) ask_values(1);
 #pragma unroll
@@ -302,7 +326,8 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     f32x4& to = o[u][half * (DT / HALVES) + d];
-                    to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf[u], to, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < PIECES; ++i) to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf[u][i], to, 0, 0, 0);
                 }
             }
         }
@@ -330,7 +355,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         float* part = a.ws_o + at_col * (DT * 16) + 4 * q4;
 #pragma unroll
         for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4*>(part + 16 * d) = o[0][d];
-    } else if (!a.talk) {
+    } else if constexpr (!MIXED) {
         // the second map's waves leave their results in LDS, lane by lane, for those of the first with the same columns
         float mul[U];
 #pragma unroll
@@ -496,26 +521,33 @@ __global__ __launch_bounds__(64) void combine_maps_kernel(const WideArgs a) {
     }
 }
 
+template <int TK, int DT, int U, bool PARTS, bool MIXED, bool SHARED = false>
+static int launch_one(const WideArgs& a, dim3 grid, int threads, size_t lds, hipStream_t stream) {
+    auto kernel = attend_wide_kernel<TK, DT, U, PARTS, SHARED, MIXED>;
+    if (lds > 48 * 1024) LLMS_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    kernel<<<grid, threads, lds, stream>>>(a);
+    LLMS_LAUNCH_CHECK();
+}
+
+template <int U, bool PARTS, bool MIXED>
+static int launch(const WideArgs& a, int dk, int width, dim3 grid, int threads, size_t lds, hipStream_t stream) {
+    if constexpr (U == 1 && MIXED) {
+        if (width == 256)
+            return dk == 64 ? launch_one<2, 16, U, PARTS, MIXED>(a, grid, threads, lds, stream)
+                            : launch_one<4, 16, U, PARTS, MIXED>(a, grid, threads, lds, stream);
+    }
+    LLMS_REQUIRE(width <= 128, "attend_composed_wide: 256 columns of values go with mixed heads and one unit");
+    if (dk == 64)
+        return width == 64 ? launch_one<2, 4, U, PARTS, MIXED>(a, grid, threads, lds, stream)
+                           : launch_one<2, 8, U, PARTS, MIXED>(a, grid, threads, lds, stream);
+    return width == 64 ? launch_one<4, 4, U, PARTS, MIXED>(a, grid, threads, lds, stream)
+                       : launch_one<4, 8, U, PARTS, MIXED>(a, grid, threads, lds, stream);
+}
+
 template <int U, bool PARTS>
 static int launch(const WideArgs& a, int dk, int width, dim3 grid, int threads, size_t lds, hipStream_t stream) {
-#define AW_LAUNCH(TK, DT)                                                                                              \
-    do {                                                                                                               \
-        auto kernel = attend_wide_kernel<TK, DT, U, PARTS, false>;                                                            \
-        if (lds > 48 * 1024)                                                                                           \
-            LLMS_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
-        kernel<<<grid, threads, lds, stream>>>(a);                                                                     \
-    } while (0)
-    if (width == 256) {
-        if constexpr (U == 1) {
-            if (dk == 64) AW_LAUNCH(2, 16);
-            else AW_LAUNCH(4, 16);
-        }
-    } else if (dk == 64 && width == 64) AW_LAUNCH(2, 4);
-    else if (dk == 64) AW_LAUNCH(2, 8);
-    else if (width == 64) AW_LAUNCH(4, 4);
-    else AW_LAUNCH(4, 8);
-#undef AW_LAUNCH
-    LLMS_LAUNCH_CHECK();
+    return a.talk ? launch<U, PARTS, true>(a, dk, width, grid, threads, lds, stream)
+                  : launch<U, PARTS, false>(a, dk, width, grid, threads, lds, stream);
 }
 
 extern "C" {
@@ -562,11 +594,7 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
         if (shared) {
             LLMS_REQUIRE(talk && units == 1 && kv_heads >= 4 && dk == 64 && width == 256, "attend_composed_wide: shared values with 4 to 8 mixed key/value heads, keys of 64 and 256 columns of values");
             const size_t turns = 2 * (size_t)width * 64, all = lds > turns ? lds : turns;
-            auto kernel = attend_wide_kernel<2, 16, 1, false, true>;
-            if (all > 48 * 1024)
-                LLMS_HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)all));
-            kernel<<<grid, kv_heads * LLMS_WAVE, all, stream>>>(a);
-            LLMS_LAUNCH_CHECK();
+            return launch_one<2, 16, 1, false, true, true>(a, grid, kv_heads * LLMS_WAVE, all, stream);
         }
         return units == 2 ? launch<2, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream)
                           : launch<1, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream);

@@ -1451,8 +1451,8 @@ def attend_composed_wide_supported(q: torch.Tensor, k_pool: torch.Tensor, v_pool
                                    dv: int, block_size: int, talk: bool) -> bool:
     """Whether `attend_composed_wide` takes this attention: bfloat16, keys of 64 or 128, pages of a multiple of 16 keys, aligned
     rows; one token a request, or mixed heads; and 64, 128 or 256 columns of values for a score column: those of its key/value
-    head, with mixed heads those of all.  (With 512 a lane's results would need 128 registers, and the value products would be 8
-    of 9: the kernel that mixes weights has 1 in 3.)"""
+    head, with mixed heads those of all.  (With 512 a lane's results would need 128 registers, and 64 of 68 matrix instructions
+    would be value products: the kernel that mixes weights has 1 in 3.)"""
     width = kv_heads * dv if talk else dv
     return (q.dtype == torch.bfloat16 and heads % kv_heads == 0 and heads // kv_heads <= 16 and dk in (64, 128) and dv % 16 == 0
             and dv <= 128 and width in (64, 128, 256) and block_size % 16 == 0 and kv_heads <= 8 and heads <= 128
@@ -1502,18 +1502,20 @@ def wide_prompt_units(heads: int, kv_heads: int, dv: int, talk: bool, n_seqs: in
     """Units of 16 columns a wave of `attend_composed_wide` takes over portions of prompts.  Two share every key and value a wave
     reads, one gives twice the workgroups (16 heads of two maps over 64, values of 128: 2,000 tokens of 4 requests in 440
     workgroups of two 56 microseconds, in 890 of one 105; 100 tokens in 112 or 224 of them 48 and 39).  The results of two
-    units of 256 columns do not fit a wave's registers."""
-    tpw, width = 16 // (heads // kv_heads), kv_heads * dv if talk else dv
-    workgroups = n_seqs * -(-max_new // (2 * tpw)) * (1 if talk else kv_heads)
-    return 2 if width <= 128 and workgroups >= cus else 1
+    units of 256 columns do not fit a wave's registers, and mixed heads, whose weights are two numbers each, are faster with one (8
+    heads of 128 on 1, 2,048 tokens: 72 against 95; 4 requests of 512: 26 and 35; 16 heads on 4 of 32, 2,048 tokens: 92 and 95)."""
+    if talk or dv > 128:
+        return 1
+    workgroups = n_seqs * -(-max_new // (2 * (16 // (heads // kv_heads)))) * kv_heads
+    return 2 if workgroups >= cus else 1
 
 
 def wide_prompt_shared(heads: int, kv_heads: int, dk: int, dv: int, talk: bool, n_seqs: int, max_new: int, cus: int) -> bool:
     """Whether the waves of a workgroup of `attend_composed_wide` share the values of a step through LDS (256 columns of values, all
     read by at least 4 waves).  Where a SIMD has two waves or more, reading them once a workgroup counts for more than the
-    barrier a step and the way through LDS (microseconds, each wave for itself -> shared, 32 heads of 64 on 4: 1,100 tokens 84 -> 71,
-    2,048 tokens 201 -> 154; 8 heads on 8 of 32: 333 tokens 45 -> 41); a single wave a SIMD waits for each step's barrier (333
-    tokens 25.9 -> 29.2, 512 behind 488 others 53 -> 61)."""
+    barrier a step and the way through LDS (microseconds, each wave for itself -> shared, 32 heads of 64 on 4: 1,100 tokens 84 -> 75,
+    2,048 tokens 206 -> 167; 8 heads on 8 of 32: 333 tokens 46 -> 42); a single wave a SIMD waits for each step's barrier (333
+    tokens 26.9 -> 30.7, 512 behind 488 others 54 -> 66)."""
     workgroups = n_seqs * -(-max_new // (16 // (heads // kv_heads)))
     return talk and dk == 64 and kv_heads * dv == 256 and kv_heads >= 4 and (kv_heads > 4 or workgroups > cus)
 

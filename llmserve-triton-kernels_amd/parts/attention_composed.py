@@ -453,8 +453,8 @@ class ComposedAttention(Mixer):
         without) is one workgroup, which alone keeps one compute unit busy for as long as its keys last; while the batch
         leaves compute units idle its keys go to several, down to one group of 64 keys a share, at the price of one more
         launch, or two more where the heads' weights are mixed and not their results.  Measured, microseconds: 4 requests
-        behind 1,000 keys, 32 heads of 64 mixed: 49 in one share, 19 in 4, 12 in 16; 64 requests 53, 24, 33; 256 requests
-        72, 84, 136."""
+        behind 1,000 keys, 32 heads of 64 mixed: 51 in one share, 21 in 4, 13 in 16; 64 requests 55, 26, 33; 256 requests
+        72, 83, 135."""
         reach = min(x for x in (max_context, self.chunk, None if self.window is None else self.window + self.keep_first)
                     if x is not None)
         return max(1, min(16, cus // max(n_requests, 1), -(-int(reach) // 64)))

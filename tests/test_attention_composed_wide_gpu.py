@@ -118,3 +118,31 @@ def test_values_behind_the_end_and_pages_of_other_requests_are_not_seen():
         ops.attend_composed_wide(out, q, k_pool.to(DEV), v_pool.to(DEV), table, i32(0, new), i32(t), 0, 1, new, heads=heads, kv_heads=kv,
                                  dk=d, dv=d, block_size=bs, scale=0.1, talk=talk, shares=2)
         assert torch.isfinite(out.float()).all()
+
+
+def _relative_error(got, want):
+    got, want = torch.cat([g.double().cpu().flatten() for g in got]), torch.cat([w.flatten() for w in want])
+    return float((got - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.3, 0.1, 0.03])  # of the queries: the flatter the weights, the more of them cancels
+@pytest.mark.parametrize("heads,kv,dk,dv", [(32, 4, 64, 64), (8, 8, 64, 32), (8, 1, 128, 128)])
+def test_heads_that_are_subtracted_from_one_another(heads, kv, dk, dv, scale, monkeypatch):
+    """A head minus the next one, and minus the mean of all: what is left is small beside the heads' own results.  In the norm the
+    result is as near as where the mixed weights are rounded: a rounding of 2^-9 at most of each weight and one of each number."""
+    from llmserve.ops import library as ops
+
+    subtracting = (torch.eye(heads, dtype=F64) - torch.eye(heads, dtype=F64).roll(1, 1), torch.eye(heads, dtype=F64) - 1.0 / heads)
+    for talk in subtracting:
+        seqs, refs = [], []
+        for i, (t, first) in enumerate(REQUESTS[3:]):
+            q, k, v = (rounded(s * x, torch.bfloat16) for s, x in ((scale, rnd(t, heads, dk, seed=60 + i)), (1, rnd(t, kv, dk, seed=70 + i)),
+                                                                   (1, rnd(t, kv, dv, seed=80 + i))))
+            ref = pd.talking_heads(q, k, v, pd.visible_chunk(t, None), dk ** -0.5, torch.zeros(heads, dtype=F64), talk.float().double())
+            refs.append(ref.reshape(t, -1)[first:])
+            seqs.append((q, k, v, first, t - first))
+        kw = dict(heads=heads, kv_heads=kv, chunk=0, scale=dk ** -0.5, talk=talk.float().to(DEV))
+        for shared in {False, kv >= 4 and kv * dv == 256 and dk == 64}:
+            monkeypatch.setattr(ops, "wide_prompt_shared", lambda *a: shared)
+            assert _relative_error(run(seqs, 16, shares=3, **kw), refs) <= 2.0 ** -8
+        assert _relative_error(attend_mfma(seqs, 16, **kw), refs) <= 2.0 ** -8
