@@ -489,7 +489,7 @@ def gemv(args) -> int:
                     run = lambda w: ops.gemm_decode(out, x, w, swiglu=True, norm=norm)  # noqa: E731
                 elif lin.few_rows(m, weights[0]):
                     run = lambda w: ops.gemm_stream(out, x, w, swiglu=True)  # noqa: E731
-                elif lin.tiles_fit(x, weights[0]):
+                elif lin.tiles_product(x, weights[0], "gated"):
                     run = lambda w: ops.gemm_tiles(out, x, w, swiglu=True)  # noqa: E731
                     how = "gemm_tiles"
                 else:
@@ -509,7 +509,7 @@ def gemv(args) -> int:
                     run = lambda w: ops.gemm_decode(q, x, w, rope=rope, norm=norm)  # noqa: E731
                 elif lin.few_rows(m, weights[0]):
                     run = lambda w: ops.gemm_stream(q, x, w, rope=rope)  # noqa: E731
-                elif lin.tiles_fit(x, weights[0]) and d % 32 == 0:
+                elif lin.tiles_product(x, weights[0], "rotary") and d % 32 == 0:
                     rope["angles"] = ops.rotary_angles(positions, inv_freq)
                     run = lambda w: ops.gemm_tiles(q, x, w, rope=rope)  # noqa: E731
                     how = "gemm_tiles"

@@ -16,7 +16,7 @@ import math
 import torch
 
 from ..ops import library as ops
-from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums, tiles_fit
+from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums, tiles_product
 from .registry import ADDED_IN_PLACE, POSITION_ENCODINGS, DeferredNorm, Mixer, register_mixer
 from .spec import PagedCacheSpec, ParamInfo
 
@@ -100,9 +100,7 @@ class Attention(Mixer):
         return not (decode_product(rows, self.qkv_weight) or few_rows(rows.shape[0], self.qkv_weight) or self._fits_tiles(rows))
 
     def _fits_tiles(self, rows) -> bool:
-        # (whatever the weight's size: the rotation and the cache store that the library's product leaves to a kernel of their
-        # own cost more than it gains)
-        return self.head_dim % 32 == 0 and tiles_fit(rows, self.qkv_weight)
+        return self.head_dim % 32 == 0 and tiles_product(rows, self.qkv_weight, "rotary")
 
     def project_and_store(self, x, batch, cache, slots):
         """With bfloat16 rows one kernel does the projection, the rotation and the cache store

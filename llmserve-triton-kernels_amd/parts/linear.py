@@ -16,7 +16,7 @@ bfloat16, few rows otherwise: the hand-written kernel that streams the weight on
 bfloat16, more rows: ops.gemm_tiles, tiles on the matrix cores with the activation, the rotation and cache store, or the
   partial sums of a product that goes to a norm in the epilogue; the library's matrix product (hipBLASLt through
   torch.mm), which is where the reference's engine uses a library too (nn.Linear, src/llmserve/model/llama.py:64-67), only
-  for the sizes where it is still the faster one (tiles_product) and for K or N that the tiles cannot take.
+  for the sizes where it is still the faster one (tiles_pay) and for K or N that the tiles cannot take.
 Operands the matrix-core kernels cannot take (K not a multiple of 8) fall to the 32-bit
 multiply-add kernel, which takes anything.
 
@@ -71,15 +71,34 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
         return m > 0
     return m <= STREAM_MAX_ROWS and -(-m // 16) * weight.numel() * 2 <= STREAM_REREAD_BYTES
 
-# A plain product against a weight this large (the vocabulary's) stays with the library from some rows on: it has tiles for
-# every compute unit several times over, and the library shares the last round's out.  Microseconds, tiles and library:
-# 32000 x 2048 40 and 39 at 160 rows, 54 and 44 at 256, 68 and 65 at 512, 268 and 262 at 2,048; 12288 x 4096 53 and 53 at
-# 333, 56 and 55 at 512, 97 and 87 at 1,024.  Smaller weights win or tie (2048 x 5632 22 and 28 at 333, 56 and 60 at
-# 2,048; 4608 x 2048 12 and 22 at 200), and gated products mostly, with the activation that the library's leaves to a kernel
-# of its own (11264 x 2048 34 and 40 at 333, 101 and 103 at 2,048; 22016 x 4096 75 and 82 at 333, 111 and 96 at 512, 197 and
-# 183 at 1,024, 321 and 424 at 2,048).
-LIBRARY_WEIGHT = 48e6
-LIBRARY_ROWS = 160
+
+# Up to how many multiply-adds ops.gemm_tiles is the faster way; larger products go to the library.  Tiles gain by what they
+# spare (a kernel behind the product, a pass over its result, a short K walk where K comes in parts); the library gains by sharing
+# the last round of tiles out, which the tiles do not, and that weighs more the more rounds there are.  Means over 1,900
+# products of 33 to 2,048 rows (tiles' time over the library's with the kernel behind it; below the line, and beyond): plain 0.89
+# (1.05), gated 0.93 (1.04), rotation and cache store 0.77 (1.00), parts of K for a norm 0.81 (1.04).  The library's times jump from
+# size to size, so single products lie on the wrong side: 1 in 18 below the line is more than 5 percent slower in tiles, at most 19, and 1
+# in 6 beyond it more than 5 percent faster.  Single sizes, microseconds, tiles and library:
+#   plain   4608 x 2048 12 and 16 at 333 rows; 6144 x 2048 16 and 20 at 333, 57 and 46 at 2,048; 32000 x 2048 65 and 61 at 512
+#   gated   11264 x 2048 36 and 38 at 512 rows, 86 and 73 at 1,300; 22016 x 4096 61 and 62 at 200, 107 and 88 at 512, 188 and 162 at
+#           1,024; 28672 x 4096 428 and 355 at 2,048
+#   rotary  2560 x 2048 12 and 20 at 512 rows; 12288 x 4096 57 and 62 at 512, 106 and 90 at 1,024
+#   parts   4096 x 11008 57 and 78 at 512 rows; 8192 x 28672 159 and 313 at 200, 446 and 261 at 640
+# Gated products of TILES_GATED_WORK and more against a weight below TILES_GATED_WEIGHT (200 MB, which the 256 MB memory-side cache
+# holds) are the tiles' again: 27 such products of 17 weights 0.95 in the mean, 0.72 to 1.19, where larger weights are at 1.05; 22016 x
+# 4096 at 2,048 rows 314 and 424.
+TILES_WORK = {"plain": 18e9, "gated": 18e9, "rotary": 40e9, "parts": 60e9}
+TILES_GATED_WORK = 130e9
+TILES_GATED_WEIGHT = 100e6
+
+
+def tiles_pay(kind: str, m: int, n: int, k: int) -> bool:
+    """Whether m rows against a weight [n, k] are faster by ops.gemm_tiles ("plain", "gated" or "rotary" with what follows in the
+    epilogue, "parts": K in parts for a norm to add up) than by the library: a rule by sizes alone."""
+    work = m * n * k
+    if kind == "gated" and work >= TILES_GATED_WORK and n * k < TILES_GATED_WEIGHT:
+        return True
+    return work < TILES_WORK[kind]
 
 
 def tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -87,9 +106,9 @@ def tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return x.shape[0] > STREAM_ROWS and ops.gemm_tiles_supported(x, weight)
 
 
-def tiles_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """Whether a plain product goes there."""
-    return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or not (weight.numel() >= LIBRARY_WEIGHT and x.shape[0] >= LIBRARY_ROWS))
+def tiles_product(x: torch.Tensor, weight: torch.Tensor, kind: str = "plain") -> bool:
+    """Whether a product of this kind goes there."""
+    return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or tiles_pay(kind, x.shape[0], *weight.shape))
 
 
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and
@@ -138,7 +157,7 @@ def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor):
         parts = torch.empty((-(-weight.shape[1] // ops.SLICE_K), m, weight.shape[0]), dtype=torch.float32, device=x.device)
         return PartialSums(ops.gemm_slices(parts, x, weight), x.dtype)
     if not few_rows(m, weight):
-        if tiles_product(x, weight):
+        if tiles_product(x, weight, "parts"):
             k_parts = ops.gemm_tiles_plan(m, weight.shape[0], weight.shape[1], 4, ops.compute_units(x.device))[1]
             if k_parts > 1:
                 parts = torch.empty((k_parts, m, weight.shape[0]), dtype=torch.float32, device=x.device)

@@ -11,7 +11,7 @@ from __future__ import annotations
 import torch
 
 from ..ops import library as ops
-from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums, tiles_fit
+from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums, tiles_product
 from .registry import ADDED_IN_PLACE, DeferredNorm, FeedForward, register_feed_forward
 from .spec import ParamInfo
 
@@ -66,7 +66,7 @@ class SwiGLU(FeedForward):
             few = dtype == torch.bfloat16 and few_rows(m, self.gate_up) and self.intermediate % 8 == 0
             if few and ops.gemm_bf16_supported(rows, self.gate_up):
                 ops.gemm_stream(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # activation in the product's epilogue
-            elif not few and tiles_fit(rows, self.gate_up) and self.intermediate % 16 == 0:
+            elif not few and self.intermediate % 16 == 0 and tiles_product(rows, self.gate_up, "gated"):
                 ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # the same
             else:
                 ops.silu_mul(act, linear(rows, self.gate_up), self.limit, self.gelu)

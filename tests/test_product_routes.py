@@ -1,0 +1,35 @@
+"""Which products of many bfloat16 rows go to the tiles and which to the library: a rule on sizes alone (no GPU)."""
+import pytest
+
+from llmserve.parts.linear import TILES_WORK, tiles_pay
+
+MEASURED = [  # kind, rows, weight [n, k], microseconds of the tiles and of the library with the kernel behind it
+    ("gated", 333, 11264, 2048, 34, 36), ("gated", 512, 11264, 2048, 36, 38), ("gated", 768, 11264, 2048, 45, 48),
+    ("gated", 1300, 11264, 2048, 86, 73), ("gated", 1536, 11264, 2048, 88, 80),
+    ("gated", 400, 22016, 4096, 103, 85), ("gated", 512, 22016, 4096, 107, 88), ("gated", 896, 22016, 4096, 160, 153),
+    ("gated", 1024, 22016, 4096, 188, 162), ("gated", 1100, 22016, 4096, 212, 179), ("gated", 1536, 22016, 4096, 253, 312),
+    ("gated", 2048, 22016, 4096, 314, 424), ("gated", 400, 57344, 8192, 424, 360), ("gated", 512, 57344, 8192, 430, 376),
+    ("gated", 1300, 57344, 8192, 1249, 1009), ("gated", 2048, 57344, 8192, 1415, 1299), ("gated", 640, 28672, 4096, 171, 140),
+    ("gated", 2048, 28672, 4096, 428, 355), ("gated", 544, 16384, 3072, 91, 62), ("gated", 256, 8192, 1536, 13, 21),
+    ("rotary", 512, 2560, 2048, 12, 20), ("rotary", 2048, 2560, 2048, 28, 33), ("rotary", 512, 12288, 4096, 57, 62),
+    ("rotary", 1024, 12288, 4096, 106, 90), ("rotary", 2048, 12288, 4096, 185, 172), ("rotary", 256, 10240, 8192, 67, 95),
+    ("rotary", 1024, 10240, 8192, 157, 142), ("rotary", 2048, 10240, 8192, 320, 275),
+    ("plain", 333, 6144, 2048, 16, 20), ("plain", 2048, 6144, 2048, 57, 46), ("plain", 333, 4608, 2048, 12, 16),
+    ("plain", 2048, 4608, 2048, 44, 40), ("plain", 1024, 12288, 4096, 101, 81), ("plain", 2048, 5120, 5120, 119, 103),
+    ("parts", 512, 4096, 11008, 57, 78), ("parts", 200, 8192, 28672, 159, 313), ("parts", 1024, 8192, 28672, 479, 375),
+    ("parts", 1100, 8192, 8192, 182, 137), ("parts", 128, 2048, 5632, 13, 17),
+]
+
+
+@pytest.mark.parametrize("kind,m,n,k,tiles,library", MEASURED)
+def test_the_faster_way_is_taken(kind, m, n, k, tiles, library):
+    assert tiles_pay(kind, m, n, k) == (tiles < library)
+
+
+def test_what_the_tiles_leave_behind_is_the_librarys():
+    """A gated product, a rotation or parts of K that the tiles decline become a plain product and a kernel: the plain product must
+    then not be theirs either, as it was the library's product that was the faster one."""
+    for kind in TILES_WORK:
+        for m in (65, 200, 512, 700, 1100, 2048, 8192):
+            for n, k in ((2560, 2048), (11264, 2048), (22016, 4096), (4096, 11008), (57344, 8192)):
+                assert tiles_pay(kind, m, n, k) or not tiles_pay("plain", m, n, k)
