@@ -390,9 +390,9 @@ class ComposedAttention(Mixer):
         args = (out, q, paged.k_pool, paged.v_pool, view.block_tables, batch.cu_seqlens, batch.context_lens)
         common.update(dist_bias=self.dist_bias, gate=gate, sink=self.sink, gate_heads=self.gate_heads)
         n_dec = batch.num_decode
-        # one walk over the keys by a short kernel, and the results mixed, wherever it takes the sizes: it was the faster one from 1
-        # request to 256, 64 keys to 4,000 and 16 tokens to 2,048 (12 against 24 microseconds for 4 decoding requests behind
-        # 1,000 keys, 26 against 153 for a prompt of 333)
+        # one walk over the keys by a short kernel, and the results mixed, wherever it takes the sizes and a portion is not short
+        # behind many keys (shares_long_keys): it was the faster one from 1 request to 256, 64 keys to 4,000 and 16 tokens to 2,048
+        # (13 against 25 microseconds for 4 decoding requests behind 1,000 keys, 27 against 152 for a prompt of 333)
         wide = self.dist_bias is None and gate is None and not (self.talking and self.head_norm_eps is not None) and \
             ops.attend_composed_wide_supported(q, paged.k_pool, paged.v_pool, self.num_heads, self.num_kv_heads, self.head_dim,
                                                self.value_dim, paged.block_size, self.talking)
@@ -413,9 +413,11 @@ class ComposedAttention(Mixer):
                                         head_dim=self.head_dim, block_size=paged.block_size, scale=self.scale,
                                         dist_bias=self.dist_bias, gate=gate, table_rows=batch.state_slots)
             return
-        if n_dec < batch.num_seqs and batch.max_count > 1 and wide:
+        if n_dec == batch.num_seqs:
+            return
+        if batch.max_count > 1 and wide and not self.shares_long_keys(batch.max_count, batch.max_context):
             ops.attend_composed_wide(*args, n_dec, batch.num_seqs - n_dec, batch.max_count, **plain)
-        elif n_dec < batch.num_seqs:
+        else:
             shares = self.prompt_shares(batch.num_seqs - n_dec, batch.max_count, batch.max_context,
                                         ops.compute_units(q.device))
             ops.attend_composed_mfma(*args, n_dec, batch.num_seqs - n_dec, batch.max_count, shares=shares, **common)
@@ -433,6 +435,17 @@ class ComposedAttention(Mixer):
             splits = prompt_splits(heads, kv, self.window, batch.num_seqs - n_dec, batch.max_count, batch.max_context, cus)
             ops.attention_mfma(*common, n_dec, batch.num_seqs - n_dec, batch.max_count, n_dec, batch.num_tokens - n_dec, heads,
                                kv, d, bs, window, self.scale, num_splits=splits, table_rows=batch.state_slots, head_gate=gate)
+
+    def shares_long_keys(self, max_new: int, max_context: int) -> bool:
+        """Whether portions with mixed heads go to the kernel that mixes weights although the one that mixes results takes their
+        sizes.  The latter walks a block's keys in one workgroup, at 75 nanoseconds a key with 8 key/value heads and 40 with 4;
+        the former walks them twice, but in up to 4 shares, and while the columns of the portion fill one unit of 16 that is
+        less from some 1,500 keys on (microseconds, mixing results and weights: 8 heads of 64 on 8 of 32, 8 tokens behind 1,000
+        keys 84 and 89, 4,000 keys 307 and 221, 16,000 keys 1,179 and 862; 4 heads on 4 of 64 53 and 64, 172 and 152, 652 and 590;
+        with twice the tokens, two units, 318 and 416, 180 and 259 behind 4,000 keys; with 2 key/value heads 107 and 158)."""
+        reach = max_context if self.chunk is None else min(max_context, self.chunk)
+        return (self.talking and self.num_kv_heads >= 4 and max_new * (self.num_heads // self.num_kv_heads) <= 16
+                and self.num_heads <= 32 and reach >= 1500)
 
     def prompt_shares(self, n_requests: int, max_new: int, max_context: int, cus: int = 256) -> int:
         """Workgroups that share the keys of one block of prompt tokens when the heads' weights are mixed.  All heads

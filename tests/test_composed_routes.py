@@ -1,0 +1,56 @@
+"""Which kernel of the composed attention a step's requests go to (a rule on sizes alone; no GPU)."""
+from types import SimpleNamespace
+
+import pytest
+
+from llmserve.ops import library as ops
+from llmserve.parts.attention_composed import ComposedAttention
+
+
+def route(monkeypatch, heads, kv, new, context, n=1, n_dec=0, chunk=None, talking=True, dk=64, dv=32):
+    """(kernel, first request, requests, most new tokens, shares) of every launch."""
+    calls = []
+    for name in ("attend_composed_wide", "attend_composed_mfma"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, **kw: calls.append((name, *a[7:10], kw.get("shares"))))
+    for name in ("attend_composed_wide_supported", "attend_composed_mfma_supported"):
+        monkeypatch.setattr(ops, name, lambda *a: True)
+    monkeypatch.setattr(ops, "compute_units", lambda device: 256)
+    monkeypatch.setattr(ops, "attend_composed_mfma_tokens", lambda *a: 16)
+    part = ComposedAttention({"hidden": 64, "num_heads": heads, "num_kv_heads": kv, "head_dim": dk, "value_dim": dv, "chunk": chunk,
+                              "talking_heads": talking, "differential": not talking}, None)
+    batch = SimpleNamespace(num_decode=n_dec, num_seqs=n + n_dec, max_count=new, max_context=context, max_decode_context=context,
+                            state_slots=None, cu_seqlens=None, context_lens=None, num_tokens=n * new + n_dec)
+    part.attend(None, SimpleNamespace(dtype=None, device=None), SimpleNamespace(k_pool=None, v_pool=None, block_size=16),
+                SimpleNamespace(block_tables=None), batch)
+    return calls
+
+
+@pytest.mark.parametrize("heads,kv,new,context,chunk,dv,kernel", [
+    (8, 8, 8, 4000, None, 32, "mfma"), (8, 8, 16, 16000, None, 32, "mfma"), (16, 8, 8, 4000, None, 32, "mfma"),
+    (4, 4, 8, 4000, None, 64, "mfma"), (16, 4, 2, 4000, None, 64, "mfma"),
+    (8, 8, 8, 1000, None, 32, "wide"),      # few keys
+    (8, 8, 8, 4000, 1024, 32, "wide"),      # (its own chunk's)
+    (8, 8, 32, 4000, None, 32, "wide"),     # more than one unit of columns
+    (16, 8, 16, 4000, None, 32, "wide"),
+    (64, 8, 2, 4000, None, 32, "wide"),     # many heads to mix
+    (4, 2, 8, 16000, None, 64, "wide"),     # few key/value heads
+])
+def test_short_portions_behind_many_keys_share_them(heads, kv, new, context, chunk, dv, kernel, monkeypatch):
+    (call,) = route(monkeypatch, heads, kv, new, context, chunk=chunk, dv=dv)
+    assert call[:4] == (f"attend_composed_{kernel}", 0, 1, new)
+    assert kernel == "wide" or call[4] == 4
+
+
+def test_single_tokens_beside_them_do_not_change(monkeypatch):
+    decode, portion = route(monkeypatch, 8, 8, 8, 4000, n=2, n_dec=3)
+    assert decode[:4] == ("attend_composed_wide", 0, 3, 1) and portion[:4] == ("attend_composed_mfma", 3, 2, 8)
+
+
+def test_two_maps_have_one_walk_whatever_the_keys(monkeypatch):
+    (call,) = route(monkeypatch, 8, 8, 8, 16000, talking=False, dv=64)
+    assert call[0] == "attend_composed_wide"
+
+
+def test_nothing_but_single_tokens_is_one_launch(monkeypatch):
+    (call,) = route(monkeypatch, 8, 8, 1, 4000, n=0, n_dec=5)
+    assert call[:4] == ("attend_composed_wide", 0, 5, 1)
