@@ -637,8 +637,11 @@ def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256)
 
 
 def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 64, blocks of 16 weight rows, 16-byte rows."""
-    return gemm_bf16_supported(x, w) and x.shape[1] % 64 == 0 and w.shape[0] % 16 == 0 and w.dtype == torch.bfloat16
+    """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 64, blocks of 16 weight rows, rows of x of 16-byte pieces
+    that do not overlap, a contiguous w, and neither without columns or rows."""
+    n, k = w.shape
+    return (gemm_bf16_supported(x, w) and x.stride(1) == 1 and k <= x.stride(0) < 1 << 26 and k > 0 and k % 64 == 0 and n > 0 and n % 16 == 0
+            and w.dtype == torch.bfloat16 and w.is_contiguous())
 
 
 def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *, swiglu: bool = False,

@@ -171,6 +171,13 @@ def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor):
     return PartialSums(parts, x.dtype)
 
 
+def _tiles_take(out: torch.Tensor, bias: torch.Tensor | None, n: int) -> bool:
+    """Whether ops.gemm_tiles stores into `out` and adds `bias` (the library's product takes any strides, and a bias of another
+    dtype or of one number)."""
+    return (out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0 and
+            (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == (n,))))
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
            out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """x [M, K] (unit inner stride), weight [N, K] -> [M, N] in out_dtype (default: x's)."""
@@ -185,7 +192,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
             return ops.gemm_decode(out, x, weight, bias)
         if few_rows(m, weight):
             return ops.gemm_stream(out, x, weight, bias)
-        if tiles_product(x, weight) and out.stride(0) % 4 == 0 and out.data_ptr() % (4 * out.element_size()) == 0:
+        if tiles_product(x, weight) and _tiles_take(out, bias, n):
             return ops.gemm_tiles(out, x, weight, bias)
         if OWN_KERNELS_ONLY:
             return ops.gemm_bf16(out, x, weight, bias, kernel="skinny" if m <= 64 else "tile")

@@ -118,6 +118,47 @@ def test_rotary(tile, nh, nkv, d, bs, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("what", ["plain", "columns of a wider weight", "transposed weight", "every other column of x", "one row many times",
+                                  "no weight rows", "no columns", "32-bit bias", "every other number of a bias", "bias of one number",
+                                  "bias of rows", "every other column of out", "transposed out"])
+def test_what_the_tiles_do_not_take_goes_to_the_library(what):
+    """`linear` with many rows takes any strides of its operands and its result, no rows or columns, and any bias that can be added."""
+    from llmserve.parts.linear import linear
+
+    m, n, k = 100, 256, 512
+    x, w, bias = rnd(m, k, seed=1).to(DEV), rnd(n, k, seed=2, scale=k ** -0.5).to(DEV), None
+    wide, out = rnd(m, 2 * k, seed=3).to(DEV), None
+    if what == "columns of a wider weight":
+        w = rnd(n, k + 8, seed=4, scale=k ** -0.5).to(DEV)[:, :k]
+    elif what == "transposed weight":
+        w = rnd(k, n, seed=4, scale=k ** -0.5).to(DEV).t()
+    elif what == "every other column of x":
+        x = wide[:, ::2]
+    elif what == "one row many times":
+        x = wide[:1, :k].expand(m, k)
+    elif what == "no weight rows":
+        w = w[:0]
+    elif what == "no columns":
+        x, w = x[:, :0], w[:, :0].contiguous()
+    elif what == "32-bit bias":
+        bias = rnd(n, seed=5).float().to(DEV)
+    elif what == "every other number of a bias":
+        bias = rnd(2 * n, seed=5).to(DEV)[::2]
+    elif what == "bias of one number":
+        bias = rnd(1, seed=5).to(DEV)
+    elif what == "bias of rows":
+        bias = rnd(m, n, seed=5).to(DEV)
+    elif what == "every other column of out":
+        out = torch.empty(m, 2 * n, dtype=torch.bfloat16, device=DEV)[:, ::2]
+    elif what == "transposed out":
+        out = torch.empty(n, m, dtype=torch.bfloat16, device=DEV).t()
+    got = linear(x, w, bias, out=out)
+    assert tuple(got.shape) == (m, w.shape[0]) and (out is None or got.data_ptr() == out.data_ptr())
+    if got.numel():
+        close(got, product(x.cpu(), w.cpu(), None if bias is None else bias.cpu()), k)
+
+
+@pytest.mark.gpu
 def test_what_the_kernel_cannot_take_is_refused():
     x, w = rnd(70, 256).to(DEV), rnd(64, 256).to(DEV)
     out = torch.empty(70, 64, dtype=torch.bfloat16, device=DEV)
