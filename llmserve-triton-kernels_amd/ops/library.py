@@ -688,6 +688,7 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
         nh, nkv, d = r["n_heads"], r["n_kv_heads"], r["head_dim"]
         if d % 32 or n != (nh + 2 * nkv) * d:
             raise ValueError("the rotary epilogue needs head_dim in multiples of 32 and N = (heads + 2 kv heads) * head_dim")
+        _dev(x, r["inv_freq"], r["angles"], r["positions"], r["slots"], r["k_pool"], r["v_pool"])
         if r["angles"] is None and r["inv_freq"] is not None:
             _i32(r["positions"], "positions", m)
             _f32(r["inv_freq"], "inv_freq", d // 2)
@@ -701,8 +702,6 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
             if (tuple(kp.shape) != (pages, nkv, bs, d) or tuple(vp.shape) != (pages, nkv, d, bs) or kp.dtype != torch.bfloat16
                     or vp.dtype != torch.bfloat16 or not kp.is_contiguous() or not vp.is_contiguous()):
                 raise ValueError("k_pool and v_pool must be contiguous bfloat16 pools of these heads and pages")
-            if kp.device != dev or vp.device != dev or r["slots"].device != dev:
-                raise ValueError("pools and slots must be on the operands' device")
         epilogue, cols = 3, nh * d
     if tuple(out.shape[-2:]) != (m, cols):
         raise ValueError(f"out shape {tuple(out.shape)} does not end in {(m, cols)}")

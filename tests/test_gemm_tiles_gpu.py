@@ -173,6 +173,19 @@ def test_what_the_kernel_cannot_take_is_refused():
             bad()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["angles", "slots", "k_pool", "v_pool"])
+def test_a_rotation_from_host_memory_is_refused(name):
+    m, d, k = 70, 64, 128
+    rope = dict(n_heads=2, n_kv_heads=1, head_dim=d, inv_freq=None, positions=torch.zeros(m, dtype=torch.int32, device=DEV),
+                angles=torch.zeros(m, d // 2, 2, device=DEV), slots=torch.zeros(m, dtype=torch.int32, device=DEV),
+                k_pool=torch.zeros(5, 1, 16, d, dtype=torch.bfloat16, device=DEV),
+                v_pool=torch.zeros(5, 1, d, 16, dtype=torch.bfloat16, device=DEV), block_size=16)
+    rope[name] = rope[name].cpu()
+    with pytest.raises(ValueError):
+        ops().gemm_tiles(torch.empty(m, 2 * d, dtype=torch.bfloat16, device=DEV), rnd(m, k).to(DEV), rnd(4 * d, k).to(DEV), rope=rope)
+
+
 def test_plan():
     """The plan names a tile, and no more parts than were allowed or than K has steps for."""
     for m in (17, 64, 65, 128, 333, 512, 2048, 8191):
