@@ -33,11 +33,6 @@
 
 #define AM_PAGE_CACHE 1024  // page ids (4 bytes each) a workgroup keeps in LDS
 
-// Heads are mixed on the matrix cores, in 32-bit, up to this many blocks of 16 of them (their sums stay in registers).  On the
-// vector units every column read all heads' weights of its keys from LDS, 262 KB a token and 64 keys at 32 heads, and LDS
-// bounded the kernel; now a token's weights are read once for every 16 heads.
-#define AM_MIX_TILES 2
-
 #define LOG2E 1.4426950408889634f
 #define NOTHING_YET (-1.0e30f)
 
@@ -432,12 +427,6 @@ __global__ __launch_bounds__(THREADS) void attend_mfma_kernel(const MfmaArgs a) 
         const int group_keys = 16 * TG;
         float* pbuf = lds + (size_t)slice * a.tok * H * group_keys;  // [slice][tok][H][16 TG]
         float* talk_s = lds + (size_t)NS * a.tok * H * group_keys;    // [g][h]
-        // 16 weights of a token's head; a head's tiles change places with the heads, so that 4 heads' weights of the same keys
-        // lie in different banks
-        auto weights_at = [&](int token, int head, int tile) {
-            return pbuf + ((size_t)token * H + head) * group_keys + 16 * (tile ^ (head & (TG - 1)));
-        };
-        const bool on_cores = H <= 16 * AM_MIX_TILES;
         float* stats = talk_s + H * H;                               // [unit][slice][2][16]
         for (int i = threadIdx.x; i < H * H; i += blockDim.x) talk_s[(i % H) * H + i / H] = a.talk[i];
         // first walk: every column's maximum and sum
@@ -517,53 +506,26 @@ __global__ __launch_bounds__(THREADS) void attend_mfma_kernel(const MfmaArgs a) 
                         f32x4 w;
 #pragma unroll
                         for (int r = 0; r < 4; ++r) w[r] = fast_exp2(sc[tt][r] - run_m[uu][0]) * inv_l[uu];
-                        if (col < used_cols) *reinterpret_cast<f32x4*>(weights_at(u_tl[uu], u_h[uu], tt) + 4 * q4) = w;
+                        if (col < used_cols)
+                            *reinterpret_cast<f32x4*>(pbuf + ((size_t)u_tl[uu] * H + u_h[uu]) * group_keys + 16 * tt + 4 * q4) = w;
                     }
                 }
             };
             if (some) walk(std::false_type{});
             __syncthreads();
-            if (on_cores) {
-                // A job is a token's 16 keys: sum_g w_g(key) talk[h, g] for all heads h, 4 heads g an instruction (32-bit operands
-                // and sums, the heads in order).  It reads and then overwrites only its own weights.
-                for (int job = some ? uw : ntok * TG; job < ntok * TG; job += n_uw) {
-                    const int tl = job / TG, tt = job % TG;
-                    f32x4 mixed[AM_MIX_TILES];
-#pragma unroll
-                    for (int ht = 0; ht < AM_MIX_TILES; ++ht) mixed[ht] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    for (int g0 = 0; g0 < H; g0 += 4) {
-                        const int g = g0 + q4;
-                        const float wg = g < H ? weights_at(tl, g, tt)[col] : 0.f;
-#pragma unroll
-                        for (int ht = 0; ht < AM_MIX_TILES; ++ht) {
-                            if (16 * ht >= H) break;
-                            const int h = 16 * ht + col;
-                            const float tg = (g < H && h < H) ? talk_s[g * H + h] : 0.f;
-                            mixed[ht] = __builtin_amdgcn_mfma_f32_16x16x4f32(wg, tg, mixed[ht], 0, 0, 0);
-                        }
-                    }
-#pragma unroll
-                    for (int ht = 0; ht < AM_MIX_TILES; ++ht)
-                        if (16 * ht + col < H) *reinterpret_cast<f32x4*>(weights_at(tl, 16 * ht + col, tt) + 4 * q4) = mixed[ht];
-                }
-                __syncthreads();
-            }
 #pragma unroll
             for (int uu = 0; uu < MAXU; ++uu) {
                 if (!mine[uu] || !some) continue;
                 f32x4 w[TG];
 #pragma unroll
                 for (int tt = 0; tt < TG; ++tt) w[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if (on_cores) {
-                    if (valid[uu])
-#pragma unroll
-                        for (int tt = 0; tt < TG; ++tt) w[tt] = *reinterpret_cast<const f32x4*>(weights_at(u_tl[uu], u_h[uu], tt) + 4 * q4);
-                } else if (col < used_cols) {
+                if (col < used_cols) {
+                    const float* prow = pbuf + (size_t)u_tl[uu] * H * group_keys + 4 * q4;
                     const float* trow = talk_s + u_h[uu];
                     for (int g = 0; g < H; ++g) {
                         const float tg = trow[g * H];
 #pragma unroll
-                        for (int tt = 0; tt < TG; ++tt) w[tt] += tg * *reinterpret_cast<const f32x4*>(weights_at(u_tl[uu], g, tt) + 4 * q4);
+                        for (int tt = 0; tt < TG; ++tt) w[tt] += tg * *reinterpret_cast<const f32x4*>(prow + g * group_keys + 16 * tt);
                     }
                 }
                 s16x4 pf[TG];
