@@ -167,9 +167,8 @@ __global__ void rmsnorm_bf16_vec_kernel(bf16* __restrict__ out, const bf16* x, c
     }
 }
 
-// The same for float rows of hidden % 4 == 0 and hidden <= 4 * RV_CHUNKS * 256: the row, what is added to
-// it and the norm's weight are asked for at once (one wait for memory; the plain kernel waits three times: rows of 2,048
-// take 4.8 microseconds under the profiler, 5.7 there).
+// The same for few float rows of hidden % 4 == 0 and hidden <= 4 * RV_CHUNKS * 256: the row, what is added to it and the norm's
+// weight are asked for at once (one wait for memory; the plain kernel waits three times).  See f32_rows_at_once for what it takes.
 __global__ __launch_bounds__(256) void rmsnorm_f32_vec_kernel(float* __restrict__ out, const float* x, const float* __restrict__ delta,
                                                               float* resid_out, const float* __restrict__ weight,
                                                               const int* __restrict__ rows, float eps, int hidden,
@@ -543,6 +542,16 @@ __global__ void rotary_angles_kernel(float2* out, const int* positions, const fl
     if (i < total) out[i] = rotary_angle((float)positions[i / half], inv_freq[i % half]);
 }
 
+// Which float rows are normed by the kernel that asks for everything at once: long rows, few of them.  With short rows most of
+// its four pieces a thread hold nothing, and with many rows other rows hide the waits while its registers leave room for fewer.
+// Microseconds, the plain kernel and this one, with a sum written back, the row warm and the weight cold as behind a product:
+// rows of 4,096 at 1 row 8.9 and 6.1, at 256 9.9 and 7.9, at 1,024 17.7 and 21.2; of 2,048 at 1 row 5.7 and 4.9, at 256 6.9 and
+// 6.6, at 1,024 9.8 and 12.0; of 1,024 at 1 row 4.8 and 3.7, at 16 4.6 and 4.6, at 64 5.0 and 5.6; of 512 at 4 rows 4.1 and 3.9, at
+// 64 4.1 and 5.1.
+static bool f32_rows_at_once(int n_rows, int hidden) {
+    return hidden % 4 == 0 && hidden <= 4 * RV_CHUNKS * 256 && ((hidden >= 2048 && n_rows <= 256) || (hidden >= 1024 && n_rows <= 16));
+}
+
 extern "C" {
 
 int llms_embed_gather(int dtype, void* out, const void* table, const int* ids, int n_tokens, int hidden,
@@ -572,8 +581,9 @@ int llms_rmsnorm(int dtype, void* out, const void* x, const void* delta, void* r
                                                                 hidden, parts, n_parts, part_stride);
         LLMS_LAUNCH_CHECK();
     }
-    if (dtype == 0 && (!parts || (((uintptr_t)parts % 16) == 0 && part_stride % 4 == 0)) && hidden % 4 == 0 && hidden <= 4 * RV_CHUNKS * 256 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0 &&
-        ((uintptr_t)weight % 16) == 0 && ((uintptr_t)delta % 16) == 0 && ((uintptr_t)resid_out % 16) == 0) {
+    if (dtype == 0 && f32_rows_at_once(n_rows, hidden) && (!parts || (((uintptr_t)parts % 16) == 0 && part_stride % 4 == 0)) &&
+        ((uintptr_t)x % 16) == 0 && ((uintptr_t)out % 16) == 0 && ((uintptr_t)weight % 16) == 0 && ((uintptr_t)delta % 16) == 0 &&
+        ((uintptr_t)resid_out % 16) == 0) {
         rmsnorm_f32_vec_kernel<<<n_rows, 256, 0, stream>>>((float*)out, (const float*)x, (const float*)delta, (float*)resid_out,
                                                            (const float*)weight, rows, eps, hidden, parts, n_parts, part_stride);
         LLMS_LAUNCH_CHECK();

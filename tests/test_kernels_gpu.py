@@ -95,6 +95,19 @@ def test_rmsnorm_takes_the_delta_as_partial_sums(dtype, hidden, parts):
         ops().rmsnorm(torch.empty_like(resid), resid, w.to(DEV), 1e-5, delta=p[:, :8].contiguous().to(DEV))
 
 
+# both kernels of 32-bit rows, at the lines between them (few long rows ask for everything at once)
+@pytest.mark.parametrize("rows,hidden", [(16, 1024), (17, 1024), (3, 1020), (256, 2048), (257, 2048), (2, 2044), (300, 4096), (2, 4096), (2, 4100)])
+def test_rmsnorm_of_32_bit_rows(rows, hidden):
+    x, delta, w = rnd(rows, hidden, seed=2, scale=3.0), rnd(rows, hidden, seed=3), 1 + 0.1 * rnd(hidden, seed=4)
+    resid = x.to(DEV)
+    out = ops().rmsnorm(torch.empty_like(resid), resid, w.to(DEV), 1e-5, delta=delta.to(DEV), resid_out=resid)
+    assert torch.equal(resid.cpu(), x + delta)
+    summed = (x + delta).double()
+    want = summed / torch.sqrt((summed * summed).mean(-1, keepdim=True) + 1e-5) * w.double()
+    # three roundings of 2^-24 of a number, and the sum of squares: positive terms, a chain of at most 16 + 10 of them
+    assert ((out.cpu().double() - want).abs() <= 30 * 2.0 ** -24 * want.abs() + 1e-30).all()
+
+
 def test_rmsnorm_tiny_inputs_feel_eps():
     x = rnd(2, 96, seed=5, scale=1e-3)
     w = torch.ones(96)
