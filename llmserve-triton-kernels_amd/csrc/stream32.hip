@@ -112,35 +112,27 @@ __global__ __launch_bounds__(S32_THREADS) void gated_add_norm_vec_kernel(
     const int n = blockIdx.x, n4 = hidden / 4;
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f), one = make_float4(1.f, 1.f, 1.f, 1.f);
     auto at = [](const float* p) { return *reinterpret_cast<const float4*>(p); };
-    // everything the row needs is asked for before the first number is used, the norm's weight too (behind the sum's barrier
-    // it cost a trip to memory of its own)
-    float4 r[S32_VEC], w[S32_VEC], a0[S32_VEC], a1[S32_VEC], z0[S32_VEC], z1[S32_VEC], b0[S32_VEC], b1[S32_VEC];
-    const bool gate0 = y0 && z_col0 >= 0, gate1 = y1 && z_col1 >= 0;
+    float4 r[S32_VEC];
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < S32_VEC; ++i) {
         const int c = 4 * (threadIdx.x + i * S32_THREADS);
-        const bool in = c < hidden;
-        r[i] = in ? at(x + (size_t)n * hidden + c) : zero;
-        a0[i] = (in && y0) ? at(y0 + (size_t)n * y0_stride + c) : zero;
-        a1[i] = (in && y1) ? at(y1 + (size_t)n * y1_stride + c) : zero;
-        z0[i] = (in && gate0) ? at(z + (size_t)n * z_stride + z_col0 + c) : zero;
-        z1[i] = (in && gate1) ? at(z + (size_t)n * z_stride + z_col1 + c) : zero;
-        b0[i] = (in && gate0 && bias0) ? at(bias0 + c) : zero;
-        b1[i] = (in && gate1 && bias1) ? at(bias1 + c) : zero;
-        w[i] = in ? at(weight + c) : zero;
-    }
-#pragma unroll
-    for (int i = 0; i < S32_VEC; ++i) {
-        const int c = 4 * (threadIdx.x + i * S32_THREADS);
+        r[i] = zero;
         if (c < hidden) {
-            const float4 g0 = gate0 ? gate4(z0[i], b0[i]) : one;
-            const float4 g1 = gate1 ? gate4(z1[i], b1[i]) : one;
+            const float4 xv = at(x + (size_t)n * hidden + c);
+            const float4 a0 = y0 ? at(y0 + (size_t)n * y0_stride + c) : zero;
+            const float4 a1 = y1 ? at(y1 + (size_t)n * y1_stride + c) : zero;
+            const float4 z0 = (y0 && z_col0 >= 0) ? at(z + (size_t)n * z_stride + z_col0 + c) : zero;
+            const float4 z1 = (y1 && z_col1 >= 0) ? at(z + (size_t)n * z_stride + z_col1 + c) : zero;
+            const float4 b0 = (y0 && z_col0 >= 0 && bias0) ? at(bias0 + c) : zero;
+            const float4 b1 = (y1 && z_col1 >= 0 && bias1) ? at(bias1 + c) : zero;
+            const float4 g0 = (y0 && z_col0 >= 0) ? gate4(z0, b0) : one;
+            const float4 g1 = (y1 && z_col1 >= 0) ? gate4(z1, b1) : one;
             float4 s;
-            s.x = r[i].x + (g0.x * a0[i].x + g1.x * a1[i].x);
-            s.y = r[i].y + (g0.y * a0[i].y + g1.y * a1[i].y);
-            s.z = r[i].z + (g0.z * a0[i].z + g1.z * a1[i].z);
-            s.w = r[i].w + (g0.w * a0[i].w + g1.w * a1[i].w);
+            s.x = xv.x + (g0.x * a0.x + g1.x * a1.x);
+            s.y = xv.y + (g0.y * a0.y + g1.y * a1.y);
+            s.z = xv.z + (g0.z * a0.z + g1.z * a1.z);
+            s.w = xv.w + (g0.w * a0.w + g1.w * a1.w);
             *reinterpret_cast<float4*>(x + (size_t)n * hidden + c) = s;
             r[i] = s;
             ss += s.x * s.x + s.y * s.y + s.z * s.z + s.w * s.w;
@@ -152,10 +144,11 @@ __global__ __launch_bounds__(S32_THREADS) void gated_add_norm_vec_kernel(
     for (int i = 0; i < S32_VEC; ++i) {
         const int c = 4 * (threadIdx.x + i * S32_THREADS);
         if (c < hidden) {
-            orow[c + 0] = from_f32<T>(r[i].x * inv * (offset + w[i].x));
-            orow[c + 1] = from_f32<T>(r[i].y * inv * (offset + w[i].y));
-            orow[c + 2] = from_f32<T>(r[i].z * inv * (offset + w[i].z));
-            orow[c + 3] = from_f32<T>(r[i].w * inv * (offset + w[i].w));
+            const float4 w = at(weight + c);
+            orow[c + 0] = from_f32<T>(r[i].x * inv * (offset + w.x));
+            orow[c + 1] = from_f32<T>(r[i].y * inv * (offset + w.y));
+            orow[c + 2] = from_f32<T>(r[i].z * inv * (offset + w.z));
+            orow[c + 3] = from_f32<T>(r[i].w * inv * (offset + w.w));
         }
     }
     (void)n4;
@@ -455,13 +448,11 @@ __global__ __launch_bounds__(S32_THREADS) void normed_add_norm_kernel(T* __restr
                      ((uintptr_t)w % 16) == 0 && ((uintptr_t)out % 16) == 0;
     if (vec && hidden <= 4 * NAN_VEC * S32_THREADS) {
         // the row, what joins it and that norm's weight in registers, all asked for at once: one trip to memory
-        // (the second norm's weight among them: behind the sums' barriers it cost a trip of its own)
-        float4 xv[NAN_VEC], yv[NAN_VEC], bv[NAN_VEC], wv[NAN_VEC];
+        float4 xv[NAN_VEC], yv[NAN_VEC], bv[NAN_VEC];
 #pragma unroll
         for (int i = 0; i < NAN_VEC; ++i) {
             const int c = 4 * (threadIdx.x + i * S32_THREADS);
             const bool in = c < hidden;
-            wv[i] = (in && w && out) ? *reinterpret_cast<const float4*>(w + c) : make_float4(1.f, 1.f, 1.f, 1.f);
             xv[i] = in ? *reinterpret_cast<const float4*>(xr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
             yv[i] = (in && yr) ? *reinterpret_cast<const float4*>(yr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
             bv[i] = (in && yr) ? *reinterpret_cast<const float4*>(wb + c) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -491,7 +482,8 @@ __global__ __launch_bounds__(S32_THREADS) void normed_add_norm_kernel(T* __restr
         for (int i = 0; i < NAN_VEC; ++i) {
             const int c = 4 * (threadIdx.x + i * S32_THREADS);
             if (c >= hidden) continue;
-            const float a = xv[i].x * inv * wv[i].x, b = xv[i].y * inv * wv[i].y, cc = xv[i].z * inv * wv[i].z, d = xv[i].w * inv * wv[i].w;
+            const float4 wv = w ? *reinterpret_cast<const float4*>(w + c) : make_float4(1.f, 1.f, 1.f, 1.f);
+            const float a = xv[i].x * inv * wv.x, b = xv[i].y * inv * wv.y, cc = xv[i].z * inv * wv.z, d = xv[i].w * inv * wv.w;
             if constexpr (sizeof(T) == 2) {
                 uint2 packed = make_uint2(pack_bf16x2(a, b), pack_bf16x2(cc, d));
                 *reinterpret_cast<uint2*>(orow + c) = packed;
