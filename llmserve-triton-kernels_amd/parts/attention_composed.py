@@ -437,15 +437,26 @@ class ComposedAttention(Mixer):
                                kv, d, bs, window, self.scale, num_splits=splits, table_rows=batch.state_slots, head_gate=gate)
 
     def shares_long_keys(self, max_new: int, max_context: int) -> bool:
-        """Whether portions with mixed heads go to the kernel that mixes weights although the one that mixes results takes their
-        sizes.  The latter walks a block's keys in one workgroup, at 75 nanoseconds a key with 8 key/value heads and 40 with 4;
-        the former walks them twice, but in up to 4 shares, and while the columns of the portion fill one unit of 16 that is
-        less from some 1,500 keys on (microseconds, mixing results and weights: 8 heads of 64 on 8 of 32, 8 tokens behind 1,000
-        keys 84 and 89, 4,000 keys 307 and 221, 16,000 keys 1,179 and 862; 4 heads on 4 of 64 53 and 64, 172 and 152, 652 and 590;
-        with twice the tokens, two units, 318 and 416, 180 and 259 behind 4,000 keys; with 2 key/value heads 107 and 158)."""
-        reach = max_context if self.chunk is None else min(max_context, self.chunk)
-        return (self.talking and self.num_kv_heads >= 4 and max_new * (self.num_heads // self.num_kv_heads) <= 16
-                and self.num_heads <= 32 and reach >= 1500)
+        """Whether portions go to attend_composed_mfma although attend_composed_wide takes their sizes.  The latter walks the
+        keys of a block of columns in one wave (with mixed heads in one workgroup); the former deals them to 4 or 8 waves where
+        the columns of a portion fill one unit of 16 (with mixed heads to 4 workgroups, in two walks), which is less from some
+        number of keys on.  Microseconds, wide and mfma, a portion of 4 tokens (8 with mixed heads):
+          one map   16 heads of 64 on 4: behind 128 keys 8 and 9, 500 13 and 12, 1,000 23 and 17, 4,000 80 and 42; 32 heads of 128 on 8:
+                    behind 1,000 28 and 28, 4,000 94 and 78
+          two maps  4 heads of 64 on 4, values of 64: behind 1,000 keys 24 and 28, 4,000 84 and 72; keys of 128 never
+          mixed     8 heads of 64 on 8 of 32: behind 1,000 keys 84 and 89, 4,000 307 and 221, 16,000 1,179 and 862; 4 heads on 4 of
+                    64 53 and 64, 172 and 152, 652 and 590; with 2 key/value heads behind 4,000 107 and 158
+        and with twice the tokens, two units, behind 4,000 keys: mixed 318 and 416, 180 and 259.  (32 portions side by side
+        feel it from fewer keys on, 43 and 36 behind 1,000 with two maps, but 64 of them do not, 41 and 41.)"""
+        if max_new * (self.num_heads // self.num_kv_heads) > 16:
+            return False
+        reach = min(x for x in (max_context, self.chunk, None if self.window is None else self.window + self.keep_first + max_new)
+                    if x is not None)
+        if self.talking:
+            return self.num_kv_heads >= 4 and self.num_heads <= 32 and reach >= 1500
+        if self.maps == 2:
+            return self.head_dim <= 64 and reach >= 2000
+        return reach >= 500 * self.head_dim // 64
 
     def prompt_shares(self, n_requests: int, max_new: int, max_context: int, cus: int = 256) -> int:
         """Workgroups that share the keys of one block of prompt tokens when the heads' weights are mixed.  All heads

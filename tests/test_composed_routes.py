@@ -7,7 +7,7 @@ from llmserve.ops import library as ops
 from llmserve.parts.attention_composed import ComposedAttention
 
 
-def route(monkeypatch, heads, kv, new, context, n=1, n_dec=0, chunk=None, talking=True, dk=64, dv=32):
+def route(monkeypatch, heads, kv, new, context, n=1, n_dec=0, chunk=None, talking=True, maps=1, dk=64, dv=32, **params):
     """(kernel, first request, requests, most new tokens, shares) of every launch."""
     calls = []
     for name in ("attend_composed_wide", "attend_composed_mfma"):
@@ -17,7 +17,7 @@ def route(monkeypatch, heads, kv, new, context, n=1, n_dec=0, chunk=None, talkin
     monkeypatch.setattr(ops, "compute_units", lambda device: 256)
     monkeypatch.setattr(ops, "attend_composed_mfma_tokens", lambda *a: 16)
     part = ComposedAttention({"hidden": 64, "num_heads": heads, "num_kv_heads": kv, "head_dim": dk, "value_dim": dv, "chunk": chunk,
-                              "talking_heads": talking, "differential": not talking}, None)
+                              "talking_heads": talking, "differential": maps == 2, **params}, None)
     batch = SimpleNamespace(num_decode=n_dec, num_seqs=n + n_dec, max_count=new, max_context=context, max_decode_context=context,
                             state_slots=None, cu_seqlens=None, context_lens=None, num_tokens=n * new + n_dec)
     part.attend(None, SimpleNamespace(dtype=None, device=None), SimpleNamespace(k_pool=None, v_pool=None, block_size=16),
@@ -46,9 +46,17 @@ def test_single_tokens_beside_them_do_not_change(monkeypatch):
     assert decode[:4] == ("attend_composed_wide", 0, 3, 1) and portion[:4] == ("attend_composed_mfma", 3, 2, 8)
 
 
-def test_two_maps_have_one_walk_whatever_the_keys(monkeypatch):
-    (call,) = route(monkeypatch, 8, 8, 8, 16000, talking=False, dv=64)
-    assert call[0] == "attend_composed_wide"
+@pytest.mark.parametrize("heads,kv,maps,dk,new,context,params,kernel", [
+    (16, 4, 1, 64, 4, 1000, {}, "mfma"), (8, 8, 1, 64, 16, 500, {}, "mfma"), (8, 8, 1, 64, 16, 4000, {"window": 512}, "mfma"),
+    (32, 8, 1, 128, 4, 4000, {}, "mfma"), (4, 4, 2, 64, 16, 4000, {}, "mfma"),
+    (16, 4, 1, 64, 4, 300, {}, "wide"),     # few keys
+    (16, 4, 1, 64, 4, 4000, {"chunk": 256}, "wide"), (16, 4, 1, 64, 4, 4000, {"window": 100}, "wide"),
+    (16, 4, 1, 64, 5, 4000, {}, "wide"),    # more than one unit of columns
+    (32, 8, 1, 128, 4, 800, {}, "wide"), (4, 4, 2, 64, 16, 1000, {}, "wide"), (8, 8, 2, 128, 8, 16000, {}, "wide"),
+])
+def test_without_mixing_too(heads, kv, maps, dk, new, context, params, kernel, monkeypatch):
+    (call,) = route(monkeypatch, heads, kv, new, context, talking=False, maps=maps, dk=dk, dv=64, distance_slope_base=8, **params)
+    assert call[:4] == (f"attend_composed_{kernel}", 0, 1, new)
 
 
 def test_nothing_but_single_tokens_is_one_launch(monkeypatch):
