@@ -185,14 +185,20 @@ class LatentAttention(Mixer):
                                n_seqs=batch.num_seqs, max_count=batch.max_count, splits=splits, **common)
 
     def key_shares(self, n_requests: int, max_new: int, max_context: int, cus: int = 256, tokens: int | None = None) -> int:
-        """Workgroups that share the keys of one block of 64 (token, head) pairs.  While the blocks alone leave
+        """Workgroups that share the keys of one block of 128 (token, head) pairs.  While the blocks alone leave
         compute units idle (decoding, short portions), the tiles of 32 keys of each go to several workgroups, two
         tiles a share at least, and a second kernel adds the shares up.  A step of portions beside single tokens has the blocks
-        of its `tokens`, not the longest portion's for every request (456 tokens of 6 requests, 16 heads, behind up to 900
-        keys: 63 blocks and not 336, 111 microseconds in one share, 59 and 24 for adding up in 4)."""
+        of its `tokens`, not the longest portion's for every request, and its keys are shared out by those where that spares more
+        than writing and adding up the shares of every (token, head) pair costs: some 0.0125 r microseconds a tile against 7e-6 r
+        a pair and share (16 heads of 256 in 1, 4 shares: 448 tokens beside 5 behind 900 keys 90 and 76 microseconds, 200 beside 20
+        behind 1,500 142 and 59; 32 heads in 1, 2: 92 and 131, 144 and 101; 400 tokens beside 100 behind 400 46 and 79).  Not with
+        mostly single tokens, whose blocks may all lie on one XCD (60 tokens beside 60 behind 800 keys, in 1 and 3: 143 and 163)."""
         blocks = n_requests * -(-max_new * self.heads // ops.LATENT_MFMA_PAIRS)
-        if tokens is not None:
-            blocks = min(blocks, n_requests + tokens * self.heads // ops.LATENT_MFMA_PAIRS)
         reach = max_context if self.window is None else min(max_context, self.window + max_new - 1)
         tiles = -(-reach // ops.LATENT_MFMA_KEYS) + 1
-        return max(1, min(16, cus // max(blocks, 1), tiles // 2))
+        shares = max(1, min(16, cus // max(blocks, 1), tiles // 2))
+        if tokens is None or shares > 1 or tokens < 2 * n_requests:
+            return shares
+        pairs = tokens * self.heads
+        by_tokens = max(1, min(16, cus // (n_requests + pairs // ops.LATENT_MFMA_PAIRS), tiles // 2))
+        return by_tokens if tiles * (1 - 1 / by_tokens) > 5.4e-4 * pairs * by_tokens else 1

@@ -27,3 +27,19 @@ def test_blocks_times_shares_never_pass_the_compute_units():
             got = shares(heads, n, tokens, 4000, tokens)
             assert 1 <= got <= 16
             assert got == 1 or got * tokens * heads <= 256 * 128
+
+
+@pytest.mark.parametrize("heads,n,max_new,reach,tokens,expected", [
+    (16, 21, 200, 1500, 220, 5), (16, 13, 500, 3000, 512, 3), (32, 21, 200, 1500, 220, 3),  # measured: shared keys are the faster way
+    (32, 6, 448, 900, 453, 1), (32, 2, 400, 400, 500, 1), (32, 31, 30, 100, 60, 1),         # adding the shares up costs more
+    (128, 4, 100, 300, 103, 1), (128, 5, 40, 200, 44, 1),
+    (16, 61, 60, 800, 120, 1),                                                              # mostly single tokens
+])
+def test_shares_that_cost_more_than_they_spare_are_not_made(heads, n, max_new, reach, tokens, expected):
+    assert shares(heads, n, max_new, reach, tokens) == expected
+
+
+def test_where_the_longest_portion_leaves_compute_units_idle_nothing_changes():
+    for heads, n, max_new, reach, tokens in ((32, 8, 16, 4000, 23), (128, 8, 16, 4000, 23), (16, 4, 100, 300, 103), (8, 4, 500, 1000, 802)):
+        same = shares(heads, n, max_new, reach)
+        assert same > 1 and shares(heads, n, max_new, reach, tokens) == same
