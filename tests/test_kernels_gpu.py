@@ -253,6 +253,20 @@ def test_gemm32(m, n, k):
         ops().gemm32(whole, a.bfloat16().to(DEV), w.bfloat16().to(DEV))
 
 
+@pytest.mark.parametrize("n,k", [(512, 512), (2048, 2048), (333, 5632)])
+def test_gemm32_rows_in_other_company(n, k):
+    """Up to 64 rows of 512 columns and more are summed by several waves, more rows in the order of the columns: a row's result
+    depends on how many others come with it, by no more than either differs from 64 bits."""
+    a, w = rnd(65, k, seed=8), rnd(n, k, seed=9)
+    ref = a.double() @ w.double().t()
+    bound = 2e-6 * math.sqrt(k) * float(ref.abs().max())  # (as in test_gemm32)
+    rows = {m: ops().gemm32(torch.empty(m, n, device=DEV), a[:m].to(DEV), w.to(DEV)).cpu().double() for m in (1, 16, 17, 64, 65)}
+    for m, got in rows.items():
+        assert (got - ref[:m]).abs().max() <= bound
+        assert (got - rows[65][:m]).abs().max() <= bound
+    assert torch.equal(rows[65].float(), ops().gemm_fma(torch.empty(65, n, device=DEV), a.to(DEV), w.to(DEV)).cpu())
+
+
 @pytest.mark.parametrize("kernel,m", [("skinny", 1), ("skinny", 7), ("skinny", 16), ("skinny", 17), ("skinny", 33),
                                       ("skinny", 64), ("tile", 5), ("tile", 65), ("tile", 128), ("tile", 300)])
 @pytest.mark.parametrize("n,k", [(16, 64), (333, 96), (100, 176), (2056, 2048), (512, 5632)])
