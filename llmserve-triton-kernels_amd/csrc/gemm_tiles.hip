@@ -16,10 +16,12 @@
 // the fewer bytes of LDS per product (a 64 x 64 wave tile already asks LDS for as much as it can give), so the large tiles
 // run at 1.4 PFLOP/s in the loop and the small ones fill the chip when there are few rows.
 //
-// Measured (microseconds, weights from memory; in brackets the library's product, and with it the kernel behind):
-//   1.1B shape    333 rows: q, k, v 9 (12), o_proj in 2 parts 8 (12), gate and up with SiLU 28 (32 + 5), down_proj in 4 parts 16 (25)
-//                 512 rows: 10 (15), 9 (12), 31 (33 + 6), 22 (27);  2,048 rows: 26 (28), 20 (22), 87 (92 + 13), 50 (50 to 60)
-//   7B shape      330 rows: q, k, v 50 (56), o_proj 21 (26), down_proj 40 (60);  2,048 rows: gate and up 310 (402), down_proj 155 (167)
+// Measured (microseconds, weights from memory, the norm behind o_proj and down_proj included; in brackets the library's product
+// with the kernels behind it):
+//   1.1B shape    333 rows: q, k, v 11 (17), o_proj in 2 parts 14 (15), gate and up with SiLU 34 (36), down_proj in 4 parts 20 (24)
+//                 512 rows: 12 (20), 13 (16), 36 (38), 23 (25) in 2 parts;  2,048 rows: 28 (33), 27 (29), 95 (94), 59 (59)
+//   7B shape      333 rows: 54 (61), 27 (30), 77 (78), 48 (62);  512 rows: 57 (62), 32 (35), 107 (88), 57 (78);  2,048 rows: 185 (172), 71
+//                 (70), 314 (424), 160 (172)
 // What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times
 // its matrix instructions); beyond, LDS and matrix cores together, and how evenly the tiles fill 256 compute units.
 //

@@ -1453,8 +1453,8 @@ def attend_composed_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
 def attend_composed_wide_supported(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, heads: int, kv_heads: int, dk: int,
                                    dv: int, block_size: int, talk: bool) -> bool:
     """Whether `attend_composed_wide` takes this attention: bfloat16, keys of 64 or 128, pages of a multiple of 16 keys, aligned
-    rows; one token a request, or mixed heads; and 64, 128 or 256 columns of values for a score column: those of its key/value
-    head, with mixed heads those of all.  (With 512 a lane's results would need 128 registers, and 64 of 68 matrix instructions
+    rows; and 64 or 128 columns of values for a score column, those of its key/value head, or with mixed heads those of all, up to
+    256.  (With 512 a lane's results would need 128 registers, and 64 of 68 matrix instructions
     would be value products: the kernel that mixes weights has 1 in 3.)"""
     width = kv_heads * dv if talk else dv
     return (q.dtype == torch.bfloat16 and heads % kv_heads == 0 and heads // kv_heads <= 16 and dk in (64, 128) and dv % 16 == 0
@@ -1469,8 +1469,8 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
                          chunk: int = 0, slopes: torch.Tensor | None = None, talk: torch.Tensor | None = None,
                          lam: float = 0.0, head_norm: bool = False, eps: float = 0.0, out_scale: float = 1.0,
                          table_rows: torch.Tensor | None = None, sink: bool = False, shares: int = 1) -> torch.Tensor:
-    """`attend_composed_mfma` for one token a request (`max_new` = 1; their keys shared out to `shares` workgroups), and for
-    portions of prompts with mixed heads, in one walk over the keys: a head's weights meet the values of all key/value heads
+    """`attend_composed_mfma` for one token a request (`max_new` = 1; their keys shared out to `shares` workgroups) and for
+    portions of prompts, in one walk over the keys: with mixed heads a head's weights meet the values of all key/value heads
     and the results are mixed, not the weights.  Same arguments and results; see attend_composed_wide_supported."""
     dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, slopes, talk, table_rows)
     if not attend_composed_wide_supported(q, k_pool, v_pool, heads, kv_heads, dk, dv, block_size, talk is not None):

@@ -392,7 +392,8 @@ class ComposedAttention(Mixer):
         n_dec = batch.num_decode
         # one walk over the keys by a short kernel, and the results mixed, wherever it takes the sizes and a portion is not short
         # behind many keys (shares_long_keys): it was the faster one from 1 request to 256, 64 keys to 4,000 and 16 tokens to 2,048
-        # (13 against 25 microseconds for 4 decoding requests behind 1,000 keys, 27 against 152 for a prompt of 333)
+        # (13 against 25 microseconds for 4 decoding requests behind 1,000 keys, 27 against 152 for a prompt of 333); only mixed heads
+        # of some 200 single tokens and more behind fewer than 100 keys each lose up to a fifth (64 heads 36 and 32)
         wide = self.dist_bias is None and gate is None and not (self.talking and self.head_norm_eps is not None) and \
             ops.attend_composed_wide_supported(q, paged.k_pool, paged.v_pool, self.num_heads, self.num_kv_heads, self.head_dim,
                                                self.value_dim, paged.block_size, self.talking)
