@@ -87,17 +87,25 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 # Gated products of TILES_GATED_WORK and more against a weight below TILES_GATED_WEIGHT (200 MB, which the 256 MB memory-side cache
 # holds) are the tiles' again: 27 such products of 17 weights 0.95 in the mean, 0.72 to 1.19, where larger weights are at 1.05; 22016 x
 # 4096 at 2,048 rows 314 and 424.
+# Plain products of TILES_LONG_K columns and more whose tiles leave half the compute units without one are the library's, which
+# shares their K out (a bfloat16 result cannot come in parts, and each tile walks all of K): 65 such products of 9 weights, from 65 rows
+# on, 1.17 in the mean.  2048 x 5632 28 and 16 at 128 rows, 25 and 21 at 228, but 28 and 33 at 613; 1024 x 4096 13 and 9 at 96.
 TILES_WORK = {"plain": 18e9, "gated": 18e9, "rotary": 40e9, "parts": 60e9}
 TILES_GATED_WORK = 130e9
 TILES_GATED_WEIGHT = 100e6
+TILES_LONG_K = 4096
 
 
-def tiles_pay(kind: str, m: int, n: int, k: int) -> bool:
+def tiles_pay(kind: str, m: int, n: int, k: int, cus: int = 256) -> bool:
     """Whether m rows against a weight [n, k] are faster by ops.gemm_tiles ("plain", "gated" or "rotary" with what follows in the
     epilogue, "parts": K in parts for a norm to add up) than by the library: a rule by sizes alone."""
     work = m * n * k
     if kind == "gated" and work >= TILES_GATED_WORK and n * k < TILES_GATED_WEIGHT:
         return True
+    if kind == "plain" and m > 64 and k >= TILES_LONG_K:
+        rows, weight_rows = ops.GEMM_TILES[ops.gemm_tiles_plan(m, n, k, 1, cus)[0]][:2]
+        if 2 * -(-m // rows) * -(-n // weight_rows) <= cus:
+            return False
     return work < TILES_WORK[kind]
 
 
@@ -108,7 +116,7 @@ def tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def tiles_product(x: torch.Tensor, weight: torch.Tensor, kind: str = "plain") -> bool:
     """Whether a product of this kind goes there."""
-    return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or tiles_pay(kind, x.shape[0], *weight.shape))
+    return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or tiles_pay(kind, x.shape[0], *weight.shape, ops.compute_units(x.device)))
 
 
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and

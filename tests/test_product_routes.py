@@ -16,6 +16,9 @@ MEASURED = [  # kind, rows, weight [n, k], microseconds of the tiles and of the 
     ("rotary", 1024, 10240, 8192, 157, 142), ("rotary", 2048, 10240, 8192, 320, 275),
     ("plain", 333, 6144, 2048, 16, 20), ("plain", 2048, 6144, 2048, 57, 46), ("plain", 333, 4608, 2048, 12, 16),
     ("plain", 2048, 4608, 2048, 44, 40), ("plain", 1024, 12288, 4096, 101, 81), ("plain", 2048, 5120, 5120, 119, 103),
+    ("plain", 128, 2048, 5632, 28, 16), ("plain", 228, 2048, 5632, 25, 21), ("plain", 613, 2048, 5632, 28, 33),
+    ("plain", 128, 2048, 8192, 36, 22), ("plain", 96, 1024, 4096, 13, 9), ("plain", 560, 1024, 4096, 14, 18),
+    ("plain", 512, 2048, 4096, 15, 20), ("plain", 228, 2048, 2048, 9, 10),
     ("parts", 512, 4096, 11008, 57, 78), ("parts", 200, 8192, 28672, 159, 313), ("parts", 1024, 8192, 28672, 479, 375),
     ("parts", 1100, 8192, 8192, 182, 137), ("parts", 128, 2048, 5632, 13, 17),
 ]
