@@ -88,8 +88,8 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 # holds) are the tiles' again: 27 such products of 17 weights 0.95 in the mean, 0.72 to 1.19, where larger weights are at 1.05; 22016 x
 # 4096 at 2,048 rows 314 and 424.
 # Plain products of TILES_LONG_K columns and more whose tiles leave half the compute units without one are the library's, which
-# shares their K out (a bfloat16 result cannot come in parts, and each tile walks all of K): 65 such products of 9 weights, from 65 rows
-# on, 1.17 in the mean.  2048 x 5632 28 and 16 at 128 rows, 25 and 21 at 228, but 28 and 33 at 613; 1024 x 4096 13 and 9 at 96.
+# shares their K out (one result cannot come in parts, and each tile walks all of K): 65 such products of 9 weights, from 65 rows on,
+# 1.17 in the mean.  2048 x 5632 28 and 16 at 128 rows, 25 and 21 at 228, but 28 and 33 at 613; 1024 x 4096 13 and 9 at 96.
 TILES_WORK = {"plain": 18e9, "gated": 18e9, "rotary": 40e9, "parts": 60e9}
 TILES_GATED_WORK = 130e9
 TILES_GATED_WEIGHT = 100e6
