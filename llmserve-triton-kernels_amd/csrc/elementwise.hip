@@ -480,7 +480,7 @@ __global__ void silu_mul_bf16_vec_kernel(bf16* __restrict__ out, const bf16* __r
             const float u = bf16_bits_to_f32((uint16_t)(h ? uw[j] >> 16 : uw[j] & 0xffffu));
             r2[h] = UNIT == UNIT_CLAMPED ? clamped_unit(g, u, limit)
                     : UNIT == UNIT_GELU  ? gelu_tanh(g) * u
-                                         : round_to<bf16>(g / (1.f + expf(-g))) * u;
+                                         : round_to<bf16>(silu_of_bf16(g)) * u;
         }
         ow[j] = pack_bf16x2(r2[0], r2[1]);
     }

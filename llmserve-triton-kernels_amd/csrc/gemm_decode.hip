@@ -217,7 +217,7 @@ __device__ __forceinline__ void gd_finish_pair(const DecodeGemmArgs& a, int m, i
             return;
         }
         const float gate = gd_bfr(lo), up = gd_bfr(hi);
-        gd_store<TOut>(reinterpret_cast<TOut*>(a.C) + (size_t)m * a.ldc + u, gd_bfr(gate / (1.f + expf(-gate))) * up);
+        gd_store<TOut>(reinterpret_cast<TOut*>(a.C) + (size_t)m * a.ldc + u, gd_bfr(silu_of_bf16(gate)) * up);
         return;
     }
     const int nh = a.n_heads, nkv = a.n_kv_heads, D = a.head_dim, half = D / 2, bs = a.block_size;

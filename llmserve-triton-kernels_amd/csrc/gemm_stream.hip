@@ -229,7 +229,7 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void gemm_stream_kernel(const Stream
                 return;
             }
             const float gate = bfr(lo), up = bfr(hi);
-            store_out<TOut>(C + (size_t)m * a.ldc + f, bfr(gate / (1.f + expf(-gate))) * up);
+            store_out<TOut>(C + (size_t)m * a.ldc + f, bfr(silu_of_bf16(gate)) * up);
         }
     } else {
         const int nh = a.n_heads, nkv = a.n_kv_heads, bs = a.block_size;

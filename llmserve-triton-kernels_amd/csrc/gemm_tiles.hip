@@ -32,6 +32,7 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 #define GT_PLAIN 0
 #define GT_FLOAT 1  // plain or parts, 32-bit result
@@ -53,6 +54,7 @@ struct TilesArgs {
     const float* angles;         // [M][head_dim / 2] (sine, cosine), or null: nothing turns
     const int* slots;            // or null: nothing is stored
     bf16 *k_pool, *v_pool;
+    int wide;                    // PLAIN, GATED: rows of C start on 16 bytes, not only on 8
 };
 
 template <int N>
@@ -80,14 +82,41 @@ __device__ __forceinline__ void gt_store4(bf16* p, float a, float b, float c, fl
     *reinterpret_cast<u32x2*>(p) = (u32x2){pack_bf16x2(a, b), pack_bf16x2(c, d)};
 }
 
-__device__ __forceinline__ float gt_unit(const TilesArgs& a, float gate, float up) {
-    if (a.unit == 1) {
-        const float g = fminf(gate, a.limit), v = fminf(fmaxf(up, -a.limit), a.limit);
-        return g / (1.f + expf(-1.702f * g)) * (v + 1.f);
+// 16 bytes of a result's row; `wide`: rows start on 16 bytes, not on 8
+__device__ __forceinline__ void gt_store16(void* p, u32x4 v, int wide) {
+    if (wide) {
+        *reinterpret_cast<u32x4*>(p) = v;
+    } else {
+        reinterpret_cast<u32x2*>(p)[0] = (u32x2){v[0], v[1]};
+        reinterpret_cast<u32x2*>(p)[1] = (u32x2){v[2], v[3]};
     }
-    if (a.unit == 3) return gelu_tanh(gate) * up;
-    gate = round_to<bf16>(gate);  // (the projections' results and SiLU are bfloat16 before they are multiplied)
-    return round_to<bf16>(gate / (1.f + expf(-gate))) * round_to<bf16>(up);
+}
+
+// Four units at once.  (UNIT is a constant: with a branch on it around every unit the compiler works one after the other, each a
+// chain of some 35 instructions.)
+template <int UNIT>
+__device__ __forceinline__ u32x2 gt_units(const TilesArgs& a, const f32x4& gate, const f32x4& up) {
+    float y[4];
+    if constexpr (UNIT == 0) {  // (the projections' results and SiLU are bfloat16 before they are multiplied)
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+            const uint32_t g = pack_bf16x2(gate[r], gate[r + 1]), u = pack_bf16x2(up[r], up[r + 1]);
+            const uint32_t s = pack_bf16x2(silu_of_bf16(__uint_as_float(g << 16)), silu_of_bf16(__uint_as_float(g & 0xffff0000u)));
+            y[r] = __uint_as_float(s << 16) * __uint_as_float(u << 16);
+            y[r + 1] = __uint_as_float(s & 0xffff0000u) * __uint_as_float(u & 0xffff0000u);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (UNIT == 1) {
+                const float g = fminf(gate[r], a.limit), v = fminf(fmaxf(up[r], -a.limit), a.limit);
+                y[r] = g / (1.f + expf(-1.702f * g)) * (v + 1.f);
+            } else {
+                y[r] = gelu_tanh(gate[r]) * up[r];
+            }
+        }
+    }
+    return (u32x2){pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
 }
 
 template <int BM, int BN, int WM, int WN, int S, int EPI>
@@ -313,20 +342,11 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
         }
         return;
     }
+    if constexpr (EPI == GT_FLOAT) {
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-        const int m = m0 + wm + j * 16 + r16;
-        if (m >= a.M) continue;
-        if constexpr (EPI == GT_GATED) {
-#pragma unroll
-            for (int i = 0; i < TN; i += 2) {
-                const int n = (n0 + wn) / 2 + i * 8 + g * 4;
-                if (n >= a.inter) continue;
-                const f32x4 lo = acc[i][j], hi = acc[i + 1][j];
-                gt_store4(reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + n, gt_unit(a, lo[0], hi[0]), gt_unit(a, lo[1], hi[1]),
-                          gt_unit(a, lo[2], hi[2]), gt_unit(a, lo[3], hi[3]));
-            }
-        } else {
+        for (int j = 0; j < TM; ++j) {
+            const int m = m0 + wm + j * 16 + r16;
+            if (m >= a.M) continue;
 #pragma unroll
             for (int i = 0; i < TN; ++i) {
                 const int n = n0 + wn + i * 16 + g * 4;
@@ -336,11 +356,67 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
 #pragma unroll
                     for (int r = 0; r < 4; ++r) s[r] += bf16_bits_to_f32(a.bias[n + r].bits);
                 }
-                if constexpr (EPI == GT_FLOAT)
-                    *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.C) + part * a.part_stride + (size_t)m * a.ldc + n) = s;
-                else
-                    gt_store4(reinterpret_cast<bf16*>(a.C) + (size_t)m * a.ldc + n, s[0], s[1], s[2], s[3]);
+                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.C) + part * a.part_stride + (size_t)m * a.ldc + n) = s;
             }
+        }
+        return;
+    }
+    // bfloat16 rows go through LDS, a chunk of JC blocks of rows at a time, and leave in 16-byte pieces along whole rows of the
+    // tile: as the lanes hold them (8 bytes of 16 rows an instruction) a matrix of 2,048 x 5,632 takes 11.2 microseconds to
+    // store, in pieces along rows 5.6.  (32-bit rows have 64 bytes together as the lanes hold them: through LDS 17.3 microseconds for
+    // 512 rows of 2048 x 2048, directly 17.0.)  With four units worked out side by side gate and up of the 1.1B shape went from 33.8
+    // to 29.1 microseconds at 333 rows, from 37.2 to 31.9 at 512, and from 117.7 to 98.4 at 2,048 (tiles of 160 x 192).
+    constexpr int ROW = EPI == GT_GATED ? BN : BN * 2, PITCH = ROW + 16;  // bytes
+    constexpr int FIT = TILE / (WM * 16 * PITCH), JC = FIT < TM ? FIT : TM, CHUNKS = (TM + JC - 1) / JC;
+    static_assert(JC > 0, "a block of rows fits");
+    constexpr int RC = WM * JC * 16, PP = ROW / 16, THREADS = NW * LLMS_WAVE;
+    const int left = EPI == GT_GATED ? a.inter - n0 / 2 : a.N - n0;  // columns from the tile's first on
+    bf16* const first_row = reinterpret_cast<bf16*>(a.C) + (size_t)m0 * a.ldc + (EPI == GT_GATED ? n0 / 2 : n0);
+#pragma unroll
+    for (int chunk = 0; chunk < CHUNKS; ++chunk) {
+        const int j0 = chunk * JC;
+        uint8_t* const stage = chunk % 2 ? lds1 : lds0;
+        uint8_t* const mine = stage + ((wave % WM) * (JC * 16) + r16) * PITCH;
+        if constexpr (EPI == GT_GATED) {
+            auto units = [&](auto unit) {
+#pragma unroll
+                for (int j = j0; j < j0 + JC && j < TM; ++j)
+#pragma unroll
+                    for (int i = 0; i < TN; i += 2)
+                        *reinterpret_cast<u32x2*>(mine + (j - j0) * 16 * PITCH + (wn / 2 + i * 8 + g * 4) * 2) =
+                            gt_units<decltype(unit)::n>(a, acc[i][j], acc[i + 1][j]);
+            };
+            if (a.unit == 0) units(Number<0>());
+            else if (a.unit == 1) units(Number<1>());
+            else units(Number<3>());
+        } else {
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const int n = n0 + wn + i * 16 + g * 4;
+                f32x4 b = (f32x4){0.f, 0.f, 0.f, 0.f};
+                if (a.bias && n < a.N) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) b[r] = bf16_bits_to_f32(a.bias[n + r].bits);
+                }
+#pragma unroll
+                for (int j = j0; j < j0 + JC && j < TM; ++j) {
+                    const f32x4 s = acc[i][j] + b;
+                    *reinterpret_cast<u32x2*>(mine + (j - j0) * 16 * PITCH + (wn + i * 16 + g * 4) * 2) =
+                        (u32x2){pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+                }
+            }
+        }
+        // (LDS alone is waited for: stores to memory stay in flight)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int k = 0; k < (RC * PP + THREADS - 1) / THREADS; ++k) {
+            const int p = tid + k * THREADS, r = p / PP, q = p % PP, within = r % (JC * 16);
+            const int row = r / (JC * 16) * (BM / WM) + j0 * 16 + within;  // (of the tile; the last chunk may have fewer blocks)
+            if (p >= RC * PP || j0 * 16 + within >= TM * 16 || m0 + row >= a.M || q * 8 >= left) continue;
+            gt_store16(first_row + (size_t)row * a.ldc + q * 8, *reinterpret_cast<const u32x4*>(stage + r * PITCH + q * 16), a.wide);
         }
     }
 }
@@ -390,6 +466,7 @@ int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* 
     a.ldx = ldx;
     a.ldc = ldc;
     a.part_stride = part_stride;
+    a.wide = ldc % 8 == 0 && (uintptr_t)C % 16 == 0;
     if (epilogue == GT_GATED) {
         LLMS_REQUIRE(N % 32 == 0 && bias == nullptr, "gemm_tiles: the gated epilogue takes blocks of 16 units and no bias");
         LLMS_REQUIRE(unit == 0 || unit == 1 || unit == 3, "gemm_tiles: unit 0, 1 or 3");

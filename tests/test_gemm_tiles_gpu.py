@@ -125,6 +125,57 @@ def test_rotary(tile, nh, nkv, d, bs, bias):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("pad", [0, 4, 8])
+def test_rows_of_every_alignment(tile, pad):
+    """Results leave in 16-byte pieces along rows, or in 8-byte ones where rows do not start on 16: the same numbers, and none
+    beside them."""
+    bm, bn, step = sizes_of(tile)
+    m, n, k = bm + 19, bn + 32, step
+    x, w = rnd(m, k, seed=11).to(DEV), rnd(n, k, seed=12, scale=k ** -0.5).to(DEV)
+    want = product(x.cpu(), w.cpu())
+    for dtype in (torch.bfloat16, torch.float32):
+        out = torch.full((m + 1, n + pad), 7.0, dtype=dtype, device=DEV)
+        ops().gemm_tiles(out[:m, :n], x, w, tile=tile)
+        close(out[:m, :n], want, k, dtype == torch.bfloat16)
+        assert bool((out[m:] == 7.0).all()) and bool((out[:, n:] == 7.0).all())
+    wide = ops().gemm_tiles(torch.empty(m, n, dtype=torch.bfloat16, device=DEV), x, w, tile=tile)
+    out = torch.full((m + 1, n // 2 + pad), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_tiles(out[:m, :n // 2], x, w, swiglu=True, tile=tile)
+    assert torch.equal(out[:m, :n // 2], ops().silu_mul(torch.empty(m, n // 2, dtype=torch.bfloat16, device=DEV), wide))
+    assert bool((out[m:] == 7.0).all()) and bool((out[:, n // 2:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("bs,first,pad", [(16, 0, 0), (16, 8, 8), (16, 5, 0), (24, 8, 4), (20, 0, 0)])
+def test_rotary_values_in_runs(tile, bs, first, pad):
+    """8 tokens side by side in a page leave in one piece where they start on 8 and the page is of eights, on their own
+    otherwise; several heads a tile, and a tile between q, k and v: to the bit what the rotation's own kernel stores."""
+    bm, _, step = sizes_of(tile)
+    m, k, nh, nkv, d = bm + 40, step, 5, 3, 64
+    n = (nh + 2 * nkv) * d
+    x, w = rnd(m, k, seed=13).to(DEV), rnd(n, k, seed=14, scale=k ** -0.5).to(DEV)
+    positions = torch.arange(m, dtype=torch.int32, device=DEV)
+    inv_freq = (1.0 / (1e4 ** (torch.arange(0, d, 2, dtype=torch.float32) / d))).to(DEV)
+    pages = -(-(m + first) // bs) + 1
+    slots = torch.arange(first, m + first, dtype=torch.int32)
+    slots[9] = -1                                       # a hole in a run
+    slots[24:32] = torch.flip(slots[24:32], [0])        # eight tokens backwards
+    slots = slots.to(DEV)
+    pools = [torch.full(shape, 7.0, dtype=torch.bfloat16, device=DEV)
+             for shape in ((pages, nkv, bs, d), (pages, nkv, d, bs)) for _ in range(2)]
+    qkv = ops().gemm_tiles(torch.empty(m, n, dtype=torch.bfloat16, device=DEV), x, w, tile=tile)
+    ops().rope_store(qkv, inv_freq, positions, slots, pools[0], pools[2], nh, nkv, d, bs)
+    q = torch.full((m, nh * d + pad), 7.0, dtype=torch.bfloat16, device=DEV)
+    rope = dict(n_heads=nh, n_kv_heads=nkv, head_dim=d, inv_freq=inv_freq, positions=positions, slots=slots, k_pool=pools[1],
+                v_pool=pools[3], block_size=bs)
+    ops().gemm_tiles(q[:, :nh * d], x, w, rope=rope, tile=tile)
+    assert torch.equal(q[:, :nh * d], qkv[:, :nh * d]) and bool((q[:, nh * d:] == 7.0).all())
+    assert torch.equal(pools[0], pools[1]) and torch.equal(pools[2], pools[3])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("what", ["plain", "columns of a wider weight", "transposed weight", "every other column of x", "one row many times",
                                   "no weight rows", "no columns", "32-bit bias", "every other number of a bias", "bias of one number",
                                   "bias of rows", "every other column of out", "transposed out"])

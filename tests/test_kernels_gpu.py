@@ -219,6 +219,21 @@ def test_silu_mul(dtype, inter):
     assert (out.float().cpu() - ref).abs().max() <= ulp(dtype, ref)
 
 
+def test_silu_of_every_bfloat16():
+    """silu of all 65,536 numbers: half a step of bfloat16 (8 bits: up to 2^-8 of the value), a few
+    roundings of 32-bit arithmetic, and 89 * 2^-128 < 2^-121 where exp(-x) is beyond 2^128 and the result 0; infinities and NaN as the formula
+    gives them."""
+    x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    rows = torch.stack([x.view(8, -1), torch.ones(8, 8192, dtype=torch.bfloat16)], 1).reshape(8, -1).contiguous()
+    got = ops().silu_mul(torch.empty(8, 8192, dtype=torch.bfloat16, device=DEV), rows.to(DEV)).cpu().reshape(-1).double()
+    x = x.double()
+    want = x / (1 + torch.exp(-x))
+    odd = want.isnan() | want.isinf()
+    assert int(odd.sum()) == 2 * 127 + 2  # (NaN of both signs and the infinities)
+    assert torch.equal(got[odd].isnan(), want[odd].isnan()) and bool((got[x == math.inf] == math.inf).all())
+    assert ((got - want).abs() <= (2.0 ** -8 + 2.0 ** -19) * want.abs() + 2.0 ** -121)[~odd].all()
+
+
 # ------------------------------------------------------------------ matrix products
 @pytest.mark.parametrize("m,n,k", [(1, 256, 64), (5, 333, 96), (64, 100, 176), (130, 65, 17), (300, 513, 1000)])
 def test_gemm_fma(m, n, k):
