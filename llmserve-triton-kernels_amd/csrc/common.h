@@ -56,6 +56,32 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, v);
 }
 
+// A weight that a kernel further on reads, for workgroups of a kernel that leaves memory and compute units idle to bring nearer: into the
+// 256 MB memory-side cache.
+struct Near {
+    const void* from;
+    unsigned bytes;  // (the host checks: below 2 GB)
+    int workers;     // workgroups that do so, behind those of the kernel's own work; 0: none
+};
+
+// Worker `at` of them, NW waves: a number of every 128-byte line goes to LDS, where nobody looks at it; `lds`: 256 bytes per wave.  Reads
+// stay inside the weight (its buffer descriptor), nothing is written to memory.
+template <int NW>
+__device__ __forceinline__ void bring_near(const Near& n, int at, void* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(n.from), 0, n.bytes, 0x00020000);
+    const unsigned piece = LLMS_WAVE * 128u, stride = (unsigned)(n.workers * NW) * piece;  // (up to 2^30: no offset wraps)
+    for (unsigned o = (unsigned)(at * NW + wave) * piece; o < n.bytes; o += stride)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)((char*)lds + wave * 256), 4, o + lane * 128u, 0, 0, 0);
+    __builtin_amdgcn_s_waitcnt(0);  // (no load may find the workgroup gone)
+#endif
+}
+
+#define LLMS_REQUIRE_NEAR(n)                                                                                              \
+    LLMS_REQUIRE((n).workers >= 0 && (n).workers <= 4096 && ((n).workers == 0 || ((n).from && (uintptr_t)(n).from % 4 == 0 && (n).bytes < (1u << 31))), \
+                 "up to 4,096 workgroups bring up to 2 GB nearer, aligned to 4 bytes")
+
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(bf16 v) { return bf16_bits_to_f32(v.bits); }
 

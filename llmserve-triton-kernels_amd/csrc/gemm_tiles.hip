@@ -25,6 +25,8 @@
 // What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times
 // its matrix instructions); beyond, LDS and matrix cores together, and how evenly the tiles fill 256 compute units.
 //
+// Compute units without a tile bring a weight that a later kernel multiplies with nearer (`near`).
+//
 // K must be a multiple of 64 (the host checks), N of 16, rows of X and W 16-byte aligned; M is arbitrary: rows beyond M
 // are read as zeros or as row 0 and never stored.
 #include "common.h"
@@ -46,6 +48,7 @@ struct TilesArgs {
     void* C;
     int M, N, K, ldx, ldc;
     int tiles_m, tiles;          // tiles along M, tiles in all (of one part)
+    int workgroups;              // of the tiles in all parts
     int steps;                   // of 64 columns, of one part
     long long part_stride;       // elements from one part's sums to the next's
     int inter, unit;             // GATED; unit 0 SiLU, 1 clamped, 3 gelu
@@ -55,6 +58,7 @@ struct TilesArgs {
     const int* slots;            // or null: nothing is stored
     bf16 *k_pool, *v_pool;
     int wide;                    // PLAIN, GATED: rows of C start on 16 bytes, not only on 8
+    Near near;                   // for the workgroups behind those of the tiles
 };
 
 template <int N>
@@ -119,6 +123,12 @@ __device__ __forceinline__ u32x2 gt_units(const TilesArgs& a, const f32x4& gate,
     return (u32x2){pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
 }
 
+// Workgroups beyond those of the tiles bring a weight that a later kernel multiplies with nearer (`near`).  A tile's loads are
+// answered in order, those of weights from memory hold up those of rows from L2 behind them, and no depth of fetching ahead made
+// up for it (buffers of 4, 5 and 6 steps: the same times); with its weight in the memory-side cache 2048 x 5632 at 512 rows in 2
+// parts takes 17.1 microseconds where it takes 22.9 from memory, 2048 x 2048 8.9 and 11.8.  A layer's four products of the 1.1B shape at
+// 512 rows: 93.7 microseconds, 85.8 where q, k, v bring o_proj's weight (16 compute units without a tile) and gate and up
+// down_proj's (20).  What bounds a worker is what a compute unit has of misses in flight: 57 GB/s.
 template <int BM, int BN, int WM, int WN, int S, int EPI>
 __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const TilesArgs a) {
     constexpr int NW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
@@ -241,6 +251,15 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
         __builtin_amdgcn_sched_barrier(0);
         ++step;
     };
+    // (Here and not at the start: behind a branch there the arguments would be asked for a second time, 0.4 microseconds a launch; what
+    // a worker has worked out so far is in bounds and not used.  Products that come in parts have no workers, and were 0.4 slower with
+    // this code in their kernel.)
+    if constexpr (EPI == GT_GATED || EPI == GT_ROTARY) {
+        if (__builtin_expect((int)blockIdx.x >= a.workgroups, 0)) {
+            bring_near<NW>(a.near, blockIdx.x - a.workgroups, lds0);
+            return;
+        }
+    }
     fetch(lds0, 0);
     fetch(lds1, 1);
     if constexpr (S > 2) fetch(lds2, 2);
@@ -430,7 +449,9 @@ static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
     a.tiles = a.tiles_m * tiles_n;
     a.steps = (a.K / 64 + parts - 1) / parts;
     LLMS_REQUIRE((long long)(parts - 1) * a.steps < a.K / 64, "gemm_tiles: a part of K is empty");
-    const dim3 grid((unsigned)(a.tiles * parts)), block(WM * WN * LLMS_WAVE);
+    a.workgroups = a.tiles * parts;
+    LLMS_REQUIRE((long long)a.workgroups + a.near.workers < (1ll << 31), "gemm_tiles: too many workgroups");
+    const dim3 grid((unsigned)(a.workgroups + a.near.workers)), block(WM * WN * LLMS_WAVE);
     if (epilogue == GT_PLAIN) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_PLAIN><<<grid, block, 0, stream>>>(a);
     else if (epilogue == GT_FLOAT) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_FLOAT><<<grid, block, 0, stream>>>(a);
     else if (epilogue == GT_GATED) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_GATED><<<grid, block, 0, stream>>>(a);
@@ -442,9 +463,11 @@ extern "C" {
 
 // epilogue: 0 plain bfloat16, 1 plain float (parts > 1: `parts` arrays of sums, part_stride elements apart), 2 gated, 3 rotary.
 // tile: a place in the table of ops/library.py (GEMM_TILES).
+// near_workers (gated, rotary): that many workgroups more bring `near_bytes` of `near` nearer.
 int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* W, const void* bias, int M, int N, int K, int ldx,
                     int ldc, int parts, long long part_stride, int unit, float limit, int n_heads, int n_kv_heads, int head_dim,
-                    int block_size, const float* angles, const int* slots, void* k_pool, void* v_pool, hipStream_t stream) {
+                    int block_size, const float* angles, const int* slots, void* k_pool, void* v_pool, const void* near,
+                    unsigned near_bytes, int near_workers, hipStream_t stream) {
     LLMS_REQUIRE(M > 0 && N > 0 && K > 0 && parts > 0, "gemm_tiles: sizes must be positive");
     LLMS_REQUIRE(N % 16 == 0 && ldx % 8 == 0 && ldx >= K, "gemm_tiles: N in multiples of 16, rows of X of multiples of 8");
     LLMS_REQUIRE((uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0, "gemm_tiles: X and W must be 16-byte aligned");
@@ -466,6 +489,9 @@ int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* 
     a.ldx = ldx;
     a.ldc = ldc;
     a.part_stride = part_stride;
+    a.near = Near{near, near_bytes, near_workers};
+    LLMS_REQUIRE_NEAR(a.near);
+    LLMS_REQUIRE(near_workers == 0 || epilogue == GT_GATED || epilogue == GT_ROTARY, "gemm_tiles: workers go with the gated and rotary epilogues");
     a.wide = ldc % 8 == 0 && (uintptr_t)C % 16 == 0;
     if (epilogue == GT_GATED) {
         LLMS_REQUIRE(N % 32 == 0 && bias == nullptr, "gemm_tiles: the gated epilogue takes blocks of 16 units and no bias");

@@ -636,6 +636,42 @@ def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256)
     return best[1:]
 
 
+def _near_bytes(near: torch.Tensor) -> int:
+    """Bytes of a weight that is to be brought nearer; 0 where it starts between two words (it stays where it is)."""
+    if not near.is_contiguous():
+        raise ValueError("near must be contiguous")
+    return 0 if near.data_ptr() % 4 else min(near.numel() * near.element_size(), (1 << 31) - 1)
+
+
+# What a compute unit without a tile brings from memory, bytes a microsecond (10 and 20 of them: 60 and 57 GB/s each); up to which
+# weight that is done, and up to how many bytes a microsecond of both products' weights.
+GEMM_TILES_WORKER_RATE = 57e3
+GEMM_TILES_NEAR_BYTES = 40e6
+GEMM_TILES_NEAR_RATE = 2.9e6
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: int, cus: int = 256) -> int:
+    """How many workgroups beyond those of the tiles bring a weight of `nbytes` nearer: as many as do so in four fifths of a round's
+    time, if there are as many compute units without a tile in the last round and memory has time for both weights; otherwise none.
+    Time saved in both products together, microseconds: gate and up with down_proj behind them (1.1B shape, 23 MB) 4.7 at 512 rows, 6.8
+    at 560, 3.1 at 700; q, k, v with o_proj (8 MB) 1.3 at 512, 2.3 at 593, 5.7 at 2,048.  A part of a weight gains nothing, since the
+    last tile decides (8 of 23 MB: -0.1 at 333 rows, -0.8 at 512); a large one gets in the way of the tiles' own (down_proj of the 7B
+    shape, 90 MB: -10.7 at 330 rows, -4.6 at 448), and so does any where the tiles themselves wait for memory (gate and up at 333 rows
+    take 2.2 more, down_proj 2.2 less).  With more workers than there are such compute units each would take a tile's place or be a
+    round of its own.  A rule by sizes alone."""
+    if not 0 < nbytes <= GEMM_TILES_NEAR_BYTES:
+        return 0
+    bm, bn, held, stages, one, full = GEMM_TILES[tile]
+    rounds, rest = divmod(-(-m // bm) * -(-n // bn) * parts, held * cus)
+    steps = -(-(-(-(k // 64) // parts)) // stages) * stages
+    last = steps * (one if rounds == 0 else full) + 2.0
+    idle = cus - rest if 0 < rest < cus else 0
+    if idle * GEMM_TILES_WORKER_RATE * last < nbytes or 2 * n * k + nbytes > GEMM_TILES_NEAR_RATE * (rounds * steps * full + last):
+        return 0
+    return min(idle, -(-nbytes // int(0.8 * GEMM_TILES_WORKER_RATE * last)))
+
+
 def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 64, blocks of 16 weight rows, rows of x of 16-byte pieces
     that do not overlap, a contiguous w, and neither without columns or rows."""
@@ -645,7 +681,8 @@ def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *, swiglu: bool = False,
-               rope: dict | None = None, limit: float | None = None, gelu: bool = False, tile: int | None = None) -> torch.Tensor:
+               rope: dict | None = None, limit: float | None = None, gelu: bool = False, tile: int | None = None,
+               near: torch.Tensor | None = None) -> torch.Tensor:
     """The product of many bfloat16 rows, and what follows it fused in.
 
     plain:   out[M, N] = x w^T (+ bias), bfloat16 or float32; float32 [parts, M, N]: the sums of that many parts of K.
@@ -653,8 +690,10 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
              `silu_mul` (in 32-bit, rounded once).
     rope:    as for `gemm_decode` (head_dim a multiple of 32): out[M, n_heads * head_dim] = rotated q, rotated k and v go to
              the tokens' cache slots.
-    `tile`: a place in GEMM_TILES; default by gemm_tiles_plan."""
-    dev = _dev(out, x, w, bias)
+    `tile`: a place in GEMM_TILES; default by gemm_tiles_plan.
+    `near` (with swiglu or rope): a contiguous weight that a kernel after this one reads: compute units without a tile bring it into the memory-side
+            cache meanwhile, where that pays (gemm_tiles_workers).  No result depends on it."""
+    dev = _dev(out, x, w, bias, near)
     if x.dim() != 2 or x.stride(1) != 1 or out.dim() not in (2, 3) or out.stride(-1) != 1:
         raise ValueError("x must be 2-d, x and out with unit inner stride")
     _rows(w, "w", x.shape[1])
@@ -709,12 +748,18 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
         return out
     if tile is None:
         tile = gemm_tiles_plan(m, n, k, 1, compute_units(dev))[0] if parts == 1 else _tile_for_parts(m, n, k, parts, compute_units(dev))
+    workers = near_bytes = 0
+    if near is not None:
+        if epilogue not in (2, 3):
+            raise ValueError("near goes with the gated and the rotary epilogue")
+        near_bytes = _near_bytes(near)
+        workers = gemm_tiles_workers(tile, m, n, k, parts, near_bytes, compute_units(dev))
     _check(load("gemm_tiles").llms_gemm_tiles(
         c_int(tile), c_int(epilogue), _ptr(out), _ptr(x), _ptr(w), _ptr(bias), c_int(m), c_int(n), c_int(k), c_int(x.stride(0)),
         c_int(out.stride(-2)), c_int(parts), ctypes.c_longlong(part_stride), c_int(_gated_unit(limit, gelu)),
         c_float(0.0 if limit is None else limit), c_int(r["n_heads"]), c_int(r["n_kv_heads"]), c_int(r["head_dim"]),
-        c_int(r["block_size"]), _ptr(r["angles"]), _ptr(r["slots"]), _ptr(r["k_pool"]), _ptr(r["v_pool"]), _stream(dev)),
-        "gemm_tiles")
+        c_int(r["block_size"]), _ptr(r["angles"]), _ptr(r["slots"]), _ptr(r["k_pool"]), _ptr(r["v_pool"]),
+        _ptr(near), ctypes.c_uint(near_bytes), c_int(workers), _stream(dev)), "gemm_tiles")
     return out
 
 

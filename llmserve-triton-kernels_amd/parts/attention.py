@@ -130,7 +130,7 @@ class Attention(Mixer):
             if angles is not None and getattr(batch, "shared", None) is not None:
                 rope["angles"] = angles(batch)  # worked out once per step, not once per layer and workgroup
             if tiles:
-                ops.gemm_tiles(q, rows, self.qkv_weight, self.qkv_bias, rope=rope)
+                ops.gemm_tiles(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, near=self.o_weight)
             else:
                 ops.gemm_decode(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, norm=norm)
         else:

@@ -67,7 +67,7 @@ class SwiGLU(FeedForward):
             if few and ops.gemm_bf16_supported(rows, self.gate_up):
                 ops.gemm_stream(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # activation in the product's epilogue
             elif not few and self.intermediate % 16 == 0 and tiles_product(rows, self.gate_up, "gated"):
-                ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # the same
+                ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu, near=self.down)  # the same
             else:
                 ops.silu_mul(act, linear(rows, self.gate_up), self.limit, self.gelu)
         if deferred and x.may_add_in_place and adds_residual_in_epilogue(act, self.down):

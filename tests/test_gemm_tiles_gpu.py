@@ -253,3 +253,34 @@ def test_plan():
                 assert 0 <= tile < len(ops().GEMM_TILES) and 1 <= parts <= most
                 assert (parts - 1) * -(-(k // 64) // parts) < k // 64
     assert ops().gemm_tiles_plan(128, 2048, 5632, 4)[1] == 4 and ops().gemm_tiles_plan(2048, 2048, 2048, 4)[1] == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("epilogue", ["gated", "rotary"])
+@pytest.mark.parametrize("m,rows", [(512, 2048), (560, 2047), (700, 1), (512, 33), (512, 9000), (333, 2048)])
+def test_a_weight_brought_nearer_changes_nothing(epilogue, m, rows):
+    """Compute units without a tile read a weight of `rows` rows meanwhile (more, fewer and odd numbers of pieces, too large a one, none
+    where all have a tile): the same bits, and the weight as it was."""
+    k, nh, nkv, d = 2048, 32, 4, 64
+    near = rnd(rows, k, seed=21).to(DEV)
+    before, x = near.clone(), rnd(m, k, seed=22).to(DEV)
+    n = 2 * 5632 if epilogue == "gated" else (nh + 2 * nkv) * d
+    w = rnd(n, k, seed=23, scale=k ** -0.5).to(DEV)
+    rope = dict(n_heads=nh, n_kv_heads=nkv, head_dim=d, inv_freq=None, positions=None, slots=None, k_pool=None, v_pool=None, block_size=16)
+    form = dict(swiglu=True) if epilogue == "gated" else dict(rope=rope)
+    outs = [ops().gemm_tiles(torch.empty(m, 5632 if epilogue == "gated" else nh * d, dtype=torch.bfloat16, device=DEV), x, w, near=v, **form)
+            for v in (None, near, near[rows // 2:])]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2]) and torch.equal(near, before)
+    tile = ops().gemm_tiles_plan(m, n, k)[0]
+    workers = ops().gemm_tiles_workers(tile, m, n, k, 1, near.numel() * 2, ops().compute_units(near.device))
+    bm, bn = sizes_of(tile)[:2]
+    assert workers == 0 if rows == 9000 else workers <= -(-(-(-m // bm) * -(-n // bn)) // 256) * 256 - -(-m // bm) * -(-n // bn)
+
+
+@pytest.mark.gpu
+def test_a_weight_to_bring_nearer_that_is_refused():
+    x, w = rnd(128, 64, seed=24).to(DEV), rnd(64, 64, seed=25).to(DEV)
+    with pytest.raises(ValueError, match="contiguous"):
+        ops().gemm_tiles(torch.empty(128, 32, dtype=torch.bfloat16, device=DEV), x, w, swiglu=True, near=w.t())
+    with pytest.raises(ValueError, match="near goes"):
+        ops().gemm_tiles(torch.empty(128, 64, dtype=torch.bfloat16, device=DEV), x, w, near=w)
