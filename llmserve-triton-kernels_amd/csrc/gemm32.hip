@@ -4,13 +4,15 @@
 //
 //   gemm32_stream  M <= 64, K >= 512: the weight is read once, straight into the matrix instruction; a workgroup owns 16 or 32 weight
 //                  rows, its waves share K out in chunks of 32 and add their sums up in LDS in a fixed order.
-//   gemm32_tile    the rest: tiles through LDS, the next tile's loads in flight while the present one is multiplied; a result is
+//   gemm32_tile    the rest: tiles through LDS, the next steps' loads in flight while the present one is multiplied; a result is
 //                  the sum of its products from the first column to the last, to the bit what gemm_fma gives.
 //
 // Both: K and the row stride of A multiples of 4, A and W 16-byte aligned (the host checks; what does not fit goes to
 // gemm_fma); M and N are arbitrary.  Loads go through a buffer that ends with the workgroup's last row; rows and columns that
 // do not exist are asked for beyond its end, which brings zeros and touches no memory (and no branch surrounds a load).
 #include "common.h"
+
+#include <algorithm>
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
@@ -40,16 +42,23 @@ __device__ __forceinline__ unsigned row_offset(int row, int rows, int ld) { retu
 // 2048 x 2048 9 (a launch and one wait for memory); the multiply-add kernel, whose workgroup brings 64 weight rows through
 // LDS 4 bytes a load whatever the number of rows, takes 282, 216 and 197.  At 64 rows 111, 56 and 23: from some 20 rows on
 // every workgroup's reading of all rows of X out of L2 weighs more than the weight.
-template <int MB, int NT, int WAVES, int UNROLL>
+// HALVES (up to 8 rows of A): a tile is 8 weight rows, and rows 8 to 15 of both operands hold the same rows' next 32 columns, so
+// that D[i][j] and D[i + 8][j + 8] are two parts of one sum (the other two blocks of D mean nothing).  A weight of few rows then
+// has a workgroup on twice as many compute units, and each spends half the time in its matrix instructions: 2 rows against 2048 x
+// 5632 18.6 -> 12.6 microseconds, 1024 x 4096 13.0 -> 8.8, 2048 x 2048 7.7 -> 6.8 (with more loads a round 7.6 to 9.3 there, the waves'
+// registers being asked for in vain).
+template <int MB, int NT, int WAVES, int UNROLL, bool HALVES = false>
 __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* __restrict__ C, const float* __restrict__ X,
                                                                          const float* __restrict__ W,
                                                                          const float* __restrict__ bias, int M, int N, int K,
                                                                          int ldx, int ldc, int wide) {
+    static_assert(!HALVES || (MB == 1 && NT == 1), "halves: one tile of up to 8 rows");
+    constexpr int ROWS = HALVES ? 8 : 16, CHUNK = HALVES ? 64 : 32;  // rows of a tile, columns of a chunk
     __shared__ f32x4 red[WAVES][NT * MB][LLMS_WAVE];
     const int wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE;
-    const int r16 = lane % 16, g = lane / 16;
-    const int n0 = blockIdx.x * 16 * NT;
-    const __amdgpu_buffer_rsrc_t w_buf = rows_buffer(W, n0, 16 * NT, N, K, K), x_buf = rows_buffer(X, 0, 16 * MB, M, ldx, K);
+    const int r16 = lane % ROWS, g = lane / 16, later = HALVES ? (lane / 8 % 2) * 32 : 0;
+    const int n0 = blockIdx.x * ROWS * NT;
+    const __amdgpu_buffer_rsrc_t w_buf = rows_buffer(W, n0, ROWS * NT, N, K, K), x_buf = rows_buffer(X, 0, ROWS * MB, M, ldx, K);
     unsigned wrow[NT], xrow[MB];
 #pragma unroll
     for (int t = 0; t < NT; ++t) wrow[t] = row_offset(t * 16 + r16, N - n0, K);
@@ -61,7 +70,7 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
 #pragma unroll
         for (int b = 0; b < MB; ++b) acc[t][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-    const int chunks = (K + 31) / 32;
+    const int chunks = (K + CHUNK - 1) / CHUNK;
     for (int c0 = wave; c0 < chunks; c0 += WAVES * UNROLL) {
         f32x4 wv[UNROLL][NT][2];
 #pragma unroll
@@ -69,14 +78,14 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) wv[u][t][s] = load_columns(w_buf, wrow[t], (c0 + u * WAVES) * 32 + s * 16 + g * 4, K);
+                for (int s = 0; s < 2; ++s) wv[u][t][s] = load_columns(w_buf, wrow[t], (c0 + u * WAVES) * CHUNK + later + s * 16 + g * 4, K);
         f32x4 xv[UNROLL][MB][2];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
             for (int b = 0; b < MB; ++b)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) xv[u][b][s] = load_columns(x_buf, xrow[b], (c0 + u * WAVES) * 32 + s * 16 + g * 4, K);
+                for (int s = 0; s < 2; ++s) xv[u][b][s] = load_columns(x_buf, xrow[b], (c0 + u * WAVES) * CHUNK + later + s * 16 + g * 4, K);
         // (all of them are asked for before the first is used: with the rows of X asked for one by one behind the weights,
         // 2048 x 5632 at 2 rows took 21 microseconds instead of 19)
         __builtin_amdgcn_sched_barrier(0);
@@ -97,13 +106,16 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
     for (int idx = threadIdx.x; idx < NT * MB * LLMS_WAVE; idx += WAVES * LLMS_WAVE) {
         const int part = idx / LLMS_WAVE, l = idx % LLMS_WAVE;
         const int n = n0 + (part / MB) * 16 + 4 * (l / 16), m = (part % MB) * 16 + l % 16;
-        if (m >= M || n >= N) continue;
+        if (m >= M || n >= N || (HALVES && l >= 32)) continue;
         // (added up in 64 bits and rounded once: the few sums of a thread wait for LDS, not for arithmetic)
         double wide_sum[4] = {};
 #pragma unroll
         for (int w = 0; w < WAVES; ++w)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) wide_sum[r] += (double)red[w][part][l][r];
+            for (int r = 0; r < 4; ++r) {
+                wide_sum[r] += (double)red[w][part][l][r];
+                if constexpr (HALVES) wide_sum[r] += (double)red[w][part][l + 40][r];  // (rows 8 .. 15 by rows 8 .. 15 of X)
+            }
         f32x4 s = {(float)wide_sum[0], (float)wide_sum[1], (float)wide_sum[2], (float)wide_sum[3]};
         float* c = C + (size_t)m * ldc + n;
         if (wide && n + 4 <= N) {
@@ -120,17 +132,25 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
 }
 
 // ------------------------------------------------------------------------------ tiles
-// Bound by the matrix cores (157 TFLOP/s in 32-bit) once there are tiles for every compute unit: an instruction of 32 cycles
-// needs 8 bytes of LDS per lane, so one buffer and a plain order of stages are enough.  Measured: 4096 x 4096 at 2,048 rows 502
-// microseconds (137 TFLOP/s), 11264 x 2048 at 130 rows 106 (56; the multiply-add kernel 378), 2048 x 2048 at 130 rows 31 (220).
-template <int BM, int BN, int BK, int WM>
+template <int N>
+struct Number {
+    static constexpr int n = N;
+};
+
+// Bound by the matrix cores (157 TFLOP/s in 32-bit) once there are several large tiles for every compute unit: an instruction of 32
+// cycles needs 8 bytes of LDS per lane, so one buffer and a plain order of stages are enough (4096 x 4096 at 2,048 rows 502
+// microseconds, 137 TFLOP/s).  With few rows a compute unit has one or two workgroups, which wait for each stage in turn: the small
+// tiles have two buffers (TWO), and a step's products run beside the writing of the next one's tile and the loads of the two behind it,
+// which made a step of 32 x 64 x 64 1.0 -> 0.72 microseconds (0.43 in its matrix instructions).  Two buffers for 64 x 64 gain
+// nothing (105 and 104 microseconds for 11264 x 2048 at 130 rows): fewer workgroups fit.
+template <int BM, int BN, int BK, int WM, bool TWO>
 __global__ __launch_bounds__(256) void gemm32_tile_kernel(float* __restrict__ C, const float* __restrict__ A,
                                                           const float* __restrict__ W, const float* __restrict__ bias, int M,
                                                           int N, int K, int lda, int ldc, int tiles_m, int wide) {
     constexpr int WN = 4 / WM, TM = BM / WM / 16, TN = BN / WN / 16, LD = BK + 4;
     constexpr int PER_ROW = BK / 4, CA = BM * PER_ROW / 256, CB = BN * PER_ROW / 256, STEP = 256 / PER_ROW;
-    __shared__ __attribute__((aligned(16))) float As[BM * LD];
-    __shared__ __attribute__((aligned(16))) float Bs[BN * LD];
+    __shared__ __attribute__((aligned(16))) float As[TWO ? 2 : 1][BM * LD];
+    __shared__ __attribute__((aligned(16))) float Bs[TWO ? 2 : 1][BN * LD];
     // workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, rows fastest, so that the tiles
     // which share a weight slab share an L2
     const int nblk = gridDim.x, pid = blockIdx.x;
@@ -148,46 +168,103 @@ __global__ __launch_bounds__(256) void gemm32_tile_kernel(float* __restrict__ C,
     for (int c = 0; c < CA; ++c) ap[c] = row_offset(row + c * STEP, M - m0, lda);
 #pragma unroll
     for (int c = 0; c < CB; ++c) wp[c] = row_offset(row + c * STEP, N - n0, K);
-    f32x4 ra[CA], rb[CB], acc[TM][TN];
+    f32x4 ra[TWO ? 2 : 1][CA], rb[TWO ? 2 : 1][CB], acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int c = 0; c < CA; ++c) ra[c] = load_columns(a_buf, ap[c], k0 + col, K);
-#pragma unroll
-        for (int c = 0; c < CB; ++c) rb[c] = load_columns(w_buf, wp[c], k0 + col, K);
+    // piece p of a step's loads (rows of A, then of W; beyond K: from nowhere)
+    auto fetch = [&](auto set, int p, int k0) {
+        constexpr int q = decltype(set)::n;
+        if (p < CA) ra[q][p] = load_columns(a_buf, ap[p], k0 + col, K);
+        else rb[q][p - CA] = load_columns(w_buf, wp[p - CA], k0 + col, K);
     };
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += BK) {
-        __syncthreads();  // (every wave is done with the tile before)
+    auto put = [&](auto set, int p) {
+        constexpr int q = decltype(set)::n;
         // column 4 q + r of a group of 16 lies at 4 r + q: what a lane reads in one piece, its instructions take in the order
         // of the columns, so that a result is the sum of its products from the first column to the last
 #pragma unroll
-        for (int c = 0; c < CA; ++c)
+        for (int r = 0; r < 4; ++r) {
+            if (p < CA) As[q][(row + p * STEP) * LD + place + 4 * r] = ra[q][p][r];
+            else Bs[q][(row + (p - CA) * STEP) * LD + place + 4 * r] = rb[q][p - CA][r];
+        }
+    };
+    f32x4 xf[2][TM], wf[2][TN];
+    auto read = [&](auto set, int s) {
+        constexpr int q = decltype(set)::n;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) As[(row + c * STEP) * LD + place + 4 * r] = ra[c][r];
+        for (int i = 0; i < TM; ++i) xf[s % 2][i] = *reinterpret_cast<const f32x4*>(&As[q][(wm + i * 16 + r16) * LD + s * 16 + g * 4]);
 #pragma unroll
-        for (int c = 0; c < CB; ++c)
+        for (int j = 0; j < TN; ++j) wf[s % 2][j] = *reinterpret_cast<const f32x4*>(&Bs[q][(wn + j * 16 + r16) * LD + s * 16 + g * 4]);
+    };
+    auto multiply = [&](int s) {
+        // (four columns of K for every tile before the next four: a tile's instructions do not follow on one another)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) Bs[(row + c * STEP) * LD + place + 4 * r] = rb[c][r];
-        __syncthreads();
-        if (k0 + BK < K) fetch(k0 + BK);
+        for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int s = 0; s < BK / 16; ++s) {
-            f32x4 xf[TM], wf[TN];
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int i = 0; i < TM; ++i) xf[i] = *reinterpret_cast<const f32x4*>(&As[(wm + i * 16 + r16) * LD + s * 16 + g * 4]);
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[s % 2][j][r], xf[s % 2][i][r], acc[i][j], 0, 0, 0);
+    };
+    // LDS only is waited for: the loads of the steps behind stay in flight
+    auto meet = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // A step: its tile lies in one buffer; the next step's goes into the other (whose readers met behind the step before), the one
+    // behind that is asked for, and the step's products run beside both, a group of 16 columns at a time.  (With all of the next
+    // tile written before the first read, the reads queued behind 96 writes of the workgroup.)
+    constexpr int GROUPS = BK / 16, PIECES = CA + CB;
+    auto one = [&](auto now, auto next, int k0) {
+        read(now, 0);
 #pragma unroll
-            for (int j = 0; j < TN; ++j) wf[j] = *reinterpret_cast<const f32x4*>(&Bs[(wn + j * 16 + r16) * LD + s * 16 + g * 4]);
-            // (four columns of K for every tile before the next four: a tile's instructions do not follow on one another)
+        for (int s = 0; s < GROUPS; ++s) {
+            if (s + 1 < GROUPS) read(now, s + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(s);
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+            for (int p = PIECES * s / GROUPS; p < PIECES * (s + 1) / GROUPS; ++p) {
+                put(next, p);
+                fetch(next, p, k0 + 3 * BK);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        meet();
+    };
+    if constexpr (TWO) {
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+        for (int p = 0; p < PIECES; ++p) fetch(Number<0>(), p, 0);
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][r], xf[i][r], acc[i][j], 0, 0, 0);
+        for (int p = 0; p < PIECES; ++p) fetch(Number<1>(), p, BK);
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) {
+            put(Number<0>(), p);
+            fetch(Number<0>(), p, 2 * BK);
+        }
+        meet();
+        for (int k0 = 0; k0 < K; k0 += 2 * BK) {  // (a step beyond K adds zeros; a branch around it made the compiler wait for every load)
+            one(Number<0>(), Number<1>(), k0);
+            one(Number<1>(), Number<0>(), k0 + BK);
+        }
+    } else {
+#pragma unroll
+        for (int p = 0; p < PIECES; ++p) fetch(Number<0>(), p, 0);
+        for (int k0 = 0; k0 < K; k0 += BK) {
+            __syncthreads();  // (every wave is done with the tile before)
+#pragma unroll
+            for (int p = 0; p < PIECES; ++p) put(Number<0>(), p);
+            __syncthreads();
+            if (k0 + BK < K)
+#pragma unroll
+                for (int p = 0; p < PIECES; ++p) fetch(Number<0>(), p, k0 + BK);
+#pragma unroll
+            for (int s = 0; s < GROUPS; ++s) {
+                read(Number<0>(), s);
+                multiply(s);
+            }
         }
     }
 #pragma unroll
@@ -213,13 +290,13 @@ __global__ __launch_bounds__(256) void gemm32_tile_kernel(float* __restrict__ C,
     }
 }
 
-template <int BM, int BN, int BK, int WM>
+template <int BM, int BN, int BK, int WM, bool TWO>
 static int launch_tile(float* C, const float* A, const float* W, const float* bias, int M, int N, int K, int lda, int ldc, int wide,
                        hipStream_t stream) {
     const int tiles_m = (M + BM - 1) / BM;
     const long long blocks = (long long)tiles_m * ((N + BN - 1) / BN);
     LLMS_REQUIRE(blocks < (1ll << 31), "gemm32: too many tiles");
-    gemm32_tile_kernel<BM, BN, BK, WM><<<(unsigned)blocks, 256, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, tiles_m, wide);
+    gemm32_tile_kernel<BM, BN, BK, WM, TWO><<<(unsigned)blocks, 256, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, tiles_m, wide);
     LLMS_LAUNCH_CHECK();
 }
 
@@ -244,7 +321,9 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
         const unsigned tiles = (N + 15) / 16, pairs = (N + 31) / 32;
         if (M <= 16) {
             // 16 waves a tile while the tiles alone do not fill the chip, 8 beyond
-            if (tiles <= 2u * cus) gemm32_stream_kernel<1, 1, 16, 4><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+            // tiles of 8 weight rows where there are no more of them than compute units and up to 8 rows of A
+            if (M <= 8 && (N + 7) / 8 <= cus) gemm32_stream_kernel<1, 1, 16, 2, true><<<(N + 7) / 8, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+            else if (tiles <= 2u * cus) gemm32_stream_kernel<1, 1, 16, 4><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
             else gemm32_stream_kernel<1, 1, 8, 4><<<tiles, 512, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
         } else if (M <= 32) {
             if (tiles <= 2u * cus) gemm32_stream_kernel<2, 1, 16, 4><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
@@ -255,11 +334,17 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
         }
         LLMS_LAUNCH_CHECK();
     }
-    // the largest tile of which there are two for every compute unit (a larger tile reads each operand less often)
-    const auto tiles_of = [&](int bm, int bn) { return (long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-    if (tiles_of(128, 128) >= 2ll * cus) return launch_tile<128, 128, 32, 2>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
-    if (tiles_of(64, 64) >= 2ll * cus) return launch_tile<64, 64, 64, 2>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
-    return launch_tile<32, 64, 64, 1>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+    // The tile that takes least: microseconds per round of tiles over the compute units and what the first costs beyond, for 2,048
+    // columns (measured at 65 to 1,500 rows against 1,024 to 11,264 weight rows; the larger ones read each operand less often).  65
+    // rows: 2048 x 2048 31 -> 16 microseconds by the two smallest as they are now, 2048 x 5632 78 -> 37; 130 rows: 31 -> 25, 78 -> 59,
+    // 11264 x 2048 105 -> 72; 333 rows: 46 -> 33, 117 -> 85, 170 -> 143.
+    const auto rounds = [&](int bm, int bn) { return (float)(((long long)((M + bm - 1) / bm) * ((N + bn - 1) / bn) + cus - 1) / cus); };
+    const float r32 = rounds(32, 32), c32 = 8.2f * r32 + 1.5f * std::max(0.f, r32 - 4.f) + 8.f, c64 = 17.f * rounds(32, 64) + 8.4f;
+    const float c4 = 30.f * rounds(64, 64) + 16.f, c16 = 105.f * rounds(128, 128) + 40.f;
+    if (c16 <= std::min(c4, std::min(c64, c32))) return launch_tile<128, 128, 32, 2, false>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+    if (c4 <= std::min(c64, c32)) return launch_tile<64, 64, 64, 2, false>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+    if (c64 <= c32) return launch_tile<32, 64, 64, 1, true>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+    return launch_tile<32, 32, 64, 2, true>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
 }
 
 }  // extern "C"

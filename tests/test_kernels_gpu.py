@@ -268,6 +268,26 @@ def test_gemm32(m, n, k):
         ops().gemm32(whole, a.bfloat16().to(DEV), w.bfloat16().to(DEV))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 8, 512), (8, 2048, 512), (7, 2041, 516), (8, 2043, 2108), (2, 2048, 5632), (9, 2048, 516),
+                                   (8, 2049, 516), (65, 31, 64), (97, 2050, 68), (130, 2079, 196), (66, 4099, 4), (333, 2560, 132),
+                                   (700, 2048, 72), (1500, 2559, 60)])
+def test_gemm32_by_arrangement(m, n, k):
+    """Halves of K side by side (up to 8 rows, a tile of 8 weight rows a compute unit), and each of the tiles: remainders of tiles and of
+    K, steps of K that do not fill the buffers, nothing beside the result."""
+    g = torch.Generator().manual_seed(m * 131 + n)
+    a, w, b = (torch.randn(*s, generator=g).to(DEV) for s in ((m, k + 4), (n, k), (n,)))
+    a = a[:, :k]  # (rows of a wider matrix)
+    out = torch.full((m + 1, n + 3), 7.0, device=DEV)
+    ops().gemm32(out[:m, :n], a, w, b)
+    assert bool((out[m:] == 7.0).all()) and bool((out[:, n:] == 7.0).all())
+    if m > 64 or k < 512:  # the sums of the multiply-add kernel, column after column
+        assert torch.equal(out[:m, :n], ops().gemm_fma(torch.empty(m, n, device=DEV), a.contiguous(), w, b))
+    else:
+        # sums of k products in 32-bit, in any order: k roundings of at most 2^-24 of the sum of the products' sizes each
+        size = a.double().abs() @ w.double().abs().T + b.double().abs()
+        assert ((out[:m, :n].double() - (a.double() @ w.double().T + b.double())).abs() <= k * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("n,k", [(512, 512), (2048, 2048), (333, 5632)])
 def test_gemm32_rows_in_other_company(n, k):
     """Up to 64 rows of 512 columns and more are summed by several waves, more rows in the order of the columns: a row's result
