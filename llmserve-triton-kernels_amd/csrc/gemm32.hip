@@ -47,21 +47,26 @@ __device__ __forceinline__ unsigned row_offset(int row, int rows, int ld) { retu
 // has a workgroup on twice as many compute units, and each spends half the time in its matrix instructions: 2 rows against 2048 x
 // 5632 18.6 -> 12.6 microseconds, 1024 x 4096 13.0 -> 8.8, 2048 x 2048 7.7 -> 6.8 (with more loads a round 7.6 to 9.3 there, the waves'
 // registers being asked for in vain).
-template <int MB, int NT, int WAVES, int UNROLL, bool HALVES = false>
+template <int MB, int NT, int WAVES, int UNROLL, bool HALVES = false, bool GATED = false>
 __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* __restrict__ C, const float* __restrict__ X,
                                                                          const float* __restrict__ W,
                                                                          const float* __restrict__ bias, int M, int N, int K,
                                                                          int ldx, int ldc, int wide) {
     static_assert(!HALVES || (MB == 1 && NT == 1), "halves: one tile of up to 8 rows");
+    static_assert(!GATED || (MB == 1 && NT == 1 && !HALVES), "gated: one tile of 8 units");
     constexpr int ROWS = HALVES ? 8 : 16, CHUNK = HALVES ? 64 : 32;  // rows of a tile, columns of a chunk
     __shared__ f32x4 red[WAVES][NT * MB][LLMS_WAVE];
     const int wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE;
     const int r16 = lane % ROWS, g = lane / 16, later = HALVES ? (lane / 8 % 2) * 32 : 0;
-    const int n0 = blockIdx.x * ROWS * NT;
-    const __amdgpu_buffer_rsrc_t w_buf = rows_buffer(W, n0, ROWS * NT, N, K, K), x_buf = rows_buffer(X, 0, ROWS * MB, M, ldx, K);
+    const int n0 = blockIdx.x * (GATED ? 8 : ROWS * NT);
+    // (gated: from the first gate row to the last up row, W = [gate; up] of N units each)
+    const __amdgpu_buffer_rsrc_t w_buf = rows_buffer(W, n0, GATED ? N + 8 : ROWS * NT, GATED ? 2 * N : N, K, K), x_buf = rows_buffer(X, 0, ROWS * MB, M, ldx, K);
     unsigned wrow[NT], xrow[MB];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wrow[t] = row_offset(t * 16 + r16, N - n0, K);
+    for (int t = 0; t < NT; ++t) {
+        if constexpr (GATED) wrow[t] = n0 + r16 % 8 < N ? row_offset(r16 % 8 + (r16 < 8 ? 0 : N), 2 * N, K) : NOWHERE / 2;
+        else wrow[t] = row_offset(t * 16 + r16, N - n0, K);
+    }
 #pragma unroll
     for (int b = 0; b < MB; ++b) xrow[b] = row_offset(b * 16 + r16, M, ldx);
     f32x4 acc[NT][MB];
@@ -106,7 +111,7 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
     for (int idx = threadIdx.x; idx < NT * MB * LLMS_WAVE; idx += WAVES * LLMS_WAVE) {
         const int part = idx / LLMS_WAVE, l = idx % LLMS_WAVE;
         const int n = n0 + (part / MB) * 16 + 4 * (l / 16), m = (part % MB) * 16 + l % 16;
-        if (m >= M || n >= N || (HALVES && l >= 32)) continue;
+        if (m >= M || n >= N || ((HALVES || GATED) && l >= 32)) continue;
         // (added up in 64 bits and rounded once: the few sums of a thread wait for LDS, not for arithmetic)
         double wide_sum[4] = {};
 #pragma unroll
@@ -117,6 +122,15 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
                 if constexpr (HALVES) wide_sum[r] += (double)red[w][part][l + 40][r];  // (rows 8 .. 15 by rows 8 .. 15 of X)
             }
         f32x4 s = {(float)wide_sum[0], (float)wide_sum[1], (float)wide_sum[2], (float)wide_sum[3]};
+        if constexpr (GATED) {  // (rows 8 .. 15: the same units' up)
+            double up[4] = {};
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) up[r] += (double)red[w][part][l + 32][r];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] = s[r] / (1.f + expf(-s[r])) * (float)up[r];
+        }
         float* c = C + (size_t)m * ldc + n;
         if (wide && n + 4 <= N) {
             if (bias)
@@ -345,6 +359,22 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
     if (c4 <= std::min(c64, c32)) return launch_tile<64, 64, 64, 2, false>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
     if (c64 <= c32) return launch_tile<32, 64, 64, 1, true>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
     return launch_tile<32, 32, 64, 2, true>(C, A, W, bias, M, N, K, lda, ldc, wide, stream);
+}
+
+// c[M, inter] = silu(a wg^T) * (a wu^T), w = [wg; wu] of `inter` rows each: up to 16 rows, the activation in the product's epilogue (4.7
+// microseconds a launch of its own), with the sums and the arithmetic of llms_gemm32 and the activation behind it.
+int llms_gemm32_gated(void* c, const void* a, const void* w, int M, int inter, int K, int lda, int ldc, int cus, hipStream_t stream) {
+    LLMS_REQUIRE(M > 0 && M <= 16 && inter > 0 && K >= 512 && cus > 0, "gemm32_gated: 1 to 16 rows of 512 columns and more");
+    LLMS_REQUIRE(K % 4 == 0 && lda % 4 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0, "gemm32_gated: rows of multiples of 4, 16-byte aligned");
+    LLMS_REQUIRE(lda >= K && ldc >= inter, "gemm32_gated: leading dimensions too small");
+    LLMS_REQUIRE((long long)(inter + 8) * K * 4 < (1ll << 30) && (long long)lda * 4 * 128 < (1ll << 30), "gemm32_gated: too large");
+    float* C = (float*)c;
+    const float *A = (const float*)a, *W = (const float*)w;
+    const int wide = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
+    const unsigned tiles = (inter + 7) / 8;
+    if ((2 * inter + 15) / 16 <= 2 * cus) gemm32_stream_kernel<1, 1, 16, 4, false, true><<<tiles, 1024, 0, stream>>>(C, A, W, nullptr, M, inter, K, lda, ldc, wide);
+    else gemm32_stream_kernel<1, 1, 8, 4, false, true><<<tiles, 512, 0, stream>>>(C, A, W, nullptr, M, inter, K, lda, ldc, wide);
+    LLMS_LAUNCH_CHECK();
 }
 
 }  // extern "C"

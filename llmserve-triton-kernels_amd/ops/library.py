@@ -332,6 +332,28 @@ def gemm32(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: torch.Tens
     return out
 
 
+def gemm32_gated_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether `gemm32_gated` takes these operands: up to 16 rows of 512 columns and more, [gate; up] of less than 2 GB."""
+    return (0 < a.shape[0] <= 16 and a.shape[1] >= 512 and w.shape[0] % 2 == 0 and w.is_contiguous() and gemm32_supported(a, w) and
+            a.stride(1) == 1 and (w.shape[0] // 2 + 8) * a.shape[1] * 4 < 1 << 30)
+
+
+def gemm32_gated(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """out[M, I] = silu(gate) * up with [gate, up] = a w^T, w = [gate; up] [2I, K]: float32, as `gemm32` and `silu_mul` behind it
+    give it, in one launch."""
+    dev = _dev(out, a, w)
+    _rows(w, "w", a.shape[1])
+    m, k = a.shape
+    inter = w.shape[0] // 2
+    if out.dim() != 2 or out.stride(1) != 1 or tuple(out.shape) != (m, inter) or out.dtype != torch.float32:
+        raise ValueError(f"out must be float32 {(m, inter)} with unit inner stride")
+    if not gemm32_gated_supported(a, w):
+        raise ValueError("gemm32_gated takes 1 to 16 float32 rows of 512 columns and more, multiples of 4, 16-byte aligned")
+    _check(load("gemm32").llms_gemm32_gated(_ptr(out), _ptr(a), _ptr(w), c_int(m), c_int(inter), c_int(k), c_int(a.stride(0)),
+                                            c_int(out.stride(0)), c_int(compute_units(dev)), _stream(dev)), "gemm32_gated")
+    return out
+
+
 def gemm_bf16_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the matrix-core kernels take these operands (else `gemm_fma` does)."""
     k = a.shape[1]

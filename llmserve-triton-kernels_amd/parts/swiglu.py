@@ -68,6 +68,8 @@ class SwiGLU(FeedForward):
                 ops.gemm_stream(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # activation in the product's epilogue
             elif not few and self.intermediate % 16 == 0 and tiles_product(rows, self.gate_up, "gated"):
                 ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu, near=self.down)  # the same
+            elif self.unit == "silu" and ops.gemm32_gated_supported(rows, self.gate_up):
+                ops.gemm32_gated(act, rows, self.gate_up)  # the same, in 32-bit
             else:
                 ops.silu_mul(act, linear(rows, self.gate_up), self.limit, self.gelu)
         if deferred and x.may_add_in_place and adds_residual_in_epilogue(act, self.down):

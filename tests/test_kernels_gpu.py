@@ -288,6 +288,25 @@ def test_gemm32_by_arrangement(m, n, k):
         assert ((out[:m, :n].double() - (a.double() @ w.double().T + b.double())).abs() <= k * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("m,inter,k", [(1, 4100, 512), (2, 5632, 2048), (16, 4099, 516), (9, 2041, 1028), (3, 5, 512)])
+def test_gemm32_gated(m, inter, k):
+    """To the bit the product and the activation behind it, where the product is summed by the same waves (its tiles of 8 weight rows
+    are not); units that do not fill a tile, rows of a wider matrix, nothing beside the result."""
+    a, w = rnd(m, k + 4, seed=31).to(DEV)[:, :k], rnd(2 * inter, k, seed=32, scale=k ** -0.5).to(DEV)
+    out = torch.full((m + 1, inter + 3), 7.0, device=DEV)
+    ops().gemm32_gated(out[:m, :inter], a, w)
+    assert bool((out[m:] == 7.0).all()) and bool((out[:, inter:] == 7.0).all())
+    both = ops().gemm32(torch.empty(m, 2 * inter, device=DEV), a, w)
+    want = ops().silu_mul(torch.empty(m, inter, device=DEV), both)
+    if m > 8 or 2 * inter > 2048:
+        assert torch.equal(out[:m, :inter], want)
+    # |silu'| <= 1.1 and |silu(g)| <= |g|: the sums' errors (test_gemm32_by_arrangement), and some roundings of the unit
+    size = a.double().abs() @ w.double().abs().T * k * 2.0 ** -24
+    g, u = (a.double() @ w.double().T).split(inter, 1)
+    bound = 1.1 * size[:, :inter] * (u.abs() + size[:, inter:]) + g.abs() * size[:, inter:] + 2.0 ** -20 * (g * u).abs()
+    assert ((out[:m, :inter].double() - torch.nn.functional.silu(g) * u).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("n,k", [(512, 512), (2048, 2048), (333, 5632)])
 def test_gemm32_rows_in_other_company(n, k):
     """Up to 64 rows of 512 columns and more are summed by several waves, more rows in the order of the columns: a row's result
