@@ -18,8 +18,8 @@
 //
 // Measured (microseconds, weights from memory, the norm behind o_proj and down_proj included; in brackets the library's product
 // with the kernels behind it):
-//   1.1B shape    333 rows: q, k, v 11 (17), o_proj in 2 parts 14 (15), gate and up with SiLU 34 (36), down_proj in 4 parts 20 (24)
-//                 512 rows: 12 (20), 13 (16), 36 (38), 23 (25) in 2 parts;  2,048 rows: 28 (33), 27 (29), 95 (94), 59 (59)
+//   1.1B shape    333 rows: q, k, v 11 (17), o_proj in 2 parts 14 (15), gate and up with SiLU 29 (36), down_proj in 4 parts 20 (24)
+//                 512 rows: 12 (20), 13 (16), 32 (38), 23 (25) in 2 parts;  2,048 rows: 28 (33), 27 (29), 95 (94), 59 (59)
 //   7B shape      333 rows: 54 (61), 27 (30), 77 (78), 48 (62);  512 rows: 57 (62), 32 (35), 107 (88), 57 (78);  2,048 rows: 185 (172), 71
 //                 (70), 314 (424), 160 (172)
 // What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times

@@ -1,6 +1,6 @@
 """y = x W^T (+ b) for the parts: picks the matrix product by dtype and shape.
 
-float32: the 32-bit matrix-core kernels (ops.gemm32: multiply-adds in 32-bit, no reduced-precision mode), or the
+float32: the 32-bit matrix-core kernels (ops.gemm32: multiply-adds in 32-bit, no reduced-precision mode; ops.gemm32_gated), or the
   multiply-add kernel of the vector units where rows are no multiples of 16 bytes.
 bfloat16, up to 16 rows of up to 6,144 columns, 17 to 32 rows of up to 4,096, or 33 to 64 rows of up to 2,048:
   ops.gemm_decode, one workgroup per compute unit, with the activation or the rotation and cache store in
@@ -80,7 +80,7 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 # size to size, so single products lie on the wrong side: 1 in 18 below the line is more than 5 percent slower in tiles, at most 19, and 1
 # in 6 beyond it more than 5 percent faster.  Single sizes, microseconds, tiles and library:
 #   plain   4608 x 2048 12 and 16 at 333 rows; 6144 x 2048 16 and 20 at 333, 57 and 46 at 2,048; 32000 x 2048 65 and 61 at 512
-#   gated   11264 x 2048 36 and 38 at 512 rows, 86 and 73 at 1,300; 22016 x 4096 61 and 62 at 200, 107 and 88 at 512, 188 and 162 at
+#   gated   11264 x 2048 32 and 38 at 512 rows, 86 and 73 at 1,300; 22016 x 4096 61 and 62 at 200, 107 and 88 at 512, 188 and 162 at
 #           1,024; 28672 x 4096 428 and 355 at 2,048
 #   rotary  2560 x 2048 12 and 20 at 512 rows; 12288 x 4096 57 and 62 at 512, 106 and 90 at 1,024
 #   parts   4096 x 11008 57 and 78 at 512 rows; 8192 x 28672 159 and 313 at 200, 446 and 261 at 640
