@@ -270,7 +270,7 @@ def test_gemm32(m, n, k):
 
 @pytest.mark.parametrize("m,n,k", [(1, 8, 512), (8, 2048, 512), (7, 2041, 516), (8, 2043, 2108), (2, 2048, 5632), (9, 2048, 516),
                                    (8, 2049, 516), (65, 31, 64), (97, 2050, 68), (130, 2079, 196), (66, 4099, 4), (333, 2560, 132),
-                                   (700, 2048, 72), (1500, 2559, 60)])
+                                   (700, 2048, 72), (1500, 2559, 60), (333, 2563, 324), (500, 11270, 132), (700, 2563, 260)])
 def test_gemm32_by_arrangement(m, n, k):
     """Halves of K side by side (up to 8 rows, a tile of 8 weight rows a compute unit), and each of the tiles: remainders of tiles and of
     K, steps of K that do not fill the buffers, nothing beside the result."""

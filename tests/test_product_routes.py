@@ -36,3 +36,20 @@ def test_what_the_tiles_leave_behind_is_the_librarys():
         for m in (65, 200, 512, 700, 1100, 2048, 8192):
             for n, k in ((2560, 2048), (11264, 2048), (22016, 4096), (4096, 11008), (57344, 8192)):
                 assert tiles_pay(kind, m, n, k) or not tiles_pay("plain", m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,micros", [
+    # microseconds of 32 x 32 and 32 x 64 with two buffers, 32 x 64, 64 x 64 and 128 x 128 with one
+    (512, 11264, 64, (22.5, 22.0, 13.3, 14.1, 16.1)), (100, 2560, 64, (4.05, 4.32, 3.34, 4.08, 8.17)),
+    (1900, 2560, 64, (20.1, 20.3, 11.9, 12.8, 16.1)), (65, 11264, 64, (7.15, 7.44, 5.12, 6.25, 8.36)),
+    (200, 11264, 128, (12.3, 13.0, 10.5, 11.5, 14.6)), (512, 2560, 128, (7.77, 7.84, 7.19, 8.57, 13.7)),
+    (64, 512, 128, (3.29, 4.16, 3.96, 5.28, 11.9)), (512, 11264, 256, (36.2, 35.4, 32.4, 33.1, 39.8)),
+    (65, 256, 1024, (8.57, 13.7, 15.9, 24.3, 72.6)), (1900, 11264, 1024, (446, 415, 391, 371, 385)),
+    (65, 512, 11008, (66.9, 120, 151, 237, 762)), (1900, 11264, 5632, (2405, 2178, 2119, 1977, 2019)),
+])
+def test_the_tile_of_a_32_bit_product_by_all_its_sizes(m, n, k, micros):
+    """The number of columns counts too: what two buffers gain they gain from the steps of K."""
+    from llmserve.ops import library
+
+    tile = library.load("gemm32").llms_gemm32_tile(m, n, k, 256)
+    assert micros[tile] <= 1.1 * min(micros)
