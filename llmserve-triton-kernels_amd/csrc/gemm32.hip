@@ -2,8 +2,9 @@
 // v_mfma_f32_16x16x4_f32 multiplies and adds in 32-bit (no reduced-precision mode) at the rate of the vector units, but takes
 // its operands from registers that a wave fills with 16-byte loads, so nothing but memory bounds the products of few rows.
 //
-//   gemm32_stream  M <= 64, K >= 512: the weight is read once, straight into the matrix instruction; a workgroup owns 16 or 32 weight
-//                  rows, its waves share K out in chunks of 32 and add their sums up in LDS in a fixed order.
+//   gemm32_stream  M <= 64, K >= 512: the weight is read once, straight into the matrix instruction; a workgroup owns 8, 16 or 32
+//                  weight rows, its waves share K out in chunks of 32 and add their sums up in LDS in a fixed order, which the
+//                  number of weight rows decides and the number of rows does not.
 //   gemm32_tile    the rest: tiles through LDS, the next steps' loads in flight while the present one is multiplied; a result is
 //                  the sum of its products from the first column to the last, to the bit what gemm_fma gives.
 //
@@ -40,11 +41,12 @@ __device__ __forceinline__ unsigned row_offset(int row, int rows, int ld) { retu
 // 2048 x 2048 9 (a launch and one wait for memory); the multiply-add kernel, whose workgroup brings 64 weight rows through
 // LDS 4 bytes a load whatever the number of rows, takes 282, 216 and 197.  At 64 rows 111, 56 and 23: from some 20 rows on
 // every workgroup's reading of all rows of X out of L2 weighs more than the weight.
-// HALVES (up to 8 rows of A): a tile is 8 weight rows, and rows 8 to 15 of both operands hold the same rows' next 32 columns, so
-// that D[i][j] and D[i + 8][j + 8] are two parts of one sum (the other two blocks of D mean nothing).  A weight of few rows then
-// has a workgroup on twice as many compute units, and each spends half the time in its matrix instructions: 2 rows against 2048 x
-// 5632 18.6 -> 12.6 microseconds, 1024 x 4096 13.0 -> 8.8, 2048 x 2048 7.7 -> 6.8 (with more loads a round 7.6 to 9.3 there, the waves'
-// registers being asked for in vain).
+// HALVES (up to 8 rows of A): a tile is 8 weight rows, and rows 8 to 15 of both operands hold the same rows' columns of another share of
+// K, so that D[i][j] and D[i + 8][j + 8] are two parts of one sum (the other two blocks of D mean nothing).  A weight of few rows
+// then has a workgroup on twice as many compute units, and each spends half the time in its matrix instructions.  8 waves with two
+// shares each sum what 16 waves sum elsewhere, in the same order: a row's result is the same bits whether 1 or 64 rows come with it.
+// 2 rows against 2048 x 5632 17.3 -> 10.9 microseconds, 1024 x 4096 12.9 -> 8.0, 2048 x 2048 7.9 -> 6.3, 512 x 512 5.5 -> 3.6 (16 waves
+// with two shares each, whose sums are others: 12.1, 8.6, 7.0 and 4.0; with 4 chunks a round instead of 2: 12.1, 8.4, 6.4 and 4.1).
 template <int MB, int NT, int WAVES, int UNROLL, bool HALVES = false, bool GATED = false>
 __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* __restrict__ C, const float* __restrict__ X,
                                                                          const float* __restrict__ W,
@@ -52,10 +54,10 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
                                                                          int ldx, int ldc, int wide) {
     static_assert(!HALVES || (MB == 1 && NT == 1), "halves: one tile of up to 8 rows");
     static_assert(!GATED || (MB == 1 && NT == 1 && !HALVES), "gated: one tile of 8 units");
-    constexpr int ROWS = HALVES ? 8 : 16, CHUNK = HALVES ? 64 : 32;  // rows of a tile, columns of a chunk
+    constexpr int ROWS = HALVES ? 8 : 16, SHARES = HALVES ? 2 * WAVES : WAVES;  // rows of a tile, sums that K is shared out to
     __shared__ f32x4 red[WAVES][NT * MB][LLMS_WAVE];
     const int wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE;
-    const int r16 = lane % ROWS, g = lane / 16, later = HALVES ? (lane / 8 % 2) * 32 : 0;
+    const int r16 = lane % ROWS, g = lane / 16, later = HALVES ? (lane / 8 % 2) * WAVES * 32 : 0;
     const int n0 = blockIdx.x * (GATED ? 8 : ROWS * NT);
     // (gated: from the first gate row to the last up row, W = [gate; up] of N units each)
     const __amdgpu_buffer_rsrc_t w_buf = rows_buffer(W, n0, GATED ? N + 8 : ROWS * NT, GATED ? 2 * N : N, K, K), x_buf = rows_buffer(X, 0, ROWS * MB, M, ldx, K);
@@ -73,22 +75,22 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
 #pragma unroll
         for (int b = 0; b < MB; ++b) acc[t][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-    const int chunks = (K + CHUNK - 1) / CHUNK;
-    for (int c0 = wave; c0 < chunks; c0 += WAVES * UNROLL) {
+    const int chunks = (K + 31) / 32;
+    for (int c0 = wave; c0 < chunks; c0 += SHARES * UNROLL) {
         f32x4 wv[UNROLL][NT][2];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) wv[u][t][s] = load_columns(w_buf, wrow[t], (c0 + u * WAVES) * CHUNK + later + s * 16 + g * 4, K);
+                for (int s = 0; s < 2; ++s) wv[u][t][s] = load_columns(w_buf, wrow[t], (c0 + u * SHARES) * 32 + later + s * 16 + g * 4, K);
         f32x4 xv[UNROLL][MB][2];
 #pragma unroll
         for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
             for (int b = 0; b < MB; ++b)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) xv[u][b][s] = load_columns(x_buf, xrow[b], (c0 + u * WAVES) * CHUNK + later + s * 16 + g * 4, K);
+                for (int s = 0; s < 2; ++s) xv[u][b][s] = load_columns(x_buf, xrow[b], (c0 + u * SHARES) * 32 + later + s * 16 + g * 4, K);
         // (all of them are asked for before the first is used: with the rows of X asked for one by one behind the weights,
         // 2048 x 5632 at 2 rows took 21 microseconds instead of 19)
         __builtin_amdgcn_sched_barrier(0);
@@ -115,10 +117,13 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
 #pragma unroll
         for (int w = 0; w < WAVES; ++w)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                wide_sum[r] += (double)red[w][part][l][r];
-                if constexpr (HALVES) wide_sum[r] += (double)red[w][part][l + 40][r];  // (rows 8 .. 15 by rows 8 .. 15 of X)
-            }
+            for (int r = 0; r < 4; ++r) wide_sum[r] += (double)red[w][part][l][r];
+        if constexpr (HALVES) {  // (rows 8 .. 15 by rows 8 .. 15 of X)
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) wide_sum[r] += (double)red[w][part][l + 40][r];
+        }
         f32x4 s = {(float)wide_sum[0], (float)wide_sum[1], (float)wide_sum[2], (float)wide_sum[3]};
         if constexpr (GATED) {  // (rows 8 .. 15: the same units' up)
             double up[4] = {};
@@ -369,7 +374,7 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
         if (M <= 16) {
             // 16 waves a tile while the tiles alone do not fill the chip, 8 beyond
             // tiles of 8 weight rows where there are no more of them than compute units and up to 8 rows of A
-            if (M <= 8 && (N + 7) / 8 <= cus) gemm32_stream_kernel<1, 1, 16, 2, true><<<(N + 7) / 8, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
+            if (M <= 8 && (N + 7) / 8 <= cus) gemm32_stream_kernel<1, 1, 8, 2, true><<<(N + 7) / 8, 512, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
             else if (tiles <= 2u * cus) gemm32_stream_kernel<1, 1, 16, 4><<<tiles, 1024, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
             else gemm32_stream_kernel<1, 1, 8, 4><<<tiles, 512, 0, stream>>>(C, A, W, bias, M, N, K, lda, ldc, wide);
         } else if (M <= 32) {

@@ -272,7 +272,7 @@ def test_gemm32(m, n, k):
                                    (8, 2049, 516), (65, 31, 64), (97, 2050, 68), (130, 2079, 196), (66, 4099, 4), (333, 2560, 132),
                                    (700, 2048, 72), (1500, 2559, 60), (333, 2563, 324), (500, 11270, 132), (700, 2563, 260)])
 def test_gemm32_by_arrangement(m, n, k):
-    """Halves of K side by side (up to 8 rows, a tile of 8 weight rows a compute unit), and each of the tiles: remainders of tiles and of
+    """Two shares of K side by side (up to 8 rows, a tile of 8 weight rows a compute unit), and each of the tiles: remainders of tiles and of
     K, steps of K that do not fill the buffers, nothing beside the result."""
     g = torch.Generator().manual_seed(m * 131 + n)
     a, w, b = (torch.randn(*s, generator=g).to(DEV) for s in ((m, k + 4), (n, k), (n,)))
@@ -288,18 +288,31 @@ def test_gemm32_by_arrangement(m, n, k):
         assert ((out[:m, :n].double() - (a.double() @ w.double().T + b.double())).abs() <= k * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("n,k", [(8, 512), (512, 516), (2041, 1028), (2048, 2048), (2056, 512), (2048, 5632), (8200, 640)])
+def test_gemm32_rows_of_few(n, k):
+    """A row's result is the same bits whichever of 1 to 64 rows come with it: whatever the tile, K is shared out in the same way and
+    the shares' sums are added in the same order.  The activation in the product's epilogue takes the same sums."""
+    a, w = rnd(64, k, seed=41).to(DEV), rnd(n, k, seed=42, scale=k ** -0.5).to(DEV)
+    whole = ops().gemm32(torch.empty(64, n, device=DEV), a, w)
+    for m in (1, 2, 7, 8, 9, 16, 17, 32, 33):
+        assert torch.equal(ops().gemm32(torch.empty(m, n, device=DEV), a[:m], w), whole[:m])
+    if n % 2 == 0:
+        unit = ops().silu_mul(torch.empty(64, n // 2, device=DEV), whole)
+        for m in (1, 8, 9, 16):
+            assert torch.equal(ops().gemm32_gated(torch.empty(m, n // 2, device=DEV), a[:m], w), unit[:m])
+
+
 @pytest.mark.parametrize("m,inter,k", [(1, 4100, 512), (2, 5632, 2048), (16, 4099, 516), (9, 2041, 1028), (3, 5, 512)])
 def test_gemm32_gated(m, inter, k):
-    """To the bit the product and the activation behind it, where the product is summed by the same waves (its tiles of 8 weight rows
-    are not); units that do not fill a tile, rows of a wider matrix, nothing beside the result."""
+    """To the bit the product and the activation behind it; units that do not fill a tile, rows of a wider matrix, nothing beside the
+    result."""
     a, w = rnd(m, k + 4, seed=31).to(DEV)[:, :k], rnd(2 * inter, k, seed=32, scale=k ** -0.5).to(DEV)
     out = torch.full((m + 1, inter + 3), 7.0, device=DEV)
     ops().gemm32_gated(out[:m, :inter], a, w)
     assert bool((out[m:] == 7.0).all()) and bool((out[:, inter:] == 7.0).all())
     both = ops().gemm32(torch.empty(m, 2 * inter, device=DEV), a, w)
     want = ops().silu_mul(torch.empty(m, inter, device=DEV), both)
-    if m > 8 or 2 * inter > 2048:
-        assert torch.equal(out[:m, :inter], want)
+    assert torch.equal(out[:m, :inter], want)
     # |silu'| <= 1.1 and |silu(g)| <= |g|: the sums' errors (test_gemm32_by_arrangement), and some roundings of the unit
     size = a.double().abs() @ w.double().abs().T * k * 2.0 ** -24
     g, u = (a.double() @ w.double().T).split(inter, 1)
