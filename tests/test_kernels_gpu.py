@@ -222,10 +222,15 @@ def test_silu_mul(dtype, inter):
 def test_silu_of_every_bfloat16():
     """silu of all 65,536 numbers: half a step of bfloat16 (8 bits: up to 2^-8 of the value), a few
     roundings of 32-bit arithmetic, and 89 * 2^-128 < 2^-121 where exp(-x) is beyond 2^128 and the result 0; infinities and NaN as the formula
-    gives them."""
+    gives them.  And the very number that expf and a division give: rows of an odd width go to the kernel that has them."""
     x = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
     rows = torch.stack([x.view(8, -1), torch.ones(8, 8192, dtype=torch.bfloat16)], 1).reshape(8, -1).contiguous()
     got = ops().silu_mul(torch.empty(8, 8192, dtype=torch.bfloat16, device=DEV), rows.to(DEV)).cpu().reshape(-1).double()
+    wide = torch.zeros(8, 2 * 8193, dtype=torch.bfloat16)
+    wide[:, :8192], wide[:, 8193:] = x.view(8, -1), 1.0
+    plain = ops().silu_mul(torch.empty(8, 8193, dtype=torch.bfloat16, device=DEV), wide.to(DEV)).cpu()[:, :8192].reshape(-1).double()
+    assert torch.equal(got.nan_to_num(7.0), plain.nan_to_num(7.0)) and torch.equal(got.isnan(), plain.isnan())
+    assert torch.equal(got.signbit()[~got.isnan()], plain.signbit()[~got.isnan()])
     x = x.double()
     want = x / (1 + torch.exp(-x))
     odd = want.isnan() | want.isinf()

@@ -53,3 +53,22 @@ def test_the_tile_of_a_32_bit_product_by_all_its_sizes(m, n, k, micros):
 
     tile = library.load("gemm32").llms_gemm32_tile(m, n, k, 256)
     assert micros[tile] <= 1.1 * min(micros)
+
+
+def test_which_compute_units_bring_a_weight_nearer():
+    """Those without a tile, where they are enough for the whole weight and memory has time for it (1.1B shape: q, k, v bring o_proj's,
+    gate and up down_proj's); none where every compute unit has a tile."""
+    from llmserve.ops import library
+
+    def workers(m, n, rows, k=2048):
+        return library.gemm_tiles_workers(library.gemm_tiles_plan(m, n, k)[0], m, n, k, 1, rows * k * 2)
+
+    for m in (65, 130, 256, 320, 512, 560, 700, 1300, 2048):
+        assert workers(m, 2560, 2048) > 0
+    for m in (512, 560, 700, 1300):
+        assert workers(m, 11264, 5632) > 0
+    for m in (65, 130, 333):  # (the tiles wait for memory themselves)
+        assert workers(m, 11264, 5632) == 0
+    for m, n in ((1024, 2048), (2048, 4096), (4096, 8192)):
+        bm, bn, held = library.GEMM_TILES[library.gemm_tiles_plan(m, n, 2048)[0]][:3]
+        assert -(-m // bm) * -(-n // bn) % (256 * held) == 0 and workers(m, n, 1) == 0
