@@ -56,31 +56,11 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, v);
 }
 
-// A weight that a kernel further on reads, for workgroups of a kernel that leaves memory and compute units idle to bring nearer: into the
-// 256 MB memory-side cache.
-struct Near {
-    const void* from;
-    unsigned bytes;  // (the host checks: below 2 GB)
-    int workers;     // workgroups that do so, behind those of the kernel's own work; 0: none
+// A constant as the type of an argument.
+template <int N>
+struct Number {
+    static constexpr int n = N;
 };
-
-// Worker `at` of them, NW waves: a number of every 128-byte line goes to LDS, where nobody looks at it; `lds`: 256 bytes per wave.  Reads
-// stay inside the weight (its buffer descriptor), nothing is written to memory.
-template <int NW>
-__device__ __forceinline__ void bring_near(const Near& n, int at, void* lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
-    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(n.from), 0, n.bytes, 0x00020000);
-    const unsigned piece = LLMS_WAVE * 128u, stride = (unsigned)(n.workers * NW) * piece;  // (up to 2^30: no offset wraps)
-    for (unsigned o = (unsigned)(at * NW + wave) * piece; o < n.bytes; o += stride)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)((char*)lds + wave * 256), 4, o + lane * 128u, 0, 0, 0);
-    __builtin_amdgcn_s_waitcnt(0);  // (no load may find the workgroup gone)
-#endif
-}
-
-#define LLMS_REQUIRE_NEAR(n)                                                                                              \
-    LLMS_REQUIRE((n).workers >= 0 && (n).workers <= 4096 && ((n).workers == 0 || ((n).from && (uintptr_t)(n).from % 4 == 0 && (n).bytes < (1u << 31))), \
-                 "up to 4,096 workgroups bring up to 2 GB nearer, aligned to 4 bytes")
 
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(bf16 v) { return bf16_bits_to_f32(v.bits); }
@@ -122,8 +102,9 @@ __device__ __forceinline__ float2 rotate_pair(float a, float b, float cs, float 
 // x / (1 + exp(-x)) of an x that is a bfloat16 number: once rounded to bfloat16 again, for each of the 65,536 such x the number
 // that expf and a division in 32-bit give.  The hardware's exp2 and reciprocal (one Newton step) are 9 instructions where those
 // are some 35, which is what an epilogue of a product spends its time on.  Numerator and denominator are a quarter of what
-// they stand for, so that the reciprocal of up to 2^128 is no denormal number; the bound keeps the Newton step free of
-// infinities.
+// they stand for, so that the reciprocal of up to 2^126 is no denormal number.  The bound keeps the Newton step free of infinities, and
+// what it relies on is that the hardware's reciprocal gives 0 where its result would be a denormal number, as beyond the bound: x
+// below -89 gives -0 and -infinity NaN, as the formula does.
 __device__ __forceinline__ float silu_of_bf16(float x) {
     const float d = fminf(0.25f + __builtin_amdgcn_exp2f(fmaf(x, -1.44269504f, -2.f)), 1.5e38f);
     const float r = __builtin_amdgcn_rcpf(d);

@@ -149,11 +149,6 @@ __global__ __launch_bounds__(WAVES* LLMS_WAVE) void gemm32_stream_kernel(float* 
 }
 
 // ------------------------------------------------------------------------------ tiles
-template <int N>
-struct Number {
-    static constexpr int n = N;
-};
-
 // Bound by the matrix cores (157 TFLOP/s in 32-bit) once there are several large tiles for every compute unit: an instruction of 32
 // cycles needs 8 bytes of LDS per lane, so one buffer and a plain order of stages are enough (4096 x 4096 at 2,048 rows 502
 // microseconds, 137 TFLOP/s).  With few rows a compute unit has one or two workgroups, which wait for each stage in turn: the small

@@ -41,6 +41,27 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 #define GT_GATED 2
 #define GT_ROTARY 3
 
+// A weight that a kernel further on reads, for workgroups to bring nearer: into the 256 MB memory-side cache.
+struct Near {
+    const void* from;
+    unsigned bytes;  // (the host checks: below 2 GB)
+    int workers;     // workgroups that do so, behind those of the kernel's own work; 0: none
+};
+
+// Worker `at` of them, NW waves: a number of every 128-byte line goes to LDS, where nobody looks at it; `lds`: 256 bytes per wave.  Reads
+// stay inside the weight (its buffer descriptor), nothing is written to memory.
+template <int NW>
+__device__ __forceinline__ void bring_near(const Near& n, int at, void* lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(n.from), 0, n.bytes, 0x00020000);
+    const unsigned piece = LLMS_WAVE * 128u, stride = (unsigned)(n.workers * NW) * piece;  // (up to 2^30: no offset wraps)
+    for (unsigned o = (unsigned)(at * NW + wave) * piece; o < n.bytes; o += stride)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)((char*)lds + wave * 256), 4, o + lane * 128u, 0, 0, 0);
+    __builtin_amdgcn_s_waitcnt(0);  // (no load may find the workgroup gone)
+#endif
+}
+
 struct TilesArgs {
     const bf16* X;
     const bf16* W;
@@ -59,11 +80,6 @@ struct TilesArgs {
     bf16 *k_pool, *v_pool;
     int wide;                    // PLAIN, GATED: rows of C start on 16 bytes, not only on 8
     Near near;                   // for the workgroups behind those of the tiles
-};
-
-template <int N>
-struct Number {
-    static constexpr int n = N;
 };
 
 // Row of W behind row `r` (a multiple of 8) of the product's columns in the order the epilogue wants them: blocks of 16
@@ -490,7 +506,8 @@ int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* 
     a.ldc = ldc;
     a.part_stride = part_stride;
     a.near = Near{near, near_bytes, near_workers};
-    LLMS_REQUIRE_NEAR(a.near);
+    LLMS_REQUIRE(near_workers >= 0 && near_workers <= 4096 && (near_workers == 0 || (near && (uintptr_t)near % 4 == 0 && near_bytes < (1u << 31))),
+                 "gemm_tiles: up to 4,096 workgroups bring up to 2 GB nearer, aligned to 4 bytes");
     LLMS_REQUIRE(near_workers == 0 || epilogue == GT_GATED || epilogue == GT_ROTARY, "gemm_tiles: workers go with the gated and rotary epilogues");
     a.wide = ldc % 8 == 0 && (uintptr_t)C % 16 == 0;
     if (epilogue == GT_GATED) {
