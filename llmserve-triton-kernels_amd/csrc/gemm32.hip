@@ -391,7 +391,7 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
 }
 
 // c[M, inter] = silu(a wg^T) * (a wu^T), w = [wg; wu] of `inter` rows each: up to 16 rows, the activation in the product's epilogue (4.7
-// microseconds a launch of its own), with the sums and the arithmetic of llms_gemm32 and the activation behind it.
+// microseconds a launch of its own), with the sums and the arithmetic of llms_gemm32 and the activation behind it, to the bit.
 int llms_gemm32_gated(void* c, const void* a, const void* w, int M, int inter, int K, int lda, int ldc, int cus, hipStream_t stream) {
     LLMS_REQUIRE(M > 0 && M <= 16 && inter > 0 && K >= 512 && cus > 0, "gemm32_gated: 1 to 16 rows of 512 columns and more");
     LLMS_REQUIRE(K % 4 == 0 && lda % 4 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0, "gemm32_gated: rows of multiples of 4, 16-byte aligned");

@@ -18,10 +18,10 @@
 //
 // Measured (microseconds, weights from memory, the norm behind o_proj and down_proj included; in brackets the library's product
 // with the kernels behind it):
-//   1.1B shape    333 rows: q, k, v 11 (17), o_proj in 2 parts 14 (15), gate and up with SiLU 29 (36), down_proj in 4 parts 20 (24)
-//                 512 rows: 12 (20), 13 (16), 32 (38), 23 (25) in 2 parts;  2,048 rows: 28 (33), 27 (29), 95 (94), 59 (59)
-//   7B shape      333 rows: 54 (61), 27 (30), 77 (78), 48 (62);  512 rows: 57 (62), 32 (35), 107 (88), 57 (78);  2,048 rows: 185 (172), 71
-//                 (70), 314 (424), 160 (172)
+//   1.1B shape    333 rows: q, k, v 10 (16), o_proj in 2 parts 14 (15), gate and up with SiLU 27 (34), down_proj in 4 parts 24 (25)
+//                 512 rows: 11 (19), 13 (15), 30 (37), 26 (27) in 2 parts;  2,048 rows: 29 (34), 28 (29), 86 (95), 60 (59)
+//   7B shape      333 rows: 54 (59), 25 (27), 70 (78), 47 (59);  512 rows: 60 (63), 32 (32), 102 (88), 59 (75);  2,048 rows: 198 (179), 74
+//                 (72), 304 (422), 165 (174)
 // What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times
 // its matrix instructions); beyond, LDS and matrix cores together, and how evenly the tiles fill 256 compute units.
 //
@@ -399,8 +399,8 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     // bfloat16 rows go through LDS, a chunk of JC blocks of rows at a time, and leave in 16-byte pieces along whole rows of the
     // tile: as the lanes hold them (8 bytes of 16 rows an instruction) a matrix of 2,048 x 5,632 takes 11.2 microseconds to
     // store, in pieces along rows 5.6.  (32-bit rows have 64 bytes together as the lanes hold them: through LDS 17.3 microseconds for
-    // 512 rows of 2048 x 2048, directly 17.0.)  With four units worked out side by side gate and up of the 1.1B shape went from 33.8
-    // to 29.1 microseconds at 333 rows, from 37.2 to 31.9 at 512, and from 117.7 to 98.4 at 2,048 (tiles of 160 x 192).
+    // 512 rows of 2048 x 2048, directly 17.0.)  With four units worked out side by side gate and up of the 1.1B shape went from 32.2
+    // to 26.4 microseconds at 333 rows, from 34.9 to 29.3 at 512, and from 92.9 to 82.5 at 2,048.
     constexpr int ROW = EPI == GT_GATED ? BN : BN * 2, PITCH = ROW + 16;  // bytes
     constexpr int FIT = TILE / (WM * 16 * PITCH), JC = FIT < TM ? FIT : TM, CHUNKS = (TM + JC - 1) / JC;
     static_assert(JC > 0, "a block of rows fits");

@@ -339,8 +339,8 @@ def gemm32_gated_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def gemm32_gated(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """out[M, I] = silu(gate) * up with [gate, up] = a w^T, w = [gate; up] [2I, K]: float32, as `gemm32` and `silu_mul` behind it
-    give it, in one launch."""
+    """out[M, I] = silu(gate) * up with [gate, up] = a w^T, w = [gate; up] [2I, K]: float32, to the bit as `gemm32` and `silu_mul` behind
+    it give it, in one launch."""
     dev = _dev(out, a, w)
     _rows(w, "w", a.shape[1])
     m, k = a.shape
@@ -627,8 +627,9 @@ SLICE_K = 512  # what one workgroup of gemm_slices takes of K
 # Tiles of ops.gemm_tiles (the order is the launcher's): rows of x, rows of w, workgroups a compute unit holds, steps of 64
 # columns its LDS holds, and the microseconds a step takes with one workgroup on every compute unit and with all it holds:
 # fitted to 150 products (65 to 2,048 rows; K of 2,048 to 11,008, N of 2,048 to 22,016).  Over 600 products of 27 weights (K to
-# 28,672, N to 57,344) the plan below is 1.7 % off the best tile in the mean and 28 % at most (gated 16384 x 3072 at 544 rows 92
-# microseconds and 72; 2048 x 2048 there 20 and 17); refitted on them it was no better on weights left out of the fit.
+# 28,672, N to 57,344) the plan below was 1.7 % off the best tile in the mean and 28 % at most; refitted on them it was no better on
+# weights left out of the fit.  With the gated epilogue as it is now 72 gated products of 6 weights are 1.0 % off in the mean and 25 %
+# at most (16384 x 3072 at 544 rows 78 microseconds and 62).
 GEMM_TILES = ((64, 64, 2, 4, 0.20, 0.33), (96, 64, 2, 4, 0.255, 0.40), (128, 64, 1, 4, 0.31, 0.31), (96, 128, 1, 4, 0.39, 0.39),
               (128, 128, 1, 4, 0.50, 0.50), (128, 192, 1, 4, 0.755, 0.755), (192, 128, 1, 4, 0.62, 0.62), (192, 128, 2, 2, 0.94, 1.23),
               (256, 128, 1, 3, 0.85, 0.85), (160, 192, 1, 3, 0.81, 0.81), (192, 192, 1, 3, 0.90, 0.90), (256, 256, 1, 2, 1.47, 1.47))
@@ -676,12 +677,14 @@ GEMM_TILES_NEAR_RATE = 2.9e6
 def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: int, cus: int = 256) -> int:
     """How many workgroups beyond those of the tiles bring a weight of `nbytes` nearer: as many as do so in four fifths of a round's
     time, if there are as many compute units without a tile in the last round and memory has time for both weights; otherwise none.
-    Time saved in both products together, microseconds: gate and up with down_proj behind them (1.1B shape, 23 MB) 4.7 at 512 rows, 6.8
-    at 560, 3.1 at 700; q, k, v with o_proj (8 MB) 1.3 at 512, 2.3 at 593, 5.7 at 2,048.  A part of a weight gains nothing, since the
-    last tile decides (8 of 23 MB: -0.1 at 333 rows, -0.8 at 512); a large one gets in the way of the tiles' own (down_proj of the 7B
-    shape, 90 MB: -10.7 at 330 rows, -4.6 at 448), and so does any where the tiles themselves wait for memory (gate and up at 333 rows
-    take 2.2 more, down_proj 2.2 less).  With more workers than there are such compute units each would take a tile's place or be a
-    round of its own.  A rule by sizes alone."""
+    Time saved in both products together, microseconds: gate and up with down_proj behind them (1.1B shape, 23 MB) 4.5 at 512 rows, 6.0
+    at 560, 2.0 at 700, 4.0 at 1,300; q, k, v with o_proj (8 MB) 0.2 to 0.5 at 65 to 160 rows, 1.0 to 1.6 at 200 to 320, 3.0 at 512, 1.5
+    at 593, 3.1 at 2,048.  Over 119 such pairs of 7 layer shapes (2 to 34 MB, 65 to 2,048 rows) 0.9 in the median, -0.2 of 17.5 at worst
+    (2 MB, 512 rows).  A part of a weight gains nothing, since the last tile decides (8 of 23 MB: -0.1 at 333 rows, -0.8 at 512); a large
+    one gets in the way of the tiles' own (down_proj of the 7B shape, 90 MB: -10.7 at 330 rows, -4.6 at 448), and so does any where the
+    tiles themselves wait for memory (gate and up at 333 rows take 2.2 more, down_proj 2.2 less).  With more workers than there are
+    such compute units each would take a tile's place or be a round of its own.  A rule by sizes alone: it takes the compute units
+    without a tile to be idle, and where another stream's kernel is on them the two share them."""
     if not 0 < nbytes <= GEMM_TILES_NEAR_BYTES:
         return 0
     bm, bn, held, stages, one, full = GEMM_TILES[tile]

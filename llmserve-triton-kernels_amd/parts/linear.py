@@ -79,14 +79,18 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 # (1.05), gated 0.93 (1.04), rotation and cache store 0.77 (1.00), parts of K for a norm 0.81 (1.04).  The library's times jump from
 # size to size, so single products lie on the wrong side: 1 in 18 below the line is more than 5 percent slower in tiles, at most 19, and 1
 # in 6 beyond it more than 5 percent faster.  Single sizes, microseconds, tiles and library:
-#   plain   4608 x 2048 12 and 16 at 333 rows; 6144 x 2048 16 and 20 at 333, 57 and 46 at 2,048; 32000 x 2048 65 and 61 at 512
-#   gated   11264 x 2048 32 and 38 at 512 rows, 86 and 73 at 1,300; 22016 x 4096 61 and 62 at 200, 107 and 88 at 512, 188 and 162 at
-#           1,024; 28672 x 4096 428 and 355 at 2,048
-#   rotary  2560 x 2048 12 and 20 at 512 rows; 12288 x 4096 57 and 62 at 512, 106 and 90 at 1,024
-#   parts   4096 x 11008 57 and 78 at 512 rows; 8192 x 28672 159 and 313 at 200, 446 and 261 at 640
+#   plain   4608 x 2048 15 and 16 at 333 rows; 6144 x 2048 18 and 25 at 333, 52 and 46 at 2,048; 32000 x 2048 60 and 57 at 512
+#   gated   11264 x 2048 30 and 37 at 512 rows; 22016 x 4096 59 and 66 at 200, 101 and 87 at 512, 169 and 167 at 1,024; 28672 x 4096
+#           398 and 374 at 2,048
+#   rotary  2560 x 2048 11 and 19 at 512 rows; 12288 x 4096 60 and 62 at 512, 104 and 92 at 1,024
+#   parts   4096 x 11008 51 and 73 at 512 rows; 8192 x 28672 151 and 306 at 200, 430 and 263 at 640 (without the norm)
+# The gated line was drawn when the tiles' epilogue took up to a quarter longer than it does now: 5 to 20 % of such a product.  Beyond
+# it 11264 x 2048 is now the tiles' in truth (54 and 57 at 1,024 rows, 68 and 73 at 1,300, 72 and 81 at 1,536, 86 and 96 at 2,048), while
+# 22016 x 4096 and larger weights are still the library's where the line says so (98 and 85 at 400 rows, 28672 x 4096 152 and 145 at 640):
+# it has not been drawn anew.
 # Gated products of TILES_GATED_WORK and more against a weight below TILES_GATED_WEIGHT (200 MB, which the 256 MB memory-side cache
 # holds) are the tiles' again: 27 such products of 17 weights 0.95 in the mean, 0.72 to 1.19, where larger weights are at 1.05; 22016 x
-# 4096 at 2,048 rows 314 and 424.
+# 4096 at 2,048 rows 299 and 425 (the means, too, from before).
 # Plain products of TILES_LONG_K columns and more whose tiles leave half the compute units without one are the library's, which
 # shares their K out (one result cannot come in parts, and each tile walks all of K): 65 such products of 9 weights, from 65 rows on,
 # 1.17 in the mean.  2048 x 5632 28 and 16 at 128 rows, 25 and 21 at 228, but 28 and 33 at 613; 1024 x 4096 13 and 9 at 96.

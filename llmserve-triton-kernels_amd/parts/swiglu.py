@@ -3,8 +3,9 @@
 `limit`: down(g sigmoid(1.702 g) (u + 1)), g = min(gate(x), limit), u = clamp(up(x), -limit, limit); or "gelu_tanh":
 down(gelu(gate(x)) * up(x)) with the tanh form of gelu).
 gate_proj and up_proj are stacked into one [2I, H] matrix at load, so one product feeds
-the activation.  With few bfloat16 rows that product also does the activation after it
-(ops.gemm_stream); otherwise the product and the activation are kernels of their own."""
+the activation.  In bfloat16 that product does the activation in its epilogue (ops.gemm_decode, which also norms its rows,
+ops.gemm_stream, ops.gemm_tiles), and in 32-bit with up to 16 rows and SiLU (ops.gemm32_gated); products that go to the
+library, more 32-bit rows, and sizes those kernels do not take have the activation as a kernel of its own."""
 
 from __future__ import annotations
 
