@@ -38,8 +38,8 @@ __device__ __forceinline__ unsigned row_offset(int row, int rows, int ld) { retu
 
 // ------------------------------------------------------------------------------ few rows
 // Bound by reading the weight: 32000 x 2048 (262 MB) at 2 rows takes 48 microseconds (5.4 TB/s), 11264 x 2048 22 (4.1 TB/s),
-// 2048 x 2048 9 (a launch and one wait for memory); the multiply-add kernel, whose workgroup brings 64 weight rows through
-// LDS 4 bytes a load whatever the number of rows, takes 282, 216 and 197.  At 64 rows 111, 56 and 23: from some 20 rows on
+// 2048 x 2048 6 (a launch and one wait for memory); the multiply-add kernel, whose workgroup brings 64 weight rows through
+// LDS 4 bytes a load whatever the number of rows, takes 272, 210 and 202.  At 64 rows 118, 58 and 22: from some 20 rows on
 // every workgroup's reading of all rows of X out of L2 weighs more than the weight.
 // HALVES (up to 8 rows of A): a tile is 8 weight rows, and rows 8 to 15 of both operands hold the same rows' columns of another share of
 // K, so that D[i][j] and D[i + 8][j + 8] are two parts of one sum (the other two blocks of D mean nothing).  A weight of few rows
@@ -361,9 +361,9 @@ int llms_gemm32(void* c, const void* a, const void* w, const void* b, int M, int
     float* C = (float*)c;
     const float *A = (const float*)a, *W = (const float*)w, *bias = (const float*)b;
     const int wide = ldc % 4 == 0 && (uintptr_t)c % 16 == 0;
-    // Rows of fewer than 512 columns give the stream's waves a chunk each at most.  Tiles take some microseconds more there (2
-    // rows of 508 columns against 512 weight rows 8.6, of 512 columns in the stream 5.4; 40 rows 8.8 and 8.1; the multiply-add
-    // kernel 43 to 51), and what they sum in the order of the columns stays to the bit what small models gave before.
+    // Rows of fewer than 512 columns give the stream's waves a chunk each at most.  They go to the tiles (2 rows of 508 columns
+    // against 512 weight rows 5.4 microseconds, of 512 columns in the stream 3.5; 40 rows 5.6 and 8.1; the multiply-add kernel 48 to
+    // 53), whose sums in the order of the columns are to the bit what small models gave before.
     if (M <= 64 && K >= 512) {
         const unsigned tiles = (N + 15) / 16, pairs = (N + 31) / 32;
         if (M <= 16) {
