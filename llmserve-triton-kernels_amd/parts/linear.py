@@ -84,8 +84,7 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 #           398 and 374 at 2,048
 #   rotary  2560 x 2048 11 and 19 at 512 rows; 12288 x 4096 60 and 62 at 512, 104 and 92 at 1,024
 #   parts   4096 x 11008 51 and 73 at 512 rows; 8192 x 28672 151 and 306 at 200, 430 and 263 at 640 (without the norm)
-# The gated line was drawn when the tiles' epilogue took up to a quarter longer than it does now: 5 to 20 % of such a product.  Beyond
-# it 11264 x 2048 is now the tiles' in truth (54 and 57 at 1,024 rows, 68 and 73 at 1,300, 72 and 81 at 1,536, 86 and 96 at 2,048), while
+# The gated line was drawn when such products took 5 to 25 % longer in tiles, all of it in their epilogue.  Beyond it 11264 x 2048 is now the tiles' in truth (54 and 57 at 1,024 rows, 68 and 73 at 1,300, 72 and 81 at 1,536, 86 and 96 at 2,048), while
 # 22016 x 4096 and larger weights are still the library's where the line says so (98 and 85 at 400 rows, 28672 x 4096 152 and 145 at 640):
 # it has not been drawn anew.
 # Gated products of TILES_GATED_WORK and more against a weight below TILES_GATED_WEIGHT (200 MB, which the 256 MB memory-side cache
