@@ -6,24 +6,33 @@
 //   gated    W = [gate; up]: C[M,N/2] = silu(gate) * up (or the clamped unit, or gelu(gate) * up)
 //   rotary   W = [q; k; v]: C = rotated q; rotated k and v go to the tokens' cache slots
 //
-// Arrangement.  A workgroup of 4 or 8 waves owns a tile of BM rows of X by BN rows of W and walks K in steps of 64.  A step's
-// rows come into one of S buffers of LDS by loads that go there directly (8 rows of 128 bytes an instruction), S - 1 steps
-// ahead; a piece of 16 bytes lies at its place XOR the row, so that the 16 rows of a matrix operand are read without bank
-// conflicts.  Fragments are held twice: while the first half of a step is multiplied its second half is read, and while
-// that is multiplied the next step's first half is, so LDS and matrix cores work side by side and a step needs one barrier.
-// The buffers are variables of their own, and the loop is unrolled over them: only so does the compiler know that a read
-// of one buffer need not wait for the loads into another.  Instructions per wave tile of (BM / WM) x (BN / WN): the larger,
-// the fewer bytes of LDS per product (a 64 x 64 wave tile already asks LDS for as much as it can give), so the large tiles
-// run at 1.4 PFLOP/s in the loop and the small ones fill the chip when there are few rows.
+// Arrangement.  A workgroup owns a tile of BM rows of X by BN rows of W and walks K in steps of 64.  A step's rows come into LDS by
+// loads that go there directly (8 rows of 128 bytes an instruction), some steps ahead; a piece of 16 bytes lies at its place XOR
+// the row, so that the 16 rows of a matrix operand are read without bank conflicts.  Fragments are held twice: while the first half
+// of a step is multiplied its second half is read, and while that is multiplied the next step's first half is, so LDS and matrix
+// cores work side by side and a step needs one barrier.  Instructions per wave tile of (BM / WM) x (BN / WN): the larger, the fewer
+// bytes of LDS per product, so the large tiles run at 1.4 PFLOP/s in the loop and the small ones fill the chip when there are few rows.
 //
-// Measured (microseconds, weights from memory, the norm behind o_proj and down_proj included; in brackets the library's product
-// with the kernels behind it):
-//   1.1B shape    333 rows: q, k, v 10 (16), o_proj in 2 parts 14 (15), gate and up with SiLU 27 (34), down_proj in 4 parts 24 (25)
-//                 512 rows: 11 (19), 13 (15), 30 (37), 26 (27) in 2 parts;  2,048 rows: 29 (34), 28 (29), 86 (95), 60 (59)
-//   7B shape      333 rows: 54 (59), 25 (27), 70 (78), 47 (59);  512 rows: 60 (63), 32 (32), 102 (88), 59 (75);  2,048 rows: 198 (179), 74
-//                 (72), 304 (422), 165 (174)
-// What bounds them: up to some 300 rows the answer of memory (a step of a 64 x 64 tile takes 0.17 microseconds, four times
-// its matrix instructions); beyond, LDS and matrix cores together, and how evenly the tiles fill 256 compute units.
+// Who loads, and in which order.  A compute unit has some 40 KB of answers outstanding, however many buffers there are (more than 10
+// instructions of 1 KB a wave in flight change nothing), and they come back in the order they were asked for: a row of X from L2 behind
+// a row of W from memory waits as long as that.  So what counts is how often the queue stands still for memory, and the order decides
+// it: U = 2 to 4 steps of W asked for in one piece, then X step by step, stand still once where a step of X and a step of W in turn
+// stand still every time (loads alone, 128 x 128 tiles of 2048 x 5632 at 2,048 rows 52.8 -> 45.3 microseconds; 192 x 128 of 11264 x
+// 2048 at 333 22.8 -> 19.7; weights in the memory-side cache: no difference).  That needs waves that do nothing but load (NP of them,
+// one per SIMD): where the waves that multiply ask for four steps' worth at once, their matrix instructions wait behind their own loads
+// (192 x 128 at 333 rows 26.6 -> 27.8, and 25.5 with waves for it).  The rings of X (SX steps) and of W (SW) are as long as LDS allows.
+// Taller tiles of fewer weight rows (192 x 96, 256 x 96) ask memory for less.  Tiles of one wave per SIMD that load for themselves (NP
+// = 0) stay where a compute unit holds two workgroups, where the weight mostly lies in the memory-side cache, and for 256 x 256, whose
+// accumulators leave no registers for more waves.  There the buffers are variables of their own and the loop is unrolled over them: only
+// so does the compiler know that a read of one buffer need not wait for the loads into another.
+//
+// Measured (microseconds, weights from memory; in brackets one wave per SIMD that loads for itself):
+//   11264 x 2048 gated     333 rows 23.4 (26.5), 512: 27.6 (29.8), 544: 31.7 (32.6), 768: 35.9 (39.7)
+//   2048 x 5632 in parts   512 rows 21.2 (24.4), 640: 26.4 (29.0); one part, 2,048 rows: 51.5 (57.1)
+//   2560 x 2048            333 rows 10.3 (11.0), 640: 13.5 (15.6), 2,048: 26.1 (27.4);   2048 x 2048, 2,048 rows 21.5 (22.9)
+//   12288 x 4096           256 rows 36.9 (46.8), 333: 42.1 (47.8), 2,048: 170.8 (181.7); 22016 x 4096 gated, 1,024 rows 162 (175)
+// What bounds them: the loads, up to some 600 rows (without matrix instructions the same launches take 0.85 to 0.95 of the time);
+// beyond, matrix cores at the clock they hold (1.5 to 1.7 PFLOP/s without loads) and how evenly the tiles fill 256 compute units.
 //
 // Compute units without a tile bring a weight that a later kernel multiplies with nearer (`near`).
 //
@@ -141,22 +150,26 @@ __device__ __forceinline__ u32x2 gt_units(const TilesArgs& a, const f32x4& gate,
 
 // Workgroups beyond those of the tiles bring a weight that a later kernel multiplies with nearer (`near`).  A tile's loads are
 // answered in order, those of weights from memory hold up those of rows from L2 behind them, and no depth of fetching ahead made
-// up for it (buffers of 4, 5 and 6 steps: the same times); with its weight in the memory-side cache 2048 x 5632 at 512 rows in 2
+// up for it; with its weight in the memory-side cache 2048 x 5632 at 512 rows in 2
 // parts takes 17.1 microseconds where it takes 22.9 from memory, 2048 x 2048 8.9 and 11.8.  A layer's four products of the 1.1B shape at
 // 512 rows: 93.7 microseconds, 85.8 where q, k, v bring o_proj's weight (16 compute units without a tile) and gate and up
 // down_proj's (20).  What bounds a worker is what a compute unit has of misses in flight: 57 GB/s.
-template <int BM, int BN, int WM, int WN, int S, int EPI>
-__global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const TilesArgs a) {
+//
+// NP: waves that only load; without, every wave loads.  SX, SW: steps that LDS holds of X and of W; U: steps of W asked for at once.
+template <int BM, int BN, int WM, int WN, int NP, int SX, int SW, int U, int EPI>
+__global__ __launch_bounds__((WM * WN + NP) * LLMS_WAVE) void gemm_tiles_kernel(const TilesArgs a) {
     constexpr int NW = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
-    constexpr int LM = BM / 8 / NW, LN = BN / 8 / NW;  // loads of 8 rows, per wave
-    static_assert(LM * NW * 8 == BM && LN * NW * 8 == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile does not divide");
+    constexpr int NL = NP ? NP : NW;                   // waves that load
+    constexpr int LM = BM / 8 / NL, LN = BN / 8 / NL;  // loads of 8 rows, per wave
+    static_assert(LM * NL * 8 == BM && LN * NL * 8 == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile does not divide");
     static_assert(TN % 2 == 0, "columns that belong together lie in one wave");
-    static_assert(S >= 2 && S <= 4, "buffers");
-    constexpr int TILE = (BM + BN) * 128;
-    __shared__ __attribute__((aligned(1024))) uint8_t lds0[TILE];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds1[TILE];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds2[S > 2 ? TILE : 16];
-    __shared__ __attribute__((aligned(1024))) uint8_t lds3[S > 3 ? TILE : 16];
+    static_assert(NP ? SW % U == 0 && SW > U && SX > 2 : SX == SW && U == 1 && (SX == 2 || SX == 4), "buffers");
+    // lds0 with NP: SX steps of rows of X, then SW steps of rows of W.  Without: each buffer holds a step of both.
+    constexpr int XT = BM * 128, WT = BN * 128, LDS = NP ? SX * XT + SW * WT : XT + WT;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds0[LDS];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds1[NP ? 16 : LDS];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds2[NP || SX < 4 ? 16 : LDS];
+    __shared__ __attribute__((aligned(1024))) uint8_t lds3[NP || SX < 4 ? 16 : LDS];
 
     const int part = EPI == GT_FLOAT ? blockIdx.x / a.tiles : 0, pid = blockIdx.x - part * a.tiles;
     const int first = part * a.steps, steps = min(a.steps, a.K / 64 - first);
@@ -166,6 +179,7 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     const int t = xcd * full + min(xcd, rem) + pid / 8;
     const int m0 = (t % a.tiles_m) * BM, n0 = (t / a.tiles_m) * BN;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / LLMS_WAVE), lane = tid % LLMS_WAVE;
+    const int loader = NP ? wave - NW : wave;  // (NP: the last waves load, the others multiply)
     const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
     const int r16 = lane % 16, g = lane / 16;
 
@@ -183,30 +197,35 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     __amdgpu_buffer_rsrc_t xb[LM], wb[LN];
 #pragma unroll
     for (int i = 0; i < LM; ++i) {
-        int r = m0 + (wave * LM + i) * 8;
+        int r = m0 + (loader * LM + i) * 8;
         r = r < a.M ? r : 0;
         xb[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.X + (size_t)r * a.ldx), 0,
                                                   (unsigned)((min(8, a.M - r) - 1) * a.ldx + a.K) * 2u, 0x00020000);
     }
 #pragma unroll
     for (int i = 0; i < LN; ++i) {
-        const int c = n0 + (wave * LN + i) * 8;
+        const int c = n0 + (loader * LN + i) * 8;
         wb[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a.W + (size_t)(c < a.N ? gt_weight_row<EPI>(a, c) : 0) * a.K), 0,
                                                   (unsigned)(8 * a.K) * 2u, 0x00020000);
     }
-    auto fetch = [&](uint8_t* lds, int step) {
+    auto fetch_x = [&](uint8_t* x, int step) {
 #if defined(__HIP_DEVICE_COMPILE__)
         const bool live = step < steps;
         const int so = live ? (first + step) * 128 : 0;
-        const unsigned xo = live ? x_off : 0x80000000u, wo = live ? w_off : 0x80000000u;
+        const unsigned off = live ? x_off : 0x80000000u;
 #pragma unroll
         for (int i = 0; i < LM; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(xb[i], (__attribute__((address_space(3))) void*)(lds + (wave * LM + i) * 1024), 16, xo,
-                                                     so, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xb[i], (__attribute__((address_space(3))) void*)(x + (loader * LM + i) * 1024), 16, off, so, 0, 0);
+#endif
+    };
+    auto fetch_w = [&](uint8_t* w, int step) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        const bool live = step < steps;
+        const int so = live ? (first + step) * 128 : 0;
+        const unsigned off = live ? w_off : 0x80000000u;
 #pragma unroll
         for (int i = 0; i < LN; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                wb[i], (__attribute__((address_space(3))) void*)(lds + BM * 128 + (wave * LN + i) * 1024), 16, wo, so, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(wb[i], (__attribute__((address_space(3))) void*)(w + (loader * LN + i) * 1024), 16, off, so, 0, 0);
 #endif
     };
 
@@ -217,12 +236,12 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
 #pragma unroll
         for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     bf16x8 wf[2][TN], xf[2][TM];
-    auto read = [&](const uint8_t* lds, int half) {
+    auto read = [&](const uint8_t* x, const uint8_t* w, int half) {
         const int q = ((half * 4 + g) ^ (r16 & 7)) * 16;
 #pragma unroll
-        for (int i = 0; i < TN; ++i) wf[half][i] = *reinterpret_cast<const bf16x8*>(lds + BM * 128 + (wn + i * 16 + r16) * 128 + q);
+        for (int i = 0; i < TN; ++i) wf[half][i] = *reinterpret_cast<const bf16x8*>(w + (wn + i * 16 + r16) * 128 + q);
 #pragma unroll
-        for (int j = 0; j < TM; ++j) xf[half][j] = *reinterpret_cast<const bf16x8*>(lds + (wm + j * 16 + r16) * 128 + q);
+        for (int j = 0; j < TM; ++j) xf[half][j] = *reinterpret_cast<const bf16x8*>(x + (wm + j * 16 + r16) * 128 + q);
     };
     auto multiply = [&](int half) {
 #pragma unroll
@@ -241,61 +260,145 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
         }
         __builtin_amdgcn_sched_group_barrier(0x8, TM * TN, 0);
     };
-    // waits until at most `left` steps' loads of this wave are in flight (and its LDS reads are done), then for all waves
+    // waits until at most `left` loads of this wave are in flight (and its LDS reads are done), then for all waves
     auto arrive = [&](auto left) {
-        constexpr int n = decltype(left)::n * (LM + LN);
+        constexpr int n = decltype(left)::n;
         static_assert(n < 64, "the counter of loads in flight");
         __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | 0x0070);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    // One step: `now` holds it, its first half is in registers; `next` holds the step behind it.  At the barrier every wave
-    // has read all of `now`, which then takes the step S further on.
-    int step = 0;
-    auto one = [&](uint8_t* now, uint8_t* next) {
-        read(now, 1);
-        multiply(0);
-        interleave(Number<0>());
-        __builtin_amdgcn_sched_barrier(0);
-        arrive(Number<S - 2>());
-        __builtin_amdgcn_sched_barrier(0);
-        fetch(now, step + S);
-        read(next, 0);
-        multiply(1);
-        interleave(Number<LM + LN>());
-        __builtin_amdgcn_sched_barrier(0);
-        ++step;
-    };
     // (Here and not at the start: behind a branch there the arguments would be asked for a second time, 0.4 microseconds a launch; what
     // a worker has worked out so far is in bounds and not used.  Products that come in parts have no workers, and were 0.4 slower with
     // this code in their kernel.)
     if constexpr (EPI == GT_GATED || EPI == GT_ROTARY) {
         if (__builtin_expect((int)blockIdx.x >= a.workgroups, 0)) {
-            bring_near<NW>(a.near, blockIdx.x - a.workgroups, lds0);
+            bring_near<NW + NP>(a.near, blockIdx.x - a.workgroups, lds0);
             return;
         }
     }
-    fetch(lds0, 0);
-    fetch(lds1, 1);
-    if constexpr (S > 2) fetch(lds2, 2);
-    if constexpr (S > 3) fetch(lds3, 3);
-    arrive(Number<S - 1>());
-    read(lds0, 0);
-    for (int rounds = (steps + S - 1) / S; rounds > 0; --rounds) {
-        one(lds0, lds1);
-        if constexpr (S == 2) {
-            one(lds1, lds0);
-        } else if constexpr (S == 3) {
-            one(lds1, lds2);
-            one(lds2, lds0);
-        } else {
-            one(lds1, lds2);
-            one(lds2, lds3);
-            one(lds3, lds0);
+    if constexpr (NP == 0) {
+        // One step: `now` holds it, its first half is in registers; `next` holds the step behind it.  At the barrier every wave
+        // has read all of `now`, which then takes the step SX further on.
+        int step = 0;
+        auto fetch = [&](uint8_t* lds, int at) {
+            fetch_x(lds, at);
+            fetch_w(lds + XT, at);
+        };
+        auto one = [&](uint8_t* now, uint8_t* next) {
+            read(now, now + XT, 1);
+            multiply(0);
+            interleave(Number<0>());
+            __builtin_amdgcn_sched_barrier(0);
+            arrive(Number<(SX - 2) * (LM + LN)>());
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(now, step + SX);
+            read(next, next + XT, 0);
+            multiply(1);
+            interleave(Number<LM + LN>());
+            __builtin_amdgcn_sched_barrier(0);
+            ++step;
+        };
+        fetch(lds0, 0);
+        fetch(lds1, 1);
+        if constexpr (SX == 4) {
+            fetch(lds2, 2);
+            fetch(lds3, 3);
         }
+        arrive(Number<(SX - 1) * (LM + LN)>());
+        read(lds0, lds0 + XT, 0);
+        for (int rounds = (steps + SX - 1) / SX; rounds > 0; --rounds) {
+            one(lds0, lds1);
+            if constexpr (SX == 2) {
+                one(lds1, lds0);
+            } else {
+                one(lds1, lds2);
+                one(lds2, lds3);
+                one(lds3, lds0);
+            }
+        }
+        arrive(Number<0>());  // (no load may find the workgroup gone)
+    } else if (wave >= NW) {
+        // What is asked for at the barrier behind step t, where the places of that step are free: if it is the last of U, U steps of W,
+        // then a step of X.  Step s + 1 is there when at most `left` loads are in flight: those asked for behind it until then.
+        int xs = 0, ws = 0;  // the places that are asked for next
+        auto next_x = [&](int step) {
+            fetch_x(lds0 + xs * XT, step);
+            xs = xs + 1 < SX ? xs + 1 : 0;
+        };
+        auto next_w = [&](int from) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                fetch_w(lds0 + SX * XT + ws * WT, from + u);
+                ws = ws + 1 < SW ? ws + 1 : 0;
+            }
+        };
+        constexpr int BEFORE = SX > SW - U + 1 ? SX : SW - U + 1;
+#pragma unroll
+        for (int t = -BEFORE; t < -1; ++t) {
+            if ((t + 64 * U) % U == U - 1 && t + SW - U + 1 >= 0) next_w(t + SW - U + 1);
+            if (t + SX >= 0) next_x(t + SX);
+        }
+        // (from -1 on: there the first step is waited for)
+        auto go = [&](int t, auto phase) {  // phase: t modulo U
+            constexpr int P = decltype(phase)::n, J = (P + 1) % U;
+            constexpr int BACK_X = SX - 1, BACK_W = SW - U + J;  // step t + 1 was asked for that many barriers ago: X, W
+            constexpr auto asked = [](int back) {      // loads asked for at the `back - 1` barriers before this one
+                int n = 0;
+                for (int b = 1; b < back; ++b) n += LM + ((P - b + 64 * U) % U == U - 1 ? U * LN : 0);
+                return n;
+            };
+            constexpr int X_LEFT = asked(BACK_X), W_LEFT = asked(BACK_W) + (U - 1 - J) * LN + LM;
+            constexpr int LEFT = X_LEFT < W_LEFT ? X_LEFT : W_LEFT;
+            arrive(Number<(LEFT < 63 ? LEFT : 63)>());
+            if (P == U - 1) next_w(t + SW - U + 1);
+            next_x(t + SX);
+        };
+        int t = -1;
+        go(t++, Number<U - 1>());
+        while (t < steps - 1) {
+            go(t++, Number<0>());
+            if constexpr (U > 1) {
+                if (t >= steps - 1) break;
+                go(t++, Number<1>());
+            }
+            if constexpr (U > 2) {
+                if (t >= steps - 1) break;
+                go(t++, Number<2>());
+            }
+            if constexpr (U > 3) {
+                if (t >= steps - 1) break;
+                go(t++, Number<3>());
+            }
+        }
+        arrive(Number<0>());  // (no load may find the workgroup gone, nor what the epilogue keeps in LDS)
+        return;
+    } else {
+        int xs = 0, ws = 0;
+        arrive(Number<63>());
+        read(lds0, lds0 + SX * XT, 0);
+        for (int step = 0; step < steps - 1; ++step) {
+            const uint8_t* x = lds0 + xs * XT;
+            const uint8_t* w = lds0 + SX * XT + ws * WT;
+            read(x, w, 1);
+            multiply(0);
+            interleave(Number<0>());
+            __builtin_amdgcn_sched_barrier(0);
+            arrive(Number<63>());
+            __builtin_amdgcn_sched_barrier(0);
+            xs = xs + 1 < SX ? xs + 1 : 0;
+            ws = ws + 1 < SW ? ws + 1 : 0;
+            read(lds0 + xs * XT, lds0 + SX * XT + ws * WT, 0);
+            multiply(1);
+            interleave(Number<0>());
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        read(lds0 + xs * XT, lds0 + SX * XT + ws * WT, 1);
+        multiply(0);
+        multiply(1);
+        arrive(Number<63>());
     }
-    arrive(Number<0>());  // (no load may find the workgroup gone)
 
     // ---- epilogue: a lane holds 4 consecutive columns of row m in each acc[i][j]; blocks i and i + 1 (i even) belong together
     if constexpr (EPI == GT_ROTARY) {
@@ -303,7 +406,7 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
         // The angles of a pair of blocks are asked for before the pair in front of them is stored: behind the stores, each row's
         // would be waited for on its own (the compiler cannot know that they do not overlap), which took 10 microseconds of
         // the 36 that q, k and v of 2,048 rows of the 1.1B shape took.
-        constexpr int AHEAD = NW == 4 ? 2 : 1;  // (8 waves leave no registers for a second pair's)
+        constexpr int AHEAD = NW + NP == 4 || TM * TN <= 24 ? 2 : 1;  // (8 waves with large tiles leave no registers for a second pair's)
         f32x4 table[AHEAD][TM][2];
         auto ask = [&](int i) {
             const int c = n0 + wn + i * 16;  // (the same for all lanes: the branches on it are uniform)
@@ -402,7 +505,7 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     // 512 rows of 2048 x 2048, directly 17.0.)  With four units worked out side by side gate and up of the 1.1B shape went from 32.2
     // to 26.4 microseconds at 333 rows, from 34.9 to 29.3 at 512, and from 92.9 to 82.5 at 2,048.
     constexpr int ROW = EPI == GT_GATED ? BN : BN * 2, PITCH = ROW + 16;  // bytes
-    constexpr int FIT = TILE / (WM * 16 * PITCH), JC = FIT < TM ? FIT : TM, CHUNKS = (TM + JC - 1) / JC;
+    constexpr int FIT = LDS / (WM * 16 * PITCH), JC = FIT < TM ? FIT : TM, CHUNKS = (TM + JC - 1) / JC;
     static_assert(JC > 0, "a block of rows fits");
     constexpr int RC = WM * JC * 16, PP = ROW / 16, THREADS = NW * LLMS_WAVE;
     const int left = EPI == GT_GATED ? a.inter - n0 / 2 : a.N - n0;  // columns from the tile's first on
@@ -410,6 +513,7 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
 #pragma unroll
     for (int chunk = 0; chunk < CHUNKS; ++chunk) {
         const int j0 = chunk * JC;
+        static_assert(NP == 0 || CHUNKS == 1, "the tile fits");
         uint8_t* const stage = chunk % 2 ? lds1 : lds0;
         uint8_t* const mine = stage + ((wave % WM) * (JC * 16) + r16) * PITCH;
         if constexpr (EPI == GT_GATED) {
@@ -456,7 +560,7 @@ __global__ __launch_bounds__(WM* WN* LLMS_WAVE) void gemm_tiles_kernel(const Til
     }
 }
 
-template <int BM, int BN, int WM, int WN, int S>
+template <int BM, int BN, int WM, int WN, int NP, int SX, int SW, int U>
 static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
     LLMS_REQUIRE(a.K % 64 == 0, "gemm_tiles: K must be a multiple of 64");
     const int tiles_n = (a.N + BN - 1) / BN;
@@ -467,11 +571,11 @@ static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
     LLMS_REQUIRE((long long)(parts - 1) * a.steps < a.K / 64, "gemm_tiles: a part of K is empty");
     a.workgroups = a.tiles * parts;
     LLMS_REQUIRE((long long)a.workgroups + a.near.workers < (1ll << 31), "gemm_tiles: too many workgroups");
-    const dim3 grid((unsigned)(a.workgroups + a.near.workers)), block(WM * WN * LLMS_WAVE);
-    if (epilogue == GT_PLAIN) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_PLAIN><<<grid, block, 0, stream>>>(a);
-    else if (epilogue == GT_FLOAT) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_FLOAT><<<grid, block, 0, stream>>>(a);
-    else if (epilogue == GT_GATED) gemm_tiles_kernel<BM, BN, WM, WN, S, GT_GATED><<<grid, block, 0, stream>>>(a);
-    else gemm_tiles_kernel<BM, BN, WM, WN, S, GT_ROTARY><<<grid, block, 0, stream>>>(a);
+    const dim3 grid((unsigned)(a.workgroups + a.near.workers)), block((WM * WN + NP) * LLMS_WAVE);
+    if (epilogue == GT_PLAIN) gemm_tiles_kernel<BM, BN, WM, WN, NP, SX, SW, U, GT_PLAIN><<<grid, block, 0, stream>>>(a);
+    else if (epilogue == GT_FLOAT) gemm_tiles_kernel<BM, BN, WM, WN, NP, SX, SW, U, GT_FLOAT><<<grid, block, 0, stream>>>(a);
+    else if (epilogue == GT_GATED) gemm_tiles_kernel<BM, BN, WM, WN, NP, SX, SW, U, GT_GATED><<<grid, block, 0, stream>>>(a);
+    else gemm_tiles_kernel<BM, BN, WM, WN, NP, SX, SW, U, GT_ROTARY><<<grid, block, 0, stream>>>(a);
     LLMS_LAUNCH_CHECK();
 }
 
@@ -535,18 +639,23 @@ int llms_gemm_tiles(int tile, int epilogue, void* C, const void* X, const void* 
         a.v_pool = (bf16*)v_pool;
     }
     switch (tile) {
-        case 0: return launch<64, 64, 2, 2, 4>(epilogue, a, parts, stream);
-        case 1: return launch<96, 64, 2, 2, 4>(epilogue, a, parts, stream);
-        case 2: return launch<128, 64, 2, 2, 4>(epilogue, a, parts, stream);
-        case 3: return launch<96, 128, 2, 2, 4>(epilogue, a, parts, stream);
-        case 4: return launch<128, 128, 2, 2, 4>(epilogue, a, parts, stream);
-        case 5: return launch<128, 192, 2, 2, 4>(epilogue, a, parts, stream);
-        case 6: return launch<192, 128, 2, 2, 4>(epilogue, a, parts, stream);
-        case 7: return launch<192, 128, 2, 2, 2>(epilogue, a, parts, stream);
-        case 8: return launch<256, 128, 2, 2, 3>(epilogue, a, parts, stream);
-        case 9: return launch<160, 192, 2, 2, 3>(epilogue, a, parts, stream);
-        case 10: return launch<192, 192, 2, 2, 3>(epilogue, a, parts, stream);
-        case 11: return launch<256, 256, 2, 4, 2>(epilogue, a, parts, stream);
+        case 0: return launch<64, 64, 2, 2, 0, 4, 4, 1>(epilogue, a, parts, stream);
+        case 1: return launch<96, 64, 2, 2, 0, 4, 4, 1>(epilogue, a, parts, stream);
+        case 2: return launch<128, 64, 2, 2, 0, 4, 4, 1>(epilogue, a, parts, stream);
+        case 3: return launch<96, 128, 2, 2, 4, 4, 4, 2>(epilogue, a, parts, stream);
+        case 4: return launch<128, 128, 2, 2, 4, 4, 4, 2>(epilogue, a, parts, stream);
+        case 5: return launch<160, 192, 2, 2, 4, 3, 3, 1>(epilogue, a, parts, stream);
+        case 6: return launch<192, 128, 2, 2, 4, 4, 4, 2>(epilogue, a, parts, stream);
+        case 7: return launch<192, 128, 2, 2, 0, 2, 2, 1>(epilogue, a, parts, stream);
+        case 8: return launch<256, 128, 2, 2, 4, 3, 4, 2>(epilogue, a, parts, stream);
+        case 9: return launch<192, 96, 4, 1, 4, 4, 4, 2>(epilogue, a, parts, stream);
+        case 10: return launch<192, 192, 2, 2, 4, 3, 3, 1>(epilogue, a, parts, stream);
+        case 11: return launch<256, 256, 2, 4, 0, 2, 2, 1>(epilogue, a, parts, stream);
+        case 12: return launch<64, 64, 2, 2, 4, 8, 8, 4>(epilogue, a, parts, stream);
+        case 13: return launch<96, 64, 2, 2, 4, 6, 8, 4>(epilogue, a, parts, stream);
+        case 14: return launch<128, 64, 2, 2, 4, 4, 8, 4>(epilogue, a, parts, stream);
+        case 15: return launch<192, 64, 2, 2, 4, 4, 8, 4>(epilogue, a, parts, stream);
+        case 16: return launch<256, 96, 4, 1, 4, 3, 4, 2>(epilogue, a, parts, stream);
     }
     LLMS_REQUIRE(false, "gemm_tiles: no such tile");
 }

@@ -624,36 +624,54 @@ def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias
 SLICE_K = 512  # what one workgroup of gemm_slices takes of K
 
 
-# Tiles of ops.gemm_tiles (the order is the launcher's): rows of x, rows of w, workgroups a compute unit holds, steps of 64
-# columns its LDS holds, and the microseconds a step takes with one workgroup on every compute unit and with all it holds:
-# fitted to 150 products (65 to 2,048 rows; K of 2,048 to 11,008, N of 2,048 to 22,016).  Over 600 products of 27 weights (K to
-# 28,672, N to 57,344) the plan below was 1.7 % off the best tile in the mean and 28 % at most; refitted on them it was no better on
-# weights left out of the fit.  With the gated epilogue as it is now 72 gated products of 6 weights are 1.0 % off in the mean and 25 %
-# at most (16384 x 3072 at 544 rows 78 microseconds and 62).
-GEMM_TILES = ((64, 64, 2, 4, 0.20, 0.33), (96, 64, 2, 4, 0.255, 0.40), (128, 64, 1, 4, 0.31, 0.31), (96, 128, 1, 4, 0.39, 0.39),
-              (128, 128, 1, 4, 0.50, 0.50), (128, 192, 1, 4, 0.755, 0.755), (192, 128, 1, 4, 0.62, 0.62), (192, 128, 2, 2, 0.94, 1.23),
-              (256, 128, 1, 3, 0.85, 0.85), (160, 192, 1, 3, 0.81, 0.81), (192, 192, 1, 3, 0.90, 0.90), (256, 256, 1, 2, 1.47, 1.47))
+# Tiles of ops.gemm_tiles (the order is the launcher's): rows of x, rows of w, workgroups a compute unit holds, steps of 64 columns that it
+# holds of w, then what a workgroup costs, microseconds: once, a step with all that a compute unit holds on every one, a step with one on
+# almost none, what comes to that with one on every compute unit; and the waves that only load.  Fitted to 9,700 products (17 weights of 1024
+# x 2048 to 22016 x 4096, 65 to 2,048 rows, up to 4 parts of K; weights from memory and, for what goes to a norm, from the memory-side
+# cache too).  The plan below is 0.7 % off the best tile in the mean over them and 13 % at most (900 rows against 1024 x 2048: 9.8
+# microseconds and 8.7).
+GEMM_TILES = ((64, 64, 2, 4, 0.098, 0.484, 0.198, 0.079, 0), (96, 64, 2, 4, 0.305, 0.587, 0.229, 0.093, 0),
+              (128, 64, 1, 4, 0.837, 0.409, 0.260, 0.137, 0), (96, 128, 1, 4, 1.070, 0.468, 0.327, 0.126, 4),
+              (128, 128, 1, 4, 1.725, 0.540, 0.405, 0.133, 4), (160, 192, 1, 3, 2.825, 0.822, 0.626, 0.190, 4),
+              (192, 128, 1, 4, 2.452, 0.684, 0.497, 0.197, 4), (192, 128, 2, 2, 1.132, 1.200, 0.810, 0.216, 0),
+              (256, 128, 1, 4, 2.769, 0.828, 0.598, 0.239, 4), (192, 96, 1, 4, 2.047, 0.561, 0.383, 0.204, 4),
+              (192, 192, 1, 3, 3.828, 0.900, 0.676, 0.222, 4), (256, 256, 1, 2, 4.870, 1.460, 1.268, 0.268, 0),
+              (64, 64, 1, 8, 0.963, 0.234, 0.176, 0.060, 4), (96, 64, 1, 8, 1.262, 0.308, 0.238, 0.056, 4),
+              (128, 64, 1, 8, 1.082, 0.354, 0.270, 0.096, 4), (192, 64, 1, 8, 1.651, 0.461, 0.332, 0.125, 4),
+              (256, 96, 1, 4, 2.267, 0.676, 0.481, 0.250, 4))
+
+# A weight that lies in the memory-side cache already: what a step takes where the waves that multiply load as well, of what it takes from
+# memory.  (Tiles whose loading waves wait for the weight together gain less.)  0.90 and 0.83: 1.0 and 1.5 % off for such weights, 0.7 here.
+GEMM_TILES_FROM_CACHE = 0.86
+
+
+def _gemm_tiles_rounds(tile: int, m: int, n: int, k: int, parts: int, cus: int) -> tuple[int, float, float]:
+    """Workgroups of the last round (0: it is full), microseconds of the rounds in front of it, and of it."""
+    bm, bn, held, buffers, once, full, one, fill, loaders = GEMM_TILES[tile]
+    steps = -(-(k // 64) // parts)
+    if not loaders:  # (these walk whole rounds of their buffers)
+        steps = -(-steps // buffers) * buffers
+    rounds, rest = divmod(-(-m // bm) * -(-n // bn) * parts, held * cus)
+    last = 0.0 if rest == 0 else once + steps * (full if rest > cus else one + fill * rest / cus)
+    return rest, rounds * (once + steps * full), last
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256) -> tuple[int, int]:
+def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256, near: bool = False) -> tuple[int, int]:
     """(tile, parts of K) for m rows against a weight [n, k]: the least of what the rounds over the compute units cost.  A
     round takes a tile's steps; the last one as much as its fullest compute unit has.  Parts of K (2 or 4, where the caller
     takes partial sums) fill the chip when there are few tiles, and cost writing and reading their 32-bit sums (2048 x 5632
-    with the norm behind it at 128 rows: 16.6 microseconds in four parts, 33 in one; at 1,024 rows 42 and 37.6).  A rule by
-    sizes alone."""
+    with the norm behind it at 128 rows: 16.6 microseconds in four parts, 33 in one; at 1,024 rows 42 and 37.6).  `near`: the weight
+    lies in the memory-side cache (a product in front brought it there).  A rule by sizes alone."""
     best = None
-    for tile, (bm, bn, held, stages, one, full) in enumerate(GEMM_TILES):
+    for tile in range(len(GEMM_TILES)):
         for parts in (1, 2, 4):
-            steps = -(-(k // 64) // parts)
-            if parts > most_parts or (parts - 1) * steps >= k // 64:
+            if parts > most_parts or (parts - 1) * -(-(k // 64) // parts) >= k // 64:
                 continue
-            steps = -(-steps // stages) * stages
-            workgroups = -(-m // bm) * -(-n // bn) * parts
-            rounds, rest = divmod(workgroups, held * cus)
-            cost = steps * (rounds * full + (0.0 if rest == 0 else one if rounds == 0 and rest <= cus else full)) + rounds + (rest > 0)
+            _, rounds, last = _gemm_tiles_rounds(tile, m, n, k, parts, cus)
+            cost = (rounds + last) * (GEMM_TILES_FROM_CACHE if near and not GEMM_TILES[tile][-1] else 1.0)
             if parts > 1:
-                cost += m * n * (6 * parts - 4) / 5.0e6
+                cost += m * n * ((6 * parts - 4) / 5.0e6 + parts / 2.0e6)
             if best is None or cost < best[0]:
                 best = (cost, tile, parts)
     return best[1:]
@@ -687,12 +705,10 @@ def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: in
     without a tile to be idle, and where another stream's kernel is on them the two share them."""
     if not 0 < nbytes <= GEMM_TILES_NEAR_BYTES:
         return 0
-    bm, bn, held, stages, one, full = GEMM_TILES[tile]
-    rounds, rest = divmod(-(-m // bm) * -(-n // bn) * parts, held * cus)
-    steps = -(-(-(-(k // 64) // parts)) // stages) * stages
-    last = steps * (one if rounds == 0 else full) + 2.0
+    rest, rounds, last = _gemm_tiles_rounds(tile, m, n, k, parts, cus)
+    last += 2.5  # (before the first step and behind the last)
     idle = cus - rest if 0 < rest < cus else 0
-    if idle * GEMM_TILES_WORKER_RATE * last < nbytes or 2 * n * k + nbytes > GEMM_TILES_NEAR_RATE * (rounds * steps * full + last):
+    if idle * GEMM_TILES_WORKER_RATE * 0.8 * last < nbytes or 2 * n * k + nbytes > GEMM_TILES_NEAR_RATE * (rounds + last):
         return 0
     return min(idle, -(-nbytes // int(0.8 * GEMM_TILES_WORKER_RATE * last)))
 
@@ -707,7 +723,7 @@ def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *, swiglu: bool = False,
                rope: dict | None = None, limit: float | None = None, gelu: bool = False, tile: int | None = None,
-               near: torch.Tensor | None = None) -> torch.Tensor:
+               near: torch.Tensor | None = None, from_cache: bool = False) -> torch.Tensor:
     """The product of many bfloat16 rows, and what follows it fused in.
 
     plain:   out[M, N] = x w^T (+ bias), bfloat16 or float32; float32 [parts, M, N]: the sums of that many parts of K.
@@ -717,7 +733,8 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
              the tokens' cache slots.
     `tile`: a place in GEMM_TILES; default by gemm_tiles_plan.
     `near` (with swiglu or rope): a contiguous weight that a kernel after this one reads: compute units without a tile bring it into the memory-side
-            cache meanwhile, where that pays (gemm_tiles_workers).  No result depends on it."""
+            cache meanwhile, where that pays (gemm_tiles_workers).  No result depends on it.
+    `from_cache`: w is such a weight, which the product in front brought there (another tile may then be the best)."""
     dev = _dev(out, x, w, bias, near)
     if x.dim() != 2 or x.stride(1) != 1 or out.dim() not in (2, 3) or out.stride(-1) != 1:
         raise ValueError("x must be 2-d, x and out with unit inner stride")
@@ -772,7 +789,8 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
     if m == 0:
         return out
     if tile is None:
-        tile = gemm_tiles_plan(m, n, k, 1, compute_units(dev))[0] if parts == 1 else _tile_for_parts(m, n, k, parts, compute_units(dev))
+        cus = compute_units(dev)
+        tile = gemm_tiles_plan(m, n, k, 1, cus, from_cache)[0] if parts == 1 else _tile_for_parts(m, n, k, parts, cus, from_cache)
     workers = near_bytes = 0
     if near is not None:
         if epilogue not in (2, 3):
@@ -788,8 +806,8 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
     return out
 
 
-def _tile_for_parts(m: int, n: int, k: int, parts: int, cus: int) -> int:
-    tile, planned = gemm_tiles_plan(m, n, k, 4, cus)
+def _tile_for_parts(m: int, n: int, k: int, parts: int, cus: int, near: bool) -> int:
+    tile, planned = gemm_tiles_plan(m, n, k, 4, cus, near)
     if planned != parts:
         raise ValueError(f"{m} rows against [{n}, {k}] are planned in {planned} parts of K; for {parts} name the tile")
     return tile

@@ -16,7 +16,7 @@ import math
 import torch
 
 from ..ops import library as ops
-from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums, tiles_product
+from .linear import adds_residual_in_epilogue, brings_near, decode_product, few_rows, linear, linear_partial_sums, tiles_product
 from .registry import ADDED_IN_PLACE, POSITION_ENCODINGS, DeferredNorm, Mixer, register_mixer
 from .spec import PagedCacheSpec, ParamInfo
 
@@ -75,6 +75,8 @@ class Attention(Mixer):
         slots = view.slots if cache.store else None
         deferred = x if isinstance(x, DeferredNorm) else None  # (then the result goes to a norm, which takes partial sums)
         q = self.project_and_store(x, batch, cache, slots)
+        rows = deferred.residual if deferred is not None else x
+        near = q is not None and self._in_tiles(rows) and brings_near(rows, self.qkv_weight, self.o_weight)
         if q is None:
             if deferred is not None:
                 x = deferred.materialize()
@@ -92,12 +94,16 @@ class Attention(Mixer):
         if deferred is not None and deferred.may_add_in_place and adds_residual_in_epilogue(out, self.o_weight):
             ops.gemm_decode(None, out, self.o_weight, residual=deferred.residual)  # the residual sum in the epilogue
             return ADDED_IN_PLACE
-        return (linear_partial_sums(out, self.o_weight) if deferred is not None else None) or linear(out, self.o_weight)
+        return (linear_partial_sums(out, self.o_weight, near) if deferred is not None else None) or linear(out, self.o_weight, from_cache=near)
 
     def _few_rows_unfit(self, rows) -> bool:
         if rows.dtype != torch.bfloat16 or self.head_dim % 16 != 0 or not ops.gemm_bf16_supported(rows, self.qkv_weight):
             return True
         return not (decode_product(rows, self.qkv_weight) or few_rows(rows.shape[0], self.qkv_weight) or self._fits_tiles(rows))
+
+    def _in_tiles(self, rows) -> bool:
+        """Of rows that project_and_store takes."""
+        return not decode_product(rows, self.qkv_weight) and not few_rows(rows.shape[0], self.qkv_weight)
 
     def _fits_tiles(self, rows) -> bool:
         return self.head_dim % 32 == 0 and tiles_product(rows, self.qkv_weight, "rotary")
@@ -124,7 +130,7 @@ class Attention(Mixer):
                     inv_freq=frequencies() if frequencies is not None else None, positions=batch.positions,
                     slots=slots, k_pool=cache.k_pool, v_pool=cache.v_pool, block_size=cache.block_size)
         q = torch.empty((m, self.num_heads * self.head_dim), dtype=rows.dtype, device=rows.device)
-        tiles = not decode and not few_rows(m, self.qkv_weight)
+        tiles = self._in_tiles(rows)
         if decode or tiles:
             angles = getattr(self.position, "rotary_angles", None)
             if angles is not None and getattr(batch, "shared", None) is not None:

@@ -84,31 +84,40 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 #           398 and 374 at 2,048
 #   rotary  2560 x 2048 11 and 19 at 512 rows; 12288 x 4096 60 and 62 at 512, 104 and 92 at 1,024
 #   parts   4096 x 11008 51 and 73 at 512 rows; 8192 x 28672 151 and 306 at 200, 430 and 263 at 640 (without the norm)
-# The gated line was drawn when such products took 5 to 25 % longer in tiles, all of it in their epilogue.  Beyond it 11264 x 2048 is now the tiles' in truth (54 and 57 at 1,024 rows, 68 and 73 at 1,300, 72 and 81 at 1,536, 86 and 96 at 2,048), while
-# 22016 x 4096 and larger weights are still the library's where the line says so (98 and 85 at 400 rows, 28672 x 4096 152 and 145 at 640):
-# it has not been drawn anew.
+# The gated line was drawn when such products took 10 to 30 % longer in tiles.  Against a weight below TILES_GATED_SMALL they are the tiles'
+# but in TILES_GATED_BAND, where only the measurements of then stand against it (11264 x 2048: 36 and 47 at 768 rows, 52 and 56 at 1,024,
+# 66 and 75 at 1,300, 78 and 99 at 1,629, 88 and 95 at 2,048); 22016 x 4096 and larger weights are still the library's at few rows (95 and
+# 89 at 512 rows).
 # Gated products of TILES_GATED_WORK and more against a weight below TILES_GATED_WEIGHT (200 MB, which the 256 MB memory-side cache
 # holds) are the tiles' again: 27 such products of 17 weights 0.95 in the mean, 0.72 to 1.19, where larger weights are at 1.05; 22016 x
 # 4096 at 2,048 rows 299 and 425 (the means, too, from before).
 # Plain products of TILES_LONG_K columns and more whose tiles leave half the compute units without one are the library's, which
 # shares their K out (one result cannot come in parts, and each tile walks all of K): 65 such products of 9 weights, from 65 rows on,
 # 1.17 in the mean.  2048 x 5632 28 and 16 at 128 rows, 25 and 21 at 228, but 28 and 33 at 613; 1024 x 4096 13 and 9 at 96.
+# Plain products whose tiles are one round that nine tenths of the compute units have a part in leave the library nothing to share out:
+# they are the tiles' up to where the band begins (2048 x 5632 at 2,048 rows 52 and 55).
 TILES_WORK = {"plain": 18e9, "gated": 18e9, "rotary": 40e9, "parts": 60e9}
 TILES_GATED_WORK = 130e9
 TILES_GATED_WEIGHT = 100e6
 TILES_LONG_K = 4096
+TILES_GATED_SMALL = 50e6
+TILES_GATED_BAND = (29e9, 36e9)
 
 
 def tiles_pay(kind: str, m: int, n: int, k: int, cus: int = 256) -> bool:
     """Whether m rows against a weight [n, k] are faster by ops.gemm_tiles ("plain", "gated" or "rotary" with what follows in the
     epilogue, "parts": K in parts for a norm to add up) than by the library: a rule by sizes alone."""
     work = m * n * k
-    if kind == "gated" and work >= TILES_GATED_WORK and n * k < TILES_GATED_WEIGHT:
-        return True
-    if kind == "plain" and m > 64 and k >= TILES_LONG_K:
+    if kind == "gated" and n * k < TILES_GATED_WEIGHT:
+        if work >= TILES_GATED_WORK or n * k < TILES_GATED_SMALL and not TILES_GATED_BAND[0] <= work < TILES_GATED_BAND[1]:
+            return True
+    if kind == "plain" and m > 64:
         rows, weight_rows = ops.GEMM_TILES[ops.gemm_tiles_plan(m, n, k, 1, cus)[0]][:2]
-        if 2 * -(-m // rows) * -(-n // weight_rows) <= cus:
+        tiles = -(-m // rows) * -(-n // weight_rows)
+        if k >= TILES_LONG_K and 2 * tiles <= cus:
             return False
+        if 0.9 * cus <= tiles <= cus and n * k < TILES_GATED_SMALL and work < TILES_GATED_BAND[0]:
+            return True
     return work < TILES_WORK[kind]
 
 
@@ -120,6 +129,13 @@ def tiles_fit(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def tiles_product(x: torch.Tensor, weight: torch.Tensor, kind: str = "plain") -> bool:
     """Whether a product of this kind goes there."""
     return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or tiles_pay(kind, x.shape[0], *weight.shape, ops.compute_units(x.device)))
+
+
+def brings_near(x: torch.Tensor, weight: torch.Tensor, near: torch.Tensor) -> bool:
+    """Whether ops.gemm_tiles, given x against weight with `near` behind it, has compute units left that bring `near` into the
+    memory-side cache: what the product of `near` is told (`from_cache`)."""
+    m, (n, k), cus = x.shape[0], weight.shape, ops.compute_units(x.device)
+    return ops.gemm_tiles_workers(ops.gemm_tiles_plan(m, n, k, 1, cus)[0], m, n, k, 1, near.numel() * near.element_size(), cus) > 0
 
 
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and
@@ -151,9 +167,9 @@ def slices_pay(m: int, weight: torch.Tensor) -> bool:
     return SPLIT_K and STREAM_ROWS < m <= STREAM_MAX_ROWS and weight.numel() * 2 <= SLICES_MAX_WEIGHT_BYTES
 
 
-def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor):
+def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor, from_cache: bool = False):
     """x W^T as `PartialSums` (K shared out to several workgroups per tile), or None where that does not
-    pay or does not apply; for callers whose result goes to a norm next."""
+    pay or does not apply; for callers whose result goes to a norm next.  `from_cache`: as for ops.gemm_tiles."""
     from .registry import PartialSums
 
     m = x.shape[0]
@@ -169,10 +185,10 @@ def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor):
         return PartialSums(ops.gemm_slices(parts, x, weight), x.dtype)
     if not few_rows(m, weight):
         if tiles_product(x, weight, "parts"):
-            k_parts = ops.gemm_tiles_plan(m, weight.shape[0], weight.shape[1], 4, ops.compute_units(x.device))[1]
+            k_parts = ops.gemm_tiles_plan(m, weight.shape[0], weight.shape[1], 4, ops.compute_units(x.device), from_cache)[1]
             if k_parts > 1:
                 parts = torch.empty((k_parts, m, weight.shape[0]), dtype=torch.float32, device=x.device)
-                return PartialSums(ops.gemm_tiles(parts, x, weight), x.dtype)
+                return PartialSums(ops.gemm_tiles(parts, x, weight, from_cache=from_cache), x.dtype)
         return None
     splits = k_splits_for(m, weight)
     if splits < 2:
@@ -190,8 +206,8 @@ def _tiles_take(out: torch.Tensor, bias: torch.Tensor | None, n: int) -> bool:
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
-           out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
-    """x [M, K] (unit inner stride), weight [N, K] -> [M, N] in out_dtype (default: x's)."""
+           out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None, from_cache: bool = False) -> torch.Tensor:
+    """x [M, K] (unit inner stride), weight [N, K] -> [M, N] in out_dtype (default: x's).  `from_cache`: as for ops.gemm_tiles."""
     out_dtype = out_dtype or x.dtype
     m, n = x.shape[0], weight.shape[0]
     if out is None:
@@ -204,7 +220,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
         if few_rows(m, weight):
             return ops.gemm_stream(out, x, weight, bias)
         if tiles_product(x, weight) and _tiles_take(out, bias, n):
-            return ops.gemm_tiles(out, x, weight, bias)
+            return ops.gemm_tiles(out, x, weight, bias, from_cache=from_cache)
         if OWN_KERNELS_ONLY:
             return ops.gemm_bf16(out, x, weight, bias, kernel="skinny" if m <= 64 else "tile")
         if bias is None:

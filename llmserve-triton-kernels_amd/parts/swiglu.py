@@ -12,7 +12,7 @@ from __future__ import annotations
 import torch
 
 from ..ops import library as ops
-from .linear import adds_residual_in_epilogue, decode_product, few_rows, linear, linear_partial_sums, tiles_product
+from .linear import adds_residual_in_epilogue, brings_near, decode_product, few_rows, linear, linear_partial_sums, tiles_product
 from .registry import ADDED_IN_PLACE, DeferredNorm, FeedForward, register_feed_forward
 from .spec import ParamInfo
 
@@ -54,6 +54,7 @@ class SwiGLU(FeedForward):
         m = rows.shape[0]
         dtype, device = self.gate_up.dtype, self.gate_up.device
         act = torch.empty((m, self.intermediate), dtype=dtype, device=device)
+        near = False
         if decode_product(rows, self.gate_up):
             norm = x.fused() if deferred and m <= ops.GEMM_DECODE_NORM_ROWS else None
             if norm is not None:
@@ -69,6 +70,7 @@ class SwiGLU(FeedForward):
                 ops.gemm_stream(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # activation in the product's epilogue
             elif not few and self.intermediate % 16 == 0 and tiles_product(rows, self.gate_up, "gated"):
                 ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu, near=self.down)  # the same
+                near = brings_near(rows, self.gate_up, self.down)
             elif self.unit == "silu" and ops.gemm32_gated_supported(rows, self.gate_up):
                 ops.gemm32_gated(act, rows, self.gate_up)  # the same, in 32-bit
             else:
@@ -76,8 +78,8 @@ class SwiGLU(FeedForward):
         if deferred and x.may_add_in_place and adds_residual_in_epilogue(act, self.down):
             ops.gemm_decode(None, act, self.down, residual=x.residual)  # the residual sum in the product's epilogue
             return ADDED_IN_PLACE
-        return (linear_partial_sums(act, self.down) if deferred else None) or linear(act, self.down,
-                                                                                       out_dtype=self.result_dtype)
+        return (linear_partial_sums(act, self.down, near) if deferred else None) or linear(act, self.down, out_dtype=self.result_dtype,
+                                                                                             from_cache=near)
 
 
 @register_feed_forward("none")

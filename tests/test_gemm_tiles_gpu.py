@@ -286,3 +286,48 @@ def test_a_weight_to_bring_nearer_that_is_refused():
         ops().gemm_tiles(torch.empty(128, 32, dtype=torch.bfloat16, device=DEV), x, w, swiglu=True, near=w.t())
     with pytest.raises(ValueError, match="near goes"):
         ops().gemm_tiles(torch.empty(128, 64, dtype=torch.bfloat16, device=DEV), x, w, near=w)
+
+
+def tiles_with(loading):
+    from llmserve.ops.library import GEMM_TILES
+
+    return [t for t, tile in enumerate(GEMM_TILES) if tile[-1] == loading]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(12, 17))
+def test_the_tiles_added_later(tile):
+    """As the others: edges of tiles, activations, rotation and cache store."""
+    test_plain_and_parts(tile)
+    for limit, gelu in ((None, False), (1.5, False), (None, True)):
+        test_gated(tile, limit, gelu)
+    for shape in ((4, 2, 64, 16, True), (2, 2, 128, 5, True)):
+        test_rotary(tile, *shape)
+    test_rows_of_every_alignment(tile, 4)
+    test_rotary_tokens_anywhere_in_their_pages(tile, 16, 5, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", tiles_with(4))
+def test_steps_of_k_where_some_waves_only_load(tile):
+    """From one step of K to beyond two rounds of the buffers, step by step: first, last and middle steps of what is asked for at once.
+    Rows beyond the matrix and two tiles; the parts are told apart by numbers that grow with the column."""
+    bm, bn, step = sizes_of(tile)
+    m, n = bm + 5, bn + 16
+    for steps in range(1, 2 * step // 64 + 4):
+        k = 64 * steps
+        x, w = rnd(m, k, seed=steps), rnd(n, k, seed=100 + steps) * (1 + torch.arange(k) // 64).to(torch.bfloat16)
+        out = torch.full((m, n), 7.0, device=DEV)
+        ops().gemm_tiles(out, x.to(DEV), w.to(DEV), tile=tile)
+        close(out, product(x, w), k, False)
+        if steps > 3 and 2 * -(-steps // 3) < steps:
+            sums = torch.full((3, m, n), 7.0, device=DEV)
+            ops().gemm_tiles(sums, x.to(DEV), w.to(DEV), tile=tile)
+            close(sums.double().sum(0), product(x, w), k, False)
+
+
+def test_plan_of_a_weight_in_the_cache():
+    """What lies in the memory-side cache already goes rather to tiles whose multiplying waves load."""
+    plan = ops().gemm_tiles_plan
+    loading = [ops().GEMM_TILES[plan(512, 2048, 2048, 1, 256, near)[0]][-1] for near in (False, True)]
+    assert loading == [4, 0]
