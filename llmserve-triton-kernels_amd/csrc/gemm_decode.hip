@@ -6,9 +6,9 @@
 //
 // A decode step is a chain of short launches; what each of them costs beyond the bytes of its weight is what it
 // does before its first load is out, the rows of X that every workgroup pulls in, and every launch that only
-// norms or adds.  Here a compute unit gets one workgroup of 16 waves, which owns an equal share of the weight rows
+// norms or adds.  Here a compute unit gets one workgroup of 8 waves, which owns an equal share of the weight rows
 // (every unit reads the same number of bytes) and whose waves share K out in chunks of 128 for good: wave w takes
-// chunks w, w + 16, ... of every tile.  So the part of X a wave needs is the same for all its tiles: it loads its
+// chunks w, w + 8, ... of every tile.  So the part of X a wave needs is the same for all its tiles: it loads its
 // chunks of the rows that exist (a load instruction per 4 rows), once, and leaves them in LDS, where the matrix
 // instruction's second operand is read from.  Because X enters a compute unit once, what is done to X on the way
 // in is paid once per unit as well: the RMSNorm of the rows (src/llmserve/model/llama.py:18-28; the workgroup
@@ -23,6 +23,12 @@
 // under a condition: the compiler counts the loads issued after the one it waits for, and where paths differ in
 // that count it waits for all.  Lanes whose row or column does not exist load through the buffer descriptor from
 // beyond its end, which brings zeros and touches no memory.
+//
+// Few waves, few loads in flight: a wave has two items (tile, chunk) asked for, 64 KB a compute unit.  With 16 waves and up to four items
+// each a layer's four products of the 1.1B shape took 25.3 microseconds at 1 row and 26.9 at 8, of the 7B shape (without down_proj) 66.0
+// and 68.2; with 8 waves and six or four items 24.6, 26.2, 63.1 and 65.6 (half the waves start and meet), with two items 23.8, 25.2, 58.0
+// and 60.7, with one 25.9, 27.6, 61.4 and 64.1: memory answers a compute unit some 40 KB at a time, and what all compute units ask for
+// beyond that comes from more open rows of memory at once.  The vocabulary's product, 32000 x 2048: 29.2 -> 22.8 (5.8 TB/s).
 //
 // Epilogues (the waves' partial sums meet in LDS in the order of the waves):
 //   PLAIN     C = sums (+ bias), float32 or bfloat16; `unit` 2: max(sums, 0)^2.
@@ -41,9 +47,9 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
-#define GD_NW 16     // waves of a workgroup
+#define GD_NW 8      // waves of a workgroup
 #define GD_KC 128    // elements of K per item
-#define GD_MAX_XC 3  // chunks of K per wave
+#define GD_MAX_XC 6  // chunks of K per wave
 #define GD_MAX_K (GD_NW * GD_MAX_XC * GD_KC)
 // LDS: the waves' tiles (later their partial sums), the rows' sums of squares, then the rows of X
 #define GD_LDS_TILES (GD_NW * 16 * (GD_KC / 8) * 16)
@@ -145,7 +151,7 @@ __device__ __forceinline__ int gd_weight_row(const DecodeGemmArgs& a, int u0, in
 // 1 / rms of M <= 16 rows whose waves' sums of squares lie in LDS, [row][wave]: lane l of a wave works out row l / 16 + 4 (l % 4),
 // once for all the rows its lanes will norm (up to 4 rows: row l / 16, the lanes of a group then read one address).  With every lane
 // working out each row in turn, 16 additions, a division and a root a row, that was half the vector instructions of the norm, which
-// 16 waves of a compute unit share its vector units for: q, k, v with the norm at 8 rows 5.85 -> 5.65 microseconds, at 16 rows 7.3 -> 6.5,
+// the waves of a compute unit share its vector units for (then 16 of them): q, k, v with the norm at 8 rows 5.85 -> 5.65 microseconds, at 16 rows 7.3 -> 6.5,
 // the same bits.
 template <int NW>
 __device__ __forceinline__ float gd_inverse_rms(const float* sq, int lane, int M, int K, float eps) {
@@ -296,7 +302,9 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     constexpr int UPT = PAIRS ? 8 : 4 * LPI;  // units per tile
     constexpr int ITEMS = NT * XC;            // items (tile, chunk) of a group
     // items in flight per wave; a divisor of ITEMS, so that an item has the same place in the ring in every group
-    constexpr int RING = ITEMS == 4 ? (XC == 1 ? 4 : 2) : (ITEMS < 3 ? ITEMS : 3);
+    constexpr int RING = ITEMS % 2 == 0 ? 2 : (ITEMS < 3 ? ITEMS : 3);
+    // ... of which this many are asked for before the rows of X are in LDS
+    constexpr int FIRST = PAIRS || XC > 2 ? RING : 1;
     static_assert(ITEMS % RING == 0, "the ring must go round a whole number of times per group");
     constexpr int THREADS = NW * LLMS_WAVE;
     constexpr int PLACES = PAIRS ? 128 : 16 * UPT;  // (unit or row, row of X) pairs of a tile: one thread each
@@ -369,9 +377,11 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
             w[i] = gd_load_streaming(w_buf, n >= 0 && kl < K ? (unsigned)(n * K + kl) * 2 : GD_NOWHERE);
         }
     };
-    // (a wave issues in order and waits when the memory pipeline is full: with all its loads asked for here it
-    // would get to the norm of its rows only after the pipeline has taken them all)
-    issue(ring[0], 0, 0);
+    // (a wave issues in order and waits when the memory pipeline is full: with much more asked for here it would get to the norm
+    // of its rows only after the pipeline has taken it all; q, k, v with the norm at 8 rows 5.68 microseconds with one item, 5.43 with
+    // both; gate and up 9.8 with two, 11.9 with six)
+#pragma unroll
+    for (int q = 0; q < FIRST; ++q) issue(ring[q], 0, q);
 
     // ---- the rows of X, normed if asked, go to LDS: only this wave reads its chunks there
     if (a.norm_weight) {
@@ -425,7 +435,7 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     }
 
 #pragma unroll
-    for (int q = 1; q < RING; ++q) issue(ring[q], 0, q);
+    for (int q = FIRST; q < RING; ++q) issue(ring[q], 0, q);
 
     u32x4* tile = lds + wave * 16 * (GD_KC / 8);
     const char* x_mine = x_lds + (r16 & (a.x_rows - 1)) * a.x_pitch + wave * (GD_KC * 2) + 16 * g;
@@ -508,15 +518,15 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
 // share of a large weight; with one workgroup per block of 16 rows it would enter four times as many workgroups.
 // Where the sums go to a norm (plain 32-bit output), K may be shared out as well: k_parts sets of workgroups, each
 // with all of N and a part of K, leave one array of partial sums each, and a compute unit pulls 1/k_parts of X.
-// With 16 waves and one block of rows the same kernel takes 9 to 16 rows whose K is too long for LDS (up to 6,144: three
-// chunks of 16 rows are 48 of a wave's 128 registers).
+// With one block of rows the same kernel takes 9 to 16 rows whose K is too long for LDS (up to 6,144: six chunks of 16 rows are 96 of a
+// wave's registers; 12288 x 4096 with the norm at 16 rows 26.7 -> 22.7 microseconds against 16 waves with half as many each).
 #define GR_NW 8
 
-template <typename TOut, int EPI, int XC, int RB, int NT, bool NORM, int NW = GR_NW, int LPI = 4>
-__global__ __launch_bounds__(NW* LLMS_WAVE) void gemm_decode_rows_kernel(const DecodeGemmArgs a) {
+template <typename TOut, int EPI, int XC, int RB, int NT, bool NORM, int LPI = 4>
+__global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(const DecodeGemmArgs a) {
+    constexpr int NW = GR_NW;
     static_assert(!NORM || RB == 1, "the norm on the way in is for up to 16 rows");
-    static_assert(NW == GR_NW || (NW == 16 && RB == 1), "16 waves have registers for one block of rows");
-    constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
+        constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
     static_assert(!PAIRS || LPI == 4, "units with partners fill rows 0..7 and 8..15");
     constexpr int UPT = PAIRS ? 8 : 4 * LPI;  // units per tile (rows of the tile beyond them hold whatever lies in LDS)
     constexpr int ITEMS = NT * XC;
@@ -749,28 +759,21 @@ static void gd_launch_rows_long_k(int tiles, unsigned grid, DecodeGemmArgs& a, h
 }
 #undef GR_GO
 
-// 9 to 16 rows whose K does not fit LDS: 16 waves, two or three chunks each.  LPI = 2: tiles of 8 weight rows, for a
-// share whose last tile of 16 would be half empty (two load instructions less per chunk, and with three chunks a group
-// of one tile whose ring of three fits the registers).
+// 9 to 16 rows whose K does not fit LDS: four or six chunks a wave.  LPI = 2: tiles of 8 weight rows, for a share whose last tile of 16
+// would be half empty (two load instructions less per chunk).
 template <typename TOut, int EPI, bool NORM, int LPI>
-static void gd_launch_rows_16_waves(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
-#define GR_GO16(XC, NT)                                                                                          \
-    do {                                                                                                         \
-        a.groups = (tiles + NT - 1) / NT;                                                                        \
-        gemm_decode_rows_kernel<TOut, EPI, XC, 1, NT, NORM, 16, LPI><<<grid, 16 * LLMS_WAVE, 0, stream>>>(a);    \
+static void gd_launch_rows_one_block(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
+#define GR_GO16(XC, NT)                                                                                             \
+    do {                                                                                                            \
+        a.groups = (tiles + NT - 1) / NT;                                                                           \
+        gemm_decode_rows_kernel<TOut, EPI, XC, 1, NT, NORM, LPI><<<grid, GR_NW * LLMS_WAVE, 0, stream>>>(a);        \
     } while (0)
-    if (chunks <= 32) {
-        if (tiles == 1) GR_GO16(2, 1);
-        else GR_GO16(2, 2);
+    if (chunks <= 4 * GR_NW) {
+        if (tiles == 1) GR_GO16(4, 1);
+        else GR_GO16(4, 2);
     } else {
-        if constexpr (LPI == 2) {
-            if (tiles == 1) {
-                GR_GO16(3, 1);
-                return;
-            }
-        }
-        GR_GO16(3, 2);  // (a ring of three whole chunks beside three chunks of X would not fit the registers: two tiles
-                        // a group, of which the second may not exist, and a ring of two)
+        if (tiles == 1) GR_GO16(6, 1);
+        else GR_GO16(6, 2);
     }
 #undef GR_GO16
 }
@@ -780,11 +783,11 @@ static int gd_launch_rows(int chunks, int rows, int tiles, bool low, unsigned gr
     if (rows <= 16) {
         if (low) {
             if constexpr (EPI == GD_PLAIN || EPI == GD_RESIDUAL) {
-                if (a.norm_weight) gd_launch_rows_16_waves<TOut, EPI, true, 2>(chunks, tiles, grid, a, stream);
-                else gd_launch_rows_16_waves<TOut, EPI, false, 2>(chunks, tiles, grid, a, stream);
+                if (a.norm_weight) gd_launch_rows_one_block<TOut, EPI, true, 2>(chunks, tiles, grid, a, stream);
+                else gd_launch_rows_one_block<TOut, EPI, false, 2>(chunks, tiles, grid, a, stream);
             }
-        } else if (a.norm_weight) gd_launch_rows_16_waves<TOut, EPI, true, 4>(chunks, tiles, grid, a, stream);
-        else gd_launch_rows_16_waves<TOut, EPI, false, 4>(chunks, tiles, grid, a, stream);
+        } else if (a.norm_weight) gd_launch_rows_one_block<TOut, EPI, true, 4>(chunks, tiles, grid, a, stream);
+        else gd_launch_rows_one_block<TOut, EPI, false, 4>(chunks, tiles, grid, a, stream);
         return LLMS_OK;
     }
     if (chunks > 2 * GR_NW) {  // (17 to 32 rows: checked by the caller)
@@ -816,18 +819,23 @@ static int gd_launch(int chunks, int tiles, unsigned grid, unsigned lds_bytes, D
         a.groups = (tiles + NT - 1) / NT;                                                                        \
         gemm_decode_kernel<TOut, EPI, XC, LPI, NT><<<grid, GD_NW * LLMS_WAVE, lds_bytes, stream>>>(a);           \
     } while (0)
+    // tiles of a group: as few groups as possible, and then as few tiles that do not exist
+    const int groups = (tiles + 3) / 4, nt = (tiles + groups - 1) / groups;
     if (chunks <= GD_NW) {
-        // tiles of a group: as few groups as possible, and then as few tiles that do not exist
-        const int groups = (tiles + 3) / 4, nt = (tiles + groups - 1) / groups;
         if (nt == 1) GD_GO(1, 1);
         else if (nt == 2) GD_GO(1, 2);
         else if (nt == 3) GD_GO(1, 3);
         else GD_GO(1, 4);
     } else if (chunks <= 2 * GD_NW) {
-        if (tiles % 2) GD_GO(2, 1);
-        else GD_GO(2, 2);
+        if (nt == 1) GD_GO(2, 1);
+        else if (nt == 2) GD_GO(2, 2);
+        else if (nt == 3) GD_GO(2, 3);
+        else GD_GO(2, 4);
+    } else if (chunks <= 4 * GD_NW) {
+        if (tiles % 2) GD_GO(4, 1);
+        else GD_GO(4, 2);
     } else {
-        GD_GO(3, 1);
+        GD_GO(6, 1);
     }
 #undef GD_GO
     return LLMS_OK;
@@ -840,8 +848,8 @@ static bool gd_rows_fit_lds(int M, int K) {
     return (M <= 8 ? 8 : 16) * ((K + GD_KC - 1) / GD_KC * (GD_KC * 2) + 16) <= GD_LDS_X_MAX;
 }
 
-// Whether M rows of K elements fit: up to 16 rows in LDS, or where K is too long for that in the registers of 16
-// waves, three chunks of 128 each; 17 to 64 rows in the registers of 8 waves, two chunks each (four up to 32 rows).
+// Whether M rows of K elements fit: up to 16 rows in LDS, or where K is too long for that in the registers of the 8
+// waves, six chunks of 128 each; 17 to 64 rows in registers too, two chunks each (four up to 32 rows).
 int llms_gemm_decode_fits(int M, int K) {
     if (M <= 0 || M > 64 || K <= 0 || K > GD_MAX_K) return 0;
     if (M > 32) return K <= 2 * GR_NW * GD_KC;

@@ -480,12 +480,12 @@ def compute_units(dev: torch.device) -> int:
 GEMM_DECODE_MAX_ROWS = 64
 GEMM_DECODE_NORM_ROWS = 16  # up to here the kernel norms its rows on the way in (with more rows that costs a compute
 # unit more vector arithmetic than a norm kernel of its own: measured at 32 rows, 4 microseconds)
-GEMM_DECODE_MAX_K = 16 * 3 * 128  # 16 waves with up to three chunks of 128 each
+GEMM_DECODE_MAX_K = 8 * 6 * 128  # 8 waves with up to six chunks of 128 each
 
 
 def gemm_decode_fits(m: int, k: int) -> bool:
     """Whether m rows of k elements fit ops.gemm_decode: up to 16 rows stay in LDS or, where K is too long for that, in
-    the registers of 16 waves (k up to 6,144 either way); 17 to 64 rows in the registers of 8 waves: four chunks of
+    the registers of 8 waves (k up to 6,144 either way); 17 to 64 rows in the registers too: four chunks of
     128 each up to 32 rows (k up to 4,096), two beyond (k up to 2,048)."""
     if not (0 < m <= GEMM_DECODE_MAX_ROWS and 0 < k <= GEMM_DECODE_MAX_K):
         return False

@@ -42,12 +42,6 @@ STREAM_MAX_ROWS = 64
 STREAM_REREAD_BYTES = 64e6
 
 
-# A plain product of up to 8 rows against a weight this large (the vocabulary's) stays with the streaming kernel:
-# its two thousand small workgroups even out better than 256 large ones with a barrier per group of tiles
-# (measured on 32000 x 2048: 25.8 and 27.0 microseconds at 1 and 8 rows against 27.9 and 28.3).
-STREAM_LARGE_ROWS = 8
-STREAM_LARGE_BYTES = 100e6
-
 DECODE_KERNEL = os.environ.get("LLMSERVE_DECODE_GEMM", "1") != "0"
 
 
@@ -215,7 +209,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     if m == 0:
         return out
     if x.dtype == torch.bfloat16 and ops.gemm_bf16_supported(x, weight):
-        if decode_product(x, weight) and not (m <= STREAM_LARGE_ROWS and weight.numel() * 2 >= STREAM_LARGE_BYTES):
+        if decode_product(x, weight):
             return ops.gemm_decode(out, x, weight, bias)
         if few_rows(m, weight):
             return ops.gemm_stream(out, x, weight, bias)

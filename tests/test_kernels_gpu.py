@@ -484,6 +484,23 @@ def test_gemm_decode_plain(m, n, k):
     assert torch.equal(ops().gemm_decode(torch.empty(m, n, dtype=torch.bfloat16, device=DEV), wide[:, :k], w.to(DEV)), out)
 
 
+@pytest.mark.parametrize("k", [1024, 1032, 2040, 2056, 3072, 3968, 3976, 4096, 4104, 5120, 5128, 6144])
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+def test_gemm_decode_chunks_of_k(m, k):
+    """One, two, four and six chunks a wave, the last ones empty, half empty or full; rows in LDS and in registers; one tile, several and
+    several groups of them."""
+    for n in (40, 4104, 20000):
+        x, w, b = rnd(m, k, seed=11).bfloat16(), rnd(n, k, seed=12).bfloat16(), rnd(n, seed=13).bfloat16()
+        got = ops().gemm_decode(torch.empty(m, n, device=DEV), x.to(DEV), w.to(DEV), b.to(DEV))
+        ref = x.to(DEV).double() @ w.to(DEV).double().t() + b.to(DEV).double()
+        assert (got.double() - ref).abs().max() <= 2e-6 * math.sqrt(k) * float(ref.abs().max())
+        # the norm on the way in: its own kernel in front, but for a rounding where a row's sum of squares has another order
+        nw = (1 + 0.1 * rnd(k, seed=4)).bfloat16().to(DEV)
+        want = ops().gemm_decode(torch.empty(m, n, device=DEV), ops().rmsnorm(torch.empty_like(x).to(DEV), x.to(DEV), nw, 1e-5), w.to(DEV))
+        got = ops().gemm_decode(torch.empty(m, n, device=DEV), x.to(DEV), w.to(DEV), norm=(nw, 1e-5))
+        assert (got - want).abs().max() <= 2.0 ** -7 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("m,n,k,parts", [(64, 2048, 5632, 3), (17, 333, 2048 + 8, 2), (33, 4096, 11008, 6), (40, 100, 520, 5),
                                          (24, 2048, 5632, 3), (64, 48, 256, 2)])
 def test_gemm_decode_shares_k_out_for_many_rows(m, n, k, parts):
