@@ -404,8 +404,14 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
     // first and last tile whose 32 keys every column of the group sees
     const int lo_max = (a.window > 0 && p_max - a.window + 1 > 0) ? p_max - a.window + 1 : 0;
 
-    // this workgroup's share of the tiles, dealt to its waves
-    const int per_split = (n_tiles + a.num_splits - 1) / a.num_splits;
+    // this workgroup's share of the tiles, dealt to its waves.  What one workgroup brings in at once is not shared out (num_splits goes by
+    // the longest context that a step may have: a shared request of 600 keys costs 1 microsecond more): the other workgroups leave, or
+    // where a kernel adds the shares up leave one without keys, which changes no bit of the sum.
+    constexpr int AHEAD = DB <= 4 ? 3 : DB <= 8 ? 2 : 1;  // tiles a wave asks for at once (what the registers hold beside the sums)
+    const bool alone = a.num_splits == 1 || (DB <= 8 && n_tiles <= AHEAD * NW);
+    if (alone && split > 0 && a.arrive) return;
+    const bool direct = a.num_splits == 1 || (alone && a.arrive);
+    const int per_split = alone ? n_tiles : (n_tiles + a.num_splits - 1) / a.num_splits;
     const int t_begin = split * per_split + wave;
     const int t_end = min(n_tiles, (split + 1) * per_split);
     constexpr int t_step = NW;
@@ -466,21 +472,28 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
 
     // Few tiles per wave (a decoded token behind a context of some hundred keys: up to AHEAD each, whose pages one
     // register per lane holds): every tile's operands are asked for at once, so the wave's way through memory is
-    // one trip and not one per tile.  Every wave issues the same loads (a tile it does not have is the workgroup's
-    // last once more, which some other wave brings in anyway), so the compiler knows how many are in flight when
-    // it waits for the first.
-    constexpr int AHEAD = DB <= 4 ? 3 : DB <= 8 ? 2 : 1;  // (what the registers hold beside the sums)
-    const int t_first_here = split * per_split;
-    const bool at_once = t_end > t_first_here && t_end - t_first_here <= AHEAD * NW &&
+    // one trip and not one per tile.  With as many tiles for each wave as the first has (a number that the code knows: no branch
+    // around a load), so that a compute unit takes in no more than it needs: with three for every wave, those that do not exist as
+    // the last once more, a launch behind 27 keys brought 192 KB into a compute unit for the 8 it uses.
+    const int t_first_here = split * per_split, tiles_here = t_end - t_first_here;
+    const bool at_once = tiles_here > 0 && tiles_here <= AHEAD * NW &&
                          block_of(min(j_begin + 32 * t_end - 1, p_max)) - block_of(j_begin + 32 * t_first_here) < LLMS_WAVE;
+    auto all_at_once = [&](auto tiles) {
+        constexpr int n = decltype(tiles)::n;
+        uint4 kfa[n][2][KS], vfa[n][DB];
+#pragma unroll
+        for (int i = 0; i < n; ++i) fetch_tile(j_begin + 32 * min(t_begin + i * NW, t_end - 1), kfa[i], vfa[i]);
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+            if (t_begin + i * NW < t_end) attend(j_begin + 32 * (t_begin + i * NW), kfa[i], vfa[i]);
+    };
     if (at_once) {
         load_pages(block_of(j_begin + 32 * t_first_here));
-        uint4 kfa[AHEAD][2][KS], vfa[AHEAD][DB];
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) fetch_tile(j_begin + 32 * min(t_begin + i * NW, t_end - 1), kfa[i], vfa[i]);
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i)
-            if (t_begin + i * NW < t_end) attend(j_begin + 32 * (t_begin + i * NW), kfa[i], vfa[i]);
+        if (t_begin < t_end) {  // (the same for all lanes of a wave; a wave without a tile asks for nothing)
+            if (AHEAD == 1 || tiles_here <= NW) all_at_once(Number<1>());
+            else if (AHEAD == 2 || tiles_here <= 2 * NW) all_at_once(Number<(AHEAD < 2 ? 1 : 2)>());
+            else all_at_once(Number<AHEAD>());
+        }
     } else {
         // the next tile's operands are requested before this tile's arithmetic starts
         uint4 kf_next[2][KS], vf_next[DB];
@@ -540,7 +553,7 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
             o.w += p.w * weight[w];
         }
         if (!col_ok) continue;
-        if (a.num_splits == 1) {
+        if (direct) {
             const float inv = column_factor(l_tot, gate_z);
             uint2 pk;
             pk.x = pack_bf16(o.x * inv, o.y * inv);
@@ -553,7 +566,8 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
             *reinterpret_cast<float4*>(a.ws_o + item * D + 16 * m + 4 * g) = o;
         }
     }
-    if (a.num_splits > 1 && wave == 0 && g == 0 && col_ok) {
+    if (direct) return;
+    if (wave == 0 && g == 0 && col_ok) {
         if (a.arrive) {
             store_across(a.ws_ml + item * 2, m_tot, l_tot);
         } else {
@@ -561,7 +575,7 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
             a.ws_ml[item * 2 + 1] = l_tot;
         }
     }
-    if (a.num_splits > 1 && a.arrive) {  // (the same in every thread of the launch)
+    if (a.arrive) {  // (the same in every thread of the launch)
         // A thread's stores have been taken by memory before its workgroup is counted; the one that finds all
         // others counted reads their shares.  Nobody waits for anybody: a workgroup that is not the last leaves.
         __shared__ unsigned is_last;

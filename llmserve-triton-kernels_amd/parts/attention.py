@@ -199,13 +199,16 @@ def prompt_splits(num_heads: int, num_kv_heads: int, window: int | None, n_reque
 
 def decode_arrangement(num_heads: int, num_kv_heads: int, head_dim: int, window: int | None, n_requests: int, max_context: int,
                        cus: int = 256) -> tuple[int, int]:
-    """(workgroups per request and KV head, waves per workgroup) for decoding.  The waves of a
-    workgroup take 32 keys at a time each and merge in LDS; workgroups that share a request hand
-    their shares to the one that finishes last, through memory, which costs more (2 to 3
-    microseconds) than a few extra tiles per wave.  So a small batch first gets 8 waves, and is
-    split over workgroups only when a wave would still walk more than 4 tiles (measured: at a
-    context of 512 no split pays at any batch size, at 4,096 four to eight do up to batch 8); once
-    the batch alone fills the chip (a workgroup for each of its `cus` compute units) nothing is split."""
+    """(workgroups per request and KV head, waves per workgroup) for decoding.  The waves of a workgroup take 32 keys at a time each
+    and merge in LDS; workgroups that share a request hand their shares to the one that finishes last, through memory, which costs 1
+    to 1.5 microseconds and little more for four of them than for two.  A compute unit takes in some 60 GB/s of keys and values, so what
+    does not come in one trip (three tiles a wave up to a head size of 64, two up to 128) is shared out, to at least four, of at most
+    two tiles a wave (microseconds with one workgroup, two, four and eight, 4 KV heads of 64 numbers: 1 request of 600 keys 6.1, 6.9, 6.3,
+    7.1, of 1,000 8.5, 7.3, 7.1, 7.7, of 4,000 21.9, 14.9, 10.9, 9.6; 8 requests of 768 7.2, 8.1, 7.9, 9.2, of 1,000 8.7, 8.3, 8.2,
+    9.5, of 2,048 16.2, 12.5, 10.6, 11.4; 8 KV heads of 128, 4 requests of 600 keys 10.4, 10.7, 9.1, 10.6, of 1,000 17.1, 12.6, 11.3,
+    12.1).  Once the batch alone fills the chip (a workgroup for each of its `cus` compute units) nothing is split.  More than
+    16 shares would need a kernel to add them up: they wait until a wave would walk more than 4 tiles.  Wider heads are split
+    where a wave would walk more than 4 tiles."""
     g = num_heads // num_kv_heads
     groups = n_requests * num_kv_heads * -(-g // 16)
     reach = min(max_context, window) if window else max_context
@@ -213,5 +216,10 @@ def decode_arrangement(num_heads: int, num_kv_heads: int, head_dim: int, window:
     if groups >= cus:
         return 1, waves
     tiles = -(-reach // 32)
-    splits = max(1, min(cus // groups, -(-tiles // (4 * waves))))
+    splits = -(-tiles // (4 * waves))
+    if head_dim <= 128:
+        if tiles <= (3 if head_dim <= 64 else 2) * waves:
+            return 1, waves
+        splits = max(min(16, max(4, -(-tiles // (2 * waves)))), splits)
+    splits = max(1, min(cus // groups, splits))
     return splits, waves

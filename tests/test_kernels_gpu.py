@@ -915,6 +915,27 @@ def test_attention_mfma(case, arrangement):
     assert (got - ref).abs().max() <= 2.0 ** -7 * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("window", [0, 700])
+@pytest.mark.parametrize("nh,nkv,d,waves,lens", [
+    (8, 1, 64, 8, [1, 32, 33, 256, 257, 512, 513, 768, 769, 1500]),   # three tiles a wave at once: up to 768 keys
+    (8, 2, 64, 4, [128, 129, 384, 385, 1000]),
+    (4, 2, 128, 8, [255, 256, 257, 512, 513, 1100]),                  # two tiles a wave: up to 512
+    (3, 1, 144, 8, [200, 256, 257, 900]), (2, 1, 16, 8, [767, 770])])
+def test_decode_keys_at_once_or_shared_out(nh, nkv, d, waves, lens, window):
+    """One, two and three tiles a wave in one trip, one key more than that, and many: requests of all lengths in one launch, each
+    shared out to workgroups or not by its own length.  The last workgroup and the second kernel give the same bits, and one
+    workgroup to a request what they give for requests that are not shared out."""
+    new, got = [1] * len(lens), {}
+    for splits, kernel in ((1, False), (4, False), (4, True), (7, False), (7, True)):
+        got[splits, kernel], ref = run_attention_mfma(nh, nkv, d, 16, lens, new, window, seed=70, split_waves=True, num_splits=splits,
+                                                      waves=waves, merge_kernel=kernel)
+        assert (got[splits, kernel] - ref).abs().max() <= 2.0 ** -7 * float(ref.abs().max())
+    assert torch.equal(got[4, False], got[4, True]) and torch.equal(got[7, False], got[7, True])
+    if d <= 128:
+        short = [i for i, n in enumerate(lens) if n <= 32 * waves * (3 if d <= 64 else 2)]
+        assert torch.equal(got[1, False][short], got[4, False][short])
+
+
 @pytest.mark.parametrize("case", [(8, 2, 64, 16, [300, 64, 129, 1, 17, 600, 33, 90], 4, 8), (32, 4, 64, 16, [520], 8, 8),
                                   (64, 8, 128, 16, [700, 33], 2, 8), (3, 1, 32, 8, [1, 7, 40, 100], 3, 4),
                                   (6, 2, 80, 8, [70, 19, 300], 16, 4), (4, 4, 256, 16, [257, 31], 5, 4),
