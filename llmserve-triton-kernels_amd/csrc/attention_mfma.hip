@@ -335,8 +335,14 @@ __device__ __forceinline__ void merge_shares(const AttnArgs& a, size_t item0, bo
     }
 }
 
-template <int DB, int NW>  // blocks of 16 dimensions of a head; waves of the workgroup (4 or 8), which share the keys
-__global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs a) {
+// A workgroup's place in its launch, and the launch's size.
+struct Place {
+    int x, y, z, gx, gy;
+};
+
+// DB: blocks of 16 dimensions of a head; NW: waves of the workgroup (4 or 8), which share the keys; AHEAD: tiles a wave asks for at once.
+template <int DB, int NW, int AHEAD>
+__device__ __forceinline__ void attn_decode(const AttnArgs& a, const Place at) {
     constexpr int D = DB * 16;
     constexpr int KS = (D + 31) / 32;  // k-steps of the score product
     const int wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE;
@@ -346,10 +352,10 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
     const int HG = G < 16 ? G : 16;       // heads of one column group
     const int TPG = 16 / HG;              // tokens of one column group
     const int HB = (G + HG - 1) / HG;     // column groups needed to cover a KV head's query heads
-    const int kvh = blockIdx.y / HB, hb = blockIdx.y % HB;
-    const int b = a.seq_begin + blockIdx.z;
+    const int kvh = at.y / HB, hb = at.y % HB;
+    const int b = a.seq_begin + at.z;
     const bool one_each = a.one_token_from >= 0;
-    const int tok0 = one_each ? a.one_token_from + (int)blockIdx.z : a.cu_seqlens[b];
+    const int tok0 = one_each ? a.one_token_from + at.z : a.cu_seqlens[b];
     const int n_new = one_each ? 1 : a.cu_seqlens[b + 1] - tok0;
     const int ctx = a.context_lens[b];
     // (asked for together with the lengths: one trip to memory earlier than where the block table is first needed)
@@ -360,7 +366,7 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
     const int* table = a.block_tables + (size_t)table_row * a.max_blocks;
     int blk_base = 0, pages_reg = table[min(lane, a.max_blocks - 1)];
 
-    const int tile = blockIdx.x / a.num_splits, split = blockIdx.x % a.num_splits;
+    const int tile = at.x / a.num_splits, split = at.x % a.num_splits;
     const int t_first = tile * TPG;  // first token (within the request's new tokens) of this group
 
     // this lane's column
@@ -407,7 +413,6 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
     // this workgroup's share of the tiles, dealt to its waves.  What one workgroup brings in at once is not shared out (num_splits goes by
     // the longest context that a step may have: a shared request of 600 keys costs 1 microsecond more): the other workgroups leave, or
     // where a kernel adds the shares up leave one without keys, which changes no bit of the sum.
-    constexpr int AHEAD = DB <= 4 ? 3 : DB <= 8 ? 2 : 1;  // tiles a wave asks for at once (what the registers hold beside the sums)
     const bool alone = a.num_splits == 1 || (DB <= 8 && n_tiles <= AHEAD * NW);
     if (alone && split > 0 && a.arrive) return;
     const bool direct = a.num_splits == 1 || (alone && a.arrive);
@@ -582,7 +587,7 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         if (threadIdx.x == 0) {
-            unsigned* counter = a.arrive + ((size_t)blockIdx.z * gridDim.y + blockIdx.y) * (gridDim.x / a.num_splits) + tile;
+            unsigned* counter = a.arrive + ((size_t)at.z * at.gy + at.y) * (at.gx / a.num_splits) + tile;
             const unsigned before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             is_last = before + 1 == (unsigned)a.num_splits;
             if (is_last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // zero again for the next launch
@@ -596,6 +601,12 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
         else if (a.num_splits <= 8) merge_shares<DB, 8>(a, item0, col_ok, wave, nw, g, orow, gate_z);
         else merge_shares<DB, 16>(a, item0, col_ok, wave, nw, g, orow, gate_z);
     }
+}
+
+template <int DB, int NW>
+__global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs a) {
+    // (as many tiles at once as the registers hold beside the sums)
+    attn_decode<DB, NW, (DB <= 4 ? 3 : DB <= 8 ? 2 : 1)>(a, Place{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.x, (int)gridDim.y});
 }
 
 // Prompt portions: a block of WB * CG consecutive column groups of one request and KV head per workgroup, CG per
@@ -615,7 +626,7 @@ __global__ __launch_bounds__(NW* LLMS_WAVE) void attn_mfma_kernel(const AttnArgs
 // blocks are handed out in an order (see `rank` below) in which a CU that was given a long one gets a short one
 // beside or after it.
 template <int DB, bool TWIN, int CG, int WB, bool BIAS = false>
-__global__ __launch_bounds__((TWIN ? 2 : 1) * WB * LLMS_WAVE, (TWIN && DB <= 4) ? 4 : 1) void attn_prompt_kernel(const AttnArgs a) {
+__device__ __forceinline__ void attn_prompt(const AttnArgs& a, const Place at) {
     constexpr int D = DB * 16;
     constexpr int KS = (D + 31) / 32;
     constexpr int KCH = D / 8;          // 16-byte chunks of a key row
@@ -632,9 +643,9 @@ __global__ __launch_bounds__((TWIN ? 2 : 1) * WB * LLMS_WAVE, (TWIN && DB <= 4) 
 
     const int G = a.n_heads / a.n_kv_heads;
     const int HG = G < 16 ? G : 16, TPG = 16 / HG, HB = (G + HG - 1) / HG;
-    const int head_block = TWIN ? blockIdx.x : blockIdx.y;
+    const int head_block = TWIN ? at.x : at.y;
     const int kvh = head_block / HB, hb = head_block % HB;
-    const int b = a.seq_begin + blockIdx.z;
+    const int b = a.seq_begin + at.z;
     const int tok0 = a.cu_seqlens[b], n_new = a.cu_seqlens[b + 1] - tok0;
     const int ctx = a.context_lens[b];
     // (asked for together with the lengths: one trip to memory earlier than where the block table is first needed)
@@ -643,19 +654,19 @@ __global__ __launch_bounds__((TWIN ? 2 : 1) * WB * LLMS_WAVE, (TWIN && DB <= 4) 
     int wg_first;                   // first token (within the request's new tokens) of the workgroup's block
     if (TWIN) {
         // rank 0: the last block of the prompt, which sees the most keys.  Workgroups are handed out in the order
-        // of blockIdx.y: the first on every CU get the longest blocks, and the CU that was given the shortest of
+        // of at.y: the first on every CU get the longest blocks, and the CU that was given the shortest of
         // these gets the longest of the rest
-        const int blocks = (n_new + BLK - 1) / BLK, by = blockIdx.y;
+        const int blocks = (n_new + BLK - 1) / BLK, by = at.y;
         const int rank = by < a.first_blocks ? a.first_blocks - 1 - by : by;
         if (rank >= blocks || ctx <= 0) return;
         wg_first = (blocks - 1 - rank) * BLK;
     } else {
-        wg_first = ((int)blockIdx.x / a.num_splits) * BLK;
+        wg_first = (at.x / a.num_splits) * BLK;
         if (wg_first >= n_new || ctx <= 0) return;
     }
-    // Without twins the keys of a block may be shared out to num_splits workgroups (blockIdx.x % num_splits), whose
+    // Without twins the keys of a block may be shared out to num_splits workgroups (at.x % num_splits), whose
     // partial results attn_merge adds up: a short portion with a long prefix has few blocks and many keys.
-    const int n_splits = TWIN ? 1 : a.num_splits, split = TWIN ? 0 : (int)blockIdx.x % a.num_splits;
+    const int n_splits = TWIN ? 1 : a.num_splits, split = TWIN ? 0 : at.x % a.num_splits;
 
     // this wave's CG column groups: consecutive tokens, the same heads
     const int w_first = wg_first + (wave % WB) * CG * TPG;
@@ -924,6 +935,31 @@ __global__ __launch_bounds__((TWIN ? 2 : 1) * WB * LLMS_WAVE, (TWIN && DB <= 4) 
     }
 }
 
+template <int DB, bool TWIN, int CG, int WB, bool BIAS = false>
+__global__ __launch_bounds__((TWIN ? 2 : 1) * WB * LLMS_WAVE, (TWIN && DB <= 4) ? 4 : 1) void attn_prompt_kernel(const AttnArgs a) {
+    attn_prompt<DB, TWIN, CG, WB, BIAS>(a, Place{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z, (int)gridDim.x, (int)gridDim.y});
+}
+
+#if !defined(LLMS_ATTENTION_BIASED) && !defined(LLMS_ATTENTION_HEAD_GATED)
+// A step that has both: the first `n_decode` workgroups are those of the single tokens, the others those of the portions with twins.  Neither
+// needs what the other leaves, but as two launches the single tokens' waited for memory with most of the chip idle while the portions' had
+// not begun: 32 heads of 64 with 4 KV heads, 32 tokens with 512 keys and a portion of 512, 15.7 us as two and 13.0 as one; 48 tokens with
+// 1024 keys, 27.1 and 21.7; 8 tokens with 2000 keys and a portion of 2048, 46.3 and 36.5; 32 heads of 128 with 8, 16 tokens with 1024, 38.8
+// and 36.9.  The single tokens come first because each is one chain of trips to memory (last: the same to 1 % slower, steps with long
+// contexts).  They ask for two tiles a wave at once, not three: the kernel's registers are then those of the portions.
+template <int DB, int CG>
+__global__ __launch_bounds__(8 * LLMS_WAVE, DB <= 4 ? 4 : 1) void attn_both_kernel(const AttnArgs decode, const AttnArgs prompt, int n_decode,
+                                                                                  int dx, int dy, int px, int py) {
+    const int w = blockIdx.x;
+    if (w < n_decode) {
+        attn_decode<DB, 8, 2>(decode, Place{w % dx, w / dx % dy, w / (dx * dy), dx, dy});
+    } else {
+        const int v = w - n_decode;
+        attn_prompt<DB, true, CG, 4>(prompt, Place{v % px, v / px % py, v / (px * py), px, py});
+    }
+}
+#endif
+
 // Merge of the splits of every (token, head), split 0 first: a thread per token, head and 4 dimensions (blockIdx.x:
 // token, blockIdx.y: which blockDim.x of the token's heads * head_dim / 4 pieces).
 __global__ __launch_bounds__(256) void attn_merge_kernel(bf16* __restrict__ out, int out_stride, const float* __restrict__ ws_o,
@@ -1077,7 +1113,13 @@ extern "C" {
 // ws_ml [tokens * heads * splits * 2] floats, indexed by absolute token row.  `arrive` (may be null): n_arrive
 // counters in device memory, all zero, which the kernel leaves zero: decoding with 2 to 16 splits then adds the
 // shares up in the workgroup that finishes last instead of in a second kernel.
-static int attention_mfma_launch(void* out, int out_stride, const void* q, int q_stride, const void* k_pool,
+struct AttnLaunch {  // what a launch of one of the kernels above would be
+    AttnArgs a;
+    dim3 grid;
+    int cg;     // prompts
+    bool twin;  // prompts
+};
+static int attention_mfma_launch(AttnLaunch* only, void* out, int out_stride, const void* q, int q_stride, const void* k_pool,
                         const void* v_pool, const int* block_tables, const int* table_rows, int max_blocks,
                         const int* cu_seqlens,
                         const int* context_lens, int seq_begin, int n_seqs, int max_new, int token_begin,
@@ -1118,6 +1160,10 @@ static int attention_mfma_launch(void* out, int out_stride, const void* q, int q
     if (split_waves > 0) {
         dim3 grid(groups * num_splits, n_kv_heads * HB, n_seqs);
         if (arrive && num_splits > 1 && num_splits <= 16 && (long long)groups * grid.y * grid.z <= n_arrive) a.arrive = arrive;
+        if (only) {
+            *only = AttnLaunch{a, grid, 0, false};
+            return LLMS_OK;
+        }
         if (int e = launch_attn(head_dim / 16, grid, waves * LLMS_WAVE, a, stream)) return e;
         if (num_splits > 1 && a.arrive == nullptr) {
             hipError_t e1 = hipGetLastError();
@@ -1152,6 +1198,10 @@ static int attention_mfma_launch(void* out, int out_stride, const void* q, int q
             // short one that add up to the same.
             a.first_blocks = n_seqs == 1 ? (int)std::min<long long>(grid.y, cus / grid.x) : 0;
         }
+        if (only) {
+            *only = AttnLaunch{a, grid, cg, twin};
+            return LLMS_OK;
+        }
         if (int e = launch_prompt(head_dim / 16, cg, grid, twin, a, stream)) return e;
         if (num_splits > 1) {
             hipError_t e1 = hipGetLastError();
@@ -1174,10 +1224,50 @@ int llms_attention_mfma(void* out, int out_stride, const void* q, int q_stride, 
                         int n_tokens, int n_heads, int n_kv_heads, int head_dim, int block_size, int window,
                         float scale, int split_waves, int num_splits, int waves, float* ws_o, float* ws_ml,
                         unsigned* arrive, int n_arrive, hipStream_t stream) {
-    return attention_mfma_launch(out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
+    return attention_mfma_launch(nullptr, out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
                                  context_lens, seq_begin, n_seqs, max_new, token_begin, n_tokens, n_heads, n_kv_heads, head_dim,
                                  block_size, window, scale, split_waves, num_splits, waves, ws_o, ws_ml, arrive, n_arrive,
                                  nullptr, 0, nullptr, 0, stream);
+}
+
+// A step's attention in one call: n_decode requests of one token each (rows 0 ..), then n_seqs portions of up to max_new tokens, n_tokens in all.
+// One launch where the portions have twins, no window and heads of up to 128 numbers, and 8 waves share a single token's keys; otherwise one each.
+int llms_attention_mfma_step(void* out, int out_stride, const void* q, int q_stride, const void* k_pool, const void* v_pool,
+                             const int* block_tables, const int* table_rows, int max_blocks, const int* cu_seqlens,
+                             const int* context_lens, int n_heads, int n_kv_heads, int head_dim, int block_size, int window, float scale,
+                             int n_decode, int num_splits, int waves, float* ws_o, float* ws_ml, unsigned* arrive, int n_arrive, int n_seqs,
+                             int max_new, int n_tokens, int prompt_splits, float* prompt_ws_o, float* prompt_ws_ml, hipStream_t stream) {
+    auto decode = [&](AttnLaunch* only) {
+        return attention_mfma_launch(only, out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
+                                     context_lens, 0, n_decode, 1, 0, n_decode, n_heads, n_kv_heads, head_dim, block_size, window, scale, 1,
+                                     num_splits, waves, ws_o, ws_ml, arrive, n_arrive, nullptr, 0, nullptr, 0, stream);
+    };
+    auto prompt = [&](AttnLaunch* only) {
+        return attention_mfma_launch(only, out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
+                                     context_lens, n_decode, n_seqs, max_new, n_decode, n_tokens, n_heads, n_kv_heads, head_dim, block_size,
+                                     window, scale, 0, prompt_splits, 4, prompt_ws_o, prompt_ws_ml, nullptr, 0, nullptr, 0, nullptr, 0, stream);
+    };
+    AttnLaunch d{}, p{};
+    if (int e = decode(&d)) return e;
+    if (int e = prompt(&p)) return e;
+    const long long n_d = (long long)d.grid.x * d.grid.y * d.grid.z, n_p = (long long)p.grid.x * p.grid.y * p.grid.z;
+    if (!(waves == 8 && p.twin && head_dim <= 128 && (num_splits == 1 || d.a.arrive) && n_d + n_p < (1ll << 31))) {
+        if (int e = decode(nullptr)) return e;
+        return prompt(nullptr);
+    }
+    const dim3 grid((unsigned)(n_d + n_p));
+#define ATT_BOTH(N, C) attn_both_kernel<N, C><<<grid, 8 * LLMS_WAVE, 0, stream>>>(d.a, p.a, (int)n_d, d.grid.x, d.grid.y, p.grid.x, p.grid.y)
+#define ATT_CASE(N)                     \
+    case N:                             \
+        if (p.cg == 2) ATT_BOTH(N, 2);  \
+        else ATT_BOTH(N, 1);            \
+        break;
+    switch (head_dim / 16) {
+        ATT_CASE(1) ATT_CASE(2) ATT_CASE(3) ATT_CASE(4) ATT_CASE(5) ATT_CASE(6) ATT_CASE(7) ATT_CASE(8)
+    }
+#undef ATT_CASE
+#undef ATT_BOTH
+    LLMS_LAUNCH_CHECK();
 }
 #elif defined(LLMS_ATTENTION_HEAD_GATED)
 // The plain attention with every head's result multiplied by the sigmoid of one 32-bit number per token and head,
@@ -1189,7 +1279,7 @@ int llms_attention_mfma_gated(void* out, int out_stride, const void* q, int q_st
                               int window, float scale, int split_waves, int num_splits, int waves, float* ws_o, float* ws_ml,
                               unsigned* arrive, int n_arrive, const float* gate, int gate_stride, hipStream_t stream) {
     LLMS_REQUIRE(gate && gate_stride >= n_heads, "attention_mfma_gated: a gate row has a number per head");
-    return attention_mfma_launch(out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
+    return attention_mfma_launch(nullptr, out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
                                  context_lens, seq_begin, n_seqs, max_new, token_begin, n_tokens, n_heads, n_kv_heads, head_dim,
                                  block_size, window, scale, split_waves, num_splits, waves, ws_o, ws_ml, arrive, n_arrive,
                                  nullptr, 0, gate, gate_stride, stream);
@@ -1208,7 +1298,7 @@ int llms_attention_prompt_biased(void* out, int out_stride, const void* q, int q
     LLMS_REQUIRE(head_dim == 32 || head_dim == 64 || head_dim == 96 || head_dim == 128,
                  "attention_prompt_biased: head_dim is 32, 64, 96 or 128");
     LLMS_REQUIRE(!gate || (gate_stride % 4 == 0 && ((uintptr_t)gate % 16) == 0), "attention_prompt_biased: gate rows must be 16-byte aligned");
-    return attention_mfma_launch(out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
+    return attention_mfma_launch(nullptr, out, out_stride, q, q_stride, k_pool, v_pool, block_tables, table_rows, max_blocks, cu_seqlens,
                                  context_lens, seq_begin, n_seqs, max_new, token_begin, n_tokens, n_heads, n_kv_heads, head_dim,
                                  block_size, /*window=*/0, scale, /*split_waves=*/0, /*num_splits=*/1, /*waves=*/4, nullptr,
                                  nullptr, nullptr, 0, dist_bias, dist_reach, gate, gate_stride, stream);

@@ -937,26 +937,8 @@ def attention_mfma_supported(dtype: torch.dtype, head_dim: int, block_size: int)
     return dtype == torch.bfloat16 and head_dim % 16 == 0 and 16 <= head_dim <= 256 and block_size % 8 == 0
 
 
-def attention_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
-                   block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
-                   seq_begin: int, n_seqs: int, max_new: int, token_begin: int, n_tokens: int,
-                   n_heads: int, n_kv_heads: int, head_dim: int, block_size: int, window: int = 0,
-                   scale: float | None = None, split_waves: bool = False, num_splits: int = 1,
-                   table_rows: torch.Tensor | None = None, waves: int = 4, merge_kernel: bool = False,
-                   head_gate: torch.Tensor | None = None) -> torch.Tensor:
-    """bfloat16 causal attention on the matrix cores for requests [seq_begin, seq_begin + n_seqs) of a
-    step, whose new tokens are rows [token_begin, token_begin + n_tokens) of q and out and bring at most
-    `max_new` tokens each.  `split_waves` (with `waves` = 4 or 8 and `num_splits`) spreads each request's keys
-    over the waves of a workgroup and over workgroups: the arrangement for single decoded tokens.  Without
-    it the 4 waves of a block of tokens take neighbouring tokens and share each tile of keys through LDS (in a
-    large launch without a window each has a twin wave that takes every other tile); `num_splits` instead
-    shares the keys of such a block of tokens out to several workgroups (short portions, long prefixes).
-    The shares of workgroups are added up, in the order of the splits, by a second kernel, or for decoding with up
-    to 16 splits by the workgroup of each group that finishes last (`merge_kernel=True` asks for the second kernel
-    there too: the same bits).  (For prompt portions the last workgroup was tried as well: no faster.)
-    `head_gate` float32 [N, >= n_heads] (unit inner stride): every head's result is multiplied by the sigmoid of the
-    token's number for it."""
-    dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, table_rows, head_gate)
+def _check_attention_mfma(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, seq_begin, n_seqs, token_begin, n_tokens,
+                          n_heads, n_kv_heads, head_dim, block_size, window, split_waves, num_splits, table_rows, waves) -> None:
     _check_paged(q, out, k_pool, v_pool, block_tables, n_heads, n_kv_heads, head_dim, block_size)
     if not attention_mfma_supported(q.dtype, head_dim, block_size):
         raise ValueError(f"attention_mfma needs bfloat16, head_dim a multiple of 16 up to 256 and block_size a "
@@ -980,6 +962,30 @@ def attention_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_p
         raise ValueError("4 waves, or 8 when the waves share the keys")
     if waves == 8 and head_dim > 160:
         raise ValueError("8 waves take head_dim up to 160 (wider heads would not fit the registers)")
+
+
+def attention_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor,
+                   block_tables: torch.Tensor, cu_seqlens: torch.Tensor, context_lens: torch.Tensor,
+                   seq_begin: int, n_seqs: int, max_new: int, token_begin: int, n_tokens: int,
+                   n_heads: int, n_kv_heads: int, head_dim: int, block_size: int, window: int = 0,
+                   scale: float | None = None, split_waves: bool = False, num_splits: int = 1,
+                   table_rows: torch.Tensor | None = None, waves: int = 4, merge_kernel: bool = False,
+                   head_gate: torch.Tensor | None = None) -> torch.Tensor:
+    """bfloat16 causal attention on the matrix cores for requests [seq_begin, seq_begin + n_seqs) of a
+    step, whose new tokens are rows [token_begin, token_begin + n_tokens) of q and out and bring at most
+    `max_new` tokens each.  `split_waves` (with `waves` = 4 or 8 and `num_splits`) spreads each request's keys
+    over the waves of a workgroup and over workgroups: the arrangement for single decoded tokens.  Without
+    it the 4 waves of a block of tokens take neighbouring tokens and share each tile of keys through LDS (in a
+    large launch without a window each has a twin wave that takes every other tile); `num_splits` instead
+    shares the keys of such a block of tokens out to several workgroups (short portions, long prefixes).
+    The shares of workgroups are added up, in the order of the splits, by a second kernel, or for decoding with up
+    to 16 splits by the workgroup of each group that finishes last (`merge_kernel=True` asks for the second kernel
+    there too: the same bits).  (For prompt portions the last workgroup was tried as well: no faster.)
+    `head_gate` float32 [N, >= n_heads] (unit inner stride): every head's result is multiplied by the sigmoid of the
+    token's number for it."""
+    dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, table_rows, head_gate)
+    _check_attention_mfma(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, seq_begin, n_seqs, token_begin, n_tokens,
+                          n_heads, n_kv_heads, head_dim, block_size, window, split_waves, num_splits, table_rows, waves)
     if head_gate is not None and (head_gate.dtype != torch.float32 or head_gate.dim() != 2 or head_gate.stride(1) != 1
                                   or head_gate.shape[0] != q.shape[0] or head_gate.shape[1] < n_heads):
         raise ValueError("head_gate must be float32 [N, >= n_heads] with unit inner stride")
@@ -1005,6 +1011,40 @@ def attention_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_p
         c_int(1 if split_waves else 0),
         c_int(num_splits), c_int(waves), _ptr(ws_o), _ptr(ws_ml), _ptr(arrive),
         c_int(arrive.numel() if arrive is not None else 0), *gate_args, _stream(dev)), "attention_mfma")
+    return out
+
+
+def attention_mfma_step(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Tensor,
+                        cu_seqlens: torch.Tensor, context_lens: torch.Tensor, n_decode: int, n_seqs: int, max_new: int, n_tokens: int,
+                        n_heads: int, n_kv_heads: int, head_dim: int, block_size: int, window: int = 0, scale: float | None = None,
+                        num_splits: int = 1, waves: int = 4, prompt_splits: int = 1,
+                        table_rows: torch.Tensor | None = None) -> torch.Tensor:
+    """Both of a step's attentions: `n_decode` requests of one token each (rows 0 to n_decode of q and out; `num_splits`, `waves` as for
+    attention_mfma with split_waves), then `n_seqs` portions of at most `max_new` tokens, `n_tokens` in all (`prompt_splits`).  One
+    launch where the portions are many enough for twins, their heads up to 128 numbers and 8 waves share a token's keys; else two."""
+    dev = _dev(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, table_rows)
+    for first, seqs, row, rows, split, splits, w in ((0, n_decode, 0, n_decode, True, num_splits, waves),
+                                                     (n_decode, n_seqs, n_decode, n_tokens, False, prompt_splits, 4)):
+        _check_attention_mfma(out, q, k_pool, v_pool, block_tables, cu_seqlens, context_lens, first, seqs, row, rows, n_heads, n_kv_heads,
+                              head_dim, block_size, window, split, splits, table_rows, w)
+    if n_decode < 1 or n_seqs < 1 or n_tokens < 1:
+        raise ValueError("a step of single tokens and portions has some of each")
+
+    def workspace(splits):
+        if splits == 1:
+            return None, None
+        return (torch.empty((q.shape[0] * n_heads * splits * head_dim,), dtype=torch.float32, device=dev),
+                torch.empty((q.shape[0] * n_heads * splits * 2,), dtype=torch.float32, device=dev))
+
+    arrive = _arrival_counters(dev) if num_splits > 1 and not MERGE_BY_KERNEL else None
+    (ws_o, ws_ml), (prompt_ws_o, prompt_ws_ml) = workspace(num_splits), workspace(prompt_splits)
+    _check(load("attention_mfma").llms_attention_mfma_step(
+        _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables), _ptr(table_rows),
+        c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), c_int(n_heads), c_int(n_kv_heads), c_int(head_dim),
+        c_int(block_size), c_int(window), c_float(1.0 / math.sqrt(head_dim) if scale is None else scale), c_int(n_decode),
+        c_int(num_splits), c_int(waves), _ptr(ws_o), _ptr(ws_ml), _ptr(arrive), c_int(arrive.numel() if arrive is not None else 0),
+        c_int(n_seqs), c_int(max_new), c_int(n_tokens), c_int(prompt_splits), _ptr(prompt_ws_o), _ptr(prompt_ws_ml), _stream(dev)),
+        "attention_mfma_step")
     return out
 
 

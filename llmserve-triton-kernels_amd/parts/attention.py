@@ -152,16 +152,20 @@ class Attention(Mixer):
                                batch.positions, nh, nkv, d, bs, window, self.scale, table_rows=batch.state_slots)
             return
         common = (out, qkv, cache.k_pool, cache.v_pool, view.block_tables, batch.cu_seqlens, batch.context_lens)
-        n_dec = batch.num_decode
+        n_dec, n_prompt, cus = batch.num_decode, batch.num_seqs - batch.num_decode, ops.compute_units(qkv.device)
         if n_dec:  # requests that bring one token: their keys are spread over waves and workgroups
-            splits, waves = self.decode_arrangement(n_dec, batch.max_decode_context, ops.compute_units(qkv.device))
+            splits, waves = self.decode_arrangement(n_dec, batch.max_decode_context, cus)
+        if n_prompt:  # portions of prompts: one wave per group of tokens and heads
+            prompt_splits = self.prompt_splits(n_prompt, batch.max_count, batch.max_context, cus)
+        if n_dec and n_prompt and batch.num_tokens > n_dec:
+            ops.attention_mfma_step(*common, n_dec, n_prompt, batch.max_count, batch.num_tokens - n_dec, nh, nkv, d, bs, window, self.scale,
+                                    num_splits=splits, waves=waves, prompt_splits=prompt_splits, table_rows=batch.state_slots)
+        elif n_dec:
             ops.attention_mfma(*common, 0, n_dec, 1, 0, n_dec, nh, nkv, d, bs, window, self.scale,
                                split_waves=True, num_splits=splits, waves=waves, table_rows=batch.state_slots)
-        if n_dec < batch.num_seqs:  # portions of prompts: one wave per group of tokens and heads
-            splits = self.prompt_splits(batch.num_seqs - n_dec, batch.max_count, batch.max_context, ops.compute_units(qkv.device))
-            ops.attention_mfma(*common, n_dec, batch.num_seqs - n_dec, batch.max_count, n_dec,
-                               batch.num_tokens - n_dec, nh, nkv, d, bs, window, self.scale, num_splits=splits,
-                               table_rows=batch.state_slots)
+        elif n_prompt:
+            ops.attention_mfma(*common, 0, n_prompt, batch.max_count, 0, batch.num_tokens, nh, nkv, d, bs, window, self.scale,
+                               num_splits=prompt_splits, table_rows=batch.state_slots)
 
     def prompt_splits(self, n_requests: int, max_new: int, max_context: int, cus: int = 256) -> int:
         return prompt_splits(self.num_heads, self.num_kv_heads, self.window, n_requests, max_new, max_context, cus)

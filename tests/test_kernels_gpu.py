@@ -842,8 +842,9 @@ def test_sample_rows_do_not_depend_on_the_batch_or_the_run(vocab):
 
 # ------------------------------------------------------------------ attention on the matrix cores
 def run_attention_mfma(nh, nkv, d, bs, lens, new, window=0, seed=0, craft=None, split_waves=False, num_splits=1,
-                       waves=4, merge_kernel=False, repeat=1):
-    """As `run_attention`, for the bfloat16 matrix-core kernel and its request-wise arguments."""
+                       waves=4, merge_kernel=False, repeat=1, n_decode=None, prompt_splits=1):
+    """As `run_attention`, for the bfloat16 matrix-core kernel and its request-wise arguments; with `n_decode` for a step of that many
+    single tokens and portions after them."""
     dtype = torch.bfloat16
     qs = [rnd(s, nh, d, seed=seed + 3 * b) for b, s in enumerate(lens)]
     ks = [rnd(s, nkv, d, seed=seed + 3 * b + 1) for b, s in enumerate(lens)]
@@ -865,6 +866,10 @@ def run_attention_mfma(nh, nkv, d, bs, lens, new, window=0, seed=0, craft=None, 
     operands = (q, k_pool.to(DEV), v_pool.to(DEV), tables.to(DEV), i32(cu), i32(lens))
     for _ in range(repeat):  # (launches in a row find the counters of the one before zero again)
         out.fill_(float("nan"))
+        if n_decode is not None:
+            ops().attention_mfma_step(out, *operands, n_decode, len(lens) - n_decode, max(new), cu[-1] - n_decode, nh, nkv, d, bs, window,
+                                      num_splits=num_splits, waves=waves, prompt_splits=prompt_splits)
+            continue
         ops().attention_mfma(out, *operands, 0, len(lens), max(new), 0, cu[-1], nh, nkv, d, bs, window, None,
                              split_waves=split_waves, num_splits=num_splits, waves=waves, merge_kernel=merge_kernel)
     got = out.float().cpu()
@@ -934,6 +939,29 @@ def test_decode_keys_at_once_or_shared_out(nh, nkv, d, waves, lens, window):
     if d <= 128:
         short = [i for i, n in enumerate(lens) if n <= 32 * waves * (3 if d <= 64 else 2)]
         assert torch.equal(got[1, False][short], got[4, False][short])
+
+
+@pytest.mark.parametrize("nh,nkv,d,window,singles,splits,waves,portions,new,prompt_splits", [
+    (32, 4, 64, 0, [1, 33, 512, 600, 1300], 1, 8, [300, 700], [300, 257], 1),   # one launch: one column group a wave
+    (32, 4, 64, 0, [1, 512, 513, 1300], 4, 8, [1030, 90], [1030, 20], 1),       # two, and the last workgroup adds shares up
+    (64, 8, 128, 0, [700, 20], 3, 8, [300, 64], [300, 40], 1),
+    (32, 4, 16, 0, [700], 16, 8, [600], [600], 1),
+    (32, 4, 64, 0, [700, 1300], 17, 8, [300, 700], [300, 257], 1),              # more shares than the last workgroup adds up
+    (32, 4, 64, 0, [40, 600], 2, 4, [300, 700], [300, 257], 1),                 # 4 waves to a single token
+    (32, 4, 64, 90, [40, 600], 2, 8, [300, 700], [300, 257], 1), (8, 2, 64, 0, [40, 600], 2, 8, [700], [9], 3),
+    (32, 4, 144, 0, [600, 17], 2, 8, [300, 40], [300, 40], 1)])
+def test_attention_of_single_tokens_and_portions(nh, nkv, d, window, singles, splits, waves, portions, new, prompt_splits):
+    """A step's single tokens and portions, in one launch (the first four) and in two: the same launch after launch."""
+    n = len(singles)
+    got, ref = run_attention_mfma(nh, nkv, d, 16, singles + portions, [1] * n + new, window, seed=75, num_splits=splits, waves=waves,
+                                  n_decode=n, prompt_splits=prompt_splits)
+    assert (got - ref).abs().max() <= 2.0 ** -7 * float(ref.abs().max())
+    again, _ = run_attention_mfma(nh, nkv, d, 16, singles + portions, [1] * n + new, window, seed=75, num_splits=splits, waves=waves,
+                                  n_decode=n, prompt_splits=prompt_splits, repeat=3)
+    assert torch.equal(got, again)
+    from llmserve.ops import library
+
+    assert int(library._arrival_counters(torch.device(DEV)).abs().sum()) == 0
 
 
 @pytest.mark.parametrize("case", [(8, 2, 64, 16, [300, 64, 129, 1, 17, 600, 33, 90], 4, 8), (32, 4, 64, 16, [520], 8, 8),
