@@ -88,14 +88,19 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 # Plain products of TILES_LONG_K columns and more whose tiles leave half the compute units without one are the library's, which
 # shares their K out (one result cannot come in parts, and each tile walks all of K): 65 such products of 9 weights, from 65 rows on,
 # 1.17 in the mean.  2048 x 5632 28 and 16 at 128 rows, 25 and 21 at 228, but 28 and 33 at 613; 1024 x 4096 13 and 9 at 96.
-# Plain products whose tiles are one round that nine tenths of the compute units have a part in leave the library nothing to share out:
-# they are the tiles' up to where the band begins (2048 x 5632 at 2,048 rows 52 and 55).
+# Products whose tiles are one round that three quarters of the compute units have a part in leave the library nothing to share out.  Beyond
+# TILES_WORK, 67 plain ones of 14 weights up to 28672 x 4096 and 128 to 4,096 rows, 0.92 in the mean, 0.72 to 1.02 (2048 x 5632 46 and 51 at
+# 1,629 rows, 4096 x 4096 54 and 58 at 2,048, 4096 x 11008 145 and 164 at 2,048, 8192 x 8192 96 and 103 at 768), and 40 gated ones, 0.87,
+# 0.70 to 0.96 (22016 x 4096 64 and 78 at 330, 12288 x 4096 60 and 67 at 610).  Of columns beyond TILES_ROUND_K and of tiles of 256 x
+# 256 (one wave to a SIMD) too many were slower: 2048 x 16384 151 and 141 at 2,048, 6144 x 2048 53 and 48 at 2,500.  Rotations and parts gain
+# what they spare behind the product on top (parts: the plan says whether K comes in any).
 TILES_WORK = {"plain": 18e9, "gated": 18e9, "rotary": 40e9, "parts": 60e9}
 TILES_GATED_WORK = 130e9
 TILES_GATED_WEIGHT = 100e6
 TILES_LONG_K = 4096
 TILES_GATED_SMALL = 50e6
 TILES_GATED_BAND = (29e9, 36e9)
+TILES_ROUND_K = 12288
 
 
 def tiles_pay(kind: str, m: int, n: int, k: int, cus: int = 256) -> bool:
@@ -105,12 +110,12 @@ def tiles_pay(kind: str, m: int, n: int, k: int, cus: int = 256) -> bool:
     if kind == "gated" and n * k < TILES_GATED_WEIGHT:
         if work >= TILES_GATED_WORK or n * k < TILES_GATED_SMALL and not TILES_GATED_BAND[0] <= work < TILES_GATED_BAND[1]:
             return True
-    if kind == "plain" and m > 64:
+    if m > 64:
         rows, weight_rows = ops.GEMM_TILES[ops.gemm_tiles_plan(m, n, k, 1, cus)[0]][:2]
         tiles = -(-m // rows) * -(-n // weight_rows)
-        if k >= TILES_LONG_K and 2 * tiles <= cus:
+        if kind == "plain" and k >= TILES_LONG_K and 2 * tiles <= cus:
             return False
-        if 0.9 * cus <= tiles <= cus and n * k < TILES_GATED_SMALL and work < TILES_GATED_BAND[0]:
+        if 0.75 * cus <= tiles <= cus and k <= TILES_ROUND_K and rows * weight_rows < 65536:
             return True
     return work < TILES_WORK[kind]
 

@@ -31,6 +31,15 @@ def test_the_faster_way_is_taken(kind, m, n, k, tiles, library):
     assert tiles_pay(kind, m, n, k) == (tiles < library)
 
 
+@pytest.mark.parametrize("kind,m,n,k,tiles,library", [
+    ("plain", 2048, 4096, 11008, 145, 164), ("plain", 1629, 2048, 5632, 46, 51), ("plain", 768, 8192, 8192, 96, 103),
+    ("gated", 330, 22016, 4096, 64, 78), ("gated", 610, 12288, 4096, 60, 67),
+    ("plain", 2048, 2048, 16384, 151, 141), ("plain", 2500, 6144, 2048, 53, 48), ("plain", 1600, 6144, 2048, 41, 36)])
+def test_large_products_of_one_round(kind, m, n, k, tiles, library):
+    """One round of tiles, of up to 12,288 columns and not of 256 x 256; longer rows, those tiles and more rounds stay as they were."""
+    assert tiles_pay(kind, m, n, k) == (tiles < library)
+
+
 def test_what_the_tiles_leave_behind_is_the_librarys():
     """A gated product, a rotation or parts of K that the tiles decline become a plain product and a kernel: the plain product must
     then not be theirs either, as it was the library's product that was the faster one."""
