@@ -211,8 +211,9 @@ def decode_arrangement(num_heads: int, num_kv_heads: int, head_dim: int, window:
     7.1, of 1,000 8.5, 7.3, 7.1, 7.7, of 4,000 21.9, 14.9, 10.9, 9.6; 8 requests of 768 7.2, 8.1, 7.9, 9.2, of 1,000 8.7, 8.3, 8.2,
     9.5, of 2,048 16.2, 12.5, 10.6, 11.4; 8 KV heads of 128, 4 requests of 600 keys 10.4, 10.7, 9.1, 10.6, of 1,000 17.1, 12.6, 11.3,
     12.1).  Once the batch alone fills the chip (a workgroup for each of its `cus` compute units) nothing is split.  More than
-    16 shares would need a kernel to add them up: they wait until a wave would walk more than 4 tiles.  Wider heads are split
-    where a wave would walk more than 4 tiles."""
+    16 shares would need a kernel to add them up: they wait until a wave would walk more than 4 tiles.  Wider heads, and batches
+    that leave fewer than four compute units to a workgroup, are split where a wave would walk more than 4 tiles (two shares by the
+    reach of 1,024 that 32 requests of 580 keys have cost a step of the 1.1B shape 1.105 ms, one share 1.095)."""
     g = num_heads // num_kv_heads
     groups = n_requests * num_kv_heads * -(-g // 16)
     reach = min(max_context, window) if window else max_context
@@ -224,6 +225,7 @@ def decode_arrangement(num_heads: int, num_kv_heads: int, head_dim: int, window:
     if head_dim <= 128:
         if tiles <= (3 if head_dim <= 64 else 2) * waves:
             return 1, waves
-        splits = max(min(16, max(4, -(-tiles // (2 * waves)))), splits)
+        if 4 * groups <= cus:
+            splits = max(min(16, max(4, -(-tiles // (2 * waves)))), splits)
     splits = max(1, min(cus // groups, splits))
     return splits, waves
