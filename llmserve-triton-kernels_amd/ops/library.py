@@ -512,9 +512,15 @@ def gemm_decode_k_parts(m: int, k: int) -> int:
     return first if (first - 1) * (-(-chunks // first) * 128) < k else 0
 
 
+def gemm_decode_reaches(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ops.gemm_decode's 32-bit offsets reach all of x and w: less than 2 GB each."""
+    return w.numel() < 1 << 30 and x.shape[0] * x.stride(0) < 1 << 30
+
+
 def gemm_decode_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ops.gemm_decode takes x [M, K] against w [N, K]."""
-    return x.dtype == torch.bfloat16 and gemm_decode_fits(x.shape[0], x.shape[1]) and gemm_bf16_supported(x, w)
+    return (x.dtype == torch.bfloat16 and gemm_decode_fits(x.shape[0], x.shape[1]) and gemm_bf16_supported(x, w)
+            and gemm_decode_reaches(x, w))
 
 
 def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,

@@ -174,7 +174,7 @@ def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor, from_cache: bool 
     m = x.shape[0]
     if not (SPLIT_K and x.dtype == torch.bfloat16 and ops.gemm_bf16_supported(x, weight)):
         return None
-    if STREAM_ROWS < m <= STREAM_MAX_ROWS and DECODE_KERNEL:
+    if STREAM_ROWS < m <= STREAM_MAX_ROWS and DECODE_KERNEL and ops.gemm_decode_reaches(x, weight):
         k_parts = ops.gemm_decode_k_parts(m, weight.shape[1])
         if k_parts > 1:  # the rows in registers, K shared out to a few sets of workgroups
             parts = torch.empty((k_parts, m, weight.shape[0]), dtype=torch.float32, device=x.device)

@@ -537,6 +537,21 @@ def test_gemm_decode_refuses_what_it_cannot_take():
     assert not ops().gemm_decode_supported(x, w) and ops().gemm_decode_supported(x[:64], w)
 
 
+@pytest.mark.parametrize("m", [1, 9, 40])
+def test_a_vocabulary_weight_of_2_gb(m):
+    """2^30 elements, beyond the decode kernel's offsets: the product goes elsewhere and is right at both ends."""
+    from llmserve.parts.linear import linear, linear_partial_sums
+
+    n, k = 1 << 18, 4096
+    w = torch.empty(n, k, dtype=torch.bfloat16, device=DEV).normal_(0, 0.02)
+    x = rnd(m, k, seed=21).bfloat16().to(DEV)
+    out = linear(x, w, out_dtype=torch.float32)
+    for rows in (slice(0, 300), slice(n - 300, n)):
+        ref = x.double() @ w[rows].double().t()
+        assert (out[:, rows].double() - ref).abs().max() <= 2e-6 * math.sqrt(k) * float(ref.abs().max())
+    assert linear_partial_sums(x, w) is None
+
+
 @pytest.mark.parametrize("m,n,k,eps", [(1, 64, 64, 1e-5), (8, 2560, 2048, 1e-5), (16, 333, 96, 1e-6), (5, 100, 4096, 1e-5),
                                        (3, 48, 5888 - 8, 1e-6), (13, 200, 2560, 1e-5), (16, 11264, 2048, 1e-5),
                                        (16, 2560, 4096, 1e-5), (9, 100, 5632, 1e-6), (12, 333, 3072 + 8, 1e-6)])

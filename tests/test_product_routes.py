@@ -1,5 +1,6 @@
 """Which products of many bfloat16 rows go to the tiles and which to the library: a rule on sizes alone (no GPU)."""
 import pytest
+import torch
 
 from llmserve.parts.linear import TILES_WORK, tiles_pay
 
@@ -83,3 +84,22 @@ def test_which_compute_units_bring_a_weight_nearer():
     for m, n in ((1024, 2048), (2048, 4096), (4096, 8192)):
         bm, bn, held = library.GEMM_TILES[library.gemm_tiles_plan(m, n, 2048)[0]][:3]
         assert -(-m // bm) * -(-n // bn) % (256 * held) == 0 and workers(m, n, 1) == 0
+
+
+@pytest.mark.parametrize("n,k", [(262144, 4096), (262208, 5376)])
+def test_weights_of_2_gb_and_more_do_not_go_to_the_decode_kernel(n, k):
+    """Its offsets are 32-bit (the launcher refuses 2^30 elements): such a weight goes to the streaming kernel, the tiles or the
+    library, whatever the rows.  Shapes alone, on the meta device."""
+    from llmserve.ops import library
+    from llmserve.parts import linear
+
+    def bf16(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="meta")
+
+    for m in (1, 8, 9, 16, 17, 64):
+        fits = library.gemm_decode_fits(m, k)
+        assert not linear.decode_product(bf16(m, k), bf16(n, k))
+        assert linear.decode_product(bf16(m, k), bf16((1 << 30) // k - 1, k)) == fits
+    assert linear.few_rows(16, bf16(n, k))
+    assert not library.gemm_decode_reaches(bf16(40, 2048), bf16(1 << 19, 2048)) and library.gemm_decode_reaches(bf16(40, 2048), bf16((1 << 19) - 1, 2048))
+    assert not library.gemm_decode_supported(bf16(4, 1 << 28)[:, :4096], bf16(64, 4096))
