@@ -1103,6 +1103,31 @@ static int launch_attn(int db, dim3 grid, int threads, const AttnArgs& a, hipStr
 
 #endif
 
+// How portions of prompts are dealt out.
+struct PromptGrid {
+    dim3 grid;
+    int cg;
+    bool twin;
+};
+static PromptGrid prompt_grid(int n_heads, int n_kv_heads, int head_dim, int window, int n_seqs, int max_new, int num_splits) {
+    const int G = n_heads / n_kv_heads, HG = G < 16 ? G : 16, TPG = 16 / HG, HB = (G + HG - 1) / HG;
+    const int groups = (max_new + TPG - 1) / TPG;
+    // twins (8 waves, two tiles a round) where a workgroup per CU is left that way; wider heads would not fit
+    // the registers of 8 waves, a window or splits have their own arrangement
+    bool twin = window == 0 && head_dim <= 16 * PROMPT_TWIN_MAX_DB && num_splits == 1;
+    auto grid_for = [&](int cg) {
+        const int per_block = PROMPT_WB * cg;  // column groups of a block of tokens
+        return dim3((groups + per_block - 1) / per_block * num_splits, n_kv_heads * HB, n_seqs);
+    };
+    auto workgroups = [](dim3 g) { return (long long)g.x * g.y * g.z; };
+    int cg = PROMPT_CG_MAX(head_dim / 16);
+    dim3 grid = grid_for(cg);
+    if (cg == 2 && workgroups(grid) < PROMPT_FULL_CHIP * (twin && head_dim <= 64 ? 2 : 1)) grid = grid_for(cg = 1);
+    if (twin && workgroups(grid) < PROMPT_FULL_CHIP) twin = false;  // a short portion: workgroups for more CUs matter more
+    if (twin) grid = dim3(grid.y, grid.x, grid.z);  // heads in x, blocks of tokens in y: the order in which workgroups are handed out
+    return {grid, cg, twin};
+}
+
 extern "C" {
 
 // Attention for the requests [seq_begin, seq_begin + n_seqs) of a step.  max_new: most new tokens any of
@@ -1116,8 +1141,7 @@ extern "C" {
 struct AttnLaunch {  // what a launch of one of the kernels above would be
     AttnArgs a;
     dim3 grid;
-    int cg;     // prompts
-    bool twin;  // prompts
+    int cg;  // prompts
 };
 static int attention_mfma_launch(AttnLaunch* only, void* out, int out_stride, const void* q, int q_stride, const void* k_pool,
                         const void* v_pool, const int* block_tables, const int* table_rows, int max_blocks,
@@ -1161,7 +1185,7 @@ static int attention_mfma_launch(AttnLaunch* only, void* out, int out_stride, co
         dim3 grid(groups * num_splits, n_kv_heads * HB, n_seqs);
         if (arrive && num_splits > 1 && num_splits <= 16 && (long long)groups * grid.y * grid.z <= n_arrive) a.arrive = arrive;
         if (only) {
-            *only = AttnLaunch{a, grid, 0, false};
+            *only = AttnLaunch{a, grid, 0};
             return LLMS_OK;
         }
         if (int e = launch_attn(head_dim / 16, grid, waves * LLMS_WAVE, a, stream)) return e;
@@ -1174,21 +1198,12 @@ static int attention_mfma_launch(AttnLaunch* only, void* out, int out_stride, co
             launch_merge(out, out_stride, ws_o, ws_ml, token_begin, n_tokens, n_heads, head_dim, num_splits, gate, gate_stride, stream);
         }
     } else {
-        // twins (8 waves, two tiles a round) where a workgroup per CU is left that way; wider heads would not fit
-        // the registers of 8 waves, a window or splits have their own arrangement
-        bool twin = window == 0 && head_dim <= 16 * PROMPT_TWIN_MAX_DB && num_splits == 1;
-        auto grid_for = [&](int cg) {
-            const int per_block = PROMPT_WB * cg;  // column groups of a block of tokens
-            return dim3((groups + per_block - 1) / per_block * num_splits, n_kv_heads * HB, n_seqs);
-        };
-        auto workgroups = [](dim3 g) { return (long long)g.x * g.y * g.z; };
-        int cg = PROMPT_CG_MAX(head_dim / 16);
-        dim3 grid = grid_for(cg);
-        if (cg == 2 && workgroups(grid) < PROMPT_FULL_CHIP * (twin && head_dim <= 64 ? 2 : 1)) grid = grid_for(cg = 1);
-        if (twin && workgroups(grid) < PROMPT_FULL_CHIP) twin = false;  // a short portion: workgroups for more CUs matter more
-        if (twin) {  // heads in x, blocks of tokens in y: the order in which workgroups are handed out
-            LLMS_REQUIRE(grid.x <= 65535, "attention_mfma: too many tokens per request for one launch");
-            grid = dim3(grid.y, grid.x, grid.z);
+        const PromptGrid way = prompt_grid(n_heads, n_kv_heads, head_dim, window, n_seqs, max_new, num_splits);
+        const dim3 grid = way.grid;
+        const int cg = way.cg;
+        const bool twin = way.twin;
+        if (twin) {
+            LLMS_REQUIRE(grid.y <= 65535, "attention_mfma: too many tokens per request for one launch");
             int cus = 0;
             if (int e = compute_units(&cus)) return e;
             // The first workgroup of every CU: the longest blocks, shortest of them first; then from the longest
@@ -1199,7 +1214,7 @@ static int attention_mfma_launch(AttnLaunch* only, void* out, int out_stride, co
             a.first_blocks = n_seqs == 1 ? (int)std::min<long long>(grid.y, cus / grid.x) : 0;
         }
         if (only) {
-            *only = AttnLaunch{a, grid, cg, twin};
+            *only = AttnLaunch{a, grid, cg};
             return LLMS_OK;
         }
         if (int e = launch_prompt(head_dim / 16, cg, grid, twin, a, stream)) return e;
@@ -1230,8 +1245,19 @@ int llms_attention_mfma(void* out, int out_stride, const void* q, int q_stride, 
                                  nullptr, 0, nullptr, 0, stream);
 }
 
+// How a step of both is launched: column groups a wave of the portions where both are one launch, 0 where they are two.  One where the portions
+// have twins, no window and heads of up to 128 numbers, 8 waves share a single token's keys, n_arrive counters (0: none) let the last
+// workgroup add shares up, and the launch, which counts workgroups in one dimension, has fewer than 2^32 threads.
+int llms_attention_mfma_step_in_one(int n_heads, int n_kv_heads, int head_dim, int window, int n_decode, int num_splits, int waves,
+                                    int n_arrive, int n_seqs, int max_new, int prompt_splits) {
+    const int G = n_heads / n_kv_heads, HB = (G + 15) / 16;
+    const PromptGrid p = prompt_grid(n_heads, n_kv_heads, head_dim, window, n_seqs, max_new, prompt_splits);
+    const long long keys = (long long)n_kv_heads * HB * n_decode, all = keys * num_splits + (long long)p.grid.x * p.grid.y * p.grid.z;
+    const bool merges = num_splits == 1 || (num_splits <= 16 && keys <= n_arrive);
+    return waves == 8 && p.twin && head_dim <= 128 && merges && all < (1ll << 32) / (8 * LLMS_WAVE) ? p.cg : 0;
+}
+
 // A step's attention in one call: n_decode requests of one token each (rows 0 ..), then n_seqs portions of up to max_new tokens, n_tokens in all.
-// One launch where the portions have twins, no window and heads of up to 128 numbers, and 8 waves share a single token's keys; otherwise one each.
 int llms_attention_mfma_step(void* out, int out_stride, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                              const int* block_tables, const int* table_rows, int max_blocks, const int* cu_seqlens,
                              const int* context_lens, int n_heads, int n_kv_heads, int head_dim, int block_size, int window, float scale,
@@ -1250,12 +1276,13 @@ int llms_attention_mfma_step(void* out, int out_stride, const void* q, int q_str
     AttnLaunch d{}, p{};
     if (int e = decode(&d)) return e;
     if (int e = prompt(&p)) return e;
-    const long long n_d = (long long)d.grid.x * d.grid.y * d.grid.z, n_p = (long long)p.grid.x * p.grid.y * p.grid.z;
-    if (!(waves == 8 && p.twin && head_dim <= 128 && (num_splits == 1 || d.a.arrive) && n_d + n_p < (1ll << 31))) {
+    if (!llms_attention_mfma_step_in_one(n_heads, n_kv_heads, head_dim, window, n_decode, num_splits, waves, arrive ? n_arrive : 0, n_seqs,
+                                         max_new, prompt_splits)) {
         if (int e = decode(nullptr)) return e;
         return prompt(nullptr);
     }
-    const dim3 grid((unsigned)(n_d + n_p));
+    const unsigned n_d = d.grid.x * d.grid.y * d.grid.z;
+    const dim3 grid(n_d + p.grid.x * p.grid.y * p.grid.z);
 #define ATT_BOTH(N, C) attn_both_kernel<N, C><<<grid, 8 * LLMS_WAVE, 0, stream>>>(d.a, p.a, (int)n_d, d.grid.x, d.grid.y, p.grid.x, p.grid.y)
 #define ATT_CASE(N)                     \
     case N:                             \

@@ -968,6 +968,9 @@ def test_decode_keys_at_once_or_shared_out(nh, nkv, d, waves, lens, window):
 def test_attention_of_single_tokens_and_portions(nh, nkv, d, window, singles, splits, waves, portions, new, prompt_splits):
     """A step's single tokens and portions, in one launch (the first four) and in two: the same launch after launch."""
     n = len(singles)
+    way = ops().load("attention_mfma").llms_attention_mfma_step_in_one(nh, nkv, d, window, n, splits, waves, ops().ARRIVAL_COUNTERS,
+                                                                       len(portions), max(new), prompt_splits)
+    assert way == {(300, 700): 1, (1030, 90): 2, (300, 64): 2, (600,): 1}.get(tuple(portions), 0) * (waves == 8 and window == 0 and splits <= 16)
     got, ref = run_attention_mfma(nh, nkv, d, 16, singles + portions, [1] * n + new, window, seed=75, num_splits=splits, waves=waves,
                                   n_decode=n, prompt_splits=prompt_splits)
     assert (got - ref).abs().max() <= 2.0 ** -7 * float(ref.abs().max())
