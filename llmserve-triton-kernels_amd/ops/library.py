@@ -1001,8 +1001,9 @@ def attention_mfma(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor, v_p
     if num_splits > 1 and split_waves and not (merge_kernel or MERGE_BY_KERNEL):
         arrive = _arrival_counters(dev)
     if num_splits > 1:
-        ws_o = torch.empty((q.shape[0] * n_heads * num_splits * head_dim,), dtype=torch.float32, device=dev)
-        ws_ml = torch.empty((q.shape[0] * n_heads * num_splits * 2,), dtype=torch.float32, device=dev)
+        rows = token_begin + n_tokens  # (the shares are indexed by row of q)
+        ws_o = torch.empty((rows * n_heads * num_splits * head_dim,), dtype=torch.float32, device=dev)
+        ws_ml = torch.empty((rows * n_heads * num_splits * 2,), dtype=torch.float32, device=dev)
     scale = 1.0 / math.sqrt(head_dim) if scale is None else scale
     if head_gate is None:
         entry, gate_args = load("attention_mfma").llms_attention_mfma, ()
@@ -1036,14 +1037,14 @@ def attention_mfma_step(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tensor
     if n_decode < 1 or n_seqs < 1 or n_tokens < 1:
         raise ValueError("a step of single tokens and portions has some of each")
 
-    def workspace(splits):
+    def workspace(splits, rows):  # (indexed by row: the single tokens' are the first ones)
         if splits == 1:
             return None, None
-        return (torch.empty((q.shape[0] * n_heads * splits * head_dim,), dtype=torch.float32, device=dev),
-                torch.empty((q.shape[0] * n_heads * splits * 2,), dtype=torch.float32, device=dev))
+        return (torch.empty((rows * n_heads * splits * head_dim,), dtype=torch.float32, device=dev),
+                torch.empty((rows * n_heads * splits * 2,), dtype=torch.float32, device=dev))
 
     arrive = _arrival_counters(dev) if num_splits > 1 and not MERGE_BY_KERNEL else None
-    (ws_o, ws_ml), (prompt_ws_o, prompt_ws_ml) = workspace(num_splits), workspace(prompt_splits)
+    (ws_o, ws_ml), (prompt_ws_o, prompt_ws_ml) = workspace(num_splits, n_decode), workspace(prompt_splits, n_decode + n_tokens)
     _check(load("attention_mfma").llms_attention_mfma_step(
         _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables), _ptr(table_rows),
         c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), c_int(n_heads), c_int(n_kv_heads), c_int(head_dim),

@@ -982,6 +982,28 @@ def test_attention_of_single_tokens_and_portions(nh, nkv, d, window, singles, sp
     assert int(library._arrival_counters(torch.device(DEV)).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("together", [True, False])
+def test_shares_of_single_tokens_take_no_room_for_a_steps_other_rows(together):
+    """Two single tokens in front of 4,094 rows of portions: their shares are two rows."""
+    nh, nkv, d, bs, portion, splits = 32, 4, 64, 16, 4094, 16
+    q = rnd(2 + portion, nh * d, seed=3).bfloat16().to(DEV)
+    out, pages = torch.empty_like(q), portion // bs + 1
+    k_pool, v_pool = rnd(pages, nkv, bs, d, seed=4).bfloat16().to(DEV), rnd(pages, nkv, d, bs, seed=5).bfloat16().to(DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    operands = (out, q, k_pool, v_pool, torch.arange(pages, dtype=torch.int32, device=DEV).repeat(3, 1), i32([0, 1, 2, 2 + portion]),
+                i32([2000, 1200, portion]))
+    ops()._arrival_counters(torch.device(DEV))
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    if together:
+        ops().attention_mfma_step(*operands, 2, 1, portion, portion, nh, nkv, d, bs, num_splits=splits, waves=8)
+    else:
+        ops().attention_mfma(*operands, 0, 2, 1, 0, 2, nh, nkv, d, bs, split_waves=True, num_splits=splits, waves=8)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - before <= 2 * nh * splits * (d + 2) * 4 + 2 * 512  # (two blocks, rounded up)
+
+
 @pytest.mark.parametrize("case", [(8, 2, 64, 16, [300, 64, 129, 1, 17, 600, 33, 90], 4, 8), (32, 4, 64, 16, [520], 8, 8),
                                   (64, 8, 128, 16, [700, 33], 2, 8), (3, 1, 32, 8, [1, 7, 40, 100], 3, 4),
                                   (6, 2, 80, 8, [70, 19, 300], 16, 4), (4, 4, 256, 16, [257, 31], 5, 4),
