@@ -940,13 +940,13 @@ def test_attention_mfma(case, arrangement):
     (8, 1, 64, 8, [1, 32, 33, 256, 257, 512, 513, 768, 769, 1500]),   # three tiles a wave at once: up to 768 keys
     (8, 2, 64, 4, [128, 129, 384, 385, 1000]),
     (4, 2, 128, 8, [255, 256, 257, 512, 513, 1100]),                  # two tiles a wave: up to 512
-    (3, 1, 144, 8, [200, 256, 257, 900]), (2, 1, 16, 8, [767, 770])])
+    (3, 1, 144, 8, [200, 256, 257, 900]), (2, 1, 16, 8, [767, 770]), (7, 7, 64, 8, [600, 20, 900] * 5)])
 def test_decode_keys_at_once_or_shared_out(nh, nkv, d, waves, lens, window):
     """One, two and three tiles a wave in one trip, one key more than that, and many: requests of all lengths in one launch, each
     shared out to workgroups or not by its own length.  The last workgroup and the second kernel give the same bits, and one
     workgroup to a request what they give for requests that are not shared out."""
     new, got = [1] * len(lens), {}
-    for splits, kernel in ((1, False), (4, False), (4, True), (7, False), (7, True)):
+    for splits, kernel in ((1, False), (2, False), (4, False), (4, True), (7, False), (7, True), (8, False), (12, False), (16, False)):
         got[splits, kernel], ref = run_attention_mfma(nh, nkv, d, 16, lens, new, window, seed=70, split_waves=True, num_splits=splits,
                                                       waves=waves, merge_kernel=kernel)
         assert (got[splits, kernel] - ref).abs().max() <= 2.0 ** -7 * float(ref.abs().max())
