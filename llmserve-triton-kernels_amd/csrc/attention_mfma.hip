@@ -437,10 +437,10 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, const Place at) {
     // first and last tile whose 32 keys every column of the group sees
     const int lo_max = (a.window > 0 && p_max - a.window + 1 > 0) ? p_max - a.window + 1 : 0;
 
-    // this workgroup's share of the tiles, dealt to its waves.  What one workgroup brings in at once is not shared out (num_splits goes by
-    // the longest context that a step may have: a shared request of 600 keys costs 1 microsecond more): the other workgroups leave, or
-    // where a kernel adds the shares up leave one without keys, which changes no bit of the sum.
-    const bool alone = a.num_splits == 1 || (DB <= 8 && n_tiles <= AHEAD * NW);
+    // this workgroup's share of the tiles, dealt to its waves.  A request of few tiles (the line of decode_arrangement in parts/attention.py,
+    // whichever kernel this is part of) is not shared out, whatever num_splits, which goes by the longest context that a step may have: the
+    // other workgroups leave, or where a kernel adds the shares up leave one without keys, which changes no bit of the sum.
+    const bool alone = a.num_splits == 1 || (DB <= 8 && n_tiles <= (DB <= 6 ? 3 : 2) * NW);
     if (alone && split > 0 && a.arrive) return;
     const bool direct = a.num_splits == 1 || (alone && a.arrive);
     const int per_split = alone ? n_tiles : (n_tiles + a.num_splits - 1) / a.num_splits;

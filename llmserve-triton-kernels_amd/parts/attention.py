@@ -204,16 +204,18 @@ def prompt_splits(num_heads: int, num_kv_heads: int, window: int | None, n_reque
 def decode_arrangement(num_heads: int, num_kv_heads: int, head_dim: int, window: int | None, n_requests: int, max_context: int,
                        cus: int = 256) -> tuple[int, int]:
     """(workgroups per request and KV head, waves per workgroup) for decoding.  The waves of a workgroup take 32 keys at a time each
-    and merge in LDS; workgroups that share a request hand their shares to the one that finishes last, through memory, which costs 1
-    to 1.5 microseconds and little more for four of them than for two.  A compute unit takes in some 60 GB/s of keys and values, so what
-    does not come in one trip (three tiles a wave up to a head size of 64, two up to 128) is shared out, to at least four, of at most
-    two tiles a wave (microseconds with one workgroup, two, four and eight, 4 KV heads of 64 numbers: 1 request of 600 keys 6.1, 6.9, 6.3,
-    7.1, of 1,000 8.5, 7.3, 7.1, 7.7, of 4,000 21.9, 14.9, 10.9, 9.6; 8 requests of 768 7.2, 8.1, 7.9, 9.2, of 1,000 8.7, 8.3, 8.2,
-    9.5, of 2,048 16.2, 12.5, 10.6, 11.4; 8 KV heads of 128, 4 requests of 600 keys 10.4, 10.7, 9.1, 10.6, of 1,000 17.1, 12.6, 11.3,
-    12.1).  Once the batch alone fills the chip (a workgroup for each of its `cus` compute units) nothing is split.  More than
-    16 shares would need a kernel to add them up: they wait until a wave would walk more than 4 tiles.  Wider heads, and batches
-    that leave fewer than four compute units to a workgroup, are split where a wave would walk more than 4 tiles (two shares by the
-    reach of 1,024 that 32 requests of 580 keys have cost a step of the 1.1B shape 1.105 ms, one share 1.095)."""
+    and merge in LDS; workgroups that share a request hand their shares to the one that finishes last, through memory, which costs
+    some 1.5 microseconds and little more for four of them than for two.  A compute unit takes in some 60 GB/s of keys and values, so what
+    is more than three tiles a wave (two beyond a head size of 96) is shared out, to at least four, of at most two tiles a wave.
+    Microseconds with one workgroup, two, four and eight, 4 KV heads of 64 numbers: 1 request of 800 keys 7.2, 7.1, 6.5, 7.2, of 1,000 8.2,
+    7.3, 6.6, 7.4, of 4,000 21.7, 14.7, 10.6, 9.2; 8 requests of 800 7.5, 8.2, 7.4, 8.7, of 1,000 8.5, 8.3, 7.7, 9.2, of 2,048 16.2, 12.4,
+    10.4, 11.1; 8 KV heads of 128, 4 requests of 600 keys 10.0, 10.7, 8.6, 10.0, of 1,000 16.7, 12.6, 10.7, 11.8.  More than eight
+    of them only pay for up to cus / 32 requests and heads (16 of 8,000 keys: 1 request with 8 heads of 64 13.7 with eight and 12.9 with
+    sixteen, 4 with 4 15.6 and 16.5, 4 with 8 19.4 and 26.0) or where a wave would walk more than 4 tiles; beyond 16 a kernel adds
+    them up.  Wider heads, and batches that leave fewer than four compute units to a workgroup (eight up to a head size of 48: 16 requests
+    of 800 keys 6.4 with one, 8.0 with four), are split where a wave would walk more than 4 tiles (32 requests of 1,000 keys 12.2
+    with one, 12.3 with two, 24 of them 11.5 and 10.9).  Once the batch alone fills the chip (a workgroup for each of its `cus` compute
+    units) nothing is split."""
     g = num_heads // num_kv_heads
     groups = n_requests * num_kv_heads * -(-g // 16)
     reach = min(max_context, window) if window else max_context
@@ -223,9 +225,9 @@ def decode_arrangement(num_heads: int, num_kv_heads: int, head_dim: int, window:
     tiles = -(-reach // 32)
     splits = -(-tiles // (4 * waves))
     if head_dim <= 128:
-        if tiles <= (3 if head_dim <= 64 else 2) * waves:
+        if tiles <= (3 if head_dim <= 96 else 2) * waves:
             return 1, waves
-        if 4 * groups <= cus:
-            splits = max(min(16, max(4, -(-tiles // (2 * waves)))), splits)
+        if (4 if head_dim > 48 else 8) * groups <= cus:
+            splits = max(min(16 if 32 * groups <= cus else 8, max(4, -(-tiles // (2 * waves)))), splits)
     splits = max(1, min(cus // groups, splits))
     return splits, waves

@@ -940,7 +940,8 @@ def test_attention_mfma(case, arrangement):
     (8, 1, 64, 8, [1, 32, 33, 256, 257, 512, 513, 768, 769, 1500]),   # three tiles a wave at once: up to 768 keys
     (8, 2, 64, 4, [128, 129, 384, 385, 1000]),
     (4, 2, 128, 8, [255, 256, 257, 512, 513, 1100]),                  # two tiles a wave: up to 512
-    (3, 1, 144, 8, [200, 256, 257, 900]), (2, 1, 16, 8, [767, 770]), (7, 7, 64, 8, [600, 20, 900] * 5)])
+    (3, 1, 144, 8, [200, 256, 257, 900]), (2, 1, 16, 8, [767, 770]),
+    (20, 1, 96, 8, [300, 512, 513, 768, 769, 1500]), (7, 7, 64, 8, [600, 20, 900] * 5)])      # over 16 heads a KV head; turns of all places
 def test_decode_keys_at_once_or_shared_out(nh, nkv, d, waves, lens, window):
     """One, two and three tiles a wave in one trip, one key more than that, and many: requests of all lengths in one launch, each
     shared out to workgroups or not by its own length.  The last workgroup and the second kernel give the same bits, and one
@@ -952,7 +953,7 @@ def test_decode_keys_at_once_or_shared_out(nh, nkv, d, waves, lens, window):
         assert (got[splits, kernel] - ref).abs().max() <= 2.0 ** -7 * float(ref.abs().max())
     assert torch.equal(got[4, False], got[4, True]) and torch.equal(got[7, False], got[7, True])
     if d <= 128:
-        short = [i for i, n in enumerate(lens) if n <= 32 * waves * (3 if d <= 64 else 2)]
+        short = [i for i, n in enumerate(lens) if n <= 32 * waves * (3 if d <= 96 else 2)]
         assert torch.equal(got[1, False][short], got[4, False][short])
 
 
@@ -977,6 +978,9 @@ def test_attention_of_single_tokens_and_portions(nh, nkv, d, window, singles, sp
     again, _ = run_attention_mfma(nh, nkv, d, 16, singles + portions, [1] * n + new, window, seed=75, num_splits=splits, waves=waves,
                                   n_decode=n, prompt_splits=prompt_splits, repeat=3)
     assert torch.equal(got, again)
+    # a single token has the bits that it has without portions beside it: its keys are shared out or not by the same line
+    without, _ = run_attention_mfma(nh, nkv, d, 16, singles, [1] * n, window, seed=75, split_waves=True, num_splits=splits, waves=waves)
+    assert torch.equal(got[:n], without)
     from llmserve.ops import library
 
     assert int(library._arrival_counters(torch.device(DEV)).abs().sum()) == 0
