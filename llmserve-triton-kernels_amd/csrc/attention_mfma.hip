@@ -968,20 +968,20 @@ __global__ __launch_bounds__((TWIN ? 2 : 1) * WB * LLMS_WAVE, (TWIN && DB <= 4) 
 }
 
 #if !defined(LLMS_ATTENTION_BIASED) && !defined(LLMS_ATTENTION_HEAD_GATED)
-// A step that has both: the first `n_decode` workgroups are those of the single tokens, the others those of the portions with twins.  Neither
-// needs what the other leaves, but as two launches the single tokens' waited for memory with most of the chip idle while the portions' had
-// not begun: 32 heads of 64 with 4 KV heads, 32 tokens with 512 keys and a portion of 512, 15.7 us as two and 13.0 as one; 48 tokens with
-// 1024 keys, 27.1 and 21.7; 8 tokens with 2000 keys and a portion of 2048, 46.3 and 36.5; 32 heads of 128 with 8, 16 tokens with 1024, 38.8
-// and 36.9.  The single tokens come first because each is one chain of trips to memory (last: the same to 1 % slower, steps with long
-// contexts).  They ask for two tiles a wave at once, not three: the kernel's registers are then those of the portions.
+// A step that has both: `n_decode` workgroups from `decode_at` on are those of the single tokens, the others those of the portions with twins.
+// Neither needs what the other leaves, but as two launches the single tokens' waited for memory with most of the chip idle while the portions'
+// had not begun: 32 heads of 64 with 4 KV heads, 32 tokens with 500 keys and a portion of 512, 17.2 us as two and 10.8 as one; 3 tokens with
+// 1,900 keys and a portion of 512 behind 1,388, 32.1 and 24.2; 8 tokens with 2,000 keys and a portion of 2,048, 43.0 and 35.0; 32 heads of 128
+// with 8, 16 tokens with 1,000 and a portion of 512 behind 1,388, 52.9 and 47.3.
+// They ask for two tiles a wave at once, not three: the kernel's registers are then those of the portions.
 template <int DB, int CG>
 __global__ __launch_bounds__(8 * LLMS_WAVE, DB <= 4 ? 4 : 1) void attn_both_kernel(const AttnArgs decode, const AttnArgs prompt, int n_decode,
-                                                                                  int dx, int dy, int px, int py) {
-    const int w = blockIdx.x;
-    if (w < n_decode) {
+                                                                                  int dx, int dy, int px, int py, int decode_at) {
+    const int w = (int)blockIdx.x - decode_at;
+    if ((unsigned)w < (unsigned)n_decode) {
         attn_decode<DB, 8, 2>(decode, Place{w % dx, w / dx % dy, w / (dx * dy), dy});
     } else {
-        const int v = w - n_decode;
+        const int v = decode_at ? (int)blockIdx.x : w - n_decode;
         attn_prompt<DB, true, CG, 4>(prompt, Place{v % px, v / px % py, v / (px * py), py});
     }
 }
@@ -1312,9 +1312,21 @@ int llms_attention_mfma_step(void* out, int out_stride, const void* q, int q_str
         if (int e = decode(nullptr)) return e;
         return prompt(nullptr);
     }
-    const unsigned n_d = d.grid.x * d.grid.y * d.grid.z;
-    const dim3 grid(n_d + p.grid.x * p.grid.y * p.grid.z);
-#define ATT_BOTH(N, C) attn_both_kernel<N, C><<<grid, 8 * LLMS_WAVE, 0, stream>>>(d.a, p.a, (int)n_d, d.grid.x, d.grid.y, p.grid.x, p.grid.y)
+    const int n_d = (int)(d.grid.x * d.grid.y * d.grid.z), n_p = (int)(p.grid.x * p.grid.y * p.grid.z);
+    // Single tokens first: each is one chain of trips to memory.  The order of a lone portion's blocks counts on the first workgroup of every
+    // compute unit, and those are then the single tokens' on as many of them; many single tokens of narrow heads come last instead
+    // (two workgroups a compute unit: theirs fill the second places).  Without either, 48 tokens of 700 keys and 8 KV heads of 64 beside 512 tokens
+    // behind 1,388 took 41.5 microseconds for 39.3 as two launches, now 27.7; 3 of 1,900 keys and 4 KV heads 27.1, now 24.2; 480 steps of
+    // both in the mean 0.87 of two launches, now 0.82.  Several portions have no such order, and single tokens last were up to 36 % slower.
+    int decode_at = 0;
+    if (n_seqs == 1) {
+        int cus = 0;
+        if (int e = compute_units(&cus)) return e;
+        if (head_dim <= 64 && 4 * n_d > cus) decode_at = n_p;
+        else p.a.first_blocks = std::min(p.a.first_blocks, std::max(0, cus - n_d) / (int)p.grid.x);
+    }
+    const dim3 grid((unsigned)(n_d + n_p));
+#define ATT_BOTH(N, C) attn_both_kernel<N, C><<<grid, 8 * LLMS_WAVE, 0, stream>>>(d.a, p.a, n_d, d.grid.x, d.grid.y, p.grid.x, p.grid.y, decode_at)
 #define ATT_CASE(N)                     \
     case N:                             \
         if (p.cg == 2) ATT_BOTH(N, 2);  \
