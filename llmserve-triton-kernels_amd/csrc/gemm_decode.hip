@@ -302,7 +302,8 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     constexpr int UPT = PAIRS ? 8 : 4 * LPI;  // units per tile
     constexpr int ITEMS = NT * XC;            // items (tile, chunk) of a group
     // items in flight per wave; a divisor of ITEMS, so that an item has the same place in the ring in every group
-    constexpr int RING = ITEMS % 2 == 0 ? 2 : (ITEMS < 3 ? ITEMS : 3);
+    // (three of the half items of 8 weight rows and six chunks: 896 x 4864 at 1 row 4.66 -> 4.52 microseconds, 4608 x 4608 10.8 -> 10.2)
+    constexpr int RING = LPI == 2 && XC == 6 ? 3 : ITEMS % 2 == 0 ? 2 : (ITEMS < 3 ? ITEMS : 3);
     // ... of which this many are asked for before the rows of X are in LDS
     constexpr int FIRST = PAIRS || XC > 2 ? RING : 1;
     static_assert(ITEMS % RING == 0, "the ring must go round a whole number of times per group");
@@ -759,7 +760,7 @@ static void gd_launch_rows_long_k(int tiles, unsigned grid, DecodeGemmArgs& a, h
 }
 #undef GR_GO
 
-// 9 to 16 rows whose K does not fit LDS: four or six chunks a wave.  LPI = 2: tiles of 8 weight rows, for a share whose last tile of 16
+// 9 to 16 rows whose K does not fit LDS: four, five or six chunks a wave.  LPI = 2: tiles of 8 weight rows, for a share whose last tile of 16
 // would be half empty (two load instructions less per chunk).
 template <typename TOut, int EPI, bool NORM, int LPI>
 static void gd_launch_rows_one_block(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
@@ -771,6 +772,8 @@ static void gd_launch_rows_one_block(int chunks, int tiles, unsigned grid, Decod
     if (chunks <= 4 * GR_NW) {
         if (tiles == 1) GR_GO16(4, 1);
         else GR_GO16(4, 2);
+    } else if (chunks <= 5 * GR_NW && tiles > 1) {
+        GR_GO16(5, 2);
     } else {
         if (tiles == 1) GR_GO16(6, 1);
         else GR_GO16(6, 2);
@@ -831,9 +834,19 @@ static int gd_launch(int chunks, int tiles, unsigned grid, unsigned lds_bytes, D
         else if (nt == 2) GD_GO(2, 2);
         else if (nt == 3) GD_GO(2, 3);
         else GD_GO(2, 4);
+    }
+    // An item beyond K is a place in the ring with nothing in flight: with 18 chunks of four places a wave half of them are, and 256000 x 2304
+    // at 1 row took 196 microseconds (169 with 16 waves), 171 with three; 6144 x 2304 8.1 and 7.0; gate and up of 5120 x 5120 with
+    // the norm 12.5 and 11.9 with five for six.  Three and five items go round a ring of two in groups of two tiles, so few odd
+    // tiles stay as they are; of three items, all asked for in front of the norm, 3840 x 2560 took 6.7 for 6.4.
+    else if (chunks <= 3 * GD_NW && (tiles % 2 == 0 || tiles > 3 || !a.norm_weight)) {
+        if (tiles % 2 && tiles <= 3) GD_GO(3, 1);
+        else GD_GO(3, 2);
     } else if (chunks <= 4 * GD_NW) {
         if (tiles % 2) GD_GO(4, 1);
         else GD_GO(4, 2);
+    } else if (chunks <= 5 * GD_NW && (tiles % 2 == 0 || tiles > 5)) {
+        GD_GO(5, 2);
     } else {
         GD_GO(6, 1);
     }

@@ -484,12 +484,12 @@ def test_gemm_decode_plain(m, n, k):
     assert torch.equal(ops().gemm_decode(torch.empty(m, n, dtype=torch.bfloat16, device=DEV), wide[:, :k], w.to(DEV)), out)
 
 
-@pytest.mark.parametrize("k", [1024, 1032, 2040, 2056, 3072, 3968, 3976, 4096, 4104, 5120, 5128, 6144])
+@pytest.mark.parametrize("k", [1024, 1032, 2040, 2056, 2304, 3072, 3968, 3976, 4096, 4104, 5120, 5128, 6144])
 @pytest.mark.parametrize("m", [1, 8, 9, 16])
 def test_gemm_decode_chunks_of_k(m, k):
-    """One, two, four and six chunks a wave, the last ones empty, half empty or full; rows in LDS and in registers; one tile, several and
-    several groups of them."""
-    for n in (40, 4104, 20000):
+    """One to six chunks a wave, the last ones empty, half empty or full; rows in LDS and in registers; one tile, several (odd and even
+    numbers of them) and several groups of them."""
+    for n in (40, 4104, 8192, 20000, 28000):
         x, w, b = rnd(m, k, seed=11).bfloat16(), rnd(n, k, seed=12).bfloat16(), rnd(n, seed=13).bfloat16()
         got = ops().gemm_decode(torch.empty(m, n, device=DEV), x.to(DEV), w.to(DEV), b.to(DEV))
         ref = x.to(DEV).double() @ w.to(DEV).double().t() + b.to(DEV).double()
