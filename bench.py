@@ -528,6 +528,8 @@ def gemv(args) -> int:
                     how = "partial sums" if lin.linear_partial_sums(x, weights[0]) is not None else how
             else:
                 run = lambda w: lin.linear(x, w, out_dtype=torch.float32)  # noqa: E731
+                if decode and lin.streams_large(m, n, k, ops.compute_units(dev)):
+                    how = "gemm_stream"
             if norm is not None and name in ("qkv", "gate_up"):
                 how += " + norm"
             for w in weights[:2]:

@@ -42,6 +42,33 @@ STREAM_MAX_ROWS = 64
 STREAM_REREAD_BYTES = 64e6
 
 
+# A plain product of up to 8 rows against a weight this large (the vocabulary's): ops.gemm_decode shares it out to the compute units in
+# one stretch each and streams it faster than ops.gemm_stream's thousands of small workgroups where all its waves have whole chunks of K
+# (two, three, four or six of 128 columns each) or beyond 4 rows.  Microseconds, gemm_decode and gemm_stream: 32000 x 2048 22.1 and 24.2 at 1
+# row, 22.5 and 26.2 at 8; 128256 x 2048 78 and 82, 82 and 90; 32000 x 4096 41.4 and 43.4, 42.5 and 46.9; 32064 x 3072 31.0 and 31.9; 100352 x
+# 6144 188 and 189, 190 and 206.  Otherwise 50304 x 1024 19.8 and 18.2 at 1 row, 50264 x 1600 28.5 and 26.3, 262144 x 1152 94 and 85, 151936 x
+# 896 42.1 and 40.1, 64000 x 2560 50.4 and 49.1, but at 8 rows 20.2 and 19.9, 29.0 and 29.6, 101 and 105, 44.8 and 45.5, 52.3 and 56.6.
+STREAM_LARGE_ROWS = 8
+STREAM_LARGE_BYTES = 100e6
+STREAM_LARGE_ODD_ROWS = 4
+
+
+def streams_large(m: int, n: int, k: int, cus: int = 256) -> bool:
+    """Whether a plain product of `m` rows against a large weight [n, k] that ops.gemm_decode takes is faster by ops.gemm_stream."""
+    if m > STREAM_LARGE_ROWS or 2 * n * k < STREAM_LARGE_BYTES:
+        return False
+    return (m <= STREAM_LARGE_ODD_ROWS and k not in (2048, 3072, 4096, 6144)) or _shares_meet(n, k, cus)
+
+
+def _shares_meet(n: int, k: int, cus: int) -> bool:
+    """Whether the compute units' stretches of a weight [n, k] start on the same channels of memory.  Starts 127 or 129 times a
+    power of two apart are slow, their neighbours are not, whatever that power: as if fields of 7 bits of an address, added without carry,
+    chose the channel, where such starts cancel out and all units walk the weight side by side on few channels.  TB/s of gemm_decode at 1 row, K = 4096, by rows a compute unit:
+    126 6.4, 127 5.2, 128 6.4; 253 6.6, 254 5.5, 255 6.6, 257 6.6, 258 5.7, 260 6.6 (gemm_stream 5.9 and 6.3 to 6.4)."""
+    apart = n // cus * k
+    return n % cus == 0 and apart > 0 and ((apart & -apart) * 127 == apart or (apart & -apart) * 129 == apart)
+
+
 DECODE_KERNEL = os.environ.get("LLMSERVE_DECODE_GEMM", "1") != "0"
 
 
@@ -214,7 +241,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     if m == 0:
         return out
     if x.dtype == torch.bfloat16 and ops.gemm_bf16_supported(x, weight):
-        if decode_product(x, weight):
+        if decode_product(x, weight) and not streams_large(m, n, weight.shape[1], ops.compute_units(x.device)):
             return ops.gemm_decode(out, x, weight, bias)
         if few_rows(m, weight):
             return ops.gemm_stream(out, x, weight, bias)

@@ -103,3 +103,24 @@ def test_weights_of_2_gb_and_more_do_not_go_to_the_decode_kernel(n, k):
     assert linear.few_rows(16, bf16(n, k))
     assert not library.gemm_decode_reaches(bf16(40, 2048), bf16(1 << 19, 2048)) and library.gemm_decode_reaches(bf16(40, 2048), bf16((1 << 19) - 1, 2048))
     assert not library.gemm_decode_supported(bf16(4, 1 << 28)[:, :4096], bf16(64, 4096))
+
+
+@pytest.mark.parametrize("m,n,k,decode,stream", [  # microseconds
+    (1, 32000, 2048, 22.1, 24.2), (8, 32000, 2048, 22.5, 26.2), (1, 32000, 4096, 41.4, 43.4), (4, 128256, 2048, 79.7, 84.1),
+    (1, 32064, 3072, 31.0, 31.9), (8, 100352, 6144, 190, 206), (8, 51200, 2560, 42.5, 46.0), (8, 256000, 2304, 185, 197),
+    (8, 262144, 1152, 101, 105), (8, 151936, 896, 44.8, 45.5), (1, 50304, 1024, 19.8, 18.2), (4, 50264, 1600, 28.7, 27.2),
+    (1, 262144, 1152, 94, 85), (1, 151936, 896, 42.1, 40.1), (1, 64000, 2560, 50.4, 49.1), (1, 256000, 2304, 171, 167),
+    (1, 65024, 4096, 94, 83), (8, 65024, 4096, 97, 88), (1, 32512, 4096, 51, 44.5), (8, 32512, 2048, 31, 26.7), (1, 66048, 2048, 51, 48),
+    (1, 65536, 4096, 79.7, 80.8), (1, 64768, 4096, 80.5, 83.3)])
+def test_the_vocabularys_product_of_few_rows(m, n, k, decode, stream):
+    """One stretch of the weight for each compute unit, or small workgroups: the faster one."""
+    from llmserve.parts.linear import streams_large
+
+    assert streams_large(m, n, k) == (stream < decode)
+
+
+def test_smaller_weights_and_more_rows_do_not_go_to_the_streaming_kernel():
+    from llmserve.parts.linear import streams_large
+
+    assert not streams_large(9, 65024, 4096) and not streams_large(1, 8128, 4096) and not streams_large(1, 11264, 2048)
+    assert not streams_large(1, 49152, 576)  # 57 MB
