@@ -635,7 +635,11 @@ SLICE_K = 512  # what one workgroup of gemm_slices takes of K
 # almost none, what comes to that with one on every compute unit; and the waves that only load.  Fitted to 9,700 products (17 weights of 1024
 # x 2048 to 22016 x 4096, 65 to 2,048 rows, up to 4 parts of K; weights from memory and, for what goes to a norm, from the memory-side
 # cache too).  The plan below is 0.7 % off the best tile in the mean over them and 13 % at most (900 rows against 1024 x 2048: 9.8
-# microseconds and 8.7).
+# microseconds and 8.7).  Beyond 2,048 rows, which the fit does not cover, tiles of more than one round take longer than that, the more the
+# fewer weight rows they have, since the rows of x no longer stay in L2 from one round to the next: 24 % in the mean with 64 weight rows, 13
+# with 96, 9 with 128, 3 with 192 and more (37 weights at 2,500, 3,000 and 4,096 rows).  With that counted in the plan is 0.8, 0.6 and 0.3 % off the best
+# tile for them, plain, gated and rotated, where it was 1.2, 1.2 and 1.3 (3072 x 1024 at 4,096 rows 34.8 microseconds -> 30.1, gate and up of 9728 x
+# 896 at 3,000 64.1 -> 59.6, 3072 x 2048 rotated at 4,096 67.1 -> 60.5).
 GEMM_TILES = ((64, 64, 2, 4, 0.098, 0.484, 0.198, 0.079, 0), (96, 64, 2, 4, 0.305, 0.587, 0.229, 0.093, 0),
               (128, 64, 1, 4, 0.837, 0.409, 0.260, 0.137, 0), (96, 128, 1, 4, 1.070, 0.468, 0.327, 0.126, 4),
               (128, 128, 1, 4, 1.725, 0.540, 0.405, 0.133, 4), (160, 192, 1, 3, 2.825, 0.822, 0.626, 0.190, 4),
@@ -676,6 +680,8 @@ def gemm_tiles_plan(m: int, n: int, k: int, most_parts: int = 1, cus: int = 256,
                 continue
             _, rounds, last = _gemm_tiles_rounds(tile, m, n, k, parts, cus)
             cost = (rounds + last) * (GEMM_TILES_FROM_CACHE if near and not GEMM_TILES[tile][-1] else 1.0)
+            if m > 2048 and rounds > 0:
+                cost *= 1.0 + max(0.0, 20.0 / GEMM_TILES[tile][1] - 0.07)
             if parts > 1:
                 cost += m * n * ((6 * parts - 4) / 5.0e6 + parts / 2.0e6)
             if best is None or cost < best[0]:

@@ -124,3 +124,14 @@ def test_smaller_weights_and_more_rows_do_not_go_to_the_streaming_kernel():
 
     assert not streams_large(9, 65024, 4096) and not streams_large(1, 8128, 4096) and not streams_large(1, 11264, 2048)
     assert not streams_large(1, 49152, 576)  # 57 MB
+
+
+@pytest.mark.parametrize("m,n,k,micros", [  # microseconds by tile (those of the best third)
+    (4096, 3072, 1024, {5: 34.5, 7: 37.5, 8: 37.4, 10: 37.0, 11: 30.1, 16: 34.8}), (4096, 3072, 2048, {5: 69.5, 7: 76.0, 11: 60.5, 16: 67.1}),
+    (4096, 14336, 3072, {5: 347, 7: 341, 8: 315, 10: 338, 11: 319}), (3000, 9728, 896, {5: 67.2, 7: 64.1, 8: 66.2, 11: 59.6}),
+    (2500, 5120, 3072, {5: 100, 8: 99, 11: 82.5}), (2500, 3072, 2048, {5: 37.7, 7: 45.1, 8: 39.3, 10: 41.5})])
+def test_the_tile_beyond_2048_rows(m, n, k, micros):
+    """Rows of x do not stay in L2 from one round of tiles to the next: tiles of few weight rows read them more often."""
+    from llmserve.ops.library import gemm_tiles_plan
+
+    assert micros[gemm_tiles_plan(m, n, k)[0]] <= 1.05 * min(micros.values())
