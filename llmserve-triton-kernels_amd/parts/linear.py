@@ -105,10 +105,10 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 #           398 and 374 at 2,048
 #   rotary  2560 x 2048 11 and 19 at 512 rows; 12288 x 4096 60 and 62 at 512, 104 and 92 at 1,024
 #   parts   4096 x 11008 51 and 73 at 512 rows; 8192 x 28672 151 and 306 at 200, 430 and 263 at 640 (without the norm)
-# The gated line was drawn when such products took 10 to 30 % longer in tiles.  Against a weight below TILES_GATED_SMALL they are the tiles'
-# but in TILES_GATED_BAND, where only the measurements of then stand against it (11264 x 2048: 36 and 47 at 768 rows, 52 and 56 at 1,024,
-# 66 and 75 at 1,300, 78 and 99 at 1,629, 88 and 95 at 2,048); 22016 x 4096 and larger weights are still the library's at few rows (95 and
-# 89 at 512 rows).
+# The gated line was drawn when such products took 10 to 30 % longer in tiles.  Against a weight below TILES_GATED_SMALL they are the tiles',
+# whatever the rows: 8 such weights of 5632 x 1024 to 14336 x 3072 at 72 to 4,096 rows, 192 products, 0.78 in the mean, 1.08 at most (14336 x 3072 at
+# 2,500); 11264 x 2048: 36 and 49 at 768 rows, 53 and 58 at 1,024, 66 and 75 at 1,300, 68 and 81 at 1,536, 90 and 99 at 2,048; 17920 x 1536 71
+# and 83 at 1,300; 16384 x 2048 85 and 94.  22016 x 4096 and larger weights are the library's at some sizes still (1.06 at 512 rows).
 # Gated products of TILES_GATED_WORK and more against a weight below TILES_GATED_WEIGHT (200 MB, which the 256 MB memory-side cache
 # holds) are the tiles' again: 27 such products of 17 weights 0.95 in the mean, 0.72 to 1.19, where larger weights are at 1.05; 22016 x
 # 4096 at 2,048 rows 299 and 425 (the means, too, from before).
@@ -120,13 +120,13 @@ def few_rows(m: int, weight: torch.Tensor) -> bool:
 # 1,629 rows, 4096 x 4096 54 and 58 at 2,048, 4096 x 11008 145 and 164 at 2,048, 8192 x 8192 96 and 103 at 768), and 40 gated ones, 0.87,
 # 0.70 to 0.96 (22016 x 4096 64 and 78 at 330, 12288 x 4096 60 and 67 at 610).  Of columns beyond TILES_ROUND_K and of tiles of 256 x
 # 256 (one wave to a SIMD) too many were slower: 2048 x 16384 151 and 141 at 2,048, 6144 x 2048 53 and 48 at 2,500.  Rotations and parts gain
-# what they spare behind the product on top (parts: the plan says whether K comes in any).
+# what they spare behind the product on top: 15360 x 5120 rotated at 512 and 528 rows 0.85 and 0.88, and 9 products that go to a norm, in the parts
+# of K that their plan has, 0.90, at most 0.95 (8192 x 8192 at 1,024 rows 0.93, 3072 x 8192 at 3,000 0.91).
 TILES_WORK = {"plain": 18e9, "gated": 18e9, "rotary": 40e9, "parts": 60e9}
 TILES_GATED_WORK = 130e9
 TILES_GATED_WEIGHT = 100e6
 TILES_LONG_K = 4096
 TILES_GATED_SMALL = 50e6
-TILES_GATED_BAND = (29e9, 36e9)
 TILES_ROUND_K = 12288
 
 
@@ -135,7 +135,7 @@ def tiles_pay(kind: str, m: int, n: int, k: int, cus: int = 256) -> bool:
     epilogue, "parts": K in parts for a norm to add up) than by the library: a rule by sizes alone."""
     work = m * n * k
     if kind == "gated" and n * k < TILES_GATED_WEIGHT:
-        if work >= TILES_GATED_WORK or n * k < TILES_GATED_SMALL and not TILES_GATED_BAND[0] <= work < TILES_GATED_BAND[1]:
+        if work >= TILES_GATED_WORK or n * k < TILES_GATED_SMALL:
             return True
     if m > 64:
         rows, weight_rows = ops.GEMM_TILES[ops.gemm_tiles_plan(m, n, k, 1, cus)[0]][:2]

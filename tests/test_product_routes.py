@@ -8,7 +8,9 @@ from llmserve.parts.linear import TILES_WORK, tiles_pay
 # tiles' gated products take 5 to 20 % less since)
 MEASURED = [
     ("gated", 333, 11264, 2048, 34, 36), ("gated", 512, 11264, 2048, 36, 38), ("gated", 768, 11264, 2048, 45, 48),
-    ("gated", 1300, 11264, 2048, 86, 73), ("gated", 1536, 11264, 2048, 88, 80),
+    ("gated", 1300, 11264, 2048, 66, 75), ("gated", 1536, 11264, 2048, 68, 81),  # (as they are now; 86 and 73, 88 and 80 then)
+    ("gated", 1258, 11264, 2048, 57, 62), ("gated", 1560, 11264, 2048, 77, 95), ("gated", 1300, 17920, 1536, 71, 83),
+    ("gated", 1200, 17920, 1536, 70, 80), ("gated", 1300, 16384, 2048, 85, 94), ("gated", 700, 14336, 3072, 67, 72),
     ("gated", 400, 22016, 4096, 103, 85), ("gated", 512, 22016, 4096, 107, 88), ("gated", 896, 22016, 4096, 160, 153),
     ("gated", 1024, 22016, 4096, 188, 162), ("gated", 1100, 22016, 4096, 212, 179), ("gated", 1536, 22016, 4096, 253, 312),
     ("gated", 2048, 22016, 4096, 314, 424), ("gated", 400, 57344, 8192, 424, 360), ("gated", 512, 57344, 8192, 430, 376),
