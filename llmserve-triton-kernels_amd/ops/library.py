@@ -725,6 +725,12 @@ def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: in
     return min(idle, -(-nbytes // int(0.8 * GEMM_TILES_WORKER_RATE * last)))
 
 
+def gemm_tiles_brings(m: int, n: int, k: int, near: torch.Tensor, cus: int = 256, tile: int | None = None) -> tuple[int, int]:
+    """(workers, bytes) with which ops.gemm_tiles, given m rows against a weight [n, k], brings `near` into the memory-side cache."""
+    nbytes = _near_bytes(near)
+    return gemm_tiles_workers(gemm_tiles_plan(m, n, k, 1, cus)[0] if tile is None else tile, m, n, k, 1, nbytes, cus), nbytes
+
+
 def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ops.gemm_tiles takes x [M, K] against w [N, K]: K in steps of 64, blocks of 16 weight rows, rows of x of 16-byte pieces
     that do not overlap, a contiguous w, and neither without columns or rows."""
@@ -807,8 +813,7 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
     if near is not None:
         if epilogue not in (2, 3):
             raise ValueError("near goes with the gated and the rotary epilogue")
-        near_bytes = _near_bytes(near)
-        workers = gemm_tiles_workers(tile, m, n, k, parts, near_bytes, compute_units(dev))
+        workers, near_bytes = gemm_tiles_brings(m, n, k, near, compute_units(dev), tile)
     _check(load("gemm_tiles").llms_gemm_tiles(
         c_int(tile), c_int(epilogue), _ptr(out), _ptr(x), _ptr(w), _ptr(bias), c_int(m), c_int(n), c_int(k), c_int(x.stride(0)),
         c_int(out.stride(-2)), c_int(parts), ctypes.c_longlong(part_stride), c_int(_gated_unit(limit, gelu)),

@@ -160,8 +160,7 @@ def tiles_product(x: torch.Tensor, weight: torch.Tensor, kind: str = "plain") ->
 def brings_near(x: torch.Tensor, weight: torch.Tensor, near: torch.Tensor) -> bool:
     """Whether ops.gemm_tiles, given x against weight with `near` behind it, has compute units left that bring `near` into the
     memory-side cache: what the product of `near` is told (`from_cache`)."""
-    m, (n, k), cus = x.shape[0], weight.shape, ops.compute_units(x.device)
-    return ops.gemm_tiles_workers(ops.gemm_tiles_plan(m, n, k, 1, cus)[0], m, n, k, 1, near.numel() * near.element_size(), cus) > 0
+    return ops.gemm_tiles_brings(x.shape[0], *weight.shape, near, ops.compute_units(x.device))[0] > 0
 
 
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and
