@@ -877,7 +877,8 @@ def _arrival_counters(dev) -> torch.Tensor | None:
     if key not in _ARRIVAL_COUNTERS:
         if torch.cuda.is_current_stream_capturing():
             return None
-        _ARRIVAL_COUNTERS[key] = torch.zeros(ARRIVAL_COUNTERS, dtype=torch.int32, device=dev)
+        with torch.inference_mode(False):  # (steps run in inference mode, and are not the only ones that write here)
+            _ARRIVAL_COUNTERS[key] = torch.zeros(ARRIVAL_COUNTERS, dtype=torch.int32, device=dev)
     return _ARRIVAL_COUNTERS[key]
 
 

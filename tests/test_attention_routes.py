@@ -1,5 +1,6 @@
 """Which launches a step's attention becomes: rules by sizes alone (no GPU)."""
 import pytest
+import torch
 
 
 def step_in_one(nh, nkv, d, n_decode, n_portions, max_new, window=0, splits=1, waves=8, counters=1 << 14, prompt_splits=1):
@@ -55,3 +56,17 @@ def test_the_kernel_shares_keys_out_from_the_line_of_the_rule():
     for d, tiles in ((16, 3), (64, 3), (80, 3), (96, 3), (112, 2), (128, 2)):
         assert decode_arrangement(8, 2, d, None, 2, 32 * 8 * tiles) == (1, 8)
         assert decode_arrangement(8, 2, d, None, 2, 32 * 8 * tiles + 1) == (4, 8)
+
+
+def test_counters_made_inside_a_step_can_be_zeroed_outside_one(monkeypatch):
+    """A step runs in inference mode, and the first one whose attention shares keys out makes the counters; a runner that is built later
+    zeroes them, outside."""
+    from llmserve.ops import library
+
+    monkeypatch.setattr(library, "_ARRIVAL_COUNTERS", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    with torch.inference_mode():
+        counters = library._arrival_counters(torch.device("cpu"))
+        counters[3] = 7
+    library.reset_arrival_counters()
+    assert library.arrival_counters_are_zero() and int(counters.sum()) == 0
