@@ -513,14 +513,14 @@ def gemm_decode_k_parts(m: int, k: int) -> int:
 
 
 def gemm_decode_reaches(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ops.gemm_decode's 32-bit offsets reach all of x and w: less than 2 GB each."""
-    return w.numel() < 1 << 30 and x.shape[0] * x.stride(0) < 1 << 30
+    """Whether ops.gemm_decode's 32-bit offsets reach all of x [M, K] and w [N, K]: less than 2 GB each."""
+    m, k = x.shape
+    return w.shape[0] * k < 1 << 30 and m * x.stride(0) < 1 << 30
 
 
 def gemm_decode_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ops.gemm_decode takes x [M, K] against w [N, K]."""
-    return (x.dtype == torch.bfloat16 and gemm_decode_fits(x.shape[0], x.shape[1]) and gemm_bf16_supported(x, w)
-            and gemm_decode_reaches(x, w))
+    return x.dtype == torch.bfloat16 and gemm_decode_fits(*x.shape) and gemm_bf16_supported(x, w) and gemm_decode_reaches(x, w)
 
 
 def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
@@ -704,7 +704,8 @@ GEMM_TILES_NEAR_RATE = 2.9e6
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: int, cus: int = 256) -> int:
+@functools.lru_cache(maxsize=4096)
+def gemm_tiles_workers(tile: int | None, m: int, n: int, k: int, parts: int, nbytes: int, cus: int = 256) -> int:
     """How many workgroups beyond those of the tiles bring a weight of `nbytes` nearer: as many as do so in four fifths of a round's
     time, if there are as many compute units without a tile in the last round and memory has time for both weights; otherwise none.
     Time saved in both products together, microseconds: gate and up with down_proj behind them (1.1B shape, 23 MB) 4.5 at 512 rows, 6.0
@@ -714,9 +715,11 @@ def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: in
     one gets in the way of the tiles' own (down_proj of the 7B shape, 90 MB: -10.7 at 330 rows, -4.6 at 448), and so does any where the
     tiles themselves wait for memory (gate and up at 333 rows take 2.2 more, down_proj 2.2 less).  With more workers than there are
     such compute units each would take a tile's place or be a round of its own.  A rule by sizes alone: it takes the compute units
-    without a tile to be idle, and where another stream's kernel is on them the two share them."""
+    without a tile to be idle, and where another stream's kernel is on them the two share them.  (Without a `tile`: the plan's.)"""
     if not 0 < nbytes <= GEMM_TILES_NEAR_BYTES:
         return 0
+    if tile is None:
+        tile = gemm_tiles_plan(m, n, k, 1, cus)[0]
     rest, rounds, last = _gemm_tiles_rounds(tile, m, n, k, parts, cus)
     last += 2.5  # (before the first step and behind the last)
     idle = cus - rest if 0 < rest < cus else 0
@@ -728,7 +731,7 @@ def gemm_tiles_workers(tile: int, m: int, n: int, k: int, parts: int, nbytes: in
 def gemm_tiles_brings(m: int, n: int, k: int, near: torch.Tensor, cus: int = 256, tile: int | None = None) -> tuple[int, int]:
     """(workers, bytes) with which ops.gemm_tiles, given m rows against a weight [n, k], brings `near` into the memory-side cache."""
     nbytes = _near_bytes(near)
-    return gemm_tiles_workers(gemm_tiles_plan(m, n, k, 1, cus)[0] if tile is None else tile, m, n, k, 1, nbytes, cus), nbytes
+    return gemm_tiles_workers(tile, m, n, k, 1, nbytes, cus), nbytes
 
 
 def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -741,7 +744,7 @@ def gemm_tiles_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *, swiglu: bool = False,
                rope: dict | None = None, limit: float | None = None, gelu: bool = False, tile: int | None = None,
-               near: torch.Tensor | None = None, from_cache: bool = False) -> torch.Tensor:
+               near: torch.Tensor | None = None, brings: tuple[int, int] | None = None, from_cache: bool = False) -> torch.Tensor:
     """The product of many bfloat16 rows, and what follows it fused in.
 
     plain:   out[M, N] = x w^T (+ bias), bfloat16 or float32; float32 [parts, M, N]: the sums of that many parts of K.
@@ -752,6 +755,7 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
     `tile`: a place in GEMM_TILES; default by gemm_tiles_plan.
     `near` (with swiglu or rope): a contiguous weight that a kernel after this one reads: compute units without a tile bring it into the memory-side
             cache meanwhile, where that pays (gemm_tiles_workers).  No result depends on it.
+    `brings`: what gemm_tiles_brings says of `near`, for a caller who has asked (the tile is the plan's then).
     `from_cache`: w is such a weight, which the product in front brought there (another tile may then be the best)."""
     dev = _dev(out, x, w, bias, near)
     if x.dim() != 2 or x.stride(1) != 1 or out.dim() not in (2, 3) or out.stride(-1) != 1:
@@ -806,14 +810,14 @@ def gemm_tiles(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.
         raise ValueError(f"out shape {tuple(out.shape)} does not end in {(m, cols)}")
     if m == 0:
         return out
+    cus = compute_units(dev)
     if tile is None:
-        cus = compute_units(dev)
         tile = gemm_tiles_plan(m, n, k, 1, cus, from_cache)[0] if parts == 1 else _tile_for_parts(m, n, k, parts, cus, from_cache)
     workers = near_bytes = 0
     if near is not None:
         if epilogue not in (2, 3):
             raise ValueError("near goes with the gated and the rotary epilogue")
-        workers, near_bytes = gemm_tiles_brings(m, n, k, near, compute_units(dev), tile)
+        workers, near_bytes = gemm_tiles_brings(m, n, k, near, cus, tile) if brings is None else brings
     _check(load("gemm_tiles").llms_gemm_tiles(
         c_int(tile), c_int(epilogue), _ptr(out), _ptr(x), _ptr(w), _ptr(bias), c_int(m), c_int(n), c_int(k), c_int(x.stride(0)),
         c_int(out.stride(-2)), c_int(parts), ctypes.c_longlong(part_stride), c_int(_gated_unit(limit, gelu)),

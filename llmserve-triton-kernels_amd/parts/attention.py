@@ -74,9 +74,7 @@ class Attention(Mixer):
         view = batch.groups[cache.group_id]
         slots = view.slots if cache.store else None
         deferred = x if isinstance(x, DeferredNorm) else None  # (then the result goes to a norm, which takes partial sums)
-        q = self.project_and_store(x, batch, cache, slots)
-        rows = deferred.residual if deferred is not None else x
-        near = q is not None and self._in_tiles(rows) and brings_near(rows, self.qkv_weight, self.o_weight)
+        q, near = self.project_and_store(x, batch, cache, slots)
         if q is None:
             if deferred is not None:
                 x = deferred.materialize()
@@ -101,25 +99,21 @@ class Attention(Mixer):
             return True
         return not (decode_product(rows, self.qkv_weight) or few_rows(rows.shape[0], self.qkv_weight) or self._fits_tiles(rows))
 
-    def _in_tiles(self, rows) -> bool:
-        """Of rows that project_and_store takes."""
-        return not decode_product(rows, self.qkv_weight) and not few_rows(rows.shape[0], self.qkv_weight)
-
     def _fits_tiles(self, rows) -> bool:
         return self.head_dim % 32 == 0 and tiles_product(rows, self.qkv_weight, "rotary")
 
     def project_and_store(self, x, batch, cache, slots):
         """With bfloat16 rows one kernel does the projection, the rotation and the cache store
         (ops.gemm_decode, which also norms its rows on the way in, ops.gemm_stream or ops.gemm_tiles).  Returns the rotated
-        queries, or None when none of them applies."""
+        queries, or None when none of them applies, and whether it brought o_proj's weight into the memory-side cache."""
         deferred = isinstance(x, DeferredNorm)
         rows = x.residual if deferred else x
         m = rows.shape[0]
         if self._few_rows_unfit(rows):
-            return None
+            return None, False
         frequencies = getattr(self.position, "rotary_frequencies", None)
         if frequencies is None and not getattr(self.position, "identity", False):
-            return None  # a position encoding this kernel does not know
+            return None, False  # a position encoding this kernel does not know
         decode = decode_product(rows, self.qkv_weight)
         norm = x.fused() if deferred and decode and m <= ops.GEMM_DECODE_NORM_ROWS else None
         if norm is not None:
@@ -130,18 +124,19 @@ class Attention(Mixer):
                     inv_freq=frequencies() if frequencies is not None else None, positions=batch.positions,
                     slots=slots, k_pool=cache.k_pool, v_pool=cache.v_pool, block_size=cache.block_size)
         q = torch.empty((m, self.num_heads * self.head_dim), dtype=rows.dtype, device=rows.device)
-        tiles = self._in_tiles(rows)
+        tiles, brings = not decode and not few_rows(m, self.qkv_weight), (0, 0)
         if decode or tiles:
             angles = getattr(self.position, "rotary_angles", None)
             if angles is not None and getattr(batch, "shared", None) is not None:
                 rope["angles"] = angles(batch)  # worked out once per step, not once per layer and workgroup
             if tiles:
-                ops.gemm_tiles(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, near=self.o_weight)
+                brings = brings_near(rows, self.qkv_weight, self.o_weight)
+                ops.gemm_tiles(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, near=self.o_weight, brings=brings)
             else:
                 ops.gemm_decode(q, rows, self.qkv_weight, self.qkv_bias, rope=rope, norm=norm)
         else:
             ops.gemm_stream(q, rows, self.qkv_weight, self.qkv_bias, rope=rope)
-        return q
+        return q, brings[0] > 0
 
     def attend(self, out, qkv, cache, view, batch):
         """out[n] = attention of token n's query heads (the first nh*D columns of qkv) over its

@@ -157,10 +157,11 @@ def tiles_product(x: torch.Tensor, weight: torch.Tensor, kind: str = "plain") ->
     return tiles_fit(x, weight) and (OWN_KERNELS_ONLY or tiles_pay(kind, x.shape[0], *weight.shape, ops.compute_units(x.device)))
 
 
-def brings_near(x: torch.Tensor, weight: torch.Tensor, near: torch.Tensor) -> bool:
-    """Whether ops.gemm_tiles, given x against weight with `near` behind it, has compute units left that bring `near` into the
-    memory-side cache: what the product of `near` is told (`from_cache`)."""
-    return ops.gemm_tiles_brings(x.shape[0], *weight.shape, near, ops.compute_units(x.device))[0] > 0
+def brings_near(x: torch.Tensor, weight: torch.Tensor, near: torch.Tensor) -> tuple[int, int]:
+    """With how many compute units ops.gemm_tiles, given x against weight with `near` behind it, brings `near` into the memory-side cache,
+    and how many bytes: what it is told (`brings`), and where there are any the product of `near` is (`from_cache`)."""
+    n, k = weight.shape
+    return ops.gemm_tiles_brings(x.shape[0], n, k, near, ops.compute_units(x.device))
 
 
 # A short, wide weight gives the streaming kernel fewer tiles than the chip has CUs (TinyLlama's o_proj and

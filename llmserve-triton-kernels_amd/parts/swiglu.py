@@ -69,8 +69,9 @@ class SwiGLU(FeedForward):
             if few and ops.gemm_bf16_supported(rows, self.gate_up):
                 ops.gemm_stream(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu)  # activation in the product's epilogue
             elif not few and self.intermediate % 16 == 0 and tiles_product(rows, self.gate_up, "gated"):
-                ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu, near=self.down)  # the same
-                near = brings_near(rows, self.gate_up, self.down)
+                brings = brings_near(rows, self.gate_up, self.down)
+                ops.gemm_tiles(act, rows, self.gate_up, swiglu=True, limit=self.limit, gelu=self.gelu, near=self.down, brings=brings)  # the same
+                near = brings[0] > 0
             elif self.unit == "silu" and ops.gemm32_gated_supported(rows, self.gate_up):
                 ops.gemm32_gated(act, rows, self.gate_up)  # the same, in 32-bit
             else:
