@@ -28,7 +28,8 @@
 // each a layer's four products of the 1.1B shape took 25.3 microseconds at 1 row and 26.9 at 8, of the 7B shape (without down_proj) 66.0
 // and 68.2; with 8 waves and six or four items 24.6, 26.2, 63.1 and 65.6 (half the waves start and meet), with two items 23.8, 25.2, 58.0
 // and 60.7, with one 25.9, 27.6, 61.4 and 64.1: memory answers a compute unit some 40 KB at a time, and what all compute units ask for
-// beyond that comes from more open rows of memory at once.  The vocabulary's product, 32000 x 2048: 29.2 -> 22.8 (5.8 TB/s).
+// beyond that comes from more open rows of memory at once.  That the sums still have no more terms than 16 waves' (gd_sums) takes 0.2 to
+// 0.9 of them back: 24.5, 25.9, 58.2 and 61.3.  The vocabulary's product, 32000 x 2048: 29.2 -> 23.1 (5.7 TB/s).
 //
 // Epilogues (the waves' partial sums meet in LDS in the order of the waves):
 //   PLAIN     C = sums (+ bias), float32 or bfloat16; `unit` 2: max(sums, 0)^2.
@@ -51,10 +52,23 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 #define GD_KC 128    // elements of K per item
 #define GD_MAX_XC 6  // chunks of K per wave
 #define GD_MAX_K (GD_NW * GD_MAX_XC * GD_KC)
+// Sums of a wave with `xc` chunks: one of every other chunk, so that a sum has no more terms than 16 waves' and the sums are added up in
+// their order (chunks c, c + 16, ... are a sum; sum 0 first).  With one sum a wave 5632 columns were 24 % further from 64 bits
+// (1.62e-7 for 1.31e-7), 4096 19 %, 2048 5 %.  (17 to 64 rows: one sum of a wave's up to four chunks.)
+constexpr int gd_sums(int xc) { return xc > 1 ? 2 : 1; }
+// Where a lane's 4 sums (rows 4 g .. of the tile for row m of X, lane 16 g + m) lie among those of 64 lanes: turned by 8 or 4 places a g, so that
+// the 64 places a wave reads (8 rows of the tile for 8 of X, or 16 for 4) are in different banks; in the order of the lanes they were 2
+// or 4 to a bank.
+template <int UPT>
+__device__ __forceinline__ int gd_place(int g, int m) { return 16 * g + ((m + (UPT == 8 ? 8 : 4) * g) & 15); }
+
 // LDS: the waves' tiles (later their partial sums), the rows' sums of squares, then the rows of X
-#define GD_LDS_TILES (GD_NW * 16 * (GD_KC / 8) * 16)
-#define GD_LDS_SQ (16 * GD_NW * 4)
-#define GD_LDS_X_MAX (160 * 1024 - GD_LDS_TILES - GD_LDS_SQ)
+constexpr int gd_lds_tiles(int xc, int nt) {
+    const int tiles = GD_NW * 16 * (GD_KC / 8) * 16, sums = nt * gd_sums(xc) * GD_NW * LLMS_WAVE * 16;
+    return tiles > sums ? tiles : sums;
+}
+#define GD_LDS_SQ (16 * 2 * GD_NW * 4)
+#define GD_LDS_X_MAX (160 * 1024 - gd_lds_tiles(3, 2) - GD_LDS_SQ)  // (more only with up to 2,048 columns, whose rows are small)
 
 #define GD_PLAIN 0
 #define GD_SWIGLU 1
@@ -146,6 +160,24 @@ __device__ __forceinline__ int gd_weight_row(const DecodeGemmArgs& a, int u0, in
         return h * D + j + (hi ? half : 0);
     }
     return (a.n_heads + a.n_kv_heads) * D + (u - rot_units) + (hi ? a.n_kv_heads * half : 0);
+}
+
+// The sums over 16 lanes of N <= 2 values each, the first one's in the last lane and the second one's in the last but one.
+template <int N>
+__device__ __forceinline__ float gd_sum_of_16(const float (&a)[N], int lane) {
+#define GD_DPP(x, how) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), how, 0xf, 0xf, true))
+    float v;
+    if constexpr (N == 2) {  // odd lanes add up the first, even lanes the second: two sums of 8 lanes each from here on
+        const bool odd = lane & 1;
+        v = (odd ? a[0] : a[1]) + GD_DPP(odd ? a[1] : a[0], 0xb1);  // (the neighbour's)
+    } else {
+        v = a[0] + GD_DPP(a[0], 0x111);  // (lanes shifted by 1, then 2, 4, 8, with zeros coming in)
+    }
+    v += GD_DPP(v, 0x112);
+    v += GD_DPP(v, 0x114);
+    v += GD_DPP(v, 0x118);
+#undef GD_DPP
+    return v;
 }
 
 // 1 / rms of M <= 16 rows whose waves' sums of squares lie in LDS, [row][wave]: lane l of a wave works out row l / 16 + 4 (l % 4),
@@ -291,12 +323,12 @@ __device__ __forceinline__ void gd_finish_pair(const DecodeGemmArgs& a, int m, i
     }
 }
 
-// XC: chunks of K a wave holds (ceil(K / 128 / 16)); LPI: load instructions per item, each 4 rows of 256 bytes (a
+// XC: chunks of K a wave holds (at least ceil(K / 128 / 8); the launcher says which are built); LPI: load instructions per item, each 4 rows of 256 bytes (a
 // tile is 4 LPI rows); NT: tiles of a group, whose partial sums meet in LDS together (the items of a group,
 // NT * XC, are unrolled).
 template <typename TOut, int EPI, int XC, int LPI, int NT>
 __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const DecodeGemmArgs a) {
-    constexpr int NW = GD_NW;
+    constexpr int NW = GD_NW, SUMS = gd_sums(XC), NS = SUMS * NW;  // sums of the waves: the first of each, then the second
     constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
     static_assert(!PAIRS || LPI == 4, "units with partners fill rows 0..7 and 8..15");
     constexpr int UPT = PAIRS ? 8 : 4 * LPI;  // units per tile
@@ -312,9 +344,9 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     constexpr int EPI_ROUNDS = (NT * PLACES + THREADS - 1) / THREADS;
     extern __shared__ __attribute__((aligned(16))) char gd_lds[];
     u32x4* lds = reinterpret_cast<u32x4*>(gd_lds);                      // per wave 16 rows x 16 pieces of 16 bytes
-    float* red = reinterpret_cast<float*>(gd_lds);                       // later [tile of the group][wave][lane][4]
-    float* sq_lds = reinterpret_cast<float*>(gd_lds + GD_LDS_TILES);     // [row][wave]
-    char* x_lds = gd_lds + GD_LDS_TILES + GD_LDS_SQ;                     // [row][x_pitch bytes]
+    float* red = reinterpret_cast<float*>(gd_lds);                       // later [tile of the group][sum][lane][4]
+    float* sq_lds = reinterpret_cast<float*>(gd_lds + gd_lds_tiles(XC, NT));  // [row][sum]
+    char* x_lds = gd_lds + gd_lds_tiles(XC, NT) + GD_LDS_SQ;             // [row][x_pitch bytes]
     const int tid = threadIdx.x, wave = tid / LLMS_WAVE, lane = tid % LLMS_WAVE;
     const int r16 = lane % 16, g = lane / 16;
     const int M = a.M, K = a.K, n_chunks = (K + GD_KC - 1) / GD_KC;
@@ -391,22 +423,18 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (4 * i < M) {
-                float ss = 0.f;
+                float ss[SUMS] = {};
 #pragma unroll
                 for (int j = 0; j < XC; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) ss = gd_dot2(xf[i][j][e], xf[i][j][e], ss);
-                // (within the 16 lanes: shifts by 1, 2, 4, 8 lanes with zeros coming in; the last lane has the sum)
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x111, 0xf, 0xf, true));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x112, 0xf, 0xf, true));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x114, 0xf, 0xf, true));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x118, 0xf, 0xf, true));
-                if (r16 == 15) sq_lds[(g + 4 * i) * NW + wave] = ss;
+                    for (int e = 0; e < 4; ++e) ss[j % SUMS] = gd_dot2(xf[i][j][e], xf[i][j][e], ss[j % SUMS]);
+                const float sum = gd_sum_of_16<SUMS>(ss, lane);
+                if (r16 > 15 - SUMS) sq_lds[(g + 4 * i) * NS + (15 - r16) * NW + wave] = sum;
             }
         }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // (LDS writes done; the weights stay in flight across the barrier)
         __builtin_amdgcn_s_barrier();
-        const float invs = gd_inverse_rms<NW>(sq_lds, lane, M, K, a.eps);
+        const float invs = gd_inverse_rms<NS>(sq_lds, lane, M, K, a.eps);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (4 * i < M) {
@@ -459,20 +487,24 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     // the items of one group; `more`: another group follows, whose first items are asked for as the ring frees.  The
     // partial sums take the place of the waves' tiles once every wave is done with its own.
     auto run_group = [&](int tile0, const bool more) {
-        f32x4 acc[NT];
+        f32x4 acc[NT][SUMS];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int h = 0; h < SUMS; ++h) acc[t][h] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < ITEMS; ++q) {
             const bool live = wave + NW * (q % XC) < n_chunks;  // (a chunk beyond K: its loads brought zeros)
             if (live) stage(ring[q % RING]);
             if (q + RING < ITEMS) issue(ring[q % RING], tile0, q + RING);  // the registers are free again
             else if (more) issue(ring[q % RING], tile0 + NT, q + RING - ITEMS);
-            if (live) multiply(acc[q / XC], q % XC);
+            if (live) multiply(acc[q / XC][q % XC % SUMS], q % XC);
         }
         __syncthreads();
 #pragma unroll
-        for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(red + ((t * NW + wave) * LLMS_WAVE + lane) * 4) = acc[t];
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int h = 0; h < SUMS; ++h) *reinterpret_cast<f32x4*>(red + ((t * NS + h * NW + wave) * LLMS_WAVE + gd_place<UPT>(g, r16)) * 4) = acc[t][h];
     };
     auto finish_group = [&](int tile0) {
         __syncthreads();
@@ -482,12 +514,14 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
             place_of(e, te, idx);
             const int eu0 = u_begin + (tile0 + te) * UPT;  // first unit of the tile
             if (te >= NT) continue;
-            // sum of the waves for row i (0..15) of the tile and row ml of X, wave 0 first
+            // sum of the waves' sums for row i (0..15) of the tile and row ml of X, wave 0's first
             auto total_of = [&](int i, int ml) -> float {
-                const int src_lane = (i / 4) * 16 + ml, r = i % 4;
-                float s = 0.f;
+                const int src_lane = gd_place<UPT>(i / 4, ml), r = i % 4;
+                float each[NS], s = 0.f;  // (all asked for before the first is added)
 #pragma unroll
-                for (int w = 0; w < NW; ++w) s += red[((te * NW + w) * LLMS_WAVE + src_lane) * 4 + r];
+                for (int w = 0; w < NS; ++w) each[w] = red[((te * NS + w) * LLMS_WAVE + src_lane) * 4 + r];
+#pragma unroll
+                for (int w = 0; w < NS; ++w) s += each[w];
                 return s;
             };
             if (!PAIRS) {
@@ -512,8 +546,7 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     finish_group(tile0);
 }
 
-// 17 to 64 rows of X (RB blocks of 16): the same sharing out of weight rows and of K, with 8 waves that have
-// twice the registers.  A wave keeps its chunks of all rows of X in registers (asked for as whole lines, then
+// 17 to 64 rows of X (RB blocks of 16): the same sharing out of weight rows and of K.  A wave keeps its chunks of all rows of X in registers (asked for as whole lines, then
 // turned into the operand layout through the wave's LDS tile), and every chunk of weights it stages meets RB blocks
 // of rows: RB matrix instructions per fragment read from LDS.  X enters a compute unit once, as much as the unit's
 // share of a large weight; with one workgroup per block of 16 rows it would enter four times as many workgroups.
@@ -525,20 +558,20 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
 
 template <typename TOut, int EPI, int XC, int RB, int NT, bool NORM, int LPI = 4>
 __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(const DecodeGemmArgs a) {
-    constexpr int NW = GR_NW;
+    constexpr int NW = GR_NW, SUMS = RB == 1 ? gd_sums(XC) : 1, NS = SUMS * NW;  // sums of the waves, as in the kernel above
     static_assert(!NORM || RB == 1, "the norm on the way in is for up to 16 rows");
-        constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
+    constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
     static_assert(!PAIRS || LPI == 4, "units with partners fill rows 0..7 and 8..15");
     constexpr int UPT = PAIRS ? 8 : 4 * LPI;  // units per tile (rows of the tile beyond them hold whatever lies in LDS)
     constexpr int ITEMS = NT * XC;
-    constexpr int RING = ITEMS % 2 == 0 ? 2 : (ITEMS < 3 ? ITEMS : 3);  // (1, 2, 3, 4, 6 items: 1, 2, 3, 2, 2)
+    constexpr int RING = ITEMS % 2 == 0 ? 2 : (ITEMS < 3 ? ITEMS : 3);  // (of an even number of items two, of one or three all)
     static_assert(ITEMS % RING == 0, "the ring must go round a whole number of times per group");
     constexpr int THREADS = NW * LLMS_WAVE;
     constexpr int PLACES = UPT * RB * 16;  // (unit or row, row of X) pairs of a tile: one thread each
     constexpr int EPI_ROUNDS = (NT * PLACES + THREADS - 1) / THREADS;
     __shared__ u32x4 lds[NW * 16 * (GD_KC / 8)];         // per wave 16 rows x 16 pieces of 16 bytes
-    __shared__ __attribute__((aligned(16))) float red[NT * NW * RB * LLMS_WAVE * 4];  // [tile of the group][wave][block of rows][lane][4]
-    float* sq_lds = red;  // the norm's sums of squares, [row][wave], before the first sums of the product
+    __shared__ __attribute__((aligned(16))) float red[NT * NS * RB * LLMS_WAVE * 4];  // [tile of the group][sum][block of rows][lane][4]
+    float* sq_lds = red;  // the norm's sums of squares, [row][sum], before the first sums of the product
     const int tid = threadIdx.x, wave = tid / LLMS_WAVE, lane = tid % LLMS_WAVE;
     const int r16 = lane % 16, g = lane / 16;
     const int part = (int)blockIdx.x / a.wgs_per_part, wg = (int)blockIdx.x - part * a.wgs_per_part;
@@ -610,20 +643,17 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (16 * rb + 4 * i >= M) continue;  // (rows that do not exist are zeros and stay zeros)
-                float ss = 0.f;
+                float ss[SUMS] = {};
 #pragma unroll
                 for (int j = 0; j < XC; ++j)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) ss = gd_dot2(xr[j][rb][i][e], xr[j][rb][i][e], ss);
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x111, 0xf, 0xf, true));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x112, 0xf, 0xf, true));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x114, 0xf, 0xf, true));
-                ss += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, ss), 0x118, 0xf, 0xf, true));
-                if (r16 == 15) sq_lds[(16 * rb + 4 * i + g) * NW + wave] = ss;
+                    for (int e = 0; e < 4; ++e) ss[j % SUMS] = gd_dot2(xr[j][rb][i][e], xr[j][rb][i][e], ss[j % SUMS]);
+                const float sum = gd_sum_of_16<SUMS>(ss, lane);
+                if (r16 > 15 - SUMS) sq_lds[(16 * rb + 4 * i + g) * NS + (15 - r16) * NW + wave] = sum;
             }
         __builtin_amdgcn_s_waitcnt(0xc07f);  // (LDS writes done; the weights stay in flight across the barrier)
         __builtin_amdgcn_s_barrier();
-        const float invs = gd_inverse_rms<NW>(sq_lds, lane, M, K, a.eps);  // (one block of rows)
+        const float invs = gd_inverse_rms<NS>(sq_lds, lane, M, K, a.eps);  // (one block of rows)
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -657,9 +687,11 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
             for (int s_ = 0; s_ < 4; ++s_) xr[j][rb][s_] = tile[r16 * 16 + ((4 * s_ + g) ^ r16)];
         }
     auto run_group = [&](int tile0, const bool more) {
-        f32x4 acc[RB];  // (of the tile under way: its sums go to LDS when its last chunk is in)
+        f32x4 acc[SUMS][RB];  // (of the tile under way: its sums go to LDS when its last chunk is in)
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) acc[rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < SUMS; ++h)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) acc[h][rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < ITEMS; ++q) {
             const bool live = wave + NW * (q % XC) < n_chunks;  // (a chunk beyond K: its loads brought zeros)
@@ -678,15 +710,17 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
                     const u32x4 av = tile[r16 * 16 + ((4 * s + g) ^ r16)];
 #pragma unroll
                     for (int rb = 0; rb < RB; ++rb)
-                        acc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gd_as_bf16x8(av), gd_as_bf16x8(xr[q % XC][rb][s]), acc[rb], 0, 0, 0);
+                        acc[q % XC % SUMS][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gd_as_bf16x8(av), gd_as_bf16x8(xr[q % XC][rb][s]), acc[q % XC % SUMS][rb], 0, 0, 0);
                 }
             }
             if (q % XC == XC - 1) {
 #pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    *reinterpret_cast<f32x4*>(red + ((((q / XC) * NW + wave) * RB + rb) * LLMS_WAVE + lane) * 4) = acc[rb];
-                    acc[rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                }
+                for (int h = 0; h < SUMS; ++h)
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) {
+                        *reinterpret_cast<f32x4*>(red + ((((q / XC) * NS + h * NW + wave) * RB + rb) * LLMS_WAVE + gd_place<UPT>(g, r16)) * 4) = acc[h][rb];
+                        acc[h][rb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                    }
             }
         }
     };
@@ -698,12 +732,14 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
             place_of(e, te, idx);
             if (te >= NT) continue;
             const int i = idx % UPT, m = idx / UPT, u = u_begin + (tile0 + te) * UPT + i;
-            // sum of the waves for row i (0..15) of the tile and row m of X, wave 0 first
+            // sum of the waves' sums for row i (0..15) of the tile and row m of X, wave 0's first
             auto total_of = [&](int row) -> float {
-                const int src_lane = (row / 4) * 16 + m % 16, r = row % 4;
-                float sum = 0.f;
+                const int src_lane = gd_place<UPT>(row / 4, m % 16), r = row % 4;
+                float each[NS], sum = 0.f;
 #pragma unroll
-                for (int w = 0; w < NW; ++w) sum += red[(((te * NW + w) * RB + m / 16) * LLMS_WAVE + src_lane) * 4 + r];
+                for (int w = 0; w < NS; ++w) each[w] = red[(((te * NS + w) * RB + m / 16) * LLMS_WAVE + src_lane) * 4 + r];
+#pragma unroll
+                for (int w = 0; w < NS; ++w) sum += each[w];
                 return sum;
             };
             if (m >= M || u >= u_last) continue;
@@ -764,21 +800,21 @@ static void gd_launch_rows_long_k(int tiles, unsigned grid, DecodeGemmArgs& a, h
 // would be half empty (two load instructions less per chunk).
 template <typename TOut, int EPI, bool NORM, int LPI>
 static void gd_launch_rows_one_block(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
-#define GR_GO16(XC, NT)                                                                                             \
+#define GR_GO1(XC, NT)                                                                                              \
     do {                                                                                                            \
         a.groups = (tiles + NT - 1) / NT;                                                                           \
         gemm_decode_rows_kernel<TOut, EPI, XC, 1, NT, NORM, LPI><<<grid, GR_NW * LLMS_WAVE, 0, stream>>>(a);        \
     } while (0)
     if (chunks <= 4 * GR_NW) {
-        if (tiles == 1) GR_GO16(4, 1);
-        else GR_GO16(4, 2);
+        if (tiles == 1) GR_GO1(4, 1);
+        else GR_GO1(4, 2);
     } else if (chunks <= 5 * GR_NW && tiles > 1) {
-        GR_GO16(5, 2);
+        GR_GO1(5, 2);
     } else {
-        if (tiles == 1) GR_GO16(6, 1);
-        else GR_GO16(6, 2);
+        if (tiles == 1) GR_GO1(6, 1);
+        else GR_GO1(6, 2);
     }
-#undef GR_GO16
+#undef GR_GO1
 }
 
 template <typename TOut, int EPI>
@@ -808,9 +844,9 @@ static int gd_launch_rows(int chunks, int rows, int tiles, bool low, unsigned gr
     return LLMS_OK;
 }
 
-// `tiles`: tiles of the workgroup with the most units; `lds_bytes`: what the kernel needs of LDS.
+// `tiles`: tiles of the workgroup with the most units.
 template <typename TOut, int EPI, int LPI>
-static int gd_launch(int chunks, int tiles, unsigned grid, unsigned lds_bytes, DecodeGemmArgs& a, hipStream_t stream) {
+static int gd_launch(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
 #define GD_GO(XC, NT)                                                                                            \
     do {                                                                                                         \
         static bool large_lds_allowed = false;                                                                   \
@@ -820,7 +856,7 @@ static int gd_launch(int chunks, int tiles, unsigned grid, unsigned lds_bytes, D
             large_lds_allowed = true;                                                                            \
         }                                                                                                        \
         a.groups = (tiles + NT - 1) / NT;                                                                        \
-        gemm_decode_kernel<TOut, EPI, XC, LPI, NT><<<grid, GD_NW * LLMS_WAVE, lds_bytes, stream>>>(a);           \
+        gemm_decode_kernel<TOut, EPI, XC, LPI, NT><<<grid, GD_NW * LLMS_WAVE, gd_lds_tiles(XC, NT) + GD_LDS_SQ + a.x_rows * a.x_pitch, stream>>>(a); \
     } while (0)
     // tiles of a group: as few groups as possible, and then as few tiles that do not exist
     const int groups = (tiles + 3) / 4, nt = (tiles + groups - 1) / groups;
@@ -945,7 +981,6 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
     a.units_more = a.units % (int)wgs;
     const int most = a.units_each + (a.units_more ? 1 : 0);  // units of the largest share
     const int chunks = (a.k_each + GD_KC - 1) / GD_KC;
-    const unsigned lds = GD_LDS_TILES + GD_LDS_SQ + (unsigned)(x_rows * x_pitch);
     int rc;
     if (M > 16 || !gd_rows_fit_lds(M, K)) {  // the rows in registers: tiles of 16 weight rows (8 units with partners)
         const bool pairs = epilogue == GD_SWIGLU || epilogue == GD_ROPE_QKV;
@@ -957,22 +992,22 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
         else if (epilogue == GD_RESIDUAL) rc = gd_launch_rows<bf16, GD_RESIDUAL>(chunks, M, tiles, low, grid, a, stream);
         else if (out_dtype == 0) rc = gd_launch_rows<float, GD_PLAIN>(chunks, M, tiles, low, grid, a, stream);
         else rc = gd_launch_rows<bf16, GD_PLAIN>(chunks, M, tiles, low, grid, a, stream);
-    } else if (epilogue == GD_SWIGLU) rc = gd_launch<bf16, GD_SWIGLU, 4>(chunks, (most + 7) / 8, grid, lds, a, stream);
-    else if (epilogue == GD_ROPE_QKV) rc = gd_launch<bf16, GD_ROPE_QKV, 4>(chunks, (most + 7) / 8, grid, lds, a, stream);
+    } else if (epilogue == GD_SWIGLU) rc = gd_launch<bf16, GD_SWIGLU, 4>(chunks, (most + 7) / 8, grid, a, stream);
+    else if (epilogue == GD_ROPE_QKV) rc = gd_launch<bf16, GD_ROPE_QKV, 4>(chunks, (most + 7) / 8, grid, a, stream);
     else {
         // tiles of 8 rows where the last tile of 16 would be half empty (a share of up to 8 rows, of 17 to 24, ...):
         // two load instructions less per chunk
         const bool low = ((most + 7) / 8) % 2 == 1;
         const int tiles = low ? (most + 7) / 8 : (most + 15) / 16;
         if (epilogue == GD_RESIDUAL) {
-            if (low) rc = gd_launch<bf16, GD_RESIDUAL, 2>(chunks, tiles, grid, lds, a, stream);
-            else rc = gd_launch<bf16, GD_RESIDUAL, 4>(chunks, tiles, grid, lds, a, stream);
+            if (low) rc = gd_launch<bf16, GD_RESIDUAL, 2>(chunks, tiles, grid, a, stream);
+            else rc = gd_launch<bf16, GD_RESIDUAL, 4>(chunks, tiles, grid, a, stream);
         } else if (out_dtype == 0) {
-            if (low) rc = gd_launch<float, GD_PLAIN, 2>(chunks, tiles, grid, lds, a, stream);
-            else rc = gd_launch<float, GD_PLAIN, 4>(chunks, tiles, grid, lds, a, stream);
+            if (low) rc = gd_launch<float, GD_PLAIN, 2>(chunks, tiles, grid, a, stream);
+            else rc = gd_launch<float, GD_PLAIN, 4>(chunks, tiles, grid, a, stream);
         } else {
-            if (low) rc = gd_launch<bf16, GD_PLAIN, 2>(chunks, tiles, grid, lds, a, stream);
-            else rc = gd_launch<bf16, GD_PLAIN, 4>(chunks, tiles, grid, lds, a, stream);
+            if (low) rc = gd_launch<bf16, GD_PLAIN, 2>(chunks, tiles, grid, a, stream);
+            else rc = gd_launch<bf16, GD_PLAIN, 4>(chunks, tiles, grid, a, stream);
         }
     }
     if (rc != LLMS_OK) return rc;

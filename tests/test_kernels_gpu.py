@@ -501,6 +501,19 @@ def test_gemm_decode_chunks_of_k(m, k):
         assert (got - want).abs().max() <= 2.0 ** -7 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("k", [1000, 1024, 1032, 2048, 2304, 4096, 5120, 5632, 6144])
+@pytest.mark.parametrize("m", [1, 8, 9, 16])
+def test_gemm_decode_adds_up_sixteen_sums(m, k):
+    """The precision of up to 16 rows: 16 sums over a 16th of the chunks of 128 columns each (c, c + 16, ...), added up in order.  With x
+    zero in all other chunks the product is one of those sums, to the bit; fewer, longer sums would round differently."""
+    for n in (40, 2048, 12288):
+        x, w = rnd(m, k, seed=81).bfloat16().to(DEV), rnd(n, k, seed=82).bfloat16().to(DEV)
+        chunk, want = torch.arange(k, device=DEV) // 128, torch.zeros(m, n, device=DEV)
+        for c in range(16):
+            want += ops().gemm_decode(torch.empty(m, n, device=DEV), x.masked_fill(chunk % 16 != c, 0), w)
+        assert torch.equal(ops().gemm_decode(torch.empty(m, n, device=DEV), x, w), want), n
+
+
 @pytest.mark.parametrize("m,n,k,parts", [(64, 2048, 5632, 3), (17, 333, 2048 + 8, 2), (33, 4096, 11008, 6), (40, 100, 520, 5),
                                          (24, 2048, 5632, 3), (64, 48, 256, 2)])
 def test_gemm_decode_shares_k_out_for_many_rows(m, n, k, parts):
