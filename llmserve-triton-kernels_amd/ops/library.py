@@ -704,7 +704,6 @@ GEMM_TILES_NEAR_RATE = 2.9e6
 
 
 @functools.lru_cache(maxsize=4096)
-@functools.lru_cache(maxsize=4096)
 def gemm_tiles_workers(tile: int | None, m: int, n: int, k: int, parts: int, nbytes: int, cus: int = 256) -> int:
     """How many workgroups beyond those of the tiles bring a weight of `nbytes` nearer: as many as do so in four fifths of a round's
     time, if there are as many compute units without a tile in the last round and memory has time for both weights; otherwise none.
