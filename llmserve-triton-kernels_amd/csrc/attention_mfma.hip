@@ -1212,8 +1212,16 @@ static int attention_mfma_launch(AttnLaunch* only, void* out, int out_stride, co
         dim3 grid(groups * num_splits, n_kv_heads * HB, n_seqs);
         if (arrive && num_splits > 1 && num_splits <= 16 && (long long)groups * grid.y * grid.z <= n_arrive) {
             a.arrive = arrive;
-            a.split_inv = (unsigned)((1ull << 32) / num_splits + 1);
-            a.split_shift = std::max(0, 3 - __builtin_ctz((unsigned)num_splits));
+            int cus = 0;
+            if (int e = compute_units(&cus)) return e;
+            // Places are turned where those that stay would otherwise take more than five eighths of the compute units of their XCDs; few are
+            // better on few XCDs, by the kernels around them too: a step of the 1.1B shape behind 512 keys, 4 KV heads, in 4 shares, turned
+            // and not: 2 requests 0.765 ms and 0.741, 6 0.791 and 0.766, 8 0.791 and 0.780, 10 0.879 and 0.877, 12 0.876 and 0.884, 16
+            // 0.878 and 0.904.
+            if (8ll * groups * grid.y * grid.z * num_splits > 5ll * cus) {
+                a.split_inv = (unsigned)((1ull << 32) / num_splits + 1);
+                a.split_shift = std::max(0, 3 - __builtin_ctz((unsigned)num_splits));
+            }
         }
         if (only) {
             *only = AttnLaunch{a, grid, 0};
