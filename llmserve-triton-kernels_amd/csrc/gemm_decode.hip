@@ -29,7 +29,7 @@
 // and 68.2; with 8 waves and six or four items 24.6, 26.2, 63.1 and 65.6 (half the waves start and meet), with two items 23.8, 25.2, 58.0
 // and 60.7, with one 25.9, 27.6, 61.4 and 64.1: memory answers a compute unit some 40 KB at a time, and what all compute units ask for
 // beyond that comes from more open rows of memory at once.  That the sums still have no more terms than 16 waves' (gd_sums) takes 0.2 to
-// 0.9 of them back: 24.5, 25.9, 58.2 and 61.3.  The vocabulary's product, 32000 x 2048: 29.2 -> 23.1 (5.7 TB/s).
+// 0.8 of them back: 24.4, 25.7, 58.2 and 61.3.  The vocabulary's product, 32000 x 2048: 29.2 -> 23.1 (5.7 TB/s).
 //
 // Epilogues (the waves' partial sums meet in LDS in the order of the waves):
 //   PLAIN     C = sums (+ bias), float32 or bfloat16; `unit` 2: max(sums, 0)^2.
@@ -62,13 +62,15 @@ constexpr int gd_sums(int xc) { return xc > 1 ? 2 : 1; }
 template <int UPT>
 __device__ __forceinline__ int gd_place(int g, int m) { return 16 * g + ((m + (UPT == 8 ? 8 : 4) * g) & 15); }
 
-// LDS: the waves' tiles (later their partial sums), the rows' sums of squares, then the rows of X
-constexpr int gd_lds_tiles(int xc, int nt) {
-    const int tiles = GD_NW * 16 * (GD_KC / 8) * 16, sums = nt * gd_sums(xc) * GD_NW * LLMS_WAVE * 16;
-    return tiles > sums ? tiles : sums;
-}
+// LDS: the waves' tiles, the rows' sums of squares, the rows of X, then the partial sums, which a wave leaves as soon as it has them.  Where
+// that is more than there is, the sums take the tiles' place once every wave is done with its own (a layer's four products of the 1.1B shape
+// at 8 rows 26.9 microseconds so, 26.7 apart, gate and up 10.4 and 10.2; a step of 16 requests 0.895 ms and 0.890).
+#define GD_LDS 163840
+#define GD_LDS_TILES (GD_NW * 16 * (GD_KC / 8) * 16)
+constexpr int gd_lds_sums(int xc, int nt) { return nt * gd_sums(xc) * GD_NW * LLMS_WAVE * 16; }
+constexpr int gd_lds_tiles(int xc, int nt) { return GD_LDS_TILES > gd_lds_sums(xc, nt) ? GD_LDS_TILES : gd_lds_sums(xc, nt); }
 #define GD_LDS_SQ (16 * 2 * GD_NW * 4)
-#define GD_LDS_X_MAX (160 * 1024 - gd_lds_tiles(3, 2) - GD_LDS_SQ)  // (more only with up to 2,048 columns, whose rows are small)
+#define GD_LDS_X_MAX (GD_LDS - gd_lds_tiles(3, 2) - GD_LDS_SQ)  // (more only with up to 2,048 columns, whose rows are small)
 
 #define GD_PLAIN 0
 #define GD_SWIGLU 1
@@ -114,6 +116,7 @@ struct DecodeGemmArgs {
     // parts up.  ldw is the row stride of W (K of the whole weight).
     int ldw, k_parts, k_each, wgs_per_part;
     long long part_stride;
+    int sq_at, sums_at;  // up to 16 rows: where the sums of squares and the partial sums (0: in the tiles' place) lie in LDS
 };
 
 __device__ __forceinline__ bf16x8 gd_as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -344,9 +347,9 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     constexpr int EPI_ROUNDS = (NT * PLACES + THREADS - 1) / THREADS;
     extern __shared__ __attribute__((aligned(16))) char gd_lds[];
     u32x4* lds = reinterpret_cast<u32x4*>(gd_lds);                      // per wave 16 rows x 16 pieces of 16 bytes
-    float* red = reinterpret_cast<float*>(gd_lds);                       // later [tile of the group][sum][lane][4]
-    float* sq_lds = reinterpret_cast<float*>(gd_lds + gd_lds_tiles(XC, NT));  // [row][sum]
-    char* x_lds = gd_lds + gd_lds_tiles(XC, NT) + GD_LDS_SQ;             // [row][x_pitch bytes]
+    float* red = reinterpret_cast<float*>(gd_lds + a.sums_at);           // [tile of the group][sum][lane][4]
+    float* sq_lds = reinterpret_cast<float*>(gd_lds + a.sq_at);          // [row][sum]
+    char* x_lds = gd_lds + a.sq_at + GD_LDS_SQ;                          // [row][x_pitch bytes]
     const int tid = threadIdx.x, wave = tid / LLMS_WAVE, lane = tid % LLMS_WAVE;
     const int r16 = lane % 16, g = lane / 16;
     const int M = a.M, K = a.K, n_chunks = (K + GD_KC - 1) / GD_KC;
@@ -484,8 +487,7 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gd_as_bf16x8(av), gd_as_bf16x8(xv), acc, 0, 0, 0);
         }
     };
-    // the items of one group; `more`: another group follows, whose first items are asked for as the ring frees.  The
-    // partial sums take the place of the waves' tiles once every wave is done with its own.
+    // the items of one group; `more`: another group follows, whose first items are asked for as the ring frees.
     auto run_group = [&](int tile0, const bool more) {
         f32x4 acc[NT][SUMS];
 #pragma unroll
@@ -500,7 +502,7 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
             else if (more) issue(ring[q % RING], tile0 + NT, q + RING - ITEMS);
             if (live) multiply(acc[q / XC][q % XC % SUMS], q % XC);
         }
-        __syncthreads();
+        if (!a.sums_at) __syncthreads();  // (the waves' tiles lie there)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -852,11 +854,15 @@ static int gd_launch(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hi
         static bool large_lds_allowed = false;                                                                   \
         if (!large_lds_allowed) {                                                                                \
             LLMS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_decode_kernel<TOut, EPI, XC, LPI, NT>), \
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));         \
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, GD_LDS));             \
             large_lds_allowed = true;                                                                            \
         }                                                                                                        \
         a.groups = (tiles + NT - 1) / NT;                                                                        \
-        gemm_decode_kernel<TOut, EPI, XC, LPI, NT><<<grid, GD_NW * LLMS_WAVE, gd_lds_tiles(XC, NT) + GD_LDS_SQ + a.x_rows * a.x_pitch, stream>>>(a); \
+        const int rest = GD_LDS_SQ + a.x_rows * a.x_pitch, sums = gd_lds_sums(XC, NT);                           \
+        const bool apart = GD_LDS_TILES + rest + sums <= GD_LDS;                                                 \
+        a.sq_at = apart ? GD_LDS_TILES : gd_lds_tiles(XC, NT);                                                   \
+        a.sums_at = apart ? GD_LDS_TILES + rest : 0;                                                             \
+        gemm_decode_kernel<TOut, EPI, XC, LPI, NT><<<grid, GD_NW * LLMS_WAVE, a.sq_at + rest + (apart ? sums : 0), stream>>>(a); \
     } while (0)
     // tiles of a group: as few groups as possible, and then as few tiles that do not exist
     const int groups = (tiles + 3) / 4, nt = (tiles + groups - 1) / groups;

@@ -514,6 +514,18 @@ def test_gemm_decode_adds_up_sixteen_sums(m, k):
         assert torch.equal(ops().gemm_decode(torch.empty(m, n, device=DEV), x, w), want), n
 
 
+@pytest.mark.parametrize("n,k", [(16384, 2048), (32768, 2048), (2048, 3840), (16400, 3456)])
+def test_gemm_decode_sums_apart_from_the_tiles_or_in_their_place(n, k):
+    """In one group of tiles and in more: with 8 rows the partial sums have room of their own in LDS, with 16 (but for one tile of 3456 columns)
+    they do not and take the place of the waves' tiles.  A row's result is the same bits either way."""
+    x, w = rnd(16, k, seed=83).bfloat16().to(DEV), rnd(n, k, seed=84).bfloat16().to(DEV)
+    got = ops().gemm_decode(torch.empty(16, n, device=DEV), x, w)
+    for first in (0, 8):
+        assert torch.equal(ops().gemm_decode(torch.empty(8, n, device=DEV), x[first:first + 8], w), got[first:first + 8])
+    ref = x.double() @ w.double().t()
+    assert (got.double() - ref).abs().max() <= 2e-6 * math.sqrt(k) * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("m,n,k,parts", [(64, 2048, 5632, 3), (17, 333, 2048 + 8, 2), (33, 4096, 11008, 6), (40, 100, 520, 5),
                                          (24, 2048, 5632, 3), (64, 48, 256, 2)])
 def test_gemm_decode_shares_k_out_for_many_rows(m, n, k, parts):
