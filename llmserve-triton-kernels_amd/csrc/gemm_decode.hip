@@ -28,8 +28,9 @@
 // each a layer's four products of the 1.1B shape took 25.3 microseconds at 1 row and 26.9 at 8, of the 7B shape (without down_proj) 66.0
 // and 68.2; with 8 waves and six or four items 24.6, 26.2, 63.1 and 65.6 (half the waves start and meet), with two items 23.8, 25.2, 58.0
 // and 60.7, with one 25.9, 27.6, 61.4 and 64.1: memory answers a compute unit some 40 KB at a time, and what all compute units ask for
-// beyond that comes from more open rows of memory at once.  That the sums still have no more terms than 16 waves' (gd_sums) takes 0.2 to
-// 0.8 of them back: 24.4, 25.7, 58.2 and 61.3.  The vocabulary's product, 32000 x 2048: 29.2 -> 23.1 (5.7 TB/s).
+// beyond that comes from more open rows of memory at once.  That the sums still have no more terms than 16 waves' (gd_sums) takes 0.4 to
+// 0.6 of them back (in turn, 16 waves, 8 with one sum each, 8 with two: 26.4, 24.9 and 25.4 at 1 row, 27.6, 26.1 and 26.7 at 8, 66.0, 59.2 and
+// 59.7, 67.2, 60.8 and 61.5).  The vocabulary's product, 32000 x 2048: 26.1 -> 23.3 (5.6 TB/s).
 //
 // Epilogues (the waves' partial sums meet in LDS in the order of the waves):
 //   PLAIN     C = sums (+ bias), float32 or bfloat16; `unit` 2: max(sums, 0)^2.
