@@ -78,6 +78,7 @@ struct TilesArgs {
     void* C;
     int M, N, K, ldx, ldc;
     int tiles_m, tiles;          // tiles along M, tiles in all (of one part)
+    int band, band_tiles;        // tiles along M that are walked together, tiles of such a band
     int workgroups;              // of the tiles in all parts
     int steps;                   // of 64 columns, of one part
     long long part_stride;       // elements from one part's sums to the next's
@@ -173,11 +174,18 @@ __global__ __launch_bounds__((WM * WN + NP) * LLMS_WAVE) void gemm_tiles_kernel(
 
     const int part = EPI == GT_FLOAT ? blockIdx.x / a.tiles : 0, pid = blockIdx.x - part * a.tiles;
     const int first = part * a.steps, steps = min(a.steps, a.K / 64 - first);
-    // workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, rows fastest, so that the tiles
-    // which share weight rows share an L2
+    // workgroups are dealt round-robin to the 8 XCDs: each XCD gets a contiguous run of tiles, in bands of `band` tiles along M, rows
+    // fastest, so that the tiles which share rows of X or weight rows share an L2
     const int full = a.tiles / 8, rem = a.tiles % 8, xcd = pid % 8;
     const int t = xcd * full + min(xcd, rem) + pid / 8;
-    const int m0 = (t % a.tiles_m) * BM, n0 = (t / a.tiles_m) * BN;
+    int above = 0, in_band = t, high = a.tiles_m;
+    if (a.band < a.tiles_m) {  // (a division that most launches do without)
+        const int b = t / a.band_tiles;
+        above = b * a.band;
+        in_band = t - b * a.band_tiles;
+        high = min(a.band, a.tiles_m - above);
+    }
+    const int m0 = (above + in_band % high) * BM, n0 = in_band / high * BN;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / LLMS_WAVE), lane = tid % LLMS_WAVE;
     const int loader = NP ? wave - NW : wave;  // (NP: the last waves load, the others multiply)
     const int wm = (wave % WM) * (BM / WM), wn = (wave / WM) * (BN / WN);
@@ -560,6 +568,27 @@ __global__ __launch_bounds__((WM * WN + NP) * LLMS_WAVE) void gemm_tiles_kernel(
     }
 }
 
+// How many tiles along M an XCD walks together.  Of the rows that its `run` of tiles asks L2 for, those of X that lie in the band and those of W
+// behind the columns that the run then reaches, the fewest: what the tiles do not share comes from the memory-side cache, and a row from
+// there holds up those behind it.  (All of M together, as it is where few rows leave few tiles along M, and in bands, microseconds, weights from
+// memory, at 2,048 rows: 2560 x 2048 23.4 and 22.0, 2048 x 2048 18.7 and 18.0, 2048 x 5632 52.1 and 49.2, 4096 x 4096 57.4 and 56.2, 4096 x
+// 11008 147.5 and 144.6; 11264 x 2048 gated 87.9 and 87.3, 22016 x 4096 gated 303.3 and 301.4.  A
+// few rows less are not worth it, since a weight row that two XCDs ask for comes from memory and one of X does not: 2048 x 5632 in two parts at
+// 513 rows, 800 for 832.)
+static int gt_band(int tiles_m, int bm, int bn, int run) {
+    int best = tiles_m;
+    long long least = -1;
+    for (int bands = 1; bands <= tiles_m && bands <= 64; ++bands) {
+        const int high = (tiles_m + bands - 1) / bands;
+        const long long rows = (long long)high * bm + (long long)((run + high - 1) / high) * bn;
+        if (least < 0 || rows < least - least / 8) {
+            least = rows;
+            best = high;
+        }
+    }
+    return best;
+}
+
 template <int BM, int BN, int WM, int WN, int NP, int SX, int SW, int U>
 static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
     LLMS_REQUIRE(a.K % 64 == 0, "gemm_tiles: K must be a multiple of 64");
@@ -567,6 +596,9 @@ static int launch(int epilogue, TilesArgs a, int parts, hipStream_t stream) {
     a.tiles_m = (a.M + BM - 1) / BM;
     LLMS_REQUIRE((long long)a.tiles_m * tiles_n * parts < (1ll << 31), "gemm_tiles: too many tiles");
     a.tiles = a.tiles_m * tiles_n;
+    const int held = 2 * (SX * BM + SW * BN) * 128 <= 163840 ? 2 : 1, each = (a.tiles + 7) / 8;  // tiles a compute unit has at once; of an XCD
+    a.band = gt_band(a.tiles_m, BM, BN, each < 32 * held ? each : 32 * held);
+    a.band_tiles = a.band * tiles_n;
     a.steps = (a.K / 64 + parts - 1) / parts;
     LLMS_REQUIRE((long long)(parts - 1) * a.steps < a.K / 64, "gemm_tiles: a part of K is empty");
     a.workgroups = a.tiles * parts;

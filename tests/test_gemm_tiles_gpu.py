@@ -63,6 +63,23 @@ def test_plain_and_parts(tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile", range(17))
+def test_bands(tile):
+    """Seven tiles along M are walked in bands, the last of which is lower: every tile is there once, in one part of K and in two."""
+    bm, bn, _ = sizes_of(tile)
+    m, n, k = 7 * bm - 5, 13 * bn - 16, 128
+    x, w = rnd(m, k, seed=11).to(DEV), rnd(n, k, seed=12).to(DEV)
+    want = (x.double() @ w.double().t()).cpu()
+    out = torch.full((m + 1, n), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_tiles(out[:m], x, w, tile=tile)
+    close(out[:m], want, k)
+    assert bool((out[m:] == 7.0).all())
+    sums = torch.full((2, m, n), 7.0, device=DEV)
+    ops().gemm_tiles(sums, x, w, tile=tile)
+    close(sums.double().sum(0), want, k, False)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("tile", TILES)
 @pytest.mark.parametrize("limit,gelu", [(None, False), (1.5, False), (None, True)])
 def test_gated(tile, limit, gelu):
