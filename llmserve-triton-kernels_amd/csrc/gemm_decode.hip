@@ -39,11 +39,14 @@
 //   ROPE_QKV  W = [q; k; v]; q and k rotated (src/llmserve/model/llama.py:31-54), q written, k and v stored at the
 //             tokens' slots of the paged cache (values transposed inside a page).
 //   RESIDUAL  residual[m, n] = bf16(residual[m, n] + bf16(sums)) in place: the layer's residual sum
-//             (src/llmserve/model/llama.py:131-135), so that the next product's prologue finds whole rows to norm.
+//             (src/llmserve/model/llama.py:131-135), so that the next product's prologue finds whole rows to norm.  A 32-bit
+//             stream takes the unrounded sums, times a gate sigmoid(z) where there is one.
 // What is shared out to the workgroups are units: a weight row (PLAIN, RESIDUAL), a feature's gate and up rows
 // (SWIGLU), a rotary pair (i, i + D/2) of a query or key head or two value rows (ROPE_QKV).  A tile is up to 16
 // rows of the matrix instruction: 8 or 16 units, or 8 units with their partners in rows 8 to 15.
 #include "common.h"
+
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -82,6 +85,18 @@ constexpr int gd_lds_tiles(int xc, int nt) { return GD_LDS_TILES > gd_lds_sums(x
 #define GD_UNIT_RELU2 2
 #define GD_UNIT_GELU 3
 
+// Rows of a 32-bit stream, which the product makes its own rows of on the way in (up to 8 rows):
+//   GD_FROM_OPEN  the stream has an open sum, which is closed: x + y / sqrt(mean(y^2) + eps) * w, rounded once
+//   GD_FROM_NORM  the rows are normed: x / sqrt(mean(x^2) + eps) * (offset + w), rounded once
+#define GD_FROM_OPEN 1
+#define GD_FROM_NORM 2
+struct DecodeStream {
+    const float *x, *y, *w;  // x, y [M, K] without gaps, w [K]
+    float* x_out;            // OPEN: the stream with its sum closed: not x itself, which other workgroups read
+    bf16* h_out;             // or null: the rows of the product, for who reads them next
+    float offset;
+};
+
 struct DecodeGemmArgs {
     const bf16* W;
     const bf16* X;
@@ -119,6 +134,17 @@ struct DecodeGemmArgs {
     long long part_stride;
     int sq_at, sums_at;  // up to 16 rows: where the sums of squares and the partial sums (0: in the tiles' place) lie in LDS
 };
+
+// ... and of the few kernels that read rows of a 32-bit stream or add to one.
+struct DecodeStreamArgs : DecodeGemmArgs {
+    DecodeStream from;
+    // RESIDUAL with 32-bit rows: residual32[m, n] += g * sums, g = sigmoid(gate_z[m, gate_col + n] + gate_bias[n]) or 1 (no gate_z)
+    float* residual32;
+    const float *gate_z, *gate_bias;
+    int ldz, gate_col;
+};
+template <typename TOut, int EPI, int FROM>
+using GdArgs = typename std::conditional<FROM != 0 || (EPI == GD_RESIDUAL && sizeof(TOut) == 4), DecodeStreamArgs, DecodeGemmArgs>::type;
 
 __device__ __forceinline__ bf16x8 gd_as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 // Loads through a buffer descriptor: an offset beyond the buffer's end (GD_NOWHERE) brings zeros and touches no
@@ -188,8 +214,8 @@ __device__ __forceinline__ float gd_sum_of_16(const float (&a)[N], int lane) {
 // once for all the rows its lanes will norm (up to 4 rows: row l / 16, the lanes of a group then read one address).  With every lane
 // working out each row in turn, 16 additions, a division and a root a row, that was half the vector instructions of the norm, which
 // the waves of a compute unit share its vector units for (then 16 of them): q, k, v with the norm at 8 rows 5.85 -> 5.65 microseconds, at 16 rows 7.3 -> 6.5,
-// the same bits.
-template <int NW>
+// the same bits.  EXACT: a division and a root instead of the hardware's inverse root.
+template <int NW, bool EXACT = false>
 __device__ __forceinline__ float gd_inverse_rms(const float* sq, int lane, int M, int K, float eps) {
     const float* mine = sq + (lane / 16 + (M > 4 ? 4 * (lane % 4) : 0)) * NW;
     float total = 0.f;
@@ -201,7 +227,7 @@ __device__ __forceinline__ float gd_inverse_rms(const float* sq, int lane, int M
         total += part[2];
         total += part[3];
     }
-    return rsqrtf(total / (float)K + eps);
+    return EXACT ? 1.f / sqrtf(total / (float)K + eps) : rsqrtf(total / (float)K + eps);
 }
 // ... of row lane / 16 + 4 i: what lane i of the quad has
 __device__ __forceinline__ float gd_of_quad(float v, int i) {
@@ -219,25 +245,32 @@ struct GdFinish {
     float freq;
     float sn, cs;
     unsigned res;
+    float res32, z, gate_bias;
 };
 
 struct GdFinishBuffers {
-    __amdgpu_buffer_rsrc_t pos, slot, freq, angles, res;
+    __amdgpu_buffer_rsrc_t pos, slot, freq, angles, res, res32, z, gate_bias;
 };
 
-__device__ __forceinline__ GdFinishBuffers gd_finish_buffers(const DecodeGemmArgs& a) {
+template <typename Args>
+__device__ __forceinline__ GdFinishBuffers gd_finish_buffers(const Args& a) {
     GdFinishBuffers b;
     b.pos = gd_buffer(a.positions, a.positions ? (unsigned)a.M * 4 : 0u);
     b.slot = gd_buffer(a.slots, a.slots ? (unsigned)a.M * 4 : 0u);
     b.freq = gd_buffer(a.inv_freq, a.inv_freq ? (unsigned)a.head_dim * 2 : 0u);
     b.angles = gd_buffer(a.angles, a.angles ? (unsigned)a.M * a.head_dim * 4 : 0u);
     b.res = gd_buffer(a.residual, a.residual ? (unsigned)(((size_t)(a.M - 1) * a.ldr + a.N) * 2) : 0u);
+    if constexpr (std::is_same<Args, DecodeStreamArgs>::value) {
+        b.res32 = gd_buffer(a.residual32, a.residual32 ? (unsigned)(((size_t)(a.M - 1) * a.ldr + a.N) * 4) : 0u);
+        b.z = gd_buffer(a.gate_z, a.gate_z ? (unsigned)(((size_t)(a.M - 1) * a.ldz + a.gate_col + a.N) * 4) : 0u);
+        b.gate_bias = gd_buffer(a.gate_bias, a.gate_bias ? (unsigned)a.N * 4 : 0u);
+    }
     return b;
 }
 
 // `u`: the unit (pairs) or weight row (plain, residual) of the place, `m` its row of X; `live`: the place exists.
-template <int EPI>
-__device__ __forceinline__ void gd_ask(const DecodeGemmArgs& a, const GdFinishBuffers& b, bool live, int m, int u, GdFinish& f) {
+template <typename TOut, int EPI, typename Args>
+__device__ __forceinline__ void gd_ask(const Args& a, const GdFinishBuffers& b, bool live, int m, int u, GdFinish& f) {
     if (EPI == GD_ROPE_QKV) {
         const int half = a.head_dim / 2;
         f.slot = (int)__builtin_amdgcn_raw_buffer_load_b32(b.slot, live ? (unsigned)m * 4 : GD_NOWHERE, 0, 0);
@@ -254,21 +287,27 @@ __device__ __forceinline__ void gd_ask(const DecodeGemmArgs& a, const GdFinishBu
         f.sn = __uint_as_float(sc[0]);
         f.cs = __uint_as_float(sc[1]);
     }
-    if (EPI == GD_RESIDUAL)
+    if constexpr (EPI == GD_RESIDUAL && sizeof(TOut) == 4) {
+        f.res32 = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b.res32, live ? (unsigned)(m * a.ldr + u) * 4 : GD_NOWHERE, 0, 0));
+        f.z = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b.z, live ? (unsigned)(m * a.ldz + a.gate_col + u) * 4 : GD_NOWHERE, 0, 0));
+        f.gate_bias = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b.gate_bias, live ? (unsigned)u * 4 : GD_NOWHERE, 0, 0));
+    } else if (EPI == GD_RESIDUAL)
         f.res = __builtin_amdgcn_raw_buffer_load_b16(b.res, live ? (unsigned)(m * a.ldr + u) * 2 : GD_NOWHERE, 0, 0);
 }
 
 // PLAIN, RESIDUAL: the sum `s` of weight row n and row m of X.
-template <typename TOut, int EPI>
-__device__ __forceinline__ void gd_finish_row(const DecodeGemmArgs& a, int m, int n, float s, const GdFinish& f,
+template <typename TOut, int EPI, typename Args>
+__device__ __forceinline__ void gd_finish_row(const Args& a, int m, int n, float s, const GdFinish& f,
                                               size_t part_offset = 0) {
     if (a.bias) s += bf16_bits_to_f32(a.bias[n].bits);
     if (EPI == GD_PLAIN && a.unit == GD_UNIT_RELU2) {
         const float r = fmaxf(s, 0.f);
         s = r * r;
     }
-    if (EPI == GD_PLAIN)
+    if constexpr (EPI == GD_PLAIN)
         gd_store<TOut>(reinterpret_cast<TOut*>(a.C) + part_offset + (size_t)m * a.ldc + n, s);
+    else if constexpr (sizeof(TOut) == 4)
+        a.residual32[(size_t)m * a.ldr + n] = f.res32 + (a.gate_z ? 1.f / (1.f + expf(-(f.z + f.gate_bias))) : 1.f) * s;
     else
         a.residual[(size_t)m * a.ldr + n].bits = f32_to_bf16_bits(bf16_bits_to_f32((uint16_t)f.res) + gd_bfr(s));
 }
@@ -327,11 +366,104 @@ __device__ __forceinline__ void gd_finish_pair(const DecodeGemmArgs& a, int m, i
     }
 }
 
+// What a lane has of a chunk in 32-bit: columns k .. k + 7.
+struct GdEight {
+    float at[8];
+};
+__device__ __forceinline__ GdEight gd_load_eight(__amdgpu_buffer_rsrc_t b, unsigned offset) {
+    GdEight v;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const u32x4 four = gd_load(b, offset + 16 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v.at[4 * h + e] = __uint_as_float(four[e]);
+    }
+    return v;
+}
+
+// The rows of the product from those of a stream (`FROM`), as packed pairs of bfloat16 in xf: lane (g, r16) of a wave has columns 8 r16 .. 8 r16
+// + 7 of its chunks of rows g and g + 4.  Every workgroup works out all rows, which costs what is pulled in from L2 (4 rows of 2,048 with an open
+// sum 0.6 microseconds, where the kernel it saves takes 4.3); workgroup c, c + the grid, ... stores chunk c of what others will read.  (A sum
+// through two sigmoid gates was closed here as well: five rows for one, and 64 exponentials a lane in every workgroup, took 5 of
+// the 5.5 microseconds that its kernel takes.  Gates are the epilogue's, where an element meets its gate once.)  `asked` is called when
+// everything is asked for: weights may be from there on.
+template <int XC, int FROM, typename Asked>
+__device__ __forceinline__ void gd_rows_from_stream(const DecodeStreamArgs& a, float* sq_lds, u32x4 (&xf)[4][XC], Asked asked) {
+    constexpr int NW = GD_NW, SUMS = gd_sums(XC), NS = SUMS * NW, RI = 2;
+    const DecodeStream& t = a.from;
+    const int wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE, r16 = lane % 16, g = lane / 16;
+    const int M = a.M, K = a.K, n_chunks = (K + GD_KC - 1) / GD_KC;
+    const unsigned bytes = (unsigned)M * K * 4u;
+    const __amdgpu_buffer_rsrc_t xb = gd_buffer(t.x, bytes), yb = gd_buffer(t.y, FROM == GD_FROM_OPEN ? bytes : 0u), wb = gd_buffer(t.w, (unsigned)K * 4u);
+    GdEight x[RI][XC], y[FROM == GD_FROM_OPEN ? RI : 1][XC], w[XC];
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+        if (4 * i < M) {
+#pragma unroll
+            for (int j = 0; j < XC; ++j) {
+                const int row = g + 4 * i, k = (wave + NW * j) * GD_KC + 8 * r16;
+                const unsigned at = row < M && k < K ? (unsigned)(row * K + k) * 4u : GD_NOWHERE;
+                x[i][j] = gd_load_eight(xb, at);
+                if constexpr (FROM == GD_FROM_OPEN) y[i][j] = gd_load_eight(yb, at);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < XC; ++j) {
+        const int k = (wave + NW * j) * GD_KC + 8 * r16;
+        w[j] = gd_load_eight(wb, k < K ? (unsigned)k * 4u : GD_NOWHERE);
+    }
+    __builtin_amdgcn_s_barrier();  // (no wave asks for weights before every wave has asked for its rows)
+    asked();
+    // sums of squares, of what joins or of the stream: the lane's, the 16 lanes of a row's chunk, then the waves in their order
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+        if (4 * i < M) {
+            float ss[SUMS] = {};
+#pragma unroll
+            for (int j = 0; j < XC; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = FROM == GD_FROM_OPEN ? y[i][j].at[e] : x[i][j].at[e];
+                    ss[j % SUMS] = fmaf(v, v, ss[j % SUMS]);
+                }
+            const float sum = gd_sum_of_16<SUMS>(ss, lane);
+            if (r16 > 15 - SUMS) sq_lds[(g + 4 * i) * NS + (15 - r16) * NW + wave] = sum;
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // (LDS writes done; the weights stay in flight across the barrier)
+    __builtin_amdgcn_s_barrier();
+    const float invs = gd_inverse_rms<NS, true>(sq_lds, lane, M, K, a.eps);
+#pragma unroll
+    for (int i = 0; i < RI; ++i) {
+        if (4 * i >= M) continue;
+        const float inv = gd_of_quad(invs, i);
+#pragma unroll
+        for (int j = 0; j < XC; ++j) {
+            GdEight h;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                h.at[e] = FROM == GD_FROM_OPEN ? x[i][j].at[e] + y[i][j].at[e] * inv * w[j].at[e] : x[i][j].at[e] * inv * (t.offset + w[j].at[e]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) xf[i][j][e] = pack_bf16x2(h.at[2 * e], h.at[2 * e + 1]);
+            const int c = wave + NW * j, k = c * GD_KC + 8 * r16, row = g + 4 * i;
+            if (c < n_chunks && c % gridDim.x == blockIdx.x && row < M && k < K) {
+                if constexpr (FROM == GD_FROM_OPEN) {
+                    float* to = t.x_out + (size_t)row * K + k;
+                    *reinterpret_cast<f32x4*>(to) = (f32x4){h.at[0], h.at[1], h.at[2], h.at[3]};
+                    *reinterpret_cast<f32x4*>(to + 4) = (f32x4){h.at[4], h.at[5], h.at[6], h.at[7]};
+                }
+                if (t.h_out) *reinterpret_cast<u32x4*>(t.h_out + (size_t)row * K + k) = xf[i][j];
+            }
+        }
+    }
+}
+
 // XC: chunks of K a wave holds (at least ceil(K / 128 / 8); the launcher says which are built); LPI: load instructions per item, each 4 rows of 256 bytes (a
 // tile is 4 LPI rows); NT: tiles of a group, whose partial sums meet in LDS together (the items of a group,
 // NT * XC, are unrolled).
-template <typename TOut, int EPI, int XC, int LPI, int NT>
-__global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const DecodeGemmArgs a) {
+template <typename TOut, int EPI, int XC, int LPI, int NT, int FROM>
+__global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const GdArgs<TOut, EPI, FROM> a) {
     constexpr int NW = GD_NW, SUMS = gd_sums(XC), NS = SUMS * NW;  // sums of the waves: the first of each, then the second
     constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
     static_assert(!PAIRS || LPI == 4, "units with partners fill rows 0..7 and 8..15");
@@ -361,24 +493,26 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     // ---- first what is small and needed early: this wave's chunks of the rows of X that exist (lane (g, p) brings
     // piece p of 16 bytes of rows g, g + 4, ...), and the norm's weight for the same columns
     u32x4 xf[4][XC], nwf[XC];
-    const __amdgpu_buffer_rsrc_t x_buf = gd_buffer(a.X, (unsigned)(((size_t)(M - 1) * a.ldx + K) * 2));
+    if constexpr (!FROM) {
+        const __amdgpu_buffer_rsrc_t x_buf = gd_buffer(a.X, (unsigned)(((size_t)(M - 1) * a.ldx + K) * 2));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (4 * i < M) {
+        for (int i = 0; i < 4; ++i) {
+            if (4 * i < M) {
 #pragma unroll
-            for (int j = 0; j < XC; ++j) {
-                const int row = g + 4 * i, k = (wave + NW * j) * GD_KC + 8 * r16;
-                xf[i][j] = gd_load(x_buf, row < M && k < K ? (unsigned)(row * a.ldx + k) * 2 : GD_NOWHERE);
+                for (int j = 0; j < XC; ++j) {
+                    const int row = g + 4 * i, k = (wave + NW * j) * GD_KC + 8 * r16;
+                    xf[i][j] = gd_load(x_buf, row < M && k < K ? (unsigned)(row * a.ldx + k) * 2 : GD_NOWHERE);
+                }
             }
         }
-    }
-    if (a.norm_weight) {
-        const __amdgpu_buffer_rsrc_t nw_buf = gd_buffer(a.norm_weight, (unsigned)K * 2);
+        if (a.norm_weight) {
+            const __amdgpu_buffer_rsrc_t nw_buf = gd_buffer(a.norm_weight, (unsigned)K * 2);
 #pragma unroll
-        for (int j = 0; j < XC; ++j) nwf[j] = gd_load(nw_buf, (unsigned)((wave + NW * j) * GD_KC + 8 * r16) * 2);
-        // The sum of squares waits for the rows of every wave: no wave asks for weights before every wave has asked
-        // for its rows, or the last wave's rows would queue behind the others' weights.
-        __builtin_amdgcn_s_barrier();
+            for (int j = 0; j < XC; ++j) nwf[j] = gd_load(nw_buf, (unsigned)((wave + NW * j) * GD_KC + 8 * r16) * 2);
+            // The sum of squares waits for the rows of every wave: no wave asks for weights before every wave has asked
+            // for its rows, or the last wave's rows would queue behind the others' weights.
+            __builtin_amdgcn_s_barrier();
+        }
     }
 
     // ---- what a thread needs from memory to finish its places of a group of tiles
@@ -395,7 +529,7 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
             place_of(e, te, idx);
             const int per = PAIRS ? 8 : UPT;
             const int m = idx / per, u = u_begin + (tile0 + te) * UPT + idx % per;
-            gd_ask<EPI>(a, fin_bufs, te < NT && m < M && u < u_last, m, u, f[e]);
+            gd_ask<TOut, EPI>(a, fin_bufs, te < NT && m < M && u < u_last, m, u, f[e]);
         }
     };
     GdFinish fin[EPI_ROUNDS];
@@ -417,11 +551,19 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
     // (a wave issues in order and waits when the memory pipeline is full: with much more asked for here it would get to the norm
     // of its rows only after the pipeline has taken it all; q, k, v with the norm at 8 rows 5.68 microseconds with one item, 5.43 with
     // both; gate and up 9.8 with two, 11.9 with six)
+    // (the loop stands here twice: called from a function object in every kernel it left other registers, and a step of one row 1 % longer)
+    if constexpr (FROM) {
+        gd_rows_from_stream<XC, FROM>(a, sq_lds, xf, [&]() {
 #pragma unroll
-    for (int q = 0; q < FIRST; ++q) issue(ring[q], 0, q);
+            for (int q = 0; q < FIRST; ++q) issue(ring[q], 0, q);
+        });
+    } else {
+#pragma unroll
+        for (int q = 0; q < FIRST; ++q) issue(ring[q], 0, q);
+    }
 
     // ---- the rows of X, normed if asked, go to LDS: only this wave reads its chunks there
-    if (a.norm_weight) {
+    if (!FROM && a.norm_weight) {
         // sum of squares of a row: the lane's elements, the 16 lanes that hold the row's pieces of a chunk, then the
         // waves (in their order)
 #pragma unroll
@@ -560,7 +702,7 @@ __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_kernel(const Dec
 #define GR_NW 8
 
 template <typename TOut, int EPI, int XC, int RB, int NT, bool NORM, int LPI = 4>
-__global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(const DecodeGemmArgs a) {
+__global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(const GdArgs<TOut, EPI, 0> a) {
     constexpr int NW = GR_NW, SUMS = RB == 1 ? gd_sums(XC) : 1, NS = SUMS * NW;  // sums of the waves, as in the kernel above
     static_assert(!NORM || RB == 1, "the norm on the way in is for up to 16 rows");
     constexpr bool PAIRS = EPI == GD_SWIGLU || EPI == GD_ROPE_QKV;
@@ -618,7 +760,7 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
             int te, idx;
             place_of(e, te, idx);
             const int m = idx / UPT, u = u_begin + (tile0 + te) * UPT + idx % UPT;
-            gd_ask<EPI>(a, fin_bufs, te < NT && m < M && u < u_last, m, u, f[e]);
+            gd_ask<TOut, EPI>(a, fin_bufs, te < NT && m < M && u < u_last, m, u, f[e]);
         }
     };
     GdFinish fin[EPI_ROUNDS];
@@ -802,7 +944,7 @@ static void gd_launch_rows_long_k(int tiles, unsigned grid, DecodeGemmArgs& a, h
 // 9 to 16 rows whose K does not fit LDS: four, five or six chunks a wave.  LPI = 2: tiles of 8 weight rows, for a share whose last tile of 16
 // would be half empty (two load instructions less per chunk).
 template <typename TOut, int EPI, bool NORM, int LPI>
-static void gd_launch_rows_one_block(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
+static void gd_launch_rows_one_block(int chunks, int tiles, unsigned grid, GdArgs<TOut, EPI, 0>& a, hipStream_t stream) {
 #define GR_GO1(XC, NT)                                                                                              \
     do {                                                                                                            \
         a.groups = (tiles + NT - 1) / NT;                                                                           \
@@ -848,13 +990,13 @@ static int gd_launch_rows(int chunks, int rows, int tiles, bool low, unsigned gr
 }
 
 // `tiles`: tiles of the workgroup with the most units.
-template <typename TOut, int EPI, int LPI>
-static int gd_launch(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hipStream_t stream) {
+template <typename TOut, int EPI, int LPI, int FROM = 0>
+static int gd_launch(int chunks, int tiles, unsigned grid, GdArgs<TOut, EPI, FROM>& a, hipStream_t stream) {
 #define GD_GO(XC, NT)                                                                                            \
     do {                                                                                                         \
         static bool large_lds_allowed = false;                                                                   \
         if (!large_lds_allowed) {                                                                                \
-            LLMS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_decode_kernel<TOut, EPI, XC, LPI, NT>), \
+            LLMS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_decode_kernel<TOut, EPI, XC, LPI, NT, FROM>), \
                                                hipFuncAttributeMaxDynamicSharedMemorySize, GD_LDS));             \
             large_lds_allowed = true;                                                                            \
         }                                                                                                        \
@@ -863,7 +1005,7 @@ static int gd_launch(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hi
         const bool apart = GD_LDS_TILES + rest + sums <= GD_LDS;                                                 \
         a.sq_at = apart ? GD_LDS_TILES : gd_lds_tiles(XC, NT);                                                   \
         a.sums_at = apart ? GD_LDS_TILES + rest : 0;                                                             \
-        gemm_decode_kernel<TOut, EPI, XC, LPI, NT><<<grid, GD_NW * LLMS_WAVE, a.sq_at + rest + (apart ? sums : 0), stream>>>(a); \
+        gemm_decode_kernel<TOut, EPI, XC, LPI, NT, FROM><<<grid, GD_NW * LLMS_WAVE, a.sq_at + rest + (apart ? sums : 0), stream>>>(a); \
     } while (0)
     // tiles of a group: as few groups as possible, and then as few tiles that do not exist
     const int groups = (tiles + 3) / 4, nt = (tiles + groups - 1) / groups;
@@ -888,6 +1030,8 @@ static int gd_launch(int chunks, int tiles, unsigned grid, DecodeGemmArgs& a, hi
     } else if (chunks <= 4 * GD_NW) {
         if (tiles % 2) GD_GO(4, 1);
         else GD_GO(4, 2);
+    } else if constexpr (FROM != 0) {
+        LLMS_REQUIRE(false, "gemm_decode: rows from a stream are of up to 4,096 numbers");
     } else if (chunks <= 5 * GD_NW && (tiles % 2 == 0 || tiles > 5)) {
         GD_GO(5, 2);
     } else {
@@ -916,7 +1060,8 @@ int llms_gemm_decode_fits(int M, int K) {
 // epilogue: 0 plain (C [M,N] + bias; out_dtype 0 float32, 1 bfloat16), 1 gated (W = [gate; up] of `inter` rows each,
 // C [M, inter] bfloat16), 2 rotary q/k/v (W = [q; k; v], C = q [M, n_heads*head_dim] bfloat16, k and v stored at
 // `slots` when given; the angles as position times inv_freq, or their sines and cosines as `angles` [M][head_dim / 2][2],
-// or neither: no rotation), 3 residual (residual[M, N] += X W^T in place, bfloat16; C unused).
+// or neither: no rotation), 3 residual (residual[M, N] += X W^T in place, bfloat16, or with out_dtype 0 (up to 16 rows, no norm) float32 and
+// unrounded, times sigmoid(gate_z[m, gate_col + n] + gate_bias[n]) where gate_z is given; C unused).
 // norm_weight (bfloat16 [K]) given: the rows of X are replaced by RMSNorm(X) * norm_weight with `eps` on the way in.
 // unit: 0, or what is made of the sums instead: 1 (gated epilogue) the clamped unit with `limit`, 2 (plain) max(sum, 0)^2,
 // 3 (gated epilogue) gelu(gate) * up in 32-bit, rounded once (the tanh form).
@@ -927,7 +1072,8 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
                      const void* bias, const void* norm_weight, float eps, int M, int N, int K, int inter,
                      int n_heads, int n_kv_heads, int head_dim, int block_size, const float* inv_freq,
                      const float* angles, const int* positions, const int* slots, void* k_pool, void* v_pool,
-                     void* residual, int ldr, int workgroups, int k_parts, int unit, float limit, hipStream_t stream) {
+                     void* residual, int ldr, int workgroups, int k_parts, int unit, float limit, const float* gate_z, int ldz, int gate_col,
+                     const float* gate_bias, hipStream_t stream) {
     LLMS_REQUIRE(M > 0 && M <= 64 && N > 0 && K > 0, "gemm_decode: needs 1 <= M <= 64 and positive sizes");
     LLMS_REQUIRE((long long)N * K < (1ll << 30) && (long long)M * ldx < (1ll << 30), "gemm_decode: operands of 2 GB or more");
     const int x_rows = M <= 8 ? 8 : 16, x_pitch = (K + GD_KC - 1) / GD_KC * (GD_KC * 2) + 16;
@@ -941,11 +1087,23 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
     LLMS_REQUIRE(((uintptr_t)X % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)norm_weight % 16) == 0,
                  "gemm_decode: X, W and the norm's weight must be 16-byte aligned");
     LLMS_REQUIRE(epilogue >= 0 && epilogue <= 3, "gemm_decode: epilogue must be 0..3");
-    LLMS_REQUIRE(out_dtype == 1 || (out_dtype == 0 && epilogue == GD_PLAIN), "gemm_decode: 32-bit output goes with the plain epilogue");
+    LLMS_REQUIRE(out_dtype == 1 || (out_dtype == 0 && (epilogue == GD_PLAIN || (epilogue == GD_RESIDUAL && M <= 16))),
+                 "gemm_decode: 32-bit output goes with the plain epilogue, or the residual one of up to 16 rows");
+    LLMS_REQUIRE(gate_z == nullptr ? gate_bias == nullptr : epilogue == GD_RESIDUAL && out_dtype == 0 && gate_col >= 0 && (M == 1 || ldz >= gate_col + N) && ldz < (1 << 24) && gate_col < (1 << 24),
+                 "gemm_decode: a gate goes with a 32-bit residual");
     LLMS_REQUIRE(workgroups > 0 && workgroups <= 4096, "gemm_decode: bad number of workgroups");
-    DecodeGemmArgs a = {(const bf16*)W, (const bf16*)X, (const bf16*)bias, (const bf16*)norm_weight, eps, C, ldc, ldx,
+    DecodeStreamArgs all = {{(const bf16*)W, (const bf16*)X, (const bf16*)bias, (const bf16*)norm_weight, eps, C, ldc, ldx,
                         M, N, K, 0, 0, 0, 0, x_rows, x_pitch, inter, unit, limit, n_heads, n_kv_heads, head_dim, block_size, 0u, -1, inv_freq, angles, positions, slots,
-                        (bf16*)k_pool, (bf16*)v_pool, (bf16*)residual, ldr, K, 1, K, 0, 0};
+                        (bf16*)k_pool, (bf16*)v_pool, (bf16*)residual, ldr, K, 1, K, 0, 0}};
+    DecodeGemmArgs& a = all;
+    if (epilogue == GD_RESIDUAL && out_dtype == 0) {
+        all.residual = nullptr;
+        all.residual32 = (float*)residual;
+        all.gate_z = gate_z;
+        all.ldz = ldz;
+        all.gate_col = gate_col;
+        all.gate_bias = gate_bias;
+    }
     LLMS_REQUIRE(unit == 0 || ((unit == GD_UNIT_CLAMPED || unit == GD_UNIT_GELU) && epilogue == GD_SWIGLU) || (unit == GD_UNIT_RELU2 && epilogue == GD_PLAIN && k_parts == 1),
                  "gemm_decode: the clamped unit goes with the gated epilogue, the squared relu with the plain one");
     if (epilogue == GD_PLAIN) {
@@ -996,7 +1154,11 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
         const int tiles = pairs || low ? (most + 7) / 8 : (most + 15) / 16;
         if (epilogue == GD_SWIGLU) rc = gd_launch_rows<bf16, GD_SWIGLU>(chunks, M, tiles, low, grid, a, stream);
         else if (epilogue == GD_ROPE_QKV) rc = gd_launch_rows<bf16, GD_ROPE_QKV>(chunks, M, tiles, low, grid, a, stream);
-        else if (epilogue == GD_RESIDUAL) rc = gd_launch_rows<bf16, GD_RESIDUAL>(chunks, M, tiles, low, grid, a, stream);
+        else if (epilogue == GD_RESIDUAL && out_dtype == 0) {
+            rc = LLMS_OK;
+            if (low) gd_launch_rows_one_block<float, GD_RESIDUAL, false, 2>(chunks, tiles, grid, all, stream);
+            else gd_launch_rows_one_block<float, GD_RESIDUAL, false, 4>(chunks, tiles, grid, all, stream);
+        } else if (epilogue == GD_RESIDUAL) rc = gd_launch_rows<bf16, GD_RESIDUAL>(chunks, M, tiles, low, grid, a, stream);
         else if (out_dtype == 0) rc = gd_launch_rows<float, GD_PLAIN>(chunks, M, tiles, low, grid, a, stream);
         else rc = gd_launch_rows<bf16, GD_PLAIN>(chunks, M, tiles, low, grid, a, stream);
     } else if (epilogue == GD_SWIGLU) rc = gd_launch<bf16, GD_SWIGLU, 4>(chunks, (most + 7) / 8, grid, a, stream);
@@ -1006,7 +1168,10 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
         // two load instructions less per chunk
         const bool low = ((most + 7) / 8) % 2 == 1;
         const int tiles = low ? (most + 7) / 8 : (most + 15) / 16;
-        if (epilogue == GD_RESIDUAL) {
+        if (epilogue == GD_RESIDUAL && out_dtype == 0) {
+            if (low) rc = gd_launch<float, GD_RESIDUAL, 2>(chunks, tiles, grid, all, stream);
+            else rc = gd_launch<float, GD_RESIDUAL, 4>(chunks, tiles, grid, all, stream);
+        } else if (epilogue == GD_RESIDUAL) {
             if (low) rc = gd_launch<bf16, GD_RESIDUAL, 2>(chunks, tiles, grid, a, stream);
             else rc = gd_launch<bf16, GD_RESIDUAL, 4>(chunks, tiles, grid, a, stream);
         } else if (out_dtype == 0) {
@@ -1017,6 +1182,58 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
             else rc = gd_launch<bf16, GD_PLAIN, 4>(chunks, tiles, grid, a, stream);
         }
     }
+    if (rc != LLMS_OK) return rc;
+    LLMS_LAUNCH_CHECK();
+}
+
+// The product of up to 8 rows (K up to 4,096) that are made from a 32-bit stream x [M, K].  from 1: x + y / sqrt(mean(y^2) + eps) * w, rounded
+// to bfloat16, with that sum to x_out [M, K], which is not x (epilogue 0 with out_dtype 0, or 1).  from 2: x / sqrt(mean(x^2) + eps) *
+// (offset + w), rounded (epilogue 0 with out_dtype 0).  The product's rows go to h_out [M, K] if given.
+int llms_gemm_decode_stream(int out_dtype, int epilogue, void* C, int ldc, const void* W, const void* bias, int M, int N, int K, int inter, int unit,
+                            float limit, int from, const float* x, float* x_out, void* h_out, const float* y, const float* w, float offset,
+                            float eps, int workgroups, hipStream_t stream) {
+    LLMS_REQUIRE(M > 0 && M <= 8 && N > 0 && K > 0 && K % 8 == 0 && K <= 4 * GD_NW * GD_KC,
+                 "gemm_decode_stream: needs 1 <= M <= 8 and K a multiple of 8 up to 4,096");
+    LLMS_REQUIRE(from == GD_FROM_OPEN || from == GD_FROM_NORM, "gemm_decode_stream: from must be 1 or 2");
+    LLMS_REQUIRE((long long)N * K < (1ll << 30), "gemm_decode_stream: a weight of 2 GB or more");
+    LLMS_REQUIRE(C && W && x && w && (from == GD_FROM_NORM || (y && x_out && x_out != x)), "gemm_decode_stream: an operand is missing, or x_out is x");
+    LLMS_REQUIRE((uintptr_t)W % 16 == 0 && (uintptr_t)x_out % 16 == 0 && (uintptr_t)h_out % 16 == 0, "gemm_decode_stream: W and what is stored must be 16-byte aligned");
+    LLMS_REQUIRE((epilogue == GD_PLAIN && out_dtype == 0 && ldc >= N && unit == 0) ||
+                     (epilogue == GD_SWIGLU && out_dtype == 1 && from == GD_FROM_OPEN && inter > 0 && N == 2 * inter && ldc >= inter && !bias &&
+                      (unit == 0 || unit == GD_UNIT_CLAMPED || unit == GD_UNIT_GELU)),
+                 "gemm_decode_stream: 32-bit rows, or the gated epilogue with an open sum");
+    LLMS_REQUIRE(workgroups > 0 && workgroups <= 4096, "gemm_decode_stream: bad number of workgroups");
+    DecodeStreamArgs a{};
+    a.W = (const bf16*)W;
+    a.bias = (const bf16*)bias;
+    a.eps = eps;
+    a.C = C;
+    a.ldc = ldc;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.x_rows = 8;
+    a.x_pitch = (K + GD_KC - 1) / GD_KC * (GD_KC * 2) + 16;
+    a.inter = inter;
+    a.unit = unit;
+    a.limit = limit;
+    a.ldw = K;
+    a.k_parts = 1;
+    a.k_each = K;
+    a.from = DecodeStream{x, y, w, x_out, (bf16*)h_out, offset};
+    a.units = epilogue == GD_SWIGLU ? inter : N;
+    const int wgs = workgroups < a.units ? workgroups : a.units;
+    a.wgs_per_part = wgs;
+    a.units_each = a.units / wgs;
+    a.units_more = a.units % wgs;
+    const int most = a.units_each + (a.units_more ? 1 : 0), chunks = (K + GD_KC - 1) / GD_KC, tiles8 = (most + 7) / 8;
+    const bool low = tiles8 % 2 == 1;  // (as in llms_gemm_decode)
+    int rc;
+    if (epilogue == GD_SWIGLU) rc = gd_launch<bf16, GD_SWIGLU, 4, GD_FROM_OPEN>(chunks, tiles8, wgs, a, stream);
+    else if (from == GD_FROM_OPEN) rc = low ? gd_launch<float, GD_PLAIN, 2, GD_FROM_OPEN>(chunks, tiles8, wgs, a, stream)
+                                            : gd_launch<float, GD_PLAIN, 4, GD_FROM_OPEN>(chunks, (most + 15) / 16, wgs, a, stream);
+    else rc = low ? gd_launch<float, GD_PLAIN, 2, GD_FROM_NORM>(chunks, tiles8, wgs, a, stream)
+                  : gd_launch<float, GD_PLAIN, 4, GD_FROM_NORM>(chunks, (most + 15) / 16, wgs, a, stream);
     if (rc != LLMS_OK) return rc;
     LLMS_LAUNCH_CHECK();
 }

@@ -526,7 +526,7 @@ def gemm_decode_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
                 norm: tuple[torch.Tensor, float] | None = None, swiglu: bool = False, rope: dict | None = None,
                 residual: torch.Tensor | None = None, k_parts: int = 1, limit: float | None = None,
-                squared_relu: bool = False, gelu: bool = False) -> torch.Tensor:
+                squared_relu: bool = False, gelu: bool = False, gate: tuple | None = None) -> torch.Tensor:
     """The product for up to 64 bfloat16 rows with one workgroup per compute unit, and what surrounds it fused in.
 
     norm = (weight [K], eps): the rows of x are replaced by RMSNorm(x) * weight on the way in (up to 16 rows).
@@ -538,7 +538,8 @@ def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias
                are stored at the tokens' cache slots.  `angles` (rotary_angles(positions, inv_freq), float32
                [M, head_dim / 2, 2]) saves the kernel the sines and cosines; the result is the same to the bit.
     residual:  residual[M, N] += x w^T (+ bias) in place (32-bit sum of the rounded product and the row, rounded
-               once); `out` is not used and `residual` is returned.
+               once); `out` is not used and `residual` is returned.  A float32 residual (up to 16 rows, no norm) takes the sums
+               unrounded, with gate = (z, column, bias | None) times sigmoid(z[:, column : column + N] + bias), all float32.
     k_parts > 1 (17 to 64 rows, plain, no bias, no norm): K is shared out to that many sets of workgroups and `out` is
                float32 [k_parts, M, N], the parts' sums, for a norm to add up (gemm_decode_k_parts says how many
                parts a K needs)."""
@@ -607,24 +608,98 @@ def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias
         _dev(x, r["inv_freq"], r["angles"], r["positions"], r["slots"], r["k_pool"], r["v_pool"])
         epilogue, cols = 2, nh * d
     elif residual is not None:
+        wide = residual.dtype == torch.float32 and m <= GEMM_DECODE_NORM_ROWS and norm is None
         if (residual.dim() != 2 or residual.stride(1) != 1 or tuple(residual.shape) != (m, n)
-                or residual.dtype != torch.bfloat16):
-            raise ValueError(f"residual must be a bfloat16 [{m}, {n}] tensor with unit inner stride")
+                or not (residual.dtype == torch.bfloat16 or wide)):
+            raise ValueError(f"residual must be a bfloat16 [{m}, {n}] tensor with unit inner stride, or float32 (up to "
+                             f"{GEMM_DECODE_NORM_ROWS} rows, no norm)")
         epilogue = 3
+    gate_z, gate_col, gate_bias = (None, 0, None) if gate is None else gate
+    if gate is not None:
+        if epilogue != 3 or residual.dtype != torch.float32:
+            raise ValueError("a gate goes with a float32 residual")
+        if (gate_z.dim() != 2 or gate_z.stride(1) != 1 or gate_z.dtype != torch.float32 or gate_z.shape[0] != m
+                or not 0 <= gate_col <= gate_z.shape[1] - n):
+            raise ValueError(f"a gate's products must be float32 [{m}, columns] with unit inner stride and {n} columns from the gate's on")
+        if gate_bias is not None:
+            _f32(gate_bias, "the gate's bias", n)
+        _dev(x, gate_z, gate_bias)
     if epilogue != 3 and k_parts == 1:
         if out is None or out.dim() != 2 or out.stride(1) != 1 or tuple(out.shape) != (m, cols):
             raise ValueError(f"out must be 2-d [{m}, {cols}] with unit inner stride")
         if out.dtype != torch.bfloat16 and not (epilogue == 0 and out.dtype == torch.float32):
             raise ValueError("gemm_decode stores bfloat16 (the plain epilogue also float32)")
     _check(load("gemm_decode").llms_gemm_decode(
-        c_int(1 if epilogue == 3 else _code(out)), c_int(epilogue), _ptr(None if epilogue == 3 else out),
+        c_int(_code(residual if epilogue == 3 else out)), c_int(epilogue), _ptr(None if epilogue == 3 else out),
         c_int(0 if epilogue == 3 else out.stride(-2)), _ptr(x), c_int(x.stride(0)), _ptr(w), _ptr(bias),
         _ptr(norm_weight), c_float(eps), c_int(m), c_int(n), c_int(k), c_int(inter), c_int(r["n_heads"]),
         c_int(r["n_kv_heads"]), c_int(r["head_dim"]), c_int(r["block_size"]), _ptr(r["inv_freq"]), _ptr(r["angles"]), _ptr(r["positions"]),
         _ptr(r["slots"]), _ptr(r["k_pool"]), _ptr(r["v_pool"]), _ptr(residual),
         c_int(residual.stride(0) if residual is not None else 0), c_int(compute_units(dev)), c_int(k_parts),
-        c_int(2 if squared_relu else _gated_unit(limit, gelu)), c_float(limit or 0.0), _stream(dev)), "gemm_decode")
+        c_int(2 if squared_relu else _gated_unit(limit, gelu)), c_float(limit or 0.0), _ptr(gate_z), c_int(_row_stride(gate_z)),
+        c_int(gate_col), _ptr(gate_bias), _stream(dev)), "gemm_decode")
     return residual if epilogue == 3 else out
+
+
+# Up to how many rows, and of how many numbers, ops.gemm_decode_stream takes: a row of 2,048 costs every workgroup 8 or, with what
+# joins it, 16 KB from L2, which the kernel of some 4.3 microseconds that it stands for stops being worth.
+GEMM_DECODE_STREAM_ROWS = 8
+GEMM_DECODE_STREAM_K = 4096
+
+
+def _row_stride(t: torch.Tensor | None) -> int:
+    """Elements from row to row (of one row: its length, whatever the tensor says)."""
+    return 0 if t is None else t.stride(0) if t.shape[0] > 1 else t.shape[1]
+
+
+def gemm_decode_stream_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ops.gemm_decode_stream takes the float32 rows x [N, K] against the bfloat16 weight w."""
+    n, k = x.shape
+    return (0 < n <= GEMM_DECODE_STREAM_ROWS and x.dtype == torch.float32 and x.is_contiguous() and w.dtype == torch.bfloat16
+            and w.is_contiguous() and w.data_ptr() % 16 == 0 and w.shape[1] == k and k % 8 == 0 and 0 < k <= GEMM_DECODE_STREAM_K
+            and 0 < w.numel() < 1 << 30)
+
+
+def gemm_decode_stream(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, *,
+                       joins: tuple[torch.Tensor, torch.Tensor, float, torch.Tensor] | None = None,
+                       norm: tuple[torch.Tensor, float, float] | None = None, h_out: torch.Tensor | None = None, swiglu: bool = False,
+                       limit: float | None = None, gelu: bool = False) -> torch.Tensor:
+    """`gemm_decode` of up to 8 rows that the product makes from a float32 stream x [N, K] on its way in:
+
+    joins = (y, y_weight, y_eps, x_out): the stream's open sum is closed, as `normed_add_norm` does without a norm behind it: the rows are
+            bf16(x + y / sqrt(mean(y^2) + y_eps) * y_weight); that sum goes to x_out (another tensor: x stays as it is).
+    norm = (weight, eps, offset): the rows are `rmsnorm32` of x.
+    h_out (bfloat16 [N, K]): takes the rows, for who else reads them.
+    out: float32 [N, rows of w] (+ bias), or with `swiglu` (with `joins`) bfloat16 as for `gemm_decode`."""
+    (n, k), cols = x.shape, w.shape[0] // 2 if swiglu else w.shape[0]
+    if (joins is None) == (norm is None):
+        raise ValueError("either joins or norm")
+    y, weight, eps, x_out = joins if joins is not None else (None, norm[0], norm[1], None)
+    for t, what, dtype in ((x, "x", torch.float32), (y, "y", torch.float32), (x_out, "x_out", torch.float32), (h_out, "h_out", torch.bfloat16)):
+        if t is not None and (t.dtype != dtype or tuple(t.shape) != (n, k) or not t.is_contiguous()):
+            raise ValueError(f"{what} must be a contiguous {dtype} [{n}, {k}] tensor")
+    if x_out is not None and x_out.data_ptr() == x.data_ptr():
+        raise ValueError("x_out must not be x, which every workgroup reads")
+    _f32(weight, "weight", k)
+    _rows(w, "w", k)
+    if not gemm_decode_stream_supported(x, w):
+        raise ValueError(f"gemm_decode_stream takes up to {GEMM_DECODE_STREAM_ROWS} rows of up to {GEMM_DECODE_STREAM_K} numbers (multiples "
+                         "of 8) against an aligned bfloat16 weight")
+    if bias is not None and (swiglu or bias.dtype != torch.bfloat16 or bias.numel() != w.shape[0] or not bias.is_contiguous()):
+        raise ValueError("bias must be a contiguous bfloat16 vector of N elements (none for the gated epilogue)")
+    if swiglu and (joins is None or w.shape[0] % 2):
+        raise ValueError("the gated epilogue goes with an open sum and an even number of weight rows")
+    if (limit is not None or gelu) and not swiglu:
+        raise ValueError("a limit and gelu go with the gated epilogue")
+    if out.dim() != 2 or out.stride(1) != 1 or tuple(out.shape) != (n, cols) or out.dtype != (torch.bfloat16 if swiglu else torch.float32):
+        raise ValueError(f"out must be [{n}, {cols}] with unit inner stride, float32 or for the gated epilogue bfloat16")
+    dev = _dev(out, x, w, bias, y, x_out, weight, h_out)
+    _check(load("gemm_decode").llms_gemm_decode_stream(
+        c_int(1 if swiglu else 0), c_int(1 if swiglu else 0), _ptr(out), c_int(_row_stride(out)), _ptr(w), _ptr(bias), c_int(n),
+        c_int(w.shape[0]), c_int(k), c_int(cols if swiglu else 0), c_int(_gated_unit(limit, gelu) if swiglu else 0), c_float(limit or 0.0),
+        c_int(1 if joins is not None else 2), _ptr(x), _ptr(x_out), _ptr(h_out), _ptr(y), _ptr(weight),
+        c_float(0.0 if norm is None else norm[2]), c_float(eps), c_int(compute_units(dev)), _stream(dev)), "gemm_decode_stream")
+    return out
 
 
 SLICE_K = 512  # what one workgroup of gemm_slices takes of K

@@ -129,6 +129,7 @@ def _fill_talk(shape, generator, device, options):
 @register_mixer("composed_attention")
 class ComposedAttention(Mixer):
     graph_safe = True
+    accepts_joined_rows = True  # (its input meets one product, which comes first)
 
     def __init__(self, spec, ctx):
         super().__init__(spec, ctx)
@@ -329,7 +330,9 @@ class ComposedAttention(Mixer):
     def input_weight(self, weight):
         self.qkv_weight = weight
 
-    def forward(self, x, batch, cache, projected=None):
+    adds_to_stream_by = "o_weight"
+
+    def forward(self, x, batch, cache, projected=None, joins=None):
         paged, state = cache if isinstance(cache, tuple) else (cache, None)
         view = batch.groups[paged.group_id]
         heads, kv, dk, dv = self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim
@@ -348,7 +351,7 @@ class ComposedAttention(Mixer):
                            norm_first=self.norm_first, q_scale=self.temp, values_from_keys=self.values_from_keys, joint=self.joint_norm, bias=self.late_bias)
             out = torch.empty((proj.shape[0], heads * dv), dtype=x.dtype, device=x.device)
             self.attend(out, q, paged, view, batch, gate)
-            return linear(out, self.o_weight, out_dtype=self.result_dtype)
+            return self._result(out, joins)
         if self.output_gate:
             proj = proj[:, : self.cq + self.ck + self.cv]
         conv, taps = self.taps > 1, self.taps > 0  # (one tap is a factor per channel and needs no state)
@@ -364,7 +367,10 @@ class ComposedAttention(Mixer):
             ops.conv_state(state.state, proj, batch.state_slots, batch.cu_seqlens, batch.context_lens)
         out = torch.empty((proj.shape[0], heads * dv), dtype=x.dtype, device=x.device)
         self.attend(out, q, paged, view, batch, gate)
-        return linear(out, self.o_weight, out_dtype=self.result_dtype)
+        return self._result(out, joins)
+
+    def _result(self, out, joins):
+        return linear(out, self.o_weight, out_dtype=self.result_dtype) if joins is None else joins.add(out, self.o_weight)
 
     def attend(self, out, q, paged, view, batch, gate=None):
         """out[n] = this attention of token n's heads over its request's pages: on the matrix cores where the

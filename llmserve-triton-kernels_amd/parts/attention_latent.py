@@ -44,6 +44,7 @@ _DEFAULT_NAMES = {"dq": "dq", "dq_norm": "dq.norm", "uq": "uq", "q": "q", "sink"
 @register_mixer("latent_attention")
 class LatentAttention(Mixer):
     graph_safe = True
+    accepts_joined_rows = True  # (its input meets one product, which comes first)
 
     def __init__(self, spec, ctx):
         super().__init__(spec, ctx)

@@ -30,8 +30,8 @@ from __future__ import annotations
 import torch
 
 from ..ops import library as ops
-from .linear import linear
-from .registry import ADDED_IN_PLACE, Block, DeferredNorm, GatedSum, NormedSum, OpenStreams, register_block
+from .linear import adds_to_stream, linear, takes_stream
+from .registry import ADDED_IN_PLACE, Block, DeferredNorm, GatedStream, GatedSum, JoinedRows, NormedSum, OpenStreams, register_block
 
 
 @register_block("prenorm")
@@ -84,16 +84,47 @@ class ParallelBlock(Block):
                 self._mixer_columns = (b, self._stacked.shape[0])
         return True
 
+    def _columns(self, out):
+        """What the product with the stacked weights holds: (column of the mixer's gate, of the feed-forward's, the mixer's input or None)."""
+        projected = None
+        if self._mixer_columns is not None:
+            projected = out[:, self._mixer_columns[0]: self._mixer_columns[1]]
+        return 0, self.mixer_gate.weight.shape[0], projected
+
+    def _adds_by_products(self, x):
+        """Whether the branches' last products add to the stream themselves, each times its gate, and the product of the gates norms the
+        stream on its way in or behind the norm's kernel: few rows (a rule by sizes alone, the same for every layer of a kind)."""
+        parts = [self.mixer] if getattr(self.feed_forward, "absent", False) else [self.mixer, self.feed_forward]
+        last = [getattr(p, p.adds_to_stream_by) if p.adds_to_stream_by and p.result_dtype == torch.float32 else None for p in parts]
+        return (x.is_contiguous() and getattr(self.norm, "closes_gated_sums", False) and self.norm.ctx.dtype == torch.bfloat16
+                and all(w is not None and adds_to_stream(x.shape[0], w) for w in last) and self._stack())
+
+    def _few_rows(self, x, batch, cache):
+        """The layer where every sum into x is a product's epilogue."""
+        norm = self.norm
+        if takes_stream(x, self._stacked):
+            h = torch.empty(x.shape, dtype=norm.ctx.dtype, device=x.device)
+            z = torch.empty((x.shape[0], self._stacked.shape[0]), dtype=torch.float32, device=x.device)
+            ops.gemm_decode_stream(z, x, self._stacked, norm=(norm.weight, norm.eps, norm.offset), h_out=h)
+        else:
+            h = norm.forward(x)
+            z = linear(h, self._stacked, out_dtype=torch.float32)
+        col_m, col_f, projected = self._columns(z)
+        extra = {} if projected is None else {"projected": projected}
+        results = [self.mixer.forward(h, batch, cache, joins=GatedStream(x, z, col_m, self.mixer_gate.bias), **extra)]
+        if not getattr(self.feed_forward, "absent", False):
+            results.append(self.feed_forward.forward(h, joins=GatedStream(x, z, col_f, self.feed_forward_gate.bias)))
+        if any(y is not ADDED_IN_PLACE for y in results):
+            raise RuntimeError("a branch took a stream to add to and did not")
+        return x
+
     def _gate_products(self, h):
         """(products [N, columns] or None, column of the mixer's gate or None, column of the feed-forward's,
         the mixer's projected input or None)."""
         gm, gf = self.mixer_gate, self.feed_forward_gate
         if self._stack():  # one product for all
             out = linear(h, self._stacked, out_dtype=torch.float32)
-            projected = None
-            if self._mixer_columns is not None:
-                projected = out[:, self._mixer_columns[0]: self._mixer_columns[1]]
-            return out, 0, gm.weight.shape[0], projected
+            return out, *self._columns(out)
         zm, zf = gm.products(h), gf.products(h)
         if zm is not None and zf is not None:
             return torch.cat([zm, zf], dim=1), 0, zm.shape[1], None
@@ -103,6 +134,8 @@ class ParallelBlock(Block):
     def forward(self, x, delta, batch, cache):
         if x.dtype != torch.float32:
             raise ValueError("the parallel arrangement keeps a 32-bit residual stream")
+        if delta is None and self._adds_by_products(x):
+            return self._few_rows(x, batch, cache), None
         # (the layer before may have left its gated sum open: this layer's norm closes it in its own kernel)
         h = self.norm.add_norm(x, delta)
         z, col_m, col_f, projected = self._gate_products(h)
@@ -188,27 +221,47 @@ class PostNormBlock(Block):
 
     ROLES = {"mixer": "mixer", "feed_forward": "feed_forward", "mixer_post_norm": "norm", "feed_forward_post_norm": "norm"}
 
-    def _read(self, x, delta):
-        """(the sublayer's input, the stream after the open sum `delta`)"""
+    def _read(self, x, delta, takes_joined: bool):
+        """(the sublayer's input, the stream [N, hidden] after the open sum `delta` as far as it is known: `_after`)"""
         if x.dtype != torch.float32 or (x.dim() == 3 and x.shape[1] != 1):
             raise ValueError("the postnorm arrangement keeps one 32-bit stream")
         if delta is not None and not isinstance(delta, NormedSum):
             raise ValueError("the postnorm arrangement closes a sum through a norm or nothing")
         rows = x.view(x.shape[0], x.shape[-1])
-        joins = {} if delta is None else {"y": delta.y, "y_weight": delta.weight, "y_eps": delta.eps}
         dtype = self.mixer.ctx.dtype
         if dtype == torch.float32:  # (the stream itself is the input: the next sum comes after the sublayer has read it)
-            if joins:
-                ops.normed_add_norm(None, rows, None, 0.0, **joins)
-            return rows, x
-        return ops.normed_add_norm(torch.empty(rows.shape, dtype=dtype, device=x.device), rows, None, 0.0, **joins), x
+            if delta is not None:
+                ops.normed_add_norm(None, rows, None, 0.0, **self._joins(delta))
+            return rows, rows
+        if delta is not None and takes_joined:
+            return JoinedRows(rows, delta, dtype, self._close), rows
+        return self._close(rows, delta, dtype), rows
+
+    @staticmethod
+    def _joins(delta):
+        return {} if delta is None else {"y": delta.y, "y_weight": delta.weight, "y_eps": delta.eps}
+
+    @classmethod
+    def _close(cls, rows, delta, dtype):
+        """The rows rounded once, after `delta` has been added to them in place."""
+        return ops.normed_add_norm(torch.empty(rows.shape, dtype=dtype, device=rows.device), rows, None, 0.0, **cls._joins(delta))
+
+    @staticmethod
+    def _after(h, rows, x, part):
+        """The stream behind the sublayer that read `h`, in x's shape."""
+        if isinstance(h, JoinedRows):
+            if not h.resolved:
+                raise RuntimeError(f"{type(part).__name__} took an input whose sum is open and left it unresolved")
+            rows = h.stream
+        return rows.view(x.shape)
 
     def forward(self, x, delta, batch, cache):
-        h, x = self._read(x, delta)
+        h, rows = self._read(x, delta, self.mixer.accepts_joined_rows)
         y, post = self.mixer.forward(h, batch, cache), self.mixer_post_norm
+        x = self._after(h, rows, x, self.mixer)
         delta = NormedSum(StreamsBlock._result(y), post.weight, post.eps)
         if getattr(self.feed_forward, "absent", False):
             return x, delta
-        h, x = self._read(x, delta)
+        h, rows = self._read(x, delta, self.feed_forward.accepts_joined_rows)
         y, post = self.feed_forward.forward(h), self.feed_forward_post_norm
-        return x, NormedSum(StreamsBlock._result(y), post.weight, post.eps)
+        return self._after(h, rows, x, self.feed_forward), NormedSum(StreamsBlock._result(y), post.weight, post.eps)

@@ -31,6 +31,7 @@ import os
 import torch
 
 from ..ops import library as ops
+from .registry import JoinedRows
 
 OWN_KERNELS_ONLY = os.environ.get("LLMSERVE_GEMM", "") == "own"
 
@@ -231,13 +232,45 @@ def _tiles_take(out: torch.Tensor, bias: torch.Tensor | None, n: int) -> bool:
             (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous() and bias.shape == (n,))))
 
 
+def takes_stream(stream: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the product of few rows against `weight` makes them from a 32-bit stream on its way in (ops.gemm_decode_stream), and not behind
+    a kernel that does: a launch less, where the product is ops.gemm_decode's anyway."""
+    m, (n, k) = stream.shape[0], weight.shape
+    return (DECODE_KERNEL and ops.gemm_decode_stream_supported(stream, weight) and ops.gemm_decode_fits(m, k)
+            and not streams_large(m, n, k, ops.compute_units(stream.device)))
+
+
+def joined_product(x, weight: torch.Tensor, out: torch.Tensor, bias: torch.Tensor | None = None, **epilogue) -> bool:
+    """The product of `JoinedRows` x into `out` (float32, or bfloat16 with the gated `epilogue`) with x's sum closed on the way in, where that is
+    done; False, with nothing done, otherwise."""
+    if x.dtype != torch.bfloat16 or not takes_stream(x.stream, weight):
+        return False
+    stream = torch.empty_like(x.stream)
+    ops.gemm_decode_stream(out, x.stream, weight, bias, joins=(x.delta.y, x.delta.weight, x.delta.eps, stream), **epilogue)
+    x.resolve(stream)
+    return True
+
+
+def adds_to_stream(rows: int, weight: torch.Tensor) -> bool:
+    """Whether the product of `rows` bfloat16 rows against `weight` adds its result, times its gate, to a 32-bit stream in its epilogue
+    (`GatedStream.add`): where it is ops.gemm_decode's and the norm behind the sum is no kernel of its own, or one that adds nothing up."""
+    return (DECODE_KERNEL and 0 < rows <= ops.GEMM_DECODE_NORM_ROWS and weight.dtype == torch.bfloat16 and weight.is_contiguous()
+            and weight.data_ptr() % 16 == 0 and weight.shape[1] % 8 == 0 and 0 < weight.numel() < 1 << 30
+            and ops.gemm_decode_fits(rows, weight.shape[1]))
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None,
            out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None, from_cache: bool = False) -> torch.Tensor:
-    """x [M, K] (unit inner stride), weight [N, K] -> [M, N] in out_dtype (default: x's).  `from_cache`: as for ops.gemm_tiles."""
+    """x [M, K] (unit inner stride; or `JoinedRows`), weight [N, K] -> [M, N] in out_dtype (default: x's).  `from_cache`: as for
+    ops.gemm_tiles."""
     out_dtype = out_dtype or x.dtype
     m, n = x.shape[0], weight.shape[0]
     if out is None:
         out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+    if isinstance(x, JoinedRows):
+        if out.dtype == torch.float32 and joined_product(x, weight, out, bias):
+            return out
+        x = x.materialize()
     if m == 0:
         return out
     if x.dtype == torch.bfloat16 and ops.gemm_bf16_supported(x, weight):

@@ -113,6 +113,24 @@ class GatedSum:
 
 
 @dataclass
+class GatedStream:
+    """Where a branch's result y goes with few rows: `stream` += g * y in the epilogue of y's last product, g by the columns of the gates' products
+    z [N, columns] from `column` on, and `bias` (`column` None: 1).  The branch returns `ADDED_IN_PLACE` then.  The stream is 32-bit."""
+
+    stream: torch.Tensor
+    z: "torch.Tensor | None"
+    column: "int | None"
+    bias: "torch.Tensor | None"
+
+    def add(self, x: torch.Tensor, weight: torch.Tensor):
+        from ..ops import library as ops
+
+        gate = None if self.column is None else (self.z, self.column, self.bias)
+        ops.gemm_decode(None, x, weight, residual=self.stream, gate=gate)
+        return ADDED_IN_PLACE
+
+
+@dataclass
 class OpenStreams:
     """A write into a residual stream of several copies that is still open: new_t = sum_s mix[s, t] x_s + write[t] y,
     with the coefficients of `connection` (a `Connection`).  It travels in the place of `delta`; a norm that sets
@@ -131,6 +149,33 @@ class NormedSum:
     y: torch.Tensor
     weight: torch.Tensor
     eps: float
+
+
+class JoinedRows:
+    """The input of a sublayer before it is computed: the rows of a 32-bit stream [N, hidden] after the open sum `delta` (a `NormedSum`),
+    rounded once to `dtype`.  Its consumer either calls `materialize()` or closes the sum in the first product's kernel
+    (`linear.joined_product`, which calls `resolve`).  Afterwards `stream` is the stream with its sum closed.  A part that sets
+    `accepts_joined_rows` is handed this in the place of a tensor."""
+
+    def __init__(self, stream: torch.Tensor, delta: NormedSum, dtype: torch.dtype, close: Callable):
+        self.stream = stream
+        self.delta = delta
+        self.dtype = dtype
+        self.shape = stream.shape
+        self.device = stream.device
+        self.resolved = False
+        self._close = close  # (stream, delta, dtype) -> the rows, with the sum added to the stream in place
+
+    def materialize(self) -> torch.Tensor:
+        rows = self._close(self.stream, self.delta, self.dtype)
+        self.resolve(self.stream)
+        return rows
+
+    def resolve(self, stream: torch.Tensor) -> None:
+        if self.resolved:
+            raise RuntimeError("this input was already consumed")
+        self.resolved = True
+        self.stream = stream
 
 
 def as_tensor(delta):
@@ -203,6 +248,9 @@ class Mixer(Part):
     the arrangement formed together with products of its own."""
 
     accepts_deferred_norm = False
+    accepts_joined_rows = False
+    # the weight of the last product, where `forward(..., joins=GatedStream)` leaves the sum to that product: a name, or None
+    adds_to_stream_by = None
 
     def cache_spec(self) -> PagedCacheSpec | StateCacheSpec | None:
         return None
@@ -213,6 +261,8 @@ class Mixer(Part):
 
 class FeedForward(Part):
     accepts_deferred_norm = False
+    accepts_joined_rows = False
+    adds_to_stream_by = None  # as a mixer's
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         raise NotImplementedError

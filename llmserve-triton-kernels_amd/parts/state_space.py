@@ -43,6 +43,7 @@ def _fill_rates(shape, generator, device, options):
 @register_mixer("state_space")
 class StateSpace(Mixer):
     graph_safe = True
+    accepts_joined_rows = True  # (its input meets one product, which comes first)
     SCAN_UP_TO = 16  # new tokens of the longest portion up to which the recurrence runs token by token
 
     def __init__(self, spec, ctx):

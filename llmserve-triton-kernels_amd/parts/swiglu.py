@@ -12,8 +12,8 @@ from __future__ import annotations
 import torch
 
 from ..ops import library as ops
-from .linear import adds_residual_in_epilogue, brings_near, decode_product, few_rows, linear, linear_partial_sums, tiles_product
-from .registry import ADDED_IN_PLACE, DeferredNorm, FeedForward, register_feed_forward
+from .linear import adds_residual_in_epilogue, brings_near, decode_product, few_rows, joined_product, linear, linear_partial_sums, tiles_product
+from .registry import ADDED_IN_PLACE, DeferredNorm, FeedForward, JoinedRows, register_feed_forward
 from .spec import ParamInfo
 
 
@@ -21,6 +21,7 @@ from .spec import ParamInfo
 class SwiGLU(FeedForward):
     graph_safe = True
     accepts_deferred_norm = True
+    accepts_joined_rows = True
 
     def __init__(self, spec, ctx):
         super().__init__(spec, ctx)
@@ -48,14 +49,20 @@ class SwiGLU(FeedForward):
         self.gate_up = torch.cat([tensors[self.names["gate"]], tensors[self.names["up"]]], dim=0).contiguous()
         self.down = tensors[self.names["down"]].contiguous()
 
-    def forward(self, x):
+    adds_to_stream_by = "down"
+
+    def forward(self, x, joins=None):
         deferred = isinstance(x, DeferredNorm)  # the caller hands the result to a norm, which takes partial sums
         rows = x.residual if deferred else x
         m = rows.shape[0]
         dtype, device = self.gate_up.dtype, self.gate_up.device
         act = torch.empty((m, self.intermediate), dtype=dtype, device=device)
         near = False
-        if decode_product(rows, self.gate_up):
+        if isinstance(x, JoinedRows):
+            rows = None if joined_product(x, self.gate_up, act, swiglu=True, limit=self.limit, gelu=self.gelu) else x.materialize()
+        if rows is None:
+            pass  # (done)
+        elif decode_product(rows, self.gate_up):
             norm = x.fused() if deferred and m <= ops.GEMM_DECODE_NORM_ROWS else None
             if norm is not None:
                 x.resolve(None)  # nothing is left to add: the kernel norms the residual rows as they are
@@ -76,6 +83,8 @@ class SwiGLU(FeedForward):
                 ops.gemm32_gated(act, rows, self.gate_up)  # the same, in 32-bit
             else:
                 ops.silu_mul(act, linear(rows, self.gate_up), self.limit, self.gelu)
+        if joins is not None:
+            return joins.add(act, self.down)
         if deferred and x.may_add_in_place and adds_residual_in_epilogue(act, self.down):
             ops.gemm_decode(None, act, self.down, residual=x.residual)  # the residual sum in the product's epilogue
             return ADDED_IN_PLACE
@@ -90,5 +99,5 @@ class NoFeedForward(FeedForward):
     graph_safe = True
     absent = True
 
-    def forward(self, x):
+    def forward(self, x, joins=None):
         return None
