@@ -16,7 +16,7 @@ from pathlib import Path
 
 import torch
 
-from ..cache.manager import CacheManager, group_layers
+from ..cache.manager import CacheManager, StepLayout, group_layers
 from ..cache.storage import CacheStorage, pool_sizes_for_budget
 from ..config.engine_config import EngineConfig
 from ..config.registry import architecture_of, read_config
@@ -28,6 +28,14 @@ from ..weights.random import random_tensors
 from .batch import BatchUploader, StaticDecodeBatch, StaticStepBatch, build_batch
 
 _TORCH_DTYPES = {"bfloat16": torch.bfloat16, "float32": torch.float32}
+
+
+def _pow2(x: int, least: int = 1) -> int:
+    """The first of least, 2 least, 4 least, ... that is not below x."""
+    p = least
+    while p < x:
+        p *= 2
+    return p
 
 
 @dataclass
@@ -299,14 +307,48 @@ class ModelRunner:
     @classmethod
     def _step_shape(cls, n_decode: int, n_prefill: int, n_prefill_tokens: int, n_logits: int, context: int) -> tuple:
         """The sizes a step is padded to: powers of two for the requests, the wanted rows and the reach of
-        the contexts (which only sets how attention spreads its work), `_row_bucket` for the rows of the portions."""
-        def pow2(x, least=1):
-            p = least
-            while p < x:
-                p *= 2
-            return p
-        return (pow2(n_decode) if n_decode else 0, pow2(n_prefill), cls._row_bucket(n_prefill_tokens),
-                pow2(max(n_logits, 1)), pow2(context, 256))
+        the contexts (which only sets how attention spreads its work), `_row_bucket` for the rows of the portions, alone or with
+        the single tokens in front of them, whichever leaves fewer."""
+        decode = _pow2(n_decode) if n_decode else 0
+        rows = min(cls._row_bucket(n_prefill_tokens), cls._row_bucket(decode + n_prefill_tokens) - decode)
+        return (decode, _pow2(n_prefill), rows, _pow2(max(n_logits, 1)), _pow2(context, 256))
+
+    @classmethod
+    def _spare_rows_filled(cls, layout, tokens: list[list[int]], logit_rows: list[int]):
+        """The same step with the first tokens of its longest portion in the places that a power of two of single tokens leaves empty, where
+        that leaves fewer rows: (layout, tokens, logit_rows).  A token attends to the keys up to its own place, which all are stored
+        before, so for layers that keep keys and nothing else a portion may be cut anywhere.  A step of 512 tokens, 3 of them
+        decoding, has 512 rows so, and 516 otherwise, and one row past 512 takes the four products of a layer of the 1.1B shape from 60.6
+        microseconds to 68.4."""
+        counts = layout.counts
+        n_dec = next((i for i, c in enumerate(counts) if c != 1), len(counts))
+        if not 0 < n_dec < len(counts):
+            return layout, tokens, logit_rows
+        total = sum(counts[n_dec:])
+        longest = max(range(n_dec, len(counts)), key=lambda i: counts[i])
+        moved = min(_pow2(n_dec) - n_dec, counts[longest] - 2)  # (a portion stays one)
+
+        def rows_with(m):
+            decode, _, rows, *_ = cls._step_shape(n_dec + m, 1, total - m, 1, 1)
+            return decode + rows
+
+        if moved <= 0 or rows_with(moved) >= rows_with(0):
+            return layout, tokens, logit_rows
+        at = n_dec + sum(counts[n_dec:longest])  # the portion's first row
+        order = [*range(n_dec), *range(at, at + moved), *range(n_dec, at), *range(at + moved, n_dec + total)]
+        place = {row: i for i, row in enumerate(order)}
+
+        def each(values, cut, rest):  # of every request: the singles', the moved tokens', the portions' with the longest one's rest
+            return [*values[:n_dec], *cut, *values[n_dec:longest], rest, *values[longest + 1:]]
+
+        start, slot, seq = layout.starts[longest], layout.state_slots[longest], layout.seq_ids[longest]
+        filled = StepLayout(
+            seq_ids=each(layout.seq_ids, [seq] * moved, seq), counts=each(counts, [1] * moved, counts[longest] - moved),
+            starts=each(layout.starts, range(start, start + moved), start + moved), state_slots=each(layout.state_slots, [slot] * moved, slot),
+            fresh_slots=layout.fresh_slots, slots={g: [s[row] for row in order] for g, s in layout.slots.items()},
+            table_updates=layout.table_updates)
+        own = tokens[longest]
+        return filled, each(tokens, [[t] for t in own[:moved]], own[moved:]), [place[row] for row in logit_rows]
 
     def _shape_of(self, layout, n_logits: int) -> tuple:
         n_dec = 0
@@ -322,6 +364,8 @@ class ModelRunner:
         from then on.  Which kernels run, and in which arrangement, is therefore a function of the bucket
         alone: the first run and every replay give the same bits, and so do two runs of one trace.
         Returns (logits, whether the caller owns them)."""
+        if len(self.manager.paged_groups) == len(self.manager.groups):  # (no layer keeps a state that a portion runs through)
+            layout, tokens, logit_rows = self._spare_rows_filled(layout, tokens, logit_rows)
         shape = self._shape_of(layout, len(logit_rows))
         bucket = self._buckets.pop(shape, None)
         if bucket is None:
