@@ -903,6 +903,99 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
     finish_group(tile0);
 }
 
+// Up to 16 rows of any K whose result is added to the residual rows (down_proj of larger shapes: 4096 x 11008).  A share of such a weight is a
+// tile or two of 16 rows, so the rows of X are needed once or twice and need not stay: a chunk of them comes with the weights' (XL loads
+// of 4 rows, from L2) and goes through a tile of its own in LDS.  The waves share K out as above, two items each in flight; the loop is
+// over four items, whose sums stay apart (a sum has no more terms than where K was shared out to workgroups), so K is not a constant of the kernel.
+// 4096 x 11008 with the residual's sum 18.5, 19.4 and 20.8 microseconds at 1, 8 and 16 rows, and the norm behind it goes into the next product;
+// gemm_stream, which leaves partial sums, and the norm that adds them up 21.4, 23.4 and 26.8.  8192 x 28672 75.5 and 78.9 at 1 and 8 rows (6.2 TB/s),
+// 85.9 and 93.3.  What bounds it: memory, and with 16 rows the rows of X beside it.
+#define GL_SUMS 4
+template <int LPI, int XL>
+__global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_long_kernel(const DecodeGemmArgs a) {
+    constexpr int NW = GD_NW, NS = GL_SUMS * NW, UPT = 4 * LPI, RING = 2, THREADS = NW * LLMS_WAVE, PLACES = 16 * UPT;
+    static_assert(PLACES <= THREADS, "a thread per place");
+    __shared__ u32x4 w_lds[NW * 16 * (GD_KC / 8)], x_lds[NW * 16 * (GD_KC / 8)];
+    __shared__ __attribute__((aligned(16))) float red[NS * LLMS_WAVE * 4];  // [sum][lane][4]
+    const int tid = threadIdx.x, wave = tid / LLMS_WAVE, lane = tid % LLMS_WAVE, r16 = lane % 16, g = lane / 16;
+    const int M = a.M, K = a.K, n_chunks = (K + GD_KC - 1) / GD_KC, wg = blockIdx.x;
+    const int per = ((n_chunks + NW - 1) / NW + GL_SUMS - 1) / GL_SUMS * GL_SUMS;  // items of a tile; those beyond K are nowhere
+    const int u_begin = wg * a.units_each + min(wg, a.units_more);
+    const int u_last = u_begin + a.units_each + (wg < a.units_more ? 1 : 0);
+    const __amdgpu_buffer_rsrc_t x_buf = gd_buffer(a.X, (unsigned)(((size_t)(M - 1) * a.ldx + K) * 2));
+    const __amdgpu_buffer_rsrc_t w_buf = gd_buffer(a.W, (unsigned)((size_t)a.N * K * 2));
+    const GdFinishBuffers fin_bufs = gd_finish_buffers(a);
+    const int i_fin = tid % UPT, m_fin = tid / UPT;
+    GdFinish fin;
+    auto ask_finish = [&](int tile) {
+        const int u = u_begin + tile * UPT + i_fin;
+        gd_ask<bf16, GD_RESIDUAL>(a, fin_bufs, tid < PLACES && m_fin < M && u < u_last, m_fin, u, fin);
+    };
+    ask_finish(0);
+    u32x4 w[RING][LPI], x[RING][XL];
+    auto issue = [&](u32x4(&wi)[LPI], u32x4(&xi)[XL], int tile, int j) {
+        const int over = j >= per ? 1 : 0, k = (wave + NW * (j - over * per)) * GD_KC + 8 * r16, u0 = u_begin + (tile + over) * UPT;
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const int row = g + 4 * i;
+            xi[i] = gd_load(x_buf, row < M && k < K && u0 < u_last ? (unsigned)(row * a.ldx + k) * 2 : GD_NOWHERE);
+        }
+#pragma unroll
+        for (int i = 0; i < LPI; ++i) {
+            const int n = u0 + 4 * i + g;
+            wi[i] = gd_load_streaming(w_buf, n < u_last && k < K ? (unsigned)(n * K + k) * 2 : GD_NOWHERE);
+        }
+    };
+#pragma unroll
+    for (int q = 0; q < RING; ++q) issue(w[q], x[q], 0, q);
+    u32x4* const w_tile = w_lds + wave * 16 * (GD_KC / 8);
+    u32x4* const x_tile = x_lds + wave * 16 * (GD_KC / 8);
+    const int x_row = r16 & (4 * XL - 1);
+    for (int tile = 0; tile < a.groups; ++tile) {
+        f32x4 acc[GL_SUMS];
+#pragma unroll
+        for (int h = 0; h < GL_SUMS; ++h) acc[h] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int j0 = 0; j0 < per; j0 += GL_SUMS) {
+#pragma unroll
+            for (int h = 0; h < GL_SUMS; ++h) {
+                const bool live = wave + NW * (j0 + h) < n_chunks;
+                if (live) {
+#pragma unroll
+                    for (int i = 0; i < XL; ++i) x_tile[(g + 4 * i) * 16 + (r16 ^ (g + 4 * i))] = x[h % RING][i];
+#pragma unroll
+                    for (int i = 0; i < LPI; ++i) w_tile[(g + 4 * i) * 16 + (r16 ^ (g + 4 * i))] = w[h % RING][i];
+                }
+                issue(w[h % RING], x[h % RING], tile, j0 + h + RING);
+                if (live) {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const u32x4 wv = w_tile[r16 * 16 + ((4 * s + g) ^ r16)];
+                        const u32x4 xv = x_tile[x_row * 16 + ((4 * s + g) ^ x_row)];
+                        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gd_as_bf16x8(wv), gd_as_bf16x8(xv), acc[h], 0, 0, 0);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < GL_SUMS; ++h)
+            *reinterpret_cast<f32x4*>(red + ((h * NW + wave) * LLMS_WAVE + gd_place<UPT>(g, r16)) * 4) = acc[h];
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the next tile's loads stay in flight)
+        const int u = u_begin + tile * UPT + i_fin;
+        if (tid < PLACES && m_fin < M && u < u_last) {
+            float each[NS], sum = 0.f;
+#pragma unroll
+            for (int v = 0; v < NS; ++v) each[v] = red[(v * LLMS_WAVE + gd_place<UPT>(i_fin / 4, m_fin)) * 4 + i_fin % 4];
+#pragma unroll
+            for (int v = 0; v < NS; ++v) sum += each[v];
+            gd_finish_row<bf16, GD_RESIDUAL>(a, m_fin, u, sum, fin);
+        }
+        if (tile + 1 < a.groups) {
+            ask_finish(tile + 1);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the sums are read before the next tile's overwrite them)
+        }
+    }
+}
+
 // 17 to 64 rows: K up to 2,048 (a wave's two chunks of 64 rows are 128 registers).
 #define GR_GO(XC, RB, NT)                                                                                  \
     do {                                                                                                   \
@@ -1079,7 +1172,9 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
     const int x_rows = M <= 8 ? 8 : 16, x_pitch = (K + GD_KC - 1) / GD_KC * (GD_KC * 2) + 16;
     LLMS_REQUIRE(k_parts >= 1 && k_parts <= 16, "gemm_decode: k_parts must be 1..16");
     const int k_each = k_parts == 1 ? K : ((K + GD_KC - 1) / GD_KC + k_parts - 1) / k_parts * GD_KC;  // columns of a part
-    LLMS_REQUIRE(llms_gemm_decode_fits(M, k_each), "gemm_decode: the rows of X do not fit a compute unit (see llms_gemm_decode_fits)");
+    // (rows of X that need not stay: any K, up to 16 rows, added to the residual rows as they are)
+    const bool longer = !llms_gemm_decode_fits(M, k_each) && M <= 16 && epilogue == GD_RESIDUAL && out_dtype == 1 && norm_weight == nullptr;
+    LLMS_REQUIRE(longer || llms_gemm_decode_fits(M, k_each), "gemm_decode: the rows of X do not fit a compute unit (see llms_gemm_decode_fits)");
     LLMS_REQUIRE(K % 8 == 0 && ldx % 8 == 0 && ldx >= K, "gemm_decode: K and the row stride of X must be multiples of 8");
     // (norming 32 rows in every compute unit was built and measured: 4 microseconds of vector arithmetic in the
     // prologue, more than the norm kernel it saves)
@@ -1147,7 +1242,16 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
     const int most = a.units_each + (a.units_more ? 1 : 0);  // units of the largest share
     const int chunks = (a.k_each + GD_KC - 1) / GD_KC;
     int rc;
-    if (M > 16 || !gd_rows_fit_lds(M, K)) {  // the rows in registers: tiles of 16 weight rows (8 units with partners)
+    if (longer) {
+        const bool low = most <= 8;  // (a tile more is the rows of X once more)
+        a.groups = (most + 15) / 16;
+        const dim3 block(GD_NW * LLMS_WAVE);
+        if (M <= 8 && low) gemm_decode_long_kernel<2, 2><<<grid, block, 0, stream>>>(a);
+        else if (M <= 8) gemm_decode_long_kernel<4, 2><<<grid, block, 0, stream>>>(a);
+        else if (low) gemm_decode_long_kernel<2, 4><<<grid, block, 0, stream>>>(a);
+        else gemm_decode_long_kernel<4, 4><<<grid, block, 0, stream>>>(a);
+        rc = LLMS_OK;
+    } else if (M > 16 || !gd_rows_fit_lds(M, K)) {  // the rows in registers: tiles of 16 weight rows (8 units with partners)
         const bool pairs = epilogue == GD_SWIGLU || epilogue == GD_ROPE_QKV;
         // up to 16 rows, units without partners: tiles of 8 weight rows where the last tile of 16 would be half empty
         const bool low = M <= 16 && !pairs && ((most + 7) / 8) % 2 == 1;

@@ -492,6 +492,12 @@ def gemm_decode_fits(m: int, k: int) -> bool:
     return m <= 16 or k <= 2 * 8 * 128 or (m <= 32 and k <= 4 * 8 * 128)
 
 
+def gemm_decode_adds(m: int, k: int) -> bool:
+    """Whether ops.gemm_decode adds the product of m rows of k elements to bfloat16 residual rows: of up to 16 rows of any length, which need
+    not stay in a compute unit for that."""
+    return 0 < m <= GEMM_DECODE_NORM_ROWS and k > 0
+
+
 GEMM_DECODE_ROWS_K = 2 * 8 * 128  # 17 to 64 rows: what 8 waves hold of a row in registers
 
 
@@ -559,7 +565,8 @@ def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias
             raise ValueError(f"K = {k} has too few chunks of 128 for {k_parts} parts")
         if out is None or out.dtype != torch.float32 or tuple(out.shape) != (k_parts, m, n) or not out.is_contiguous():
             raise ValueError(f"out must be a contiguous float32 [{k_parts}, {m}, {n}] tensor")
-    if not gemm_decode_fits(m, -(-(-(-k // 128)) // k_parts) * 128 if k_parts > 1 else k):
+    adds = residual is not None and residual.dtype == torch.bfloat16 and norm is None and gemm_decode_adds(m, k)
+    if not adds and not gemm_decode_fits(m, -(-(-(-k // 128)) // k_parts) * 128 if k_parts > 1 else k):
         raise ValueError(f"gemm_decode keeps the rows of x in a compute unit: {m} rows of K = {k} do not fit (K up to "
                          f"{GEMM_DECODE_MAX_K} with up to 16 rows, 4,096 with up to 32, 2,048 beyond, per part)")
     if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:

@@ -84,7 +84,21 @@ def adds_residual_in_epilogue(x: torch.Tensor, weight: torch.Tensor) -> bool:
     GEMM_DECODE_NORM_ROWS rows): with more rows that norm is a kernel of its own, which adds up partial sums
     as it reads them, and the product is faster with its K shared out (measured at 32 rows: 1.08 against 1.12 ms
     a step of the TinyLlama shape)."""
-    return x.shape[0] <= ops.GEMM_DECODE_NORM_ROWS and decode_product(x, weight)
+    if x.shape[0] > ops.GEMM_DECODE_NORM_ROWS:
+        return False
+    return decode_product(x, weight) or (
+        DECODE_KERNEL and x.dtype == torch.bfloat16 and ops.gemm_decode_adds(*x.shape) and ops.gemm_bf16_supported(x, weight)
+        and ops.gemm_decode_reaches(x, weight) and adds_long_rows(weight.shape[0], ops.compute_units(x.device)))
+
+
+def adds_long_rows(n: int, cus: int = 256) -> bool:
+    """Whether a product of rows that are too long for a compute unit is added to the residual rows by ops.gemm_decode, in tiles of 16 weight
+    rows that each take the rows of x in again, and not by the norm behind partial sums of ops.gemm_stream.  Not where a share of the weight's
+    n rows fills less than two thirds of its tiles: 5120 x 13824, 20 rows in two tiles, 31.4 microseconds at 1 row and 32.1 at 8, with the norm still to be
+    done by the next product, where stream and norm take 31.1 and 32.9.  11 other weights of 1024 x 8192 to 12288 x 6400 at 1 to 16 rows 7 to 38 %
+    faster (4096 x 14336 21.9 and 28.3 at 8 rows, 6656 x 17920, 26 rows in two tiles, 47.0 and 57.0, 3072 x 8192 10.9 and 16.3)."""
+    most = -(-n // min(n, cus))
+    return most <= 8 or 2 * (-(-most // 16) * 16) <= 3 * most or most <= 16
 
 
 def few_rows(m: int, weight: torch.Tensor) -> bool:

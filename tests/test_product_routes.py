@@ -148,3 +148,19 @@ def test_what_a_product_is_told_of_a_weight_brought_nearer(monkeypatch):
     x, weight, near = torch.empty(512, 2048), torch.empty(11264, 2048, device="meta"), torch.empty(2048 * 5632 + 1, dtype=torch.bfloat16)
     assert brings_near(x, weight, near[:-1])[0] > 0 and brings_near(x, weight, near[1:])[0] == 0
     assert brings_near(torch.empty(2048, 2048), torch.empty(8192, 2048, device="meta"), near[:-1])[0] == 0
+
+
+@pytest.mark.parametrize("n,long", [(1, True), (256, True), (1024, True), (4096, True), (4097, False), (5120, False), (5376, False), (5632, True), (6656, True),
+                                    (8192, True), (8193, True), (12288, True)])
+def test_long_rows_are_added_where_their_tiles_are_filled(n, long):
+    """Rows of x that do not stay in a compute unit are taken in again for every tile of 16 weight rows: shares of 17 to 21 rows stay with the
+    streaming kernel.  Rows that stay, and more than 16 of them, go where they went."""
+    from llmserve.parts import linear
+
+    def bf16(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="meta")
+
+    assert linear.adds_long_rows(n) == long
+    assert linear.ops.gemm_decode_adds(16, 11008) and not linear.ops.gemm_decode_adds(17, 11008)
+    assert not linear.adds_residual_in_epilogue(bf16(17, 11008), bf16(n, 11008))
+    assert linear.adds_residual_in_epilogue(bf16(16, 6144), bf16(n, 6144))
