@@ -4,21 +4,79 @@
 // residual sum are always computed in 32-bit.
 #include "common.h"
 
-// ------------------------------------------------------------------ embedding gather
+#include <type_traits>
+
+// ------------------------------------------------------------------ what a step starts with
 // out[n, :] = table[ids[n], :].  An id outside [0, vocab) yields a row of NaN, so a bad
 // token shows in the logits and never reads outside the table.
-template <typename T>
-__global__ void embed_gather_kernel(T* __restrict__ out, const T* __restrict__ table,
-                                    const int* __restrict__ ids, int hidden, int vocab) {
-    const int n = blockIdx.x;
-    const int id = ids[n];
-    T* o = out + (size_t)n * hidden;
-    if ((unsigned)id >= (unsigned)vocab) {
-        for (int i = threadIdx.x; i < hidden; i += blockDim.x) o[i] = from_f32<T>(__uint_as_float(0x7fc00000u));
+//
+// The first launch of a step, whose parts do not depend on each other: rows of the embedding (block n: token n), the sines and cosines of the step's
+// angles (the blocks behind), and the pages it took written into the block tables (one block a table).  They were three launches of 5.8, 1.8 and 2
+// microseconds for 8 tokens of the 1.1B shape, and a row came 2 bytes a thread at a time; 23 decoding steps of 64 requests took 13 microseconds more
+// each.  What bounds it: a launch, and an answer of memory behind the ids'.
+// SCALED: rows in 32-bit times `scale`; an id outside the vocabulary is the nearest one.  Otherwise rows as they are; such an id's is NaN.
+#define STEP_START_TABLES 8
+struct StepStartArgs {
+    void* out;
+    const void* table;
+    const int* ids;
+    int n, hidden, vocab, wide;  // wide: rows in pieces of 16 bytes
+    float scale;
+    float2* angles;  // [n][half], or null
+    const int* positions;
+    const float* freq;
+    int half, angle_blocks, tables;
+    int* dst[STEP_START_TABLES];
+    const int* index[STEP_START_TABLES];  // below 0: nothing
+    const int* value[STEP_START_TABLES];
+    int count[STEP_START_TABLES];
+};
+
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(256) void step_start_kernel(const StepStartArgs a) {
+    int b = blockIdx.x;
+    if (b < a.n) {
+        typedef typename std::conditional<SCALED, float, T>::type Out;
+        Out* o = reinterpret_cast<Out*>(a.out) + (size_t)b * a.hidden;
+        int id = a.ids[b];
+        if constexpr (SCALED) {
+            id = id < 0 ? 0 : id >= a.vocab ? a.vocab - 1 : id;
+        } else if ((unsigned)id >= (unsigned)a.vocab) {
+            for (int i = threadIdx.x; i < a.hidden; i += 256) o[i] = from_f32<Out>(__uint_as_float(0x7fc00000u));
+            return;
+        }
+        const T* src = reinterpret_cast<const T*>(a.table) + (size_t)id * a.hidden;
+        constexpr int V = 16 / sizeof(T);
+        if (a.wide) {
+            for (int i = threadIdx.x * V; i < a.hidden; i += 256 * V) {
+                const uint4 v = *reinterpret_cast<const uint4*>(src + i);
+                if constexpr (!SCALED) {
+                    *reinterpret_cast<uint4*>(o + i) = v;
+                } else {
+                    const T* e = reinterpret_cast<const T*>(&v);
+#pragma unroll
+                    for (int c = 0; c < V; c += 4)
+                        *reinterpret_cast<float4*>(o + i + c) = make_float4(to_f32(e[c]) * a.scale, to_f32(e[c + 1]) * a.scale,
+                                                                            to_f32(e[c + 2]) * a.scale, to_f32(e[c + 3]) * a.scale);
+                }
+            }
+        } else {
+            for (int i = threadIdx.x; i < a.hidden; i += 256) {
+                if constexpr (SCALED) o[i] = to_f32(src[i]) * a.scale;
+                else o[i] = src[i];
+            }
+        }
         return;
     }
-    const T* src = table + (size_t)id * hidden;
-    for (int i = threadIdx.x; i < hidden; i += blockDim.x) o[i] = src[i];
+    b -= a.n;
+    if (b < a.angle_blocks) {
+        const int i = b * 256 + threadIdx.x;
+        if (i < a.n * a.half) a.angles[i] = rotary_angle((float)a.positions[i / a.half], a.freq[i % a.half]);
+        return;
+    }
+    b -= a.angle_blocks;
+    for (int i = threadIdx.x; i < a.count[b]; i += 256)
+        if (a.index[b][i] >= 0) a.dst[b][a.index[b][i]] = a.value[b][i];
 }
 
 // ------------------------------------------------------------------ RMSNorm
@@ -554,11 +612,43 @@ static bool f32_rows_at_once(int n_rows, int hidden) {
 
 extern "C" {
 
-int llms_embed_gather(int dtype, void* out, const void* table, const int* ids, int n_tokens, int hidden,
-                      int vocab, hipStream_t stream) {
-    LLMS_REQUIRE(n_tokens > 0 && hidden > 0 && vocab > 0, "embed_gather: sizes must be positive");
-    DISPATCH_DTYPE(dtype, embed_gather_kernel<T><<<n_tokens, 256, 0, stream>>>((T*)out, (const T*)table, ids,
-                                                                                hidden, vocab);)
+// Rows of the embedding table (dtype 0 float32, 1 bfloat16): out [n, hidden] of the same type, or with `scaled` float32 and times `scale`.
+// angles (or null): float32 [n][half][2].  The tables' entries: dst[t][index[t][i]] = value[t][i] for i < count[t], index below 0: nothing.
+int llms_step_start(int dtype, void* out, const void* table, const int* ids, int n, int hidden, int vocab, int scaled, float scale, float* angles,
+                    const int* positions, const float* freq, int half, int tables, int* const* dst, const int* const* index,
+                    const int* const* value, const int* count, hipStream_t stream) {
+    LLMS_REQUIRE(n > 0 && hidden > 0 && vocab > 0, "step_start: sizes must be positive");
+    LLMS_REQUIRE(dtype == 0 || dtype == 1, "step_start: dtype must be 0 (float32) or 1 (bfloat16)");
+    LLMS_REQUIRE(tables >= 0 && tables <= STEP_START_TABLES, "step_start: up to 8 tables");
+    LLMS_REQUIRE(angles == nullptr || (positions && freq && half > 0 && (long long)n * half < (1ll << 30)), "step_start: angles need positions and frequencies");
+    StepStartArgs a{};
+    a.out = out;
+    a.table = table;
+    a.ids = ids;
+    a.n = n;
+    a.hidden = hidden;
+    a.vocab = vocab;
+    a.wide = hidden % (dtype ? 8 : 4) == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)table % 16 == 0;
+    a.scale = scale;
+    a.angles = reinterpret_cast<float2*>(angles);
+    a.positions = positions;
+    a.freq = freq;
+    a.half = half;
+    a.angle_blocks = angles ? (n * half + 255) / 256 : 0;
+    a.tables = tables;
+    for (int t = 0; t < tables; ++t) {
+        LLMS_REQUIRE(dst[t] && index[t] && value[t] && count[t] >= 0, "step_start: a table's arguments");
+        a.dst[t] = dst[t];
+        a.index[t] = index[t];
+        a.value[t] = value[t];
+        a.count[t] = count[t];
+    }
+    LLMS_REQUIRE((long long)n + a.angle_blocks + tables < (1ll << 31), "step_start: too many rows");
+    const unsigned grid = (unsigned)(n + a.angle_blocks + tables);
+    if (dtype == 0 && scaled) step_start_kernel<float, true><<<grid, 256, 0, stream>>>(a);
+    else if (dtype == 0) step_start_kernel<float, false><<<grid, 256, 0, stream>>>(a);
+    else if (scaled) step_start_kernel<bf16, true><<<grid, 256, 0, stream>>>(a);
+    else step_start_kernel<bf16, false><<<grid, 256, 0, stream>>>(a);
     LLMS_LAUNCH_CHECK();
 }
 

@@ -1,5 +1,4 @@
 // Kernels of a layer whose residual stream is kept in 32-bit whatever the model's dtype:
-//   embed_scale      x[n] = table[ids[n]] * scale                                   (table T, x float)
 //   rmsnorm32        y[r] = x[s] * rsqrt(mean(x[s]^2) + eps) * (offset + w), s = rows[r] or r   (x float, y T)
 //   gated_add        x[n] += sum over branches b of g_b * y_b[n]                    (all float)
 //                    g_b = sigmoid(z_b[n] + bias_b) where the branch has a gate, else 1
@@ -15,17 +14,6 @@
 #include "common.h"
 
 #define S32_THREADS 256
-
-template <typename T>
-__global__ __launch_bounds__(S32_THREADS) void embed_scale_kernel(float* __restrict__ out, const T* __restrict__ table,
-                                                                  const int* __restrict__ ids, int hidden, int vocab,
-                                                                  float scale) {
-    const int n = blockIdx.x;
-    int id = ids[n];
-    id = id < 0 ? 0 : (id >= vocab ? vocab - 1 : id);
-    const T* row = table + (size_t)id * hidden;
-    for (int c = threadIdx.x; c < hidden; c += S32_THREADS) out[(size_t)n * hidden + c] = to_f32(row[c]) * scale;
-}
 
 // Rows whose length is a multiple of 4: a thread brings up to S32_VEC float4 of its row at once (rows of up to
 // 4 * S32_VEC * S32_THREADS), so a row costs one wait for memory and not one per 256 elements.
@@ -553,18 +541,6 @@ int llms_weighted_sum(float* out, const float* a, const float* b, float sa, floa
 int llms_softcap(float* x, size_t total, float cap, hipStream_t stream) {
     LLMS_REQUIRE(total > 0 && cap > 0.f, "softcap: a positive size and a positive cap");
     softcap_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(x, total, cap);
-    LLMS_LAUNCH_CHECK();
-}
-
-int llms_embed_scale(int dtype, float* out, const void* table, const int* ids, int n, int hidden, int vocab, float scale,
-                     hipStream_t stream) {
-    LLMS_REQUIRE(n > 0 && hidden > 0 && vocab > 0, "embed_scale: sizes must be positive");
-    if (dtype == 0)
-        embed_scale_kernel<float><<<n, S32_THREADS, 0, stream>>>(out, (const float*)table, ids, hidden, vocab, scale);
-    else if (dtype == 1)
-        embed_scale_kernel<bf16><<<n, S32_THREADS, 0, stream>>>(out, (const bf16*)table, ids, hidden, vocab, scale);
-    else
-        LLMS_REQUIRE(false, "embed_scale: dtype must be 0 (float32) or 1 (bfloat16)");
     LLMS_LAUNCH_CHECK();
 }
 

@@ -47,6 +47,8 @@ class StepBatch:
     # what a part has worked out for this step and the same kind of part in later layers can use again (the sines
     # and cosines of the tokens' angles); emptied by the model when a step starts
     shared: dict = field(default_factory=dict)
+    # block table entries that the step's first launch writes: (table, index, value) per group, an index below 0 for none
+    table_updates: list = field(default_factory=list)
     all_rows_wanted: bool = False  # logit_rows is 0, 1, ..., num_tokens - 1 (known on the host: nothing to pick)
 
 
@@ -170,6 +172,7 @@ class StaticDecodeBatch:
         v = self._view
         groups = {g: GroupView(storage.tables[g], v(7 + 3 * j)) for j, g in enumerate(group_ids)}
         self.batch = StepBatch(
+            table_updates=[(storage.tables[g], v(8 + 3 * j), v(9 + 3 * j)) for j, g in enumerate(group_ids)],
             num_tokens=c, num_seqs=c, token_ids=v(0), positions=v(1), token_seq=v(2), cu_seqlens=v(3),
             context_lens=v(4), state_slots=v(5), logit_rows=v(6), groups=groups, counts=[1] * c, starts=[0] * c,
             state_slot_list=[0] * c, num_decode=c, max_count=1, max_context=1, max_decode_context=1,
@@ -189,13 +192,6 @@ class StaticDecodeBatch:
 
     def _host_view(self, i: int):
         return self.host_np[self._offsets[i]: self._offsets[i] + self._sizes[i]]
-
-    def apply_table_updates(self) -> None:
-        """Write the step's new pages into the device block tables (part of the captured graph)."""
-        from ..ops import library as ops
-
-        for j, g in enumerate(self.group_ids):
-            ops.scatter_i32(self.storage.tables[g], self._view(8 + 3 * j), self._view(9 + 3 * j))
 
     def fill(self, layout: StepLayout, tokens: list[int]) -> None:
         """Write a decode-only step (one token per request) into the buffers."""
@@ -262,6 +258,7 @@ class StaticStepBatch:
         v = self._view
         groups = {g: GroupView(storage.tables[g], v(7 + 3 * j)) for j, g in enumerate(group_ids)}
         self.batch = StepBatch(
+            table_updates=[(storage.tables[g], v(8 + 3 * j), v(9 + 3 * j)) for j, g in enumerate(group_ids)],
             num_tokens=n, num_seqs=b, token_ids=v(0), positions=v(1), token_seq=v(2), cu_seqlens=v(3),
             context_lens=v(4), state_slots=v(5), logit_rows=v(6), groups=groups,
             counts=[1] * decode + [0] * prefill + [tokens], starts=[0] * b, state_slot_list=[0] * b,
@@ -282,13 +279,6 @@ class StaticStepBatch:
 
     def _host_view(self, i: int):
         return self.host_np[self._offsets[i]: self._offsets[i] + self._sizes[i]]
-
-    def apply_table_updates(self) -> None:
-        """Write the step's new pages into the device block tables (part of the captured graph)."""
-        from ..ops import library as ops
-
-        for j, g in enumerate(self.group_ids):
-            ops.scatter_i32(self.storage.tables[g], self._view(8 + 3 * j), self._view(9 + 3 * j))
 
     def fill(self, layout: StepLayout, tokens: list[list[int]], logit_rows: list[int]) -> None:
         """Write a step into the buffers: `layout` lists the requests that bring one token first."""

@@ -443,7 +443,6 @@ class _StepBucket:
     def run(self, runner: "ModelRunner") -> torch.Tensor:
         """Launch the step that `static.fill` described, kernel by kernel.  (The runner is an argument, not a
         field: a bucket that pointed back at its runner would keep both alive until the cycle collector runs.)"""
-        self.static.apply_table_updates()
         return runner.model.forward(self.static.batch, runner.storage)
 
     def capture(self, runner: "ModelRunner", pool) -> None:
@@ -465,10 +464,8 @@ class _DecodeGraph:
         batch = self.static.batch
         batch.max_context = batch.max_decode_context = reach
         # a first run outside the capture: libraries load, memory pools warm up
-        self.static.apply_table_updates()
         runner.model.forward(batch, runner.storage)
         torch.cuda.synchronize(runner.device)
         self.graph = torch.cuda.CUDAGraph()
         with _capturing(self.graph):
-            self.static.apply_table_updates()
             self.logits = runner.model.forward(batch, runner.storage)

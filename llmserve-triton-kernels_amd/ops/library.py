@@ -127,19 +127,54 @@ def _check(status: int, what: str) -> None:
 # ------------------------------------------------------------------------------ elementwise
 
 
-def embed_gather(out: torch.Tensor, table: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
-    """out[n] = table[ids[n]]; out [N,H], table [V,H], ids int32 [N]."""
-    dev = _dev(out, table, ids)
+STEP_START_TABLES = 8  # most block tables of ops.step_start
+
+
+def step_start(out: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, *, scale: float | None = None,
+               angles: tuple[torch.Tensor, torch.Tensor] | None = None, scatters=()) -> torch.Tensor | None:
+    """What a step starts with, in one launch: out[n] = table[ids[n]] (`embed_gather`; with `scale` `embed_scale`); with angles =
+    (positions, frequencies) what `rotary_angles` gives, which is returned; and for every (dst, index, value) of `scatters` (up to
+    STEP_START_TABLES) what `scatter_i32` does."""
+    dev = _dev(out, table, ids, *(angles or ()), *(t for entry in scatters for t in entry))
     _rows(out, "out")
     _rows(table, "table", out.shape[1])
-    _i32(ids, "ids", out.shape[0])
-    if out.dtype != table.dtype:
-        raise ValueError("out and table differ in dtype")
-    if out.shape[0] == 0:
-        return out
-    _check(load("elementwise").llms_embed_gather(
-        c_int(_code(out)), _ptr(out), _ptr(table), _ptr(ids), c_int(out.shape[0]), c_int(out.shape[1]),
-        c_int(table.shape[0]), _stream(dev)), "embed_gather")
+    n = out.shape[0]
+    _i32(ids, "ids", n)
+    if out.dtype != (table.dtype if scale is None else torch.float32):
+        raise ValueError("out and table differ in dtype" if scale is None else "out must be float32")
+    if len(scatters) > STEP_START_TABLES:
+        raise ValueError(f"up to {STEP_START_TABLES} tables")
+    turned, half = None, 0
+    if angles is not None:
+        positions, freq = angles
+        _i32(positions, "positions", n)
+        _f32(freq, "frequencies")
+        half = freq.numel()
+        turned = torch.empty((n, half, 2), dtype=torch.float32, device=dev)
+    for dst, index, value in scatters:
+        if dst.dtype != torch.int32 or not dst.is_contiguous():
+            raise ValueError("dst must be a contiguous int32 tensor")
+        _i32(index, "index")
+        _i32(value, "value", index.numel())
+    if n == 0:
+        for entry in scatters:
+            scatter_i32(*entry)
+        return turned
+    pointers = ctypes.c_void_p * max(len(scatters), 1)
+    dst, index, value = (pointers(*(entry[i].data_ptr() for entry in scatters)) for i in range(3))
+    count = (c_int * max(len(scatters), 1))(*(entry[1].numel() for entry in scatters))
+    turns = turned is not None and half > 0
+    _check(load("elementwise").llms_step_start(
+        c_int(_code(table)), _ptr(out), _ptr(table), _ptr(ids), c_int(n), c_int(out.shape[1]), c_int(table.shape[0]),
+        c_int(0 if scale is None else 1), c_float(1.0 if scale is None else scale), _ptr(turned if turns else None),
+        _ptr(angles[0] if turns else None), _ptr(angles[1] if turns else None), c_int(half), c_int(len(scatters)), dst, index, value, count,
+        _stream(dev)), "step_start")
+    return turned
+
+
+def embed_gather(out: torch.Tensor, table: torch.Tensor, ids: torch.Tensor) -> torch.Tensor:
+    """out[n] = table[ids[n]]; out [N,H], table [V,H], ids int32 [N]."""
+    step_start(out, table, ids)
     return out
 
 
@@ -1204,17 +1239,7 @@ def attention_prompt_biased(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Te
 
 def embed_scale(out: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, scale: float) -> torch.Tensor:
     """out[n] = table[ids[n]] * scale in 32-bit; out float32 [N, H], table [V, H] float32 or bfloat16."""
-    dev = _dev(out, table, ids)
-    _rows(out, "out")
-    _rows(table, "table", out.shape[1])
-    _i32(ids, "ids", out.shape[0])
-    if out.dtype != torch.float32:
-        raise ValueError("out must be float32")
-    if out.shape[0] == 0:
-        return out
-    _check(load("stream32").llms_embed_scale(
-        c_int(_code(table)), _ptr(out), _ptr(table), _ptr(ids), c_int(out.shape[0]), c_int(out.shape[1]),
-        c_int(table.shape[0]), c_float(scale), _stream(dev)), "embed_scale")
+    step_start(out, table, ids, scale=float(scale))
     return out
 
 

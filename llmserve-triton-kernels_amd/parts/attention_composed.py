@@ -56,7 +56,7 @@ import torch
 from ..ops import library as ops
 from .attention import decode_arrangement, prompt_splits
 from .linear import linear
-from .rope import step_angles
+from .rope import step_angles, step_angles_key
 from .registry import Mixer, register_mixer
 from .spec import PagedCacheSpec, ParamInfo, StateCacheSpec
 
@@ -318,6 +318,10 @@ class ComposedAttention(Mixer):
         if self.differential:  # one number for the layer, worked out once
             dot = [float((tensors[n[a]].double() * tensors[n[b]].double()).sum()) for a, b in (("lq1", "lk1"), ("lq2", "lk2"))]
             self.lam = math.exp(dot[0]) - math.exp(dot[1]) + self.diff
+
+    def step_table(self):
+        """As a position encoding's."""
+        return None if self.freq is None else (step_angles_key(self.turn_key), self.freq)
 
     # ---- one step ------------------------------------------------------------------------------------
     @property

@@ -34,7 +34,7 @@ import torch
 from ..ops import library as ops
 from .linear import linear
 from .registry import Mixer, register_mixer
-from .rope import step_angles
+from .rope import step_angles, step_angles_key
 from .spec import PagedCacheSpec, ParamInfo
 
 _DEFAULT_NAMES = {"dq": "dq", "dq_norm": "dq.norm", "uq": "uq", "q": "q", "sink": "sink", "dkv": "dkv", "dkv_norm": "dkv.norm", "uk": "uk",
@@ -138,6 +138,10 @@ class LatentAttention(Mixer):
         elif self.dims:
             exponent = torch.arange(0, self.dims, 2, dtype=torch.float64) / self.dims
             self.freq = (1.0 / (self.base ** exponent)).to(torch.float32).to(self.w_o.device)
+
+    def step_table(self):
+        """As a position encoding's."""
+        return None if self.freq is None else (step_angles_key(self.turn_key), self.freq)
 
     # ---- one step ------------------------------------------------------------------------------------
     def forward(self, x, batch, cache):

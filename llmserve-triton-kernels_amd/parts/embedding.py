@@ -41,11 +41,14 @@ class TokenEmbedding(Part):
         self.weight = tensors[self.tensor].contiguous()
 
     def forward(self, token_ids: torch.Tensor) -> torch.Tensor:
-        if self.stream == "float32":
-            out = torch.empty((token_ids.numel(), self.hidden), dtype=torch.float32, device=self.weight.device)
-            return ops.embed_scale(out, self.weight, token_ids, 1.0 if self.scale is None else float(self.scale))
-        out = torch.empty((token_ids.numel(), self.hidden), dtype=self.weight.dtype, device=self.weight.device)
-        return ops.embed_gather(out, self.weight, token_ids)
+        return self.begin(token_ids)[0]
+
+    def begin(self, token_ids: torch.Tensor, angles=None, scatters=()):
+        """(the tokens' rows, the table of `angles` or None): a step's first launch (ops.step_start)."""
+        wide = self.stream == "float32"
+        out = torch.empty((token_ids.numel(), self.hidden), dtype=torch.float32 if wide else self.weight.dtype, device=self.weight.device)
+        scale = (1.0 if self.scale is None else float(self.scale)) if wide else None
+        return out, ops.step_start(out, self.weight, token_ids, scale=scale, angles=angles, scatters=scatters)
 
 
 @HEADS.register("lm_head")

@@ -29,6 +29,7 @@ class Model:
         self.head = HEADS.build(spec.head, ctx)
         self.blocks = []
         self._sources = None
+        self._angle_table = None  # (key, frequencies), or () for none, from the first step on
         self._shift_rows = {pos: row for pos, row in spec.shifts}
         self.shift_table = None  # float32 [rows, hidden] on the device
         families = {"mixer": MIXERS, "feed_forward": FEED_FORWARDS, "norm": NORMS, "gate": GATES,
@@ -119,12 +120,33 @@ class Model:
         ops.add_vector(x, self.shift_table[row])
 
     # ---- one step ----------------------------------------------------------------------------
+    def _begin(self, batch, shared):
+        """The tokens' rows, and in the same launch the pages that the step took (`batch.table_updates`) and the table of angles that most
+        of its parts turn by (bfloat16: 32-bit parts work the angles out where they turn)."""
+        if self._angle_table is None:
+            tables = [t() for _, part in self._parts() for p in (part, getattr(part, "position", None))
+                      for t in [getattr(p, "step_table", None)] if t is not None]
+            found = [t for t in tables if t is not None]
+            keys = [key for key, _ in found]
+            self._angle_table = max(found, key=lambda t: keys.count(t[0]), default=()) if self.ctx.dtype == torch.bfloat16 else ()
+        angles = (batch.positions, self._angle_table[1]) if self._angle_table and shared is not None else None
+        updates = getattr(batch, "table_updates", ())
+        with_rows = ops.STEP_START_TABLES if hasattr(self.embedding, "begin") else 0
+        for entry in updates[with_rows:]:
+            ops.scatter_i32(*entry)
+        if not with_rows:
+            return self.embedding.forward(batch.token_ids)
+        x, turned = self.embedding.begin(batch.token_ids, angles, updates[:with_rows])
+        if turned is not None:
+            shared[self._angle_table[0]] = turned
+        return x
+
     def forward(self, batch, storage) -> torch.Tensor:
         """Logits [R, vocab] in 32-bit at `batch.logit_rows` (empty tensor when R = 0)."""
         shared = getattr(batch, "shared", None)
         if shared is not None:
             shared.clear()  # (a batch object may serve several steps)
-        x = self.embedding.forward(batch.token_ids)
+        x = self._begin(batch, shared)
         delta = None
         if self._sources is None:
             self._sources = self.cache_sources()

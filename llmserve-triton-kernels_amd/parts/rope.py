@@ -15,6 +15,10 @@ from ..ops import library as ops
 from .registry import PositionEncoding, register_position_encoding
 
 
+def step_angles_key(key):
+    return ("step_angles", key)
+
+
 def step_angles(batch, freq, key) -> "torch.Tensor | None":
     """float32 [N, len(freq), 2]: sine and cosine of every new token's position times every frequency (None: nothing
     turns).  Worked out by the first part of a step that asks; the others whose frequencies go by the same `key` find the
@@ -22,7 +26,7 @@ def step_angles(batch, freq, key) -> "torch.Tensor | None":
     shared = getattr(batch, "shared", None)
     if freq is None or shared is None:
         return None
-    key = ("step_angles", key)
+    key = step_angles_key(key)
     if key not in shared:
         shared[key] = ops.rotary_angles(batch.positions, freq)
     return shared[key]
@@ -52,10 +56,14 @@ class RotaryEncoding(PositionEncoding):
         position * frequency, which lets a mixer fold the rotation into a kernel of its own."""
         return self.inv_freq
 
+    def step_table(self):
+        """(what the table of `rotary_angles` is shared by, the frequencies): for a step's first launch, which may work it out."""
+        return ("rotary_angles", self.head_dim, self.theta), self.inv_freq
+
     def rotary_angles(self, batch):
         """float32 [N, head_dim / 2, 2]: sine and cosine of every new token's angles.  The first layer of a step
         that asks works them out (one small kernel); the others find them in what the step's parts share."""
-        key = ("rotary_angles", self.head_dim, self.theta)
+        key = self.step_table()[0]
         table = batch.shared.get(key)
         if table is None:
             table = batch.shared[key] = ops.rotary_angles(batch.positions, self.inv_freq)
