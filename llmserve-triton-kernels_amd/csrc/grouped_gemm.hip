@@ -9,8 +9,8 @@
 // (unit 0), or a * sigmoid(a) * b (unit 1);
 // "gated": the result times sigmoid(z[m, g * z_gs + n * z_ns]) with z in 32-bit (z_ns 1: a gate per element; 0: one number
 // for a row of a group).
-// Two kernels: 32-bit multiply-add (any sizes, float or bfloat16 operands, 32-bit products and sums) and bfloat16 on
-// the matrix cores (K and the strides of x in multiples of 8, 16-byte aligned operands).
+// Three kernels: 32-bit multiply-add (any sizes, float or bfloat16 operands, 32-bit products and sums) and bfloat16 on
+// the matrix cores (K and the strides of x in multiples of 8, 16-byte aligned operands), in tiles or for few rows.
 #include "common.h"
 
 #define GG_TM 64
@@ -260,6 +260,70 @@ __global__ __launch_bounds__(256) void grouped_mfma_kernel(
     }
 }
 
+// Up to 16 rows that meet every group (a step of few tokens, whose heads each have a matrix of their own).  A tile of 128 rows through LDS is
+// a chain of trips between memory, LDS and barriers for one to four steps of K; here a wave has 16 weight rows and both operands
+// come straight into the layout of v_mfma_f32_16x16x32_bf16, 256 columns asked for at once: one trip to memory, which is what bounds it.
+// Microseconds with 4 and with 16 rows, the tile's time first:
+//   32 groups of 256 x 64   4.9 -> 2.6   5.1 -> 3.0        16 groups of 128 x 512    10.0 -> 5.0   10.2 -> 6.0
+//   32 groups of 64 x 256   6.9 -> 3.5   7.2 -> 4.2        16 groups of 1024 x 1024  18.7 -> 10.3  19.1 -> 11.4
+#define GF_ROWS 16
+#define GF_WEIGHTS (1l << 24)  // at most so many numbers in w
+#define GF_STEPS 8  // of 32 columns asked for at once
+typedef __attribute__((ext_vector_type(4))) float gg_f32x4;
+
+template <typename TOut, int EPI>
+__global__ __launch_bounds__(256) void grouped_few_kernel(TOut* __restrict__ out, long out_ld, long out_gs, const bf16* __restrict__ x, long x_ld,
+                                                          long x_gs, const bf16* __restrict__ w, int M, int N, int K,
+                                                          const float* __restrict__ z, long z_ld, long z_gs, int z_ns) {
+    const int g = blockIdx.y, wave = threadIdx.x / LLMS_WAVE, lane = threadIdx.x % LLMS_WAVE, r16 = lane % 16, q = lane / 16;
+    const int n0 = (blockIdx.x * 4 + wave) * 16;
+    if (n0 >= N) return;
+    const int n = n0 + r16 < N ? n0 + r16 : N - 1, m = r16 < M ? r16 : M - 1;  // (lanes without a row of their own read the last one, and store nothing)
+    const bf16* wr = w + ((size_t)g * N + n) * K;
+    const bf16* xr = x + (size_t)g * x_gs + (size_t)m * x_ld;
+    const gg_u32x4 zero = {0, 0, 0, 0};
+    float gate[4] = {};
+    if (EPI == GG_GATED) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = n0 + 4 * q + r < N ? n0 + 4 * q + r : N - 1;
+            gate[r] = z[(size_t)m * z_ld + (size_t)g * z_gs + (size_t)c * z_ns];
+        }
+    }
+    gg_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < K; k0 += 32 * GF_STEPS) {
+        gg_u32x4 wv[GF_STEPS], xv[GF_STEPS];
+#pragma unroll
+        for (int s = 0; s < GF_STEPS; ++s) {
+            const int k = k0 + 32 * s + 8 * q;  // (K is a multiple of 8)
+            wv[s] = k < K ? *reinterpret_cast<const gg_u32x4*>(wr + k) : zero;
+            xv[s] = k < K ? *reinterpret_cast<const gg_u32x4*>(xr + k) : zero;
+        }
+#pragma unroll
+        for (int s = 0; s < GF_STEPS; ++s)
+            if (k0 + 32 * s < K)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, wv[s]), __builtin_bit_cast(gg_bf16x8, xv[s]), acc, 0, 0, 0);
+    }
+    if (r16 >= M) return;
+    TOut* o = out + (size_t)g * out_gs + (size_t)r16 * out_ld;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int c = n0 + 4 * q + r;
+        if (c < N) o[c] = from_f32<TOut>(EPI == GG_GATED ? acc[r] / (1.f + expf(-gate[r])) : acc[r]);
+    }
+}
+
+template <typename TOut>
+static int launch_few(int epilogue, hipStream_t stream, void* out, long out_ld, long out_gs, const void* x, long x_ld, long x_gs, const void* w,
+                      int M, int N, int K, int G, const float* z, long z_ld, long z_gs, int z_ns) {
+    const dim3 grid((N + 63) / 64, G);
+    if (epilogue == GG_PLAIN)
+        grouped_few_kernel<TOut, GG_PLAIN><<<grid, 256, 0, stream>>>((TOut*)out, out_ld, out_gs, (const bf16*)x, x_ld, x_gs, (const bf16*)w, M, N, K, z, z_ld, z_gs, z_ns);
+    else
+        grouped_few_kernel<TOut, GG_GATED><<<grid, 256, 0, stream>>>((TOut*)out, out_ld, out_gs, (const bf16*)x, x_ld, x_gs, (const bf16*)w, M, N, K, z, z_ld, z_gs, z_ns);
+    LLMS_LAUNCH_CHECK();
+}
+
 template <typename TOut>
 static int launch_mfma(int epilogue, dim3 grid, hipStream_t stream, void* out, long out_ld, long out_gs, const void* x, long x_ld,
                        long x_gs, const void* w, int M, int N, int K, int G, const int* seg, const int* tile_start, const float* z,
@@ -327,6 +391,11 @@ int llms_grouped_mfma(int out_dtype, int epilogue, void* out, long out_ld, long 
     LLMS_REQUIRE(k_parts >= 1 && k_parts <= 16, "grouped_mfma: 1 to 16 parts of K");
     LLMS_REQUIRE(k_parts == 1 || (seg && epilogue == GG_PLAIN && out_dtype == 0),
                  "grouped_mfma: K is shared out only with segments, the plain epilogue and a float32 result");
+    // (every wave asks for the rows again, which weights of many megabytes feel: at 16 rows 64 groups of 1024 x 512 take 20.3 us here and 18.0 in
+    // tiles, 1024 x 1024 36.5 and 30.5; 32 MB, 64 groups of 4096 x 64, are still 19.2 against 20.4)
+    if (!seg && M <= GF_ROWS && epilogue != GG_PAIRED && G <= 65535 && (long)G * N * K <= GF_WEIGHTS && (out_dtype == 0 || out_dtype == 1))
+        return out_dtype == 0 ? launch_few<float>(epilogue, stream, out, out_ld, out_gs, x, x_ld, x_gs, w, M, N, K, G, z, z_ld, z_gs, z_ns)
+                              : launch_few<bf16>(epilogue, stream, out, out_ld, out_gs, x, x_ld, x_gs, w, M, N, K, G, z, z_ld, z_gs, z_ns);
     const int k_part = k_parts == 1 ? K : ((K + k_parts - 1) / k_parts + GM_BK - 1) / GM_BK * GM_BK;
     dim3 grid((N + GM_BN - 1) / GM_BN, seg ? max_tiles : (M + GM_BM - 1) / GM_BM, seg ? k_parts : G);
     LLMS_REQUIRE(grid.y > 0 && grid.y <= 65535 && grid.z <= 65535, "grouped_mfma: too many rows or groups for one launch");
