@@ -70,12 +70,13 @@ struct WideArgs {
     float* ws_o;      // [share][request][heads * maps][DT * 16]
     float* ws_stats;  // [share][request][heads * maps][2]: maximum (units of log 2) and sum
     int out_stride, q_stride, max_blocks;
-    int seq_begin, n_seqs, blocks_per_seq;
+    int seq_begin, n_seqs;
     int heads, grp, maps, score_heads, heads_per_wg;
     int dv, block_size, k_page, v_page;  // k_page, v_page: elements of a page
     int window, keep_first, chunk;
     int tok, tpw, shares;
     unsigned bs_magic;  // ceil(2^32 / block_size)
+    unsigned tok_magic;  // ceil(2^32 / tok) (0: tok is 1)
     float scale, lambda, eps, out_scale;
     int head_norm, sink;
 };
@@ -101,16 +102,83 @@ __device__ __forceinline__ void weight_pieces(float p[2][4], bf16x8v pf[PIECES])
 
 __device__ __forceinline__ uint32_t low_half_mask(int keep) { return keep <= 0 ? 0u : keep == 1 ? 0xffffu : 0xffffffffu; }
 
+// Workgroup i's request and block of tokens; the workgroups that find none lie behind all that do.  With a grid of every request's longest
+// possible portion, workgroups without tokens lay between those with some, and as workgroups go around the parts of the chip in
+// turn, parts of it met only empty ones (32 heads of 64 on 4, microseconds: 811, 890, 150 and 197 tokens 156 -> 91, twice 1,024 beside
+// two of 1 token 190 -> 104, without those 104; 16 heads of two maps on 2: 57 -> 48 and 73 -> 56).
+// Up to AW_SORTED requests: the block with the i-th most keys, so that no long one begins late.  A block's height is its place from its
+// request's beginning, in blocks: request s has the heights from .. upto - 1.  Every lane counts the blocks of height B and more for a
+// B of its own, so that a pass narrows the heights to a 64th.  The time of a pass grows with the requests (64 of 3 tokens: 18 -> 27
+// microseconds, against 19 in the order of the requests), whose portions are short where they are many: then the requests one after the other, each
+// from its last block to its first.
+#define AW_SORTED 8
+__device__ __forceinline__ bool block_of(const WideArgs& a, int i, int lane, int& bi, int& blk, int& row0, int& count, int& end) {
+    auto blocks = [&](int tokens) { return a.tok_magic ? (int)__umulhi((unsigned)tokens, a.tok_magic) : tokens; };
+    int from, upto, row, tokens, keys;
+    auto heights = [&](int base) {  // of request base + lane
+        from = upto = row = tokens = keys = 0;
+        const int s = a.seq_begin + base + lane;
+        if (base + lane >= a.n_seqs) return;
+        row = a.cu_seqlens[s], tokens = a.cu_seqlens[s + 1] - row, keys = a.context_lens[s];
+        if (keys <= 0 || tokens <= 0) return;
+        from = blocks(keys > tokens ? keys - tokens : 0);
+        upto = from + blocks(tokens + a.tok - 1);
+    };
+    auto found = [&](int at, int request, int block) {
+        bi = request, blk = block;
+        row0 = __builtin_amdgcn_readlane(row, at), count = __builtin_amdgcn_readlane(tokens, at), end = __builtin_amdgcn_readlane(keys, at);
+        return true;
+    };
+    if (a.n_seqs > 1 && a.n_seqs <= AW_SORTED) {
+        heights(0);
+        int lo = -1, hi = blocks(a.max_blocks * a.block_size) + 2, at_hi = 0;  // (a request's keys fit its pages: no block is as high)
+        while (hi - lo > 1) {
+            const int stride = (hi - lo + LLMS_WAVE - 1) / LLMS_WAVE, height = lo + (lane + 1) * stride;
+            int higher = 0;
+            for (int j = 0; j < a.n_seqs; ++j)
+                higher += max(__builtin_amdgcn_readlane(upto, j) - max(__builtin_amdgcn_readlane(from, j), height), 0);
+            const int c = __popcll(__ballot(higher > i));  // (at most 63: none is as high as hi)
+            lo += c * stride;
+            if (lo + stride < hi) hi = lo + stride, at_hi = __builtin_amdgcn_readlane(higher, c);
+        }
+        if (lo < 0) return false;
+        const bool there = from <= lo && lo < upto;
+        const unsigned long long all = __ballot(there);
+        const int at = __ffsll(__ballot(there && __popcll(all & ((1ull << lane) - 1)) == i - at_hi)) - 1;
+        return found(at, at, lo - __builtin_amdgcn_readlane(from, at));
+    }
+    for (int base = 0; base < a.n_seqs; base += LLMS_WAVE) {
+        heights(base);
+        int last = upto - from;  // behind request base + lane's blocks
+        if (a.n_seqs > 1) {
+#pragma unroll
+            for (int d = 1; d < LLMS_WAVE; d *= 2) {
+                const int before = __shfl_up(last, d, LLMS_WAVE);
+                if (lane >= d) last += before;
+            }
+        }
+        const unsigned long long behind = __ballot(last > i);
+        if (behind) {
+            const int at = __ffsll(behind) - 1;
+            return found(at, base + at, __builtin_amdgcn_readlane(last, at) - 1 - i);
+        }
+        i -= __builtin_amdgcn_readlane(last, LLMS_WAVE - 1);
+    }
+    return false;
+}
+
 template <int TK, int DT, int U, bool PARTS, bool SHARED, bool MIXED>
 __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const WideArgs a) {
     extern __shared__ float lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / LLMS_WAVE), lane = threadIdx.x % LLMS_WAVE;
     const int nwaves = blockDim.x / LLMS_WAVE;
     const int col = lane % 16, q4 = lane / 16;
-    const int bi = blockIdx.x % a.n_seqs, b = a.seq_begin + bi, blk = a.blocks_per_seq - 1 - blockIdx.x / a.n_seqs;
-    const int row0 = a.cu_seqlens[b], count = a.cu_seqlens[b + 1] - row0, end = a.context_lens[b];
-    const int t0 = blk * a.tok;
-    if (t0 >= count || end <= 0) return;  // (the same for every thread of the workgroup)
+    int bi = blockIdx.x, blk = 0, row0, count, end;
+    if constexpr (PARTS) {
+        row0 = a.cu_seqlens[a.seq_begin + bi], count = a.cu_seqlens[a.seq_begin + bi + 1] - row0, end = a.context_lens[a.seq_begin + bi];
+        if (count <= 0 || end <= 0) return;  // (the same for every thread of the workgroup, as below)
+    } else if (!block_of(a, blockIdx.x, lane, bi, blk, row0, count, end)) return;
+    const int b = a.seq_begin + bi, t0 = blk * a.tok;
     const int ntok = count - t0 < a.tok ? count - t0 : a.tok;
     const int pos_lo = end - count + t0, pos_hi = pos_lo + ntok - 1;
     // (the constant address space: a page's number stays a scalar load also behind a barrier, where the compiler would take it for
@@ -552,16 +620,16 @@ static int launch(const WideArgs& a, int dk, int width, dim3 grid, int threads, 
 
 extern "C" {
 
-// `units` > 0: portions of prompts, workgroups of `units` (1, or 2 up to 128 columns of values) units of tokens.  units = 0:
+// `rows`: rows of q.  `units` > 0: portions of prompts, workgroups of `units` (1, or 2 up to 128 columns of values) units of tokens.  units = 0:
 // requests that bring one token, their keys shared out to `shares` workgroups, with the workspaces ws_o and ws_stats.
 int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_stride, const void* k_pool, const void* v_pool,
                               const int* block_tables, const int* table_rows, int max_blocks, const int* cu_seqlens,
-                              const int* context_lens, int seq_begin, int n_seqs, int max_new, int heads, int kv_heads, int maps,
+                              const int* context_lens, int seq_begin, int n_seqs, int max_new, int rows, int heads, int kv_heads, int maps,
                               int dk, int dv, int block_size, int window, int keep_first, int chunk, float scale,
                               const float* slopes, const float* talk, float lambda, int head_norm, float eps, float out_scale,
                               int sink, int units, int shared, int shares, float* ws_o, float* ws_stats, hipStream_t stream) {
     const int width = talk ? kv_heads * dv : dv;
-    LLMS_REQUIRE(n_seqs > 0 && max_new > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads / kv_heads <= 16,
+    LLMS_REQUIRE(n_seqs > 0 && max_new > 0 && rows >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0 && heads / kv_heads <= 16,
                  "attend_composed_wide: up to 16 query heads per key/value head");
     LLMS_REQUIRE((maps == 1 || maps == 2) && !(talk && (maps != 1 || sink || head_norm)), "attend_composed_wide: one or two maps; mixed heads with one, no sink and no norm");
     LLMS_REQUIRE((dk == 64 || dk == 128) && dv > 0 && dv % 16 == 0 && (width == 64 || width == 128 || width == 256) && (talk || dv <= 128),
@@ -585,12 +653,13 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
     if (units > 0) {
         a.heads_per_wg = talk ? kv_heads : maps, a.shares = 1;
         LLMS_REQUIRE((units == 1 || (units == 2 && width <= 128)) && a.heads_per_wg <= 8, "attend_composed_wide: up to 8 waves, of two units up to 128 columns of values");
-        a.tok = units * a.tpw, a.blocks_per_seq = (max_new + a.tok - 1) / a.tok;
+        a.tok = units * a.tpw, a.tok_magic = a.tok > 1 ? (unsigned)((0x100000000ull + a.tok - 1) / a.tok) : 0;
         const size_t lds = talk        ? ((size_t)a.tok * heads * (dv + 16) + (size_t)heads * heads) * sizeof(float)
                            : maps == 2 ? (size_t)units * 16 * dv * sizeof(float)
                                        : 0;
         LLMS_REQUIRE(lds <= 160 * 1024, "attend_composed_wide: too many heads for the LDS");
-        const dim3 grid(n_seqs * a.blocks_per_seq, 1, talk ? 1 : kv_heads);
+        const long most = (long)n_seqs * ((max_new + a.tok - 1) / a.tok), held = rows / a.tok + n_seqs;  // (blocks of portions as long as the longest, and that `rows` rows make)
+        const dim3 grid((unsigned)(held < most ? held : most), 1, talk ? 1 : kv_heads);
         if (shared) {
             LLMS_REQUIRE(talk && units == 1 && kv_heads >= 4 && dk == 64 && width == 256, "attend_composed_wide: shared values with 4 to 8 mixed key/value heads, keys of 64 and 256 columns of values");
             const size_t turns = 2 * (size_t)width * 64, all = lds > turns ? lds : turns;
@@ -601,7 +670,7 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
     }
     LLMS_REQUIRE(max_new == 1 && shares >= 1 && shares <= AW_SHARES && ws_o && ws_stats, "attend_composed_wide: one token a request, up to 16 shares, and their workspaces");
     a.heads_per_wg = a.score_heads < 4 ? a.score_heads : 4;
-    a.tok = 1, a.blocks_per_seq = 1, a.shares = shares;
+    a.tok = 1, a.shares = shares;
     const int zs = (a.score_heads + a.heads_per_wg - 1) / a.heads_per_wg;
     LLMS_REQUIRE(zs <= 65535 && heads <= 65535, "attend_composed_wide: too many heads");
     const size_t mix_lds = ((size_t)heads * 20 + (size_t)a.grp * heads) * sizeof(float);

@@ -1751,7 +1751,7 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
     _check(load("attention_composed_wide").llms_attend_composed_wide(
         _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
         _ptr(table_rows), c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), c_int(seq_begin),
-        c_int(n_seqs), c_int(max_new), c_int(heads), c_int(kv_heads), c_int(maps), c_int(dk), c_int(dv),
+        c_int(n_seqs), c_int(max_new), c_int(q.shape[0]), c_int(heads), c_int(kv_heads), c_int(maps), c_int(dk), c_int(dv),
         c_int(block_size), c_int(window), c_int(keep_first), c_int(chunk), c_float(scale), _ptr(slopes), _ptr(talk),
         c_float(lam), c_int(1 if head_norm else 0), c_float(eps), c_float(out_scale), c_int(1 if sink else 0),
         c_int(units), c_int(1 if shared else 0), c_int(shares), _ptr(ws_o), _ptr(ws_stats), _stream(dev)), "attend_composed_wide")

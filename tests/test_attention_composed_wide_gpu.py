@@ -152,3 +152,45 @@ def test_heads_that_are_subtracted_from_one_another(heads, kv, dk, dv, scale, mo
             monkeypatch.setattr(ops, "wide_prompt_shared", lambda *a: shared)
             assert _relative_error(run(seqs, 16, shares=3, **kw), refs) <= 2.0 ** -8
         assert _relative_error(attend_mfma(seqs, 16, **kw), refs) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("counts", [[2], [1, 40], [0, 33, 2], [70, 1, 0, 5, 31, 2, 64, 1], [3, 0, 50, 1, 2, 9, 0, 17, 4], [1 + i % 4 for i in range(70)]])
+def test_portions_of_ragged_lengths(counts, maps, monkeypatch):
+    """Which workgroup takes which block of which request (one request, up to 8, more, and more than a wave's lanes; requests without
+    rows and without keys between them) changes no result: each request's rows are the same numbers as in a launch of its own."""
+    from llmserve.ops import library as ops
+
+    monkeypatch.setattr(ops, "wide_prompt_units", lambda *a: 1 if maps == 1 else 2)
+    monkeypatch.setattr(ops, "wide_prompt_shared", lambda *a: False)
+    heads, kv, dk, dv, bs = (8, 2, 64, 32, 16) if maps == 1 else (4, 2, 64, 64, 16)
+    dt, gen = torch.bfloat16, torch.Generator().manual_seed(len(counts))
+    rows, n = sum(counts), len(counts)
+    ends = [c + 7 * (i % 5) if c else (11 if i % 2 else 0) for i, c in enumerate(counts)]
+    if n > 3:
+        ends[3] = 0  # padding: left alone
+    width = -(-max(ends) // bs)
+    q = torch.randn(rows, heads * maps * dk, generator=gen).to(dt).to(DEV)
+    pages = n * width
+    k_pool = torch.randn(pages, kv * maps, bs, dk, generator=gen).to(dt).to(DEV)
+    v_pool = torch.randn(pages, kv, dv, bs, generator=gen).to(dt).to(DEV)
+    table = torch.randperm(pages, generator=gen).int().view(n, width).to(DEV)
+    cu = [0]
+    for c in counts:
+        cu.append(cu[-1] + c)
+    cu_d, ends_d = torch.tensor(cu, dtype=torch.int32, device=DEV), torch.tensor(ends, dtype=torch.int32, device=DEV)
+    kw = dict(heads=heads, kv_heads=kv, dk=dk, dv=dv, block_size=bs, scale=0.1, maps=maps)
+    if maps == 1:
+        kw["talk"] = (torch.eye(heads) + 0.1 * torch.randn(heads, heads, generator=gen)).to(DEV)
+    else:
+        kw.update(lam=0.8, head_norm=True, eps=1e-5, out_scale=0.5)
+    out = torch.full((rows, heads * dv), 7.0, dtype=dt, device=DEV)
+    ops.attend_composed_wide(out, q, k_pool, v_pool, table, cu_d, ends_d, 0, n, max(2, max(counts)), **kw)
+    alone = torch.full_like(out, 7.0)
+    for s in range(n):
+        ops.attend_composed_wide(alone, q, k_pool, v_pool, table, cu_d, ends_d, s, 1, max(2, counts[s]), **kw)
+    assert torch.equal(out, alone)
+    seen = [s for s in range(n) if ends[s] > 0 and counts[s]]
+    for s in range(n):
+        part = out[cu[s]:cu[s + 1]]
+        assert bool((part != 7.0).any(1).all()) if s in seen else bool((part == 7.0).all())
