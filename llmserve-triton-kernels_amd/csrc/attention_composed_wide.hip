@@ -16,9 +16,12 @@
 // to 2.5e-3; with one rounded number a weight 2.0e-3 to 1.2e-1, the pairs up to 0.7.  A third number changes the fourth digit.
 //
 // A unit is 16 columns that share a key row: `tpw` neighbouring tokens times the `grp` query heads of a key/value head.  Per
-// step of 32 keys (two tiles of 16) a wave forms S^T = K Q^T with v_mfma_f32_16x16x32_bf16; a lane then holds keys 4 q4 .. + 3 of
-// both tiles for its column, which is the B operand of O^T = V^T P^T when the values' A operand takes its 8 keys in the
-// same order.  Pages hold a multiple of 16 keys, so a tile's page and place are scalars and a lane adds its own fixed offset.
+// step of 32 keys (two tiles of 16) a wave forms S^T = K Q^T with v_mfma_f32_16x16x32_bf16, two products whose rows are the keys
+// 8 (i / 4) + 4 u + i % 4; a lane then holds keys 8 q4 .. + 7 of the 32 for its column, which is the B operand of O^T = V^T P^T, and the
+// values' A operand is one load of 16 bytes.  (With a tile a product, a lane's keys were 4 of each tile and its values two loads of 8: a load
+// instruction takes its turn whatever it brings.  Microseconds, 32 heads of 64 on 4: 2 tokens behind 1,278 64 -> 55, 333 tokens 27.2 ->
+// 24.9, 2,048 tokens 174 -> 157, 4 single tokens behind 1,000 13.2 -> 12.3; two maps, 2,048 tokens 105 -> 91, but 210 tokens behind 890
+// 31.9 -> 33.0.)  Pages hold a multiple of 16 keys, so a tile's page and place are scalars, and a lane chooses between two.
 //
 //   attend_wide_kernel<.., PARTS = true>   requests that bring one token: the keys go to `shares` workgroups, whose maxima, sums
 //       and results (32-bit) a second kernel joins: combine_mixed_kernel or combine_maps_kernel.
@@ -31,12 +34,12 @@
 // chain of two launches and of lengths -> table -> keys -> results; for portions the answers to a step's values.
 // Measured against that kernel, microseconds (mixed: 32 heads of 64 on 4 key/value heads; maps: 16 heads of two maps of 64 on 2,
 // values of 128):
-//     4 requests, one token behind   300 keys    mixed 22.1 -> 12.1    maps 18.4 ->  9.0
-//     4 requests, one token behind 1,000 keys    mixed 24.9 -> 12.5    maps 31.7 ->  9.8
+//     4 requests, one token behind   300 keys    mixed 22.1 -> 11.1    maps 18.4 ->  8.9
+//     4 requests, one token behind 1,000 keys    mixed 24.9 -> 12.3    maps 31.7 ->  9.8
 //   256 requests, one token behind 1,000 keys    mixed  130 ->   72    maps 50.4 -> 51.1 (5 TB/s of keys and values)
-//     a prompt of   333 tokens                   mixed  152 ->   27    maps 35.7 -> 13.5
-//     a prompt of 2,048 tokens                   mixed  819 ->  167    maps  284 ->   99
-// (Mixed with one number a weight: 11.8, 12.3, 72, 26 and 154.)  Two maps, whose weights are one number in both kernels, are 2.2 to
+//     a prompt of   333 tokens                   mixed  152 ->   25    maps 35.7 -> 13.9
+//     a prompt of 2,048 tokens                   mixed  819 ->  155    maps  284 ->   89
+// (Mixed with two numbers a weight costs 0 to 8 % more than with one.)  Two maps, whose weights are one number in both kernels, are 2.2 to
 // 2.5e-3 from 64 bits in both.
 //
 // Masks as in attention_composed_mfma.hip: a column at position i sees j <= i with j >= its chunk's start and (i - j < window or
@@ -49,7 +52,6 @@
 #define AW_NO_KEY 0x40000000
 #define AW_PIECES 2  // of a weight, where heads are mixed behind the value products
 
-typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -75,6 +77,7 @@ struct WideArgs {
     int dv, block_size, k_page, v_page;  // k_page, v_page: elements of a page
     int window, keep_first, chunk;
     int tok, tpw, shares;
+    int talk_at;  // where the mixing matrix lies in LDS (portions of prompts; in floats)
     unsigned bs_magic;  // ceil(2^32 / block_size)
     unsigned tok_magic;  // ceil(2^32 / tok) (0: tok is 1)
     float scale, lambda, eps, out_scale;
@@ -105,7 +108,7 @@ __device__ __forceinline__ uint32_t low_half_mask(int keep) { return keep <= 0 ?
 // Workgroup i's request and block of tokens; the workgroups that find none lie behind all that do.  With a grid of every request's longest
 // possible portion, workgroups without tokens lay between those with some, and as workgroups go around the parts of the chip in
 // turn, parts of it met only empty ones (32 heads of 64 on 4, microseconds: 811, 890, 150 and 197 tokens 156 -> 91, twice 1,024 beside
-// two of 1 token 190 -> 104, without those 104; 16 heads of two maps on 2: 57 -> 48 and 73 -> 56).
+// two of 1 token 190 -> 104, without those 104; 16 heads of two maps on 2: 57 -> 48 and 73 -> 56; 77 and 44 are the first and third now).
 // Up to AW_SORTED requests: the block with the i-th most keys, so that no long one begins late.  A block's height is its place from its
 // request's beginning, in blocks: request s has the heights from .. upto - 1.  Every lane counts the blocks of height B and more for a
 // B of its own, so that a pass narrows the heights to a 64th.  The time of a pass grows with the requests (64 of 3 tokens: 18 -> 27
@@ -224,8 +227,12 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
     const float slope = sloped ? a.slopes[h] * LOG2E : 0.f;
     const float scale2 = a.scale * LOG2E;
 
-    const bf16* k_head = a.k_pool + (size_t)head * bs * DK + col * DK + 8 * q4;
-    const bf16* v_head = a.v_pool + (size_t)(MIXED ? 0 : kvh) * a.dv * bs + col * bs + 4 * q4;
+    // a lane's keys of a step: as a row of the score products the key 8 (col / 4) + 4 u + col % 4 of product u, as a column of them the
+    // keys 8 q4 .. 8 q4 + 7, of 32: both of one tile
+    const bool k_second = col >= 8, second = q4 >= 2;
+    const int first_key = 8 * (q4 % 2);
+    const bf16* k_head = a.k_pool + (size_t)head * bs * DK + (8 * (col / 4 % 2) + col % 4) * DK + 8 * q4;
+    const bf16* v_head = a.v_pool + (size_t)(MIXED ? 0 : kvh) * a.dv * bs + col * bs + first_key;
     struct Place {
         int page, in_page;
     };
@@ -236,11 +243,12 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         return Place{page < 0 ? 0 : page, j - block * bs};
     };
     auto ask_keys = [&](const Place at[2], bf16x8v kf[2][TK]) {
+        const size_t rows[2] = {(size_t)at[0].page * a.k_page + at[0].in_page * DK, (size_t)at[1].page * a.k_page + at[1].in_page * DK};
+        const bf16* row = k_head + (k_second ? rows[1] : rows[0]);
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int t = 0; t < TK; ++t)
-                kf[tt][t] = *reinterpret_cast<const bf16x8v*>(k_head + (size_t)at[tt].page * a.k_page + at[tt].in_page * DK + 32 * t);
+            for (int t = 0; t < TK; ++t) kf[u][t] = *reinterpret_cast<const bf16x8v*>(row + 4 * u * DK + 32 * t);
     };
 
     f32x4 o[U][DT];
@@ -252,8 +260,8 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         for (int d = 0; d < DT; ++d) o[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // SHARED: a step's values go through LDS (2,048 tokens of 32 heads on 4: 206 -> 167 microseconds), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
-    // (one per key/value head, at least 4) all read all of them.  A chunk is 32 dimensions of a tile, 16 bytes a lane;
+    // SHARED: a step's values go through LDS (1,500 tokens of 32 heads on 8 of 32: 105 -> 102 microseconds), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
+    // (one per key/value head) all read all of them.  A chunk is 32 dimensions of a tile, 16 bytes a lane;
     // the two halves of dimensions 8 to 15 of every 16 change places, so that 32 lanes read 64 banks.
     constexpr int CHUNKS = SHARED ? DT / 4 : 1;
     uint16_t* v_lds = reinterpret_cast<uint16_t*>(lds);
@@ -293,6 +301,20 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         ask_keys(at, kf);
         if constexpr (SHARED) store_chunks(0);
     }
+    if constexpr (MIXED && !PARTS) {  // the mixing matrix, [h][g] with a row of H + 1, behind what else is in LDS: it comes beside the first step's keys
+        for (int h0 = wave; h0 < a.heads; h0 += 8 * nwaves)
+            for (int g = lane; g < a.heads; g += LLMS_WAVE) {
+                float t[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int hr = h0 + e * nwaves;
+                    t[e] = a.talk[(size_t)(hr < a.heads ? hr : h0) * a.heads + g];
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (h0 + e * nwaves < a.heads) lds[a.talk_at + (h0 + e * nwaves) * (a.heads + 1) + g] = t[e];
+            }
+    }
     int turn = 0;
     for (int step = share; step < n_steps; step += a.shares) {
         const int next = step + a.shares;
@@ -300,41 +322,42 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
             __syncthreads();  // this step's values are in LDS, and the turn before has been read
             if (next < n_steps) ask_chunks(next_at, next);
         }
-        s16x4 vf[HALVES][2][DT / HALVES];
+        u32x4 vf[HALVES][DT / HALVES];
         auto ask_values = [&](int half) {
+            const size_t tiles[2] = {(size_t)at[0].page * a.v_page + at[0].in_page, (size_t)at[1].page * a.v_page + at[1].in_page};
+            const bf16* vt = v_head + (second ? tiles[1] : tiles[0]) + (size_t)half * (DT / HALVES) * 16 * bs;
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const bf16* vt = v_head + (size_t)at[tt].page * a.v_page + at[tt].in_page + (size_t)half * (DT / HALVES) * 16 * bs;
-#pragma unroll
-                for (int d = 0; d < DT / HALVES; ++d) vf[half][tt][d] = *reinterpret_cast<const s16x4*>(vt + (size_t)16 * d * bs);
-            }
+            for (int d = 0; d < DT / HALVES; ++d) vf[half][d] = *reinterpret_cast<const u32x4*>(vt + (size_t)16 * d * bs);
         };
         if constexpr (!SHARED) ask_values(0);
         if (next < n_steps) ask_keys(next_at, next_kf);
         if constexpr (SHARED) {  // (all of them, asked for before the scores: their way through LDS passes beside the softmax)
-            const uint16_t* from = v_lds + turn * (DT * 512) + col * 16 + 4 * (q4 ^ (2 * (col / 8)));
+            const uint16_t* from = v_lds + turn * (DT * 512) + (q4 / 2) * (DT * 256) + col * 16 + 8 * ((q4 % 2) ^ (col / 8));
 #pragma unroll
-            for (int d = 0; d < DT; ++d)
-                vf[0][0][d] = *reinterpret_cast<const s16x4*>(from + 256 * d), vf[0][1][d] = *reinterpret_cast<const s16x4*>(from + 256 * (DT + d));
+            for (int d = 0; d < DT; ++d) vf[0][d] = *reinterpret_cast<const u32x4*>(from + 256 * d);
             __builtin_amdgcn_sched_barrier(0);
         }
         const Place after_at[2] = {place_of(2 * (next + a.shares)), place_of(2 * (next + a.shares) + 1)};
         int j0[2];
         j0[0] = tile_start(2 * step), j0[1] = 2 * step + 1 < n_tiles ? tile_start(2 * step + 1) : AW_NO_KEY;
+        const int lane_key = (second ? j0[1] : j0[0]) + first_key;
         bf16x8v pf[U][PIECES];
         float corr[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float sc[2][4], mx = -INFINITY;
+            // every column of the unit sees all 32 keys (the same answer in every lane)
+            bool whole = true;
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+                whole = whole && j0[tt] + 15 <= pmin[u] && (a.chunk <= 0 || j0[tt] >= pmax[u] / a.chunk * a.chunk) &&
+                        (a.window <= 0 || pmax[u] - j0[tt] < a.window);
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int t = 0; t < TK; ++t) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[tt][t], qf[u][t], acc, 0, 0, 0);
-                const int key0 = j0[tt] + 4 * q4;
-                // every column of the unit sees all 16 keys (the same answer in every lane)
-                const bool whole = j0[tt] + 15 <= pmin[u] && (a.chunk <= 0 || j0[tt] >= pmax[u] / a.chunk * a.chunk) &&
-                                   (a.window <= 0 || pmax[u] - j0[tt] < a.window);
+                const int key0 = lane_key + 4 * tt;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) sc[tt][r] = acc[r] * scale2;
                 if (sloped) {
@@ -377,20 +400,13 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         for (int half = 0; half < HALVES; ++half) {
             if (!SHARED && tail) {
 #pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    const int keep = end - (j0[tt] + 4 * q4);
-                    const uint32_t lo = low_half_mask(keep), hi = low_half_mask(keep - 2);
+                for (int d = 0; d < DT / HALVES; ++d)
 #pragma unroll
-                    for (int d = 0; d < DT / HALVES; ++d) {
-                        u32x2 v = __builtin_bit_cast(u32x2, vf[half][tt][d]);
-                        v.x &= lo, v.y &= hi;
-                        vf[half][tt][d] = __builtin_bit_cast(s16x4, v);
-                    }
-                }
+                    for (int e = 0; e < 4; ++e) vf[half][d][e] &= low_half_mask(end - lane_key - 2 * e);
             }
 #pragma unroll
             for (int d = 0; d < DT / HALVES; ++d) {
-                const bf16x8v v = __builtin_bit_cast(bf16x8v, __builtin_shufflevector(vf[half][0][d], vf[half][1][d], 0, 1, 2, 3, 4, 5, 6, 7));
+                const bf16x8v v = __builtin_bit_cast(bf16x8v, vf[half][d]);
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     f32x4& to = o[u][half * (DT / HALVES) + d];
@@ -464,9 +480,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         // one key/value head's values at a time: [token][head g][dv + 16] in LDS (the pad puts 4 heads on different banks),
         // then a job is a token's 16 dimensions of that key/value head's query heads, 4 heads g an instruction
         const int H = a.heads, dv = a.dv, dvt = dv / 16, pad = dv + 16, G = H / a.grp;
-        float* talk_s = lds + (size_t)a.tok * H * pad;  // [g][h]
-        if (SHARED) __syncthreads();  // (the values' place is free)
-        for (int i = threadIdx.x; i < H * H; i += blockDim.x) talk_s[(i % H) * H + i / H] = a.talk[i];
+        const float* talk_s = lds + a.talk_at;
         float inv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) inv[u] = 1.f / run_l[u];
@@ -478,7 +492,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
                     float* at_col = lds + ((size_t)(u * a.tpw + col / a.grp) * H + h) * pad + 4 * q4;
 #pragma unroll
                     for (int d = 0; d < DT; ++d)  // (constant indexes of the results: the others are skipped)
-                        if (d / dvt == k) *reinterpret_cast<f32x4*>(at_col + 16 * (d - k * dvt)) = o[u][d] * inv[u];
+                        if (d >= k * dvt && d < (k + 1) * dvt) *reinterpret_cast<f32x4*>(at_col + 16 * (d - k * dvt)) = o[u][d] * inv[u];
                 }
             __syncthreads();
             for (int job = wave; job < ntok * dvt; job += nwaves) {
@@ -487,10 +501,17 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
                 const int ho = k * a.grp + (mine ? col : 0);
                 const float* from = lds + (size_t)tl * H * pad + d0 + col;
                 f32x4 mixed = {0.f, 0.f, 0.f, 0.f};
-                for (int g0 = 0; g0 < H; g0 += 4) {
-                    const int g = g0 + q4;
-                    const float ug = g < H ? from[g * pad] : 0.f, tg = g < H ? talk_s[g * H + ho] : 0.f;
-                    mixed = __builtin_amdgcn_mfma_f32_16x16x4f32(ug, tg, mixed, 0, 0, 0);
+                for (int g0 = 0; g0 < H; g0 += 32) {  // (32 heads asked for before the first product)
+                    float ug[8], tg[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int g = g0 + 4 * e + q4, gr = g < H ? g : H - 1;
+                        ug[e] = from[gr * pad], tg[e] = talk_s[ho * (H + 1) + gr];
+                        if (g >= H) ug[e] = 0.f, tg[e] = 0.f;
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (g0 + 4 * e < H) mixed = __builtin_amdgcn_mfma_f32_16x16x4f32(ug[e], tg[e], mixed, 0, 0, 0);
                 }
                 if (mine) {
                     *reinterpret_cast<u32x2*>(a.out + (size_t)(row0 + t0 + tl) * a.out_stride + (size_t)ho * dv + d0 + 4 * q4) =
@@ -654,7 +675,9 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
         a.heads_per_wg = talk ? kv_heads : maps, a.shares = 1;
         LLMS_REQUIRE((units == 1 || (units == 2 && width <= 128)) && a.heads_per_wg <= 8, "attend_composed_wide: up to 8 waves, of two units up to 128 columns of values");
         a.tok = units * a.tpw, a.tok_magic = a.tok > 1 ? (unsigned)((0x100000000ull + a.tok - 1) / a.tok) : 0;
-        const size_t lds = talk        ? ((size_t)a.tok * heads * (dv + 16) + (size_t)heads * heads) * sizeof(float)
+        const size_t results = (size_t)a.tok * heads * (dv + 16), turns = shared ? (size_t)width * 32 : 0;  // (floats; they take turns in LDS)
+        a.talk_at = (int)(results > turns ? results : turns);
+        const size_t lds = talk        ? ((size_t)a.talk_at + (size_t)heads * (heads + 1)) * sizeof(float)
                            : maps == 2 ? (size_t)units * 16 * dv * sizeof(float)
                                        : 0;
         LLMS_REQUIRE(lds <= 160 * 1024, "attend_composed_wide: too many heads for the LDS");
@@ -662,8 +685,7 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
         const dim3 grid((unsigned)(held < most ? held : most), 1, talk ? 1 : kv_heads);
         if (shared) {
             LLMS_REQUIRE(talk && units == 1 && kv_heads >= 4 && dk == 64 && width == 256, "attend_composed_wide: shared values with 4 to 8 mixed key/value heads, keys of 64 and 256 columns of values");
-            const size_t turns = 2 * (size_t)width * 64, all = lds > turns ? lds : turns;
-            return launch_one<2, 16, 1, false, true, true>(a, grid, kv_heads * LLMS_WAVE, all, stream);
+            return launch_one<2, 16, 1, false, true, true>(a, grid, kv_heads * LLMS_WAVE, lds, stream);
         }
         return units == 2 ? launch<2, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream)
                           : launch<1, false>(a, dk, width, grid, a.heads_per_wg * LLMS_WAVE, lds, stream);

@@ -1746,8 +1746,8 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
         ws_o = torch.empty(columns * (kv_heads * dv if talk is not None else dv), dtype=torch.float32, device=dev)
         ws_stats = torch.empty(2 * columns, dtype=torch.float32, device=dev)
     else:
-        units = wide_prompt_units(heads, kv_heads, dv, talk is not None, n_seqs, max_new, compute_units(dev))
-        shared = wide_prompt_shared(heads, kv_heads, dk, dv, talk is not None, n_seqs, max_new, compute_units(dev))
+        units = wide_prompt_units(heads, kv_heads, dv, talk is not None, n_seqs, max_new, q.shape[0], compute_units(dev))
+        shared = wide_prompt_shared(heads, kv_heads, dk, dv, talk is not None)
     _check(load("attention_composed_wide").llms_attend_composed_wide(
         _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
         _ptr(table_rows), c_int(block_tables.shape[1]), _ptr(cu_seqlens), _ptr(context_lens), c_int(seq_begin),
@@ -1758,26 +1758,28 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
     return out
 
 
-def wide_prompt_units(heads: int, kv_heads: int, dv: int, talk: bool, n_seqs: int, max_new: int, cus: int) -> int:
-    """Units of 16 columns a wave of `attend_composed_wide` takes over portions of prompts.  Two share every key and value a wave
-    reads, one gives twice the workgroups (16 heads of two maps over 64, values of 128: 2,000 tokens of 4 requests in 440
-    workgroups of two 56 microseconds, in 890 of one 105; 100 tokens in 112 or 224 of them 48 and 39).  The results of two
-    units of 256 columns do not fit a wave's registers, and mixed heads, whose weights are two numbers each, are faster with one (8
-    heads of 128 on 1, 2,048 tokens: 72 against 95; 4 requests of 512: 26 and 35; 16 heads on 4 of 32, 2,048 tokens: 92 and 95)."""
+def wide_prompt_units(heads: int, kv_heads: int, dv: int, talk: bool, n_seqs: int, max_new: int, rows: int, cus: int) -> int:
+    """Units of 16 columns a wave of `attend_composed_wide` takes over portions of prompts, of `rows` rows together.  Two share every
+    key and value a wave reads, one gives twice the workgroups, which count for more until every compute unit has several of two
+    units (16 heads of two maps over 64, values of 128, microseconds with one unit and with two: 1,100 tokens, 550 workgroups of two, 47 and
+    56; twice 700 tokens 34 and 37; 1,500 tokens, 750, 70 and 69; 2,048 tokens, 1,024, 118 and 89; 4 times 512 35 and 30; 811, 890,
+    150 and 197 52 and 44).  The results of two units of 256 columns do not fit a wave's registers, and mixed heads, whose weights
+    are two numbers each, are faster with one (8 heads of 128 on 1, 2,048 tokens: 72 against 95; 4 requests of 512: 26 and 35; 16
+    heads on 4 of 32, 2,048 tokens: 92 and 95)."""
     if talk or dv > 128:
         return 1
-    workgroups = n_seqs * -(-max_new // (2 * (16 // (heads // kv_heads)))) * kv_heads
-    return 2 if workgroups >= cus else 1
+    tokens = 2 * (16 // (heads // kv_heads))
+    workgroups = min(n_seqs * -(-max_new // tokens), rows // tokens + n_seqs) * kv_heads
+    return 2 if workgroups >= 3 * cus else 1
 
 
-def wide_prompt_shared(heads: int, kv_heads: int, dk: int, dv: int, talk: bool, n_seqs: int, max_new: int, cus: int) -> bool:
+def wide_prompt_shared(heads: int, kv_heads: int, dk: int, dv: int, talk: bool) -> bool:
     """Whether the waves of a workgroup of `attend_composed_wide` share the values of a step through LDS (256 columns of values, all
-    read by at least 4 waves).  Where a SIMD has two waves or more, reading them once a workgroup counts for more than the
-    barrier a step and the way through LDS (microseconds, each wave for itself -> shared, 32 heads of 64 on 4: 1,100 tokens 84 -> 75,
-    2,048 tokens 206 -> 167; 8 heads on 8 of 32: 333 tokens 46 -> 42); a single wave a SIMD waits for each step's barrier (333
-    tokens 26.9 -> 30.7, 512 behind 488 others 54 -> 66)."""
-    workgroups = n_seqs * -(-max_new // (16 // (heads // kv_heads)))
-    return talk and dk == 64 and kv_heads * dv == 256 and kv_heads >= 4 and (kv_heads > 4 or workgroups > cus)
+    read by at least 4 waves).  A load of 16 bytes brings what two brought, and four waves that each ask for the values are now
+    mostly ahead of a barrier a step (microseconds, each wave for itself -> shared, 32 heads of 64 on 4: 333 tokens 24.8 -> 28.8, 1,100
+    67 -> 70, 1,500 92 -> 88, 2,048 154 -> 150, behind 1,500 others 311 -> 320; ragged portions 77 -> 79); eight are not (32 heads on 8 of 32:
+    1,100 tokens 84 -> 82, 1,500 105 -> 102, 2,048 behind 1,500 328 -> 326)."""
+    return talk and dk == 64 and kv_heads * dv == 256 and kv_heads > 4
 
 
 # ------------------------------------------------------------------------------ sampling
