@@ -1290,9 +1290,16 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
     LLMS_LAUNCH_CHECK();
 }
 
+// Whether `a` of na bytes and `b` of nb bytes have a byte in common.
+static bool gd_overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && b && x < y + nb && y < x + na;
+}
+
 // The product of up to 8 rows (K up to 4,096) that are made from a 32-bit stream x [M, K].  from 1: x + y / sqrt(mean(y^2) + eps) * w, rounded
-// to bfloat16, with that sum to x_out [M, K], which is not x (epilogue 0 with out_dtype 0, or 1).  from 2: x / sqrt(mean(x^2) + eps) *
-// (offset + w), rounded (epilogue 0 with out_dtype 0).  The product's rows go to h_out [M, K] if given.
+// to bfloat16, with that sum to x_out [M, K] (epilogue 0 with out_dtype 0, or 1).  from 2: x / sqrt(mean(x^2) + eps) *
+// (offset + w), rounded (epilogue 0 with out_dtype 0).  The product's rows go to h_out [M, K] if given.  Every workgroup reads all of x and y
+// while others store: no result may lie on them, or on another result.
 int llms_gemm_decode_stream(int out_dtype, int epilogue, void* C, int ldc, const void* W, const void* bias, int M, int N, int K, int inter, int unit,
                             float limit, int from, const float* x, float* x_out, void* h_out, const float* y, const float* w, float offset,
                             float eps, int workgroups, hipStream_t stream) {
@@ -1300,12 +1307,22 @@ int llms_gemm_decode_stream(int out_dtype, int epilogue, void* C, int ldc, const
                  "gemm_decode_stream: needs 1 <= M <= 8 and K a multiple of 8 up to 4,096");
     LLMS_REQUIRE(from == GD_FROM_OPEN || from == GD_FROM_NORM, "gemm_decode_stream: from must be 1 or 2");
     LLMS_REQUIRE((long long)N * K < (1ll << 30), "gemm_decode_stream: a weight of 2 GB or more");
-    LLMS_REQUIRE(C && W && x && w && (from == GD_FROM_NORM || (y && x_out && x_out != x)), "gemm_decode_stream: an operand is missing, or x_out is x");
+    LLMS_REQUIRE(C && W && x && w && (from == GD_FROM_NORM || (y && x_out)), "gemm_decode_stream: an operand is missing");
     LLMS_REQUIRE((uintptr_t)W % 16 == 0 && (uintptr_t)x_out % 16 == 0 && (uintptr_t)h_out % 16 == 0, "gemm_decode_stream: W and what is stored must be 16-byte aligned");
     LLMS_REQUIRE((epilogue == GD_PLAIN && out_dtype == 0 && ldc >= N && unit == 0) ||
                      (epilogue == GD_SWIGLU && out_dtype == 1 && from == GD_FROM_OPEN && inter > 0 && N == 2 * inter && ldc >= inter && !bias &&
                       (unit == 0 || unit == GD_UNIT_CLAMPED || unit == GD_UNIT_GELU)),
                  "gemm_decode_stream: 32-bit rows, or the gated epilogue with an open sum");
+    const size_t rows32 = (size_t)M * K * 4, rows16 = rows32 / 2, row_out = epilogue == GD_SWIGLU ? (size_t)inter * 2 : (size_t)N * 4;
+    if (from == GD_FROM_NORM) x_out = nullptr;
+    bool apart = !gd_overlap(x_out, rows32, x, rows32) && !gd_overlap(x_out, rows32, y, rows32) && !gd_overlap(h_out, rows16, x, rows32) &&
+                 !gd_overlap(h_out, rows16, y, rows32) && !gd_overlap(h_out, rows16, x_out, rows32);
+    for (int m = 0; m < M; ++m) {
+        const char* row = (const char*)C + (size_t)m * ldc * (out_dtype == 0 ? 4 : 2);
+        apart = apart && !gd_overlap(row, row_out, x, rows32) && !gd_overlap(row, row_out, y, rows32) && !gd_overlap(row, row_out, x_out, rows32) &&
+                !gd_overlap(row, row_out, h_out, rows16);
+    }
+    LLMS_REQUIRE(apart, "gemm_decode_stream: a result lies on the stream, on what joins it or on another result");
     LLMS_REQUIRE(workgroups > 0 && workgroups <= 4096, "gemm_decode_stream: bad number of workgroups");
     DecodeStreamArgs a{};
     a.W = (const bf16*)W;

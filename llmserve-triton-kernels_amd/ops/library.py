@@ -694,6 +694,16 @@ def _row_stride(t: torch.Tensor | None) -> int:
     return 0 if t is None else t.stride(0) if t.shape[0] > 1 else t.shape[1]
 
 
+def _spans(t: torch.Tensor | None) -> list[tuple[int, int]]:
+    """Where a matrix of unit inner stride lies: its first byte and the one behind its last, or row by row where there are gaps."""
+    if t is None:
+        return []
+    at, size = t.data_ptr(), t.element_size()
+    if t.is_contiguous():
+        return [(at, at + t.numel() * size)]
+    return [(at + r * t.stride(0) * size, at + (r * t.stride(0) + t.shape[1]) * size) for r in range(t.shape[0])]
+
+
 def gemm_decode_stream_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ops.gemm_decode_stream takes the float32 rows x [N, K] against the bfloat16 weight w."""
     n, k = x.shape
@@ -709,7 +719,8 @@ def gemm_decode_stream(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias
     """`gemm_decode` of up to 8 rows that the product makes from a float32 stream x [N, K] on its way in:
 
     joins = (y, y_weight, y_eps, x_out): the stream's open sum is closed, as `normed_add_norm` does without a norm behind it: the rows are
-            bf16(x + y / sqrt(mean(y^2) + y_eps) * y_weight); that sum goes to x_out (another tensor: x stays as it is).
+            bf16(x + y / sqrt(mean(y^2) + y_eps) * y_weight); that sum goes to x_out (another tensor: x stays as it is).  Every workgroup
+            reads x and y while others store: none of out, x_out and h_out may overlap them or each other.
     norm = (weight, eps, offset): the rows are `rmsnorm32` of x.
     h_out (bfloat16 [N, K]): takes the rows, for who else reads them.
     out: float32 [N, rows of w] (+ bias), or with `swiglu` (with `joins`) bfloat16 as for `gemm_decode`."""
@@ -720,8 +731,6 @@ def gemm_decode_stream(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias
     for t, what, dtype in ((x, "x", torch.float32), (y, "y", torch.float32), (x_out, "x_out", torch.float32), (h_out, "h_out", torch.bfloat16)):
         if t is not None and (t.dtype != dtype or tuple(t.shape) != (n, k) or not t.is_contiguous()):
             raise ValueError(f"{what} must be a contiguous {dtype} [{n}, {k}] tensor")
-    if x_out is not None and x_out.data_ptr() == x.data_ptr():
-        raise ValueError("x_out must not be x, which every workgroup reads")
     _f32(weight, "weight", k)
     _rows(w, "w", k)
     if not gemm_decode_stream_supported(x, w):
@@ -735,6 +744,11 @@ def gemm_decode_stream(out: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias
         raise ValueError("a limit and gelu go with the gated epilogue")
     if out.dim() != 2 or out.stride(1) != 1 or tuple(out.shape) != (n, cols) or out.dtype != (torch.bfloat16 if swiglu else torch.float32):
         raise ValueError(f"out must be [{n}, {cols}] with unit inner stride, float32 or for the gated epilogue bfloat16")
+    stored = [("x_out", _spans(x_out)), ("h_out", _spans(h_out)), ("out", _spans(out))]
+    for i, (what, spans) in enumerate(stored):
+        for other, those in [("x", _spans(x)), ("y", _spans(y)), *stored[:i]]:
+            if any(a < d and c < b for a, b in spans for c, d in those):
+                raise ValueError(f"{what} overlaps {other}, which other workgroups read or store")
     dev = _dev(out, x, w, bias, y, x_out, weight, h_out)
     _check(load("gemm_decode").llms_gemm_decode_stream(
         c_int(1 if swiglu else 0), c_int(1 if swiglu else 0), _ptr(out), c_int(_row_stride(out)), _ptr(w), _ptr(bias), c_int(n),
