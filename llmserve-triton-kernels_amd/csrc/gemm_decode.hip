@@ -1184,6 +1184,8 @@ int llms_gemm_decode(int out_dtype, int epilogue, void* C, int ldc, const void* 
     LLMS_REQUIRE(epilogue >= 0 && epilogue <= 3, "gemm_decode: epilogue must be 0..3");
     LLMS_REQUIRE(out_dtype == 1 || (out_dtype == 0 && (epilogue == GD_PLAIN || (epilogue == GD_RESIDUAL && M <= 16))),
                  "gemm_decode: 32-bit output goes with the plain epilogue, or the residual one of up to 16 rows");
+    LLMS_REQUIRE(!(epilogue == GD_RESIDUAL && out_dtype == 0) || (norm_weight == nullptr && (long long)(M - 1) * ldr + N < (1ll << 30)),
+                 "gemm_decode: a 32-bit residual goes without a norm, and its rows span less than 4 GB");
     LLMS_REQUIRE(gate_z == nullptr ? gate_bias == nullptr : epilogue == GD_RESIDUAL && out_dtype == 0 && gate_col >= 0 && (M == 1 || ldz >= gate_col + N) && ldz < (1 << 24) && gate_col < (1 << 24),
                  "gemm_decode: a gate goes with a 32-bit residual");
     LLMS_REQUIRE(workgroups > 0 && workgroups <= 4096, "gemm_decode: bad number of workgroups");

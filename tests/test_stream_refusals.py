@@ -69,3 +69,15 @@ def test_the_launcher_refuses_them_too(x_out, h_out, out, refused):
         i(0), i(0), at[out], i(K), at[6], None, i(N), i(K), i(K), i(0), i(0), f(0), i(1), at[1], at[x_out], at[h_out], at[2], at[7], f(0), f(1e-5),
         i(256), None)
     assert status == (1 if refused else 2)
+
+
+@pytest.mark.parametrize("m,k,norm,ldr,refused", [(8, 2048, False, 64, False), (16, 5632, False, 64, False), (8, 2048, True, 64, True),
+                                                  (16, 5632, True, 64, True), (16, 2048, False, 1 << 27, True)])
+def test_a_32_bit_residual_takes_no_norm(m, k, norm, ldr, refused):
+    needs_no_gpu()
+    at = [ctypes.c_void_p(i * (1 << 24)) for i in range(9)]
+    i, f = ctypes.c_int, ctypes.c_float
+    status = library.load("gemm_decode").llms_gemm_decode(
+        i(0), i(3), None, i(0), at[1], i(k), at[2], None, at[3] if norm else None, f(1e-5), i(m), i(64), i(k), i(0), i(0), i(0), i(0), i(0), None, None,
+        None, None, None, None, at[4], i(ldr), i(256), i(1), i(0), f(0), None, i(0), i(0), None, None)
+    assert status == (1 if refused else 2)
