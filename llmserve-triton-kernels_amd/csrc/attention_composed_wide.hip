@@ -316,7 +316,12 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
             }
     }
     int turn = 0;
-    for (int step = share; step < n_steps; step += a.shares) {
+    // ALWAYS: the next keys are asked for also where there is no further step (the last tile's again).  With a branch around them the compiler
+    // counts on none of them, and the score products wait for the step's values as well.  (Mixed heads and single tokens, but those of 128
+    // columns of keys of 64, have enough waves beside one another that the needless keys weigh more: 64 single tokens of 8 heads on 8 of 32
+    // behind 1,000 keys 36.5 -> 37.6 microseconds, 16 of two maps of 64 on 2, values of 128, 23.3 -> 22.3.)
+    constexpr bool ALWAYS = !MIXED && (!PARTS || (DT == 8 && TK == 2));
+    auto walk = [&](int step, bf16x8v (&kf)[2][TK], bf16x8v (&next_kf)[2][TK]) {
         const int next = step + a.shares;
         if constexpr (SHARED) {
             __syncthreads();  // this step's values are in LDS, and the turn before has been read
@@ -330,7 +335,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
             for (int d = 0; d < DT / HALVES; ++d) vf[half][d] = *reinterpret_cast<const u32x4*>(vt + (size_t)16 * d * bs);
         };
         if constexpr (!SHARED) ask_values(0);
-        if (next < n_steps) ask_keys(next_at, next_kf);
+        if (ALWAYS || next < n_steps) ask_keys(next_at, next_kf);
         if constexpr (SHARED) {  // (all of them, asked for before the scores: their way through LDS passes beside the softmax)
             const uint16_t* from = v_lds + turn * (DT * 512) + (q4 / 2) * (DT * 256) + col * 16 + 8 * ((q4 % 2) ^ (col / 8));
 #pragma unroll
@@ -420,10 +425,24 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
             if (next < n_steps) store_chunks(turn);
         }
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            at[tt] = next_at[tt], next_at[tt] = after_at[tt];
+        for (int tt = 0; tt < 2; ++tt) at[tt] = next_at[tt], next_at[tt] = after_at[tt];
+    };
+    if constexpr (!SHARED) {
+        // Two steps a turn, whose keys change places: to copy them is to wait for them at the end of each step.  Both together, microseconds, at
+        // 2 tokens behind 1,278 others: two maps of 64 on 2, values of 128, 35.1 -> 33.1, on 4, values of 64, 32.5 -> 30.2 (16 heads);
+        // 8 mixed heads of 128 on 1 43.2 -> 41.8; 32 of 64 on 4 55.0 -> 53.4; one map of 64 on 4, 7 tokens behind 890, 24.2 -> 22.5.
+        // (Shared values wait at a barrier a step either way, and have no registers left.)
+        for (int step = share; step < n_steps; step += 2 * a.shares) {
+            walk(step, kf, next_kf);
+            if (step + a.shares < n_steps) walk(step + a.shares, next_kf, kf);
+        }
+    } else {
+        for (int step = share; step < n_steps; step += a.shares) {
+            walk(step, kf, next_kf);
 #pragma unroll
-            for (int t = 0; t < TK; ++t) kf[tt][t] = next_kf[tt][t];
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int t = 0; t < TK; ++t) kf[tt][t] = next_kf[tt][t];
         }
     }
 #pragma unroll
