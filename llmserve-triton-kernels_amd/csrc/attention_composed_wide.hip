@@ -50,6 +50,7 @@
 #define NOTHING_YET (-1.0e30f)
 #define AW_SHARES 16  // most workgroups that share a request's keys
 #define AW_NO_KEY 0x40000000
+#define AW_AT_ONCE 256  // workgroups: one a compute unit
 #define AW_PIECES 2  // of a weight, where heads are mixed behind the value products
 
 typedef __attribute__((ext_vector_type(8))) short s16x8;
@@ -77,6 +78,7 @@ struct WideArgs {
     int dv, block_size, k_page, v_page;  // k_page, v_page: elements of a page
     int window, keep_first, chunk;
     int tok, tpw, shares;
+    int ordered;  // workgroups go by their keys (`block_of`)
     int talk_at;  // where the mixing matrix lies in LDS (portions of prompts; in floats)
     unsigned bs_magic;  // ceil(2^32 / block_size)
     unsigned tok_magic;  // ceil(2^32 / tok) (0: tok is 1)
@@ -109,12 +111,23 @@ __device__ __forceinline__ uint32_t low_half_mask(int keep) { return keep <= 0 ?
 // possible portion, workgroups without tokens lay between those with some, and as workgroups go around the parts of the chip in
 // turn, parts of it met only empty ones (32 heads of 64 on 4, microseconds: 811, 890, 150 and 197 tokens 156 -> 91, twice 1,024 beside
 // two of 1 token 190 -> 104, without those 104; 16 heads of two maps on 2: 57 -> 48 and 73 -> 56; 77 and 44 are the first and third now).
-// Up to AW_SORTED requests: the block with the i-th most keys, so that no long one begins late.  A block's height is its place from its
-// request's beginning, in blocks: request s has the heights from .. upto - 1.  Every lane counts the blocks of height B and more for a
-// B of its own, so that a pass narrows the heights to a 64th.  The time of a pass grows with the requests (64 of 3 tokens: 18 -> 27
-// microseconds, against 19 in the order of the requests), whose portions are short where they are many: then the requests one after the other, each
-// from its last block to its first.
-#define AW_SORTED 8
+// One request after the other, each from its last block to its first, where the chip takes all workgroups at once or the requests are more than a
+// wave's lanes, whose portions are short.  Otherwise (`ordered`) the block with the i-th most keys, so that no long one begins late, and among equals
+// in the order of the requests, so that portions of one length meet the parts of the chip as their requests do and a part reads few requests'
+// keys.  A block's height is its place from its request's beginning, in blocks: request s has the heights from .. upto - 1; the height is looked for in
+// quarters, a turn of three sums over the lanes.  (The order for up to 8 requests alone, whose sums went over them one by one, and for more one request
+// after the other, microseconds: 16 of 64 tokens behind 100, 32 heads of 128 on 8, 20.3 -> 16.1; 32 of 64 behind 300 61 -> 41; 16 of 128, 32 mixed
+// heads of 64 on 8 of 32, 48 -> 41, on 4 of 64 42 -> 37.)
+// `add` over the numbers of a lane and of those before it.
+template <typename F>
+__device__ __forceinline__ int up_to_lane(int v, F add) {
+    v = add(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));  // from 1, 2, 4 and 8 lanes before, in rows of 16
+    v = add(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));
+    v = add(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));
+    v = add(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));
+    v = add(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // the last lane of the row before, and of the half before
+    return add(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+}
 __device__ __forceinline__ bool block_of(const WideArgs& a, int i, int lane, int& bi, int& blk, int& row0, int& count, int& end) {
     auto blocks = [&](int tokens) { return a.tok_magic ? (int)__umulhi((unsigned)tokens, a.tok_magic) : tokens; };
     int from, upto, row, tokens, keys;
@@ -132,34 +145,37 @@ __device__ __forceinline__ bool block_of(const WideArgs& a, int i, int lane, int
         row0 = __builtin_amdgcn_readlane(row, at), count = __builtin_amdgcn_readlane(tokens, at), end = __builtin_amdgcn_readlane(keys, at);
         return true;
     };
-    if (a.n_seqs > 1 && a.n_seqs <= AW_SORTED) {
+    if (a.n_seqs == 1) {  // (nothing to look for: 0.1 microseconds less)
+        row0 = a.cu_seqlens[a.seq_begin], count = a.cu_seqlens[a.seq_begin + 1] - row0, end = a.context_lens[a.seq_begin];
+        bi = 0, blk = blocks(count + a.tok - 1) - 1 - i;
+        return count > 0 && end > 0 && blk >= 0;
+    }
+    auto sum = [](int x, int y) { return x + y; };
+    if (a.ordered) {
         heights(0);
-        int lo = -1, hi = blocks(a.max_blocks * a.block_size) + 2, at_hi = 0;  // (a request's keys fit its pages: no block is as high)
+        auto most = [](int x, int y) { return x > y ? x : y; };
+        auto over_lanes = [&](int v, auto add) { return __builtin_amdgcn_readlane(up_to_lane(v, add), LLMS_WAVE - 1); };
+        auto of_height = [&](int h) { return over_lanes(most(upto - most(from, h), 0), sum); };  // blocks of height h and more
+        const int all_blocks = over_lanes(upto - from, sum), highest = over_lanes(upto, most);
+        const int depth = over_lanes(upto > from ? highest - from : 0, most);  // (from the highest block down to the lowest)
+        if (all_blocks <= i) return false;
+        int lo = highest - depth, hi = highest, above = 0;  // a height that more than i blocks reach, and one that `above` blocks do, at most i
         while (hi - lo > 1) {
-            const int stride = (hi - lo + LLMS_WAVE - 1) / LLMS_WAVE, height = lo + (lane + 1) * stride;
-            int higher = 0;
-            for (int j = 0; j < a.n_seqs; ++j)
-                higher += max(__builtin_amdgcn_readlane(upto, j) - max(__builtin_amdgcn_readlane(from, j), height), 0);
-            const int c = __popcll(__ballot(higher > i));  // (at most 63: none is as high as hi)
-            lo += c * stride;
-            if (lo + stride < hi) hi = lo + stride, at_hi = __builtin_amdgcn_readlane(higher, c);
+            const int quarter = (hi - lo + 3) / 4, m1 = lo + quarter, m2 = min(m1 + quarter, hi), m3 = min(m2 + quarter, hi);
+            const int n1 = of_height(m1), n2 = of_height(m2), n3 = of_height(m3);
+            if (n1 <= i) hi = m1, above = n1;
+            else if (n2 <= i) lo = m1, hi = m2, above = n2;
+            else if (n3 <= i) lo = m2, hi = m3, above = n3;
+            else lo = m3;
         }
-        if (lo < 0) return false;
         const bool there = from <= lo && lo < upto;
         const unsigned long long all = __ballot(there);
-        const int at = __ffsll(__ballot(there && __popcll(all & ((1ull << lane) - 1)) == i - at_hi)) - 1;
+        const int at = __ffsll(__ballot(there && __popcll(all & ((1ull << lane) - 1)) == i - above)) - 1;
         return found(at, at, lo - __builtin_amdgcn_readlane(from, at));
     }
     for (int base = 0; base < a.n_seqs; base += LLMS_WAVE) {
         heights(base);
-        int last = upto - from;  // behind request base + lane's blocks
-        if (a.n_seqs > 1) {
-#pragma unroll
-            for (int d = 1; d < LLMS_WAVE; d *= 2) {
-                const int before = __shfl_up(last, d, LLMS_WAVE);
-                if (lane >= d) last += before;
-            }
-        }
+        const int last = up_to_lane(upto - from, sum);  // behind request base + lane's blocks
         const unsigned long long behind = __ballot(last > i);
         if (behind) {
             const int at = __ffsll(behind) - 1;
@@ -708,6 +724,7 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
         LLMS_REQUIRE(lds <= 160 * 1024, "attend_composed_wide: too many heads for the LDS");
         const long most = (long)n_seqs * ((max_new + a.tok - 1) / a.tok), held = rows / a.tok + n_seqs;  // (blocks of portions as long as the longest, and that `rows` rows make)
         const dim3 grid((unsigned)(held < most ? held : most), 1, talk ? 1 : kv_heads);
+        a.ordered = n_seqs > 1 && n_seqs <= LLMS_WAVE && (long)grid.x * grid.z > AW_AT_ONCE;
         if (shared) {
             LLMS_REQUIRE(talk && units == 1 && kv_heads >= 4 && dk == 64 && width == 256, "attend_composed_wide: shared values with 4 to 8 mixed key/value heads, keys of 64 and 256 columns of values");
             return launch_one<2, 16, 1, false, true, true>(a, grid, kv_heads * LLMS_WAVE, lds, stream);
@@ -717,7 +734,7 @@ int llms_attend_composed_wide(void* out, int out_stride, const void* q, int q_st
     }
     LLMS_REQUIRE(max_new == 1 && shares >= 1 && shares <= AW_SHARES && ws_o && ws_stats, "attend_composed_wide: one token a request, up to 16 shares, and their workspaces");
     a.heads_per_wg = a.score_heads < 4 ? a.score_heads : 4;
-    a.tok = 1, a.shares = shares;
+    a.tok = 1, a.shares = shares, a.ordered = 0;
     const int zs = (a.score_heads + a.heads_per_wg - 1) / a.heads_per_wg;
     LLMS_REQUIRE(zs <= 65535 && heads <= 65535, "attend_composed_wide: too many heads");
     const size_t mix_lds = ((size_t)heads * 20 + (size_t)a.grp * heads) * sizeof(float);

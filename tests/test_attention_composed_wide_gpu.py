@@ -194,3 +194,12 @@ def test_portions_of_ragged_lengths(counts, maps, monkeypatch):
     for s in range(n):
         part = out[cu[s]:cu[s + 1]]
         assert bool((part != 7.0).any(1).all()) if s in seen else bool((part == 7.0).all())
+
+
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("counts", [[33] * 9, [7 + 5 * (i % 6) for i in range(16)], [150] + [3] * 20, [0, 90, 1] * 8, [40] * 63, [2 + i for i in range(64)],
+                                    [0] * 30 + [40, 0, 77] + [1] * 31])
+def test_portions_of_many_requests(counts, maps, monkeypatch):
+    """More than 8 requests and up to a wave's lanes, whose blocks go by their keys where the chip does not take them all at once: alike, ragged,
+    one long, some without rows, a wave full."""
+    test_portions_of_ragged_lengths(counts, maps, monkeypatch)
