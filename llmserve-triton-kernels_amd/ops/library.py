@@ -1760,7 +1760,7 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
         ws_o = torch.empty(columns * (kv_heads * dv if talk is not None else dv), dtype=torch.float32, device=dev)
         ws_stats = torch.empty(2 * columns, dtype=torch.float32, device=dev)
     else:
-        units = wide_prompt_units(heads, kv_heads, dv, talk is not None, n_seqs, max_new, q.shape[0], compute_units(dev))
+        units = wide_prompt_units(heads, kv_heads, dk, dv, maps, talk is not None, n_seqs, max_new, q.shape[0], compute_units(dev))
         shared = wide_prompt_shared(heads, kv_heads, dk, dv, talk is not None)
     _check(load("attention_composed_wide").llms_attend_composed_wide(
         _ptr(out), c_int(out.stride(0)), _ptr(q), c_int(q.stride(0)), _ptr(k_pool), _ptr(v_pool), _ptr(block_tables),
@@ -1772,19 +1772,38 @@ def attend_composed_wide(out: torch.Tensor, q: torch.Tensor, k_pool: torch.Tenso
     return out
 
 
-def wide_prompt_units(heads: int, kv_heads: int, dv: int, talk: bool, n_seqs: int, max_new: int, rows: int, cus: int) -> int:
+def wide_prompt_units(heads: int, kv_heads: int, dk: int, dv: int, maps: int, talk: bool, n_seqs: int, max_new: int, rows: int,
+                      cus: int = 256) -> int:
     """Units of 16 columns a wave of `attend_composed_wide` takes over portions of prompts, of `rows` rows together.  Two share every
-    key and value a wave reads, one gives twice the workgroups, which count for more until every compute unit has several of two
-    units (16 heads of two maps over 64, values of 128, microseconds with one unit and with two: 1,100 tokens, 550 workgroups of two, 47 and
-    56; twice 700 tokens 34 and 37; 1,500 tokens, 750, 70 and 69; 2,048 tokens, 1,024, 118 and 89; 4 times 512 35 and 30; 811, 890,
-    150 and 197 52 and 44).  The results of two units of 256 columns do not fit a wave's registers, and mixed heads, whose weights
+    key and value a wave reads, one gives twice the workgroups, which count for more until a compute unit has several waves of two units:
+    four and a half where keys are of 64 numbers, two and a quarter of 128, whose waves have twice the matrix instructions and loads a step.
+    Microseconds with one unit and with two, by waves of two units:
+      keys of 64   16 heads of two maps on 2, values of 128: 600 waves (600 tokens) 22 and 27; 1,300 53 and 61; 1,500 71 and 67; 2,048 (2,048
+                   tokens) 117 and 86; on 4, values of 64: 1,304 48 and 52; 1,408 33 and 31; 1,504 63 and 57; 32 heads of one map on 4, values
+                   of 128: 852 30 and 36; 1,000 41 and 42; 1,200 (1,200 tokens) 49 and 49, behind 900 others 95 and 81
+      keys of 128  8 heads of two maps on 4, values of 128: 376 (twice 600 tokens) 30 and 31; 600 52 and 53, behind 900 others 103 and 87; 904 109 and 78;
+                   1,024 (2,048 tokens) 144 and 99; on 2, values of 64: 752 55 and 58, behind 500 others 79 and 75; 1,024 105 and 87; 32 heads of one map
+                   on 8: 512 22 and 25; 704 35 and 33; 1,000 70 and 45
+    Just beyond the lines one unit may be the faster behind nothing and two behind many others (16 heads of two maps on 4, twice 600 tokens,
+    1,200 waves, 25 and 29): the line lies where the latter weigh more.
+    One map in no more blocks than compute units to a key/value head: a compute unit gets the same block of every head, the long ones together, and
+    half as many workgroups of two units even that out sooner (16 heads of 64 on 8, 904 waves 48 and 62, 1,024 75 and 70; on 4 65 and
+    70).  The results of two units of 256 columns do not fit a wave's registers, and mixed heads, whose weights
     are two numbers each, are faster with one (8 heads of 128 on 1, 2,048 tokens: 72 against 95; 4 requests of 512: 26 and 35; 16
     heads on 4 of 32, 2,048 tokens: 92 and 95)."""
     if talk or dv > 128:
         return 1
-    tokens = 2 * (16 // (heads // kv_heads))
-    workgroups = min(n_seqs * -(-max_new // tokens), rows // tokens + n_seqs) * kv_heads
-    return 2 if workgroups >= 3 * cus else 1
+    tokens = 16 // (heads // kv_heads)  # of a unit
+
+    def blocks(n):
+        return min(n_seqs * -(-max_new // n), rows // n + n_seqs)
+
+    waves = blocks(2 * tokens) * kv_heads * maps
+    if dk > 64:
+        line = 2.25 * cus
+    else:
+        line = 4 * cus if maps == 1 and blocks(tokens) <= cus else 4.5 * cus
+    return 2 if waves >= line else 1
 
 
 def wide_prompt_shared(heads: int, kv_heads: int, dk: int, dv: int, talk: bool) -> bool:

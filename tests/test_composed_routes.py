@@ -62,3 +62,21 @@ def test_without_mixing_too(heads, kv, maps, dk, new, context, params, kernel, m
 def test_nothing_but_single_tokens_is_one_launch(monkeypatch):
     (call,) = route(monkeypatch, 8, 8, 1, 4000, n=0, n_dec=5)
     assert call[:4] == ("attend_composed_wide", 0, 5, 1)
+
+
+@pytest.mark.parametrize("heads,kv,dk,dv,maps,counts,one,two", [  # microseconds with one unit a wave and with two
+    (8, 4, 128, 128, 2, [512], 17.6, 25.4), (8, 4, 128, 128, 2, [1000], 39.1, 43.8), (8, 4, 128, 128, 2, [2048], 144.5, 98.6),
+    (8, 4, 128, 128, 2, [512] * 4, 42.0, 31.8), (8, 4, 128, 128, 2, [256] * 8, 25.2, 20.4), (8, 4, 128, 128, 2, [128] * 16, 16.3, 13.8),
+    (8, 2, 128, 64, 2, [1100], 39.9, 43.7), (8, 2, 128, 64, 2, [2048], 105.0, 89.3), (8, 2, 128, 64, 2, [256] * 8, 19.9, 18.0),
+    (32, 8, 128, 128, 1, [512], 22.3, 24.8), (32, 8, 128, 128, 1, [850], 44.8, 39.0), (32, 8, 128, 128, 1, [128] * 16, 26.2, 21.5),
+    (16, 2, 64, 128, 2, [1100], 44.7, 53.1), (16, 2, 64, 128, 2, [1500], 70.6, 67.3), (16, 2, 64, 128, 2, [811, 890, 150, 197], 53.8, 43.0),
+    (16, 4, 64, 64, 2, [1100], 41.6, 47.2), (16, 4, 64, 64, 2, [700, 700], 33.0, 31.5), (16, 4, 64, 64, 2, [1500], 62.8, 57.3),
+    (8, 8, 64, 64, 2, [2048], 75.1, 82.5), (8, 8, 64, 64, 2, [512] * 4, 23.6, 26.3), (8, 8, 64, 64, 2, [3000], 121.3, 113.7),
+    (16, 4, 64, 64, 1, [2048], 64.9, 70.1), (16, 8, 64, 64, 1, [2048], 75.1, 70.1), (16, 8, 64, 64, 1, [1500], 38.3, 52.1),
+    (32, 4, 64, 128, 1, [850], 29.6, 36.3), (32, 4, 64, 128, 1, [1500], 73.5, 67.7), (32, 2, 128, 64, 1, [1000], 47.8, 40.9)])
+def test_units_of_a_wave_over_portions(heads, kv, dk, dv, maps, counts, one, two):
+    """As many columns a wave as is the faster: a line by the waves, the keys' length and the maps."""
+    from llmserve.ops.library import wide_prompt_units
+
+    assert wide_prompt_units(heads, kv, dk, dv, maps, False, len(counts), max(counts), sum(counts)) == (1 if one < two else 2)
+    assert wide_prompt_units(heads, kv, dk, dv, maps, True, len(counts), max(counts), sum(counts)) == 1
