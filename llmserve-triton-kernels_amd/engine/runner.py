@@ -304,13 +304,20 @@ class ModelRunner:
         unit = max(16, floor // 8)
         return -(-n // unit) * unit
 
+    # From one row past a multiple of this on, the products of a step take a round of tiles more: 512 rows of the 1.1B shape 60.6 microseconds a
+    # layer, 516 68.4.  Between two such lines a row more or less is hardly felt.
+    ROWS_LINE = 512
+
     @classmethod
     def _step_shape(cls, n_decode: int, n_prefill: int, n_prefill_tokens: int, n_logits: int, context: int) -> tuple:
         """The sizes a step is padded to: powers of two for the requests, the wanted rows and the reach of
-        the contexts (which only sets how attention spreads its work), `_row_bucket` for the rows of the portions, alone or with
-        the single tokens in front of them, whichever leaves fewer."""
+        the contexts (which only sets how attention spreads its work), `_row_bucket` for the rows of the portions, but no padding past a
+        line (`ROWS_LINE`) that the tokens do not pass.  (Rounded together with the single tokens in front of them wherever that leaves
+        fewer rows, portions had twice as many sizes: in varied traffic with steps of up to 2,048 tokens 615 steps instead of 526 in 992 met
+        theirs for the first time and were launched kernel by kernel.)"""
         decode = _pow2(n_decode) if n_decode else 0
-        rows = min(cls._row_bucket(n_prefill_tokens), cls._row_bucket(decode + n_prefill_tokens) - decode)
+        line = -(-(decode + n_prefill_tokens) // cls.ROWS_LINE) * cls.ROWS_LINE
+        rows = min(cls._row_bucket(n_prefill_tokens), line - decode)
         return (decode, _pow2(n_prefill), rows, _pow2(max(n_logits, 1)), _pow2(context, 256))
 
     @classmethod
