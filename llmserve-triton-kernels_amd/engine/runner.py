@@ -95,6 +95,11 @@ class ModelRunner:
         outer = tuple(model.spec.weights[role] for role in ("embedding", "head"))
         self._elements_per_token = sum(info.shape[0] * info.shape[1] for name, info in infos.items()
                                        if len(info.shape) == 2 and not name.startswith(outer))
+        # bytes that a key keeps in all layers, where tokens of a portion may run as single tokens beside it (0: they may not)
+        mixers = [block.mixer for block in model.blocks]
+        self._key_bytes = 0
+        if self.dtype == torch.bfloat16 and all(mixer.takes_tokens_of_portions for mixer in mixers):
+            self._key_bytes = sum(4 * spec.num_kv_heads * spec.head_dim for spec in (mixer.cache_spec() for mixer in mixers))
 
     # ---- construction ---------------------------------------------------------------------
     @staticmethod
@@ -321,25 +326,30 @@ class ModelRunner:
         return (decode, _pow2(n_prefill), rows, _pow2(max(n_logits, 1)), _pow2(context, 256))
 
     @classmethod
-    def _spare_rows_filled(cls, layout, tokens: list[list[int]], logit_rows: list[int]):
-        """The same step with the first tokens of its longest portion in the places that a power of two of single tokens leaves empty, where
-        that leaves fewer rows: (layout, tokens, logit_rows).  A token attends to the keys up to its own place, which all are stored
-        before, so for layers that keep keys and nothing else a portion may be cut anywhere.  A step of 512 tokens, 3 of them
-        decoding, has 512 rows so, and 516 otherwise, and one row past 512 takes the four products of a layer of the 1.1B shape from 60.6
-        microseconds to 68.4."""
+    def _spare_rows_filled(cls, layout, tokens: list[list[int]], logit_rows: list[int], pays=lambda moved, start: True):
+        """The same step with the first tokens of its longest portion in the places that a power of two of single tokens leaves empty, as few as
+        bring it under a line (`ROWS_LINE`) that it passes otherwise: (layout, tokens, logit_rows).  A token attends to the keys up to its own place,
+        which all are stored before, so for layers that keep keys and nothing else a portion may be cut anywhere.  But a single
+        token reads its keys alone where a portion's share them: `pays(tokens moved, keys before them)` says whether that is worth it.
+        The 1.1B shape, 12 layers, microseconds a step of 512 tokens, unfilled and filled: 3 of them decoding 1159 and 1106, 33 (31 tokens moved) 1217 and
+        1145, behind 1,500 keys 1382 and 1308, 120 behind 1,500 1559 and 1435.  Where no line is passed it costs more than it gives: 65 decoding
+        of 433 tokens 1161 and 1199, behind 1,500 keys 1330 and 1395, 33 of 700 behind 900 1480 and 1531."""
         counts = layout.counts
         n_dec = next((i for i, c in enumerate(counts) if c != 1), len(counts))
         if not 0 < n_dec < len(counts):
             return layout, tokens, logit_rows
         total = sum(counts[n_dec:])
         longest = max(range(n_dec, len(counts)), key=lambda i: counts[i])
-        moved = min(_pow2(n_dec) - n_dec, counts[longest] - 2)  # (a portion stays one)
+        most = min(_pow2(n_dec) - n_dec, counts[longest] - 2)  # (a portion stays one)
 
-        def rows_with(m):
-            decode, _, rows, *_ = cls._step_shape(n_dec + m, 1, total - m, 1, 1)
-            return decode + rows
+        def lines_passed(moved):
+            decode, _, rows, *_ = cls._step_shape(n_dec + moved, 1, total - moved, 1, 1)
+            return (decode + rows - 1) // cls.ROWS_LINE
 
-        if moved <= 0 or rows_with(moved) >= rows_with(0):
+        if most <= 0 or lines_passed(most) >= lines_passed(0):
+            return layout, tokens, logit_rows
+        moved = next(m for m in range(1, most + 1) if lines_passed(m) < lines_passed(0))
+        if not pays(moved, layout.starts[longest]):
             return layout, tokens, logit_rows
         at = n_dec + sum(counts[n_dec:longest])  # the portion's first row
         order = [*range(n_dec), *range(at, at + moved), *range(n_dec, at), *range(at + moved, n_dec + total)]
@@ -357,6 +367,12 @@ class ModelRunner:
         own = tokens[longest]
         return filled, each(tokens, [[t] for t in own[:moved]], own[moved:]), [place[row] for row in logit_rows]
 
+    def _keys_alone_pay(self, moved: int, start: int) -> bool:
+        """Whether `moved` tokens behind `start` keys may read their keys one by one for a round of tiles less: up to as many bytes as the weights of
+        the layers.  (The 1.1B shape, 88 MB a layer: 31 tokens behind 1,500 keys read 48 MB and gain 5.4 %, 58 behind 900 56 and 3.2 %, 63 behind
+        1,500 98 and 2.1 %; the 7B shape, 16 KB a key, in steps that pass no line: 15 behind 1,500 lose 12 %.)"""
+        return moved * (start + moved) * self._key_bytes <= 2 * self._elements_per_token
+
     def _shape_of(self, layout, n_logits: int) -> tuple:
         n_dec = 0
         while n_dec < len(layout.counts) and layout.counts[n_dec] == 1:
@@ -371,8 +387,8 @@ class ModelRunner:
         from then on.  Which kernels run, and in which arrangement, is therefore a function of the bucket
         alone: the first run and every replay give the same bits, and so do two runs of one trace.
         Returns (logits, whether the caller owns them)."""
-        if len(self.manager.paged_groups) == len(self.manager.groups):  # (no layer keeps a state that a portion runs through)
-            layout, tokens, logit_rows = self._spare_rows_filled(layout, tokens, logit_rows)
+        if self._key_bytes:
+            layout, tokens, logit_rows = self._spare_rows_filled(layout, tokens, logit_rows, self._keys_alone_pay)
         shape = self._shape_of(layout, len(logit_rows))
         bucket = self._buckets.pop(shape, None)
         if bucket is None:

@@ -25,6 +25,7 @@ from .spec import PagedCacheSpec, ParamInfo
 class Attention(Mixer):
     graph_safe = True
     accepts_deferred_norm = True
+    takes_tokens_of_portions = True
 
     def __init__(self, spec, ctx):
         super().__init__(spec, ctx)

@@ -249,6 +249,10 @@ class Mixer(Part):
 
     accepts_deferred_norm = False
     accepts_joined_rows = False
+    # whether a portion's tokens may as well run as single tokens beside it, each for the price of reading its keys alone: it keeps keys and
+    # nothing else, and its kernels for single tokens take a request's token for little more (measured, not only so by design: latent
+    # attention, a workgroup a token, lost up to 31 % of a step by 3 of them)
+    takes_tokens_of_portions = False
     # the weight of the last product, where `forward(..., joins=GatedStream)` leaves the sum to that product: a name, or None
     adds_to_stream_by = None
 
