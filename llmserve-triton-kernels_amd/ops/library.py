@@ -683,8 +683,8 @@ def gemm_decode(out: torch.Tensor | None, x: torch.Tensor, w: torch.Tensor, bias
     return residual if epilogue == 3 else out
 
 
-# Up to how many rows, and of how many numbers, ops.gemm_decode_stream takes: a row of 2,048 costs every workgroup 8 or, with what
-# joins it, 16 KB from L2, which the kernel of some 4.3 microseconds that it stands for stops being worth.
+# Up to how many rows, and of how many numbers, ops.gemm_decode_stream takes: what a wave has of them in its registers.  A row of 2,048 costs
+# every workgroup 8 or, with what joins it, 16 KB from L2; where the kernel that it stands for is the faster way says parts.linear.joins_pay.
 GEMM_DECODE_STREAM_ROWS = 8
 GEMM_DECODE_STREAM_K = 4096
 

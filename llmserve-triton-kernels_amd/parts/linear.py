@@ -254,10 +254,27 @@ def takes_stream(stream: torch.Tensor, weight: torch.Tensor) -> bool:
             and not streams_large(m, n, k, ops.compute_units(stream.device)))
 
 
+def joins_pay(m: int, n: int, k: int, gated: bool, cus: int = 256) -> bool:
+    """Whether `m` rows that a stream's open sum makes are closed faster by the product against a weight [n, k] on its way in than by the kernel for
+    it.  Every workgroup reads all of the stream and of what joins it, in turns of 4 rows: a second turn of more than 2,048 columns takes longer than
+    that kernel where little else is in flight, one tile of 16 weight rows to a workgroup (or 8 gated pairs), and beyond 3,072 columns anywhere.
+    Microseconds on the way in and apart, one turn of 4 rows and 8 rows: 2304 x 2304 6.7 and 7.5, 8.0 and 7.6; 2 x 2048 x 2560 gated 8.2 and 8.8, 9.5 and
+    9.0; 3072 x 3072 7.7 and 8.4, 9.2 and 8.8; 4096 x 4096 9.3 and 10.5, 11.8 and 11.1; 2 x 10240 x 4096 gated 28.7 and 29.6, 31.3 and 30.2.  Shares of other sizes,
+    8 rows: 2 x 3072 x 2560 gated 9.8 and 10.8; 6144 x 3072 11.2 and 11.5; 2048 x 3072 7.6 and 8.0.  Up to 2,048 columns 8 rows are 5 to 20 % faster.
+    A norm reads the stream alone: 8 rows of 2,304 to 4,096 columns 6 % faster in the mean, 1 of 36 sizes more than 2 % slower."""
+    if m <= 4 or k <= 2048:
+        return True
+    units = n // 2 if gated else n
+    share = -(-units // min(units, cus))
+    return k <= 3072 and not (share <= 8 if gated else 8 < share <= 16)
+
+
 def joined_product(x, weight: torch.Tensor, out: torch.Tensor, bias: torch.Tensor | None = None, **epilogue) -> bool:
     """The product of `JoinedRows` x into `out` (float32, or bfloat16 with the gated `epilogue`) with x's sum closed on the way in, where that is
-    done; False, with nothing done, otherwise."""
+    the faster way; False, with nothing done, otherwise."""
     if x.dtype != torch.bfloat16 or not takes_stream(x.stream, weight):
+        return False
+    if not joins_pay(x.shape[0], *weight.shape, epilogue.get("swiglu", False), ops.compute_units(out.device)):
         return False
     stream = torch.empty_like(x.stream)
     ops.gemm_decode_stream(out, x.stream, weight, bias, joins=(x.delta.y, x.delta.weight, x.delta.eps, stream), **epilogue)

@@ -164,3 +164,34 @@ def test_long_rows_are_added_where_their_tiles_are_filled(n, long):
     assert linear.ops.gemm_decode_adds(16, 11008) and not linear.ops.gemm_decode_adds(17, 11008)
     assert not linear.adds_residual_in_epilogue(bf16(17, 11008), bf16(n, 11008))
     assert linear.adds_residual_in_epilogue(bf16(16, 6144), bf16(n, 6144))
+
+
+@pytest.mark.parametrize("m,n,k,gated,micros,apart", [
+    (1, 2304, 2304, False, 6.50, 7.26), (4, 2304, 2304, False, 6.70, 7.45), (5, 2304, 2304, False, 7.88, 7.60), (8, 2304, 2304, False, 7.97, 7.61),
+    (8, 2048, 2304, False, 7.11, 7.47), (6, 2048, 2560, False, 7.18, 7.24), (8, 2560, 2560, False, 8.48, 8.15), (5, 3840, 2560, False, 9.05, 8.63),
+    (8, 5120, 2560, False, 9.74, 10.21), (8, 12800, 2560, True, 15.43, 16.20), (8, 4096, 2560, True, 9.50, 8.98), (4, 4096, 2560, True, 8.17, 8.76),
+    (8, 6144, 2560, True, 9.75, 10.78), (8, 10240, 3072, True, 14.96, 15.47), (5, 3072, 3072, False, 9.42, 8.67), (8, 3072, 3072, False, 9.15, 8.78),
+    (8, 6144, 3072, False, 11.19, 11.49), (8, 15360, 3072, True, 18.81, 19.46), (8, 4096, 3072, True, 10.31, 9.69), (8, 1024, 4096, False, 9.07, 8.25),
+    (4, 1024, 4096, False, 6.68, 7.75), (8, 4096, 4096, False, 11.80, 11.09), (5, 6144, 4096, False, 13.58, 13.04), (8, 20480, 4096, True, 31.27, 30.17),
+    (2, 20480, 4096, True, 28.94, 29.54), (8, 2048, 2048, False, 5.93, 6.92), (8, 1536, 1536, False, 5.45, 6.28), (8, 10240, 2048, True, 10.37, 11.83)])
+def test_an_open_sum_is_closed_the_faster_way(m, n, k, gated, micros, apart):
+    """Microseconds of the product that closes its rows' sum on the way in, and of the kernel for it and the product."""
+    from llmserve.parts.linear import joins_pay
+
+    assert joins_pay(m, n, k, gated) == (micros < apart)
+
+
+def test_rows_that_are_not_closed_on_the_way_in_stay_open(monkeypatch):
+    from llmserve.parts import linear
+    from llmserve.parts.registry import JoinedRows, NormedSum
+
+    called = []
+    monkeypatch.setattr(linear.ops, "compute_units", lambda dev: 256)
+    monkeypatch.setattr(linear.ops, "gemm_decode_stream", lambda *a, **kw: called.append(a))
+    monkeypatch.setattr(linear.ops, "gemm_decode_stream_supported", lambda x, w: True)
+    for m, k, n, taken in ((8, 2048, 2048, True), (8, 4096, 4096, False), (4, 4096, 4096, True), (8, 2560, 2560, False), (8, 2560, 4608, True)):
+        stream, weight = torch.empty(m, k, device="meta"), torch.empty(n, k, dtype=torch.bfloat16, device="meta")
+        x = JoinedRows(stream, NormedSum(stream, torch.empty(k, device="meta"), 1e-5), torch.bfloat16, None)
+        called.clear()
+        assert linear.joined_product(x, weight, torch.empty(m, n, device="meta")) == taken
+        assert x.resolved == taken and len(called) == taken
