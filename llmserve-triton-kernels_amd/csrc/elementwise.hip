@@ -14,7 +14,8 @@
 // angles (the blocks behind), and the pages it took written into the block tables (one block a table).  They were three launches of 5.8, 1.8 and 2
 // microseconds for 8 tokens of the 1.1B shape, and a row came 2 bytes a thread at a time; 23 decoding steps of 64 requests took 13 microseconds more
 // each.  What bounds it: a launch, and an answer of memory behind the ids'.
-// SCALED: rows in 32-bit times `scale`; an id outside the vocabulary is the nearest one.  Otherwise rows as they are; such an id's is NaN.
+// SCALED: rows in 32-bit times `scale`, 16 bytes a thread of what is stored (of what is read, two stores 32 bytes apart, 2,048 rows of 2,048 took 5.9
+// microseconds for 4.8); an id outside the vocabulary is the nearest one.  Otherwise rows as they are; such an id's is NaN.
 #define STEP_START_TABLES 8
 struct StepStartArgs {
     void* out;
@@ -46,18 +47,16 @@ __global__ __launch_bounds__(256) void step_start_kernel(const StepStartArgs a) 
             return;
         }
         const T* src = reinterpret_cast<const T*>(a.table) + (size_t)id * a.hidden;
-        constexpr int V = 16 / sizeof(T);
+        constexpr int V = SCALED ? 4 : 16 / sizeof(T);
+        typedef typename std::conditional<V * sizeof(T) == 16, uint4, uint2>::type Piece;
         if (a.wide) {
             for (int i = threadIdx.x * V; i < a.hidden; i += 256 * V) {
-                const uint4 v = *reinterpret_cast<const uint4*>(src + i);
+                const Piece v = *reinterpret_cast<const Piece*>(src + i);
                 if constexpr (!SCALED) {
-                    *reinterpret_cast<uint4*>(o + i) = v;
+                    *reinterpret_cast<Piece*>(o + i) = v;
                 } else {
                     const T* e = reinterpret_cast<const T*>(&v);
-#pragma unroll
-                    for (int c = 0; c < V; c += 4)
-                        *reinterpret_cast<float4*>(o + i + c) = make_float4(to_f32(e[c]) * a.scale, to_f32(e[c + 1]) * a.scale,
-                                                                            to_f32(e[c + 2]) * a.scale, to_f32(e[c + 3]) * a.scale);
+                    *reinterpret_cast<float4*>(o + i) = make_float4(to_f32(e[0]) * a.scale, to_f32(e[1]) * a.scale, to_f32(e[2]) * a.scale, to_f32(e[3]) * a.scale);
                 }
             }
         } else {
