@@ -20,8 +20,8 @@
 // 8 (i / 4) + 4 u + i % 4; a lane then holds keys 8 q4 .. + 7 of the 32 for its column, which is the B operand of O^T = V^T P^T, and the
 // values' A operand is one load of 16 bytes.  (With a tile a product, a lane's keys were 4 of each tile and its values two loads of 8: a load
 // instruction takes its turn whatever it brings.  Microseconds, 32 heads of 64 on 4: 2 tokens behind 1,278 64 -> 55, 333 tokens 27.2 ->
-// 24.9, 2,048 tokens 174 -> 157, 4 single tokens behind 1,000 13.2 -> 12.3; two maps, 2,048 tokens 105 -> 91, but 210 tokens behind 890
-// 31.9 -> 33.0.)  Pages hold a multiple of 16 keys, so a tile's page and place are scalars, and a lane chooses between two.
+// 24.9, 2,048 tokens 174 -> 157, 4 single tokens behind 1,000 13.2 -> 12.3; two maps, 2,048 tokens 105 -> 91; 210 tokens behind 890
+// 31.9 -> 33.0, and 29.8 since the scores do not wait for the values.)  Pages hold a multiple of 16 keys, so a tile's page and place are scalars, and a lane chooses between two.
 //
 //   attend_wide_kernel<.., PARTS = true>   requests that bring one token: the keys go to `shares` workgroups, whose maxima, sums
 //       and results (32-bit) a second kernel joins: combine_mixed_kernel or combine_maps_kernel.
@@ -34,11 +34,11 @@
 // chain of two launches and of lengths -> table -> keys -> results; for portions the answers to a step's values.
 // Measured against that kernel, microseconds (mixed: 32 heads of 64 on 4 key/value heads; maps: 16 heads of two maps of 64 on 2,
 // values of 128):
-//     4 requests, one token behind   300 keys    mixed 22.1 -> 11.1    maps 18.4 ->  8.9
-//     4 requests, one token behind 1,000 keys    mixed 24.9 -> 12.3    maps 31.7 ->  9.8
-//   256 requests, one token behind 1,000 keys    mixed  130 ->   72    maps 50.4 -> 51.1 (5 TB/s of keys and values)
-//     a prompt of   333 tokens                   mixed  152 ->   25    maps 35.7 -> 13.9
-//     a prompt of 2,048 tokens                   mixed  819 ->  155    maps  284 ->   89
+//     4 requests, one token behind   300 keys    mixed 22.1 -> 10.8    maps 18.4 ->  8.5
+//     4 requests, one token behind 1,000 keys    mixed 24.9 -> 12.0    maps 31.7 ->  9.4
+//   256 requests, one token behind 1,000 keys    mixed  130 ->   66    maps 50.4 -> 50.4 (5 TB/s of keys and values)
+//     a prompt of   333 tokens                   mixed  152 ->   23    maps 35.7 -> 12.3
+//     a prompt of 2,048 tokens                   mixed  819 ->  152    maps  284 ->   86
 // (Mixed with two numbers a weight costs 0 to 8 % more than with one.)  Two maps, whose weights are one number in both kernels, are 2.2 to
 // 2.5e-3 from 64 bits in both.
 //
@@ -276,7 +276,7 @@ __global__ __launch_bounds__(PARTS ? 256 : 512) void attend_wide_kernel(const Wi
         for (int d = 0; d < DT; ++d) o[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
-    // SHARED: a step's values go through LDS (1,500 tokens of 32 heads on 8 of 32: 105 -> 102 microseconds), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
+    // SHARED: a step's values go through LDS (1,500 tokens of 32 heads on 8 of 32: 100 microseconds with or without), [tile][dimension][16 keys] as in a page, in two turns: the waves of the workgroup
     // (one per key/value head) all read all of them.  A chunk is 32 dimensions of a tile, 16 bytes a lane;
     // the two halves of dimensions 8 to 15 of every 16 change places, so that 32 lanes read 64 banks.
     constexpr int CHUNKS = SHARED ? DT / 4 : 1;

@@ -907,9 +907,10 @@ __global__ __launch_bounds__(GR_NW* LLMS_WAVE) void gemm_decode_rows_kernel(cons
 // tile or two of 16 rows, so the rows of X are needed once or twice and need not stay: a chunk of them comes with the weights' (XL loads
 // of 4 rows, from L2) and goes through a tile of its own in LDS.  The waves share K out as above, two items each in flight; the loop is
 // over four items, whose sums stay apart (a sum has no more terms than where K was shared out to workgroups), so K is not a constant of the kernel.
-// 4096 x 11008 with the residual's sum 18.5, 19.4 and 20.8 microseconds at 1, 8 and 16 rows, and the norm behind it goes into the next product;
-// gemm_stream, which leaves partial sums, and the norm that adds them up 21.4, 23.4 and 26.8.  8192 x 28672 75.5 and 78.9 at 1 and 8 rows (6.2 TB/s),
-// 85.9 and 93.3.  What bounds it: memory, and with 16 rows the rows of X beside it.
+// 4096 x 11008 with the residual's sum 19.6, 20.0 and 21.5 microseconds at 1, 8 and 16 rows, and the norm behind it goes into the next product;
+// gemm_stream, which leaves partial sums, and the norm that adds them up 22.8, 25.0 and 27.4.  Rows of more than 6,144 columns meet a norm kernel behind
+// either: with it 8192 x 28672 78.8, 79.6 and 90.3 (the product alone 76.1, 6.2 TB/s), by gemm_stream 83.6, 87.7 and 103.8; 8192 x 8192 32.8, 32.8
+// and 33.3, by gemm_stream 35.0, 34.4 and 37.2.  What bounds it: memory, and with 16 rows the rows of X beside it.
 #define GL_SUMS 4
 template <int LPI, int XL>
 __global__ __launch_bounds__(GD_NW* LLMS_WAVE) void gemm_decode_long_kernel(const DecodeGemmArgs a) {
@@ -1116,7 +1117,9 @@ static int gd_launch(int chunks, int tiles, unsigned grid, GdArgs<TOut, EPI, FRO
     // An item beyond K is a place in the ring with nothing in flight: with 18 chunks of four places a wave half of them are, and 256000 x 2304
     // at 1 row took 196 microseconds (169 with 16 waves), 171 with three; 6144 x 2304 8.1 and 7.0; gate and up of 5120 x 5120 with
     // the norm 12.5 and 11.9 with five for six.  Three and five items go round a ring of two in groups of two tiles, so few odd
-    // tiles stay as they are; of three items, all asked for in front of the norm, 3840 x 2560 took 6.7 for 6.4.
+    // tiles stay as they are; of three items, all asked for in front of the norm, 3840 x 2560 took 6.7 for 6.4.  Rows from a stream
+    // are long in coming, and there three items are the better ones of three tiles, and mixed of one: 6144 x 2560 at 4 rows 8.9 and 10.0 with four, 6144 x
+    // 2304 8.4 and 9.5, 2 x 5120 x 2304 gated 11.8 and 12.0; of one tile 3840 x 2560 7.8 and 7.4, 3840 x 2056 7.5 and 7.7.
     else if (chunks <= 3 * GD_NW && (tiles % 2 == 0 || tiles > 3 || !a.norm_weight)) {
         if (tiles % 2 && tiles <= 3) GD_GO(3, 1);
         else GD_GO(3, 2);

@@ -1808,10 +1808,11 @@ def wide_prompt_units(heads: int, kv_heads: int, dk: int, dv: int, maps: int, ta
 
 def wide_prompt_shared(heads: int, kv_heads: int, dk: int, dv: int, talk: bool) -> bool:
     """Whether the waves of a workgroup of `attend_composed_wide` share the values of a step through LDS (256 columns of values, all
-    read by at least 4 waves).  A load of 16 bytes brings what two brought, and four waves that each ask for the values are now
-    mostly ahead of a barrier a step (microseconds, each wave for itself -> shared, 32 heads of 64 on 4: 333 tokens 24.8 -> 28.8, 1,100
-    67 -> 70, 1,500 92 -> 88, 2,048 154 -> 150, behind 1,500 others 311 -> 320; ragged portions 77 -> 79); eight are not (32 heads on 8 of 32:
-    1,100 tokens 84 -> 82, 1,500 105 -> 102, 2,048 behind 1,500 328 -> 326)."""
+    read by at least 4 waves).  Four waves that each ask for the values are mostly ahead of a barrier a step (microseconds, each wave for
+    itself and shared, 32 heads of 64 on 4: 333 tokens 22.7 and 27.4, 1,100 63 and 66, 1,500 87 and 86, 2,048 152 and 152, behind 1,500 others 310
+    and 324; ragged portions 76 and 79; 8 heads on 4 of 64, 2,048 tokens 82 and 110).  Eight are level with it, and ask for an eighth (32 heads on
+    8 of 32: 333 tokens 34.5 and 34.9, 1,100 78.0 and 78.2, 1,500 100.5 and 100.2, 2,048 behind 1,500 324 and 325; 8 heads on 8 of 32: 333 tokens
+    36.3 and 37.3, 2,048 133 and 134)."""
     return talk and dk == 64 and kv_heads * dv == 256 and kv_heads > 4
 
 

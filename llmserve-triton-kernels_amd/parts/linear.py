@@ -80,9 +80,9 @@ def decode_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
 
 def adds_residual_in_epilogue(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether a product whose result is added to the residual rows does that sum itself (ops.gemm_decode's
-    residual epilogue).  It pays while the norm that follows is the next product's prologue (up to
-    GEMM_DECODE_NORM_ROWS rows): with more rows that norm is a kernel of its own, which adds up partial sums
-    as it reads them, and the product is faster with its K shared out (measured at 32 rows: 1.08 against 1.12 ms
+    residual epilogue), up to GEMM_DECODE_NORM_ROWS rows.  There the norm that follows is the next product's prologue, or,
+    with rows too long for that, a kernel which then adds nothing up (`adds_long_rows`).  With more rows that kernel adds up
+    partial sums as it reads them, and the product is faster with its K shared out (measured at 32 rows: 1.08 against 1.12 ms
     a step of the TinyLlama shape)."""
     if x.shape[0] > ops.GEMM_DECODE_NORM_ROWS:
         return False
@@ -94,11 +94,12 @@ def adds_residual_in_epilogue(x: torch.Tensor, weight: torch.Tensor) -> bool:
 def adds_long_rows(n: int, cus: int = 256) -> bool:
     """Whether a product of rows that are too long for a compute unit is added to the residual rows by ops.gemm_decode, in tiles of 16 weight
     rows that each take the rows of x in again, and not by the norm behind partial sums of ops.gemm_stream.  Not where a share of the weight's
-    n rows fills less than two thirds of its tiles: 5120 x 13824, 20 rows in two tiles, 31.4 microseconds at 1 row and 32.1 at 8, with the norm still to be
-    done by the next product, where stream and norm take 31.1 and 32.9.  11 other weights of 1024 x 8192 to 12288 x 6400 at 1 to 16 rows 7 to 38 %
-    faster (4096 x 14336 21.9 and 28.3 at 8 rows, 6656 x 17920, 26 rows in two tiles, 47.0 and 57.0, 3072 x 8192 10.9 and 16.3)."""
+    n rows that takes two tiles or more fills less than two thirds of them: 5120 x 13824, 20 rows in two tiles, 29.3, 30.6 and 36.3 microseconds at 1, 8
+    and 16 rows, with the norm still to be done by the next product, where stream and norm take 30.2, 33.5 and 38.7.  Nine other weights of 4096 x
+    11008 to 12288 x 6400 at 1 to 16 rows with a norm kernel behind either 1 to 17 % faster, and up to 6,144 columns that kernel is spared as well
+    (4096 x 14336 21.7 and 28.3 at 8 rows, 3072 x 8192 10.9 and 16.3).  A single tile is taken however little of it is filled: its rows of x are read once."""
     most = -(-n // min(n, cus))
-    return most <= 8 or 2 * (-(-most // 16) * 16) <= 3 * most or most <= 16
+    return most <= 16 or 2 * (-(-most // 16) * 16) <= 3 * most
 
 
 def few_rows(m: int, weight: torch.Tensor) -> bool:

@@ -115,18 +115,17 @@ class GatedSum:
 @dataclass
 class GatedStream:
     """Where a branch's result y goes with few rows: `stream` += g * y in the epilogue of y's last product, g by the columns of the gates' products
-    z [N, columns] from `column` on, and `bias` (`column` None: 1).  The branch returns `ADDED_IN_PLACE` then.  The stream is 32-bit."""
+    z [N, columns] from `column` on, and `bias`.  The branch returns `ADDED_IN_PLACE` then.  The stream is 32-bit."""
 
     stream: torch.Tensor
-    z: "torch.Tensor | None"
-    column: "int | None"
+    z: torch.Tensor
+    column: int
     bias: "torch.Tensor | None"
 
     def add(self, x: torch.Tensor, weight: torch.Tensor):
         from ..ops import library as ops
 
-        gate = None if self.column is None else (self.z, self.column, self.bias)
-        ops.gemm_decode(None, x, weight, residual=self.stream, gate=gate)
+        ops.gemm_decode(None, x, weight, residual=self.stream, gate=(self.z, self.column, self.bias))
         return ADDED_IN_PLACE
 
 
