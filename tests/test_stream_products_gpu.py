@@ -65,6 +65,31 @@ def test_normed(n, k, cols, swiglu):
         close(h, apart.double().cpu(), rounded(after.cpu())[1])
 
 
+@pytest.mark.parametrize("n,k,inter", [(1, 8, 5), (5, 1024, 2049), (8, 2304, 1000), (3, 3072, 5000), (8, 4096, 513)])
+@pytest.mark.parametrize("unit", ["silu", "clamped"])
+def test_gated_units(n, k, inter, unit):
+    x, y, yw = rnd(n, k, seed=1), rnd(n, k, seed=2, scale=3.0), 1.0 + rnd(k, seed=3, scale=0.1)
+    w = rnd(2 * inter, k, seed=4, scale=k ** -0.5).to(torch.bfloat16)
+    h, after = torch.empty(n, k, dtype=torch.bfloat16, device=DEV), torch.empty(n, k, device=DEV)
+    out = torch.full((n, inter), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops().gemm_decode_stream(out, x.to(DEV), w.to(DEV), joins=(y.to(DEV), yw.to(DEV), 1e-5, after), h_out=h, swiglu=True,
+                             limit=1.5 if unit == "clamped" else None)
+    sums = h.double().cpu() @ w.double().t()
+    gate, up = sums[:, :inter], sums[:, inter:]
+    off = 4e-6 * math.sqrt(k) * float(sums.abs().max())  # of the sums
+    if unit == "clamped":  # in 32-bit, rounded once (half a step of 8 bits); slopes of the unit up to 1.1 and of its factor up to 1
+        g, v = gate.clamp(max=1.5), up.clamp(-1.5, 1.5) + 1.0
+        want = g * torch.sigmoid(1.702 * g) * v
+        bound = 2.0 ** -8 * want.abs() + off * (1.1 * v.abs() + 1.5)
+    else:  # gate, up and silu(gate) are rounded, and then the result: half a step each (2^-8 of a number just beyond a power of two)
+        want = gate * torch.sigmoid(gate) * up
+        bound = 2.0 ** -8 * (1.1 * gate.abs() * up.abs() + 3.0 * want.abs()) * 1.02 + off * (1.1 * up.abs() + gate.abs())
+    wrong = (out.double().cpu() - want).abs() > bound
+    assert not wrong.any(), (int(wrong.sum()), float((out.double().cpu() - want).abs().max()))
+    # beside the product of the same rows: the same sums, the same unit
+    assert torch.equal(out, ops().gemm_decode(torch.empty_like(out), h, w.to(DEV), swiglu=True, limit=1.5 if unit == "clamped" else None))
+
+
 @pytest.mark.parametrize("n,k,cols", SIZES)
 @pytest.mark.parametrize("keep", [False, True])
 def test_norm(n, k, cols, keep):
