@@ -352,7 +352,12 @@ int llms_attend_latent_mfma(void* out, const void* q, const void* pool, const in
     a.page_magic = block_size == 1 ? 0u : (uint32_t)(((1ull << 32) + block_size - 1) / block_size);
     const long long blocks = ((long long)max_count * heads + LM_PAIRS - 1) / LM_PAIRS;
     LLMS_REQUIRE(blocks < (1ll << 31) && n_seqs <= 65535, "attend_latent_mfma: too many workgroups for one launch");
-    dim3 grid((unsigned)blocks, n_seqs, splits);
+    // Workgroups go around the 8 XCDs in the grid's order, a request's row of blocks behind the other's.  With rows of a multiple of 8 every request's first
+    // block, the only one of a single token, lies on the same XCD: a block more then where at least half of the grid has no rows.  (32 heads over latents of
+    // 256, microseconds: 60 tokens beside a portion of 64 behind 800 keys 306 -> 90, in 2 shares 325 -> 65; 8 beside 256 behind 900 198 -> 116; 3 beside
+    // 210, in rows of 224, 54 -> 39.  Full rows lose by it, whose blocks would no longer be as many on every XCD: 16 portions of 64 28 and 44.)
+    const bool mostly_empty = 2ll * n_rows <= (long long)n_seqs * max_count;
+    dim3 grid((unsigned)(blocks % 8 == 0 && mostly_empty ? blocks + 1 : blocks), n_seqs, splits);
     const size_t lds = ((size_t)LM_KEYS * (a.dkp + 8) + (size_t)r * LM_CLD) * sizeof(uint16_t);
     int status = rt == 8 ? launch_latent<8>(a, grid, lds, stream)
                  : rt == 16 ? launch_latent<16>(a, grid, lds, stream)

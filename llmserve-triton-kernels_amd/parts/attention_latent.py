@@ -197,7 +197,8 @@ class LatentAttention(Mixer):
         than writing and adding up the shares of every (token, head) pair costs: some 0.0125 r microseconds a tile against 7e-6 r
         a pair and share (16 heads of 256 in 1, 4 shares: 448 tokens beside 5 behind 900 keys 90 and 76 microseconds, 200 beside 20
         behind 1,500 142 and 59; 32 heads in 1, 2: 92 and 131, 144 and 101; 400 tokens beside 100 behind 400 46 and 79).  Not with
-        mostly single tokens, whose blocks may all lie on one XCD (60 tokens beside 60 behind 800 keys, in 1 and 3: 143 and 163)."""
+        mostly single tokens: the line was drawn when their blocks might all lie on one XCD (60 tokens beside 60 behind 800 keys, 16 heads, in 1 and 2:
+        151 and 161; 88 and 58 since they lie on all, which the rule has not followed yet)."""
         blocks = n_requests * -(-max_new * self.heads // ops.LATENT_MFMA_PAIRS)
         reach = max_context if self.window is None else min(max_context, self.window + max_new - 1)
         tiles = -(-reach // ops.LATENT_MFMA_KEYS) + 1
